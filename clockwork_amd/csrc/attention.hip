@@ -331,13 +331,17 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
   const int gh = p.gh;
   const int64_t base = ((int64_t)item * gridDim.y + blockIdx.y) * p.n_splits;
   T* op = (T*)p.out;
-  for (int idx = threadIdx.x; idx < ROWS * HD; idx += 256) {
+  // a thread has one element, and its splits' numbers are asked for side by side
+  const int idx = blockIdx.z * 256 + threadIdx.x;
+  if (idx < ROWS * HD) {
     const int r = idx / HD, d = idx - r * HD;
     const int tok = r / gh, hig = chunk * gh + (r - tok * gh);
-    if (tok >= ntok || hig >= group) continue;
+    if (tok >= ntok || hig >= group) return;
     float M = -INFINITY;
+#pragma unroll 4
     for (int s = 0; s < p.n_splits; ++s) M = fmaxf(M, p.part_ml[((base + s) * ROWS + r) * 2]);
     float L = 0.0f, O = 0.0f;
+#pragma unroll 4
     for (int s = 0; s < p.n_splits; ++s) {
       const float m = p.part_ml[((base + s) * ROWS + r) * 2];
       if (m == -INFINITY) continue;
@@ -373,7 +377,7 @@ static int launch_attention(const AttnParams& p, int n_items, hipStream_t stream
   dim3 grid(n_items, p.nkv * p.n_chunks, p.n_splits), block(256);
   hipLaunchKernelGGL((attn_tile_kernel<T, HD, ROWS, BN>), grid, block, smem, stream, p);
   if (p.n_splits > 1) {
-    dim3 mgrid(n_items, p.nkv * p.n_chunks);
+    dim3 mgrid(n_items, p.nkv * p.n_chunks, (ROWS * HD + 255) / 256);
     hipLaunchKernelGGL((attn_merge_kernel<T, HD, ROWS>), mgrid, block, 0, stream, p);
   }
   return cw_launch_status();

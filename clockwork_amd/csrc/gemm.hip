@@ -1,120 +1,399 @@
 // Matrix products y = x * W^T (+ bias) for gfx950, W stored [N, K] row-major as checkpoints
 // hold it.
-//  * cw_gemm_f32: true float32 (VALU FMA, float32 operands and accumulation, no reduced-precision
-//    matrix mode). The order in which the products of one output element are summed depends on N
-//    and K alone, never on M, so a row's result does not depend on what else is in the batch.
+//  * cw_gemm_f32: true float32 on the matrix cores (v_mfma_f32_16x16x4_f32: float32 operands, products
+//    and sums). The order in which the products of one output element are summed depends on N and K
+//    alone, never on M, so a row's result does not depend on what else is in the batch.
 #include "common.h"
 
-#define GT_BM 64
-#define GT_BN 64
-#define GT_BK 16
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
-// C[M, N] = A[M, K] * W[N, K]^T + bias[N]. 256 threads, each a 4x4 tile of a 64x64 block.
-// K is summed in ``splits`` parts of k_per_split values (a multiple of 16), and the parts in their
-// order: ((p_0 + p_1) + ...) + bias. gridDim.z == 1: a block does so by itself. gridDim.z ==
-// splits: block z makes part z alone and writes it to C + z * part_stride (no bias), and
-// gemm_f32_sum_kernel adds the parts up in the same order, so both ways give the same bits.
-// ONE_PART: a block makes one part (gridDim.z == splits, or there is only one part).
-template <bool ONE_PART>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ A, int64_t lda,
-                                                       const float* __restrict__ W,
-                                                       const float* __restrict__ bias,
-                                                       float* __restrict__ C, int64_t ldc, int M,
-                                                       int N, int K, int splits, int k_per_split,
-                                                       int64_t part_stride) {
-  __shared__ float As[GT_BK][GT_BM + 4];
-  __shared__ float Ws[GT_BK][GT_BN + 4];
-  const int tid = threadIdx.x;
-  const int tx = tid & 15, ty = tid >> 4;
-  const int m0 = blockIdx.y * GT_BM, n0 = blockIdx.x * GT_BN;
-  const bool parallel = gridDim.z > 1;  // part blockIdx.z of several
-  const int z_first = ONE_PART ? blockIdx.z : 0, z_last = ONE_PART ? blockIdx.z : splits - 1;
-  float total[4][4];
-  // each thread loads 4 elements of A and 4 of W per K step: row = tid / 4, k = (tid % 4) * 4 .. +3
-  const int lr = tid >> 2, lk = (tid & 3) * 4;
-  const bool k_vec_ok = (K % 4 == 0) && (lda % 4 == 0);
-  for (int z = z_first; z <= z_last; ++z) {
-  const int k_begin = z * k_per_split;
-  const int k_end = min(K, k_begin + k_per_split);
-  float acc[4][4];
+// How these kernels load operands of few rows. An MFMA operand wants lane l to hold row l % 16 of a tile and
+// the 8 k-values of slot l / 16: loaded that way every lane asks for 16 bytes of a row of its own,
+// 64 requests an instruction to a compute unit's load path, which takes in about 30 GB/s of such.
+// So a lane loads row l / 4, slot l % 4 instead (four neighbouring lanes cover 64 bytes of one row:
+// 16 requests an instruction), and the lanes swap what they hold afterwards, lane (r, s) taking
+// from lane 4 r + s (ds_bpermute: through the LDS unit's crossbar, no memory). Measured on the
+// 1.5B shape's gate/up product: 12.8 -> 11.7 us with 8 rows of x, 19.8 -> 17.5 us with 64.
+typedef __attribute__((ext_vector_type(4))) int cw_i32x4_t;
+__device__ __forceinline__ cw_i32x4_t cw_swap_to_operand(const cw_i32x4_t& q, int lane) {
+  const int r = lane & 15, s = lane >> 4;
+  const int from = (r * 4 + s) * 4;  // byte address of the lane that loaded what lane (r, s) multiplies
+  cw_i32x4_t t;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int d = 0; d < 4; ++d) t[d] = __builtin_amdgcn_ds_bpermute(from, q[d]);
+  return t;
+}
+__device__ __forceinline__ bf16x8_t cw_to_operand_layout(const bf16x8_t& v, int lane) {
+  return __builtin_bit_cast(bf16x8_t, cw_swap_to_operand(__builtin_bit_cast(cw_i32x4_t, v), lane));
+}
+
+// =====================================================================================
+// float32. What a product of one output element is, whichever kernel makes it: K is cut into parts
+// (gemm_f32_plan), a part into blocks of 16 k-values. Lane (row, s) of an operand holds k-values
+// 4 s .. 4 s + 3 of a block; the four MFMAs of a block, the j-th with element j of every lane, sum it
+// from zero; the blocks' sums are added up in order, then the parts' in order, then the bias. (A sum of
+// 16 on its own before it joins the total: a long K, 8960 in a feed-forward, rounds about
+// sqrt(16) + sqrt(K / 16) times instead of sqrt(K).)
+__device__ __forceinline__ f32x4_t gemm_f32_block(const f32x4_t& w, const f32x4_t& x) {
+  f32x4_t t = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
-  for (int k0 = k_begin; k0 < k_end; k0 += GT_BK) {
-    {
-      const int m = m0 + lr, k = k0 + lk;
-      float v[4] = {0.f, 0.f, 0.f, 0.f};
-      if (m < M) {
-        const float* p = A + (int64_t)m * lda + k;
-        if (k_vec_ok && k + 3 < k_end) {
-          const float4 q = *reinterpret_cast<const float4*>(p);
-          v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
-        } else {
+  for (int j = 0; j < 4; ++j) t = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j], x[j], t, 0, 0, 0);
+  return t;
+}
+
+// Four k-values of a row from k on; zeros from k_end on. VEC: rows of 16-byte multiples (k and k_end are
+// multiples of 4 then), loaded from a clamped address so that the load does not hang on a condition.
+template <bool VEC>
+__device__ __forceinline__ f32x4_t gemm_f32_load4(const float* __restrict__ row, int k, int k_end) {
+  f32x4_t v;
+  if (VEC) {
+    const bool ok = k < k_end;
+    v = *reinterpret_cast<const f32x4_t*>(row + (ok ? k : 0));
 #pragma unroll
-          for (int j = 0; j < 4; ++j) if (k + j < k_end) v[j] = p[j];
-        }
+    for (int j = 0; j < 4; ++j) v[j] = ok ? v[j] : 0.0f;
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = k + j < k_end ? row[k + j] : 0.0f;
+  }
+  return v;
+}
+
+// Up to 16 rows of x (single tokens): W is streamed once, straight into the operands' registers. A wave
+// owns 16 rows of W and a run of the parts of K; ``part_waves`` waves share a tile's parts and the block
+// holds blockDim / 64 / part_waves tiles. What bounds it is the stream of W (and, for the small
+// projections, one trip to memory): eight blocks of 16 k-values are on their way while eight are multiplied.
+// With plane_stride > 0 a part's sum is written out as plane z of C (whoever reads y next adds the planes
+// in order); else the parts meet in LDS.
+// Measured on an MI355X with one row of x, the four products of a layer of the 0.5B shape: 42 us (q/k/v 9.5, output
+// 9.2, gate/up 13.6 for 35 MB, down 9.5), against 111 us of vector-unit tiles of 64 x 64 with partial sums in memory
+// and 20 us for the kernels that added them.
+template <bool VEC>
+__global__ __launch_bounds__(512) void gemm_f32_rows_kernel(const float* __restrict__ A, int64_t lda,
+                                                            const float* __restrict__ W,
+                                                            const float* __restrict__ bias,
+                                                            float* __restrict__ C, int64_t ldc, int M, int N, int K,
+                                                            int parts, int k_per_part, int part_waves,
+                                                            int64_t plane_stride) {
+  extern __shared__ __align__(16) float red[];  // [tile of the block][part][token][row of W]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, s = lane >> 4, lr = lane >> 2, ls = lane & 3;
+  const int tiles_here = (blockDim.x >> 6) / part_waves;
+  const int tile_here = wave / part_waves;
+  const int64_t n0 = ((int64_t)blockIdx.x * tiles_here + tile_here) * 16;
+  const float* wrow = W + min(n0 + lr, (int64_t)N - 1) * K;
+  const float* xrow = A + (int64_t)min(r, M - 1) * lda;
+  constexpr int U = 8;
+  const int z_step = part_waves * gridDim.y;
+  for (int z = blockIdx.y * part_waves + wave % part_waves; z < parts; z += z_step) {
+    const int k_begin = z * k_per_part, k_end = min(K, k_begin + k_per_part);
+    const int blocks = (k_end - k_begin + 15) / 16;
+    f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4_t wa[U], xa[U], wb[U], xb[U];
+    auto load = [&](f32x4_t (&w)[U], f32x4_t (&x)[U], int b0) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = k_begin + (b0 + u) * 16;
+        w[u] = gemm_f32_load4<VEC>(wrow, k + 4 * ls, k_end);
+        x[u] = gemm_f32_load4<VEC>(xrow, k + 4 * s, k_end);
       }
+    };
+    auto multiply = [&](const f32x4_t (&w)[U], const f32x4_t (&x)[U], int b0) __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) As[lk + j][lr] = v[j];
-    }
-    {
-      const int n = n0 + lr, k = k0 + lk;
-      float v[4] = {0.f, 0.f, 0.f, 0.f};
-      if (n < N) {
-        const float* p = W + (int64_t)n * K + k;
-        if (K % 4 == 0 && k + 3 < k_end) {
-          const float4 q = *reinterpret_cast<const float4*>(p);
-          v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) if (k + j < k_end) v[j] = p[j];
-        }
+      for (int u = 0; u < U; ++u) {
+        if (b0 + u >= blocks) break;
+        acc += gemm_f32_block(__builtin_bit_cast(f32x4_t, cw_swap_to_operand(__builtin_bit_cast(cw_i32x4_t, w[u]), lane)), x[u]);
       }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) Ws[lk + j][lr] = v[j];
+    };
+    load(wa, xa, 0);
+    for (int b0 = 0; b0 < blocks; b0 += 2 * U) {
+      if (b0 + U < blocks) load(wb, xb, b0 + U);
+      multiply(wa, xa, b0);
+      if (b0 + U >= blocks) break;
+      if (b0 + 2 * U < blocks) load(wa, xa, b0 + 2 * U);
+      multiply(wb, xb, b0 + U);
     }
+    // lane (r, s) holds rows 4 s .. 4 s + 3 of W for token r
+    if (plane_stride > 0) {
+      float* out = C + (int64_t)z * plane_stride + (int64_t)r * ldc + n0 + 4 * s;
+      if (r < M)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (n0 + 4 * s + i < N) out[i] = acc[i];
+    } else {
+      *reinterpret_cast<f32x4_t*>(&red[(tile_here * parts + z) * 256 + r * 16 + 4 * s]) = acc;
+    }
+  }
+  if (plane_stride > 0) return;
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < tiles_here * 256; idx += blockDim.x) {
+    const int m = (idx >> 4) & 15, t = idx >> 8;
+    const int64_t n = ((int64_t)blockIdx.x * tiles_here + t) * 16 + (idx & 15);
+    const float* p = red + t * parts * 256 + (idx & 255);
+    float total = p[0];
+    for (int z = 1; z < parts; ++z) total += p[z * 256];
+    if (m < M && n < N) C[(int64_t)m * ldc + n] = total + (bias ? bias[n] : 0.0f);
+  }
+}
+
+// A wave's sums to C, 2 x TM tiles from row m0 of x and row n0 of W: lane (r, s) holds rows 4 s .. 4 s + 3 of
+// W for token r of each.
+template <int TM>
+__device__ __forceinline__ void gemm_f32_store_tile(const f32x4_t (&total)[2][TM], float* __restrict__ C,
+                                                    const float* __restrict__ bias, int plane, int64_t plane_stride,
+                                                    int64_t ldc, int m0, int n0, int M, int N, int r, int s) {
+  const bool planes = plane_stride > 0;
+  float* out = C + (int64_t)plane * plane_stride;
+  const bool vec_store = !(ldc & 3) && !((uintptr_t)out & 15);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      const int m = m0 + 16 * j + r, n = n0 + 16 * i + 4 * s;
+      if (m >= M) continue;
+      f32x4_t v = total[i][j];
+      if (bias && !planes)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += n + e < N ? bias[n + e] : 0.0f;
+      float* p = out + (int64_t)m * ldc + n;
+      if (vec_store && n + 4 <= N) {
+        *reinterpret_cast<f32x4_t*>(p) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) p[e] = v[e];
+      }
+    }
+}
+
+// More rows, of any length: tiles of 64 rows of x by 64 rows of W, 256 threads, the K loop through registers
+// and LDS in steps of 32 (two buffers, the next step's loads on their way over the products of this one). Wave
+// (i, j) of the 2 x 2 owns 32 rows of W and 32 of x. A row of a step takes 36 floats in LDS: the 16 rows that a
+// quarter of a wave reads 16 bytes of then begin in 16 different groups of four banks.
+// gridDim.z > 1: block z makes part z alone, into plane z of C; else a block adds its parts up itself.
+// For rows that gemm_f32_ring_kernel does not take (K no multiple of 16).
+template <bool VEC, bool ONE_PART>
+__global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restrict__ A, int64_t lda,
+                                                            const float* __restrict__ W,
+                                                            const float* __restrict__ bias,
+                                                            float* __restrict__ C, int64_t ldc, int M, int N, int K,
+                                                            int parts, int k_per_part, int64_t plane_stride) {
+  constexpr int BM = 64, BN = 64, BK = 32, LD = BK + 4, TM = BM / 32, XL = BM / 32;
+  __shared__ __align__(16) float Ws[2][BN * LD];
+  __shared__ __align__(16) float Xs[2][BM * LD];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane & 15, s = lane >> 4;
+  const int wn = (wave & 1) * 32, wm = (wave >> 1) * (BM / 2);
+  const int n0 = blockIdx.x * BN, m0 = blockIdx.y * BM;
+  const int z_first = ONE_PART ? blockIdx.z : 0, z_last = ONE_PART ? blockIdx.z : parts - 1;
+
+  // what this thread brings in: 16 bytes of rows tid / 8 and tid / 8 + 32 of a step
+  const int lrow = tid >> 3, lk = (tid & 7) * 4;
+  const float* wrow[2];
+  const float* xrow[XL];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) wrow[i] = W + (int64_t)min(n0 + lrow + 32 * i, N - 1) * K;
+#pragma unroll
+  for (int i = 0; i < XL; ++i) xrow[i] = A + (int64_t)min(m0 + lrow + 32 * i, M - 1) * lda;
+  f32x4_t wreg[2], xreg[XL];
+  auto load = [&](int k0, int k_end) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) wreg[i] = gemm_f32_load4<VEC>(wrow[i], k0 + lk, k_end);
+#pragma unroll
+    for (int i = 0; i < XL; ++i) xreg[i] = gemm_f32_load4<VEC>(xrow[i], k0 + lk, k_end);
+  };
+  auto store = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) *reinterpret_cast<f32x4_t*>(&Ws[buf][(lrow + 32 * i) * LD + lk]) = wreg[i];
+#pragma unroll
+    for (int i = 0; i < XL; ++i) *reinterpret_cast<f32x4_t*>(&Xs[buf][(lrow + 32 * i) * LD + lk]) = xreg[i];
+  };
+
+  f32x4_t acc[2][TM], total[2][TM];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) acc[i][j] = total[i][j] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
+
+  int z = z_first, k0 = z * k_per_part, k_end = min(K, k0 + k_per_part), buf = 0;
+  load(k0, k_end);
+  store(0);
+  __syncthreads();
+  while (true) {
+    // the step after this one: of the same part, or the first of the next
+    int next_z = z, next_k0 = k0 + BK, next_end = k_end;
+    const bool last_of_part = next_k0 >= k_end;
+    if (last_of_part) {
+      next_z = z + 1;
+      next_k0 = next_z * k_per_part;
+      next_end = min(K, next_k0 + k_per_part);
+    }
+    const bool more = next_z <= z_last;
+    if (more) load(next_k0, next_end);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      if (b == 1 && k0 + 16 >= k_end) break;  // a part is a whole number of blocks, not of steps
+      f32x4_t wf[2], xf[TM];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) wf[i] = *reinterpret_cast<const f32x4_t*>(&Ws[buf][(wn + 16 * i + r) * LD + b * 16 + 4 * s]);
+#pragma unroll
+      for (int j = 0; j < TM; ++j) xf[j] = *reinterpret_cast<const f32x4_t*>(&Xs[buf][(wm + 16 * j + r) * LD + b * 16 + 4 * s]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) acc[i][j] += gemm_f32_block(wf[i], xf[j]);
+    }
+    if (last_of_part) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) {
+          total[i][j] = (ONE_PART || z == z_first) ? acc[i][j] : total[i][j] + acc[i][j];
+          acc[i][j] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
+    if (!more) break;
+    buf ^= 1;
+    store(buf);
     __syncthreads();
-    // the 16 products of a K step are summed on their own and then added to the total: a long K
-    // (8960 in a feed-forward) then rounds about sqrt(16) + sqrt(K / 16) times instead of sqrt(K)
-    float part[4][4];
+    z = next_z;
+    k0 = next_k0;
+    k_end = next_end;
+  }
+
+  gemm_f32_store_tile<TM>(total, C, bias, blockIdx.z, plane_stride, ldc, m0 + wm, n0 + wn, M, N, r, s);
+}
+
+// The same product, rows of whole blocks of 16 k-values: tiles of BM rows of x by 64 rows of W, K in stages of
+// 32 values that go from global memory straight into LDS (buffer loads with the LDS target), a ring of four.
+// What bounds it is the trip to memory of a tile's stages: a compute unit has one to three tiles at a time, and
+// with one stage under way over another's products (0.2 to 0.4 us against a trip of 1 us and more) it waited
+// most of the time; three are under way here. A load instruction brings eight rows of 128 bytes; the eight 16-byte
+// granules of row R change places by (R >> 1) & 7, so that the 16 lanes that read one granule of 16 rows touch
+// every bank once. The descriptors end with the matrices: rows past the end read as zeros. What a stage holds past
+// the end of its part is not multiplied. BM is 32 where 64 would leave compute units without a tile.
+// Measured on an MI355X, the four products of a layer of the 0.5B shape with 384 rows: 919 us on 64 x 64 tiles of
+// the vector units, 163 us here (q/k/v 17, output 17, gate/up 83 at 81 TFLOP/s, down 46).
+typedef __attribute__((address_space(3))) void lds_void_t;
+// s_waitcnt for "at most n vector-memory operations in flight" and nothing else
+#define GF_WAIT_LOADS(n) __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | (((n) >> 4) << 14))
+// a barrier without a fence (a fence would wait for every load in flight)
+#define GF_BARRIER()               \
+  do {                             \
+    asm volatile("" ::: "memory"); \
+    __builtin_amdgcn_s_barrier();  \
+    asm volatile("" ::: "memory"); \
+  } while (0)
+
+template <int BM, bool ONE_PART>
+__global__ __launch_bounds__(256, 2) void gemm_f32_ring_kernel(const float* __restrict__ A, int64_t lda,
+                                                            const float* __restrict__ W,
+                                                            const float* __restrict__ bias,
+                                                            float* __restrict__ C, int64_t ldc, int M, int N, int K,
+                                                            int parts, int k_per_part, int64_t plane_stride) {
+  constexpr int BN = 64, BK = 32, SLOTS = 4, TM = BM / 32;
+  constexpr int XB = BM / 8, WB = BN / 8, LOADS = (XB + WB) / 4;  // 1 KB blocks of a stage; loads of a wave
+  constexpr int STAGE = (XB + WB) * 1024;
+  extern __shared__ __align__(1024) unsigned char ring[];  // SLOTS * STAGE bytes
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, s = lane >> 4;
+  const int wn = (wave & 1) * 32, wm = (wave >> 1) * (BM / 2);
+  // Workgroups are dealt to the 8 XCDs in turn. Each XCD takes a run of neighbouring tiles, those of the same rows
+  // of W next to each other: W then comes from memory once, into one L2.
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  const int run = gridDim.x >> 3, rest = gridDim.x & 7, xcd = blockIdx.x & 7;
+  const int tile = xcd * run + min(xcd, rest) + (blockIdx.x >> 3);
+  const int m0 = tile % tiles_m * BM, n0 = tile / tiles_m % tiles_n * BN;
+  const int plane = tile / (tiles_m * tiles_n);
+  const int z_first = ONE_PART ? plane : 0, z_last = ONE_PART ? plane : parts - 1;
+
+  __amdgpu_buffer_rsrc_t xr, wr;
+  xr = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(A + (int64_t)m0 * lda), 0, (int)(uint32_t)(((int64_t)(M - m0 - 1) * lda + K) * 4), 0x00020000);
+  wr = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(W + (int64_t)n0 * K), 0, (int)(uint32_t)(((int64_t)(N - n0 - 1) * K + K) * 4), 0x00020000);
+  // load i of a wave: block wave * LOADS + i of a stage, the x blocks first
+  uint32_t at[4];  // (of a size that hangs on no template parameter, as the buffer is: the host pass drops the kernel otherwise)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < LOADS; ++i) {
+    const int block = wave * LOADS + i, row = (block < XB ? block : block - XB) * 8 + (lane >> 3);
+    const int granule = (lane & 7) ^ ((row >> 1) & 7);
+    at[i] = (uint32_t)(((int64_t)row * (block < XB ? lda : K) + granule * 4) * 4);
+  }
+  auto fetch = [&](int k0, int slot) __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) part[i][j] = 0.0f;
+    for (int i = 0; i < LOADS; ++i) {
+      const int block = wave * LOADS + i;
+      unsigned char* to = ring + (slot * STAGE + block * 1024);
+      if (block < XB) __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t*)to, 16, at[i], k0 * 4, 0, 0);
+      else __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void_t*)to, 16, at[i], k0 * 4, 0, 0);
+    }
+  };
+  // the stage that is asked for next; past the last one it is asked for again (nobody reads it, but the
+  // number of loads in flight stays what the waits count on)
+  int fz = z_first, fk = z_first * k_per_part;
+  auto fetch_next = [&](int slot) __attribute__((always_inline)) {
+    fetch(fk, slot);
+    const int end = min(K, (fz + 1) * k_per_part);
+    if (fk + BK < end) fk += BK;
+    else if (fz < z_last) fk = ++fz * k_per_part;
+  };
+  f32x4_t acc[2][TM], total[2][TM], t[2][TM];  // t: the sum of the last block, not added to acc yet
 #pragma unroll
-    for (int kk = 0; kk < GT_BK; ++kk) {
-      const float4 a = *reinterpret_cast<const float4*>(&As[kk][ty * 4]);
-      const float4 w = *reinterpret_cast<const float4*>(&Ws[kk][tx * 4]);
-      const float av[4] = {a.x, a.y, a.z, a.w};
-      const float wv[4] = {w.x, w.y, w.z, w.w};
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < TM; ++j) acc[i][j] = total[i][j] = t[i][j] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) part[i][j] = fmaf(av[i], wv[j], part[i][j]);
+  for (int i = 0; i < SLOTS - 1; ++i) fetch_next(i);
+  const unsigned char* mine = ring + r * 128;
+  const int turn = (r >> 1) & 7;
+  for (int z = z_first, slot = 0; z <= z_last; ++z) {
+    const int k_end = min(K, (z + 1) * k_per_part);
+    for (int k0 = z * k_per_part; k0 < k_end; k0 += BK, slot = (slot + 1) % SLOTS) {
+      // this wave's loads of the stage are in; behind the barrier every wave's are, and every wave has read the
+      // stage before it, whose slot the next loads take
+      GF_WAIT_LOADS((SLOTS - 2) * LOADS);
+      GF_BARRIER();
+      fetch_next((slot + SLOTS - 1) % SLOTS);
+      const unsigned char* xs = mine + slot * STAGE + wm * 128;
+      const unsigned char* ws = mine + slot * STAGE + XB * 1024 + wn * 128;
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        if (b == 1 && k0 + 16 >= k_end) break;  // a part is a whole number of blocks, not of stages
+        f32x4_t wf[2], xf[TM], next[2][TM];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) wf[i] = *reinterpret_cast<const f32x4_t*>(ws + i * 2048 + ((b * 4 + s) ^ turn) * 16);
+#pragma unroll
+        for (int j = 0; j < TM; ++j) xf[j] = *reinterpret_cast<const f32x4_t*>(xs + j * 2048 + ((b * 4 + s) ^ turn) * 16);
+        // gemm_f32_block for each pair, the pairs' products taking turns; the sums of the block before join the
+        // totals meanwhile (added at once they would wait for the last product, with the matrix core idle)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < TM; ++j)
+              next[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][q], xf[j][q], q == 0 ? (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f} : next[i][j], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < TM; ++j) {
+            acc[i][j] += t[i][j];
+            t[i][j] = next[i][j];
+          }
+      }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] += part[i][j];
-    __syncthreads();
+      for (int j = 0; j < TM; ++j) {
+        acc[i][j] += t[i][j];
+        total[i][j] = (ONE_PART || z == z_first) ? acc[i][j] : total[i][j] + acc[i][j];
+        acc[i][j] = t[i][j] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
+      }
   }
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) total[i][j] = (ONE_PART || z == z_first) ? acc[i][j] : total[i][j] + acc[i][j];
-  }
-  float* out = parallel ? C + (int64_t)blockIdx.z * part_stride : C;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty * 4 + i;
-    if (m >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx * 4 + j;
-      if (n < N) out[(int64_t)m * ldc + n] = total[i][j] + (bias && !parallel ? bias[n] : 0.0f);
-    }
-  }
+  GF_WAIT_LOADS(0);  // no load may reach LDS after the workgroup has gone
+  gemm_f32_store_tile<TM>(total, C, bias, plane, plane_stride, ldc, m0 + wm, n0 + wn, M, N, r, s);
 }
 
 // C[m, n] = ((p_0 + p_1) + ... + p_{splits-1}) + bias[n] over the partial sums p_z[m, n] (rows of N
@@ -130,9 +409,12 @@ __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(const float* __restri
   C[(int64_t)m * ldc + n] = total + (bias ? bias[n] : 0.0f);
 }
 
-// Up to this many rows of x the parts of K are made by blocks of their own (beyond, there are
+// Up to this many rows of x the parts of K are made by blocks of their own (beyond, there are mostly
 // blocks enough without, and a block sums its parts itself).
 #define GT_SPLIT_ROWS 256
+#define GT_ROWS_MAX 16    // gemm_f32_rows_kernel's rows
+#define GT_LDS_PARTS 48   // parts that may meet in that kernel's LDS (1 KB each)
+#define GT_MAX_PLANES 64  // planes that the residual-add + norm kernel adds
 
 // How the float32 product cuts K for an [N, K] weight matrix: a narrow output (24 blocks of 64
 // columns for a width of 1536) with few rows of x would leave most compute units without work and
@@ -140,21 +422,89 @@ __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(const float* __restri
 // per 64 rows, with at least 256 values of K each. A function of N and K alone: the order of the
 // sums must not depend on how many rows the step has.
 static void gemm_f32_plan(int N, int K, int* splits, int* k_per_split) {
-  const int col_blocks = (N + GT_BN - 1) / GT_BN;
+  const int col_blocks = (N + 63) / 64;
   int s = (512 + col_blocks / 2) / col_blocks;
   if (s > K / 256) s = K / 256;
   if (s < 1) s = 1;
-  const int per = ((K + s - 1) / s + GT_BK - 1) / GT_BK * GT_BK;
+  const int per = ((K + s - 1) / s + 15) / 16 * 16;
   *k_per_split = per;
   *splits = (K + per - 1) / per;
+}
+
+// Are the parts of K made apart, as planes of partial sums, for this many rows? Up to GT_SPLIT_ROWS rows
+// always (but not where the parts of few rows meet in LDS); beyond, where tiles of 64 x 64 would leave
+// compute units idle and K is long enough to pay for writing and reading the planes (300 rows of the 0.5B
+// shape's down product, 70 tiles of 4864 k-values: 65 us for the products of one tile, 46 us as 19 planes).
+static bool gemm_f32_planes(int M, int N, int K, int splits) {
+  if (splits <= 1) return false;
+  if (M <= GT_ROWS_MAX) return splits > GT_LDS_PARTS;
+  if (M <= GT_SPLIT_ROWS) return true;
+  return K >= 2048 && (int64_t)((M + 63) / 64) * ((N + 63) / 64) < 96;
 }
 
 // Floats of workspace cw_gemm_f32 needs for this product (0: none).
 CW_EXPORT int64_t cw_gemm_f32_workspace_floats(int M, int N, int K) {
   int splits, per;
-  if (M <= 0 || M > GT_SPLIT_ROWS || N <= 0 || K <= 0) return 0;
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
   gemm_f32_plan(N, K, &splits, &per);
-  return splits <= 1 ? 0 : (int64_t)splits * M * N;
+  return gemm_f32_planes(M, N, K, splits) ? (int64_t)splits * M * N : 0;
+}
+
+// Planes of partial sums that cw_gemm_f32_partial writes for this product, 0 where it should not be
+// asked: one part, blocks enough without, or more planes than the norm kernel adds.
+CW_EXPORT int cw_gemm_f32_partial_planes(int M, int N, int K) {
+  int splits, per;
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  gemm_f32_plan(N, K, &splits, &per);
+  if (splits <= 1 || splits > GT_MAX_PLANES) return 0;
+  return M <= GT_ROWS_MAX || gemm_f32_planes(M, N, K, splits) ? splits : 0;
+}
+
+// C: y [M, N] with row stride ldc, or with planes float32 [splits, M, N].
+static int launch_gemm_f32(const float* A, int64_t lda, const float* W, const float* bias, float* C, int64_t ldc, int M,
+                           int N, int K, int splits, int per, bool planes, hipStream_t stream) {
+  const bool vec = !(K & 3) && !(lda & 3);
+  const int64_t stride = planes ? (int64_t)M * N : 0;
+  if (M <= GT_ROWS_MAX) {
+    // as planes: four parts a block, each wave its own. Else all of a tile's parts in one block of up to
+    // eight waves, and as many tiles as make it four waves or more.
+    const int part_waves = planes ? (splits < 4 ? splits : 4) : (splits + (splits + 7) / 8 - 1) / ((splits + 7) / 8);
+    const int tiles_here = planes || part_waves >= 4 ? 1 : 4 / part_waves;
+    const int tiles = (N + 15) / 16;
+    const dim3 grid((tiles + tiles_here - 1) / tiles_here, planes ? (splits + part_waves - 1) / part_waves : 1);
+    const dim3 block(64 * part_waves * tiles_here);
+    const size_t lds = planes ? 0 : (size_t)tiles_here * splits * 256 * sizeof(float);
+    if (vec) hipLaunchKernelGGL(gemm_f32_rows_kernel<true>, grid, block, lds, stream, A, lda, W, bias, C, ldc, M, N, K, splits, per, part_waves, stride);
+    else hipLaunchKernelGGL(gemm_f32_rows_kernel<false>, grid, block, lds, stream, A, lda, W, bias, C, ldc, M, N, K, splits, per, part_waves, stride);
+    return cw_launch_status();
+  }
+  const int z = planes ? splits : 1;
+  const int col_tiles = (N + 63) / 64;
+  const bool one = planes || splits == 1;
+  const dim3 block(256);
+  if ((M + 63) / 64 > 65535) return CW_ERR_SIZE;
+  // whole blocks of 16, and offsets that a 32-bit buffer descriptor reaches
+  if (!(K & 15) && !(lda & 3) && ((int64_t)M * lda + K) * 4 < (int64_t)UINT32_MAX && (int64_t)N * K * 4 < (int64_t)UINT32_MAX) {
+    const bool small = M <= 32 || (int64_t)((M + 63) / 64) * col_tiles * z < 256;
+    const int64_t tiles = (int64_t)col_tiles * (small ? (M + 31) / 32 : (M + 63) / 64) * z;
+    if (tiles > 0x7fffffff) return CW_ERR_SIZE;
+    const dim3 grid((unsigned)tiles);
+#define CW_RING_F32(BM_, ONE_)                                                                                     \
+  hipLaunchKernelGGL((gemm_f32_ring_kernel<BM_, ONE_>), grid, block, 4 * (BM_ + 64) * 128, stream, A, lda, W, bias, C, ldc, M, N, K, \
+                     splits, per, stride)
+    if (small) { if (one) CW_RING_F32(32, true); else CW_RING_F32(32, false); }
+    else { if (one) CW_RING_F32(64, true); else CW_RING_F32(64, false); }
+#undef CW_RING_F32
+    return cw_launch_status();
+  }
+  const dim3 grid(col_tiles, (M + 63) / 64, z);
+#define CW_TILE_F32(VEC_, ONE_)                                                                                     \
+  hipLaunchKernelGGL((gemm_f32_tile_kernel<VEC_, ONE_>), grid, block, 0, stream, A, lda, W, bias, C, ldc, M, N, K, \
+                     splits, per, stride)
+  if (vec) { if (one) CW_TILE_F32(true, true); else CW_TILE_F32(true, false); }
+  else { if (one) CW_TILE_F32(false, true); else CW_TILE_F32(false, false); }
+#undef CW_TILE_F32
+  return cw_launch_status();
 }
 
 CW_EXPORT int cw_gemm_f32(const float* A, int64_t lda, const float* W, const float* bias, float* C,
@@ -165,26 +515,29 @@ CW_EXPORT int cw_gemm_f32(const float* A, int64_t lda, const float* W, const flo
   if (((uintptr_t)A & 15) || ((uintptr_t)W & 15)) return CW_ERR_ARG;
   int splits, per;
   gemm_f32_plan(N, K, &splits, &per);
-  const dim3 block(256);
-  dim3 grid((N + GT_BN - 1) / GT_BN, (M + GT_BM - 1) / GT_BM);
-  if (grid.y > 65535) return CW_ERR_SIZE;
-  if (splits <= 1) {
-    hipLaunchKernelGGL(gemm_f32_kernel<true>, grid, block, 0, stream, A, lda, W, bias, C, ldc, M, N, K, 1, per, (int64_t)0);
-    return cw_launch_status();
-  }
-  if (M > GT_SPLIT_ROWS) {
-    hipLaunchKernelGGL(gemm_f32_kernel<false>, grid, block, 0, stream, A, lda, W, bias, C, ldc, M, N, K, splits, per,
-                       (int64_t)0);
-    return cw_launch_status();
-  }
+  if (!gemm_f32_planes(M, N, K, splits))
+    return launch_gemm_f32(A, lda, W, bias, C, ldc, M, N, K, splits, per, false, stream);
   const int64_t part_stride = (int64_t)M * N;
   if (workspace == nullptr || workspace_floats < splits * part_stride) return CW_ERR_ARG;
-  grid.z = splits;
-  hipLaunchKernelGGL(gemm_f32_kernel<true>, grid, block, 0, stream, A, lda, W, nullptr, workspace, (int64_t)N, M, N, K,
-                     splits, per, part_stride);
-  hipLaunchKernelGGL(gemm_f32_sum_kernel, dim3((unsigned)((part_stride + 255) / 256)), block, 0, stream, workspace,
+  const int rc = launch_gemm_f32(A, lda, W, nullptr, workspace, (int64_t)N, M, N, K, splits, per, true, stream);
+  if (rc != CW_OK) return rc;
+  hipLaunchKernelGGL(gemm_f32_sum_kernel, dim3((unsigned)((part_stride + 255) / 256)), dim3(256), 0, stream, workspace,
                      splits, part_stride, bias, C, ldc, M, N);
   return cw_launch_status();
+}
+
+// The parts of the product as they are, float32 [cw_gemm_f32_partial_planes(M, N, K), M, N]: added in order
+// they are what cw_gemm_f32 gives (without a bias), bit for bit. For a result that the residual-add + norm
+// kernel reads next, which adds them itself.
+CW_EXPORT int cw_gemm_f32_partial(const float* A, int64_t lda, const float* W, float* planes, int M, int N, int K,
+                                  hipStream_t stream) {
+  if (M < 0 || N <= 0 || K <= 0 || lda < K || !planes) return CW_ERR_ARG;
+  if (M == 0) return CW_OK;
+  if (((uintptr_t)A & 15) || ((uintptr_t)W & 15)) return CW_ERR_ARG;
+  int splits, per;
+  gemm_f32_plan(N, K, &splits, &per);
+  if (cw_gemm_f32_partial_planes(M, N, K) != splits) return CW_ERR_SIZE;
+  return launch_gemm_f32(A, lda, W, nullptr, planes, (int64_t)N, M, N, K, splits, per, true, stream);
 }
 
 // =====================================================================================
@@ -204,27 +557,6 @@ CW_EXPORT int cw_gemm_f32(const float* A, int64_t lda, const float* W, const flo
 // writing its float32 partial product [split, M, N]; whoever reads y next sums the partials in
 // order (the residual-add + norm kernel does): a narrow output with a long K (96 row tiles for
 // 27 MB of weights) then streams on all compute units instead of 96.
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-
-// How these kernels load operands. An MFMA operand wants lane l to hold row l % 16 of a tile and
-// the 8 k-values of slot l / 16: loaded that way every lane asks for 16 bytes of a row of its own,
-// 64 requests an instruction to a compute unit's load path, which takes in about 30 GB/s of such.
-// So a lane loads row l / 4, slot l % 4 instead (four neighbouring lanes cover 64 bytes of one row:
-// 16 requests an instruction), and the lanes swap what they hold afterwards, lane (r, s) taking
-// from lane 4 r + s (ds_bpermute: through the LDS unit's crossbar, no memory). Measured on the
-// 1.5B shape's gate/up product: 12.8 -> 11.7 us with 8 rows of x, 19.8 -> 17.5 us with 64.
-typedef __attribute__((ext_vector_type(4))) int cw_i32x4_t;
-__device__ __forceinline__ bf16x8_t cw_to_operand_layout(const bf16x8_t& v, int lane) {
-  const int r = lane & 15, s = lane >> 4;
-  const int from = (r * 4 + s) * 4;  // byte address of the lane that loaded what lane (r, s) multiplies
-  const cw_i32x4_t q = __builtin_bit_cast(cw_i32x4_t, v);
-  cw_i32x4_t t;
-#pragma unroll
-  for (int d = 0; d < 4; ++d) t[d] = __builtin_amdgcn_ds_bpermute(from, q[d]);
-  return __builtin_bit_cast(bf16x8_t, t);
-}
-
 __device__ __forceinline__ float cw_gelu_erf(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752440f)); }
 __device__ __forceinline__ float cw_relu_squared(float z) { const float r = fmaxf(z, 0.0f); return r * r; }
 

@@ -104,6 +104,8 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
         "gemm": {
             "cw_gemm_f32": [P, L, P, P, P, L, I, I, I, P, L, P],
             "cw_gemm_f32_workspace_floats": [I, I, I],
+            "cw_gemm_f32_partial_planes": [I, I, I],
+            "cw_gemm_f32_partial": [P, L, P, P, I, I, I, P],
             "cw_gemm_bf16_skinny": [I, P, L, P, P, L, I, I, I, I, F, P],
             "cw_gemm_bf16_skinny_ksplits": [I, I, I],
             "cw_gemm_bf16_skinny_fast": [I, I, I, I],
@@ -527,12 +529,18 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias=None, out_dtype=None, par
     if x.dtype == torch.float32:
         if not (weight.dtype == torch.float32):
             raise KernelError("a float32 product needs float32 weights")
+        lib = _load("gemm")
+        # a narrow output with a long K is summed in parts over K (the same parts whatever M is)
+        if partial_ok and bias is None:
+            planes = lib.cw_gemm_f32_partial_planes(M, N, K)
+            if planes:
+                parts = torch.empty((planes, M, N), dtype=torch.float32, device=x.device)
+                _check(lib.cw_gemm_f32_partial(_ptr(x), K, _ptr(weight), _ptr(parts), M, N, K, _stream()), "gemm_f32_partial")
+                return PartialSums(parts)
         out = torch.empty((M, N), dtype=torch.float32, device=x.device)
         if bias is not None:
             if not (bias.dtype == torch.float32 and bias.numel() == N):
                 raise KernelError("bias must be float32 [N]")
-        lib = _load("gemm")
-        # a narrow output with a long K is summed in parts over K (the same parts whatever M is)
         need = lib.cw_gemm_f32_workspace_floats(M, N, K)
         parts = torch.empty(need, dtype=torch.float32, device=x.device) if need else None
         _check(lib.cw_gemm_f32(_ptr(x), K, _ptr(weight), _ptr(bias), _ptr(out), N, M, N, K, _ptr(parts), need, _stream()),

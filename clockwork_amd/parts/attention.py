@@ -67,6 +67,10 @@ def portions_have_short_ranges(q_lens, ctx_lens) -> bool:
 # is cut into at most this many parts
 MIN_PART_KEYS = 256
 MAX_PARTS = 64
+# keys of a tile of the float32 kernel for single tokens: a workgroup takes about 8 us for one and they follow
+# one another, while the kernel that merges the parts takes 5 us however many there are (one request of 300 keys
+# of the 0.5B shape: 34 + 5 us with parts of 256 keys, 14 + 5 with parts of 64)
+TILE_KEYS = 64
 
 
 def _share_long_key_ranges(items: np.ndarray, ctx, workgroups_per_item: int):
@@ -163,7 +167,7 @@ def _make_plan(ctx, nh: int, nkv: int, narrow_ok: bool) -> AttentionPlan:
     if plan.n_single:
         groups_running = plan.n_single * nkv * plan.chunks_single
         by_occupancy = -(-4 * ctx.num_compute_units // groups_running)
-        by_length = max(1, longest_single // 256)
+        by_length = max(1, longest_single // TILE_KEYS)
         plan.single_splits = max(1, min(by_occupancy, by_length, 64))
         # decode kernel: a workgroup per (request, kv head, split); a split is at least 128 keys
         # (one 32-key tile for each of its four waves). As many splits as still give every
