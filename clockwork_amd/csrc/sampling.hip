@@ -165,38 +165,61 @@ __device__ __forceinline__ uint32_t philox_first_word(uint64_t seed, uint64_t co
 }
 
 // ---------------------------------------------------------------- sampling
-// A row is cut into chunks and every step of the selection is one small kernel over
-// (chunk, row), so a row's work is spread over many compute units and a step costs little more
-// than its launch; what a step needs of the step before it goes through the workspace: the
-// chunks add their histograms into the row's with integer atomics (a sum that no order changes),
-// and every workgroup of the next step reads that one histogram.
+// A row is cut into chunks, and a pass over the logits is a kernel over (chunk, row): a row's work is spread over
+// many compute units. What is then known about a whole row is worked out by a kernel of a workgroup a row. (The
+// last of a row's workgroups to finish could do that without a launch, but what the others wrote has to be made
+// visible to it: the fences that do so cost 170 us for 64 rows, the two launches 10.)
 //
-//   MAX      per chunk: the largest logit and its first index (greedy rows end here);
-//   TOPK 0-3 the k-th largest logit by radix selection, 8 bits of the order-preserving key a
-//            step: per chunk a histogram of the next byte among the keys that share the bytes
-//            found so far. Dividing by the temperature keeps the order, so the selection runs on
-//            the raw logits and the floor of what is kept is (k-th largest) / temperature:
-//            ties at the k-th value survive, also ties that the division makes;
-//   ZSUM     per chunk: the sum of the weights exp(logit / T - max) of what top-k left;
-//   TOPP 0-3 the same radix selection with weights instead of counts: the largest key K with
-//            weight(keys >= K) > top_p * total; everything from K up stays, i.e. a token stays
-//            while the tokens strictly more likely than it weigh <= top_p * total;
-//   SUMS     the chunk sums again with the final floor (rows with top-p only);
-//   LOCATE   u * total falls into a chunk, and in it on the first index whose running sum
-//            exceeds it.
+//   MAX      per chunk: the largest logit and its first index;
+//   HIST     per chunk, over 512 bins of the distance mx - logit / T from the largest (1 / 16 wide, the last one
+//            for everything beyond): how many tokens fall into each (rows with top-k) and what they weigh, the
+//            weights being exp(logit / T - mx) (rows with top-p); and what the chunk weighs. Greedy rows end here;
+//   PICK     per row: the bin that holds the k-th largest token, or the bin in which the weight from the top exceeds
+//            top_p * total;
+//   COLLECT  per chunk: what the tokens above that bin weigh (all of them stay), and a list of the tokens in it;
+//   DRAW     per row: the k-th largest token of the list (radix selection over the order-preserving keys, 8 bits a
+//            step; dividing by the temperature keeps the order, so the floor of what is kept is
+//            (k-th largest) / temperature: ties at the k-th value survive, also ties that the division makes) and
+//            the nucleus's last token (the largest key K with weight(keys >= K) > top_p * total: a token stays
+//            while the tokens strictly more likely than it weigh <= top_p * total), then the draw. Rows without
+//            either option come here from HIST. For a row with both options whose nucleus ends in a bin above the
+//            k-th token's, COLLECT and DRAW run once more.
+//
+// A token's bin does not fall as its logit grows, and equal logits / T share a bin: what lies in bins above is kept,
+// what lies in bins below is not. A list that does not fit (a row of many equal logits) is not used: DRAW walks
+// the row instead.
+// The draw: u * total falls into a chunk, and in it on the first index whose running sum exceeds it.
 // Weights are integers, exp(.) * 2^40 rounded down: their sums do not depend on the order of
 // addition, so every comparison above gives the same answer however the row is cut and however
 // the additions are scheduled (LDS atomics included), run after run.
+// Bound by the passes over the logits, which come from the memory-side cache after the first. 64 rows of 151,936
+// logits, a quarter each greedy, temperature, top-k and top-p: 119 us as twelve kernels (a radix step of 8 bits of the
+// key each, over the whole rows), 61 us as five.
 #define SAMPLE_THREADS 256
+#define SAMPLE_WAVES (SAMPLE_THREADS / 64)
 #define SAMPLE_MAX_CHUNKS 64
+#define SAMPLE_BINS 512
+#define SAMPLE_BINS_PER_UNIT 16.0f
+#define SAMPLE_LIST 4096         // tokens of a row's list
+#define SAMPLE_BLOCK_LIST 1024   // tokens that one workgroup may add to it
 #define SAMPLE_WEIGHT_SCALE 1099511627776.0f  // 2^40
 
 typedef unsigned long long u64_t;
 
+struct SampleRow {     // what is known about a row between two kernels
+  u64_t limit;         // top_p * total (rows with top-p)
+  uint32_t bin;        // the bin to collect
+  uint32_t rank;       // rows with top-k: which of the bin's tokens, from the largest, is the k-th
+  uint32_t collect;    // 1: COLLECT has to run, 2: its second run has to
+  uint32_t listed[2];  // tokens that COLLECT's two runs found in the bin
+  uint32_t unused;     // (a whole number of 8 bytes)
+};
+
 struct SampleArgs {
   const float* logits;
   int64_t row_stride;
-  int n, V, chunks, per;
+  int n, V, chunks, per;  // per: a multiple of 4
+  int vec;                // rows begin at 16-byte boundaries
   const float* temperature;
   const int* top_k;
   const float* top_p;
@@ -204,25 +227,27 @@ struct SampleArgs {
   const int64_t* draws;
   int* out;
   // workspace
-  float* pmax;       // [n][chunks]
-  int* pmax_i;       // [n][chunks]
-  uint32_t* hist_k;  // [4 steps][n][256], zeroed by the MAX step
-  u64_t* hist_p;     // [4 steps][n][256], zeroed by the MAX step
-  uint32_t* state_k; // [2][n][2]: key bits found so far, rank still to go
-  u64_t* state_p;    // [2][n][2]: key bits found so far, weight above them
-  uint32_t* floor_k; // [n] scaled-key floor after top-k
-  u64_t* psum;       // [n][chunks] chunk sums of weights
+  u64_t* hist_w;      // [n][chunks][SAMPLE_BINS]
+  u64_t* sums;        // [n][chunks] weight of the chunk (of its bins above the collected one, after COLLECT)
+  SampleRow* rows;    // [n], zeroed by MAX
+  uint32_t* hist_n;   // [n][chunks][SAMPLE_BINS]
+  uint2* list;        // [n][SAMPLE_LIST] (key, index)
+  float* pmax;        // [n][chunks]
+  int* pmax_i;        // [n][chunks]
 };
 
-CW_EXPORT int cw_sample_chunks(int V) {
+// Chunks a row is cut into: at least 2048 tokens each; 64 for few rows, for many rows as few as still make two
+// thousand workgroups (what PICK adds up grows with them).
+static int sample_chunks(int n, int V) {
   int c = (V + 2047) / 2048;
-  return c < 1 ? 1 : (c > SAMPLE_MAX_CHUNKS ? SAMPLE_MAX_CHUNKS : c);
+  const int most = n <= 32 ? SAMPLE_MAX_CHUNKS : n >= 512 ? 4 : 2048 / n;
+  if (c > most) c = most;
+  return c < 1 ? 1 : c;
 }
 
 CW_EXPORT int64_t cw_sample_workspace_bytes(int n, int V) {
-  const int64_t rc = (int64_t)n * cw_sample_chunks(V);
-  // hist_p, state_p, psum, the second psum with a floor per row; hist_k, state_k, floor_k, pmax, pmax_i
-  return 8 * (4 * (int64_t)n * 256 + 4 * (int64_t)n + rc + rc + n) + 4 * (4 * (int64_t)n * 256 + 4 * (int64_t)n + n + 2 * rc) + 64;
+  const int64_t rc = (int64_t)n * sample_chunks(n, V);
+  return rc * SAMPLE_BINS * 12 + rc * 16 + (int64_t)n * ((int64_t)sizeof(SampleRow) + SAMPLE_LIST * 8) + 64;
 }
 
 __device__ __forceinline__ float key_to_float(uint32_t k) {
@@ -236,6 +261,71 @@ __device__ __forceinline__ bool row_has_top_p(const SampleArgs& a, int row) { re
 __device__ __forceinline__ u64_t weight_of(float v, float mx) {
   const float e = expf(v - mx);  // NaN for inf - inf: no weight
   return e == e ? (u64_t)(e * SAMPLE_WEIGHT_SCALE) : 0;
+}
+// The bin of v = logit / T (NaN goes last, with -inf).
+__device__ __forceinline__ uint32_t bin_of(float v, float mx) {
+  if (v != v) return SAMPLE_BINS - 1;
+  if (!(v < mx)) return 0;
+  const float d = (mx - v) * SAMPLE_BINS_PER_UNIT;
+  return d < (float)(SAMPLE_BINS - 1) ? (uint32_t)d : SAMPLE_BINS - 1;
+}
+__device__ __forceinline__ u64_t topp_limit(float p, u64_t total) { return (u64_t)((double)p * (double)total); }
+
+// Four neighbouring logits from token i on (i a multiple of 4); NaN from ``hi`` on.
+__device__ __forceinline__ void sample_load4(const float* x, int i, int hi, int vec, float (&o)[4]) {
+  if (vec && i + 4 <= hi) {
+    const float4 v = *reinterpret_cast<const float4*>(x + i);
+    o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = i + e < hi ? x[i + e] : NAN;
+  }
+}
+// f(index, logit) for the tokens of [lo, hi), by all threads of the workgroup, eight loads in flight a thread.
+template <typename F>
+__device__ __forceinline__ void sample_walk(const float* x, int lo, int hi, int vec, F f) {
+  for (int i0 = lo + (int)threadIdx.x * 4; i0 < hi; i0 += 8 * SAMPLE_THREADS) {
+    float a[4], b[4];
+    const int i1 = i0 + 4 * SAMPLE_THREADS;
+    sample_load4(x, i0, hi, vec, a);
+    sample_load4(x, min(i1, (int)((unsigned)(hi - 1) & ~3u)), hi, vec, b);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (i0 + e < hi) f(i0 + e, a[e]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (i1 + e < hi) f(i1 + e, b[e]);
+  }
+}
+
+// Sum over the workgroup; every thread gets it.
+__device__ __forceinline__ u64_t block_sum(u64_t v) {
+  __shared__ u64_t part[SAMPLE_WAVES];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+  __syncthreads();
+  u64_t t = 0;
+#pragma unroll
+  for (int w = 0; w < SAMPLE_WAVES; ++w) t += part[w];
+  __syncthreads();
+  return t;
+}
+// Sum of the values of this thread and of those before it.
+template <typename T>
+__device__ __forceinline__ T block_running_sum(T v) {
+  __shared__ T part[SAMPLE_WAVES];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const T up = __shfl_up(v, off, 64);
+    if (lane >= off) v += up;
+  }
+  if (lane == 63) part[wave] = v;
+  __syncthreads();
+  for (int w = 0; w < wave; ++w) v += part[w];
+  __syncthreads();
+  return v;
 }
 
 // The row's largest logit (NaN counts as -inf) and its first index, from the chunk maxima: the
@@ -264,47 +354,19 @@ __device__ __forceinline__ void row_max(const SampleArgs& a, int row, float& bv,
   __syncthreads();
 }
 
-// For every thread b < 256: suf = sum of the bins b..255 of a row's histogram (a scan through
-// LDS) and next = the bins above b.
-template <typename T>
-__device__ __forceinline__ T suffix_of_bins(const T* hist_row, T* sh, T& next) {
-  const int b = threadIdx.x;
-  const T t = hist_row[b];
-  __syncthreads();
-  sh[b] = t;
-  __syncthreads();
-  for (int off = 1; off < 256; off <<= 1) {
-    const T add = b + off < 256 ? sh[b + off] : (T)0;
-    __syncthreads();
-    sh[b] += add;
-    __syncthreads();
-  }
-  const T suf = sh[b];
-  next = suf - t;
-  return suf;
-}
-
 // MAX
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_max_kernel(SampleArgs a) {
-  __shared__ float sv[SAMPLE_THREADS / 64];
-  __shared__ int si[SAMPLE_THREADS / 64];
+  __shared__ float sv[SAMPLE_WAVES];
+  __shared__ int si[SAMPLE_WAVES];
   const int row = blockIdx.y, chunk = blockIdx.x;
-  if (chunk == 0) {  // the row's histograms start at zero
-#pragma unroll
-    for (int step = 0; step < 4; ++step) {
-      a.hist_k[((int64_t)step * a.n + row) * 256 + threadIdx.x] = 0u;
-      a.hist_p[((int64_t)step * a.n + row) * 256 + threadIdx.x] = 0;
-    }
-  }
+  if (chunk == 0 && threadIdx.x < sizeof(SampleRow) / 4) reinterpret_cast<uint32_t*>(a.rows + row)[threadIdx.x] = 0u;
   const int lo = chunk * a.per, hi = min(a.V, lo + a.per);
-  const float* x = a.logits + (int64_t)row * a.row_stride;
   float bv = -INFINITY;
   int bi = 0x7fffffff;
-  for (int i = lo + threadIdx.x; i < hi; i += SAMPLE_THREADS) {
-    float v = x[i];
+  sample_walk(a.logits + (int64_t)row * a.row_stride, lo, hi, a.vec, [&](int i, float v) __attribute__((always_inline)) {
     if (v != v) v = -INFINITY;
     argmax_merge(bv, bi, v, i);
-  }
+  });
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     const float ov = __shfl_xor(bv, off, 64);
@@ -314,351 +376,384 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_max_kernel(SampleArgs a
   if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = bv; si[threadIdx.x >> 6] = bi; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int w = 1; w < SAMPLE_THREADS / 64; ++w) argmax_merge(bv, bi, sv[w], si[w]);
+    for (int w = 1; w < SAMPLE_WAVES; ++w) argmax_merge(bv, bi, sv[w], si[w]);
     a.pmax[row * a.chunks + chunk] = bv;
     a.pmax_i[row * a.chunks + chunk] = bi;
   }
 }
 
-// State of the top-k descent after `done` steps, from the state after done - 1 steps (in the
-// workspace, written by the step before) and that step's histograms: (key bits, rank to go).
-__device__ __forceinline__ void topk_state(const SampleArgs& a, int row, int done, uint32_t* sh, uint32_t& prefix,
-                                           uint32_t& rank) {
-  __shared__ uint32_t picked[2];
-  if (done == 0) {
-    prefix = 0u;
-    rank = (uint32_t)a.top_k[row];
-    return;
-  }
-  uint32_t p0 = 0u, r0 = (uint32_t)a.top_k[row];
-  if (done > 1) {
-    const uint32_t* st = a.state_k + ((int64_t)((done - 2) & 1) * a.n + row) * 2;
-    p0 = st[0];
-    r0 = st[1];
-  }
-  const uint32_t* hist = a.hist_k + ((int64_t)(done - 1) * a.n + row) * 256;
-  if (threadIdx.x == 0) {  // what stands if no bin qualifies (it always does for counts that add up)
-    picked[0] = 0u;
-    picked[1] = r0;
-  }
-  uint32_t above;
-  const uint32_t suf = suffix_of_bins<uint32_t>(hist, sh, above);
-  // the bin that holds the rank-th largest: at least `rank` keys from it up, fewer above it
-  if (suf >= r0 && above < r0) {
-    picked[0] = threadIdx.x;
-    picked[1] = r0 - above;
-  }
+// Draws the row's token among those whose scaled key is floor_key or more; ``chunk_w`` (LDS): what each chunk's
+// such tokens weigh. All threads of one workgroup.
+__device__ __forceinline__ void sample_locate(const SampleArgs& a, int row, float temp, float mx, int mi, uint32_t floor_key,
+                                              const u64_t* chunk_w) {
+  __shared__ int sel_chunk, sel_run, found;
+  __shared__ u64_t sel_base, sel_total;
+  if (threadIdx.x == 0) sel_chunk = sel_run = 0, found = -1, sel_base = 0;
   __syncthreads();
-  prefix = p0 | (picked[0] << (24 - 8 * (done - 1)));
-  rank = picked[1];
-  __syncthreads();
-}
-
-// TOPK step `step` (0..3): histogram of byte `step` of the raw keys that share the bytes found.
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_topk_kernel(SampleArgs a, int step) {
-  __shared__ uint32_t sh[256];
-  __shared__ uint32_t bins[SAMPLE_THREADS / 64][256];
-  const int row = blockIdx.y, chunk = blockIdx.x;
-  if (!(a.temperature[row] > 0.0f) || !row_has_top_k(a, row)) return;
-  uint32_t prefix, rank;
-  topk_state(a, row, step, sh, prefix, rank);
-  if (chunk == 0 && threadIdx.x == 0 && step > 0) {
-    uint32_t* st = a.state_k + ((int64_t)((step - 1) & 1) * a.n + row) * 2;
-    st[0] = prefix;
-    st[1] = rank;
-  }
-  for (int i = threadIdx.x; i < (SAMPLE_THREADS / 64) * 256; i += SAMPLE_THREADS) (&bins[0][0])[i] = 0u;
-  __syncthreads();
-  const int lo = chunk * a.per, hi = min(a.V, lo + a.per);
-  const float* x = a.logits + (int64_t)row * a.row_stride;
-  const int shift = 24 - 8 * step;
-  const uint32_t mask = step == 0 ? 0u : (0xffffffffu << (shift + 8));
-  uint32_t* mine = bins[threadIdx.x >> 6];
-  for (int i0 = lo + threadIdx.x; i0 < hi; i0 += 4 * SAMPLE_THREADS) {  // four loads in flight
-    float raw[4];
-    bool in[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      in[u] = i0 + u * SAMPLE_THREADS < hi;
-      raw[u] = in[u] ? x[i0 + u * SAMPLE_THREADS] : 0.0f;
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const uint32_t key = order_key(raw[u]);
-      if (in[u] && (key & mask) == prefix) atomicAdd(&mine[(key >> shift) & 255u], 1u);
-    }
-  }
-  __syncthreads();
-  uint32_t t = 0u;
-#pragma unroll
-  for (int w = 0; w < SAMPLE_THREADS / 64; ++w) t += bins[w][threadIdx.x];
-  if (t) atomicAdd(&a.hist_k[((int64_t)step * a.n + row) * 256 + threadIdx.x], t);
-}
-
-// The floor top-k leaves, as a key of the scaled logits (0: nothing is cut). Every thread of the
-// workgroup gets it; after ZSUM it is in the workspace.
-__device__ __forceinline__ uint32_t topk_floor(const SampleArgs& a, int row, float temp, uint32_t* sh) {
-  if (!row_has_top_k(a, row)) return 0u;
-  uint32_t key, rank;
-  topk_state(a, row, 4, sh, key, rank);
-  return order_key(key_to_float(key) / temp);
-}
-
-// Sum of the weights of the chunk's kept tokens, every thread gets it.
-__device__ __forceinline__ u64_t chunk_weight(const SampleArgs& a, int row, int chunk, float temp, float mx,
-                                              uint32_t floor_key, u64_t* red) {
-  const int lo = chunk * a.per, hi = min(a.V, lo + a.per);
-  const float* x = a.logits + (int64_t)row * a.row_stride;
-  u64_t w = 0;
-  for (int i0 = lo + threadIdx.x; i0 < hi; i0 += 4 * SAMPLE_THREADS) {  // four loads in flight
-    float raw[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) raw[u] = i0 + u * SAMPLE_THREADS < hi ? x[i0 + u * SAMPLE_THREADS] : NAN;
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const float v = raw[u] / temp;
-      if (v == v && order_key(v) >= floor_key) w += weight_of(v, mx);
-    }
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) w += __shfl_xor(w, off, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = w;
-  __syncthreads();
-  u64_t t = 0;
-#pragma unroll
-  for (int i = 0; i < SAMPLE_THREADS / 64; ++i) t += red[i];
-  return t;
-}
-
-// ZSUM
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_zsum_kernel(SampleArgs a) {
-  __shared__ uint32_t sh[256];
-  __shared__ u64_t red[SAMPLE_THREADS / 64];
-  const int row = blockIdx.y, chunk = blockIdx.x;
-  const float temp = a.temperature[row];
-  if (!(temp > 0.0f)) return;
-  const uint32_t floor_key = topk_floor(a, row, temp, sh);
-  if (chunk == 0 && threadIdx.x == 0) a.floor_k[row] = floor_key;
-  float mraw;
-  int mi;
-  row_max(a, row, mraw, mi);
-  const u64_t w = chunk_weight(a, row, chunk, temp, mraw / temp, floor_key, red);
-  if (threadIdx.x == 0) a.psum[row * a.chunks + chunk] = w;
-}
-
-// State of the top-p descent after `done` steps: (key bits, weight of the keys above them).
-__device__ __forceinline__ void topp_state(const SampleArgs& a, int row, int done, u64_t limit, u64_t* sh,
-                                           uint32_t& prefix, u64_t& above_all) {
-  __shared__ u64_t picked[2];
-  if (done == 0) {
-    prefix = 0u;
-    above_all = 0;
-    return;
-  }
-  uint32_t p0 = 0u;
-  u64_t a0 = 0;
-  if (done > 1) {
-    const u64_t* st = a.state_p + ((int64_t)((done - 2) & 1) * a.n + row) * 2;
-    p0 = (uint32_t)st[0];
-    a0 = st[1];
-  }
-  const u64_t* hist = a.hist_p + ((int64_t)(done - 1) * a.n + row) * 256;
-  if (threadIdx.x == 0) {  // what stands if no bin qualifies (a row without any weight)
-    picked[0] = 0;
-    picked[1] = a0;
-  }
-  u64_t above;
-  const u64_t suf = suffix_of_bins<u64_t>(hist, sh, above);
-  // the largest byte b with weight(keys >= (bytes so far, b, 0...)) > limit
-  if (a0 + suf > limit && !(a0 + above > limit)) {
-    picked[0] = threadIdx.x;
-    picked[1] = a0 + above;
-  }
-  __syncthreads();
-  prefix = p0 | ((uint32_t)picked[0] << (24 - 8 * (done - 1)));
-  above_all = picked[1];
-  __syncthreads();
-}
-
-// Sum of a row's chunk sums (order does not matter: integers); every thread gets it.
-__device__ __forceinline__ u64_t row_total(const u64_t* sums, int chunks) {
-  __shared__ u64_t total;
-  if (threadIdx.x < 64) {
-    u64_t t = (int)threadIdx.x < chunks ? sums[threadIdx.x] : 0;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
-    if (threadIdx.x == 0) total = t;
-  }
-  __syncthreads();
-  const u64_t t = total;
-  __syncthreads();
-  return t;
-}
-__device__ __forceinline__ u64_t topp_limit(float p, u64_t total) { return (u64_t)((double)p * (double)total); }
-
-// TOPP step `step` (0..3): weight per value of byte `step` among the kept raw keys that share
-// the bytes found so far.
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_topp_kernel(SampleArgs a, int step) {
-  __shared__ u64_t sh[256];
-  __shared__ u64_t bins[SAMPLE_THREADS / 64][256];
-  const int row = blockIdx.y, chunk = blockIdx.x;
-  const float temp = a.temperature[row];
-  if (!(temp > 0.0f) || !row_has_top_p(a, row)) return;
-  const u64_t limit = topp_limit(a.top_p[row], row_total(a.psum + row * a.chunks, a.chunks));
-  uint32_t prefix;
-  u64_t above;
-  topp_state(a, row, step, limit, sh, prefix, above);
-  if (chunk == 0 && threadIdx.x == 0 && step > 0) {
-    u64_t* st = a.state_p + ((int64_t)((step - 1) & 1) * a.n + row) * 2;
-    st[0] = prefix;
-    st[1] = above;
-  }
-  for (int i = threadIdx.x; i < (SAMPLE_THREADS / 64) * 256; i += SAMPLE_THREADS) (&bins[0][0])[i] = 0;
-  __syncthreads();
-  float mraw;
-  int mi;
-  row_max(a, row, mraw, mi);
-  const float mx = mraw / temp;
-  const uint32_t floor_key = a.floor_k[row];
-  const int lo = chunk * a.per, hi = min(a.V, lo + a.per);
-  const float* x = a.logits + (int64_t)row * a.row_stride;
-  const int shift = 24 - 8 * step;
-  const uint32_t mask = step == 0 ? 0u : (0xffffffffu << (shift + 8));
-  u64_t* mine = bins[threadIdx.x >> 6];
-  for (int i0 = lo + threadIdx.x; i0 < hi; i0 += 4 * SAMPLE_THREADS) {  // four loads in flight
-    float raws[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) raws[u] = i0 + u * SAMPLE_THREADS < hi ? x[i0 + u * SAMPLE_THREADS] : NAN;
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const float raw = raws[u];
-      const uint32_t key = order_key(raw);
-      if (raw != raw || (key & mask) != prefix) continue;
-      const float v = raw / temp;
-      if (v == v && order_key(v) >= floor_key) atomicAdd(&mine[(key >> shift) & 255u], weight_of(v, mx));
-    }
-  }
-  __syncthreads();
-  u64_t t = 0;
-#pragma unroll
-  for (int w = 0; w < SAMPLE_THREADS / 64; ++w) t += bins[w][threadIdx.x];
-  if (t) atomicAdd(&a.hist_p[((int64_t)step * a.n + row) * 256 + threadIdx.x], t);
-}
-
-// SUMS: the chunk sums with the floor that top-p adds (rows with top-p).
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_sums_kernel(SampleArgs a, u64_t* psum_out) {
-  __shared__ u64_t sh[256];
-  __shared__ u64_t red[SAMPLE_THREADS / 64];
-  const int row = blockIdx.y, chunk = blockIdx.x;
-  const float temp = a.temperature[row];
-  if (!(temp > 0.0f) || !row_has_top_p(a, row)) return;
-  const u64_t limit = topp_limit(a.top_p[row], row_total(a.psum + row * a.chunks, a.chunks));
-  uint32_t key;
-  u64_t above;
-  topp_state(a, row, 4, limit, sh, key, above);
-  uint32_t floor_key = order_key(key_to_float(key) / temp);
-  if (floor_key < a.floor_k[row]) floor_key = a.floor_k[row];
-  float mraw;
-  int mi;
-  row_max(a, row, mraw, mi);
-  const u64_t w = chunk_weight(a, row, chunk, temp, mraw / temp, floor_key, red);
-  if (threadIdx.x == 0) {
-    psum_out[row * a.chunks + chunk] = w;
-    if (chunk == 0) psum_out[(int64_t)a.n * a.chunks + row] = floor_key;  // for LOCATE
-  }
-}
-
-// LOCATE: one workgroup per row.
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_locate_kernel(SampleArgs a, const u64_t* psum2) {
-  __shared__ u64_t scan[SAMPLE_THREADS];
-  __shared__ int found;
-  const int row = blockIdx.x;
-  const float temp = a.temperature[row];
-  float mraw;
-  int mi;
-  row_max(a, row, mraw, mi);
-  if (!(temp > 0.0f)) {  // greedy row inside a sampled batch
-    if (threadIdx.x == 0) a.out[row] = mi < a.V ? mi : 0;
-    return;
-  }
-  const bool with_p = row_has_top_p(a, row);
-  const u64_t* sums = (with_p ? psum2 : a.psum) + row * a.chunks;
-  const uint32_t floor_key = with_p ? (uint32_t)psum2[(int64_t)a.n * a.chunks + row] : a.floor_k[row];
-  const u64_t total = row_total(sums, a.chunks);
-  if (total == 0) {  // no token has any weight (every logit -inf or NaN): the first maximum, as greedy
-    if (threadIdx.x == 0) a.out[row] = mi < a.V ? mi : 0;
-    return;
-  }
   const uint32_t r = philox_first_word((uint64_t)a.seeds[row], (uint64_t)a.draws[row]);
-  // u = (r >> 8) / 2^24; the drawn token is the first whose running weight exceeds u * total
-  u64_t target = (u64_t)((double)(r >> 8) * (1.0 / 16777216.0) * (double)total);
-  if (target >= total) target = total - 1;  // (total >= 2^40: the largest logit weighs that much)
-  // the chunk the target falls into: a running sum over the chunks in the first wave
-  __shared__ int sel_chunk;
-  __shared__ u64_t sel_base;
-  if (threadIdx.x == 0) {
-    sel_chunk = 0;
-    sel_base = 0;
-  }
-  __syncthreads();
-  if (threadIdx.x < 64) {
-    const u64_t v = (int)threadIdx.x < a.chunks ? sums[threadIdx.x] : 0;
+  if (threadIdx.x < 64) {  // the chunk the target falls into: a running sum over the chunks
+    const u64_t v = (int)threadIdx.x < a.chunks ? chunk_w[threadIdx.x] : 0;
     u64_t incl = v;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
       const u64_t up = __shfl_up(incl, off, 64);
       if ((int)threadIdx.x >= off) incl += up;
     }
+    const u64_t total = __shfl(incl, 63, 64);
+    // u = (r >> 8) / 2^24; the drawn token is the first whose running weight exceeds u * total
+    u64_t target = (u64_t)((double)(r >> 8) * (1.0 / 16777216.0) * (double)total);
+    if (total > 0 && target >= total) target = total - 1;  // (total >= 2^40: the largest logit weighs that much)
     if (v > 0 && incl - v <= target && target < incl) {
       sel_chunk = threadIdx.x;
-      sel_base = incl - v;
+      sel_base = target - (incl - v);  // the target inside the chunk
     }
+    if (threadIdx.x == 0) sel_total = total;
   }
   __syncthreads();
-  const int chunk = sel_chunk;
-  const u64_t base = sel_base;
-  // in the chunk: thread t owns a run of consecutive tokens
-  const float mx = mraw / temp;
-  const int lo = chunk * a.per, hi = min(a.V, lo + a.per);
+  if (sel_total == 0) {  // no token has any weight (every logit -inf or NaN): the first maximum, as greedy
+    if (threadIdx.x == 0) a.out[row] = mi < a.V ? mi : 0;
+    return;
+  }
+  const float* x = a.logits + (int64_t)row * a.row_stride;
+  auto weight = [&](int i) __attribute__((always_inline)) -> u64_t {
+    const float v = x[i] / temp;
+    return v == v && order_key(v) >= floor_key ? weight_of(v, mx) : 0;
+  };
+  // in the chunk: thread t weighs a run of consecutive tokens; then a lane of the first wave takes a token of
+  // the run that the target falls into
+  const int lo = sel_chunk * a.per, hi = min(a.V, lo + a.per);
+  const u64_t target = sel_base;
   const int run = (hi - lo + SAMPLE_THREADS - 1) / SAMPLE_THREADS;
   const int my_lo = min(hi, lo + (int)threadIdx.x * run), my_hi = min(hi, my_lo + run);
-  const float* x = a.logits + (int64_t)row * a.row_stride;
   u64_t w = 0;
-  for (int i = my_lo; i < my_hi; ++i) {
-    const float v = x[i] / temp;
-    if (v == v && order_key(v) >= floor_key) w += weight_of(v, mx);
+#pragma unroll 8
+  for (int i = my_lo; i < my_hi; ++i) w += weight(i);
+  const u64_t incl = block_running_sum(w);
+  if (w > 0 && incl - w <= target && target < incl) {
+    sel_run = threadIdx.x;
+    sel_base = incl - w;
   }
-  scan[threadIdx.x] = w;
-  if (threadIdx.x == 0) found = -1;
   __syncthreads();
-  for (int off = 1; off < SAMPLE_THREADS; off <<= 1) {  // inclusive scan
-    const u64_t add = threadIdx.x >= off ? scan[threadIdx.x - off] : 0;
-    __syncthreads();
-    scan[threadIdx.x] += add;
-    __syncthreads();
-  }
-  const u64_t incl = base + scan[threadIdx.x], excl = incl - w;
-  if (w > 0 && excl <= target && target < incl) {
-    u64_t at = excl;
-    int chosen = my_lo;
-    for (int i = my_lo; i < my_hi; ++i) {
-      const float v = x[i] / temp;
-      if (!(v == v && order_key(v) >= floor_key)) continue;
-      const u64_t q = weight_of(v, mx);
-      if (q == 0) continue;
-      chosen = i;
-      at += q;
-      if (at > target) break;
+  if (threadIdx.x < 64) {
+    u64_t before = sel_base;
+    const int run_lo = min(hi, lo + sel_run * run), run_hi = min(hi, run_lo + run);
+    for (int i0 = run_lo; i0 < run_hi; i0 += 64) {
+      const int i = i0 + (int)threadIdx.x;
+      const u64_t q = i < run_hi ? weight(i) : 0;
+      u64_t upto = q;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const u64_t up = __shfl_up(upto, off, 64);
+        if ((int)threadIdx.x >= off) upto += up;
+      }
+      upto += before;
+      if (q > 0 && upto - q <= target && target < upto) found = i;
+      before = __shfl(upto, 63, 64);
     }
-    found = chosen;
   }
   __syncthreads();
   if (threadIdx.x == 0) a.out[row] = found >= 0 ? found : (mi < a.V ? mi : 0);
 }
 
-// flags: bit 0 some row may have top-k, bit 1 some row may have top-p (3 when unknown): the
-// steps no row needs are not launched. workspace: cw_sample_workspace_bytes(n, V) bytes, 16-byte
+// HIST
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_hist_kernel(SampleArgs a) {
+  __shared__ u64_t bins_w[SAMPLE_BINS];
+  __shared__ uint32_t bins_n[SAMPLE_BINS];
+  const int row = blockIdx.y, chunk = blockIdx.x;
+  const float temp = a.temperature[row];
+  float mraw;
+  int mi;
+  row_max(a, row, mraw, mi);
+  if (!(temp > 0.0f)) {  // greedy row inside a sampled batch
+    if (chunk == 0 && threadIdx.x == 0) a.out[row] = mi < a.V ? mi : 0;
+    return;
+  }
+  const bool with_k = row_has_top_k(a, row), with_p = row_has_top_p(a, row);
+  const float mx = mraw / temp;
+  for (int b = threadIdx.x; b < SAMPLE_BINS; b += SAMPLE_THREADS) {
+    bins_w[b] = 0;
+    bins_n[b] = 0u;
+  }
+  __syncthreads();
+  const int lo = chunk * a.per, hi = min(a.V, lo + a.per);
+  u64_t sum = 0;
+  sample_walk(a.logits + (int64_t)row * a.row_stride, lo, hi, a.vec, [&](int, float raw) __attribute__((always_inline)) {
+    const float v = raw / temp;
+    if (with_k) atomicAdd(&bins_n[bin_of(v, mx)], 1u);
+    if (with_k && !with_p) return;  // (COLLECT weighs what top-k leaves)
+    const u64_t w = v == v ? weight_of(v, mx) : 0;
+    sum += w;
+    if (with_p && w) atomicAdd(&bins_w[bin_of(v, mx)], w);
+  });
+  sum = block_sum(sum);  // (and a barrier behind the bins)
+  const int64_t rc = (int64_t)row * a.chunks + chunk;
+  if (threadIdx.x == 0) a.sums[rc] = sum;
+  for (int b = threadIdx.x; b < SAMPLE_BINS; b += SAMPLE_THREADS) {
+    if (with_k) a.hist_n[rc * SAMPLE_BINS + b] = bins_n[b];
+    if (with_p) a.hist_w[rc * SAMPLE_BINS + b] = bins_w[b];
+  }
+}
+
+// The weights of bins 2 t and 2 t + 1 of the whole row, for thread t.
+__device__ __forceinline__ void row_bins(const SampleArgs& a, int row, u64_t& w0, u64_t& w1) {
+#pragma unroll 8
+  for (int c = 0; c < a.chunks; ++c) {
+    const ulonglong2 h = *reinterpret_cast<const ulonglong2*>(a.hist_w + ((int64_t)row * a.chunks + c) * SAMPLE_BINS + 2 * threadIdx.x);
+    w0 += h.x;
+    w1 += h.y;
+  }
+}
+
+// PICK
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(SampleArgs a) {
+  __shared__ uint32_t picked_bin, picked_rank;
+  const int row = blockIdx.x;
+  if (!(a.temperature[row] > 0.0f)) return;
+  const bool with_k = row_has_top_k(a, row), with_p = row_has_top_p(a, row);
+  if (!with_k && !with_p) return;
+  SampleRow& known = a.rows[row];
+  // thread t: bins 2 t and 2 t + 1 of the whole row
+  if (threadIdx.x == 0) picked_bin = 0u, picked_rank = 1u;
+  __syncthreads();
+  if (with_k) {
+    uint32_t n0 = 0u, n1 = 0u;
+#pragma unroll 8
+    for (int c = 0; c < a.chunks; ++c) {
+      const uint2 h = *reinterpret_cast<const uint2*>(a.hist_n + ((int64_t)row * a.chunks + c) * SAMPLE_BINS + 2 * threadIdx.x);
+      n0 += h.x;
+      n1 += h.y;
+    }
+    const uint32_t upto = block_running_sum(n0 + n1), k = (uint32_t)a.top_k[row];
+    const uint32_t before = upto - n0 - n1;
+    if (before < k && k <= upto) {
+      picked_bin = 2 * threadIdx.x + (before + n0 < k ? 1 : 0);
+      picked_rank = k - (before + n0 < k ? before + n0 : before);
+    }
+  } else {
+    const u64_t total = block_sum((int)threadIdx.x < a.chunks ? a.sums[(int64_t)row * a.chunks + threadIdx.x] : 0);
+    const u64_t limit = topp_limit(a.top_p[row], total);
+    u64_t w0 = 0, w1 = 0;
+    row_bins(a, row, w0, w1);
+    const u64_t upto = block_running_sum(w0 + w1);
+    const u64_t before = upto - w0 - w1;
+    if (before <= limit && limit < upto) picked_bin = 2 * threadIdx.x + (before + w0 <= limit ? 1 : 0);
+    if (threadIdx.x == 0) known.limit = limit;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    known.bin = picked_bin;
+    known.rank = picked_rank;
+    known.collect = 1u;
+  }
+}
+
+// COLLECT; ``again``: its second run
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(SampleArgs a, int again) {
+  __shared__ uint2 mine[SAMPLE_BLOCK_LIST];
+  __shared__ uint32_t n_mine, at_list;
+  const int row = blockIdx.y, chunk = blockIdx.x;
+  SampleRow& known = a.rows[row];
+  const float temp = a.temperature[row];
+  if (!(temp > 0.0f) || known.collect != 1u + again) return;
+  float mraw;
+  int mi;
+  row_max(a, row, mraw, mi);
+  const float mx = mraw / temp;
+  const uint32_t bin = known.bin;
+  const float* x = a.logits + (int64_t)row * a.row_stride;
+  if (threadIdx.x == 0) n_mine = 0u;
+  __syncthreads();
+  const int lo = chunk * a.per, hi = min(a.V, lo + a.per);
+  u64_t sum = 0;
+  // most tokens lie below the bin, and a comparison says so (the threshold is a little lower than the bin's end,
+  // by more than the divisions and products round; NaN, which compares with nothing, goes the long way)
+  const float end = mx - (float)(bin + 1) / SAMPLE_BINS_PER_UNIT;
+  const float surely_below = bin == SAMPLE_BINS - 1 ? -INFINITY : (end - 1e-5f * (fabsf(end) + fabsf(mx) + 1.0f)) * temp;
+  sample_walk(x, lo, hi, a.vec, [&](int i, float raw) __attribute__((always_inline)) {
+    if (raw < surely_below) return;
+    const float v = raw / temp;
+    const uint32_t b = bin_of(v, mx);
+    if (b < bin) {
+      sum += weight_of(v, mx);
+    } else if (b == bin) {
+      const uint32_t at = atomicAdd(&n_mine, 1u);
+      if (at < SAMPLE_BLOCK_LIST) mine[at] = make_uint2(order_key(raw), (uint32_t)i);
+    }
+  });
+  sum = block_sum(sum);
+  // a workgroup whose tokens do not fit its own list makes the row's look too long for everybody
+  const uint32_t n_here = n_mine;
+  if (threadIdx.x == 0) {
+    a.sums[(int64_t)row * a.chunks + chunk] = sum;
+    at_list = n_here ? atomicAdd(&known.listed[again], n_here <= SAMPLE_BLOCK_LIST ? n_here : SAMPLE_LIST + 1u) : 0u;
+  }
+  __syncthreads();
+  if (n_here <= SAMPLE_BLOCK_LIST)
+    for (uint32_t i = threadIdx.x; i < n_here; i += SAMPLE_THREADS)
+      if (at_list + i < SAMPLE_LIST) a.list[(int64_t)row * SAMPLE_LIST + at_list + i] = mine[i];
+}
+
+// DRAW; ``again``: behind COLLECT's second run
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(SampleArgs a, int again) {
+  __shared__ u64_t chunk_w[SAMPLE_MAX_CHUNKS];
+  __shared__ u64_t bins_w[256];
+  __shared__ uint32_t bins_n[256];
+  __shared__ uint2 list[SAMPLE_LIST];
+  __shared__ u64_t picked_above;
+  __shared__ uint32_t picked, picked_rank, key_min, key_max;
+  const int row = blockIdx.x;
+  SampleRow& known = a.rows[row];
+  const float temp = a.temperature[row];
+  if (!(temp > 0.0f) || (again && known.collect != 2u)) return;
+  const bool with_k = row_has_top_k(a, row), with_p = row_has_top_p(a, row);
+  float mraw;
+  int mi;
+  row_max(a, row, mraw, mi);
+  const float mx = mraw / temp;
+  if ((int)threadIdx.x < a.chunks) chunk_w[threadIdx.x] = a.sums[(int64_t)row * a.chunks + threadIdx.x];
+  __syncthreads();
+  if (!with_k && !with_p) {
+    sample_locate(a, row, temp, mx, mi, 0u, chunk_w);
+    return;
+  }
+  const uint32_t bin = known.bin, listed = known.listed[again];
+  const float* x = a.logits + (int64_t)row * a.row_stride;
+  const bool fits = listed <= SAMPLE_LIST;
+  if (threadIdx.x == 0) key_min = 0xffffffffu, key_max = 0u;
+  if (fits)
+    for (uint32_t i = threadIdx.x; i < listed; i += SAMPLE_THREADS) list[i] = a.list[(int64_t)row * SAMPLE_LIST + i];
+  __syncthreads();
+  // f(key, index) for the tokens of the bin
+  auto candidates = [&](auto f) __attribute__((always_inline)) {
+    if (fits) {
+      for (uint32_t i = threadIdx.x; i < listed; i += SAMPLE_THREADS) f(list[i].x, (int)list[i].y);
+    } else {
+      for (int i = threadIdx.x; i < a.V; i += SAMPLE_THREADS)
+        if (bin_of(x[i] / temp, mx) == bin) f(order_key(x[i]), i);
+    }
+  };
+  // the keys of a bin have most of their bits in common: the selections below begin at the highest in which they differ
+  uint32_t least = 0xffffffffu, most = 0u;
+  candidates([&](uint32_t key, int) __attribute__((always_inline)) {
+    least = min(least, key);
+    most = max(most, key);
+  });
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    least = min(least, (uint32_t)__shfl_xor((int)least, off, 64));
+    most = max(most, (uint32_t)__shfl_xor((int)most, off, 64));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    atomicMin(&key_min, least);
+    atomicMax(&key_max, most);
+  }
+  __syncthreads();
+  least = key_min;
+  most = key_max;
+  const int differing = least < most ? 32 - __clz(least ^ most) : 0;  // low bits that are not the same in all
+  const uint32_t common = differing == 32 ? 0u : (most >> differing) << differing;
+  // (a NaN's key is that of -inf: neither weighs anything)
+  auto scaled = [&](uint32_t key) __attribute__((always_inline)) -> float { return key_to_float(key) / temp; };
+  const u64_t above = block_sum((int)threadIdx.x < a.chunks ? chunk_w[threadIdx.x] : 0);
+  uint32_t floor_key = 0u;
+  if (with_k && !again) {
+    // the rank-th largest key of the bin
+    uint32_t prefix = common, rank = known.rank;
+    for (int left = differing; left > 0;) {
+      const int width = min(left, 8), shift = left - width;
+      bins_n[threadIdx.x] = 0u;
+      if (threadIdx.x == 0) picked = 0u, picked_rank = rank;
+      __syncthreads();
+      candidates([&](uint32_t key, int) __attribute__((always_inline)) {
+        if (left == 32 || (key >> left) == (prefix >> left)) atomicAdd(&bins_n[(key >> shift) & ((1u << width) - 1u)], 1u);
+      });
+      __syncthreads();
+      const uint32_t b = 255u - threadIdx.x, n_b = bins_n[b];  // from the largest down
+      const uint32_t upto = block_running_sum(n_b);
+      if (upto >= rank && upto - n_b < rank) {
+        picked = b;
+        picked_rank = rank - (upto - n_b);
+      }
+      __syncthreads();
+      prefix |= picked << shift;
+      rank = picked_rank;
+      left = shift;
+      __syncthreads();
+    }
+    floor_key = order_key(scaled(prefix));
+  }
+  if (with_p) {
+    u64_t limit = known.limit;
+    if (with_k && !again) {
+      u64_t kept = 0;
+      candidates([&](uint32_t key, int) __attribute__((always_inline)) {
+        const float v = scaled(key);
+        if (order_key(v) >= floor_key) kept += weight_of(v, mx);
+      });
+      const u64_t total = above + block_sum(kept);
+      limit = topp_limit(a.top_p[row], total);
+      if (total == 0) {
+        if (threadIdx.x == 0) a.out[row] = mi < a.V ? mi : 0;
+        return;
+      }
+      if (above > limit) {
+        // the nucleus ends in a bin above this one, all of whose tokens are among the k
+        u64_t w0 = 0, w1 = 0;
+        row_bins(a, row, w0, w1);
+        const u64_t upto = block_running_sum(w0 + w1);
+        const u64_t before = upto - w0 - w1;
+        if (before <= limit && limit < upto) {
+          known.bin = 2 * threadIdx.x + (before + w0 <= limit ? 1 : 0);
+          known.limit = limit;
+          known.collect = 2u;
+        }
+        return;
+      }
+    }
+    // the largest key K of the bin with above + weight(kept keys >= K) > limit
+    uint32_t prefix = common;
+    u64_t over = above;
+    for (int left = differing; left > 0;) {
+      const int width = min(left, 8), shift = left - width;
+      bins_w[threadIdx.x] = 0;
+      if (threadIdx.x == 0) picked = 0u, picked_above = over;
+      __syncthreads();
+      candidates([&](uint32_t key, int) __attribute__((always_inline)) {
+        if (left < 32 && (key >> left) != (prefix >> left)) return;
+        const float v = scaled(key);
+        if (order_key(v) >= floor_key) atomicAdd(&bins_w[(key >> shift) & ((1u << width) - 1u)], weight_of(v, mx));
+      });
+      __syncthreads();
+      const uint32_t b = 255u - threadIdx.x;
+      const u64_t w_b = bins_w[b];
+      const u64_t upto = over + block_running_sum(w_b);
+      if (upto > limit && !(upto - w_b > limit)) {
+        picked = b;
+        picked_above = upto - w_b;
+      }
+      __syncthreads();
+      prefix |= picked << shift;
+      over = picked_above;
+      left = shift;
+      __syncthreads();
+    }
+    const uint32_t floor_p = order_key(scaled(prefix));
+    if (floor_p > floor_key) floor_key = floor_p;
+  }
+  // what is kept of the bin joins its chunks
+  candidates([&](uint32_t key, int i) __attribute__((always_inline)) {
+    const float v = scaled(key);
+    if (order_key(v) >= floor_key) {
+      const u64_t w = weight_of(v, mx);
+      if (w) atomicAdd(&chunk_w[i / a.per], w);
+    }
+  });
+  __syncthreads();
+  sample_locate(a, row, temp, mx, mi, floor_key, chunk_w);
+}
+
+// flags: bit 0 some row may have top-k, bit 1 some row may have top-p, bit 2 some row may have both (7 when
+// unknown): the steps no row needs are not launched. workspace: cw_sample_workspace_bytes(n, V) bytes, 16-byte
 // aligned.
 CW_EXPORT int cw_sample(const float* logits, int64_t row_stride, int n, int V,
                         const float* temperature, const int* top_k, const float* top_p,
@@ -671,32 +766,33 @@ CW_EXPORT int cw_sample(const float* logits, int64_t row_stride, int n, int V,
     return CW_ERR_ARG;
   SampleArgs a;
   a.logits = logits; a.row_stride = row_stride; a.n = n; a.V = V;
-  a.chunks = cw_sample_chunks(V);
-  a.per = (V + a.chunks - 1) / a.chunks;
+  a.chunks = sample_chunks(n, V);
+  a.per = ((V + a.chunks - 1) / a.chunks + 3) / 4 * 4;
+  a.vec = !(row_stride & 3) && !((uintptr_t)logits & 15);
   a.temperature = temperature; a.top_k = top_k; a.top_p = top_p; a.seeds = seeds; a.draws = draws; a.out = out;
   const int64_t rc = (int64_t)n * a.chunks;
-  // 8-byte items first
+  // 16-byte items first
   u64_t* p8 = (u64_t*)workspace;
-  a.hist_p = p8; p8 += 4 * (int64_t)n * 256;
-  a.state_p = p8; p8 += (int64_t)n * 4;
-  a.psum = p8; p8 += rc;
-  u64_t* psum2 = p8; p8 += rc + n;
-  uint32_t* p4 = (uint32_t*)p8;
-  a.hist_k = p4; p4 += 4 * (int64_t)n * 256;
-  a.state_k = p4; p4 += (int64_t)n * 4;
-  a.floor_k = p4; p4 += n;
-  a.pmax = (float*)p4; p4 += rc;
-  a.pmax_i = (int*)p4; p4 += rc;
-  if ((char*)p4 > (char*)workspace + workspace_bytes) return CW_ERR_ARG;
+  a.hist_w = p8; p8 += rc * SAMPLE_BINS;
+  a.list = (uint2*)p8; p8 += (int64_t)n * SAMPLE_LIST;
+  a.hist_n = (uint32_t*)p8; p8 += rc * SAMPLE_BINS / 2;
+  a.sums = p8; p8 += rc;
+  a.rows = (SampleRow*)p8; p8 += (int64_t)n * sizeof(SampleRow) / 8;
+  a.pmax = (float*)p8;
+  a.pmax_i = (int*)(a.pmax + rc);
+  if ((char*)(a.pmax_i + rc) > (char*)workspace + workspace_bytes) return CW_ERR_ARG;
   const dim3 grid(a.chunks, n), block(SAMPLE_THREADS);
   hipLaunchKernelGGL(sample_max_kernel, grid, block, 0, stream, a);
-  if (flags & 1)
-    for (int step = 0; step < 4; ++step) hipLaunchKernelGGL(sample_topk_kernel, grid, block, 0, stream, a, step);
-  hipLaunchKernelGGL(sample_zsum_kernel, grid, block, 0, stream, a);
-  if (flags & 2) {
-    for (int step = 0; step < 4; ++step) hipLaunchKernelGGL(sample_topp_kernel, grid, block, 0, stream, a, step);
-    hipLaunchKernelGGL(sample_sums_kernel, grid, block, 0, stream, a, psum2);
+  hipLaunchKernelGGL(sample_hist_kernel, grid, block, 0, stream, a);
+  if (flags & 3) {
+    hipLaunchKernelGGL(sample_pick_kernel, dim3(n), block, 0, stream, a);
+    hipLaunchKernelGGL(sample_collect_kernel, grid, block, 0, stream, a, 0);
   }
-  hipLaunchKernelGGL(sample_locate_kernel, dim3(n), block, 0, stream, a, psum2);
+  hipLaunchKernelGGL(sample_draw_kernel, dim3(n), block, 0, stream, a, 0);
+  if ((flags & 7) == 7) {
+    hipLaunchKernelGGL(sample_collect_kernel, grid, block, 0, stream, a, 1);
+    hipLaunchKernelGGL(sample_draw_kernel, dim3(n), block, 0, stream, a, 1);
+  }
   return cw_launch_status();
 }
+static_assert(sizeof(SampleRow) % 8 == 0 && sizeof(SampleRow) / 4 <= SAMPLE_THREADS, "MAX zeroes a row's record, a word a thread");

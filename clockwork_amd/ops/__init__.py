@@ -1309,10 +1309,10 @@ def argmax(logits: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tenso
 
 
 def sample(logits, temperature, top_k, top_p, seeds, draws, out=None, any_top_k: bool = True,
-           any_top_p: bool = True) -> torch.Tensor:
+           any_top_p: bool = True, any_both: bool = True) -> torch.Tensor:
     """One token per row: rows with temperature 0 take the arg-max, the others are drawn.
-    ``any_top_k`` / ``any_top_p`` off: the caller knows that no row has that option, and its
-    kernels are not launched."""
+    ``any_top_k`` / ``any_top_p`` / ``any_both`` off: the caller knows that no row has that option
+    (or both of them), and its kernels are not launched."""
     _gpu(logits, temperature, top_k, top_p, seeds, draws, out)
     if not (logits.dtype == torch.float32 and logits.dim() == 2):
         raise KernelError("logits must be float32 [n, V]")
@@ -1333,7 +1333,7 @@ def sample(logits, temperature, top_k, top_p, seeds, draws, out=None, any_top_k:
     ws = torch.empty(int(lib.cw_sample_workspace_bytes(n, V)), dtype=torch.uint8, device=logits.device)
     _check(
         lib.cw_sample(_ptr(logits), V, n, V, _ptr(temperature), _ptr(top_k), _ptr(top_p), _ptr(seeds), _ptr(draws),
-                      _ptr(out), _ptr(ws), ws.numel(), int(bool(any_top_k)) | (int(bool(any_top_p)) << 1), _stream()),
+                      _ptr(out), _ptr(ws), ws.numel(), int(bool(any_top_k)) | (int(bool(any_top_p)) << 1) | (int(bool(any_both)) << 2), _stream()),
         "sample",
     )
     return out

@@ -73,7 +73,7 @@ class Sampler:
         if fixed is None:
             params = [s.sampling_params for s in seqs]
             if all(p.greedy for p in params):
-                fixed = None, False, False, list(seqs)
+                fixed = None, False, False, list(seqs), False
             else:
                 vocab = logits.shape[1]
                 top_k = np.array([p.top_k if 0 < p.top_k < vocab else -1 for p in params], dtype=np.int32)
@@ -83,14 +83,15 @@ class Sampler:
                 # one buffer: seeds, (draws,) temperature, top_p, top_k; the 8-byte items first
                 packed = np.concatenate([seeds.view(np.int32), np.zeros(2 * n, dtype=np.int32),
                                          temperature.view(np.int32), top_p.view(np.int32), top_k])
-                fixed = packed, bool((top_k > 0).any()), bool((top_p < 1.0).any()), list(seqs)
+                any_both = bool(((top_k > 0) & (top_p < 1.0) & (temperature > 0)).any())
+                fixed = packed, bool((top_k > 0).any()), bool((top_p < 1.0).any()), list(seqs), any_both
             self._fixed.pop(key, None)
             while len(self._fixed) >= self._KEPT:
                 self._fixed.pop(next(iter(self._fixed)))
         else:
             self._fixed.pop(key)
         self._fixed[key] = fixed   # the newest entry last
-        packed, any_top_k, any_top_p, _ = fixed
+        packed, any_top_k, any_top_p, _, any_both = fixed
         if packed is None:
             return ops.argmax(logits)
         slot = self._pinned(7 * n)
@@ -104,5 +105,5 @@ class Sampler:
         return ops.sample(
             logits, dev[4 * n : 5 * n].view(torch.float32), dev[6 * n : 7 * n], dev[5 * n : 6 * n].view(torch.float32),
             dev[0 : 2 * n].view(torch.int64), dev[2 * n : 4 * n].view(torch.int64),
-            any_top_k=any_top_k, any_top_p=any_top_p,
+            any_top_k=any_top_k, any_top_p=any_top_p, any_both=any_both,
         )

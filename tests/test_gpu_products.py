@@ -49,3 +49,45 @@ def test_float32_infinities_stay_in_their_rows_and_columns():
         got = ops.linear(x[rows].contiguous(), w)
         assert bool(torch.isinf(got[-1]).all()) and bool(torch.isinf(got[:, 69]).all())
         assert bool((got[:-1, :69] == 528).all())
+
+
+# odd sizes (rows that do not begin at 16 bytes), values in steps of a half (bins of thousands of equal logits, more
+# than a workgroup's list and a row's list hold), nearly flat rows (all in a few bins), spread ones
+@pytest.mark.parametrize("V,kind", [(1, "spread"), (511, "spread"), (2049, "steps"), (33333, "flat"), (151936, "steps"), (151936, "spread")])
+def test_sampling_lists_bins_and_chunks(V, kind):
+    """Every option against the plain definition, and the same tokens however many rows share the launch (which
+    sets how a row is cut)."""
+    from clockwork_amd import ops
+    from tests.plain import qwen2_plain as plain
+
+    gen = torch.Generator(device=DEV).manual_seed(V)
+    n = 20
+    logits = torch.randn(n, V, device=DEV, generator=gen) * {"spread": 5.0, "steps": 2.0, "flat": 0.01}[kind]
+    if kind == "steps":
+        logits = (2.0 * logits).round() / 2.0
+    temps = torch.tensor([0.7, 1.0, 2.5, 0.0] * 5, device=DEV)
+    ks = [-1] * 4 + [7] * 4 + [-1] * 4 + [max(1, V // 2)] * 4 + [30] * 4   # the fourth: the nucleus ends far above the k-th token
+    ps = [1.0] * 8 + [0.8] * 4 + [0.3] * 4 + [0.97] * 4
+    top_k, top_p = torch.tensor(ks, dtype=torch.int32, device=DEV), torch.tensor(ps, device=DEV)
+    seeds = torch.arange(n, dtype=torch.int64, device=DEV) + 11
+    draws = torch.arange(n, dtype=torch.int64, device=DEV)
+    got = ops.sample(logits, temps, top_k, top_p, seeds, draws)
+    for i in range(n):
+        one = slice(i, i + 1)
+        both = ks[i] > 0 and ps[i] < 1.0
+        alone = ops.sample(logits[one].contiguous(), temps[one], top_k[one], top_p[one], seeds[one], draws[one],
+                           any_top_k=ks[i] > 0, any_top_p=ps[i] < 1.0, any_both=both)
+        assert int(alone) == int(got[i])
+        if float(temps[i]) == 0.0:
+            assert int(got[i]) == int(logits[i].argmax())
+            continue
+        probs = plain.sampling_probs(logits[i].cpu(), float(temps[i]), ks[i], ps[i])
+        want, margin = plain.draw(probs, plain.uniform01(int(seeds[i]), int(draws[i])))
+        # the plain nucleus takes equal tokens in the order of a sort, ours keeps all that equal its last one
+        if kind != "steps" or ps[i] == 1.0:
+            assert int(got[i]) == want or margin < 1e-4, f"row {i}: got {int(got[i])}, plain draws {want} ({margin})"
+    many = 300
+    if V <= 40000:
+        rows = torch.arange(many, device=DEV) % n
+        again = ops.sample(logits[rows], temps[rows], top_k[rows], top_p[rows], seeds[rows], draws[rows])
+        assert torch.equal(again, got[rows])
