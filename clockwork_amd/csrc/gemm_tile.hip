@@ -738,3 +738,251 @@ CW_EXPORT int cw_gemm_bf16_wide_grouped(int mode, const void* X, int64_t ldx, co
 
 // rows of a tile of cw_gemm_bf16_wide_grouped
 CW_EXPORT int cw_gemm_bf16_wide_rows(void) { return W_BM; }
+
+// ------------------------------------------------------------------------------------------------
+// Tiles for the steps between (65 to some 1000 rows): the wide tiles leave most compute units without one there,
+// and so do the library's (a step of 256 rows of the 1.5B shape: 48 tiles for its down product, on 256 units).
+//
+// A workgroup of 4 waves owns BM rows of x by BN rows of W (64 or 128 each), a wave a quarter of it. K goes in stages
+// of 64 elements straight into LDS, as blocks of 8 rows x 128 bytes (a load instruction each: whole lines, which come
+// in a fifth to a third faster than the half lines of stages of 32) through a ring of three. The eight granules of a
+// row change places by (row >> 1) & 7, so that the 16 lanes that read one granule of 16 rows touch every bank once.
+// Workgroups are dealt to the 8 XCDs in turn; an XCD takes a run of neighbouring tiles, the row tiles of one W tile next
+// to each other, so that W comes from memory once, into one L2.
+// A product whose tiles leave compute units idle is cut over K (MODE 3): run z of every tile is a work item of its own
+// and writes plane z of the partial sums, which the next norm kernel adds in their order.
+// Bound by the loads into LDS, about 50 GB/s into each compute unit (deeper rings do not help): a tile's time goes
+// with (BM + BN) K, which is what cw_gemm_bf16_mid_choice weighs.
+// Measured on an MI355X with the norm behind it, library -> here (us): down product of the 0.5B shape 14.5 -> 11.7 for 144
+// rows, 25.0 -> 18.0 for 640; of the 1.5B shape 28.1 -> 20.5 for 144, 35.8 -> 23.3 for 256, 44.0 -> 34.7 for 640; of the 7B
+// shape 165 -> 52 for 144. Gate/up product and gate of the 0.5B shape 16.5 -> 10.9 for 144 rows; of the 1.5B shape
+// 29.4 -> 26.3 for 144, and from 200 rows on the library's larger tiles, which read less, win.
+#define MID_SLOTS 3
+#define MID_MAX_PLANES 12
+
+template <int MODE, int BM, int BN>
+__global__ __launch_bounds__(256, 2) void gemm_mid_bf16_kernel(WideArgs a) {
+  extern __shared__ __align__(1024) unsigned char w_smem[];
+  constexpr int XB = BM / 8, WB = BN / 8, LOADS = (XB + WB) / 4, STAGE = (XB + WB) * W_BLOCK;
+  constexpr int TM = BM / 32, TN = BN / 32;  // 16 x 16 tiles of a wave
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int c = lane & 15, s = lane >> 4;
+  const int M = a.M, N = a.N, K = a.K, I = N / 2;
+  const int run = gridDim.x >> 3, rest = gridDim.x & 7, xcd = blockIdx.x & 7;
+  const int tile = xcd * run + min(xcd, rest) + (blockIdx.x >> 3);
+  const int tm = tile % a.tiles_m, tn = tile / a.tiles_m % a.tiles_n, plane = tile / (a.tiles_m * a.tiles_n);
+  const int m0 = tm * BM, w0 = tn * (MODE == 2 ? BN / 2 : BN);
+  const int stages = K / 64;
+  const int first = MODE == 3 ? (int)((int64_t)stages * plane / a.k_splits) : 0;
+  const int last = (MODE == 3 ? (int)((int64_t)stages * (plane + 1) / a.k_splits) : stages) - 1;
+
+  __amdgpu_buffer_rsrc_t xr, wr;
+  xr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.X + (int64_t)m0 * a.ldx), 0,
+                                         (int)(uint32_t)(((int64_t)(M - m0 - 1) * a.ldx + K) * 2), 0x00020000);
+  wr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.W + (int64_t)w0 * K), 0,
+                                         (int)(uint32_t)((int64_t)(N - w0) * K * 2), 0x00020000);
+  // load i of a wave: block wave * LOADS + i of a stage, the x blocks first. (Of a size that hangs on no template
+  // parameter, so that the host pass takes the loads below.)
+  uint32_t at[8];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int block = wave * LOADS + i;
+    int64_t from;
+    if (block < XB) {
+      from = (int64_t)(block * 8 + (lane >> 3)) * a.ldx;
+    } else {
+      const int rb = (block - XB) * 8 + (lane >> 3);
+      if (MODE == 2) {  // a wave's rows are gate rows followed by the up rows with the same indices
+        const int q = rb % (BN / 2), i2 = rb / (BN / 2) * (BN / 4) + q % (BN / 4);
+        from = (int64_t)(q < BN / 4 ? i2 : I + i2) * K;
+      } else {
+        from = (int64_t)rb * K;
+      }
+    }
+    at[i] = (uint32_t)((from + ((lane & 7) ^ ((block * 4 + (lane >> 4)) & 7)) * 8) * 2);
+  }
+  auto fetch = [&](int stage, int slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int block = wave * LOADS + i;
+      unsigned char* to = w_smem + (slot * STAGE + block * W_BLOCK);
+      if (block < XB) __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t*)to, 16, at[i], stage * 128, 0, 0);
+      else __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void_t*)to, 16, at[i], stage * 128, 0, 0);
+    }
+  };
+  f32x4_t acc[TM][TN];
+#pragma unroll
+  for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < TN; ++ni) acc[mi][ni] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int i = 0; i < MID_SLOTS - 1; ++i) fetch(min(first + i, last), i);
+  int slot = 0;
+  for (int t = first; t <= last; ++t) {
+    // this wave's loads of the stage are in; behind the barrier every wave's are, and every wave has read the stage
+    // before it, whose slot the next loads take (past the last stage it is asked for again, and nobody reads it:
+    // the number of loads in flight stays what the wait counts on)
+    W_WAIT_LOADS((MID_SLOTS - 2) * LOADS);
+    W_BARRIER();
+    fetch(min(t + MID_SLOTS - 1, last), (slot + MID_SLOTS - 1) % MID_SLOTS);
+    const unsigned char* base = w_smem + slot * STAGE + c * 128;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int g = ((kk * 4 + s) ^ ((c >> 1) & 7)) * 16;
+      bf16x8_t xf[TM], wf[TN];
+#pragma unroll
+      for (int ni = 0; ni < TN; ++ni) wf[ni] = *reinterpret_cast<const bf16x8_t*>(base + (XB * 1024 + (wn * TN + ni) * 2048) + g);
+#pragma unroll
+      for (int mi = 0; mi < TM; ++mi) xf[mi] = *reinterpret_cast<const bf16x8_t*>(base + (wm * TM + mi) * 2048 + g);
+#pragma unroll
+      for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < TN; ++ni) acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ni], xf[mi], acc[mi][ni], 0, 0, 0);
+    }
+    slot = (slot + 1) % MID_SLOTS;
+  }
+  W_WAIT_LOADS(0);  // no load may reach LDS after the workgroup has gone
+
+  // lane (c, s) holds columns 4 s .. 4 s + 3 of W block ni for row c of x block mi
+  const int out_cols = MODE == 2 ? I : N;
+#pragma unroll
+  for (int mi = 0; mi < TM; ++mi) {
+    const int m = m0 + (wm * TM + mi) * 16 + c;
+    if (m >= M) continue;
+#pragma unroll
+    for (int ni = 0; ni < (MODE == 2 ? TN / 2 : TN); ++ni) {
+      const int n = w0 + (MODE == 2 ? wn * (BN / 4) : wn * (BN / 2)) + ni * 16 + 4 * s;
+      if (n >= out_cols) continue;
+      f32x4_t v = acc[mi][ni];
+      if (MODE == 3) {
+        float* dst = (float*)a.C + ((int64_t)plane * M + m) * a.ldc + n;
+        if (n + 4 <= N && !(a.ldc & 3)) {
+          *reinterpret_cast<f32x4_t*>(dst) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) dst[e] = v[e];
+        }
+        continue;
+      }
+      if (MODE == 2) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = cw_gated(v[e], acc[mi][ni + (MODE == 2 ? TN / 2 : 0)][e], a.act);
+      } else if (a.bias != nullptr) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) v[e] += a.bias_f32 ? ((const float*)a.bias)[n + e] : __bfloat162float(((const bf16_t*)a.bias)[n + e]);
+      }
+      bf16_t* dst = (bf16_t*)a.C + (int64_t)m * a.ldc + n;
+      const uint32_t lo = w_pack_bf16(v[0], v[1]), hi = w_pack_bf16(v[2], v[3]);
+      if (n + 4 <= out_cols && !(a.ldc & 3)) {
+        *reinterpret_cast<uint2*>(dst) = make_uint2(lo, hi);
+      } else {
+        const uint32_t w2[2] = {lo, hi};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < out_cols) ((uint16_t*)dst)[e] = (uint16_t)(w2[e >> 1] >> ((e & 1) * 16));
+      }
+    }
+  }
+}
+
+template <int MODE, int BM, int BN>
+static int mid_launch(WideArgs a, hipStream_t stream) {
+  constexpr int SMEM = MID_SLOTS * (BM + BN) / 8 * W_BLOCK;
+  static bool raised = false;
+  if (!raised) {
+    if (hipFuncSetAttribute((const void*)gemm_mid_bf16_kernel<MODE, BM, BN>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) != hipSuccess)
+      return CW_ERR_LAUNCH;
+    raised = true;
+  }
+  const int out_cols = MODE == 2 ? a.N / 2 : a.N;
+  const int per_tile = MODE == 2 ? BN / 2 : BN;
+  a.tiles_n = (out_cols + per_tile - 1) / per_tile;
+  a.tiles_m = (a.M + BM - 1) / BM;
+  const int64_t total = (int64_t)a.tiles_m * a.tiles_n * (MODE == 3 ? a.k_splits : 1);
+  if (total > 0x7fffffff) return CW_ERR_SIZE;
+  hipLaunchKernelGGL((gemm_mid_bf16_kernel<MODE, BM, BN>), dim3((unsigned)total), dim3(256), SMEM, stream, a);
+  return cw_launch_status();
+}
+
+// y = x W^T through the tiles between. mode 0: bfloat16 [M, N], + bias [N] when given; 2: W = [gate; up], the gated
+// product bfloat16 [M, N / 2] (``act`` as elsewhere); 3: float32 planes [k_splits, M, N] of partial sums over runs of K.
+// bm, bn: 64 or 128 each. K a multiple of 64 (of at least 64 elements a run), both matrices below 4 GiB.
+CW_EXPORT int cw_gemm_bf16_mid(int mode, const void* X, int64_t ldx, const void* W, const void* bias, int bias_f32, void* C,
+                               int64_t ldc, int M, int N, int K, float act, int k_splits, int bm, int bn, hipStream_t stream) {
+  if (M < 0 || N <= 0 || K <= 0 || (mode != 0 && mode != 2 && mode != 3) || !(act >= 0.0f || mode == 2)) return CW_ERR_ARG;
+  if (((uintptr_t)X & 15) || ((uintptr_t)W & 15) || ((uintptr_t)C & (mode == 3 ? 15 : 7)) || !C) return CW_ERR_ARG;
+  if ((mode == 2 && (N & 1)) || (mode != 0 && bias != nullptr)) return CW_ERR_ARG;
+  if ((K & 63) || (ldx & 7) || ldx < K || ldc < (mode == 2 ? N / 2 : N)) return CW_ERR_ARG;
+  if (mode == 3 ? (k_splits < 1 || k_splits > MID_MAX_PLANES || K / 64 < k_splits) : k_splits != 1) return CW_ERR_ARG;
+  if ((bm != 64 && bm != 128) || (bn != 64 && bn != 128)) return CW_ERR_ARG;
+  if ((int64_t)N * K * 2 >= (1ll << 32) || ((int64_t)M * ldx + 128 * ldx) * 2 >= (1ll << 32)) return CW_ERR_SIZE;
+  if (M == 0) return CW_OK;
+  WideArgs a{(const bf16_t*)X, ldx, (const bf16_t*)W, bias, bias_f32, C, ldc, M, N, K, 0, 0, k_splits};
+  a.act = act;
+#define CW_MID(BM_, BN_)                                                                                                        \
+  if (bm == BM_ && bn == BN_)                                                                                                   \
+    return mode == 0 ? mid_launch<0, BM_, BN_>(a, stream) : mode == 2 ? mid_launch<2, BM_, BN_>(a, stream) : mid_launch<3, BM_, BN_>(a, stream)
+  CW_MID(64, 64);
+  CW_MID(64, 128);
+  CW_MID(128, 64);
+  CW_MID(128, 128);
+#undef CW_MID
+  return CW_ERR_ARG;
+}
+
+// Time of a product's work items in microseconds as the choice below weighs them, without what every launch costs:
+// rounds over the compute units, a stage of 64 elements of K taking what its loads take, and the planes' way to
+// memory and back. The constants are fits to the measurements above (64 x 64 and 64 x 128 tiles share a compute unit
+// with others, which covers for a part of their last round).
+static float mid_time(int M, int N, int K, int bm, int bn, int planes, int cus) {
+  const float stage = bm + bn == 128 ? 0.27f : bm + bn == 192 ? 0.38f : bm == 128 ? 0.62f : 1.04f;
+  const int64_t items = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * planes;
+  const int64_t rounds = (items + cus - 1) / cus;
+  const float share = rounds > 1 && bm + bn < 256 ? 0.85f : 1.0f;
+  const int stages = (K / 64 + planes - 1) / planes;
+  return share * (float)(rounds * stages) * stage + (planes > 1 ? 2.2e-6f * (float)planes * (float)M * (float)N : 0.0f);
+}
+
+// Which of this file's kernels a product of many rows should run on: 0 the library's, else bm | bn << 10 |
+// planes << 20 (bm 256: cw_gemm_bf16_wide_partial, else cw_gemm_bf16_mid). mode as there.
+// Where the lines lie, measured for the layers of the 0.5B, 1.5B, 3B and 7B shapes with 72 to 2048 rows:
+//  * mode 3 (a sum that the next norm adds up): K of three times N and more, up to 2048 rows: here everywhere (but for
+//    4 % at 1536 rows of the 3B shape). A squarer matrix while M N is below 1.2 M: beyond, the planes cost more than
+//    the library's idle units.
+//  * mode 2: M N K up to 4.5e9 (72 rows of the 1.5B shape: 28.0 -> 22.9 us, 208 rows 32.2 -> 31.8), and up to 690 rows for
+//    a matrix of at most 9 M elements.
+//  * mode 0: matrices of at most 2 M elements and up to 1536 rows (q/k/v of the 0.5B shape: 8.1 -> 6.3 us for 144 rows), or of
+//    4 M and 320 to 1024 (of the 1.5B shape: 14.3 -> 12.8 for 1000; 8.6 -> 8.8 for 144).
+CW_EXPORT int cw_gemm_bf16_mid_choice(int mode, int M, int N, int K, int64_t ldx, int cus) {
+  if (M <= 64 || M > 2048 || N <= 0 || K < 256 || (K & 63) || (ldx & 7) || ldx < K || cus < 8) return 0;
+  if ((int64_t)N * K * 2 >= (1ll << 32) || ((int64_t)M * ldx + 128 * ldx) * 2 >= (1ll << 32)) return 0;
+  const int64_t elements = (int64_t)N * K;
+  if (mode == 0)
+    return (elements <= 2 << 20 && M <= 1536) || (elements <= 4 << 20 && M >= 320 && M <= 1024) ? 64 | 64 << 10 | 1 << 20 : 0;
+  if (mode == 2) {
+    if ((N & 1) || !((int64_t)M * elements <= 4500000000ll || (elements <= 9 << 20 && M <= 690))) return 0;
+  } else if (mode != 3 || !(K >= 3 * N || (int64_t)M * N <= 1200000)) {
+    return 0;
+  }
+  int best = 0;
+  float least = 0.0f;
+  for (int bm = 64; bm <= 128; bm += 64)
+    for (int bn = 64; bn <= 128; bn += 64)
+      for (int planes = 1; planes <= (mode == 3 ? MID_MAX_PLANES : 1) && K / planes >= 256; ++planes) {
+        const float t = mid_time(M, N, K, bm, bn, planes, cus);
+        if (best == 0 || t < least) {
+          least = t;
+          best = bm | bn << 10 | planes << 20;
+        }
+      }
+  if (mode == 3 && M >= 512)
+    for (int planes = 2; planes <= 8; ++planes)
+      if (cw_gemm_bf16_wide_partial_ok(M, N, K, ldx, planes) && mid_time(M, N, K, W_BM, W_BN, planes, cus) < least) {
+        least = mid_time(M, N, K, W_BM, W_BN, planes, cus);
+        best = W_BM | W_BN << 10 | planes << 20;
+      }
+  return best;
+}

@@ -119,6 +119,8 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_gemm_bf16_wide": [I, P, L, P, P, I, P, L, I, I, I, F, I, P],
             "cw_gemm_bf16_wide_partial_ok": [I, I, I, L, I],
             "cw_gemm_bf16_wide_partial": [P, L, P, P, L, I, I, I, I, I, P],
+            "cw_gemm_bf16_mid_choice": [I, I, I, I, L, I],
+            "cw_gemm_bf16_mid": [I, P, L, P, P, I, P, L, I, I, I, F, I, I, I, P],
             "cw_gemm_bf16_wide_grouped": [I, P, L, P, L, P, L, I, I, P, P, I, P, P, F, I, P],
         },
         "rowwise": {
@@ -513,13 +515,14 @@ def fresh_state_rows(pool: torch.Tensor, slots: torch.Tensor, starts: torch.Tens
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias=None, out_dtype=None, partial_ok: bool = False,
-           policy: "ProductPolicy | None" = None):
+           policy: "ProductPolicy | None" = None, portions_partial_ok: bool = False):
     """y = x @ weight.T (+ bias). float32: the true-float32 HIP product. bfloat16: few rows go
     through the weight-streaming kernel, many through the library product (as the reference's
     engine uses one) or, where ``policy`` (the calling engine's :class:`ProductPolicy`) says so,
     through this package's tiled kernels; float32 accumulation either way. With ``partial_ok``
     the result may come back as :class:`PartialSums` (a narrow output with a long K, few rows):
-    only for a result that goes straight into ``add_rmsnorm``."""
+    only for a result that goes straight into ``add_rmsnorm``. ``portions_partial_ok``: with many rows
+    as well, by the rule of ``cw_gemm_bf16_mid_choice`` (csrc/gemm_tile.hip)."""
     policy = policy if policy is not None else DEFAULT_POLICY
     _gpu(x, weight, bias)
     M, K = x.shape
@@ -574,6 +577,14 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias=None, out_dtype=None, par
         splits = _wide_partial_chosen(x, weight, policy)
         if splits:
             return linear_wide_partial(x, weight, splits)
+    if M > STREAM_MAX_ROWS and x.is_contiguous() and out_dtype is None:
+        if portions_partial_ok and bias is None and not (M >= WIDE_PRODUCT_MIN_ROWS and (N, K) in policy.wide_partial_choices):
+            choice = _load("gemm_tile").cw_gemm_bf16_mid_choice(3, M, N, K, K, _compute_units(x.device))
+            if choice:
+                return linear_mid(x, weight, choice, partial=True)
+        choice = _load("gemm_tile").cw_gemm_bf16_mid_choice(0, M, N, K, K, _compute_units(x.device))
+        if choice and (bias is None or bias.dtype in (torch.bfloat16, torch.float32)):
+            return linear_mid(x, weight, choice, bias=bias)
     if policy.hip_products and K % 8 == 0 and x.is_contiguous():
         y = linear_tiled(x, weight, bias)
     elif _wide_product_chosen(x, weight, bias, policy):
@@ -738,16 +749,18 @@ def linear_tiled(x: torch.Tensor, weight: torch.Tensor, bias=None, swiglu: bool 
 WIDE_MIN_TILES = 64
 # The engine takes the wide-tile kernel for the gate/up product by itself (no ``hip_products``)
 # where it beats the library product followed by the gate kernel. Measured on an MI355X over the
-# Qwen2.5 layer shapes from 0.5B to 72B with 256 to 4096 rows: with 180 tiles or more (seven tenths
-# of the compute units busy in the last round) and 1024 rows or more it is 5 to 25 % faster; with
-# fewer rows the product is bound by reading W once, which the library does better for the large
-# shapes (and 512 rows win only for the small ones). Against the library's TUNED choice it wins for
+# Qwen2.5 layer shapes from 0.5B to 72B with 256 to 4096 rows: with 180 tiles or more and 1024 rows or
+# more it is 5 to 25 % faster. With fewer rows it is for weights of at most 64 M elements where its tiles fill seven
+# tenths of their rounds over the compute units (us, library and gate against this: 1.5B shape, 400 rows, 188 tiles
+# 41.5 / 36.1; 640 rows, 282 tiles 52.4 / 68.3; 1000 rows, 376 tiles 88.0 / 71.2; 3B shape, 400 rows, 230 tiles 56.4 / 45.1;
+# 7B shape, 400 rows 144 / 132, 640 rows 184 / 198: there reading W bounds both). Against the library's TUNED choice it wins for
 # the 0.5B, 1.5B, 3B, 14B and 32B shapes (the 1.5B shape's whole prefill step: 8.9 -> 7.9 ms) and
 # loses 3 % of the step for the 7B and 72B shapes, so a start-up that tunes (``library_tuning``)
 # times both ways on the model's own weights and keeps the faster (``ProductPolicy.swiglu_choices``).
 WIDE_SWIGLU_MIN_TILES = 180
 WIDE_SWIGLU_MIN_ROWS = 1024
-WIDE_SWIGLU_SMALL_WEIGHTS = 64 << 20    # elements of [gate; up] up to which 512 rows are enough
+WIDE_SWIGLU_FILL = 0.72
+WIDE_SWIGLU_SMALL_WEIGHTS = 64 << 20    # elements of [gate; up]
 
 _cu_counts: dict = {}
 
@@ -762,9 +775,14 @@ def _compute_units(device) -> int:
 def wide_swiglu_pays(M: int, two_i: int, K: int, ldx: int) -> bool:
     """Is the gate/up product of M rows faster through the wide-tile kernel (with the gate in its
     epilogue) than through the library and the gate kernel?"""
-    if M < WIDE_SWIGLU_MIN_ROWS and not (M >= WIDE_SWIGLU_MIN_ROWS // 2 and two_i * K <= WIDE_SWIGLU_SMALL_WEIGHTS):
+    if M < WIDE_SWIGLU_MIN_ROWS // 4:
         return False
-    return _load("gemm_tile").cw_gemm_bf16_wide_tiles(2, M, two_i, K, ldx) >= WIDE_SWIGLU_MIN_TILES
+    tiles = _load("gemm_tile").cw_gemm_bf16_wide_tiles(2, M, two_i, K, ldx)
+    if tiles < WIDE_SWIGLU_MIN_TILES:
+        return False
+    units = _compute_units(torch.device("cuda", torch.cuda.current_device()))
+    return M >= WIDE_SWIGLU_MIN_ROWS or (two_i * K <= WIDE_SWIGLU_SMALL_WEIGHTS
+                                         and tiles >= WIDE_SWIGLU_FILL * units * -(-tiles // units))
 
 
 @contextlib.contextmanager
@@ -924,6 +942,31 @@ def linear_wide_partial(x: torch.Tensor, weight: torch.Tensor, k_splits: int) ->
     _check(lib.cw_gemm_bf16_wide_partial(_ptr(x), x.stride(0), _ptr(weight), _ptr(parts), N, M, N, K, int(k_splits),
                                          _compute_units(x.device), _stream()), "gemm_bf16_wide_partial")
     return PartialSums(parts)
+
+
+def linear_mid(x: torch.Tensor, weight: torch.Tensor, choice: int, bias=None, swiglu: bool = False, partial: bool = False,
+               limit: float = 0.0):
+    """x @ weight.T through the tiles for the steps between (csrc/gemm_tile.hip), of the sizes that ``choice`` names
+    (what ``cw_gemm_bf16_mid_choice`` returned): bfloat16 (+ bias), the gated product of [gate; up] with
+    ``swiglu``, or :class:`PartialSums` over runs of K with ``partial``."""
+    _gpu(x, weight, bias)
+    M, K = x.shape
+    N = weight.shape[0]
+    bm, bn, planes = choice & 1023, choice >> 10 & 1023, choice >> 20
+    if not (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.shape[1] == K):
+        raise KernelError("a tiled product is bfloat16, x [M, K] with weight [N, K]")
+    if bias is not None and not (bias.numel() == N and bias.dtype in (torch.bfloat16, torch.float32) and not swiglu and not partial):
+        raise KernelError("bias must be [N] bfloat16 or float32")
+    if partial and bm == 256:
+        return linear_wide_partial(x, weight, planes)
+    if partial:
+        out = torch.empty((planes, M, N), dtype=torch.float32, device=x.device)
+    else:
+        out = torch.empty((M, N // 2 if swiglu else N), dtype=torch.bfloat16, device=x.device)
+    _check(_load("gemm_tile").cw_gemm_bf16_mid(3 if partial else 2 if swiglu else 0, _ptr(x), K, _ptr(weight), _ptr(bias),
+                                               int(bias is not None and bias.dtype == torch.float32), _ptr(out), out.shape[-1],
+                                               M, N, K, float(limit), planes, bm, bn, _stream()), "gemm_bf16_mid")
+    return PartialSums(out) if partial else out
 
 
 # a long portion's product is a candidate for the wide-tile kernel's partial sums when whole tiles
@@ -1086,6 +1129,9 @@ def linear_swiglu(x, gate_up_weight: torch.Tensor, policy: "ProductPolicy | None
                                                   _stream()), "gemm_bf16_skinny(swiglu)")
         return out
     if x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16 and K % 8 == 0 and x.is_contiguous():
+        choice = _load("gemm_tile").cw_gemm_bf16_mid_choice(2, M, two_i, K, K, _compute_units(x.device))
+        if choice:
+            return linear_mid(x, gate_up_weight, choice, swiglu=True, limit=limit)
         if policy.hip_products:
             return linear_tiled(x, gate_up_weight, swiglu=True, limit=limit)
         if wide_swiglu_pays(M, two_i, K, K):

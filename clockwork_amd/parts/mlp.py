@@ -34,7 +34,7 @@ class SwiGLU(Part):
 
     def forward(self, x, ctx) -> torch.Tensor:
         policy = getattr(ctx, "products", None)
-        return ops.linear(ops.linear_swiglu(x, self.gate_up, policy=policy), self.down, partial_ok=True, policy=policy)
+        return ops.linear(ops.linear_swiglu(x, self.gate_up, policy=policy), self.down, partial_ok=True, policy=policy, portions_partial_ok=True)
 
 
 class GatedMLP(Part):

@@ -91,3 +91,59 @@ def test_sampling_lists_bins_and_chunks(V, kind):
         rows = torch.arange(many, device=DEV) % n
         again = ops.sample(logits[rows], temps[rows], top_k[rows], top_p[rows], seeds[rows], draws[rows])
         assert torch.equal(again, got[rows])
+
+
+# rows and columns that end inside a tile, one tile, K of a single stage a run, runs of unequal length, every tile size
+@pytest.mark.parametrize("bm", [64, 128])
+@pytest.mark.parametrize("bn", [64, 128])
+@pytest.mark.parametrize("M,N,K", [(65, 64, 256), (130, 194, 320), (257, 1536, 1536), (1, 70, 640)])
+def test_tiles_between_the_narrow_and_the_wide(M, N, K, bm, bn):
+    """Plain with a bias, gated with each activation, and partial sums over runs of K."""
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(M + N)
+    x = torch.randn(M, K, device=DEV, generator=gen).to(torch.bfloat16)
+    w = (torch.randn(N, K, device=DEV, generator=gen) / K ** 0.5).to(torch.bfloat16)
+    want = x.float() @ w.float().t()
+    # float32 sums of K products of about 1 / sqrt(K): a few units of 2^-24 times sqrt(K); then one rounding to bfloat16
+    f32 = dict(rtol=1e-4, atol=1e-4)
+    bf16 = dict(rtol=2.0 ** -8 + 1e-4, atol=1e-4)
+    for planes in (1, 3, 4):
+        got = ops.linear_mid(x, w, bm | bn << 10 | planes << 20, partial=True)
+        assert got.parts.shape == (planes, M, N)
+        torch.testing.assert_close(got.sum(), want, **f32)
+        first = (K // 64 // planes) * 64   # the first run's elements: stages [0, stages / planes)
+        torch.testing.assert_close(got.parts[0], x[:, :first].float() @ w[:, :first].float().t(), **f32)
+    one = bm | bn << 10 | 1 << 20
+    for bias in (None, torch.randn(N, device=DEV, generator=gen), torch.randn(N, device=DEV, generator=gen).to(torch.bfloat16)):
+        got = ops.linear_mid(x, w, one, bias=bias)
+        torch.testing.assert_close(got.float(), want + (0 if bias is None else bias.float()), **bf16)
+    g, u = want[:, : N // 2], want[:, N // 2:]
+    gated = {0.0: torch.nn.functional.silu(g) * u, ops.RELU_GATE: torch.relu(g) * u,
+             0.5: torch.clamp(g, max=0.5) * torch.sigmoid(1.702 * torch.clamp(g, max=0.5)) * (torch.clamp(u, -0.5, 0.5) + 1.0)}
+    for limit, ref in gated.items():
+        torch.testing.assert_close(ops.linear_mid(x, w, one, swiglu=True, limit=limit).float(), ref, **bf16)
+
+
+def test_products_of_a_portion_by_their_rule():
+    """What the rule names runs and is the product, on every side of its lines."""
+    from clockwork_amd import ops
+
+    lib = ops._load("gemm_tile")
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    for N, K in ((256, 1024), (896, 896), (200, 320)):
+        w = (torch.randn(N, K, device=DEV, generator=gen) / K ** 0.5).to(torch.bfloat16)
+        for M in (64, 65, 100, 319, 700, 1030):
+            x = torch.randn(M, K, device=DEV, generator=gen).to(torch.bfloat16)
+            want = x.float() @ w.float().t()
+            got = ops.linear(x, w, partial_ok=True, portions_partial_ok=True)
+            if M > 64:
+                assert isinstance(got, ops.PartialSums) == bool(lib.cw_gemm_bf16_mid_choice(3, M, N, K, K, ops._compute_units(x.device)))
+            got = got.sum() if isinstance(got, ops.PartialSums) else got.float()
+            torch.testing.assert_close(got, want, rtol=2.0 ** -8 + 1e-4, atol=1e-4)
+            torch.testing.assert_close(ops.linear(x, w).float(), want, rtol=2.0 ** -8 + 1e-4, atol=1e-4)
+            h = ops.linear_swiglu(x, w).float()
+            ref = torch.nn.functional.silu(want[:, : N // 2]) * want[:, N // 2:]
+            # the library's path rounds the product to bfloat16 before the gate: two roundings of up to 2^-8 each side
+            torch.testing.assert_close(h, ref, rtol=4 * 2.0 ** -8, atol=2e-2)
+    assert lib.cw_gemm_bf16_mid_choice(3, 144, 1536, 8960 + 32, 8992, 256) == 0   # K no whole number of stages
