@@ -113,7 +113,10 @@ template <> struct Chunk4<bf16_t> {
   }
 };
 
-// KC: chunks of 4 elements a thread holds (rows of up to 1024 * KC elements)
+// KC: chunks of 4 elements a thread holds (rows of up to 1024 * KC elements).
+// Bound, for few rows, by its trips to memory, about a microsecond each: the row, the weights, the pending output and
+// up to eight planes of partial sums are all asked for before any of them is used (asked for one after the other, the
+// norm of 8 rows of 1536 with an output and six planes pending took 5.75 us in a decode step, 5.0 so).
 template <typename T, typename WT, typename DT, int KC>
 __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict__ resid, const T* __restrict__ delta0,
                                                               const DT* __restrict__ delta,
@@ -131,7 +134,8 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict_
   T* o2 = out2 ? out2 + (int64_t)i * H : nullptr;
   const bool write_back = rows == nullptr && (dl != nullptr || d0 != nullptr);
   const int n_chunks = H / 4;
-  float v[KC][4], w[KC][4];
+  constexpr int PU = KC <= 2 ? 8 : KC <= 4 ? 4 : 2;  // planes on their way at a time
+  float v[KC][4], w[KC][4], e0[KC][4], d[PU][KC][4];
 #pragma unroll
   for (int k = 0; k < KC; ++k) {
     const int ch = threadIdx.x + k * 256;
@@ -142,33 +146,35 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict_
       v[k][0] = v[k][1] = v[k][2] = v[k][3] = 0.0f;
     }
   }
-  if (d0) {  // an earlier branch's output that was not added yet: it comes first, as it would have
+  if (d0) {
 #pragma unroll
     for (int k = 0; k < KC; ++k) {
       const int ch = threadIdx.x + k * 256;
-      if (ch < n_chunks) {
-        float d[4];
-        Chunk4<T>::load(d0 + ch * 4, d);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[k][e] += d[e];
-      }
+      if (ch < n_chunks) Chunk4<T>::load(d0 + ch * 4, e0[k]);
     }
   }
-  if (dl) {
-    // the partial sums are added in order, but fetched PU at a time: every trip to memory that
-    // waits for the one before costs about a microsecond, more than the rest of this kernel
-    constexpr int PU = KC <= 4 ? 4 : 2;
+  auto load_planes = [&](int q0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < PU; ++u)
+#pragma unroll
+      for (int k = 0; k < KC; ++k) {
+        const int ch = threadIdx.x + k * 256;
+        if (q0 + u < parts && ch < n_chunks) Chunk4<DT>::load(dl + (q0 + u) * part_stride + ch * 4, d[u][k]);
+        else d[u][k][0] = d[u][k][1] = d[u][k][2] = d[u][k][3] = 0.0f;
+      }
+  };
+  if (dl) load_planes(0);
+  if (d0) {  // an earlier branch's output that was not added yet: it comes first, as it would have
+#pragma unroll
+    for (int k = 0; k < KC; ++k)
+      if ((int)threadIdx.x + k * 256 < n_chunks)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[k][e] += e0[k][e];
+  }
+  if (dl) {  // the partial sums are added in order
     float acc[KC][4];
     for (int q0 = 0; q0 < parts; q0 += PU) {
-      float d[PU][KC][4];
-#pragma unroll
-      for (int u = 0; u < PU; ++u)
-#pragma unroll
-        for (int k = 0; k < KC; ++k) {
-          const int ch = threadIdx.x + k * 256;
-          if (q0 + u < parts && ch < n_chunks) Chunk4<DT>::load(dl + (q0 + u) * part_stride + ch * 4, d[u][k]);
-          else d[u][k][0] = d[u][k][1] = d[u][k][2] = d[u][k][3] = 0.0f;
-        }
+      if (q0 > 0) load_planes(q0);
 #pragma unroll
       for (int u = 0; u < PU; ++u) {
         if (q0 + u >= parts) break;
@@ -232,7 +238,15 @@ CW_EXPORT int cw_add_rmsnorm(float* resid, const void* delta0, const void* delta
   const int64_t part_stride = (int64_t)T_rows * H;
 #define CW_LAUNCH(T, WT, DT)                                                                           \
   do {                                                                                                 \
-    if (vec && H <= 4096)                                                                              \
+    if (vec && H <= 1024)                                                                              \
+      hipLaunchKernelGGL((add_rmsnorm_vec_kernel<T, WT, DT, 1>), grid, block, 0, stream, resid,        \
+                         (const T*)delta0, (const DT*)delta, parts, part_stride, (const WT*)weight, eps, \
+                         (T*)out, rows, H, (const WT*)weight2, (T*)out2);                                                            \
+    else if (vec && H <= 2048)                                                                         \
+      hipLaunchKernelGGL((add_rmsnorm_vec_kernel<T, WT, DT, 2>), grid, block, 0, stream, resid,        \
+                         (const T*)delta0, (const DT*)delta, parts, part_stride, (const WT*)weight, eps, \
+                         (T*)out, rows, H, (const WT*)weight2, (T*)out2);                                                            \
+    else if (vec && H <= 4096)                                                                         \
       hipLaunchKernelGGL((add_rmsnorm_vec_kernel<T, WT, DT, 4>), grid, block, 0, stream, resid,        \
                          (const T*)delta0, (const DT*)delta, parts, part_stride, (const WT*)weight, eps, \
                          (T*)out, rows, H, (const WT*)weight2, (T*)out2);                                                            \
