@@ -1059,6 +1059,27 @@ CW_EXPORT int cw_gemm_bf16_skinny_ksplits(int M, int N, int K) {
     if (s <= 1 || !plan_stream(3, M, N, K, s, &mt_, &spw, &grid, &n_tiles)) return 1;
     return s;
   }
+  // up to 16 rows: a long K; or an output so wide that its norm does not run inside the next product (that kernel
+  // takes a whole sum, and rows of up to 2048 elements)
+  if (K < 4096 && !(K > 2048 && N > 2048)) return 1;
+  // Among the counts that the streaming kernel takes: a wave's steps times the tiles of its workgroup are its time
+  // (steps as the kernel is built for; 16 of them come in fours, too few on their way: 15 % more), a part costs its
+  // way to memory and back. With the norm behind it, the count before and now (us, 8 rows): 7B shape's down product 38.4
+  // (5 parts) and 33.4 (8), output product 14.3 and 12.1; 14B shape's down 38.9 and 35.2; 32B shape's down 64.4 and 59.9.
+  int best = 0;
+  float least = 0.0f;
+  for (int s = 2; s <= 12 && K / s >= 1024; ++s) {
+    int mt, spw, n_tiles;
+    dim3 grid;
+    if (!plan_stream(3, M, N, K, s, &mt, &spw, &grid, &n_tiles)) continue;
+    const int per = (n_tiles + (int)grid.x - 1) / (int)grid.x;
+    const float t = (float)(per * spw) * (spw == 16 ? 1.15f : 1.0f) + 0.6f * (float)s * (float)N / 3584.0f;
+    if (best == 0 || t < least) {
+      least = t;
+      best = s;
+    }
+  }
+  if (best) return best;
   if (K < 4096) return 1;
   int s = 512 / tiles;  // about two workgroups per compute unit,
   if (s > 8) s = 8;
@@ -1067,14 +1088,6 @@ CW_EXPORT int cw_gemm_bf16_skinny_ksplits(int M, int N, int K) {
   if (s > 16) s = 16;
   while (s > 1 && K / s < 1024) --s;
   if (s < 1) s = 1;
-  // One split more if that is what brings the streaming kernel in (two tiles for every compute unit):
-  // it keeps x in registers and its next tile's weights in flight, which the one-tile kernel does not
-  // (the 1.5B shape's down product with the norm behind it: 13.2 us with 5 splits, 11.3 with 6).
-  int mt, spw, n_tiles;
-  dim3 grid;
-  if (s < 16 && K / (s + 1) >= 1024 && !plan_stream(3, M, N, K, s, &mt, &spw, &grid, &n_tiles) &&
-      plan_stream(3, M, N, K, s + 1, &mt, &spw, &grid, &n_tiles))
-    ++s;
   return s;
 }
 
