@@ -432,7 +432,7 @@ CW_EXPORT int cw_attention(int rows, int dtype, const void* q, int64_t q_stride,
 // bfloat16 decode attention: one query token per work item, keys and values streamed at memory
 // speed, all products on the matrix cores.
 //
-// A workgroup (4 waves) takes one (request, key/value head, split of the key range); its waves
+// A workgroup (4 or 8 waves) takes one (request, key/value head, split of the key range); its waves
 // take turns on tiles of 32 keys. Per tile:
 //   S^T[key, head] = K * Q^T        v_mfma_f32_16x16x32_bf16; the up to 16 heads of the group are
 //                                   the columns, so every key is fetched once for the whole group;
@@ -440,23 +440,36 @@ CW_EXPORT int cw_attention(int rows, int dtype, const void* q, int64_t q_stride,
 //   V^T from V: V times a 0/1 selector matrix comes back with keys in the lane's registers
 //                                   (the layout the next product needs), values bit-exact;
 //   O^T[d, head] += V^T * P^T       P^T is the softmax output as it lies in the registers.
-// K and V fragments are loaded from the pages straight into operand layout with 16-byte loads;
-// the next tile's loads are issued before the current tile is computed. Waves are merged through
+// K and V fragments are loaded from the pages with 16-byte loads, four neighbouring lanes 64 bytes of a key,
+// and swapped into operand layout by lane exchanges when they are used (ds_bpermute: the LDS unit's crossbar,
+// no memory). Loaded in operand layout, where neighbouring lanes hold different keys, each load is 64 requests to a
+// compute unit's load path instead of 16, and a tile of 32 keys of 128 elements takes that path a thousand cycles:
+// 2049 keys in one workgroup of four waves take 34 us so and 30 with the exchange, with eight waves 33 and 22.
+// The next tile's loads are issued before the current tile is computed. Waves are merged through
 // LDS at the end; splits are merged by a second, small kernel.
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
-#define DEC_WAVES 4
+// lane (c, s) takes what lane 4 c + s loaded: row c, slot s of 16 rows by four slots of 16 bytes
+typedef __attribute__((ext_vector_type(4))) int i32x4_t;
+__device__ __forceinline__ bf16x8_t dec_to_operand(const bf16x8_t& v, int lane) {
+  const int from = ((lane & 15) * 4 + (lane >> 4)) * 4;  // byte address of that lane
+  const i32x4_t q = __builtin_bit_cast(i32x4_t, v);
+  i32x4_t t;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) t[d] = __builtin_amdgcn_ds_bpermute(from, q[d]);
+  return __builtin_bit_cast(bf16x8_t, t);
+}
 
-template <int HD, bool POW2>
-__global__ __launch_bounds__(256) void attn_decode_bf16_kernel(AttnParams p) {
+template <int HD, bool POW2, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void attn_decode_bf16_kernel(AttnParams p) {
   constexpr int NF = HD / 32;  // 32-element steps over the head dimension
   constexpr int ND = HD / 16;  // 16-wide blocks of the head dimension
   extern __shared__ __align__(16) float dyn_s[];  // [waves][16 heads][HD] outputs, then this split's pages
   float* o_s = dyn_s;
-  int* tbl = reinterpret_cast<int*>(dyn_s + DEC_WAVES * 16 * HD);
-  __shared__ float M_s[DEC_WAVES][16];
-  __shared__ float L_s[DEC_WAVES][16];
+  int* tbl = reinterpret_cast<int*>(dyn_s + WAVES * 16 * HD);
+  __shared__ float M_s[WAVES][16];
+  __shared__ float L_s[WAVES][16];
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane & 15, s = lane >> 4;
@@ -486,7 +499,7 @@ __global__ __launch_bounds__(256) void attn_decode_bf16_kernel(AttnParams p) {
     const int k_last = min(k_first + p.split_keys, p.table_stride * bs) - 1;
     page0 = cw_page_index<POW2>(k_first, bs, sh);
     const int n_pages = k_last >= k_first ? cw_page_index<POW2>(k_last, bs, sh) - page0 + 1 : 0;
-    for (int i = threadIdx.x; i < n_pages; i += 256) tbl[i] = table[page0 + i];
+    for (int i = threadIdx.x; i < n_pages; i += WAVES * 64) tbl[i] = table[page0 + i];
   }
   const int pos = ctx - qlen + tok0;
   const int lo = p.window > 0 ? max(0, pos - p.window + 1) : 0;
@@ -504,7 +517,7 @@ __global__ __launch_bounds__(256) void attn_decode_bf16_kernel(AttnParams p) {
     page0 = cw_page_index<POW2>(t_begin * 32, bs, sh);
     const int last_key = min(pos, t_end * 32 - 1);
     const int n_pages = t_end > t_begin ? cw_page_index<POW2>(last_key, bs, sh) - page0 + 1 : 0;
-    for (int i = threadIdx.x; i < n_pages; i += 256) tbl[i] = table[page0 + i];
+    for (int i = threadIdx.x; i < n_pages; i += WAVES * 64) tbl[i] = table[page0 + i];
   }
   __syncthreads();
 
@@ -529,7 +542,7 @@ __global__ __launch_bounds__(256) void attn_decode_bf16_kernel(AttnParams p) {
   auto load_tile = [&](int t, bf16x8_t (*kf)[NF], bf16x8_t (*vf)[NF]) {
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
-      const int kp = t * 32 + kb * 16 + c;
+      const int kp = t * 32 + kb * 16 + (lane >> 2);
       const bool ok = t < t_end && kp >= lo && kp <= pos;
       const int page = tbl[ok ? cw_page_index<POW2>(kp, bs, sh) - page0 : 0];
       const bool have = ok && page >= 0;
@@ -537,9 +550,9 @@ __global__ __launch_bounds__(256) void attn_decode_bf16_kernel(AttnParams p) {
       const bf16_t* kr = have ? kc + off : zrow;
       const bf16_t* vr = have ? vc + off : zrow;
 #pragma unroll
-      for (int j = 0; j < NF; ++j) kf[kb][j] = *reinterpret_cast<const bf16x8_t*>(kr + (j * 4 + s) * 8);
+      for (int j = 0; j < NF; ++j) kf[kb][j] = *reinterpret_cast<const bf16x8_t*>(kr + (j * 4 + (lane & 3)) * 8);
 #pragma unroll
-      for (int j = 0; j < NF; ++j) vf[kb][j] = *reinterpret_cast<const bf16x8_t*>(vr + j * 32 + s * 8);
+      for (int j = 0; j < NF; ++j) vf[kb][j] = *reinterpret_cast<const bf16x8_t*>(vr + (j * 4 + (lane & 3)) * 8);
     }
   };
 
@@ -549,9 +562,9 @@ __global__ __launch_bounds__(256) void attn_decode_bf16_kernel(AttnParams p) {
   float m_run = -INFINITY, l_run = 0.0f;  // of head c, the same in all four lane groups
   bf16x8_t kf[2][NF], vf[2][NF], kf_n[2][NF], vf_n[2][NF];
   load_tile(t_begin + wave, kf, vf);
-  for (int t = t_begin + wave; t < t_end; t += DEC_WAVES) {
+  for (int t = t_begin + wave; t < t_end; t += WAVES) {
     const int kv0 = t * 32;
-    load_tile(t + DEC_WAVES, kf_n, vf_n);  // the wave's next tile is on its way meanwhile
+    load_tile(t + WAVES, kf_n, vf_n);  // the wave's next tile is on its way meanwhile
     // ---- S^T = K Q^T, keys 4s..4s+3 of each 16-key block for head c
     float sv[8];
     float tmax = -INFINITY;
@@ -559,7 +572,7 @@ __global__ __launch_bounds__(256) void attn_decode_bf16_kernel(AttnParams p) {
     for (int kb = 0; kb < 2; ++kb) {
       f32x4_t sc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int j = 0; j < NF; ++j) sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[kb][j], qf[j], sc, 0, 0, 0);
+      for (int j = 0; j < NF; ++j) sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dec_to_operand(kf[kb][j], lane), qf[j], sc, 0, 0, 0);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int kp = kv0 + kb * 16 + 4 * s + i;
@@ -599,8 +612,9 @@ __global__ __launch_bounds__(256) void attn_decode_bf16_kernel(AttnParams p) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
         const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
-        const f32x4_t tl = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[kb][j], sel_lo, zero, 0, 0, 0);
-        const f32x4_t th = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[kb][j], sel_hi, zero, 0, 0, 0);
+        const bf16x8_t vo = dec_to_operand(vf[kb][j], lane);
+        const f32x4_t tl = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vo, sel_lo, zero, 0, 0, 0);
+        const f32x4_t th = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vo, sel_hi, zero, 0, 0, 0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           vt_lo[kb * 4 + i] = (__bf16)tl[i];
@@ -625,16 +639,16 @@ __global__ __launch_bounds__(256) void attn_decode_bf16_kernel(AttnParams p) {
     *reinterpret_cast<f32x4_t*>(&o_s[(wave * 16 + c) * HD + db * 16 + 4 * s]) = o[db];
   __syncthreads();
   const int64_t base = ((int64_t)item * gridDim.y + blockIdx.y) * p.n_splits + split;
-  for (int idx = threadIdx.x; idx < gh * HD; idx += 256) {
+  for (int idx = threadIdx.x; idx < gh * HD; idx += WAVES * 64) {
     const int g = idx / HD, d = idx - g * HD;
     const int hg = chunk * gh + g;
     if (hg >= group) continue;
     float M = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < DEC_WAVES; ++w) M = fmaxf(M, M_s[w][g]);
+    for (int w = 0; w < WAVES; ++w) M = fmaxf(M, M_s[w][g]);
     float L = 0.0f, O = 0.0f;
 #pragma unroll
-    for (int w = 0; w < DEC_WAVES; ++w) {
+    for (int w = 0; w < WAVES; ++w) {
       const float mw = M_s[w][g];
       const float wgt = mw == -INFINITY ? 0.0f : __expf(mw - M);
       L = fmaf(L_s[w][g], wgt, L);
@@ -749,24 +763,24 @@ CW_EXPORT int64_t cw_attention_decode_workspace_floats(int n_items, int nh, int 
 }
 
 #if CW_HAS_DECODE
-template <bool POW2>
+template <bool POW2, int WAVES>
 static int launch_decode(AttnParams& p, int n_items, hipStream_t stream) {
   constexpr int HD = CW_HD;
   // keys of a split: at most ceil(tiles / splits) tiles of 32; their pages go to LDS
   const int64_t max_tiles = ((int64_t)p.table_stride * p.block_size + 31) / 32;
   const int64_t tiles_per_split = p.split_keys > 0 ? p.split_keys / 32 : (max_tiles + p.n_splits - 1) / p.n_splits;
   const int64_t pages = (tiles_per_split * 32 + p.block_size - 1) / p.block_size + 2;
-  const size_t smem = sizeof(float) * DEC_WAVES * 16 * HD + sizeof(int) * (size_t)pages;
+  const size_t smem = sizeof(float) * WAVES * 16 * HD + sizeof(int) * (size_t)pages;
   if (smem > 160 * 1024) return CW_ERR_SIZE;
   static size_t raised = 0;
   if (smem > raised) {
-    if (hipFuncSetAttribute((const void*)attn_decode_bf16_kernel<HD, POW2>,
+    if (hipFuncSetAttribute((const void*)attn_decode_bf16_kernel<HD, POW2, WAVES>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
       return CW_ERR_LAUNCH;
     raised = smem;
   }
-  dim3 grid(n_items, p.nkv * p.n_chunks, p.n_splits), block(256);
-  hipLaunchKernelGGL((attn_decode_bf16_kernel<HD, POW2>), grid, block, smem, stream, p);
+  dim3 grid(n_items, p.nkv * p.n_chunks, p.n_splits), block(WAVES * 64);
+  hipLaunchKernelGGL((attn_decode_bf16_kernel<HD, POW2, WAVES>), grid, block, smem, stream, p);
   if (p.n_splits > 1) {
     dim3 mgrid(n_items, p.nkv * p.n_chunks * p.gh);
     // thread groups that share the splits: about eight splits for each, as many as 1024 threads hold
@@ -822,7 +836,15 @@ CW_EXPORT int cw_attention_decode_bf16(const void* q, int64_t q_stride, void* ou
   p.part_o = workspace;
   p.part_ml = workspace ? workspace + need / (CW_HD + 2) * CW_HD : nullptr;
   p.zeros = zeros;
-  return p.bs_shift >= 0 ? launch_decode<true>(p, n_items, stream) : launch_decode<false>(p, n_items, stream);
+  // what a split's keys are shared among: the most keys a split may have, by the caller's fixed places or by its table
+  const int64_t keys = split_keys > 0 ? split_keys : ((int64_t)table_stride * block_size + n_splits - 1) / n_splits;
+  // more than four waves can have on their way at once: eight (2049 keys of 128 elements in one workgroup: 30 us
+  // with four waves, 22 with eight; larger heads have no registers for two tiles of eight waves), where their LDS leaves
+  // room for the pages (of a table of very many small ones)
+  if constexpr (CW_HD <= 128)
+    if (keys > 128 && sizeof(float) * 8 * 16 * CW_HD + sizeof(int) * ((keys + 63) / block_size + 3) <= 160 * 1024)
+      return p.bs_shift >= 0 ? launch_decode<true, 8>(p, n_items, stream) : launch_decode<false, 8>(p, n_items, stream);
+  return p.bs_shift >= 0 ? launch_decode<true, 4>(p, n_items, stream) : launch_decode<false, 4>(p, n_items, stream);
 #else
   return CW_ERR_ARG;
 #endif

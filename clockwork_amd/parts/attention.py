@@ -102,20 +102,28 @@ def _share_long_key_ranges(items: np.ndarray, ctx, workgroups_per_item: int):
     return out.astype(np.int32).reshape(-1), most
 
 
-def attention_plan(ctx, nh: int, nkv: int, narrow_ok: bool = False) -> AttentionPlan:
+def attention_plan(ctx, nh: int, nkv: int, narrow_ok: bool = False, whole_keys: int = 0) -> AttentionPlan:
     """The step's work items for heads of this geometry, made once a step and kept in
     ``ctx.plans``. ``narrow_ok``: the matrix-core kernel for portions also comes with two row
-    blocks a workgroup (see ``ops.prefill_row_blocks_ok``)."""
+    blocks a workgroup (see ``ops.prefill_row_blocks_ok``). ``whole_keys``: up to this many keys of a single
+    token stay with one workgroup (see ``whole_single_keys``)."""
     # a batch of single tokens has no portions: one plan, whatever the kernel for portions offers
     narrow_ok = bool(narrow_ok) and any(q > 1 for q in ctx.h_q_lens)
-    key = ("attention", nh, nkv, narrow_ok)
+    key = ("attention", nh, nkv, narrow_ok, whole_keys)
     plan = ctx.plans.get(key)
     if plan is None:
-        plan = ctx.plans[key] = _make_plan(ctx, nh, nkv, narrow_ok)
+        plan = ctx.plans[key] = _make_plan(ctx, nh, nkv, narrow_ok, whole_keys)
     return plan
 
 
-def _make_plan(ctx, nh: int, nkv: int, narrow_ok: bool) -> AttentionPlan:
+def whole_single_keys(head_dim: int) -> int:
+    """Heads of up to 128 elements come with eight waves a workgroup, which take 512 keys in two turns: as
+    long as the kernel that merges the parts of a request would take alone (us for one request, one part
+    against four: heads of 64, 120 keys 4.8 / 7.8, 500 keys 6.7 / 8.0; of 128, 6.3 / 9.5 and 9.7 / 9.5)."""
+    return 512 if head_dim <= 128 else 0
+
+
+def _make_plan(ctx, nh: int, nkv: int, narrow_ok: bool, whole_keys: int = 0) -> AttentionPlan:
     group = nh // nkv
     gh_wide = min(group, 64)
     tokens_per_tile = 64 // gh_wide
@@ -176,7 +184,8 @@ def _make_plan(ctx, nh: int, nkv: int, narrow_ok: bool) -> AttentionPlan:
         # 96 requests: 42.5 us with 1, 50.6 with 3). More than 64 splits never paid: one request
         # with 30000 keys takes 16 us with 64 to 128 splits and 19 us with 235.
         base = plan.n_single * nkv * -(-group // min(group, 16))
-        plan.decode_splits = max(1, min(ctx.num_compute_units // base, longest_single // 128, 64))
+        plan.decode_splits = 1 if longest_single <= whole_keys else max(
+            1, min(ctx.num_compute_units // base, longest_single // 128, 64))
         # fixed places for the splits: a workgroup then knows its pages before it knows the
         # request's length, which saves it a trip to memory
         plan.decode_split_keys = 32 * -(-(-(-longest_single // plan.decode_splits)) // 32)
@@ -220,7 +229,8 @@ class PagedAttention(Part):
     def _plan(self, ctx, dtype) -> AttentionPlan:
         hd = self.spec.head_dim
         narrow_ok = ops.prefill_attention_supported(hd, dtype) and ops.prefill_row_blocks_ok(hd, 2)
-        return attention_plan(ctx, self.spec.num_heads, self.spec.num_kv_heads, narrow_ok=narrow_ok)
+        return attention_plan(ctx, self.spec.num_heads, self.spec.num_kv_heads, narrow_ok=narrow_ok,
+                              whole_keys=whole_single_keys(hd))
 
     def prepare(self, ctx) -> None:
         """The step's work items, before ``forward`` (a captured step must not make them)."""

@@ -26,7 +26,7 @@ import torch
 
 from clockwork_amd import ops
 from clockwork_amd.config.spec import CacheNeeds, PagedRowsSpec, ParamSpec, StateSpec
-from clockwork_amd.parts.attention import attention_plan
+from clockwork_amd.parts.attention import attention_plan, whole_single_keys
 from clockwork_amd.parts.base import EntryCache, Part
 from clockwork_amd.parts.rope import rotary_frequencies
 from clockwork_amd.parts.sink_attention import longest_key_range, query_runs
@@ -135,7 +135,7 @@ class GatedAttention(Part):
     def _plan(self, ctx):
         if self.plain:
             hd = self.spec.key_dim
-            return attention_plan(ctx, self.spec.num_heads, self.spec.num_kv_heads, narrow_ok=ops.prefill_row_blocks_ok(hd, 2))
+            return attention_plan(ctx, self.spec.num_heads, self.spec.num_kv_heads, narrow_ok=ops.prefill_row_blocks_ok(hd, 2), whole_keys=whole_single_keys(hd))
         if not self.rows_mfma:
             return (*query_runs(ctx, self.run), 1)
         s = self.spec

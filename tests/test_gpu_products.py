@@ -147,3 +147,44 @@ def test_products_of_a_portion_by_their_rule():
             # the library's path rounds the product to bfloat16 before the gate: two roundings of up to 2^-8 each side
             torch.testing.assert_close(h, ref, rtol=4 * 2.0 ** -8, atol=2e-2)
     assert lib.cw_gemm_bf16_mid_choice(3, 144, 1536, 8960 + 32, 8992, 256) == 0   # K no whole number of stages
+
+
+# 16 requests at the edges of a wave's tile of 32 keys, of the turns of four and eight waves and of the line where
+# eight take over (128 keys a split); 24 keys a page and 16; a group of more than 16 heads
+@pytest.mark.parametrize("hd,nh,nkv,bs", [(32, 4, 2, 16), (64, 14, 2, 16), (96, 6, 3, 24), (128, 12, 2, 16), (128, 20, 1, 24), (160, 4, 2, 16)])
+@pytest.mark.parametrize("splits,fixed", [(1, True), (1, False), (2, True), (5, True), (5, False)])
+def test_decode_attention_at_the_turns_of_its_waves(hd, nh, nkv, bs, splits, fixed):
+    from clockwork_amd import ops
+
+    lens = [1, 2, 31, 32, 33, 127, 128, 129, 255, 256, 257, 511, 512, 513, 640, 700]
+    gen = torch.Generator().manual_seed(hd + splits)
+    width = -(-max(lens) // bs)
+    tables = torch.randperm(len(lens) * width, generator=gen).view(len(lens), width)
+    k, v = (torch.randn(len(lens) * width, bs, nkv, hd, generator=gen).bfloat16() for _ in range(2))
+    q = torch.randn(len(lens), nh * hd, generator=gen).bfloat16()
+    ws = None
+    if splits > 1:
+        ws = torch.full((ops.decode_attention_workspace_floats(hd, len(lens), nh, nkv, splits),), float("nan"), device=DEV)
+    out = torch.empty(len(lens), nh * hd, dtype=torch.bfloat16, device=DEV)
+    ints = lambda t: torch.as_tensor(t, dtype=torch.int32, device=DEV)  # noqa: E731
+    items = ints([x for r in range(len(lens)) for x in (r, 0, 1, 0)])
+    # what no request holds is poison: a key past a length that is counted shows
+    kd, vd = (t.clone() for t in (k, v))
+    for r, n in enumerate(lens):
+        for page in range(width):
+            kd[tables[r, page], max(0, min(bs, n - page * bs)):] = float("nan")
+            vd[tables[r, page], max(0, min(bs, n - page * bs)):] = float("nan")
+    extra = dict(identity=True, split_keys=32 * -(-(-(-max(lens) // splits)) // 32), max_ctx=max(lens)) if fixed else {}
+    ops.attention_decode(q=q.to(DEV), q_stride=nh * hd, out=out, k_cache=kd.to(DEV), v_cache=vd.to(DEV), block_tables=ints(tables),
+                         ctx_lens=ints(lens), cu_q=ints(range(len(lens) + 1)), items=items, n_items=len(lens), nh=nh, nkv=nkv,
+                         hd=hd, block_size=bs, n_splits=splits, window=0, scale=hd ** -0.5, workspace=ws,
+                         n_tokens=len(lens), n_requests=len(lens), **extra)
+    got = out.view(len(lens), nh, hd).double().cpu()
+    for r, n in enumerate(lens):
+        kr = k[tables[r]].reshape(-1, nkv, hd)[:n].double().repeat_interleave(nh // nkv, 1)
+        vr = v[tables[r]].reshape(-1, nkv, hd)[:n].double().repeat_interleave(nh // nkv, 1)
+        p = torch.softmax(torch.matmul(kr.transpose(0, 1), q[r].double().view(nh, hd, 1)).squeeze(-1) * hd ** -0.5, -1)
+        want = (p[..., None] * vr.transpose(0, 1)).sum(1)
+        # the probabilities and the result are rounded to bfloat16: half of 2^-8 of each term and of the sum
+        bound = 2.0 ** -8 * ((p[..., None] * vr.transpose(0, 1)).abs().sum(1) + want.abs()) + 1e-4
+        assert bool(((got[r] - want).abs() <= bound).all()), (r, n)
