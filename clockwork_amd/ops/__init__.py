@@ -781,9 +781,9 @@ def wide_swiglu_pays(M: int, two_i: int, K: int, ldx: int) -> bool:
     if tiles < WIDE_SWIGLU_MIN_TILES:
         return False
     units = _compute_units(torch.device("cuda", torch.cuda.current_device()))
-    # fewer than 512 rows that are no multiple of 64 are a step that runs as it came, not padded for a captured graph:
+    # fewer than 512 rows that are no multiple of 16 are a step that runs as it came, not padded for a captured graph:
     # the host's launches bound it, and the library serves its product
-    if M < WIDE_SWIGLU_MIN_ROWS // 2 and M % 64:
+    if M < WIDE_SWIGLU_MIN_ROWS // 2 and M % 16:
         return False
     return M >= WIDE_SWIGLU_MIN_ROWS or (two_i * K <= WIDE_SWIGLU_SMALL_WEIGHTS
                                          and tiles >= WIDE_SWIGLU_FILL * units * -(-tiles // units))
