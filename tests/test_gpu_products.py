@@ -188,3 +188,143 @@ def test_decode_attention_at_the_turns_of_its_waves(hd, nh, nkv, bs, splits, fix
         # the probabilities and the result are rounded to bfloat16: half of 2^-8 of each term and of the sum
         bound = 2.0 ** -8 * ((p[..., None] * vr.transpose(0, 1)).abs().sum(1) + want.abs()) + 1e-4
         assert bool(((got[r] - want).abs() <= bound).all()), (r, n)
+
+
+# rows of pieces of 4: one piece, a part of a wave, around 256 pieces, the most that registers hold and one more; no
+# multiple of 4 (the kernel of any length)
+@pytest.mark.parametrize("H", [4, 100, 1020, 1024, 1028, 1536, 2048, 2052, 4096, 4100, 1535])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_rows_in_pieces_of_four(H, dtype):
+    """Residual add + LayerNorm with each kind of pending branch, the mean of two RMS norms, the q / k norm with its
+    cache rows and the gated GELU, against float64."""
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(H)
+    rand = lambda *shape, dt=dtype: torch.randn(*shape, device=DEV, generator=gen).to(dt)  # noqa: E731
+    T, f64 = 5, torch.float64
+    # values of a few units: the result's own rounding, and float32 sums of H terms
+    tol = dict(atol=0.03, rtol=0.01) if dtype == torch.bfloat16 else dict(atol=2e-5, rtol=2e-5)
+    w, b, zb, x = rand(H), rand(H), rand(2 * H), rand(T, H, dt=torch.float32)
+    one, two, z = rand(T, H), rand(T, H), rand(T, 2 * H)
+    gates = torch.sigmoid(z.to(f64) + zb.to(f64))
+    for pending, extra in ((None, 0), ((None, None, one, None), one.to(f64)), ((z[:, :H].contiguous(), None, one, None), torch.sigmoid(z[:, :H].to(f64)) * one.to(f64)),
+                           ((z, zb, one, two), gates[:, :H] * one.to(f64) + gates[:, H:] * two.to(f64))):
+        total = x.to(f64) + extra
+        want = torch.nn.functional.layer_norm(total, (H,), w.to(f64), b.to(f64), 1e-5)
+        branches = None if pending is None else ops.GatedBranches(*pending)
+        pick = torch.tensor([4, 1], dtype=torch.int32, device=DEV)
+        resid = x.clone()
+        got = ops.add_layernorm(resid, branches, w, b, 1e-5, torch.empty(2, H, dtype=dtype, device=DEV), rows=pick)
+        torch.testing.assert_close(got.to(f64), want[[4, 1]], **tol)
+        assert torch.equal(resid, x)
+        got = ops.add_layernorm(resid, branches, w, b, 1e-5, torch.empty(T, H, dtype=dtype, device=DEV))
+        torch.testing.assert_close(got.to(f64), want, **tol)
+        torch.testing.assert_close(resid.to(f64), total, atol=1e-5, rtol=1e-5)
+    rms = lambda t, u: t.to(f64) * torch.rsqrt(t.to(f64).square().mean(-1, keepdim=True) + 1e-5) * u.to(f64)  # noqa: E731
+    u, v = rand(H), rand(H)
+    torch.testing.assert_close(ops.rms_mean2(one, two, u, v, 1e-5).to(f64), 0.5 * (rms(one, u) + rms(two, v)), **tol)
+    torch.testing.assert_close(ops.rms_mean2(one, None, u, None, 1e-5).to(f64), rms(one, u), **tol)
+    nk, nv = H // 12 * 4 + 4, H // 20 * 4 + 4
+    proj, uk = rand(T, H + nk + nv), rand(nk)
+    kc, vc = torch.zeros(9, nk, dtype=dtype, device=DEV), torch.zeros(9, nv, dtype=dtype, device=DEV)
+    before, slots = proj.clone(), torch.tensor([3, -1, 0, 8, 9], dtype=torch.int32, device=DEV)
+    ops.qk_rownorm_store(proj, 0, H, H + nk, H, nk, nv, u, uk, 1e-5, slots, kc, vc)
+    torch.testing.assert_close(proj[:, :H].to(f64), rms(before[:, :H], u), **tol)
+    assert torch.equal(proj[:, H:], before[:, H:])
+    for t, slot in ((0, 3), (2, 0), (3, 8)):
+        torch.testing.assert_close(kc[slot].to(f64), rms(before[t, H:H + nk], uk), **tol)
+        assert torch.equal(vc[slot], before[t, H + nk:])
+    assert not kc[[1, 2, 4, 5, 6, 7]].any() and not vc[[1, 2, 4, 5, 6, 7]].any()
+    gu = torch.cat([torch.tensor([-200.0, -9.0, 0.0, 30.0], device=DEV), rand(T * 2 * H - 4, dt=torch.float32) * 4]).view(T, 2 * H).to(dtype)
+    want = torch.nn.functional.gelu(gu[:, :H].to(f64), approximate="tanh") * gu[:, H:].to(f64)
+    torch.testing.assert_close(ops.gelu_tanh_mul(gu, torch.empty(T, H, dtype=dtype, device=DEV)).to(f64), want, **tol)
+
+
+# four columns a thread: 1 to 64 threads a row, rows that fill the last run and rows that do not, ranks in pieces of 4
+# and not; 24 columns: a column a thread
+@pytest.mark.parametrize("dim,vdim,rank", [(64, 128, 32), (40, 64, 16), (5, 4, 3), (128, 256, 20), (100, 32, 5), (1, 16, 1), (40, 24, 16)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_recurrence_of_few_tokens(dim, vdim, rank, dtype):
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(dim + vdim)
+    heads, lens, f64 = 3, [1, 17, 0, 2], torch.float64
+    T, width = sum(lens), 3 * (2 * dim + 2 * vdim) + rank
+    width += -width % 8
+    proj = (torch.randn(T, width, device=DEV, generator=gen) * 0.7).to(dtype)
+    a2 = (torch.randn(heads * dim, rank, device=DEV, generator=gen) * 0.5).to(dtype)
+    a2b, bonus = (torch.randn(heads * dim, device=DEV, generator=gen) for _ in range(2))
+    norm = torch.rand(vdim, device=DEV, generator=gen) + 0.5
+    start = torch.randn(6, heads, dim, vdim, device=DEV, generator=gen)
+    slots = torch.tensor([4, 0, 2, 5], dtype=torch.int32, device=DEV)
+    cu = torch.tensor([0, 1, 18, 18, 20], dtype=torch.int32, device=DEV)
+    offs = (0, heads * dim, 2 * heads * dim, 2 * heads * dim + heads * vdim, 2 * heads * dim + 2 * heads * vdim)
+    for with_bonus in (False, True):
+        state = start.clone()
+        got = ops.linear_recurrence(proj, *offs, a2, a2b, norm, state, slots, cu, 4, heads, dim, vdim, dim ** -0.5, 16.0, 1e-5,
+                                    bonus=bonus if with_bonus else None)
+        cols = lambda at, n: proj[:, at:at + heads * n].to(f64).view(T, heads, n)  # noqa: E731
+        q, k, v, g = cols(offs[0], dim) * dim ** -0.5, cols(offs[1], dim), cols(offs[2], vdim), cols(offs[3], vdim)
+        z = proj[:, offs[4]:offs[4] + rank].to(f64) @ a2.to(f64).t() + a2b.to(f64)
+        decay = torch.sigmoid(z).pow(1 / 16.0).view(T, heads, dim)
+        want, at = torch.zeros(T, heads, vdim, dtype=f64, device=DEV), 0
+        after = start.to(f64)
+        for r, n in enumerate(lens):
+            for t in range(at, at + n):
+                S, kv = after[int(slots[r])], k[t, :, :, None] * v[t, :, None, :]
+                if with_bonus:
+                    want[t] = (q[t, :, :, None] * (S + bonus.to(f64).view(heads, dim, 1) * kv)).sum(1)
+                S = decay[t, :, :, None] * S + kv
+                if not with_bonus:
+                    want[t] = (q[t, :, :, None] * S).sum(1)
+                after[int(slots[r])] = S
+            at += n
+        want = want * torch.rsqrt(want.square().mean(-1, keepdim=True) + 1e-5) * norm.to(f64) * torch.nn.functional.silu(g)
+        # 17 steps and sums of up to 128 float32 terms; the result's own rounding
+        tol = dict(atol=0.02, rtol=0.01) if dtype == torch.bfloat16 else dict(atol=1e-4, rtol=1e-4)
+        torch.testing.assert_close(got.to(f64).view(T, heads, vdim), want, **tol)
+        torch.testing.assert_close(state.to(f64), after, atol=1e-4, rtol=1e-4)
+
+
+# runs of 32, 50 and 128 keys; mixed heads over one, two (two kernels) and three key/value heads (three kernels), no
+# mixing over four; sizes that are read in pieces and one by one, more columns than threads, groups of more than 16 heads
+@pytest.mark.parametrize("heads,kv,dim,vdim,talk", [(12, 2, 128, 128, True), (6, 2, 20, 24, True), (3, 1, 40, 24, True), (6, 3, 64, 64, True),
+                                                    (8, 4, 64, 96, False), (20, 1, 32, 300, True), (4, 4, 16, 16, False)])
+@pytest.mark.parametrize("sk", [32, 50, 128])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_sink_decode_runs(heads, kv, dim, vdim, talk, sk, dtype):
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(heads * sk)
+    rand = lambda *shape, dt=dtype: torch.randn(*shape, device=DEV, generator=gen).to(dt)  # noqa: E731
+    lens, window, bs, f64 = [1, 31, 32, 33, 200, 333, 700], 300, 16, torch.float64
+    R, pages = len(lens), -(-max(lens) // bs)
+    tables = torch.randperm(R * pages, device=DEV, generator=gen).view(R, pages).int()
+    kc, vc = rand(R * pages, bs, kv, dim), rand(R * pages, bs, kv, vdim)
+    stride = heads * dim + 8
+    q = rand(R, stride)
+    r1, r2, sink = (torch.rand(heads, device=DEV, generator=gen) for _ in range(3))
+    mix = torch.eye(heads, device=DEV) + 0.2 * rand(heads, heads, dt=torch.float32) if talk else None
+    out = torch.full((R, heads * vdim), float("nan"), device=DEV).to(dtype)
+    ints = lambda t: torch.as_tensor(t, dtype=torch.int32, device=DEV)  # noqa: E731
+    kd, vd = kc.clone(), vc.clone()
+    for r, n in enumerate(lens):  # what no request holds is poison
+        for page in range(pages):
+            kd[tables[r, page], max(0, min(bs, n - page * bs)):] = float("nan")
+            vd[tables[r, page], max(0, min(bs, n - page * bs)):] = float("nan")
+    ops.sink_attention_decode(q, stride, out, kd, vd, tables, ints(lens), ints(range(R + 1)), R, sk, -(-window // sk), r1, r2, sink, mix,
+                              heads, kv, dim, vdim, bs, window, dim ** -0.5)
+    for r, n in enumerate(lens):
+        lo = max(0, n - window)
+        keys = kc[tables[r].long()].reshape(-1, kv, dim)[lo:n].to(f64).repeat_interleave(heads // kv, 1)
+        values = vc[tables[r].long()].reshape(-1, kv, vdim)[lo:n].to(f64).repeat_interleave(heads // kv, 1)
+        scores = (q[r, : heads * dim].to(f64).view(heads, 1, dim) * keys.transpose(0, 1)).sum(-1) * dim ** -0.5
+        away = n - 1 - torch.arange(lo, n, device=DEV, dtype=f64)
+        scores = scores - r1.to(f64)[:, None] * torch.log1p(r2.to(f64)[:, None] * away)
+        p = torch.softmax(torch.cat([scores, sink.to(f64)[:, None]], 1), 1)[:, :-1]
+        if talk:
+            p = mix.to(f64) @ p
+        want = (p[:, :, None] * values.transpose(0, 1)).sum(1).view(-1)
+        # float32 sums of up to 300 terms of a few units; bfloat16: the result's own rounding
+        tol = dict(atol=0.005, rtol=0.005) if dtype == torch.bfloat16 else dict(atol=2e-5, rtol=2e-5)
+        torch.testing.assert_close(out[r].to(f64), want, **tol)
