@@ -309,15 +309,15 @@ __device__ __forceinline__ bool sd_range(const SinkDecodeParams& p, int r, int& 
 template <typename T> struct RowVec;
 template <> struct RowVec<float> {
   static constexpr int N = 4;
-  __device__ static void load(const float* p, float* o) {
-    const float4 v = *reinterpret_cast<const float4*>(p);
-    o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
+  __device__ static void load(const float* p, float* o) { unpack(*reinterpret_cast<const uint4*>(p), o); }
+  __device__ static void unpack(uint4 v, float* o) {
+    o[0] = __uint_as_float(v.x); o[1] = __uint_as_float(v.y); o[2] = __uint_as_float(v.z); o[3] = __uint_as_float(v.w);
   }
 };
 template <> struct RowVec<bf16_t> {
   static constexpr int N = 8;
-  __device__ static void load(const bf16_t* p, float* o) {
-    const uint4 v = *reinterpret_cast<const uint4*>(p);
+  __device__ static void load(const bf16_t* p, float* o) { unpack(*reinterpret_cast<const uint4*>(p), o); }
+  __device__ static void unpack(uint4 v, float* o) {
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int i = 0; i < 4; ++i) { o[2 * i] = __uint_as_float(w[i] << 16); o[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u); }
@@ -548,8 +548,290 @@ __global__ __launch_bounds__(256) void sink_decode_merge_kernel(SinkDecodeParams
   }
 }
 
+// ======================================================================================
+// The same in two kernels. Mixing across heads is linear, so a run's values can be multiplied with every head's own
+// exponentials before anything is known of the other runs: the merge then scales them, adds the runs and mixes.
+//
+//   runs:   scores as above; a head's exponentials against its own maximum over the run stay in LDS and meet the
+//           run's values: of all key/value heads where heads are mixed, else of the head's own;
+//   merge:  out[h] = sum over g of talk[h, g] sum over runs of exp(m[run, g] - M[g]) / L[g] * part[run, g, group of h].
+//
+// Both are bound by their trips to memory one after another (lengths, pages, keys and values; then lengths, statistics,
+// partial sums): a run's keys and values are asked for together, and no workgroup waits for another's statistics within
+// a kernel. 8 requests of 200 keys, 12 heads of 128 over 2: 32.0 us in three kernels, 19.5 in two.
+// With mixing it multiplies kv_heads times the values, hence SD_MIXED_GROUPS.
+// ======================================================================================
+#define SD_MIXED_GROUPS 2
+#define SD_COEF_FLOATS 16384   // heads * runs that the merge holds in LDS
+
+// HS, HV: heads a thread takes at a time with a key and with a value (of a group; of all, where they are mixed). What
+// fills the last turn up repeats its last head: a test for each head would wait for each one's LDS read by itself.
+template <typename T, int HS, int HV>
+__global__ __launch_bounds__(256) void sink_decode_runs_kernel(SinkDecodeParams p) {
+  extern __shared__ __align__(16) float smem[];
+  const int H = p.heads, G = p.kv_heads, D = p.dim, V = p.vdim, Hg = H / G, SK = p.sk, SP = (SK + 3) & ~3;
+  const int r = blockIdx.x, run = blockIdx.y, tid = threadIdx.x;
+  int lo, pos;
+  if (!sd_range(p, r, lo, pos)) return;
+  const int k0 = lo + run * SK;
+  if (k0 > pos) return;
+  const int nk = min(SK, pos - k0 + 1);
+  float* qs = smem;                  // [H * D], padded to a multiple of 4
+  float* sc = qs + ((H * D + 3) & ~3);  // [H][SP] scores, then exponentials
+  int* rows = (int*)(sc + H * SP);   // [SR] cache rows of the run's keys (-1: none)
+  const int SR = (SK + 31) & ~31;
+  float* rs = (float*)(rows + SR);   // [2][H] distance bias
+  const T* q = (const T*)p.q + (int64_t)p.cu_q[r] * p.q_stride;
+  const int* table = p.block_tables + (int64_t)r * p.table_width;
+  for (int jj = tid; jj < SR; jj += 256) {
+    int row = -1;
+    if (jj < nk) {
+      const int page = table[(k0 + jj) / p.block_size];
+      const int64_t at = (int64_t)page * p.block_size + (k0 + jj) % p.block_size;
+      if (page >= 0 && at < p.cache_rows) row = (int)at;
+    }
+    rows[jj] = row;
+  }
+  for (int i = tid; i < H * D; i += 256) qs[i] = cw_to_float(q[i]);
+  if (p.r1 && tid < H) { rs[tid] = p.r1[tid]; rs[H + tid] = p.r2[tid]; }
+  for (int i = tid; i < H * (SP - SK); i += 256) sc[i / (SP - SK) * SP + SK + i % (SP - SK)] = 0.0f;
+  cw_lds_barrier();
+
+  const T* kc = (const T*)p.k_cache;
+  const T* vc = (const T*)p.v_cache;
+  constexpr int N = RowVec<T>::N;
+  const bool vec = D % N == 0 && !((uintptr_t)kc & 15);
+  int tpk = 1;
+  while (vec && tpk < 8 && SK * G * tpk * 2 <= 256 && D % (tpk * 2 * N) == 0) tpk *= 2;
+  const int dpt = D / tpk;
+  // a thread's first four pieces of a key and its first 32 values; a row that is not there reads row 0 and is dropped
+  uint4 key[4];
+  if (vec && tid < SK * G * tpk) {
+    const int piece = tid % tpk, c = tid / tpk / SK, jj = tid / tpk - c * SK;
+    const T* krow = kc + ((int64_t)max(rows[jj], 0) * G + c) * D + piece * dpt;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      if (b * N < dpt) key[b] = *reinterpret_cast<const uint4*>(krow + b * N);
+  }
+  T val[32];
+  // which of the run's (at most 128) keys have a row: the same bits in every lane
+  const int l64 = tid & 63;
+  const uint64_t low = __ballot(l64 < SR && rows[l64] >= 0), high = __ballot(l64 + 64 < SR && rows[l64 + 64] >= 0);
+  uint32_t there = 0;
+  const int64_t vrow = (int64_t)G * V;
+  auto load_values = [&](int idx, int j0) __attribute__((always_inline)) {
+    there = (uint32_t)((j0 < 64 ? low : high) >> (j0 & 63));
+    const T* col = vc + idx;  // [row][kv head][vdim]: a thread's column is its number
+#pragma unroll
+    for (int u0 = 0; u0 < 32; u0 += 4) {
+      const int4 at = *reinterpret_cast<const int4*>(rows + j0 + u0);
+      val[u0] = col[max(at.x, 0) * vrow];
+      val[u0 + 1] = col[max(at.y, 0) * vrow];
+      val[u0 + 2] = col[max(at.z, 0) * vrow];
+      val[u0 + 3] = col[max(at.w, 0) * vrow];
+    }
+  };
+  if (tid < G * V) load_values(tid, 0);
+  for (int idx0 = tid; idx0 < SK * G * tpk; idx0 += 256) {
+    const int idx = idx0 / tpk, piece = idx0 - idx * tpk;
+    const int c = idx / SK, jj = idx - c * SK;
+    const T* krow = kc + ((int64_t)max(rows[jj], 0) * G + c) * D;
+    for (int h0 = 0; h0 < Hg; h0 += HS) {
+      float acc[HS];
+#pragma unroll
+      for (int e = 0; e < HS; ++e) acc[e] = 0.0f;
+      if (vec) {
+        const int d_end = (piece + 1) * dpt;
+        for (int d0 = piece * dpt; d0 < d_end; d0 += 4 * N) {
+          if (idx0 != tid || h0 || d0 != piece * dpt) {
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+              if (d0 + b * N < d_end) key[b] = *reinterpret_cast<const uint4*>(krow + d0 + b * N);
+          }
+#pragma unroll
+          for (int b = 0; b < 4; ++b) {
+            if (d0 + b * N < d_end) {
+              float kv[N];
+              RowVec<T>::unpack(key[b], kv);
+#pragma unroll
+              for (int e = 0; e < HS; ++e) {
+                const float* qv = qs + (c * Hg + min(h0 + e, Hg - 1)) * D + d0 + b * N;
+#pragma unroll
+                for (int u = 0; u < N; u += 4) {
+                  const float4 q4 = *reinterpret_cast<const float4*>(qv + u);
+                  acc[e] += q4.x * kv[u] + q4.y * kv[u + 1] + q4.z * kv[u + 2] + q4.w * kv[u + 3];
+                }
+              }
+            }
+          }
+        }
+      } else {
+        for (int d = piece * dpt; d < (piece + 1) * dpt; ++d) {
+          const float kv = cw_to_float(krow[d]);
+#pragma unroll
+          for (int e = 0; e < HS; ++e) acc[e] += qs[(c * Hg + min(h0 + e, Hg - 1)) * D + d] * kv;
+        }
+      }
+      for (int off = 1; off < tpk; off <<= 1) {
+#pragma unroll
+        for (int e = 0; e < HS; ++e) acc[e] += __shfl_xor(acc[e], off, 64);
+      }
+#pragma unroll
+      for (int e = 0; e < HS; ++e) {
+        if (h0 + e < Hg && piece == 0) sc[(c * Hg + h0 + e) * SP + jj] = acc[e];
+      }
+    }
+  }
+  cw_lds_barrier();
+  // scale, distance bias and the run's statistics: a wave takes four heads at a time, whose exchanges run side by
+  // side, a lane up to two of the (at most 128) keys
+  for (int g0 = tid >> 6; g0 < H; g0 += 16) {
+    const int lane = tid & 63;
+    float sv[4][2], m[4], l[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int g = min(g0 + 4 * i, H - 1);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int jj = lane + 64 * u;
+        sv[i][u] = -INFINITY;
+        if (jj < nk) {
+          sv[i][u] = rows[jj] >= 0 ? sc[g * SP + jj] * p.scale : 0.0f;
+          if (p.r1) sv[i][u] -= rs[g] * log1pf(rs[H + g] * (float)(pos - k0 - jj));
+        }
+      }
+      m[i] = fmaxf(sv[i][0], sv[i][1]);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) m[i] = fmaxf(m[i], __shfl_xor(m[i], off, 64));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      sv[i][0] = expf(sv[i][0] - m[i]);
+      sv[i][1] = expf(sv[i][1] - m[i]);
+      l[i] = sv[i][0] + sv[i][1];
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) l[i] += __shfl_xor(l[i], off, 64);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int g = g0 + 4 * i;
+      if (g >= H) break;
+      if (lane < SK) sc[g * SP + lane] = sv[i][0];
+      if (lane + 64 < SK) sc[g * SP + lane + 64] = sv[i][1];
+      if (lane == 0) *reinterpret_cast<float2*>(p.stats + (((int64_t)r * p.n_runs + run) * H + g) * 2) = make_float2(m[i], l[i]);
+    }
+  }
+  cw_lds_barrier();
+  const bool mixed = p.talk != nullptr;
+  const int CX = mixed ? G : 1, heads = mixed ? H : Hg;
+  float* part = p.partial + ((int64_t)r * p.n_runs + run) * ((int64_t)H * CX * V);
+  for (int idx = tid; idx < G * V; idx += 256) {
+    const int c = idx / V, dv = idx - c * V, first = mixed ? 0 : c * Hg;
+    for (int h0 = 0; h0 < heads; h0 += HV) {
+      float acc[HV];
+#pragma unroll
+      for (int e = 0; e < HV; ++e) acc[e] = 0.0f;
+      for (int j0 = 0; j0 < nk; j0 += 32) {
+        if (idx != tid || h0 || j0) load_values(idx, j0);
+#pragma unroll
+        for (int u0 = 0; u0 < 32; u0 += 4) {
+          if (j0 + u0 < nk) {
+            float v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = there >> (u0 + u) & 1 ? cw_to_float(val[u0 + u]) : 0.0f;
+#pragma unroll
+            for (int e = 0; e < HV; ++e) {
+              const float4 w = *reinterpret_cast<const float4*>(sc + (first + min(h0 + e, heads - 1)) * SP + j0 + u0);
+              acc[e] += w.x * v[0] + w.y * v[1] + w.z * v[2] + w.w * v[3];
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < HV; ++e)
+        if (h0 + e < heads) part[((int64_t)(first + h0 + e) * CX + (mixed ? c : 0)) * V + dv] = acc[e];
+    }
+  }
+}
+
+// grid: request, key/value head (mixed) or 1, 64 value columns; a wave per head, up to 16 waves
+template <typename T>
+__global__ __launch_bounds__(1024) void sink_decode_mix_kernel(SinkDecodeParams p) {
+  extern __shared__ __align__(16) float smem[];
+  const int H = p.heads, V = p.vdim, r = blockIdx.x, c = blockIdx.y, lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6, waves = blockDim.x >> 6, dv = blockIdx.z * 64 + lane;
+  int lo, pos;
+  if (!sd_range(p, r, lo, pos)) return;
+  const int runs = (pos - lo) / p.sk + 1;
+  const bool mixed = p.talk != nullptr;
+  const int CX = mixed ? p.kv_heads : 1, Hg = mixed ? H / p.kv_heads : H;
+  float* coef = smem;               // [H][n_runs]
+  float* X = coef + H * p.n_runs;   // [H][64]
+  float* tk = X + H * 64;           // [Hg][H] the mixing matrix' rows of this group
+  if (mixed)
+    for (int i = threadIdx.x; i < Hg * H; i += blockDim.x) tk[i] = p.talk[c * Hg * H + i];
+  const float2* st = reinterpret_cast<const float2*>(p.stats) + (int64_t)r * p.n_runs * H;
+  const float* part = p.partial + (int64_t)r * p.n_runs * ((int64_t)H * CX * V) + c * V + min(dv, V - 1);
+  const int64_t step = (int64_t)H * CX * V;
+  for (int g = wave; g < H; g += waves) {
+    const float sink = p.sink ? p.sink[g] : -INFINITY;
+    const float* pg = part + (int64_t)g * CX * V;
+    // the first eight runs' parts are on their way while the statistics meet
+    float x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = u < runs ? pg[u * step] : 0.0f;
+    float m = sink;
+    for (int s = lane; s < runs; s += 64) m = fmaxf(m, st[s * H + g].x);
+    m = cw_wave_max(m);
+    float l = 0.0f;
+    for (int s = lane; s < runs; s += 64) {
+      const float2 ml = st[s * H + g];
+      const float w = expf(ml.x - m);
+      coef[g * p.n_runs + s] = w;
+      l += ml.y * w;
+    }
+    l = cw_wave_sum(l);
+    if (p.sink) l += expf(sink - m);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    float sum = 0.0f;
+    for (int s0 = 0; s0 < runs; s0 += 8) {
+      if (s0) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = s0 + u < runs ? pg[(s0 + u) * step] : 0.0f;
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (s0 + u < runs) sum += coef[g * p.n_runs + s0 + u] * x[u];
+    }
+    X[g * 64 + lane] = l > 0.0f ? sum * (1.0f / l) : 0.0f;
+  }
+  __syncthreads();
+  T* out = (T*)p.out + (int64_t)p.cu_q[r] * H * V + dv;
+  for (int hh = wave; hh < Hg; hh += waves) {
+    const int h = c * Hg + hh;
+    float v = 0.0f;
+    if (mixed)
+      for (int g = 0; g < H; ++g) v += tk[hh * H + g] * X[g * 64 + lane];
+    else
+      v = X[h * 64 + lane];
+    if (dv < V) out[h * V] = cw_from_float<T>(v);
+  }
+}
+
+// Do two kernels serve it?
+static bool sd_two(int n_runs, int heads, int kv_heads, bool mixed) {
+  return (!mixed || kv_heads <= SD_MIXED_GROUPS) && heads <= 64 && (int64_t)heads * n_runs <= SD_COEF_FLOATS;
+}
+
 // floats of workspace for R single tokens whose keys are cut into n_runs runs of sk keys
-CW_EXPORT int64_t cw_sink_decode_workspace_floats(int n_requests, int n_runs, int sk, int heads, int vdim) {
+CW_EXPORT int64_t cw_sink_decode_workspace_floats(int n_requests, int n_runs, int sk, int heads, int kv_heads, int vdim,
+                                                  int mixed) {
+  if (kv_heads > 0 && sd_two(n_runs, heads, kv_heads, mixed != 0))
+    return (int64_t)n_requests * n_runs * heads * (2 + (int64_t)(mixed ? kv_heads : 1) * vdim);
   return (int64_t)n_requests * heads * n_runs * sk + (int64_t)n_requests * n_runs * heads * 2 +
          (int64_t)n_requests * n_runs * heads * vdim;
 }
@@ -580,14 +862,49 @@ CW_EXPORT int cw_sink_decode(int dtype, const void* q, int64_t q_stride, void* o
   p.q = q; p.q_stride = q_stride; p.out = out; p.k_cache = k_cache; p.v_cache = v_cache;
   p.block_tables = block_tables; p.table_width = table_width; p.ctx_lens = ctx_lens; p.cu_q = cu_q;
   p.r1 = r1; p.r2 = r2; p.sink = sink; p.talk = talk;
+  const bool two = sd_two(n_runs, heads, kv_heads, talk != nullptr) && !((uintptr_t)workspace & 7);
   p.scores = workspace;
-  p.stats = p.scores + (int64_t)n_requests * heads * n_runs * sk;
+  p.stats = two ? workspace : p.scores + (int64_t)n_requests * heads * n_runs * sk;
   p.partial = p.stats + (int64_t)n_requests * n_runs * heads * 2;
   p.heads = heads; p.kv_heads = kv_heads; p.dim = dim; p.vdim = vdim; p.block_size = block_size; p.window = window;
   p.sk = sk; p.n_runs = n_runs; p.scale = scale; p.cache_rows = cache_rows;
   const size_t smem1 = ((size_t)heads * dim + (size_t)heads * sk) * sizeof(float);
   const size_t smem2 = (2 * (size_t)heads * sk + 2 * heads + sk + (size_t)heads * heads) * sizeof(float);
   const dim3 grid(n_requests, n_runs), block(256);
+  if (two) {
+    const int sp = (sk + 3) & ~3;
+    const size_t lds = ((((size_t)heads * dim + 3) & ~(size_t)3) + (size_t)heads * sp + 2 * heads + sk + 31) * sizeof(float);
+    const int group = talk ? heads / kv_heads : heads;
+    const size_t mlds = ((size_t)heads * n_runs + (size_t)heads * 64 + (size_t)group * heads) * sizeof(float);
+    const dim3 mgrid(n_requests, talk ? kv_heads : 1, (vdim + 63) / 64), mblock(64 * (heads < 16 ? heads : 16));
+    // heads a thread takes at a time: a whole group and all mixed heads in one turn, for up to 16
+    const int hg = heads / kv_heads, hv = talk ? heads : hg;
+#define CW_TWO(T_, HS_, HV_)                                                                                           \
+  do {                                                                                                                 \
+    if (lds > 48 * 1024 && hipFuncSetAttribute((const void*)sink_decode_runs_kernel<T_, HS_, HV_>,                     \
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)    \
+      return CW_ERR_LAUNCH;                                                                                            \
+    if (mlds > 48 * 1024 && hipFuncSetAttribute((const void*)sink_decode_mix_kernel<T_>,                               \
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)mlds) != hipSuccess)  \
+      return CW_ERR_LAUNCH;                                                                                            \
+    hipLaunchKernelGGL((sink_decode_runs_kernel<T_, HS_, HV_>), grid, block, lds, stream, p);                          \
+    hipLaunchKernelGGL((sink_decode_mix_kernel<T_>), mgrid, mblock, mlds, stream, p);                                  \
+    return cw_launch_status();                                                                                         \
+  } while (0)
+#define CW_TWO_BY_HEADS(T_)                                        \
+  do {                                                             \
+    if (hg <= 4 && hv <= 4) CW_TWO(T_, 4, 4);                      \
+    if (hg <= 4) CW_TWO(T_, 4, 8);                                 \
+    if (hg <= 8 && hv <= 8) CW_TWO(T_, 8, 8);                      \
+    if (hg <= 8) CW_TWO(T_, 8, 16);                                \
+    CW_TWO(T_, 16, 16);                                            \
+  } while (0)
+    if (dtype == CW_F32) CW_TWO_BY_HEADS(float);
+    if (dtype == CW_BF16) CW_TWO_BY_HEADS(bf16_t);
+    return CW_ERR_DTYPE;
+#undef CW_TWO_BY_HEADS
+#undef CW_TWO
+  }
   int my = (heads * vdim + 255) / 256;
   if (my > 64) my = 64;
 #define CW_LAUNCH(T_)                                                                                                  \

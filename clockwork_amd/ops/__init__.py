@@ -210,7 +210,7 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
         "sink_attention": {
             "cw_sink_attention_max_bq": [I, I, I, I],
             "cw_sink_attention": [I, P, L, P, P, P, L, P, I, P, P, P, I, I, P, P, P, P, I, I, I, I, I, I, F, P],
-            "cw_sink_decode_workspace_floats": [I, I, I, I, I],
+            "cw_sink_decode_workspace_floats": [I, I, I, I, I, I, I],
             "cw_sink_prefill_mfma_supported": [I, I, I, I],
             "cw_sink_prefill_mfma": [P, L, P, P, P, L, P, I, P, P, P, I, P, P, P, P, I, I, I, I, I, I, F, I, P],
             "cw_sink_decode_supported": [I, I, I, I],
@@ -1758,7 +1758,7 @@ def sink_attention_decode(q, q_stride: int, out, k_cache, v_cache, block_tables,
                           block_size: int, window: int, scale: float) -> None:
     """``sink_attention`` for the step's requests of one token each (others are left alone): the
     keys a token sees are cut into ``n_runs`` runs of ``run_keys`` keys (the most any request of
-    the step has), a workgroup each; three kernels (scores and their sums, values, merge)."""
+    the step has), a workgroup each; the runs are merged by a kernel of its own."""
     _gpu(q, out, k_cache, v_cache, block_tables, ctx_lens, cu_q, r1, r2, sink, talk)
     T = q.shape[0]
     _need(q.dim() == 2 and q.shape[1] == q_stride and heads * dim <= q_stride, "q must be [T, q_stride] with the query heads first")
@@ -1776,7 +1776,7 @@ def sink_attention_decode(q, q_stride: int, out, k_cache, v_cache, block_tables,
     _need((r1 is None) == (r2 is None), "the distance bias takes r1 and r2 together")
     _need(1 <= run_keys <= SINK_DECODE_MAX_RUN and n_runs >= 1, "runs of 1 to 128 keys, at least one")
     lib = _load("sink_attention")
-    need = lib.cw_sink_decode_workspace_floats(n_requests, n_runs, run_keys, heads, vdim)
+    need = lib.cw_sink_decode_workspace_floats(n_requests, n_runs, run_keys, heads, kv_heads, vdim, int(talk is not None))
     workspace = torch.empty(max(int(need), 1), dtype=torch.float32, device=q.device)
     _check(lib.cw_sink_decode(
         dtype_code(q.dtype), _ptr(q), q_stride, _ptr(out), _ptr(k_cache), _ptr(v_cache), rows, _ptr(block_tables),
