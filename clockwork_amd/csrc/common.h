@@ -63,15 +63,18 @@ __device__ __forceinline__ float cw_clipped_glu(float gate, float up, float limi
   const float g = fminf(gate, limit), u = fminf(fmaxf(up, -limit), limit);
   return g / (1.0f + expf(-1.702f * g)) * (u + 1.0f);
 }
-// What the kernels of gate/up products make of a gate and an up value: ``act`` > 0 the clipped gated
-// activation of that limit, < 0 max(gate, 0) * up, else silu(gate) * up.
-__device__ __forceinline__ float cw_gated(float g, float u, float act) {
-  return act > 0.0f ? cw_clipped_glu(g, u, act) : act < 0.0f ? fmaxf(g, 0.0f) * u : g / (1.0f + expf(-g)) * u;
-}
 // The tanh form of GELU, 0.5 z (1 + tanh(y)) with y = sqrt(2 / pi) (z + 0.044715 z^3), through
 // 0.5 (1 + tanh(y)) = 1 / (1 + exp(-2 y)).
 __device__ __forceinline__ float cw_gelu_tanh(float z) {
   return z / (1.0f + expf(-1.5957691216057308f * (z + 0.044715f * z * z * z)));
+}
+// What the kernels of gate/up products make of a gate and an up value: ``act`` > 0 the clipped gated
+// activation of that limit, -1 max(gate, 0) * up, -2 gelu_tanh(gate) * up, 0 silu(gate) * up.
+__device__ __forceinline__ float cw_gated_below(float g, float u, float act) {
+  return (act < -1.5f ? cw_gelu_tanh(g) : fmaxf(g, 0.0f)) * u;
+}
+__device__ __forceinline__ float cw_gated(float g, float u, float act) {
+  return act > 0.0f ? cw_clipped_glu(g, u, act) : act < 0.0f ? cw_gated_below(g, u, act) : g / (1.0f + expf(-g)) * u;
 }
 
 // Functions from the bare exp2, log2 and reciprocal instructions: a few units in the last place, and a

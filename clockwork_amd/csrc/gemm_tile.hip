@@ -48,7 +48,7 @@ struct TileArgs {
   void* C;
   int64_t ldc;
   int M, N, K;
-  float act;          // MODE 2: > 0: the clipped gated activation with this limit, < 0: max(gate, 0) * up
+  float act;          // MODE 2: > 0: the clipped gated activation with this limit, -1: max(gate, 0) * up, -2: gelu_tanh(gate) * up
 };
 
 // Row of W that row ``rb`` (0..127) of the workgroup's W tile ``tn`` is. MODE 2: a wave's 64 tile
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_bf16_kernel(TileArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float g = acc[mi][ni][e], up = acc[mi][ni + 2][e];
-          o[e] = cw_float_to_bf16_bits(a.act > 0.0f ? cw_clipped_glu(g, up, a.act) : a.act < 0.0f ? fmaxf(g, 0.0f) * up : g / (1.0f + __expf(-g)) * up);
+          o[e] = cw_float_to_bf16_bits(a.act > 0.0f ? cw_clipped_glu(g, up, a.act) : a.act < 0.0f ? cw_gated_below(g, up, a.act) : g / (1.0f + __expf(-g)) * up);
         }
         bf16_t* dst = (bf16_t*)a.C + m * a.ldc + i0;
         if (i0 + 4 <= I && !(a.ldc & 3)) {
@@ -274,7 +274,7 @@ CW_EXPORT int cw_gemm_bf16_tiled(int mode, const void* X, int64_t ldx, const voi
 // change places between lane rows (v_permlane16_swap) so that it stores 16 bytes and four lanes
 // 64 bytes of a row.
 //
-// MODE as above (2 with ``act`` > 0: the clipped gated activation of that limit, < 0: max(gate, 0) * up), and 5: MODE 0 with
+// MODE as above (2 with ``act`` > 0: the clipped gated activation of that limit, -1: max(gate, 0) * up, -2: gelu_tanh(gate) * up), and 5: MODE 0 with
 // max(y, 0)^2, with ``act`` > 0 the tanh form of GELU, applied to the float32 sums (after the bias);
 // K a multiple of 64, at least 256; both matrices below 4 GiB. MODE 3: the product
 // of a narrow output with a long K (too few tiles to fill the card) summed in k_splits runs of K,
@@ -518,7 +518,8 @@ __global__ __launch_bounds__(256) void gemm_wide_bf16_kernel(WideArgs a) {
             const float gl = fminf(g, a.act), ul = fminf(fmaxf(up, -a.act), a.act);
             v[e] = gl * __builtin_amdgcn_rcpf(1.0f + __expf(-1.702f * gl)) * (ul + 1.0f);
           } else if (a.act < 0.0f) {
-            v[e] = fmaxf(g, 0.0f) * up;
+            const float logistic = __builtin_amdgcn_rcpf(1.0f + __expf(-1.5957691216057308f * (g + 0.044715f * g * g * g)));
+            v[e] = (a.act < -1.5f ? g * logistic : fmaxf(g, 0.0f)) * up;
           } else {
             v[e] = g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * up;
           }

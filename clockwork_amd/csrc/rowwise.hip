@@ -83,17 +83,26 @@ CW_EXPORT int cw_embedding_pos(const void* table, int dtype, const int* ids, con
 // What a block with sigmoid gates on its branches adds to the residual stream of row t, element j:
 //   s(z[t, j] + zb[j]) * a[t, j] + s(z[t, H + j] + zb[H + j]) * b[t, j]
 // z [T, 2H] (or [T, H] when there is no second branch) are the gates' products, zb their biases;
-// with z == nullptr the branches are added as they are. b may be absent.
+// with z == nullptr the branches are added as they are. b may be absent; with parts > 0 it is what a product left in
+// that many float32 planes of partial sums, ``plane`` elements apart, added in their order.
 template <typename T, typename BT>
 struct GatedPair {
   const T* z;
   const BT* zb;
   const T* a;
-  const T* b;
+  const void* b;
   int z_stride;
+  int parts;
+  int64_t plane;
+  __device__ __forceinline__ float second(int64_t at) const {
+    if (parts == 0) return cw_to_float(((const T*)b)[at]);
+    float v = ((const float*)b)[at];
+    for (int q = 1; q < parts; ++q) v += ((const float*)b)[q * plane + at];
+    return v;
+  }
   __device__ __forceinline__ float at(int64_t t, int j, int H) const {
     float va = cw_to_float(a[t * H + j]);
-    float vb = b ? cw_to_float(b[t * H + j]) : 0.0f;
+    float vb = b ? second(t * H + j) : 0.0f;
     if (z) {
       float za = cw_to_float(z[t * z_stride + j]);
       if (zb) za += cw_to_float(zb[j]);
@@ -161,7 +170,7 @@ __global__ __launch_bounds__(256) void add_layernorm_vec_kernel(float* __restric
   const int64_t t = rows ? rows[i] : i;
   float* x = resid + t * H;
   const bool has = pend.a != nullptr;
-  float v[KC][4], w[KC][4], c[KC][4], a[KC][4], b[KC][4], za[KC][4], zb[KC][4], ba[KC][4], bb[KC][4];
+  float v[KC][4], w[KC][4], c[KC][4], a[KC][4], b[KC][4], za[KC][4], zb[KC][4], ba[KC][4], bb[KC][4], planes[4][KC][4];
 #pragma unroll
   for (int k = 0; k < KC; ++k) {
     const int ch = threadIdx.x + k * 256;
@@ -173,7 +182,12 @@ __global__ __launch_bounds__(256) void add_layernorm_vec_kernel(float* __restric
       if (bias) CwVec<WT, 4>::load(bias + ch * 4, c[k]);
       if (has) {
         CwVec<T, 4>::load(pend.a + t * H + ch * 4, a[k]);
-        if (pend.b) CwVec<T, 4>::load(pend.b + t * H + ch * 4, b[k]);
+        if (pend.b && pend.parts == 0) CwVec<T, 4>::load((const T*)pend.b + t * H + ch * 4, b[k]);
+        if (pend.parts > 0) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            if (q < pend.parts) CwVec<float, 4>::load((const float*)pend.b + q * pend.plane + t * H + ch * 4, planes[q][k]);
+        }
         if (pend.z) {
           CwVec<T, 4>::load(pend.z + t * pend.z_stride + ch * 4, za[k]);
           if (pend.zb) CwVec<BT, 4>::load(pend.zb + ch * 4, ba[k]);
@@ -183,6 +197,23 @@ __global__ __launch_bounds__(256) void add_layernorm_vec_kernel(float* __restric
           }
         }
       }
+    }
+  }
+  for (int q0 = 0; q0 < pend.parts; q0 += 4) {  // in their order, four on their way at a time
+#pragma unroll
+    for (int k = 0; k < KC; ++k) {
+      const int ch = threadIdx.x + k * 256;
+      if (ch >= n_chunks) continue;
+      if (q0 > 0) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (q0 + q < pend.parts) CwVec<float, 4>::load((const float*)pend.b + (q0 + q) * pend.plane + t * H + ch * 4, planes[q][k]);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (q0 + q < pend.parts)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) b[k][e] += planes[q][k][e];
     }
   }
   float s = 0.0f;
@@ -224,18 +255,20 @@ __global__ __launch_bounds__(256) void add_layernorm_vec_kernel(float* __restric
   }
 }
 
-// z/zb/a/b: the pending gated branches (all nullptr: none); z_cols: columns of z (H or 2H).
+// z/zb/a/b: the pending gated branches (all nullptr: none); z_cols: columns of z (H or 2H); b_parts > 0: b is that many
+// float32 planes of partial sums, b_plane elements apart.
 CW_EXPORT int cw_add_layernorm(float* resid, const void* z, const void* zb, int zb_dtype, const void* a, const void* b,
-                               int z_cols, const void* weight, const void* bias, int w_dtype, float eps, void* out,
+                               int z_cols, int b_parts, int64_t b_plane, const void* weight, const void* bias, int w_dtype, float eps, void* out,
                                int dtype, const int* rows, int n, int H, hipStream_t stream) {
   if (n < 0 || H <= 0 || !resid || !weight || !out) return CW_ERR_ARG;
   if (!a && (z || b)) return CW_ERR_ARG;
+  if (b_parts < 0 || (b_parts > 0 && (!b || b_plane < (rows ? H : (int64_t)n * H)))) return CW_ERR_ARG;
   if (z && z_cols != (b ? 2 * H : H) && z_cols != 2 * H) return CW_ERR_ARG;
   if (n == 0) return CW_OK;
   dim3 grid(n), block(256);
 #define CW_LAUNCH(T, WT, BT)                                                                               \
   do {                                                                                                     \
-    GatedPair<T, BT> pend{(const T*)z, (const BT*)zb, (const T*)a, (const T*)b, z_cols};                   \
+    GatedPair<T, BT> pend{(const T*)z, (const BT*)zb, (const T*)a, b, z_cols, b_parts, b_plane};           \
     if (quads && H <= 2048)                                                                                \
       hipLaunchKernelGGL((add_layernorm_vec_kernel<T, WT, BT, 2>), grid, block, 0, stream, resid, pend,    \
                          (const WT*)weight, (const WT*)bias, eps, (T*)out, rows, H);                       \
@@ -247,7 +280,7 @@ CW_EXPORT int cw_add_layernorm(float* resid, const void* z, const void* zb, int 
                          (const WT*)weight, (const WT*)bias, eps, (T*)out, rows, H);                       \
   } while (0)
   // rows of more than 4096 elements do not fit the registers of 256 threads with all that is pending
-  const bool quads = rw_quads(H, resid, z, zb, a, b, weight, bias, out);
+  const bool quads = rw_quads(H, resid, z, zb, a, b, weight, bias, out) && b_plane % 4 == 0;
   const int zbt = zb ? zb_dtype : w_dtype;
   if (dtype == CW_F32 && w_dtype == CW_F32 && zbt == CW_F32) CW_LAUNCH(float, float, float);
   else if (dtype == CW_BF16 && w_dtype == CW_BF16 && zbt == CW_BF16) CW_LAUNCH(bf16_t, bf16_t, bf16_t);
@@ -271,8 +304,8 @@ __global__ void gated_residual_add_kernel(float* __restrict__ resid, GatedPair<T
 }
 
 CW_EXPORT int cw_gated_residual_add(float* resid, const void* z, const void* zb, int zb_dtype, const void* a,
-                                    const void* b, int z_cols, int dtype, int T, int H, hipStream_t stream) {
-  if (T < 0 || H <= 0 || !resid || !a) return CW_ERR_ARG;
+                                    const void* b, int z_cols, int b_parts, int64_t b_plane, int dtype, int T, int H, hipStream_t stream) {
+  if (T < 0 || H <= 0 || !resid || !a || b_parts < 0 || (b_parts > 0 && (!b || b_plane < (int64_t)T * H))) return CW_ERR_ARG;
   if (z && z_cols != H && z_cols != 2 * H) return CW_ERR_ARG;
   if (z && b && z_cols != 2 * H) return CW_ERR_ARG;
   if (T == 0) return CW_OK;
@@ -282,7 +315,7 @@ CW_EXPORT int cw_gated_residual_add(float* resid, const void* z, const void* zb,
   dim3 grid((unsigned)blocks), block(256);
 #define CW_LAUNCH(T_, BT_)                                                                     \
   do {                                                                                         \
-    GatedPair<T_, BT_> pend{(const T_*)z, (const BT_*)zb, (const T_*)a, (const T_*)b, z_cols}; \
+    GatedPair<T_, BT_> pend{(const T_*)z, (const BT_*)zb, (const T_*)a, b, z_cols, b_parts, b_plane}; \
     hipLaunchKernelGGL((gated_residual_add_kernel<T_, BT_>), grid, block, 0, stream, resid, pend, n, H); \
   } while (0)
   const int zbt = zb ? zb_dtype : dtype;

@@ -125,8 +125,8 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
         },
         "rowwise": {
             "cw_embedding_pos": [P, I, P, P, P, F, P, I, I, I, I, P],
-            "cw_add_layernorm": [P, P, P, I, P, P, I, P, P, I, F, P, I, P, I, I, P],
-            "cw_gated_residual_add": [P, P, P, I, P, P, I, I, I, I, P],
+            "cw_add_layernorm": [P, P, P, I, P, P, I, I, L, P, P, I, F, P, I, P, I, I, P],
+            "cw_gated_residual_add": [P, P, P, I, P, P, I, I, L, I, I, I, P],
             "cw_gelu_tanh_mul": [P, P, I, I, I, P],
             "cw_softcap": [P, L, F, P],
             "cw_rms_mean2": [P, P, P, P, I, F, P, I, I, I, P],
@@ -472,14 +472,15 @@ def rope_kv_write(qkv, bias, positions, slots, inv_freq, rotary_dim: int, nh: in
     )
 
 
-# in the place of a clipped gated activation's limit: max(gate, 0) * up
+# in the place of a clipped gated activation's limit: max(gate, 0) * up, and gelu_tanh(gate) * up
 RELU_GATE = -1.0
+GELU_GATE = -2.0
 
 
 def silu_mul(gate_up: torch.Tensor, out: torch.Tensor, limit: float = 0.0) -> torch.Tensor:
     """out[t, i] = silu(gate_up[t, i]) * gate_up[t, I + i]; ``limit`` > 0: the clipped gated activation
     g * logistic(1.702 g) * (u + 1) with g = min(gate, limit), u = up cut to [-limit, limit];
-    ``RELU_GATE``: max(gate, 0) * up."""
+    ``RELU_GATE``: max(gate, 0) * up; ``GELU_GATE``: gelu_tanh(gate) * up."""
     _gpu(gate_up, out)
     T, two_i = gate_up.shape
     if not (two_i % 2 == 0 and tuple(out.shape) == (T, two_i // 2) and out.dtype == gate_up.dtype):
@@ -1099,7 +1100,7 @@ def swiglu_norm_fusable(M: int, two_i: int, K: int, dtype, gate_up_weight, delta
 
 def linear_swiglu(x, gate_up_weight: torch.Tensor, policy: "ProductPolicy | None" = None, limit: float = 0.0) -> torch.Tensor:
     """silu(x @ gate.T) * (x @ up.T) for gate_up_weight = [gate; up] stacked along dim 0; ``limit`` > 0 or
-    ``RELU_GATE``: the other activations of the two products that ``silu_mul`` knows.
+    ``RELU_GATE`` or ``GELU_GATE``: the other activations of the two products that ``silu_mul`` knows.
 
     Few bfloat16 rows: one kernel that streams the weights once and applies the gate in its
     epilogue. Otherwise the product followed by the gate kernel, or (``policy``, see ``linear``)
@@ -1147,7 +1148,8 @@ def linear_swiglu(x, gate_up_weight: torch.Tensor, policy: "ProductPolicy | None
                 policy.swiglu_choices[(two_i, K)] = _measure_swiglu(x, gate_up_weight, out)
             if not measured or policy.swiglu_choices.get((two_i, K), True):
                 return linear_tiled(x, gate_up_weight, swiglu=True, wide=True, limit=limit)
-    return silu_mul(linear(x, gate_up_weight, policy=policy), out, limit)
+    gate_up = linear(x, gate_up_weight, policy=policy)
+    return gelu_tanh_mul(gate_up, out) if limit == GELU_GATE else silu_mul(gate_up, out, limit)
 
 
 _zero_rows: dict = {}
@@ -1416,7 +1418,8 @@ class GatedBranches:
     """What a block with gated branches still has to add to the residual stream:
     sigmoid(z[:, :H] + zb[:H]) * a + sigmoid(z[:, H:] + zb[H:]) * b. ``z`` [T, H or 2H] are the
     gates' products, ``zb`` their biases (or None); without ``z`` the branches count as they are;
-    ``b`` may be None. A norm that ``accepts_gated`` adds it inside its own kernel."""
+    ``b`` may be None, or the :class:`PartialSums` of a product. A norm that ``accepts_gated`` adds it inside its own
+    kernel."""
 
     __slots__ = ("z", "zb", "a", "b")
 
@@ -1428,9 +1431,12 @@ class GatedBranches:
         return self.a.shape
 
     def check(self, T: int, H: int, dtype) -> None:
-        _gpu(self.z, self.zb, self.a, self.b)
+        sums = isinstance(self.b, PartialSums)
+        _gpu(self.z, self.zb, self.a, self.b.parts if sums else self.b)
         _need(tuple(self.a.shape) == (T, H) and self.a.dtype == dtype, "a gated branch must be [T, H] in the activation type")
-        if self.b is not None:
+        if sums:
+            _need(tuple(self.b.shape) == (T, H) and self.b.parts.dtype == torch.float32, "a branch's partial sums must be float32 [splits, T, H]")
+        elif self.b is not None:
             _need(tuple(self.b.shape) == (T, H) and self.b.dtype == dtype, "a gated branch must be [T, H] in the activation type")
         if self.z is not None:
             cols = 2 * H if self.b is not None else H
@@ -1442,8 +1448,9 @@ class GatedBranches:
             _need(self.zb is None, "gate biases without gates")
 
     def args(self):
+        b, splits = (self.b.parts, self.b.parts.shape[0]) if isinstance(self.b, PartialSums) else (self.b, 0)
         return (_ptr(self.z), _ptr(self.zb), dtype_code(self.zb.dtype) if self.zb is not None else 0, _ptr(self.a),
-                _ptr(self.b), int(self.z.shape[1]) if self.z is not None else 0)
+                _ptr(b), int(self.z.shape[1]) if self.z is not None else 0, splits, b.stride(0) if splits else 0)
 
 
 def gated_residual_add(resid: torch.Tensor, pending: GatedBranches) -> torch.Tensor:
@@ -1474,7 +1481,7 @@ def add_layernorm(resid, pending, weight, bias, eps: float, out, rows=None) -> t
         pending.check(T, H, out.dtype)
         args = pending.args()
     else:
-        args = (None, None, 0, None, None, 0)
+        args = (None, None, 0, None, None, 0, 0, 0)
     _check(_load("rowwise").cw_add_layernorm(_ptr(resid), *args, _ptr(weight), _ptr(bias), dtype_code(weight.dtype),
                                              float(eps), _ptr(out), dtype_code(out.dtype), _ptr(rows), n, H, _stream()),
            "add_layernorm")

@@ -96,6 +96,8 @@ class ParallelBlock:
         self.mixer, self.mixer_norm, self.feed_forward, self.gate = mixer, mixer_norm, feed_forward, gate
         if gate is not None and gate.spec.branches != (2 if feed_forward is not None else 1):
             raise ValueError("a block's gate needs one set of gates per branch")
+        if hasattr(feed_forward, "partial_ok"):
+            feed_forward.partial_ok = True   # ``GatedBranches`` takes a product's partial sums
 
     def parts(self) -> dict:
         parts = {"mixer": self.mixer, "mixer_norm": self.mixer_norm}

@@ -38,9 +38,8 @@ class SwiGLU(Part):
 
 
 class GatedMLP(Part):
-    """down(act(gate(x)) * up(x)) with the activation the spec names. "silu" and "relu" take the fused
-    kernels of :class:`SwiGLU`; "gelu_tanh" runs the gate/up product, one kernel for
-    gelu_tanh(gate) * up in float32, and the down product."""
+    """down(act(gate(x)) * up(x)) with the activation the spec names ("silu", "relu" or "gelu_tanh"), through the
+    kernels of :class:`SwiGLU`."""
 
     graph_safe = True
     partial_ok = False   # may the output come as ``ops.PartialSums``? A block whose next norm adds them up sets it
@@ -61,12 +60,9 @@ class GatedMLP(Part):
 
     def forward(self, x, ctx) -> torch.Tensor:
         policy = getattr(ctx, "products", None)
-        if self.spec.activation != "gelu_tanh":
-            inner = ops.linear_swiglu(x, self.gate_up, policy=policy, limit=ops.RELU_GATE if self.spec.activation == "relu" else 0.0)
-            return ops.linear(inner, self.down, partial_ok=self.partial_ok, policy=policy)
-        gate_up = ops.linear(x, self.gate_up, policy=policy)
-        inner = torch.empty((x.shape[0], self.spec.intermediate_size), dtype=x.dtype, device=x.device)
-        return ops.linear(ops.gelu_tanh_mul(gate_up, inner), self.down, policy=policy)
+        act = {"relu": ops.RELU_GATE, "gelu_tanh": ops.GELU_GATE}.get(self.spec.activation, 0.0)
+        inner = ops.linear_swiglu(x, self.gate_up, policy=policy, limit=act)
+        return ops.linear(inner, self.down, partial_ok=self.partial_ok, policy=policy)
 
 
 class DenseMLP(Part):

@@ -205,10 +205,12 @@ def test_rows_in_pieces_of_four(H, dtype):
     # values of a few units: the result's own rounding, and float32 sums of H terms
     tol = dict(atol=0.03, rtol=0.01) if dtype == torch.bfloat16 else dict(atol=2e-5, rtol=2e-5)
     w, b, zb, x = rand(H), rand(H), rand(2 * H), rand(T, H, dt=torch.float32)
-    one, two, z = rand(T, H), rand(T, H), rand(T, 2 * H)
+    one, two, z, planes = rand(T, H), rand(T, H), rand(T, 2 * H), ops.PartialSums(rand(6, T, H, dt=torch.float32))
     gates = torch.sigmoid(z.to(f64) + zb.to(f64))
     for pending, extra in ((None, 0), ((None, None, one, None), one.to(f64)), ((z[:, :H].contiguous(), None, one, None), torch.sigmoid(z[:, :H].to(f64)) * one.to(f64)),
-                           ((z, zb, one, two), gates[:, :H] * one.to(f64) + gates[:, H:] * two.to(f64))):
+                           ((z, zb, one, two), gates[:, :H] * one.to(f64) + gates[:, H:] * two.to(f64)),
+                           ((None, None, one, planes), one.to(f64) + planes.parts.to(f64).sum(0)),
+                           ((z, zb, one, planes), gates[:, :H] * one.to(f64) + gates[:, H:] * planes.parts.to(f64).sum(0))):
         total = x.to(f64) + extra
         want = torch.nn.functional.layer_norm(total, (H,), w.to(f64), b.to(f64), 1e-5)
         branches = None if pending is None else ops.GatedBranches(*pending)
@@ -220,6 +222,8 @@ def test_rows_in_pieces_of_four(H, dtype):
         got = ops.add_layernorm(resid, branches, w, b, 1e-5, torch.empty(T, H, dtype=dtype, device=DEV))
         torch.testing.assert_close(got.to(f64), want, **tol)
         torch.testing.assert_close(resid.to(f64), total, atol=1e-5, rtol=1e-5)
+        if branches is not None:
+            torch.testing.assert_close(ops.gated_residual_add(x.clone(), branches).to(f64), total, atol=1e-5, rtol=1e-5)
     rms = lambda t, u: t.to(f64) * torch.rsqrt(t.to(f64).square().mean(-1, keepdim=True) + 1e-5) * u.to(f64)  # noqa: E731
     u, v = rand(H), rand(H)
     torch.testing.assert_close(ops.rms_mean2(one, two, u, v, 1e-5).to(f64), 0.5 * (rms(one, u) + rms(two, v)), **tol)
@@ -328,3 +332,27 @@ def test_sink_decode_runs(heads, kv, dim, vdim, talk, sk, dtype):
         # float32 sums of up to 300 terms of a few units; bfloat16: the result's own rounding
         tol = dict(atol=0.005, rtol=0.005) if dtype == torch.bfloat16 else dict(atol=2e-5, rtol=2e-5)
         torch.testing.assert_close(out[r].to(f64), want, **tol)
+
+
+# rows of the streaming kernels (one and several), of the tiles between and of the wide tiles; sizes that each takes
+@pytest.mark.parametrize("M,K,I", [(1, 96, 64), (8, 1536, 8960), (33, 256, 512), (130, 1536, 8960), (400, 1536, 8960), (1100, 1536, 8960), (9, 100, 36)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_gate_up_products_with_gelu(M, K, I, dtype):
+    from clockwork_amd import ops
+
+    if dtype == torch.float32 and M > 130:
+        pytest.skip("float32 has no epilogue of its own")
+    gen = torch.Generator(device=DEV).manual_seed(M)
+    x, w = (torch.randn(*s, device=DEV, generator=gen).to(dtype) for s in ((M, K), (2 * I, K)))
+    w *= 2.0 * K ** -0.5
+    h = x.double() @ w.double().t()
+    want = torch.nn.functional.gelu(h[:, :I], approximate="tanh") * h[:, I:]
+    got = ops.linear_swiglu(x, w, limit=ops.GELU_GATE).double()
+    # a product is off by its float32 sum (sums of K terms that come to about 2: 2^-19) and, where it is written before
+    # the gate is applied, by its rounding (2^-8 of it in bfloat16's 8 bits); the gate's slope is at most 1.13, and the result is
+    # rounded once more
+    half = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24
+    g, u = h[:, :I].abs(), h[:, I:].abs()
+    off_g, off_u = half * g + 2.0 ** -19, half * u + 2.0 ** -19
+    bound = 1.13 * (off_g * (u + off_u) + g * off_u) + (half + 2.0 ** -20) * want.abs()
+    assert bool(((got - want).abs() <= bound).all())
