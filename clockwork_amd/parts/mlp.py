@@ -62,7 +62,7 @@ class GatedMLP(Part):
         policy = getattr(ctx, "products", None)
         act = {"relu": ops.RELU_GATE, "gelu_tanh": ops.GELU_GATE}.get(self.spec.activation, 0.0)
         inner = ops.linear_swiglu(x, self.gate_up, policy=policy, limit=act)
-        return ops.linear(inner, self.down, partial_ok=self.partial_ok, policy=policy)
+        return ops.linear(inner, self.down, partial_ok=self.partial_ok, policy=policy, portions_partial_ok=self.partial_ok)
 
 
 class DenseMLP(Part):
