@@ -86,7 +86,7 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ resid, const T* __restric
   }
 }
 
-// The same for rows of up to 4096 elements with H % 4 == 0: every thread keeps its (at most four)
+// The same for rows of up to 8192 elements with H % 4 == 0: every thread keeps its (at most eight)
 // 4-element chunks of the row in registers, so the row is read once, and all loads are in flight
 // together. The order of the sum of squares depends on H alone here too.
 template <typename T> struct Chunk4;
