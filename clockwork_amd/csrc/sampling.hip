@@ -170,10 +170,10 @@ __device__ __forceinline__ uint32_t philox_first_word(uint64_t seed, uint64_t co
 // last of a row's workgroups to finish could do that without a launch, but what the others wrote has to be made
 // visible to it: the fences that do so cost 170 us for 64 rows, the two launches 10.)
 //
-//   MAX      per chunk: the largest logit and its first index;
-//   HIST     per chunk, over 512 bins of the distance mx - logit / T from the largest (1 / 16 wide, the last one
-//            for everything beyond): how many tokens fall into each (rows with top-k) and what they weigh, the
-//            weights being exp(logit / T - mx) (rows with top-p); and what the chunk weighs. Greedy rows end here;
+//   MAX      per chunk: the largest logit and its first index; and 64 logits of the row, one every V / 64;
+//   HIST     per chunk, over 512 bins of logit / T: how many tokens fall into each (rows with top-k) and what they
+//            weigh, the weights being exp(logit / T - mx) (rows with top-p); and what the chunk weighs. Greedy rows
+//            end here;
 //   PICK     per row: the bin that holds the k-th largest token, or the bin in which the weight from the top exceeds
 //            top_p * total;
 //   COLLECT  per chunk: what the tokens above that bin weigh (all of them stay), and a list of the tokens in it;
@@ -185,21 +185,32 @@ __device__ __forceinline__ uint32_t philox_first_word(uint64_t seed, uint64_t co
 //            either option come here from HIST. For a row with both options whose nucleus ends in a bin above the
 //            k-th token's, COLLECT and DRAW run once more.
 //
-// A token's bin does not fall as its logit grows, and equal logits / T share a bin: what lies in bins above is kept,
-// what lies in bins below is not. A list that does not fit (a row of many equal logits) is not used: DRAW walks
-// the row instead.
+// A token's bin does not fall as its logit falls, and equal logits / T share a bin: what lies in bins of lower number
+// is kept, what lies in bins of higher number is not.
+// The bins: 3 segments of 170 equal bins, from the row's maximum to the 9th of its 64 sampled logits in descending
+// order, from there to the 33rd, and from there on (sample_segments). However the row is spread, a segment holds about
+// as many tokens as the samples say, so that a bin of a row of 151,936 tokens holds some hundreds and its list is short:
+// rows of a spread of 0.02 to 60 (logits / T, normal) and rows that are mostly -inf take the same time. (Bins of one
+// width for all rows, 1 / 16, held 4200 tokens at a spread of 0.8 and all but a few at 60. Top-p 0.9 in us, 8 rows,
+// radix steps over whole rows / bins of one width / these: spread 3 57 / 47 / 47, spread 0.4 58 / 903 / 51; top-k 50 at a
+// spread of 60 41 / 915 / 35.)
+// A list does not fit where more than SAMPLE_LIST tokens share a bin all the same: thousands of equal logits, of which
+// only their number matters (64 rows of one value: 245 / 625 / 95 us), or a cluster much narrower than the samples lie
+// apart. DRAW then walks the row instead of the list, one workgroup a row (a third of the row within 3e-5, the nucleus's
+// last token in it, 64 rows: 169 us by radix steps over whole rows, 563 so).
 // The draw: u * total falls into a chunk, and in it on the first index whose running sum exceeds it.
 // Weights are integers, exp(.) * 2^40 rounded down: their sums do not depend on the order of
 // addition, so every comparison above gives the same answer however the row is cut and however
 // the additions are scheduled (LDS atomics included), run after run.
 // Bound by the passes over the logits, which come from the memory-side cache after the first. 64 rows of 151,936
 // logits, a quarter each greedy, temperature, top-k and top-p: 119 us as twelve kernels (a radix step of 8 bits of the
-// key each, over the whole rows), 61 us as five.
+// key each, over the whole rows), 64 us as five (61 with bins of one width).
 #define SAMPLE_THREADS 256
 #define SAMPLE_WAVES (SAMPLE_THREADS / 64)
 #define SAMPLE_MAX_CHUNKS 64
 #define SAMPLE_BINS 512
-#define SAMPLE_BINS_PER_UNIT 16.0f
+#define SAMPLE_SEGMENT_BINS 170  // of each of three segments
+#define SAMPLE_POINTS 64         // logits of a row that are sampled: a lane each
 #define SAMPLE_LIST 4096         // tokens of a row's list
 #define SAMPLE_BLOCK_LIST 1024   // tokens that one workgroup may add to it
 #define SAMPLE_WEIGHT_SCALE 1099511627776.0f  // 2^40
@@ -213,6 +224,7 @@ struct SampleRow {     // what is known about a row between two kernels
   uint32_t collect;    // 1: COLLECT has to run, 2: its second run has to
   uint32_t listed[2];  // tokens that COLLECT's two runs found in the bin
   uint32_t unused;     // (a whole number of 8 bytes)
+  float2 segments[3];  // see SampleBins
 };
 
 struct SampleArgs {
@@ -230,10 +242,12 @@ struct SampleArgs {
   u64_t* hist_w;      // [n][chunks][SAMPLE_BINS]
   u64_t* sums;        // [n][chunks] weight of the chunk (of its bins above the collected one, after COLLECT)
   SampleRow* rows;    // [n], zeroed by MAX
+  uint4* found;       // [n][chunks] smallest and largest key that COLLECT found in the bin, (~0, 0) for none, and how many
   uint32_t* hist_n;   // [n][chunks][SAMPLE_BINS]
   uint2* list;        // [n][SAMPLE_LIST] (key, index)
   float* pmax;        // [n][chunks]
   int* pmax_i;        // [n][chunks]
+  float* points;      // [n][SAMPLE_POINTS]
 };
 
 // Chunks a row is cut into: at least 2048 tokens each; 64 for few rows, for many rows as few as still make two
@@ -247,7 +261,7 @@ static int sample_chunks(int n, int V) {
 
 CW_EXPORT int64_t cw_sample_workspace_bytes(int n, int V) {
   const int64_t rc = (int64_t)n * sample_chunks(n, V);
-  return rc * SAMPLE_BINS * 12 + rc * 16 + (int64_t)n * ((int64_t)sizeof(SampleRow) + SAMPLE_LIST * 8) + 64;
+  return rc * SAMPLE_BINS * 12 + rc * 32 + (int64_t)n * ((int64_t)sizeof(SampleRow) + SAMPLE_LIST * 8 + SAMPLE_POINTS * 4) + 64;
 }
 
 __device__ __forceinline__ float key_to_float(uint32_t k) {
@@ -262,12 +276,55 @@ __device__ __forceinline__ u64_t weight_of(float v, float mx) {
   const float e = expf(v - mx);  // NaN for inf - inf: no weight
   return e == e ? (u64_t)(e * SAMPLE_WEIGHT_SCALE) : 0;
 }
-// The bin of v = logit / T (NaN goes last, with -inf).
-__device__ __forceinline__ uint32_t bin_of(float v, float mx) {
-  if (v != v) return SAMPLE_BINS - 1;
-  if (!(v < mx)) return 0;
-  const float d = (mx - v) * SAMPLE_BINS_PER_UNIT;
-  return d < (float)(SAMPLE_BINS - 1) ? (uint32_t)d : SAMPLE_BINS - 1;
+// The three segments of a row's bins: x is the largest logit / T of one, y how many bins go into a unit below that (0
+// where the segment has no width: it is one bin then).
+struct SampleBins {
+  float2 s0, s1, s2;
+};
+__device__ __forceinline__ SampleBins sample_bins(const float2* p) { return SampleBins{p[0], p[1], p[2]}; }
+// The bin of v = logit / T (-inf and NaN go last): the last segment whose top it lies below, or the first, and there
+// the distance from the top in bins.
+__device__ __forceinline__ uint32_t bin_of(const SampleBins& bins, float v) {
+  const float2 s0 = bins.s0, s1 = bins.s1, s2 = bins.s2;
+  const bool b1 = v < s1.x, b2 = v < s2.x;
+  const float x = b2 ? s2.x : b1 ? s1.x : s0.x, y = b2 ? s2.y : b1 ? s1.y : s0.y;
+  const float d = __builtin_amdgcn_fmed3f((x - v) * y, 0.0f, (float)(SAMPLE_SEGMENT_BINS - 1));  // (NaN for inf - inf: 0)
+  const uint32_t first = b2 ? 2u * SAMPLE_SEGMENT_BINS : b1 ? (uint32_t)SAMPLE_SEGMENT_BINS : 0u;
+  return v > -INFINITY ? first + (uint32_t)d : SAMPLE_BINS - 1;
+}
+__device__ __forceinline__ float bins_per_unit(float width) {
+  const float y = (float)SAMPLE_SEGMENT_BINS / width;
+  return y > 0.0f && y < INFINITY ? y : 0.0f;
+}
+// The segments of a row, by one wave: ``point`` is the lane's sample. The second and the third begin at the
+// 9th and the 33rd sample in descending order, and the bins of a segment go down to where the next one begins; the third's
+// twice as far down as the 62nd sample. Where the samples further down are masks (-inf, or as low as the type goes) a
+// segment's bins go twice as far down as the last sample that is not. ``out`` (LDS): the second and the third segment, and
+// ahead of them what the first one's bins go down to, and how many times as far.
+__device__ __forceinline__ void sample_segments(float point, float temp, float2* out) {
+  const int lane = threadIdx.x & 63;
+  // the order of the samples; those that are all but equal by their lanes
+  const uint32_t key = (order_key(point) & ~63u) | (uint32_t)lane;
+  int rank = 0;
+#pragma unroll
+  for (int l = 0; l < SAMPLE_POINTS; ++l) rank += (uint32_t)__builtin_amdgcn_readlane((int)key, l) > key ? 1 : 0;
+  const int last = SAMPLE_POINTS - 1 - __popcll(__ballot(!(point > -1e30f)));  // -1: all are masks
+  // lanes 0 to 4 take a sample each: the tops of segments 1 and 2, and the ends of 0, 1 and 2
+  const int ranks[5] = {8, 32, min(8, last), min(32, last), min(61, last)};
+  int from = 0;
+#pragma unroll
+  for (int i = 0; i < 5; ++i) {
+    const int l = __ffsll((unsigned long long)__ballot(rank == max(ranks[i], 0))) - 1;
+    from = lane == i ? l : from;
+  }
+  const float v = __shfl(point, from, 64) / temp;
+  const float mine = v == v ? v : -INFINITY;
+  const float top1 = __shfl(mine, 0, 64), top2 = __shfl(mine, 1, 64), end0 = __shfl(mine, 2, 64), end1 = __shfl(mine, 3, 64), end2 = __shfl(mine, 4, 64);
+  if (lane == 0) {
+    out[0] = make_float2(last < 0 ? -INFINITY : end0, last < 8 ? 2.0f : 1.0f);
+    out[1] = make_float2(top1, bins_per_unit((last < 32 ? 2.0f : 1.0f) * (top1 - end1)));
+    out[2] = make_float2(top2, bins_per_unit(2.0f * (top2 - end2)));
+  }
 }
 __device__ __forceinline__ u64_t topp_limit(float p, u64_t total) { return (u64_t)((double)p * (double)total); }
 
@@ -281,20 +338,20 @@ __device__ __forceinline__ void sample_load4(const float* x, int i, int hi, int 
     for (int e = 0; e < 4; ++e) o[e] = i + e < hi ? x[i + e] : NAN;
   }
 }
-// f(index, logit) for the tokens of [lo, hi), by all threads of the workgroup, eight loads in flight a thread.
-template <typename F>
+// f(index, logit) for the tokens of [lo, hi) (lo a multiple of 4), by THREADS neighbouring threads (all of the workgroup, or
+// a wave), 4 U loads in flight a thread. Up to three tokens past hi come as NaN, which everything here takes for -inf: a
+// test for each token by itself would cost as much as what most tokens need.
+template <int U = 2, int THREADS = SAMPLE_THREADS, typename F>
 __device__ __forceinline__ void sample_walk(const float* x, int lo, int hi, int vec, F f) {
-  for (int i0 = lo + (int)threadIdx.x * 4; i0 < hi; i0 += 8 * SAMPLE_THREADS) {
-    float a[4], b[4];
-    const int i1 = i0 + 4 * SAMPLE_THREADS;
-    sample_load4(x, i0, hi, vec, a);
-    sample_load4(x, min(i1, (int)((unsigned)(hi - 1) & ~3u)), hi, vec, b);
+  for (int i0 = lo + (int)(threadIdx.x & (THREADS - 1)) * 4; i0 < hi; i0 += U * 4 * THREADS) {
+    float a[U][4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (i0 + e < hi) f(i0 + e, a[e]);
+    for (int u = 0; u < U; ++u) sample_load4(x, min(i0 + u * 4 * THREADS, (int)((unsigned)(hi - 1) & ~3u)), hi, vec, a[u]);
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (i1 + e < hi) f(i1 + e, b[e]);
+    for (int u = 0; u < U; ++u)
+      if (i0 + u * 4 * THREADS < hi)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f(i0 + u * 4 * THREADS + e, a[u][e]);
   }
 }
 
@@ -361,9 +418,14 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_max_kernel(SampleArgs a
   const int row = blockIdx.y, chunk = blockIdx.x;
   if (chunk == 0 && threadIdx.x < sizeof(SampleRow) / 4) reinterpret_cast<uint32_t*>(a.rows + row)[threadIdx.x] = 0u;
   const int lo = chunk * a.per, hi = min(a.V, lo + a.per);
+  const float* x = a.logits + (int64_t)row * a.row_stride;
+  if (threadIdx.x < SAMPLE_POINTS) {
+    const int at = (int)((2 * (int64_t)threadIdx.x + 1) * a.V / (2 * SAMPLE_POINTS));
+    if (at >= lo && at < hi) a.points[(int64_t)row * SAMPLE_POINTS + threadIdx.x] = x[at];
+  }
   float bv = -INFINITY;
   int bi = 0x7fffffff;
-  sample_walk(a.logits + (int64_t)row * a.row_stride, lo, hi, a.vec, [&](int i, float v) __attribute__((always_inline)) {
+  sample_walk(x, lo, hi, a.vec, [&](int i, float v) __attribute__((always_inline)) {
     if (v != v) v = -INFINITY;
     argmax_merge(bv, bi, v, i);
   });
@@ -459,8 +521,13 @@ __device__ __forceinline__ void sample_locate(const SampleArgs& a, int row, floa
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_hist_kernel(SampleArgs a) {
   __shared__ u64_t bins_w[SAMPLE_BINS];
   __shared__ uint32_t bins_n[SAMPLE_BINS];
+  __shared__ float2 segments[3];
   const int row = blockIdx.y, chunk = blockIdx.x;
   const float temp = a.temperature[row];
+  const bool with_k = row_has_top_k(a, row), with_p = row_has_top_p(a, row);
+  // the second wave works the segments out while the first looks for the maximum
+  const float point = a.points[(int64_t)row * SAMPLE_POINTS + (threadIdx.x & 63)];
+  if (temp > 0.0f && (with_k || with_p) && threadIdx.x >> 6 == 1) sample_segments(point, temp, segments);
   float mraw;
   int mi;
   row_max(a, row, mraw, mi);
@@ -468,22 +535,34 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_hist_kernel(SampleArgs 
     if (chunk == 0 && threadIdx.x == 0) a.out[row] = mi < a.V ? mi : 0;
     return;
   }
-  const bool with_k = row_has_top_k(a, row), with_p = row_has_top_p(a, row);
   const float mx = mraw / temp;
-  for (int b = threadIdx.x; b < SAMPLE_BINS; b += SAMPLE_THREADS) {
-    bins_w[b] = 0;
-    bins_n[b] = 0u;
+  SampleBins bins = {};
+  if (with_k || with_p) {
+    bins = sample_bins(segments);  // (behind row_max's barriers)
+    // (without a sample that is no mask: bins of 1 / 16)
+    bins.s0 = make_float2(mx, bins.s0.x == -INFINITY ? 16.0f : bins_per_unit(bins.s0.y * (mx - bins.s0.x)));
+    for (int b = threadIdx.x; b < SAMPLE_BINS; b += SAMPLE_THREADS) {
+      bins_w[b] = 0;
+      bins_n[b] = 0u;
+    }
+    __syncthreads();
+    if (chunk == 0 && threadIdx.x == 0) {
+      SampleRow& known = a.rows[row];
+      known.segments[0] = bins.s0;
+      known.segments[1] = bins.s1;
+      known.segments[2] = bins.s2;
+    }
   }
-  __syncthreads();
   const int lo = chunk * a.per, hi = min(a.V, lo + a.per);
   u64_t sum = 0;
   sample_walk(a.logits + (int64_t)row * a.row_stride, lo, hi, a.vec, [&](int, float raw) __attribute__((always_inline)) {
     const float v = raw / temp;
-    if (with_k) atomicAdd(&bins_n[bin_of(v, mx)], 1u);
+    const uint32_t bin = with_k || with_p ? bin_of(bins, v) : 0u;
+    if (with_k) atomicAdd(&bins_n[bin], 1u);
     if (with_k && !with_p) return;  // (COLLECT weighs what top-k leaves)
     const u64_t w = v == v ? weight_of(v, mx) : 0;
     sum += w;
-    if (with_p && w) atomicAdd(&bins_w[bin_of(v, mx)], w);
+    if (with_p && w) atomicAdd(&bins_w[bin], w);
   });
   sum = block_sum(sum);  // (and a barrier behind the bins)
   const int64_t rc = (int64_t)row * a.chunks + chunk;
@@ -550,42 +629,61 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(SampleArgs 
 // COLLECT; ``again``: its second run
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(SampleArgs a, int again) {
   __shared__ uint2 mine[SAMPLE_BLOCK_LIST];
-  __shared__ uint32_t n_mine, at_list;
+  __shared__ uint32_t n_mine, at_list, ends[2];
   const int row = blockIdx.y, chunk = blockIdx.x;
   SampleRow& known = a.rows[row];
   const float temp = a.temperature[row];
   if (!(temp > 0.0f) || known.collect != 1u + again) return;
+  const uint32_t bin = known.bin;
+  const int lo = chunk * a.per, hi = min(a.V, lo + a.per);
+  const float* x = a.logits + (int64_t)row * a.row_stride;
+  if (threadIdx.x == 0) n_mine = ends[1] = 0u, ends[0] = 0xffffffffu;
+  const SampleBins bins = sample_bins(known.segments);
   float mraw;
   int mi;
-  row_max(a, row, mraw, mi);
+  row_max(a, row, mraw, mi);  // (and barriers behind the above)
   const float mx = mraw / temp;
-  const uint32_t bin = known.bin;
-  const float* x = a.logits + (int64_t)row * a.row_stride;
-  if (threadIdx.x == 0) n_mine = 0u;
-  __syncthreads();
-  const int lo = chunk * a.per, hi = min(a.V, lo + a.per);
   u64_t sum = 0;
+  uint32_t least = 0xffffffffu, most = 0u;  // of the bin's keys
   // most tokens lie below the bin, and a comparison says so (the threshold is a little lower than the bin's end,
   // by more than the divisions and products round; NaN, which compares with nothing, goes the long way)
-  const float end = mx - (float)(bin + 1) / SAMPLE_BINS_PER_UNIT;
-  const float surely_below = bin == SAMPLE_BINS - 1 ? -INFINITY : (end - 1e-5f * (fabsf(end) + fabsf(mx) + 1.0f)) * temp;
+  const float2 s0 = bins.s0, s1 = bins.s1, s2 = bins.s2;
+  const uint32_t segment = min(bin / SAMPLE_SEGMENT_BINS, 2u), j = bin - segment * SAMPLE_SEGMENT_BINS;
+  const float seg_top = segment == 0 ? s0.x : segment == 1 ? s1.x : s2.x, seg_y = segment == 0 ? s0.y : segment == 1 ? s1.y : s2.y;
+  float end = segment == 0 ? s1.x : segment == 1 ? s2.x : -INFINITY;
+  if (j < SAMPLE_SEGMENT_BINS - 1 && seg_y > 0.0f) end = fmaxf(end, seg_top - (float)(j + 1) / seg_y);
+  const float surely_below = (end - 1e-5f * (fabsf(end) + fabsf(seg_top)) - 1e-30f) * temp;
   sample_walk(x, lo, hi, a.vec, [&](int i, float raw) __attribute__((always_inline)) {
     if (raw < surely_below) return;
     const float v = raw / temp;
-    const uint32_t b = bin_of(v, mx);
+    const uint32_t b = bin_of(bins, v);
     if (b < bin) {
       sum += weight_of(v, mx);
     } else if (b == bin) {
-      const uint32_t at = atomicAdd(&n_mine, 1u);
-      if (at < SAMPLE_BLOCK_LIST) mine[at] = make_uint2(order_key(raw), (uint32_t)i);
+      const uint32_t key = order_key(raw), at = atomicAdd(&n_mine, 1u);
+      most = max(most, key);
+      least = min(least, key);
+      if (at < SAMPLE_BLOCK_LIST) mine[at] = make_uint2(key, (uint32_t)i);
     }
   });
-  sum = block_sum(sum);
+  if (__ballot(most >= least)) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      least = min(least, (uint32_t)__shfl_xor((int)least, off, 64));
+      most = max(most, (uint32_t)__shfl_xor((int)most, off, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+      atomicMin(&ends[0], least);
+      atomicMax(&ends[1], most);
+    }
+  }
+  sum = block_sum(sum);  // (and a barrier behind the list)
   // a workgroup whose tokens do not fit its own list makes the row's look too long for everybody
   const uint32_t n_here = n_mine;
   if (threadIdx.x == 0) {
     a.sums[(int64_t)row * a.chunks + chunk] = sum;
-    at_list = n_here ? atomicAdd(&known.listed[again], n_here <= SAMPLE_BLOCK_LIST ? n_here : SAMPLE_LIST + 1u) : 0u;
+    a.found[(int64_t)row * a.chunks + chunk] = make_uint4(ends[0], ends[1], n_here, 0u);
+    if (n_here) at_list = atomicAdd(&known.listed[again], n_here <= SAMPLE_BLOCK_LIST ? n_here : SAMPLE_LIST + 1u);
   }
   __syncthreads();
   if (n_here <= SAMPLE_BLOCK_LIST)
@@ -600,7 +698,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(SampleArgs 
   __shared__ uint32_t bins_n[256];
   __shared__ uint2 list[SAMPLE_LIST];
   __shared__ u64_t picked_above;
-  __shared__ uint32_t picked, picked_rank, key_min, key_max;
+  __shared__ uint32_t picked, picked_rank, ends[2], chunk_n[SAMPLE_MAX_CHUNKS];
   const int row = blockIdx.x;
   SampleRow& known = a.rows[row];
   const float temp = a.temperature[row];
@@ -616,47 +714,49 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(SampleArgs 
     sample_locate(a, row, temp, mx, mi, 0u, chunk_w);
     return;
   }
-  const uint32_t bin = known.bin, listed = known.listed[again];
+  const uint32_t listed = known.listed[again];
   const float* x = a.logits + (int64_t)row * a.row_stride;
   const bool fits = listed <= SAMPLE_LIST;
-  if (threadIdx.x == 0) key_min = 0xffffffffu, key_max = 0u;
   if (fits)
     for (uint32_t i = threadIdx.x; i < listed; i += SAMPLE_THREADS) list[i] = a.list[(int64_t)row * SAMPLE_LIST + i];
+  if (threadIdx.x < 64) {  // a chunk a lane (there are at most 64)
+    uint4 e = make_uint4(0xffffffffu, 0u, 0u, 0u);
+    if ((int)threadIdx.x < a.chunks) e = a.found[(int64_t)row * a.chunks + threadIdx.x];
+    chunk_n[threadIdx.x] = e.z;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      e.x = min(e.x, (uint32_t)__shfl_xor((int)e.x, off, 64));
+      e.y = max(e.y, (uint32_t)__shfl_xor((int)e.y, off, 64));
+    }
+    if (threadIdx.x == 0) ends[0] = e.x, ends[1] = e.y;
+  }
   __syncthreads();
-  // f(key, index) for the tokens of the bin
+  // the bin's tokens are those with keys from least to most
+  const uint32_t least = ends[0], most = ends[1];
+  // f(key, index) for the tokens of the bin; a row that is walked waits for its loads, 32 of them a thread at a time
   auto candidates = [&](auto f) __attribute__((always_inline)) {
     if (fits) {
       for (uint32_t i = threadIdx.x; i < listed; i += SAMPLE_THREADS) f(list[i].x, (int)list[i].y);
     } else {
-      for (int i = threadIdx.x; i < a.V; i += SAMPLE_THREADS)
-        if (bin_of(x[i] / temp, mx) == bin) f(order_key(x[i]), i);
+      sample_walk<8>(x, 0, a.V, a.vec, [&](int i, float raw) __attribute__((always_inline)) {
+        const uint32_t key = order_key(raw);
+        if (key >= least && key <= most) f(key, i);
+      });
     }
   };
   // the keys of a bin have most of their bits in common: the selections below begin at the highest in which they differ
-  uint32_t least = 0xffffffffu, most = 0u;
-  candidates([&](uint32_t key, int) __attribute__((always_inline)) {
-    least = min(least, key);
-    most = max(most, key);
-  });
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    least = min(least, (uint32_t)__shfl_xor((int)least, off, 64));
-    most = max(most, (uint32_t)__shfl_xor((int)most, off, 64));
-  }
-  if ((threadIdx.x & 63) == 0) {
-    atomicMin(&key_min, least);
-    atomicMax(&key_max, most);
-  }
-  __syncthreads();
-  least = key_min;
-  most = key_max;
   const int differing = least < most ? 32 - __clz(least ^ most) : 0;  // low bits that are not the same in all
   const uint32_t common = differing == 32 ? 0u : (most >> differing) << differing;
   // (a NaN's key is that of -inf: neither weighs anything)
   auto scaled = [&](uint32_t key) __attribute__((always_inline)) -> float { return key_to_float(key) / temp; };
   const u64_t above = block_sum((int)threadIdx.x < a.chunks ? chunk_w[threadIdx.x] : 0);
   uint32_t floor_key = 0u;
-  if (with_k && !again) {
+  // a bin whose largest token has no weight (masked tokens; at low temperatures most of a row): whichever of its
+  // tokens stay, none is drawn, and nothing below it
+  const bool weightless = listed == 0u || weight_of(scaled(most), mx) == 0;
+  // equal logits, however many: all of them stay (the k-th largest is one of them, or the nucleus ends with them)
+  const u64_t equal_weight = least == most ? weight_of(scaled(most), mx) : 0;
+  if (with_k && !again && !weightless) {
     // the rank-th largest key of the bin
     uint32_t prefix = common, rank = known.rank;
     for (int left = differing; left > 0;) {
@@ -686,10 +786,14 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(SampleArgs 
     u64_t limit = known.limit;
     if (with_k && !again) {
       u64_t kept = 0;
-      candidates([&](uint32_t key, int) __attribute__((always_inline)) {
-        const float v = scaled(key);
-        if (order_key(v) >= floor_key) kept += weight_of(v, mx);
-      });
+      if (equal_weight > 0) {
+        if ((int)threadIdx.x < a.chunks) kept = chunk_n[threadIdx.x] * equal_weight;
+      } else if (!weightless) {
+        candidates([&](uint32_t key, int) __attribute__((always_inline)) {
+          const float v = scaled(key);
+          if (order_key(v) >= floor_key) kept += weight_of(v, mx);
+        });
+      }
       const u64_t total = above + block_sum(kept);
       limit = topp_limit(a.top_p[row], total);
       if (total == 0) {
@@ -740,14 +844,31 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(SampleArgs 
     const uint32_t floor_p = order_key(scaled(prefix));
     if (floor_p > floor_key) floor_key = floor_p;
   }
-  // what is kept of the bin joins its chunks
-  candidates([&](uint32_t key, int i) __attribute__((always_inline)) {
-    const float v = scaled(key);
-    if (order_key(v) >= floor_key) {
-      const u64_t w = weight_of(v, mx);
-      if (w) atomicAdd(&chunk_w[i / a.per], w);
+  // what is kept of the bin joins its chunks; of a row that is walked a wave takes whole chunks, and adds up by itself
+  if (weightless) {
+  } else if (equal_weight > 0) {
+    if ((int)threadIdx.x < a.chunks) chunk_w[threadIdx.x] += chunk_n[threadIdx.x] * equal_weight;
+  } else if (fits) {
+    for (uint32_t i = threadIdx.x; i < listed; i += SAMPLE_THREADS) {
+      const float v = scaled(list[i].x);
+      const u64_t w = order_key(v) >= floor_key ? weight_of(v, mx) : 0;
+      if (w) atomicAdd(&chunk_w[list[i].y / a.per], w);
     }
-  });
+  } else {
+    for (int c = threadIdx.x >> 6; c < a.chunks; c += SAMPLE_WAVES) {
+      const int lo = c * a.per, hi = min(a.V, lo + a.per);
+      u64_t sum = 0;
+      sample_walk<8, 64>(x, lo, hi, a.vec, [&](int, float raw) __attribute__((always_inline)) {
+        const uint32_t key = order_key(raw);
+        if (key < least || key > most) return;
+        const float v = raw / temp;
+        if (order_key(v) >= floor_key) sum += weight_of(v, mx);
+      });
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+      if ((threadIdx.x & 63) == 0) chunk_w[c] += sum;
+    }
+  }
   __syncthreads();
   sample_locate(a, row, temp, mx, mi, floor_key, chunk_w);
 }
@@ -776,11 +897,13 @@ CW_EXPORT int cw_sample(const float* logits, int64_t row_stride, int n, int V,
   a.hist_w = p8; p8 += rc * SAMPLE_BINS;
   a.list = (uint2*)p8; p8 += (int64_t)n * SAMPLE_LIST;
   a.hist_n = (uint32_t*)p8; p8 += rc * SAMPLE_BINS / 2;
+  a.found = (uint4*)p8; p8 += 2 * rc;
   a.sums = p8; p8 += rc;
   a.rows = (SampleRow*)p8; p8 += (int64_t)n * sizeof(SampleRow) / 8;
   a.pmax = (float*)p8;
   a.pmax_i = (int*)(a.pmax + rc);
-  if ((char*)(a.pmax_i + rc) > (char*)workspace + workspace_bytes) return CW_ERR_ARG;
+  a.points = (float*)(a.pmax_i + rc);
+  if ((char*)(a.points + (int64_t)n * SAMPLE_POINTS) > (char*)workspace + workspace_bytes) return CW_ERR_ARG;
   const dim3 grid(a.chunks, n), block(SAMPLE_THREADS);
   hipLaunchKernelGGL(sample_max_kernel, grid, block, 0, stream, a);
   hipLaunchKernelGGL(sample_hist_kernel, grid, block, 0, stream, a);

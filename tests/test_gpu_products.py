@@ -51,46 +51,108 @@ def test_float32_infinities_stay_in_their_rows_and_columns():
         assert bool((got[:-1, :69] == 528).all())
 
 
-# odd sizes (rows that do not begin at 16 bytes), values in steps of a half (bins of thousands of equal logits, more
-# than a workgroup's list and a row's list hold), nearly flat rows (all in a few bins), spread ones
-@pytest.mark.parametrize("V,kind", [(1, "spread"), (511, "spread"), (2049, "steps"), (33333, "flat"), (151936, "steps"), (151936, "spread")])
+def _kept_cdf(row, temp, k, p, slack):
+    """Which tokens stay and the running sums of their weights in index order, in float64, by the sampler's definition: ties at
+    the k-th value survive, a token stays while the mass strictly above it is at most p (+ slack) of what top-k left."""
+    v = row / temp
+    keep = torch.ones_like(v, dtype=torch.bool)
+    if 0 < k < v.numel():
+        keep = v >= row.topk(k).values[-1] / temp
+    w = torch.where(keep, torch.exp(v.double() - v.max().double()), 0.0)
+    if p < 1.0:
+        values, group = torch.unique(v, return_inverse=True)   # ascending
+        mass = torch.zeros(values.numel(), dtype=torch.float64, device=row.device).index_add_(0, group, w)
+        above = mass.flip(0).cumsum(0).flip(0) - mass
+        keep &= (above <= (p + slack) * mass.sum())[group]
+        w = torch.where(keep, w, 0.0)
+    cdf = w.cumsum(0)
+    return keep, cdf / cdf[-1]
+
+
+# odd sizes (rows that do not begin at 16 bytes), values in steps of a half (thousands of equal logits in a bin, more
+# than a workgroup's list and a row's list hold), nearly flat rows, spread ones, all equal, all but some masked by -inf or by
+# the lowest value, a third of the row in a cluster that is narrower than any bin
+@pytest.mark.parametrize("V,kind", [(1, "spread"), (70, "spread"), (511, "spread"), (2049, "steps"), (33333, "flat"), (151936, "steps"), (151936, "spread"),
+                                    (151936, "flat"), (40001, "equal"), (151936, "masked"), (151936, "lowest"), (151936, "cluster")])
 def test_sampling_lists_bins_and_chunks(V, kind):
-    """Every option against the plain definition, and the same tokens however many rows share the launch (which
-    sets how a row is cut)."""
+    """Every option against its definition in float64, and the same tokens however many rows share the launch
+    (which sets how a row is cut)."""
     from clockwork_amd import ops
     from tests.plain import qwen2_plain as plain
 
     gen = torch.Generator(device=DEV).manual_seed(V)
-    n = 20
-    logits = torch.randn(n, V, device=DEV, generator=gen) * {"spread": 5.0, "steps": 2.0, "flat": 0.01}[kind]
+    n, draws_each = 24, 8
+    logits = torch.randn(n, V, device=DEV, generator=gen) * {"spread": 5.0, "steps": 2.0, "flat": 0.01, "equal": 0.0}.get(kind, 3.0)
     if kind == "steps":
         logits = (2.0 * logits).round() / 2.0
-    temps = torch.tensor([0.7, 1.0, 2.5, 0.0] * 5, device=DEV)
-    ks = [-1] * 4 + [7] * 4 + [-1] * 4 + [max(1, V // 2)] * 4 + [30] * 4   # the fourth: the nucleus ends far above the k-th token
-    ps = [1.0] * 8 + [0.8] * 4 + [0.3] * 4 + [0.97] * 4
+    logits += 0.0   # no -0: the sampler's order has it below 0, while they compare equal
+    if kind in ("masked", "lowest"):
+        hidden = torch.rand(n, V, device=DEV, generator=gen) > torch.linspace(0.0003, 0.5, n, device=DEV)[:, None]
+        hidden[:, 5] = False
+        logits[hidden] = -float("inf") if kind == "masked" else torch.finfo(torch.float32).min
+    if kind == "cluster":
+        logits[:, ::3] = 1.0 + 1e-5 * logits[:, ::3]
+    temps = torch.tensor([0.7, 1.0, 2.5, 0.0] * 5 + [0.05, 0.05, 0.05, 4.0], device=DEV)
+    ks = [-1] * 4 + [7] * 4 + [-1] * 4 + [max(1, V // 2)] * 4 + [30] * 4 + [50, -1, max(1, V // 2), -1]   # the fourth four: the nucleus ends far above the k-th token
+    ps = [1.0] * 8 + [0.8] * 4 + [0.3] * 4 + [0.97] * 4 + [1.0, 0.9, 0.9, 0.9]
     top_k, top_p = torch.tensor(ks, dtype=torch.int32, device=DEV), torch.tensor(ps, device=DEV)
     seeds = torch.arange(n, dtype=torch.int64, device=DEV) + 11
-    draws = torch.arange(n, dtype=torch.int64, device=DEV)
-    got = ops.sample(logits, temps, top_k, top_p, seeds, draws)
+    each = torch.arange(n, device=DEV).repeat_interleave(draws_each)
+    draws = torch.arange(draws_each, dtype=torch.int64, device=DEV).repeat(n)
+    args = temps[each], top_k[each], top_p[each], seeds[each]
+    got = ops.sample(logits[each], *args, draws).view(n, draws_each)
     for i in range(n):
         one = slice(i, i + 1)
         both = ks[i] > 0 and ps[i] < 1.0
-        alone = ops.sample(logits[one].contiguous(), temps[one], top_k[one], top_p[one], seeds[one], draws[one],
+        alone = ops.sample(logits[one].contiguous(), temps[one], top_k[one], top_p[one], seeds[one], draws[:1],
                            any_top_k=ks[i] > 0, any_top_p=ps[i] < 1.0, any_both=both)
-        assert int(alone) == int(got[i])
+        assert int(alone) == int(got[i, 0])
         if float(temps[i]) == 0.0:
-            assert int(got[i]) == int(logits[i].argmax())
+            assert bool((got[i] == logits[i].argmax()).all())
             continue
-        probs = plain.sampling_probs(logits[i].cpu(), float(temps[i]), ks[i], ps[i])
-        want, margin = plain.draw(probs, plain.uniform01(int(seeds[i]), int(draws[i])))
-        # the plain nucleus takes equal tokens in the order of a sort, ours keeps all that equal its last one
-        if kind != "steps" or ps[i] == 1.0:
-            assert int(got[i]) == want or margin < 1e-4, f"row {i}: got {int(got[i])}, plain draws {want} ({margin})"
+        # weights are float32 exponentials (a few units of 2^-24 each, so that running sums of up to 151,936 of them are off by less
+        # than 1e-6 of the whole) and rounded down to 2^-40; a nucleus that ends within 1e-6 of p may end on either side
+        ways = [_kept_cdf(logits[i], temps[i], ks[i], float(top_p[i]), slack) for slack in (-1e-6, 1e-6)]
+        for d, token in enumerate(got[i].tolist()):
+            u = plain.uniform01(int(seeds[i]), d)
+            assert any(bool(keep[token]) and (0.0 if token == 0 else float(cdf[token - 1])) - 2e-6 <= u <= float(cdf[token]) + 2e-6
+                       for keep, cdf in ways), (i, d, token, u)
     many = 300
-    if V <= 40000:
+    if V <= 40001:
         rows = torch.arange(many, device=DEV) % n
-        again = ops.sample(logits[rows], temps[rows], top_k[rows], top_p[rows], seeds[rows], draws[rows])
-        assert torch.equal(again, got[rows])
+        again = ops.sample(logits[rows], temps[rows], top_k[rows], top_p[rows], seeds[rows], draws[:1].expand(many).contiguous())
+        assert torch.equal(again, got[rows, 0])
+
+
+def test_sampling_takes_as_long_for_flat_and_peaked_rows():
+    """The bins follow the row's spread: rows that are nearly flat, rows far apart and masked rows take the time of
+    others. (A row whose bin did not fit its list took 15 to 40 times as long.)"""
+    from clockwork_amd import ops
+
+    V, rows = 151936, 8
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    noise = torch.randn(rows, V, device=DEV, generator=gen)
+    masked = torch.where(torch.rand(rows, V, device=DEV, generator=gen) < 0.01, 3.0 * noise, -float("inf"))
+
+    def us(logits, temperature, k, p):
+        full = lambda v, dtype=torch.float32: torch.full((rows,), v, dtype=dtype, device=DEV)  # noqa: E731
+        args = (logits, full(temperature), full(k, torch.int32), full(p), torch.arange(rows, device=DEV), torch.zeros(rows, dtype=torch.int64, device=DEV))
+        ops.sample(*args)
+        times = []
+        for _ in range(15):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            for _ in range(5):
+                ops.sample(*args)
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end) * 200)
+        return sorted(times)[len(times) // 2]
+
+    for k, p in ((-1, 0.9), (50, 1.0), (V // 2, 1.0), (V // 2, 0.9)):
+        usual = us(3.0 * noise, 1.0, k, p)
+        for logits, temperature in ((0.02 * noise, 1.0), (0.4 * noise, 1.0), (3.0 * noise, 5.0), (3.0 * noise, 0.05), (masked, 1.0)):
+            assert us(logits, temperature, k, p) < 4 * usual, (k, p, temperature)
 
 
 # rows and columns that end inside a tile, one tile, K of a single stage a run, runs of unequal length, every tile size
