@@ -873,8 +873,8 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(SampleArgs 
   sample_locate(a, row, temp, mx, mi, floor_key, chunk_w);
 }
 
-// flags: bit 0 some row may have top-k, bit 1 some row may have top-p, bit 2 some row may have both (7 when
-// unknown): the steps no row needs are not launched. workspace: cw_sample_workspace_bytes(n, V) bytes, 16-byte
+// flags: bit 0 some row may have top-k, bit 1 some row may have top-p (3 when unknown), bit 2 no row has both: the steps
+// no row needs are not launched. workspace: cw_sample_workspace_bytes(n, V) bytes, 16-byte
 // aligned.
 CW_EXPORT int cw_sample(const float* logits, int64_t row_stride, int n, int V,
                         const float* temperature, const int* top_k, const float* top_p,
@@ -912,7 +912,7 @@ CW_EXPORT int cw_sample(const float* logits, int64_t row_stride, int n, int V,
     hipLaunchKernelGGL(sample_collect_kernel, grid, block, 0, stream, a, 0);
   }
   hipLaunchKernelGGL(sample_draw_kernel, dim3(n), block, 0, stream, a, 0);
-  if ((flags & 7) == 7) {
+  if ((flags & 7) == 3) {
     hipLaunchKernelGGL(sample_collect_kernel, grid, block, 0, stream, a, 1);
     hipLaunchKernelGGL(sample_draw_kernel, dim3(n), block, 0, stream, a, 1);
   }

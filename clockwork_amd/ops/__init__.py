@@ -1385,7 +1385,7 @@ def sample(logits, temperature, top_k, top_p, seeds, draws, out=None, any_top_k:
     ws = torch.empty(int(lib.cw_sample_workspace_bytes(n, V)), dtype=torch.uint8, device=logits.device)
     _check(
         lib.cw_sample(_ptr(logits), V, n, V, _ptr(temperature), _ptr(top_k), _ptr(top_p), _ptr(seeds), _ptr(draws),
-                      _ptr(out), _ptr(ws), ws.numel(), int(bool(any_top_k)) | (int(bool(any_top_p)) << 1) | (int(bool(any_both)) << 2), _stream()),
+                      _ptr(out), _ptr(ws), ws.numel(), int(bool(any_top_k)) | (int(bool(any_top_p)) << 1) | (int(not any_both) << 2), _stream()),
         "sample",
     )
     return out

@@ -124,6 +124,23 @@ def test_sampling_lists_bins_and_chunks(V, kind):
         assert torch.equal(again, got[rows, 0])
 
 
+def test_sampling_with_flags_that_say_nothing():
+    """The C entry's flags 3, some row may have top-k and some top-p: rows with both are drawn too."""
+    from clockwork_amd import ops
+
+    V, n = 5000, 4
+    logits = 3.0 * torch.randn(n, V, device=DEV, generator=torch.Generator(device=DEV).manual_seed(2))
+    temps, ps = torch.ones(n, device=DEV), torch.full((n,), 0.3, device=DEV)
+    ks = torch.full((n,), V // 2, dtype=torch.int32, device=DEV)   # the nucleus ends far above the k-th token
+    seeds, draws = (torch.arange(n, dtype=torch.int64, device=DEV) for _ in range(2))
+    out = torch.full((n,), -7, dtype=torch.int32, device=DEV)
+    lib = ops._load("sampling")
+    ws = torch.empty(int(lib.cw_sample_workspace_bytes(n, V)), dtype=torch.uint8, device=DEV)
+    args = (ops._ptr(t) for t in (temps, ks, ps, seeds, draws, out, ws))
+    assert lib.cw_sample(ops._ptr(logits), V, n, V, *args, ws.numel(), 3, ops._stream()) == 0
+    assert torch.equal(out, ops.sample(logits, temps, ks, ps, seeds, draws)) and bool((out >= 0).all())
+
+
 def test_sampling_takes_as_long_for_flat_and_peaked_rows():
     """The bins follow the row's spread: rows that are nearly flat, rows far apart and masked rows take the time of
     others. (A row whose bin did not fit its list took 15 to 40 times as long.)"""
