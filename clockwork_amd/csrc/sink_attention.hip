@@ -708,8 +708,10 @@ __global__ __launch_bounds__(256) void sink_decode_runs_kernel(SinkDecodeParams 
       for (int i = 0; i < 4; ++i) m[i] = fmaxf(m[i], __shfl_xor(m[i], off, 64));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      sv[i][0] = expf(sv[i][0] - m[i]);
-      sv[i][1] = expf(sv[i][1] - m[i]);
+      // a run whose scores are all -inf weighs nothing; a NaN among them stays one, up to the result
+      const float from = m[i] == -INFINITY ? 0.0f : m[i];
+      sv[i][0] = expf(sv[i][0] - from);
+      sv[i][1] = expf(sv[i][1] - from);
       l[i] = sv[i][0] + sv[i][1];
     }
 #pragma unroll
@@ -787,15 +789,16 @@ __global__ __launch_bounds__(1024) void sink_decode_mix_kernel(SinkDecodeParams 
     float m = sink;
     for (int s = lane; s < runs; s += 64) m = fmaxf(m, st[s * H + g].x);
     m = cw_wave_max(m);
+    const float from = m == -INFINITY ? 0.0f : m;
     float l = 0.0f;
     for (int s = lane; s < runs; s += 64) {
       const float2 ml = st[s * H + g];
-      const float w = expf(ml.x - m);
+      const float w = expf(ml.x - from);
       coef[g * p.n_runs + s] = w;
       l += ml.y * w;
     }
     l = cw_wave_sum(l);
-    if (p.sink) l += expf(sink - m);
+    if (p.sink) l += expf(sink - from);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
     float sum = 0.0f;
     for (int s0 = 0; s0 < runs; s0 += 8) {
@@ -807,7 +810,7 @@ __global__ __launch_bounds__(1024) void sink_decode_mix_kernel(SinkDecodeParams 
       for (int u = 0; u < 8; ++u)
         if (s0 + u < runs) sum += coef[g * p.n_runs + s0 + u] * x[u];
     }
-    X[g * 64 + lane] = l > 0.0f ? sum * (1.0f / l) : 0.0f;
+    X[g * 64 + lane] = l == 0.0f ? 0.0f : sum * (1.0f / l);
   }
   __syncthreads();
   T* out = (T*)p.out + (int64_t)p.cu_q[r] * H * V + dv;

@@ -413,6 +413,40 @@ def test_sink_decode_runs(heads, kv, dim, vdim, talk, sk, dtype):
         torch.testing.assert_close(out[r].to(f64), want, **tol)
 
 
+@pytest.mark.parametrize("talk", [False, True])
+def test_sink_decode_of_scores_that_are_no_numbers(talk):
+    """A NaN reaches the result of its request (with mixing, of every head) and no other; keys whose scores are -inf weigh
+    nothing, a whole run of them as well."""
+    from clockwork_amd import ops
+
+    heads, kv, dim, n, bs, sk = 4, 2, 32, 100, 16, 32
+    gen = torch.Generator(device=DEV).manual_seed(6)
+    pages = -(-n // bs)
+    tables = torch.arange(3 * pages, dtype=torch.int32, device=DEV).view(3, pages)
+    k, v = (torch.randn(3 * pages, bs, kv, dim, device=DEV, generator=gen) for _ in range(2))
+    q = torch.rand(3, heads * dim, device=DEV, generator=gen) + 0.5
+    q[0, 0] = float("nan")                     # head 0 of request 0
+    k[pages:pages + 3] = -float("inf")         # the first 48 keys of request 1: a run and a half
+    mix = torch.eye(heads, device=DEV) + 0.2 if talk else None
+    out = torch.zeros(3, heads * dim, device=DEV)
+    ints = lambda t: torch.as_tensor(t, dtype=torch.int32, device=DEV)  # noqa: E731
+    ops.sink_attention_decode(q, heads * dim, out, k, v, tables, ints([n] * 3), ints(range(4)), 3, sk, -(-n // sk), None, None, None, mix,
+                              heads, kv, dim, dim, bs, 0, dim ** -0.5)
+    assert bool(torch.isnan(out[0] if talk else out[0, :dim]).all()) and bool(torch.isfinite(out[1:]).all())
+    for r, first in ((0, 0), (1, 48), (2, 0)):
+        keys, values = (t[r * pages:(r + 1) * pages].reshape(-1, kv, dim)[first:n].double().repeat_interleave(2, 1) for t in (k, v))
+        p = torch.softmax((q[r].double().view(heads, 1, dim) * keys.transpose(0, 1)).sum(-1) * dim ** -0.5, 1)
+        p = mix.double() @ p if talk else p
+        want = (p[:, :, None] * values.transpose(0, 1)).sum(1).view(-1)
+        if r == 0:
+            if talk:
+                continue
+            want, got = want[dim:], out[r, dim:]
+        else:
+            got = out[r]
+        torch.testing.assert_close(got.double(), want, atol=2e-5, rtol=2e-5)   # float32 sums of 100 terms of a few units
+
+
 # rows of the streaming kernels (one and several), of the tiles between and of the wide tiles; sizes that each takes
 @pytest.mark.parametrize("M,K,I", [(1, 96, 64), (8, 1536, 8960), (33, 256, 512), (130, 1536, 8960), (400, 1536, 8960), (1100, 1536, 8960), (9, 100, 36)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
