@@ -830,7 +830,7 @@ static bool sd_two(int n_runs, int heads, int kv_heads, bool mixed) {
   return (!mixed || kv_heads <= SD_MIXED_GROUPS) && heads <= 64 && (int64_t)heads * n_runs <= SD_COEF_FLOATS;
 }
 
-// floats of workspace for R single tokens whose keys are cut into n_runs runs of sk keys
+// floats of workspace (8-byte aligned) for R single tokens whose keys are cut into n_runs runs of sk keys
 CW_EXPORT int64_t cw_sink_decode_workspace_floats(int n_requests, int n_runs, int sk, int heads, int kv_heads, int vdim,
                                                   int mixed) {
   if (kv_heads > 0 && sd_two(n_runs, heads, kv_heads, mixed != 0))
@@ -865,7 +865,8 @@ CW_EXPORT int cw_sink_decode(int dtype, const void* q, int64_t q_stride, void* o
   p.q = q; p.q_stride = q_stride; p.out = out; p.k_cache = k_cache; p.v_cache = v_cache;
   p.block_tables = block_tables; p.table_width = table_width; p.ctx_lens = ctx_lens; p.cu_q = cu_q;
   p.r1 = r1; p.r2 = r2; p.sink = sink; p.talk = talk;
-  const bool two = sd_two(n_runs, heads, kv_heads, talk != nullptr) && !((uintptr_t)workspace & 7);
+  if ((uintptr_t)workspace & 7) return CW_ERR_ARG;  // (pairs of floats are read from it, and its size is not passed in)
+  const bool two = sd_two(n_runs, heads, kv_heads, talk != nullptr);
   p.scores = workspace;
   p.stats = two ? workspace : p.scores + (int64_t)n_requests * heads * n_runs * sk;
   p.partial = p.stats + (int64_t)n_requests * n_runs * heads * 2;

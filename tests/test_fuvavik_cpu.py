@@ -224,3 +224,15 @@ def test_plain_recurrence_against_its_closed_form():
     gate = x @ w["g"].t()
     want = (o.reshape(T, H * V) * gate * torch.sigmoid(gate)) @ w["o"].t()
     torch.testing.assert_close(got, want, rtol=1e-10, atol=1e-10)
+
+
+def test_a_workspace_that_is_not_aligned_is_refused_before_any_launch():
+    """The number of kernels is a rule on the sizes alone, the one that the workspace was sized by."""
+    from clockwork_amd import ops
+
+    lib = ops._load("sink_attention")
+
+    def call(workspace):
+        return lib.cw_sink_decode(0, 64, 128, 64, 64, 64, 32, 64, 2, 64, 64, 1, 32, 1, workspace, None, None, None, None, 4, 2, 32, 32, 16, 0, 1.0, None)
+
+    assert call(4) == -1 and call(12) == -1
