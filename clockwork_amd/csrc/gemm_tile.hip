@@ -949,23 +949,39 @@ static float mid_time(int M, int N, int K, int bm, int bn, int planes, int cus) 
 
 // Which of this file's kernels a product of many rows should run on: 0 the library's, else bm | bn << 10 |
 // planes << 20 (bm 256: cw_gemm_bf16_wide_partial, else cw_gemm_bf16_mid). mode as there.
-// Where the lines lie, measured for the layers of the 0.5B, 1.5B, 3B and 7B shapes with 72 to 2048 rows:
-//  * mode 3 (a sum that the next norm adds up): K of three times N and more, up to 2048 rows: here everywhere (but for
-//    4 % at 1536 rows of the 3B shape). A squarer matrix while M N is below 1.2 M: beyond, the planes cost more than
-//    the library's idle units.
-//  * mode 2: M N K up to 4.5e9 (72 rows of the 1.5B shape: 28.0 -> 22.9 us, 208 rows 32.2 -> 31.8), and up to 690 rows for
-//    a matrix of at most 9 M elements.
-//  * mode 0: matrices of at most 2 M elements and up to 1536 rows (q/k/v of the 0.5B shape: 8.1 -> 6.3 us for 144 rows), or of
-//    4 M and 320 to 1024 (of the 1.5B shape: 14.3 -> 12.8 for 1000; 8.6 -> 8.8 for 144).
+// Where the lines lie, measured with operands from memory, 72 to 2048 rows, for the layers of the 0.5B to 72B shapes
+// and for outputs of 16 to 4096 columns with K of 256 to 16384 (us, library -> here):
+//  * mode 3 (a sum that the next norm adds up): K of three times N and more. The library's product of that kind leaves
+//    units idle (32B shape's down product, 256 rows 275 -> 116, 1536 rows 565 -> 384) until M N is large: 8 M (2048 rows
+//    of the 32B shape 484 -> 513), 2.1 M for outputs of more than 5120 columns (72B shape, 256 rows 293 -> 177, 640 rows
+//    302 -> 370). Beyond 1024 rows and columns on the wide tiles only (3B shape's down product, 1434 rows 98 -> 115 on
+//    the small ones), which have to fill their rounds (7B shape, 1600 rows in 2.08 rounds 241 -> 273, 2048 in 2.4 386 ->
+//    292); beyond 640 rows not as whole sums of K (2048 x 6144, 1000 rows 49.4 -> 54.5). A squarer matrix
+//    while M N is below 1.2 M and N at most 5120: beyond, the planes cost more than the library's idle units.
+//  * mode 2: M N K up to 4.5e9 (72 rows of the 1.5B shape: 28.0 -> 22.9 us, 208 rows 32.2 -> 31.8), and up to 640 rows for
+//    a matrix of at most 9 M elements; a K of more than 1024 and half of N is a narrow output's (896 x 4864, 165 rows
+//    15.0 -> 20.6).
+//  * mode 0 (whole sums of K on 64 x 64 tiles, 0.21 us a stage): a long K is summed faster by the library in parts (64 x
+//    4096, 144 rows 11.6 -> 16.8), so K up to 512, up to 896 for 1024 columns and more (q/k/v of the 0.5B shape 8.0 ->
+//    6.4 for 144 rows; 512 columns 5.3 -> 6.1), while a compute unit has three tiles or so (4096 x 896, 400 rows 10.6 ->
+//    8.4, 700 rows 11.3 -> 12.1); and K up to 1536 for 1536 columns and more, 320 to 1024 rows (q/k/v of the 1.5B shape
+//    14.0 -> 12.7 for 1000, 8.6 -> 8.8 for 144).
 CW_EXPORT int cw_gemm_bf16_mid_choice(int mode, int M, int N, int K, int64_t ldx, int cus) {
   if (M <= 64 || M > 2048 || N <= 0 || K < 256 || (K & 63) || (ldx & 7) || ldx < K || cus < 8) return 0;
   if ((int64_t)N * K * 2 >= (1ll << 32) || ((int64_t)M * ldx + 128 * ldx) * 2 >= (1ll << 32)) return 0;
-  const int64_t elements = (int64_t)N * K;
-  if (mode == 0)
-    return (elements <= 2 << 20 && M <= 1536) || (elements <= 4 << 20 && M >= 320 && M <= 1024) ? 64 | 64 << 10 | 1 << 20 : 0;
+  const int64_t elements = (int64_t)N * K, outputs = (int64_t)M * N;
+  if (mode == 0) {
+    const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
+    const bool short_k = M <= 1536 && N >= 32 && (K <= 512 || (K <= 896 && N >= 1024)) && tiles <= 1000 && tiles * K <= 600000;
+    const bool qkv = K > 896 && K <= 1536 && N >= 1536 && elements <= 4 << 20 && M >= 320 && M <= 1024;
+    return short_k || qkv ? 64 | 64 << 10 | 1 << 20 : 0;
+  }
   if (mode == 2) {
-    if ((N & 1) || !((int64_t)M * elements <= 4500000000ll || (elements <= 9 << 20 && M <= 690))) return 0;
-  } else if (mode != 3 || !(K >= 3 * N || (int64_t)M * N <= 1200000)) {
+    if ((N & 1) || (N < 2 * K && K > 1024) || !((int64_t)M * elements <= 4500000000ll || (elements <= 9 << 20 && M <= 640))) return 0;
+  } else if (mode == 3) {
+    const int64_t most = K >= 3 * N ? (N <= 5120 ? 8000000 : 2100000) : N <= 5120 ? 1200000 : 0;
+    if (outputs > most) return 0;
+  } else {
     return 0;
   }
   int best = 0;
@@ -985,5 +1001,12 @@ CW_EXPORT int cw_gemm_bf16_mid_choice(int mode, int M, int N, int K, int64_t ldx
         least = mid_time(M, N, K, W_BM, W_BN, planes, cus);
         best = W_BM | W_BN << 10 | planes << 20;
       }
+  if (mode == 3) {
+    const int planes = best >> 20;
+    if (planes == 1 && M > 640 && N >= 512 && K >= 3 * N) return 0;
+    if ((best & 1023) != W_BM) return M > 1024 && N >= 1024 ? 0 : best;
+    const int64_t items = (int64_t)((M + W_BM - 1) / W_BM) * ((N + W_BN - 1) / W_BN) * planes;
+    if (items > cus && (float)items < 0.72f * (float)(cus * ((items + cus - 1) / cus))) return 0;
+  }
   return best;
 }
