@@ -578,13 +578,13 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias=None, out_dtype=None, par
         splits = _wide_partial_chosen(x, weight, policy)
         if splits:
             return linear_wide_partial(x, weight, splits)
-    if M > STREAM_MAX_ROWS and x.is_contiguous() and out_dtype is None:
+    if M > STREAM_MAX_ROWS and out_dtype is None and (bias is None or bias.dtype == torch.bfloat16 and tuple(bias.shape) == (N,)):
         if portions_partial_ok and bias is None and not (M >= WIDE_PRODUCT_MIN_ROWS and (N, K) in policy.wide_partial_choices):
-            choice = _load("gemm_tile").cw_gemm_bf16_mid_choice(3, M, N, K, K, _compute_units(x.device))
+            choice = _mid_choice(3, x, weight)
             if choice:
                 return linear_mid(x, weight, choice, partial=True)
-        choice = _load("gemm_tile").cw_gemm_bf16_mid_choice(0, M, N, K, K, _compute_units(x.device))
-        if choice and (bias is None or bias.dtype in (torch.bfloat16, torch.float32)):
+        choice = _mid_choice(0, x, weight)
+        if choice:
             return linear_mid(x, weight, choice, bias=bias)
     if policy.hip_products and K % 8 == 0 and x.is_contiguous():
         y = linear_tiled(x, weight, bias)
@@ -949,6 +949,19 @@ def linear_wide_partial(x: torch.Tensor, weight: torch.Tensor, k_splits: int) ->
     return PartialSums(parts)
 
 
+def _aligned(*tensors) -> bool:
+    """May the kernels of this package that load 16 bytes at a time read these? (The library takes any.)"""
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def _mid_choice(mode: int, x: torch.Tensor, weight: torch.Tensor) -> int:
+    """What ``cw_gemm_bf16_mid_choice`` says of x @ weight.T; 0 for operands that its kernels do not take."""
+    if not _aligned(x, weight):
+        return 0
+    M, K = x.shape
+    return _load("gemm_tile").cw_gemm_bf16_mid_choice(mode, M, weight.shape[0], K, K, _compute_units(x.device))
+
+
 def linear_mid(x: torch.Tensor, weight: torch.Tensor, choice: int, bias=None, swiglu: bool = False, partial: bool = False,
                limit: float = 0.0):
     """x @ weight.T through the tiles for the steps between (csrc/gemm_tile.hip), of the sizes that ``choice`` names
@@ -1134,12 +1147,12 @@ def linear_swiglu(x, gate_up_weight: torch.Tensor, policy: "ProductPolicy | None
                                                   _stream()), "gemm_bf16_skinny(swiglu)")
         return out
     if x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16 and K % 8 == 0 and x.is_contiguous():
-        choice = _load("gemm_tile").cw_gemm_bf16_mid_choice(2, M, two_i, K, K, _compute_units(x.device))
+        choice = _mid_choice(2, x, gate_up_weight)
         if choice:
             return linear_mid(x, gate_up_weight, choice, swiglu=True, limit=limit)
         if policy.hip_products:
             return linear_tiled(x, gate_up_weight, swiglu=True, limit=limit)
-        if wide_swiglu_pays(M, two_i, K, K):
+        if _aligned(x, gate_up_weight) and wide_swiglu_pays(M, two_i, K, K):
             # with enough rows the shape of the weights decides, and a start-up that tunes the
             # library's products has measured it for this model's
             measured = M >= WIDE_SWIGLU_MIN_ROWS

@@ -228,6 +228,40 @@ def test_products_of_a_portion_by_their_rule():
     assert lib.cw_gemm_bf16_mid_choice(3, 144, 1536, 8960 + 32, 8992, 256) == 0   # K no whole number of stages
 
 
+@pytest.mark.parametrize("M", [100, 400])
+def test_operands_that_only_the_library_takes(M):
+    """Rows that do not begin at 16 bytes and biases of other shapes go to the library whatever the rule names for the
+    sizes; a float32 bias, which the library refuses, stays refused."""
+    from clockwork_amd import ops
+
+    N, K = 1152, 512
+    gen = torch.Generator(device=DEV).manual_seed(M)
+    lib = ops._load("gemm_tile")
+    assert all(lib.cw_gemm_bf16_mid_choice(mode, M, N, K, K, 256) for mode in (0, 2, 3))
+    assert ops.wide_swiglu_pays(400, 2 * 8960, 1536, 1536)
+    wide = torch.randn(2 * 8960 * 1536 + 1, device=DEV, generator=gen).to(torch.bfloat16)
+
+    def odd(*shape):
+        return wide[1:1 + math.prod(shape)].view(shape)
+
+    tol = dict(rtol=4 * 2.0 ** -8, atol=2e-2)   # two roundings of up to 2^-8 each side
+    x, w = torch.randn(M, K, device=DEV, generator=gen).to(torch.bfloat16), (torch.randn(N, K, device=DEV, generator=gen) / K ** 0.5).to(torch.bfloat16)
+    for a, b in ((odd(M, K), w), (x, odd(N, K) / K ** 0.5), (odd(M, K), odd(N, K))):
+        b = odd(N, K).copy_(b) if b is not w else b
+        want = a.float() @ b.float().t()
+        for got in (ops.linear(a, b), ops.linear(a, b, partial_ok=True, portions_partial_ok=True)):
+            torch.testing.assert_close(got.float(), want, **tol)
+        g, u = want[:, : N // 2], want[:, N // 2:]
+        torch.testing.assert_close(ops.linear_swiglu(a, b).float(), torch.nn.functional.silu(g) * u, rtol=4 * 2.0 ** -8, atol=0.03 * float((g * u).abs().max()))
+    if M == 400:
+        a, b = torch.randn(M, 1536, device=DEV, generator=gen).to(torch.bfloat16), odd(2 * 8960, 1536)
+        assert ops.linear_swiglu(a, b).shape == (M, 8960)
+    one = torch.full((1,), 3.0, device=DEV, dtype=torch.bfloat16)
+    torch.testing.assert_close(ops.linear(x, w, one).float(), x.float() @ w.float().t() + 3.0, **tol)
+    with pytest.raises(RuntimeError):
+        ops.linear(x, w, torch.zeros(N, device=DEV))
+
+
 # 16 requests at the edges of a wave's tile of 32 keys, of the turns of four and eight waves and of the line where
 # eight take over (128 keys a split); 24 keys a page and 16; a group of more than 16 heads
 @pytest.mark.parametrize("hd,nh,nkv,bs", [(32, 4, 2, 16), (64, 14, 2, 16), (96, 6, 3, 24), (128, 12, 2, 16), (128, 20, 1, 24), (160, 4, 2, 16)])
