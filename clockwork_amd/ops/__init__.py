@@ -607,8 +607,8 @@ class ProductPolicy:
     ``hip_products``: such products go through this package's own LDS-tiled kernels instead of the
     library (about half as fast on an MI355X; for a run that must not depend on the library).
     ``swiglu_choices`` / ``product_choices``: for a weight shape that a tuning start-up has timed
-    both ways, whether the wide-tile kernel was the faster one ((rows of [gate; up], K) and
-    (N, K, with bias)); shapes never timed follow the fixed rules. ``k_split_choices``: for an
+    both ways, whether the wide-tile kernel was the faster one ((rows of [gate; up], K, and the activation
+    if that is not silu) and (N, K, with bias)); shapes never timed follow the fixed rules. ``k_split_choices``: for an
     (N, K) whose product of few rows is summed in parts over K (a narrow output with a long K),
     the number of parts that start-up found the fastest, the same for every step of up to 16 rows.
     ``wide_partial_choices``: for an (N, K) of a long portion's product with a narrow output and a
@@ -1055,12 +1055,23 @@ def _measure_k_splits(x: torch.Tensor, weight: torch.Tensor, default: int) -> in
     return best if times[best] < 0.97 * times[default] else default
 
 
-def _measure_swiglu(x: torch.Tensor, gate_up_weight: torch.Tensor, out: torch.Tensor) -> bool:
+def _swiglu_key(two_i: int, K: int, limit: float) -> tuple:
+    """The entry of ``ProductPolicy.swiglu_choices`` for a gated product: its sizes, and its activation if that is not
+    silu (a gate's kernel and its epilogue cost what their activation costs)."""
+    return (two_i, K) if limit == 0.0 else (two_i, K, 1 if limit > 0.0 else int(limit))
+
+
+def _gate(gate_up: torch.Tensor, out: torch.Tensor, limit: float) -> torch.Tensor:
+    """The gate kernel of ``linear_swiglu``'s activation ``limit``."""
+    return gelu_tanh_mul(gate_up, out) if limit == GELU_GATE else silu_mul(gate_up, out, limit)
+
+
+def _measure_swiglu(x: torch.Tensor, gate_up_weight: torch.Tensor, out: torch.Tensor, limit: float = 0.0) -> bool:
     """Time the two ways of a long portion's gate/up product on these operands (the library has
     just chosen its kernel for the shape): is this package's kernel at least as fast as the
     library's product followed by the gate kernel?"""
-    library = _timed_us(lambda: silu_mul(_library_product(x, gate_up_weight, None), out))
-    own = _timed_us(lambda: linear_tiled(x, gate_up_weight, swiglu=True, wide=True))
+    library = _timed_us(lambda: _gate(_library_product(x, gate_up_weight, None), out, limit))
+    own = _timed_us(lambda: linear_tiled(x, gate_up_weight, swiglu=True, wide=True, limit=limit))
     return own <= library
 
 
@@ -1155,14 +1166,12 @@ def linear_swiglu(x, gate_up_weight: torch.Tensor, policy: "ProductPolicy | None
         if _aligned(x, gate_up_weight) and wide_swiglu_pays(M, two_i, K, K):
             # with enough rows the shape of the weights decides, and a start-up that tunes the
             # library's products has measured it for this model's
-            measured = M >= WIDE_SWIGLU_MIN_ROWS
-            if (measured and policy.tuning and (two_i, K) not in policy.swiglu_choices
-                    and policy.recall("swiglu_choices", (two_i, K)) is None):
-                policy.swiglu_choices[(two_i, K)] = _measure_swiglu(x, gate_up_weight, out)
-            if not measured or policy.swiglu_choices.get((two_i, K), True):
+            measured, key = M >= WIDE_SWIGLU_MIN_ROWS, _swiglu_key(two_i, K, limit)
+            if measured and policy.tuning and key not in policy.swiglu_choices and policy.recall("swiglu_choices", key) is None:
+                policy.swiglu_choices[key] = _measure_swiglu(x, gate_up_weight, out, limit)
+            if not measured or policy.swiglu_choices.get(key, True):
                 return linear_tiled(x, gate_up_weight, swiglu=True, wide=True, limit=limit)
-    gate_up = linear(x, gate_up_weight, policy=policy)
-    return gelu_tanh_mul(gate_up, out) if limit == GELU_GATE else silu_mul(gate_up, out, limit)
+    return _gate(linear(x, gate_up_weight, policy=policy), out, limit)
 
 
 _zero_rows: dict = {}

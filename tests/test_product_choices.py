@@ -2,6 +2,8 @@
 
 import json
 
+import pytest
+
 from clockwork_amd import ops
 
 
@@ -78,3 +80,23 @@ def test_the_card_is_known_by_more_than_its_name(monkeypatch):
     assert made_for[:3] == ["gfx950:sramecc+:xnack-", 256, 1 << 38]
     monkeypatch.setattr(torch.cuda, "get_device_properties", lambda d: card("gfx950:sramecc+:xnack-", 128))
     assert ops._choices_made_for() != made_for and ops.choices_file() != path
+
+
+@pytest.mark.parametrize("limit", [0.0, 7.0, ops.RELU_GATE, ops.GELU_GATE])
+def test_a_gated_product_is_timed_and_kept_with_its_own_activation(monkeypatch, tmp_path, limit):
+    ran = []
+    monkeypatch.setattr(ops, "_timed_us", lambda fn: fn() or 1.0)
+    monkeypatch.setattr(ops, "_library_product", lambda *a: ran.append("product"))
+    monkeypatch.setattr(ops, "silu_mul", lambda gate_up, out, limit=0.0: ran.append(("gate", limit)))
+    monkeypatch.setattr(ops, "gelu_tanh_mul", lambda gate_up, out: ran.append(("gate", ops.GELU_GATE)))
+    monkeypatch.setattr(ops, "linear_tiled", lambda *a, limit=0.0, **k: ran.append(("own", limit)))
+    assert ops._measure_swiglu(None, None, None, limit)
+    assert ran == ["product", ("gate", limit), ("own", limit)]
+    # another activation's choice for the same sizes is not taken, also behind a file
+    policy, path = ops.ProductPolicy(), str(tmp_path / "choices.json")
+    policy.swiglu_choices[ops._swiglu_key(17920, 1536, limit)] = False
+    policy.write_choices(path)
+    later = ops.ProductPolicy()
+    assert later.read_choices(path) == 1
+    for other in (0.0, 7.0, ops.RELU_GATE, ops.GELU_GATE):
+        assert (later.recall("swiglu_choices", ops._swiglu_key(17920, 1536, other)) is False) == (other == limit)
