@@ -580,10 +580,10 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias=None, out_dtype=None, par
             return linear_wide_partial(x, weight, splits)
     if M > STREAM_MAX_ROWS and out_dtype is None and (bias is None or bias.dtype == torch.bfloat16 and tuple(bias.shape) == (N,)):
         if portions_partial_ok and bias is None and not (M >= WIDE_PRODUCT_MIN_ROWS and (N, K) in policy.wide_partial_choices):
-            choice = _mid_choice(3, x, weight)
+            choice = _mid_choice(3, x, weight, policy)
             if choice:
                 return linear_mid(x, weight, choice, partial=True)
-        choice = _mid_choice(0, x, weight)
+        choice = _mid_choice(0, x, weight, policy, bias=bias)
         if choice:
             return linear_mid(x, weight, choice, bias=bias)
     if policy.hip_products and K % 8 == 0 and x.is_contiguous():
@@ -613,12 +613,14 @@ class ProductPolicy:
     the number of parts that start-up found the fastest, the same for every step of up to 16 rows.
     ``wide_partial_choices``: for an (N, K) of a long portion's product with a narrow output and a
     long K, into how many runs of K the wide-tile kernel sums it (0: the library's product stays).
+    ``mid_choices``: for a product of so many rows that the tiles between would serve by their rule ((mode, rows, N, K), the
+    activation behind it as in ``swiglu_choices``), whether they were as fast as the library's tuned product.
     ``tuning``: such a start-up is under way (``library_tuning``)."""
 
-    __slots__ = ("hip_products", "swiglu_choices", "product_choices", "k_split_choices", "wide_partial_choices", "tuning",
-                 "_remembered")
+    __slots__ = ("hip_products", "swiglu_choices", "product_choices", "k_split_choices", "wide_partial_choices", "mid_choices",
+                 "tuning", "_remembered")
 
-    TABLES = ("swiglu_choices", "product_choices", "k_split_choices", "wide_partial_choices")
+    TABLES = ("swiglu_choices", "product_choices", "k_split_choices", "wide_partial_choices", "mid_choices")
 
     def __init__(self, hip_products: bool = False) -> None:
         self.hip_products = bool(hip_products)
@@ -626,6 +628,7 @@ class ProductPolicy:
         self.product_choices: dict = {}
         self.k_split_choices: dict = {}
         self.wide_partial_choices: dict = {}
+        self.mid_choices: dict = {}
         self.tuning = False
         self._remembered: dict = {name: {} for name in self.TABLES}
 
@@ -954,12 +957,41 @@ def _aligned(*tensors) -> bool:
     return all(t.data_ptr() % 16 == 0 for t in tensors)
 
 
-def _mid_choice(mode: int, x: torch.Tensor, weight: torch.Tensor) -> int:
-    """What ``cw_gemm_bf16_mid_choice`` says of x @ weight.T; 0 for operands that its kernels do not take."""
+def _mid_choice(mode: int, x: torch.Tensor, weight: torch.Tensor, policy: ProductPolicy, bias=None, limit: float = 0.0) -> int:
+    """What ``cw_gemm_bf16_mid_choice`` says of x @ weight.T; 0 for operands that its kernels do not take, and where a tuning
+    start-up has timed this very number of rows and found the library's tuned product the faster one."""
     if not _aligned(x, weight):
         return 0
     M, K = x.shape
-    return _load("gemm_tile").cw_gemm_bf16_mid_choice(mode, M, weight.shape[0], K, K, _compute_units(x.device))
+    N = weight.shape[0]
+    choice = _load("gemm_tile").cw_gemm_bf16_mid_choice(mode, M, N, K, K, _compute_units(x.device))
+    if choice and (policy.tuning or policy.mid_choices):
+        key = (mode, M, *_swiglu_key(N, K, limit))
+        if policy.tuning and key not in policy.mid_choices and policy.recall("mid_choices", key) is None:
+            policy.mid_choices[key] = _measure_mid(mode, choice, x, weight, bias, limit)
+        if not policy.mid_choices.get(key, True):
+            return 0
+    return choice
+
+
+def _measure_mid(mode: int, choice: int, x: torch.Tensor, weight: torch.Tensor, bias, limit: float) -> bool:
+    """Are the tiles between as fast as the library's product on these operands, each with the kernel that follows
+    it (for partial sums the norm that adds them, for a gated product the gate kernel)?"""
+    M, N = x.shape[0], weight.shape[0]
+    if mode == 3:
+        resid = torch.zeros((M, N), dtype=torch.float32, device=x.device)
+        norm_weight = torch.ones(N, dtype=torch.bfloat16, device=x.device)
+        out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+        library = lambda: add_rmsnorm(resid, _library_product(x, weight, None), norm_weight, 1e-6, out, write_back=False)  # noqa: E731
+        own = lambda: add_rmsnorm(resid, linear_mid(x, weight, choice, partial=True), norm_weight, 1e-6, out, write_back=False)  # noqa: E731
+    elif mode == 2:
+        out = torch.empty((M, N // 2), dtype=torch.bfloat16, device=x.device)
+        library = lambda: _gate(_library_product(x, weight, None), out, limit)  # noqa: E731
+        own = lambda: linear_mid(x, weight, choice, swiglu=True, limit=limit)  # noqa: E731
+    else:
+        library = lambda: _library_product(x, weight, bias)  # noqa: E731
+        own = lambda: linear_mid(x, weight, choice, bias=bias)  # noqa: E731
+    return _timed_us(own) <= _timed_us(library)
 
 
 def linear_mid(x: torch.Tensor, weight: torch.Tensor, choice: int, bias=None, swiglu: bool = False, partial: bool = False,
@@ -1158,7 +1190,7 @@ def linear_swiglu(x, gate_up_weight: torch.Tensor, policy: "ProductPolicy | None
                                                   _stream()), "gemm_bf16_skinny(swiglu)")
         return out
     if x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16 and K % 8 == 0 and x.is_contiguous():
-        choice = _mid_choice(2, x, gate_up_weight)
+        choice = _mid_choice(2, x, gate_up_weight, policy, limit=limit)
         if choice:
             return linear_mid(x, gate_up_weight, choice, swiglu=True, limit=limit)
         if policy.hip_products:

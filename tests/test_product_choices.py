@@ -3,6 +3,7 @@
 import json
 
 import pytest
+import torch
 
 from clockwork_amd import ops
 
@@ -68,8 +69,6 @@ def test_the_card_is_known_by_more_than_its_name(monkeypatch):
     another file."""
     import types
 
-    import torch
-
     def card(arch, units):
         return types.SimpleNamespace(name="", gcnArchName=arch, multi_processor_count=units, total_memory=1 << 38)
 
@@ -100,3 +99,29 @@ def test_a_gated_product_is_timed_and_kept_with_its_own_activation(monkeypatch, 
     assert later.read_choices(path) == 1
     for other in (0.0, 7.0, ops.RELU_GATE, ops.GELU_GATE):
         assert (later.recall("swiglu_choices", ops._swiglu_key(17920, 1536, other)) is False) == (other == limit)
+
+
+def test_the_tiles_between_leave_a_product_that_was_timed_to_the_library(monkeypatch, tmp_path):
+    """A tuning start-up times the rule's kernel against the library's tuned product, for the rows that it runs with;
+    the faster one stays, also behind a file, and other numbers of rows follow the rule."""
+    timed = []
+    monkeypatch.setattr(ops, "_compute_units", lambda device: 256)
+    monkeypatch.setattr(ops, "_measure_mid", lambda mode, choice, x, weight, bias, limit: timed.append((mode, x.shape[0], limit)) or False)
+    rows = {m: torch.zeros(m, 896, dtype=torch.bfloat16) for m in (128, 160)}
+    weight, path = torch.zeros(1152, 896, dtype=torch.bfloat16), str(tmp_path / "choices.json")
+    policy = ops.ProductPolicy()
+    by_rule = ops._mid_choice(0, rows[128], weight, policy)
+    assert by_rule and not timed
+    policy.tuning = True
+    for _ in range(2):
+        assert ops._mid_choice(0, rows[128], weight, policy) == 0
+    assert ops._mid_choice(2, rows[128], weight, policy, limit=ops.GELU_GATE) == 0
+    assert timed == [(0, 128, 0.0), (2, 128, ops.GELU_GATE)]
+    policy.tuning = False
+    assert ops._mid_choice(0, rows[128], weight, policy) == 0 and ops._mid_choice(0, rows[160], weight, policy) == by_rule
+    assert ops._mid_choice(2, rows[128], weight, policy) != 0     # another activation: not timed
+    policy.write_choices(path)
+    later = ops.ProductPolicy()
+    assert later.read_choices(path) == 2 and ops._mid_choice(0, rows[128], weight, later) == by_rule   # (not in use before it asks)
+    later.tuning = True
+    assert ops._mid_choice(0, rows[128], weight, later) == 0 and len(timed) == 2
