@@ -755,15 +755,17 @@ WIDE_MIN_TILES = 64
 # where it beats the library product followed by the gate kernel. Measured on an MI355X over the
 # Qwen2.5 layer shapes from 0.5B to 72B with 256 to 4096 rows: with 180 tiles or more and 1024 rows or
 # more it is 5 to 25 % faster. With fewer rows it is for weights of at most 64 M elements where its tiles fill seven
-# tenths of their rounds over the compute units (us, library and gate against this: 1.5B shape, 400 rows, 188 tiles
-# 41.5 / 36.1; 640 rows, 282 tiles 52.4 / 68.3; 1000 rows, 376 tiles 88.0 / 71.2; 3B shape, 400 rows, 230 tiles 56.4 / 45.1;
-# 7B shape, 400 rows 144 / 132, 640 rows 184 / 198: there reading W bounds both). Against the library's TUNED choice it wins for
+# tenths of their rounds over the compute units and its rows seven tenths of their tiles (us, library and gate against this:
+# 1.5B shape, 188 tiles of 256 rows, 304 rows 34.8 / 36.4, 368 rows 37.4 / 36.0, 408 rows 38.9 / 36.7, 512 rows 44.5 / 37.3; 282 tiles, 640 rows
+# 53.6 / 68.9; 376 tiles, 1000 rows 88.3 / 71.8; 3B shape, 230 tiles, 304 rows 44.5 / 44.8, 385 rows 55.1 / 45.8; 7B shape, 400 rows
+# 150 / 136, 640 rows 189 / 202: there reading W bounds both). Against the library's TUNED choice it wins for
 # the 0.5B, 1.5B, 3B, 14B and 32B shapes (the 1.5B shape's whole prefill step: 8.9 -> 7.9 ms) and
 # loses 3 % of the step for the 7B and 72B shapes, so a start-up that tunes (``library_tuning``)
 # times both ways on the model's own weights and keeps the faster (``ProductPolicy.swiglu_choices``).
 WIDE_SWIGLU_MIN_TILES = 180
 WIDE_SWIGLU_MIN_ROWS = 1024
-WIDE_SWIGLU_FILL = 0.72
+WIDE_SWIGLU_FILL = 0.71
+WIDE_SWIGLU_TILE_ROWS = 256
 WIDE_SWIGLU_SMALL_WEIGHTS = 64 << 20    # elements of [gate; up]
 
 _cu_counts: dict = {}
@@ -784,13 +786,11 @@ def wide_swiglu_pays(M: int, two_i: int, K: int, ldx: int) -> bool:
     tiles = _load("gemm_tile").cw_gemm_bf16_wide_tiles(2, M, two_i, K, ldx)
     if tiles < WIDE_SWIGLU_MIN_TILES:
         return False
-    units = _compute_units(torch.device("cuda", torch.cuda.current_device()))
-    # fewer than 512 rows that are no multiple of 16 are a step that runs as it came, not padded for a captured graph:
-    # the host's launches bound it, and the library serves its product
-    if M < WIDE_SWIGLU_MIN_ROWS // 2 and M % 16:
-        return False
-    return M >= WIDE_SWIGLU_MIN_ROWS or (two_i * K <= WIDE_SWIGLU_SMALL_WEIGHTS
-                                         and tiles >= WIDE_SWIGLU_FILL * units * -(-tiles // units))
+    if M >= WIDE_SWIGLU_MIN_ROWS:
+        return True
+    units, rows = _compute_units(torch.device("cuda", torch.cuda.current_device())), WIDE_SWIGLU_TILE_ROWS
+    return (two_i * K <= WIDE_SWIGLU_SMALL_WEIGHTS and tiles >= WIDE_SWIGLU_FILL * units * -(-tiles // units)
+            and M >= WIDE_SWIGLU_FILL * rows * -(-M // rows))
 
 
 @contextlib.contextmanager
@@ -1195,7 +1195,11 @@ def linear_swiglu(x, gate_up_weight: torch.Tensor, policy: "ProductPolicy | None
             return linear_mid(x, gate_up_weight, choice, swiglu=True, limit=limit)
         if policy.hip_products:
             return linear_tiled(x, gate_up_weight, swiglu=True, limit=limit)
-        if _aligned(x, gate_up_weight) and wide_swiglu_pays(M, two_i, K, K):
+        # fewer than 512 rows only inside a captured graph, where a shape's steps run from its second on. Run eagerly they
+        # keep to the library's product, as the replay tests have it (450 tokens of the 1.5B shape, bound by the host's
+        # launches: 3.9 ms, 3.65 with one launch instead of two)
+        if (_aligned(x, gate_up_weight) and wide_swiglu_pays(M, two_i, K, K)
+                and (M >= WIDE_SWIGLU_MIN_ROWS // 2 or torch.cuda.is_current_stream_capturing())):
             # with enough rows the shape of the weights decides, and a start-up that tunes the
             # library's products has measured it for this model's
             measured, key = M >= WIDE_SWIGLU_MIN_ROWS, _swiglu_key(two_i, K, limit)

@@ -262,6 +262,36 @@ def test_operands_that_only_the_library_takes(M):
         ops.linear(x, w, torch.zeros(N, device=DEV))
 
 
+def test_gate_up_of_a_captured_step_by_its_rows_and_tiles():
+    """Steps of 1 to 24 padded single tokens beside a portion padded to 384 rows are steps of 385 to 408 rows: all of them
+    take the wide tiles, no step of fewer rows does, whatever it is a multiple of."""
+    from clockwork_amd import ops
+
+    two_i, K = 2 * 8960, 1536
+    assert all(ops.wide_swiglu_pays(M, two_i, K, K) for M in (384, 385, 386, 388, 392, 400, 408, 448, 450, 512, 1000))
+    assert not any(ops.wide_swiglu_pays(M, two_i, K, K) for M in (256, 257, 264, 272, 288, 304, 320, 352, 576, 640))
+    gen = torch.Generator(device=DEV).manual_seed(4)
+    w = (torch.randn(two_i, K, device=DEV, generator=gen) / K ** 0.5).to(torch.bfloat16)
+    x = torch.randn(385, K, device=DEV, generator=gen).to(torch.bfloat16)
+    h = x.float() @ w.float().t()
+    want = torch.nn.functional.silu(h[:, :8960]) * h[:, 8960:]
+    ran, real = [], ops.linear_tiled
+    try:
+        ops.linear_tiled = lambda *a, **k: (ran.append(a[0].shape[0]), real(*a, **k))[1]
+        torch.testing.assert_close(ops.linear_swiglu(x, w).float(), want, rtol=4 * 2.0 ** -8, atol=2e-2)   # two roundings each side
+        assert not ran   # a step that is not captured
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = ops.linear_swiglu(x, w)
+        assert ran == [385]
+    finally:
+        ops.linear_tiled = real
+    for _ in range(2):
+        got.zero_()
+        graph.replay()
+        torch.testing.assert_close(got.float(), want, rtol=2.0 ** -8 + 1e-4, atol=1e-3)   # one rounding
+
+
 # 16 requests at the edges of a wave's tile of 32 keys, of the turns of four and eight waves and of the line where
 # eight take over (128 keys a split); 24 keys a page and 16; a group of more than 16 heads
 @pytest.mark.parametrize("hd,nh,nkv,bs", [(32, 4, 2, 16), (64, 14, 2, 16), (96, 6, 3, 24), (128, 12, 2, 16), (128, 20, 1, 24), (160, 4, 2, 16)])
