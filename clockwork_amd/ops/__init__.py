@@ -522,8 +522,9 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias=None, out_dtype=None, par
     engine uses one) or, where ``policy`` (the calling engine's :class:`ProductPolicy`) says so,
     through this package's tiled kernels; float32 accumulation either way. With ``partial_ok``
     the result may come back as :class:`PartialSums` (a narrow output with a long K, few rows):
-    only for a result that goes straight into ``add_rmsnorm``. ``portions_partial_ok``: with many rows
-    as well, by the rule of ``cw_gemm_bf16_mid_choice`` (csrc/gemm_tile.hip)."""
+    only for a result that goes straight into ``add_rmsnorm``. ``portions_partial_ok``: the kernel that reads it adds
+    the planes, however many there are: with many rows as well, by the rule of ``cw_gemm_bf16_mid_choice``
+    (csrc/gemm_tile.hip), and in float32 (up to 64 planes)."""
     policy = policy if policy is not None else DEFAULT_POLICY
     _gpu(x, weight, bias)
     M, K = x.shape
@@ -535,7 +536,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias=None, out_dtype=None, par
             raise KernelError("a float32 product needs float32 weights")
         lib = _load("gemm")
         # a narrow output with a long K is summed in parts over K (the same parts whatever M is)
-        if partial_ok and bias is None:
+        if partial_ok and portions_partial_ok and bias is None:
             planes = lib.cw_gemm_f32_partial_planes(M, N, K)
             if planes:
                 parts = torch.empty((planes, M, N), dtype=torch.float32, device=x.device)

@@ -271,7 +271,8 @@ class PagedAttention(Part):
             bias = self.qkv_bias[: self.q_width] if self.qkv_bias is not None else None
             self.position.rotate_and_store(qkv, bias, ctx.positions, None, nh, 0, hd, None, None)
         out = self.attend(qkv, ctx, cache)
-        return ops.linear(out, self.out_weight, self.out_bias, partial_ok=True, policy=policy, portions_partial_ok=True)
+        return ops.linear(out, self.out_weight, self.out_bias, partial_ok=True, policy=policy,
+                          portions_partial_ok=getattr(ctx, "reader_adds_sums", False))
 
     def attend(self, q: torch.Tensor, ctx, cache: EntryCache) -> torch.Tensor:
         """Attention of the step's rotated queries (the first ``num_heads * head_dim`` columns of

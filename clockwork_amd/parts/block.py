@@ -37,9 +37,12 @@ class PreNormBlock:
 
     def forward(self, resid, delta, ctx, cache):
         x = self.mixer_norm.forward(resid, delta)
+        next_adds = getattr(ctx, "next_norm_adds_sums", False)
+        ctx.reader_adds_sums = next_adds if self.feed_forward is None else getattr(self.ffn_norm, "adds_partial_sums", False)
         a = self.mixer.forward(x, ctx, cache)
         if self.feed_forward is None:
             return a
+        ctx.reader_adds_sums = next_adds
         # Few rows: the second norm can run inside the feed-forward's first product, which saves a
         # launch. That kernel writes no residual, so the mixer's output stays pending and is
         # handed on together with the feed-forward's (the next norm must be able to take both).
@@ -155,9 +158,12 @@ class TwoNormParallelBlock:
         else:
             x = self.mixer_norm.forward(resid, delta)
             y = self.ffn_norm.forward(resid, None) if self.feed_forward is not None else None
+        next_adds = getattr(ctx, "next_norm_adds_sums", False)
+        ctx.reader_adds_sums = next_adds and self.feed_forward is None   # the first of two outputs goes on as a tensor
         a = self.mixer.forward(x, ctx, cache)
         if self.feed_forward is None:
             return a
+        ctx.reader_adds_sums = next_adds and getattr(ctx, "next_norm_accepts_pending", False)
         b = self.feed_forward.forward(y, ctx)
         if isinstance(a, ops.PartialSums):
             a = a.sum(x.dtype)

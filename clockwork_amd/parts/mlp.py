@@ -34,7 +34,8 @@ class SwiGLU(Part):
 
     def forward(self, x, ctx) -> torch.Tensor:
         policy = getattr(ctx, "products", None)
-        return ops.linear(ops.linear_swiglu(x, self.gate_up, policy=policy), self.down, partial_ok=True, policy=policy, portions_partial_ok=True)
+        return ops.linear(ops.linear_swiglu(x, self.gate_up, policy=policy), self.down, partial_ok=True, policy=policy,
+                          portions_partial_ok=getattr(ctx, "reader_adds_sums", False))
 
 
 class GatedMLP(Part):

@@ -192,6 +192,10 @@ class DecoderModel:
             ctx.next_norm_accepts_pending = bool(getattr(nxt, "accepts_pending", False))
             ctx.next_norm_accepts_normed = bool(getattr(nxt, "accepts_normed_branch", False))
             ctx.next_norm_accepts_gated = bool(getattr(nxt, "accepts_gated", False))
+            # and may its output be the planes of a product of many rows? (a re-entry comes ahead of the next norm)
+            reenters = i + 1 < len(run) and run[i + 1].reenter is not None
+            ctx.next_norm_adds_sums = bool(getattr(nxt, "adds_partial_sums", False)) and not reenters
+            ctx.reader_adds_sums = False   # for a part of the block: does whoever reads its output add them? The block says so
             delta = self.layers[entry.layer].forward(resid, delta, ctx, caches[i])
         if ctx.num_logit_rows == 0:
             return None

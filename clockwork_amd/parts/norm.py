@@ -14,6 +14,9 @@ class RMSNorm(Part):
     graph_safe = True
     # takes a delta that is an ops.PendingPair (two branch outputs not yet added to the residual)
     accepts_pending = True
+    # adds a delta that is an ops.PartialSums in its kernel, however many planes there are
+    adds_partial_sums = True
+
     def __init__(self, spec: RMSNormSpec) -> None:
         self.spec = spec
 

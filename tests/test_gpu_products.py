@@ -32,10 +32,12 @@ def test_float32_rows_have_the_same_bits_in_every_kernel(N, K):
     for rows in (1, 15, 16, 17, 32, 33, 64, 65, 256, 257):
         part = x[:rows].contiguous()
         assert torch.equal(ops.linear(part, w, b), whole[:rows]), rows
-        got = ops.linear(part, w, partial_ok=True)
-        if isinstance(got, ops.PartialSums):
-            got = got.sum()
-        assert torch.equal(got, plain[:rows]), rows
+        for reader_adds in (False, True):
+            got = ops.linear(part, w, partial_ok=True, portions_partial_ok=reader_adds)
+            if isinstance(got, ops.PartialSums):
+                assert reader_adds
+                got = got.sum()
+            assert torch.equal(got, plain[:rows]), rows
 
 
 def test_float32_infinities_stay_in_their_rows_and_columns():

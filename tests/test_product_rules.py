@@ -1,5 +1,7 @@
 """Which kernel serves a product of many rows: the rule of csrc/gemm_tile.hip on both sides of its lines, without a GPU."""
 
+from types import SimpleNamespace
+
 import pytest
 
 from clockwork_amd import ops
@@ -42,3 +44,70 @@ def test_no_choice_outside_what_the_kernels_take():
         for M, N, K in ((64, 1152, 896), (2049, 1152, 896), (144, 1152, 900), (144, 1152, 192), (144, 0, 896)):
             assert _choice(mode, M, N, K) is None
     assert _choice(2, 160, 9729, 896) is None and _choice(1, 160, 1152, 896) is None
+
+
+def test_planes_of_many_rows_only_for_a_norm_that_adds_them(monkeypatch):
+    """A product of a portion, and any in float32, may come as planes of partial sums where its block hands it to a norm
+    that adds them in its kernel; any other reader would add a dozen planes with a dozen launches."""
+    from clockwork_amd.parts.block import PreNormBlock, TwoNormParallelBlock
+    from clockwork_amd.parts.mlp import SwiGLU
+    from clockwork_amd.parts.norm import LayerNorm, RMSNorm
+
+    assert RMSNorm.adds_partial_sums and not getattr(LayerNorm, "adds_partial_sums", False)
+    asked = []
+    monkeypatch.setattr(ops, "linear_swiglu", lambda x, *a, **k: x)
+    monkeypatch.setattr(ops, "linear", lambda *a, **k: asked.append(k["portions_partial_ok"]))
+    monkeypatch.setattr(ops, "gated_residual_add", lambda *a: None)
+    feed_forward = SwiGLU(None)
+    feed_forward.gate_up = feed_forward.down = None
+
+    class Mixer:
+        def forward(self, x, ctx, cache):
+            asked.append(("mixer", ctx.reader_adds_sums))
+
+    def norm(adds):
+        return SimpleNamespace(forward=lambda resid, delta: resid, adds_partial_sums=adds)
+
+    resid = SimpleNamespace(shape=(300, 8), dtype=None)
+    for inner in (False, True):
+        for after in (False, True):
+            ctx = SimpleNamespace(next_norm_adds_sums=after, next_norm_accepts_pending=False, products=None)
+            PreNormBlock(Mixer(), norm(False), feed_forward, norm(inner)).forward(resid, None, ctx, None)
+            assert asked == [("mixer", inner), after]
+            asked.clear()
+            PreNormBlock(Mixer(), norm(False)).forward(resid, None, ctx, None)
+            assert asked == [("mixer", after)]
+            asked.clear()
+            ctx.next_norm_accepts_pending = inner
+            TwoNormParallelBlock(Mixer(), norm(True), feed_forward, norm(True)).forward(resid, None, ctx, None)
+            assert asked == [("mixer", False), inner and after]
+            asked.clear()
+    # a part that no block has told anything
+    feed_forward.forward(resid, SimpleNamespace(products=None))
+    assert asked == [False]
+
+
+def test_the_model_says_whether_the_next_norm_adds_planes():
+    from clockwork_amd.config.spec import LayerSpec, ModelSpec, RunEntry
+    from clockwork_amd.parts.model import DecoderModel
+    from clockwork_amd.parts.specs import AttentionSpec, RMSNormSpec, SwiGLUSpec
+
+    norm = RMSNormSpec(16, 1e-6)
+    layer = LayerSpec("prenorm", AttentionSpec(16, 1, 1, 16, False, False, 0.25), SwiGLUSpec(16, 32), norm, norm)
+    model = DecoderModel(ModelSpec("toy", 10, 16, [layer], [RunEntry(0)] * 4, norm))
+    said = []
+
+    class Block:
+        def __init__(self, adds):
+            self.first_norm = lambda: SimpleNamespace(adds_partial_sums=adds)
+
+        def forward(self, resid, delta, ctx, cache):
+            said.append((ctx.next_norm_adds_sums, ctx.reader_adds_sums))
+            ctx.reader_adds_sums = True   # does not reach the next block
+            return delta
+
+    model.layers = [Block(True), Block(True), Block(False), Block(True)]
+    model.spec.run = [RunEntry(0), RunEntry(1), RunEntry(2), RunEntry(3)]
+    model.embedding = type("E", (), {"forward": lambda self, ctx: None})()
+    assert model.forward(SimpleNamespace(num_logit_rows=0, sequence_positions=None), [None] * 4) is None
+    assert said == [(True, False), (False, False), (True, False), (True, False)]
