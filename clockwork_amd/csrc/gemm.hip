@@ -1066,12 +1066,14 @@ CW_EXPORT int cw_gemm_bf16_skinny_ksplits(int M, int N, int K) {
   // (steps as the kernel is built for; 16 of them come in fours, too few on their way: 15 % more), a part costs its
   // way to memory and back. With the norm behind it, the count before and now (us, 8 rows): 7B shape's down product 38.4
   // (5 parts) and 33.4 (8), output product 14.3 and 12.1; 14B shape's down 38.9 and 35.2; 32B shape's down 64.4 and 59.9.
+  // A count whose shares come to more workgroups than there are units has a second round for the few beyond (4096 x
+  // 14336: 8 parts in 256 workgroups 28.9, 7 in 259 37.5; 72B shape's down: 8 in 256 105, 5 in 260 124).
   int best = 0;
   float least = 0.0f;
   for (int s = 2; s <= 12 && K / s >= 1024; ++s) {
     int mt, spw, n_tiles;
     dim3 grid;
-    if (!plan_stream(3, M, N, K, s, &mt, &spw, &grid, &n_tiles)) continue;
+    if (!plan_stream(3, M, N, K, s, &mt, &spw, &grid, &n_tiles) || (int)(grid.x * grid.y) > cw_num_compute_units()) continue;
     const int per = (n_tiles + (int)grid.x - 1) / (int)grid.x;
     const float t = (float)(per * spw) * (spw == 16 ? 1.15f : 1.0f) + 0.6f * (float)s * (float)N / 3584.0f;
     if (best == 0 || t < least) {

@@ -111,3 +111,11 @@ def test_the_model_says_whether_the_next_norm_adds_planes():
     model.embedding = type("E", (), {"forward": lambda self, ctx: None})()
     assert model.forward(SimpleNamespace(num_logit_rows=0, sequence_positions=None), [None] * 4) is None
     assert said == [(True, False), (False, False), (True, False), (True, False)]
+
+
+@pytest.mark.parametrize("N,K,parts", [(4096, 14336, 8), (8192, 29568, 8), (3584, 18944, 8), (1536, 8960, 7), (5120, 27648, 11), (896, 4864, 4)])
+def test_parts_over_k_do_not_come_to_more_workgroups_than_units(N, K, parts):
+    """Products of up to 16 rows: a workgroup takes ceil(tiles * parts / 256) tiles of a part."""
+    tiles = -(-N // 16)
+    assert -(-tiles // -(-tiles * parts // CUS)) * parts <= CUS
+    assert all(ops._load("gemm").cw_gemm_bf16_skinny_ksplits(M, N, K) == parts for M in (1, 8, 16))
