@@ -755,17 +755,18 @@ WIDE_MIN_TILES = 64
 # The engine takes the wide-tile kernel for the gate/up product by itself (no ``hip_products``)
 # where it beats the library product followed by the gate kernel. Measured on an MI355X over the
 # Qwen2.5 layer shapes from 0.5B to 72B with 256 to 4096 rows: with 180 tiles or more and 1024 rows or
-# more it is 5 to 25 % faster. With fewer rows it is for weights of at most 64 M elements where its tiles fill seven
-# tenths of their rounds over the compute units and its rows seven tenths of their tiles (us, library and gate against this:
-# 1.5B shape, 188 tiles of 256 rows, 304 rows 34.8 / 36.4, 368 rows 37.4 / 36.0, 408 rows 38.9 / 36.7, 512 rows 44.5 / 37.3; 282 tiles, 640 rows
-# 53.6 / 68.9; 376 tiles, 1000 rows 88.3 / 71.8; 3B shape, 230 tiles, 304 rows 44.5 / 44.8, 385 rows 55.1 / 45.8; 7B shape, 400 rows
-# 150 / 136, 640 rows 189 / 202: there reading W bounds both). Against the library's TUNED choice it wins for
+# more it is 5 to 25 % faster. With fewer rows it is for weights of at most 64 M elements where enough of its work is
+# not padding, of the rows to whole tiles and of the tiles to whole rounds over the compute units: 52 % in one round (the
+# library leaves units idle there as well), 58 % in several (us, library and gate against this: 1.5B shape, 188 tiles, 304 rows
+# 34.8 / 36.4, 368 rows 37.4 / 36.0, 408 rows 38.9 / 36.7, 512 rows 44.5 / 37.3; 282 tiles, 640 rows 53.6 / 68.9; 376 tiles,
+# 1000 rows 88.3 / 71.8; 3B shape, 230 tiles, 304 rows 44.5 / 44.8, 385 rows 55.1 / 45.8; 345 tiles, 640 rows 77.8 / 84.9, 700 rows
+# 97.2 / 86.0; 7B shape, 400 rows 150 / 136, 640 rows 189 / 202: there reading W bounds both). Against the library's TUNED choice it wins for
 # the 0.5B, 1.5B, 3B, 14B and 32B shapes (the 1.5B shape's whole prefill step: 8.9 -> 7.9 ms) and
 # loses 3 % of the step for the 7B and 72B shapes, so a start-up that tunes (``library_tuning``)
 # times both ways on the model's own weights and keeps the faster (``ProductPolicy.swiglu_choices``).
 WIDE_SWIGLU_MIN_TILES = 180
 WIDE_SWIGLU_MIN_ROWS = 1024
-WIDE_SWIGLU_FILL = 0.71
+WIDE_SWIGLU_WORK, WIDE_SWIGLU_WORK_ONE_ROUND = 0.58, 0.52
 WIDE_SWIGLU_TILE_ROWS = 256
 WIDE_SWIGLU_SMALL_WEIGHTS = 64 << 20    # elements of [gate; up]
 
@@ -790,8 +791,9 @@ def wide_swiglu_pays(M: int, two_i: int, K: int, ldx: int) -> bool:
     if M >= WIDE_SWIGLU_MIN_ROWS:
         return True
     units, rows = _compute_units(torch.device("cuda", torch.cuda.current_device())), WIDE_SWIGLU_TILE_ROWS
-    return (two_i * K <= WIDE_SWIGLU_SMALL_WEIGHTS and tiles >= WIDE_SWIGLU_FILL * units * -(-tiles // units)
-            and M >= WIDE_SWIGLU_FILL * rows * -(-M // rows))
+    rounds = -(-tiles // units)
+    work = tiles / (units * rounds) * M / (rows * -(-M // rows))
+    return two_i * K <= WIDE_SWIGLU_SMALL_WEIGHTS and work >= (WIDE_SWIGLU_WORK if rounds > 1 else WIDE_SWIGLU_WORK_ONE_ROUND)
 
 
 @contextlib.contextmanager
