@@ -936,13 +936,15 @@ CW_EXPORT int cw_gemm_bf16_mid(int mode, const void* X, int64_t ldx, const void*
 
 // Time of a product's work items in microseconds as the choice below weighs them, without what every launch costs:
 // rounds over the compute units, a stage of 64 elements of K taking what its loads take, and the planes' way to
-// memory and back. The constants are fits to the measurements above (64 x 64 and 64 x 128 tiles share a compute unit
-// with others, which covers for a part of their last round).
+// memory and back. The constants are fits (64 x 64 and 64 x 128 tiles share a compute unit with others, which covers
+// for a part of their last round): over 72 to 1024 rows of eight shapes what they name takes 1.0 % more than the fastest
+// tiles and counts do (2.9 % with 0.62 and 1.04 us a stage of the two largest: 700 rows of the 3B shape's down product
+// went to 64 x 128 tiles, 67.7 us, where 128 x 128 ones take 59.7).
 static float mid_time(int M, int N, int K, int bm, int bn, int planes, int cus) {
-  const float stage = bm + bn == 128 ? 0.27f : bm + bn == 192 ? 0.38f : bm == 128 ? 0.62f : 1.04f;
+  const float stage = bm + bn == 128 ? 0.27f : bm + bn == 192 ? 0.38f : bm == 128 ? 0.55f : 0.9f;
   const int64_t items = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * planes;
   const int64_t rounds = (items + cus - 1) / cus;
-  const float share = rounds > 1 && bm + bn < 256 ? 0.85f : 1.0f;
+  const float share = rounds > 1 && bm + bn < 256 ? 0.95f : 1.0f;
   const int stages = (K / 64 + planes - 1) / planes;
   return share * (float)(rounds * stages) * stage + (planes > 1 ? 2.2e-6f * (float)planes * (float)M * (float)N : 0.0f);
 }
@@ -956,8 +958,10 @@ static float mid_time(int M, int N, int K, int bm, int bn, int planes, int cus) 
 //    of the 32B shape 484 -> 513), 2.1 M for outputs of more than 5120 columns (72B shape, 256 rows 293 -> 177, 640 rows
 //    302 -> 370). Beyond 1024 rows and columns on the wide tiles only (3B shape's down product, 1434 rows 98 -> 115 on
 //    the small ones), which have to fill their rounds (7B shape, 1600 rows in 2.08 rounds 241 -> 273, 2048 in 2.4 386 ->
-//    292); beyond 640 rows not as whole sums of K (2048 x 6144, 1000 rows 49.4 -> 54.5). A squarer matrix
-//    while M N is below 1.2 M and N at most 5120: beyond, the planes cost more than the library's idle units.
+//    292; 3B shape, 1356 rows in 0.52 90 -> 103, 1600 in 0.6 112 -> 100); beyond 640 rows not as whole sums of K (2048 x
+//    6144, 1000 rows 49.4 -> 54.5; as 2 planes on 128 x 128 tiles 43.6). A squarer matrix
+//    while M N is below 1.2 M, 1.03 M for more than 1536 columns (2048 x 2048, 500 rows 17.5 -> 16.9, 522 rows 18.8 ->
+//    20.2), and N at most 5120: beyond, the planes cost more than the library's idle units.
 //  * mode 2: M N K up to 4.5e9 (72 rows of the 1.5B shape: 28.0 -> 22.9 us, 208 rows 32.2 -> 31.8), and up to 640 rows for
 //    a matrix of at most 9 M elements; a K of more than 1024 and half of N is a narrow output's (896 x 4864, 165 rows
 //    15.0 -> 20.6).
@@ -979,7 +983,7 @@ CW_EXPORT int cw_gemm_bf16_mid_choice(int mode, int M, int N, int K, int64_t ldx
   if (mode == 2) {
     if ((N & 1) || (N < 2 * K && K > 1024) || !((int64_t)M * elements <= 4500000000ll || (elements <= 9 << 20 && M <= 640))) return 0;
   } else if (mode == 3) {
-    const int64_t most = K >= 3 * N ? (N <= 5120 ? 8000000 : 2100000) : N <= 5120 ? 1200000 : 0;
+    const int64_t most = K >= 3 * N ? (N <= 5120 ? 8000000 : 2100000) : N <= 1536 ? 1200000 : N <= 5120 ? 1030000 : 0;
     if (outputs > most) return 0;
   } else {
     return 0;
@@ -1006,7 +1010,7 @@ CW_EXPORT int cw_gemm_bf16_mid_choice(int mode, int M, int N, int K, int64_t ldx
     if (planes == 1 && M > 640 && N >= 512 && K >= 3 * N) return 0;
     if ((best & 1023) != W_BM) return M > 1024 && N >= 1024 ? 0 : best;
     const int64_t items = (int64_t)((M + W_BM - 1) / W_BM) * ((N + W_BN - 1) / W_BN) * planes;
-    if (items > cus && (float)items < 0.72f * (float)(cus * ((items + cus - 1) / cus))) return 0;
+    if ((float)items < (items > cus ? 0.72f : M > 1024 ? 0.55f : 0.0f) * (float)(cus * ((items + cus - 1) / cus))) return 0;
   }
   return best;
 }

@@ -21,7 +21,7 @@ def _choice(mode, M, N, K):
     # tiles enough for the library
     (0, 700, 4096, 896), (0, 1500, 2048, 896), (0, 1500, 4096, 512), (0, 1000, 4096, 256), (0, 144, 2048, 1536),
     # sums for a norm: large outputs, small tiles beyond 1024 rows, whole sums of a long K, rounds that stay empty
-    (3, 2048, 5120, 27648), (3, 640, 8192, 29568), (3, 2048, 8192, 29568), (3, 1434, 2048, 11008), (3, 1000, 2048, 6144), (3, 1600, 3584, 18944),
+    (3, 2048, 5120, 27648), (3, 640, 8192, 29568), (3, 2048, 8192, 29568), (3, 1434, 2048, 11008), (3, 1356, 2048, 11008), (3, 1600, 3584, 18944),
     (3, 152, 7376, 2304),
     # gated products of a narrow output
     (2, 165, 896, 4864), (2, 250, 368, 9600), (2, 92, 1280, 3072), (2, 670, 9728, 896)])
@@ -32,7 +32,7 @@ def test_products_that_stay_with_the_library(mode, M, N, K):
 @pytest.mark.parametrize("mode,M,N,K,wide", [
     (0, 144, 1152, 896, False), (0, 400, 2048, 1536, False), (0, 256, 64, 512, False), (0, 1000, 1152, 512, False),
     (3, 160, 1536, 8960, False), (3, 2048, 1536, 8960, True), (3, 1024, 1536, 8960, True), (3, 2048, 3584, 18944, True), (3, 256, 8192, 29568, False),
-    (3, 1536, 5120, 27648, True), (3, 160, 1536, 1536, False), (3, 1000, 896, 896, False), (3, 2048, 256, 1024, False),
+    (3, 1536, 5120, 27648, True), (3, 160, 1536, 1536, False), (3, 1000, 896, 896, False), (3, 700, 2048, 11008, True), (3, 1600, 2048, 11008, True), (3, 1000, 2048, 6144, False), (3, 2048, 256, 1024, False),
     (2, 160, 17920, 1536, False), (2, 400, 9728, 896, False), (2, 257, 8192, 2048, False)])
 def test_products_on_the_tiles_between(mode, M, N, K, wide):
     bm, bn, planes = _choice(mode, M, N, K)
