@@ -264,7 +264,8 @@ __global__ __launch_bounds__(256) void linear_recurrence_quads_kernel(LinRecPara
           const float bonus = f.bonus && d0 + rr < D ? f.bonus[h * D + d0 + rr] : 0.0f;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const float kv = k * vv[e];
+            // (nothing for a row past dim, also where the value is infinite)
+            const float kv = d0 + rr < D ? k * vv[e] : 0.0f;
             if (f.bonus) po[e] += q * (S[rr][e] + bonus * kv);
             S[rr][e] = a * S[rr][e] + kv;
             if (!f.bonus) po[e] += q * S[rr][e];

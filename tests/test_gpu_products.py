@@ -437,6 +437,28 @@ def test_recurrence_of_few_tokens(dim, vdim, rank, dtype):
         torch.testing.assert_close(state.to(f64), after, atol=1e-4, rtol=1e-4)
 
 
+# keys whose last run of rows is padded
+@pytest.mark.parametrize("dim,vdim", [(5, 256), (100, 128)])
+@pytest.mark.parametrize("with_bonus", [False, True])
+def test_recurrence_of_infinite_values(dim, vdim, with_bonus):
+    """An infinite value makes its own column infinite, with the sign of its terms, and no other; rows that only pad a thread's
+    run add nothing to it."""
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(dim)
+    proj = torch.rand(2, 2 * dim + vdim + 16, device=DEV, generator=gen) + 0.5   # q, k, v, the decay's input
+    proj[0, 2 * dim + 3], proj[0, 2 * dim + 6] = float("inf"), -float("inf")
+    state = torch.zeros(1, 1, dim, vdim, device=DEV)
+    ints = lambda *t: torch.tensor(t, dtype=torch.int32, device=DEV)  # noqa: E731
+    got = ops.linear_recurrence(proj, 0, dim, 2 * dim, -1, 2 * dim + vdim, torch.rand(dim, 16, device=DEV, generator=gen), None, None, state,
+                                ints(0), ints(0, 2), 1, 1, dim, vdim, 1.0, 16.0, 1e-5,
+                                bonus=torch.ones(1, dim, device=DEV) if with_bonus else None)
+    assert bool((got[:, 3] == float("inf")).all()) and bool((got[:, 6] == -float("inf")).all())
+    rest = [c for c in range(vdim) if c not in (3, 6)]
+    assert bool(torch.isfinite(got[:, rest]).all()) and bool(torch.isfinite(state[..., rest]).all())
+    assert bool((state[0, 0, :, 3] == float("inf")).all()) and bool((state[0, 0, :, 6] == -float("inf")).all())
+
+
 # runs of 32, 50 and 128 keys; mixed heads over one, two (two kernels) and three key/value heads (three kernels), no
 # mixing over four; sizes that are read in pieces and one by one, more columns than threads, groups of more than 16 heads
 @pytest.mark.parametrize("heads,kv,dim,vdim,talk", [(12, 2, 128, 128, True), (6, 2, 20, 24, True), (3, 1, 40, 24, True), (6, 3, 64, 64, True),
