@@ -1,8 +1,8 @@
 // Causal attention over a paged key/value cache for gfx950, one head size per build
 // (compile with -DCW_HD=<head_dim>, a multiple of 16 from 16 to 256).
 //
-// One kernel serves portions of prompts and single decoded tokens: a work item is a run of
-// consecutive query tokens of one request; a workgroup takes one item, one key/value head and
+// The first kernel serves portions of prompts and single decoded tokens of any type: a work item is a run of
+// consecutive query tokens of one request; a workgroup takes rows of one item, one key/value head and
 // all (or a chunk of) the query heads of that head's group, so a key/value tile is fetched once
 // for the whole group. The key range of an item can be cut into splits that run in parallel
 // and are merged by a second kernel (decode with few requests and long contexts).
@@ -66,50 +66,60 @@ static inline int cw_log2_or_minus1(int v) {
   return -1;
 }
 
-template <typename T> struct Vec16;
-template <> struct Vec16<float> {
-  static constexpr int N = 4;
-  __device__ static void load(const float* p, float* o) {
+// Four neighbouring elements of a cache or query row as float32, and VW of them (1, 2 or 4).
+typedef __attribute__((ext_vector_type(4))) float attn_f32x4_t;
+template <int VW> __device__ __forceinline__ void attn_load(const float* p, float (&o)[VW]) {
+  if (VW == 4) {
     const float4 v = *reinterpret_cast<const float4*>(p);
-    o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
+    o[0] = v.x; o[1 % VW] = v.y; o[2 % VW] = v.z; o[3 % VW] = v.w;
+  } else if (VW == 2) {
+    const float2 v = *reinterpret_cast<const float2*>(p);
+    o[0] = v.x; o[1 % VW] = v.y;
+  } else {
+    o[0] = p[0];
   }
-};
-template <> struct Vec16<bf16_t> {
-  static constexpr int N = 8;
-  __device__ static void load(const bf16_t* p, float* o) {
-    const uint4 v = *reinterpret_cast<const uint4*>(p);
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+}
+template <int VW> __device__ __forceinline__ void attn_load(const bf16_t* p, float (&o)[VW]) {
+  if (VW == 1) {
+    o[0] = cw_to_float(p[0]);
+  } else {
+    uint32_t w[VW / 2 + (VW == 1)];
+    __builtin_memcpy(w, __builtin_assume_aligned(p, VW * 2), VW * 2);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      o[2 * i] = __uint_as_float(w[i] << 16);
-      o[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    for (int i = 0; i < VW / 2; ++i) {
+      o[(2 * i) % VW] = __uint_as_float(w[i] << 16);
+      o[(2 * i + 1) % VW] = __uint_as_float(w[i] & 0xffff0000u);
     }
   }
-};
+}
 
-template <int HD, int ROWS, int BN> struct TileShape {
-  static constexpr int QS = HD + 4;   // query row stride in floats (16-byte rows)
-  static constexpr int KS = HD + 1;   // key row stride: odd, so a column read hits distinct banks
-  static constexpr int VS = HD + 4;   // value row stride (16-byte rows); also the buffer's row size
-  static constexpr int SS = BN + 1;
-  static constexpr int FLOATS = ROWS * QS + BN * VS + ROWS * SS + 3 * ROWS;
-};
+// Float32 scores, softmax and sums for any cache type, all products on the matrix cores
+// (v_mfma_f32_16x16x4_f32: float32 operands, products and sums).
+//
+// A workgroup takes RB blocks of 16 rows (token, head of the group) of one item, one key/value head and one
+// split of the keys; its waves take tiles of 16 keys in turn and meet in LDS at the end. Lane (c, s) = (l % 16, l / 16):
+//   S^T[key, row] = K * Q^T    lane holds four neighbouring elements, from 4 s on, of key c / of row c: the j-th of four
+//                              products takes element j of every lane, which is the same k-value in both operands;
+//   softmax                    the lane comes out with keys 4 s .. 4 s + 3 of row c: a row is four lanes;
+//   O^T[d, row] += V^T * P^T   the j-th product takes key 4 s + j: P^T is what the lane holds, and V's elements come in
+//                              runs of VW along a row, tile e of a run's VW tiles taking element e.
+// Nothing passes through LDS in the loop, and the next tile's keys are on their way over this one's products.
+// What bounds it is the trip to memory of a wave's first tiles with short ranges (so 16 rows a workgroup while that
+// leaves compute units idle) and the matrix cores' float32 rate with long ones (32 rows: a key is read for twice the rows).
+// Measured: see launch_attention.
+template <typename T, int HD, int RB, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void attn_f32_kernel(AttnParams p, int rows, int subs) {
+  constexpr int VW = HD % 64 == 0 ? 4 : HD % 32 == 0 ? 2 : 1;  // elements of a value row that a lane loads at once
+  constexpr int KB = HD / 16, VG = HD / (16 * VW), OS = HD + 4;
+  extern __shared__ __align__(16) float smem[];  // [WAVES][16][OS] sums, then [WAVES][16][2] maxima and sums of weights
+  float* const o_s = smem;
+  float* const ml_s = smem + WAVES * 16 * OS;
 
-template <typename T, int HD, int ROWS, int BN>
-__global__ __launch_bounds__(256) void attn_tile_kernel(AttnParams p) {
-  using S = TileShape<HD, ROWS, BN>;
-  extern __shared__ __align__(16) float smem[];
-  float* Qs = smem;
-  float* KVs = Qs + ROWS * S::QS;
-  float* Ss = KVs + BN * S::VS;
-  float* m_s = Ss + ROWS * S::SS;
-  float* l_s = m_s + ROWS;
-  float* a_s = l_s + ROWS;
-
-  const int tid = threadIdx.x;
-  const int item = blockIdx.x;
-  const int kvh = blockIdx.y / p.n_chunks;
-  const int chunk = blockIdx.y % p.n_chunks;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, s = lane >> 4;
+  const int turn = gridDim.x - 1 - blockIdx.x;  // a portion's last tokens have the longest key ranges: they begin first
+  const int item = turn / subs, row0 = (turn % subs) * (16 * RB);
+  const int kvh = blockIdx.y / p.n_chunks, chunk = blockIdx.y % p.n_chunks;
   const int split = blockIdx.z;
   const int req = p.items[4 * item], tok0 = p.items[4 * item + 1];
   const int ctx = p.ctx_lens[req];
@@ -118,199 +128,226 @@ __global__ __launch_bounds__(256) void attn_tile_kernel(AttnParams p) {
   // an item may reach past the request's tokens (work items laid out for a longer portion than
   // the step brings): what lies past them is not computed
   const int ntok = min(p.items[4 * item + 2], qlen - tok0);
-  if (ntok <= 0) return;
   const int group = p.nh / p.nkv;
   const int gh = p.gh;
+  const int tok_first = row0 / gh;                              // tokens of this workgroup's rows
+  const int tok_end = min(ntok, (row0 + 16 * RB - 1) / gh + 1);
+  if (tok_first >= tok_end) return;
   const int pos0 = ctx - qlen + tok0;  // absolute position of the item's first token
-  const int kv_end = pos0 + ntok;
-  const int kv_lo = p.window > 0 ? max(0, pos0 - p.window + 1) : 0;
-  const int tile0 = kv_lo / BN;
-  const int n_tiles = (kv_end + BN - 1) / BN - tile0;
+  const int kv_end = pos0 + tok_end;
+  const int kv_lo = p.window > 0 ? max(0, pos0 + tok_first - p.window + 1) : 0;
+  const int tile0 = kv_lo / 16, n_tiles = (kv_end + 15) / 16 - tile0;
   const int tps = (n_tiles + p.n_splits - 1) / p.n_splits;
-  const int t_begin = tile0 + split * tps;
-  const int t_end = min(tile0 + n_tiles, t_begin + tps);
-  const T* qp = (const T*)p.q;
-  const T* kc = (const T*)p.k_cache;
-  const T* vc = (const T*)p.v_cache;
-  const int* table = p.block_tables + (int64_t)req * p.table_stride;
+  const int t_begin = tile0 + split * tps, t_end = min(tile0 + n_tiles, t_begin + tps);
+  const T* const qp = (const T*)p.q;
+  const T* const kc = (const T*)p.k_cache + (int64_t)kvh * HD;
+  const T* const vc = (const T*)p.v_cache + (int64_t)kvh * HD;
+  const int64_t row_stride = (int64_t)p.nkv * HD;
+  const int* const table = p.block_tables + (int64_t)req * p.table_stride;
 
-  // ---- query tile: row r = (token r / gh, head chunk * gh + r % gh); unused rows are zero
-  for (int idx = tid; idx < ROWS * HD; idx += 256) {
-    const int r = idx / HD, d = idx - r * HD;
-    const int tok = r / gh, hig = chunk * gh + (r - tok * gh);
-    float v = 0.0f;
-    if (tok < ntok && hig < group)
-      v = cw_to_float(qp[(int64_t)(q_begin + tok0 + tok) * p.q_stride + (kvh * group + hig) * HD + d]);
-    Qs[r * S::QS + d] = v;
+  // this lane's row of every block: its query, its last and first key
+  float qf[RB][KB][4];
+  int last_key[RB], first_key[RB];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    const int r = row0 + rb * 16 + c, tok = r / gh, hig = chunk * gh + (r - tok * gh);
+    const bool ok = r < rows && tok < ntok && hig < group;
+    last_key[rb] = ok ? pos0 + tok : -1;
+    first_key[rb] = p.window > 0 ? pos0 + tok - p.window + 1 : 0;
+    const T* q = qp + (int64_t)(q_begin + tok0 + (ok ? tok : tok_first)) * p.q_stride + (kvh * group + (ok ? hig : 0)) * HD + 4 * s;
+#pragma unroll
+    for (int b = 0; b < KB; ++b) {
+      // a row's start is not always a multiple of 16 bytes: the caller's stride decides
+#pragma unroll
+      for (int j = 0; j < 4; ++j) qf[rb][b][j] = ok ? cw_to_float(q[16 * b + j]) : 0.0f;
+    }
   }
-  if (tid < ROWS) { m_s[tid] = -INFINITY; l_s[tid] = 0.0f; a_s[tid] = 1.0f; }
 
-  // ---- output accumulators: thread = (dg: 4 consecutive columns, stripe: rows stripe + k * NSTRIPE)
-  constexpr int NDG = HD / 4;
-  constexpr int NSTRIPE = 256 / NDG;
-  constexpr int RPT = (ROWS + NSTRIPE - 1) / NSTRIPE;
-  const int dg = tid % NDG, stripe = tid / NDG;
-  const bool pv_active = stripe < NSTRIPE;
-  float acc[RPT][4];
+  // A tile's places in the cache: key c's and keys 4 s .. 4 s + 3's rows, -1 where the table names no page. Positions
+  // outside the range are moved to its edge: their scores are masked, and what is read lies in the request's own
+  // pages. Pages of a multiple of 16 keys hold a tile whole: one page for the wave then, by a scalar load.
+  const bool whole = !(p.block_size & 15);
+  auto places = [&](int t, int64_t (&at)[5]) __attribute__((always_inline)) {
+    int page = 0, page_first = 0;
+    if (whole) {
+      const int first = __builtin_amdgcn_readfirstlane(16 * t);
+      const int n = p.bs_shift >= 0 ? first >> p.bs_shift : first / p.block_size;
+      page = table[n];
+      page_first = n * p.block_size;
+    }
 #pragma unroll
-  for (int k = 0; k < RPT; ++k) { acc[k][0] = acc[k][1] = acc[k][2] = acc[k][3] = 0.0f; }
-
-  constexpr int VEC = Vec16<T>::N;
-  constexpr int CPR = HD / VEC;  // 16-byte chunks per cache row
-  constexpr int NRG = 256 / BN;  // row groups of the score phase
-  constexpr int RPT_S = ROWS / NRG;
-  constexpr int TPR = 256 / ROWS;  // threads per row of the softmax phase
-  static_assert(ROWS % NRG == 0 && 256 % ROWS == 0 && TPR <= 64, "tile shape");
-
-  __syncthreads();
-  for (int t = t_begin; t < t_end; ++t) {
-    const int kv0 = t * BN;
-    // ---- keys of the tile -> LDS as float32
-    for (int idx = tid; idx < BN * CPR; idx += 256) {
-      const int j = idx / CPR, ch = idx - j * CPR;
-      const int pos = kv0 + j;
-      float v[VEC];
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) v[e] = 0.0f;
-      if (pos >= kv_lo && pos < kv_end) {
-        const int page = table[pos / p.block_size];
-        if (page >= 0) {
-          const int64_t slot = (int64_t)page * p.block_size + pos % p.block_size;
-          Vec16<T>::load(kc + (slot * p.nkv + kvh) * HD + ch * VEC, v);
-        }
+    for (int i = 0; i < 5; ++i) {
+      const int pos = min(max(16 * t + (i == 0 ? c : 4 * s + i - 1), kv_lo), kv_end - 1);
+      int pg = page, off = pos - page_first;
+      if (!whole) {
+        pg = table[p.bs_shift >= 0 ? pos >> p.bs_shift : pos / p.block_size];
+        off = p.bs_shift >= 0 ? pos & (p.block_size - 1) : pos % p.block_size;
       }
+      at[i] = pg >= 0 ? (int64_t)pg * p.block_size + off : -1;
+    }
+  };
+  auto load = [&](const int64_t (&at)[5], float (&k)[KB][4], float (&v)[4][VG][VW]) __attribute__((always_inline)) {
+    const T* row = kc + max(at[0], (int64_t)0) * row_stride + 4 * s;
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) KVs[j * S::KS + ch * VEC + e] = v[e];
+    for (int b = 0; b < KB; ++b) attn_load<4>(row + 16 * b, k[b]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const T* vrow = vc + max(at[1 + j], (int64_t)0) * row_stride + VW * c;
+#pragma unroll
+      for (int g = 0; g < VG; ++g) attn_load<VW>(vrow + 16 * VW * g, v[j][g]);
+    }
+  };
+
+  attn_f32x4_t acc[RB][VG * VW];
+  float m[RB], l[RB];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    m[rb] = -INFINITY;
+    l[rb] = 0.0f;
+#pragma unroll
+    for (int e = 0; e < VG * VW; ++e) acc[rb][e] = (attn_f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
+  }
+
+  // one tile: ``at`` where it lay, ``k`` and ``v`` what lay there
+  auto compute = [&](int t, const int64_t (&at)[5], float (&k)[KB][4], float (&v)[4][VG][VW]) __attribute__((always_inline)) {
+    const int kv0 = 16 * t;
+    // no page: zeros
+    if (__builtin_amdgcn_ballot_w64(at[0] < 0 || at[1] < 0 || at[2] < 0 || at[3] < 0 || at[4] < 0)) {
+#pragma unroll
+      for (int b = 0; b < KB; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) k[b][j] = at[0] >= 0 ? k[b][j] : 0.0f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int g = 0; g < VG; ++g)
+#pragma unroll
+          for (int e = 0; e < VW; ++e) v[j][g][e] = at[1 + j] >= 0 ? v[j][g][e] : 0.0f;
+    }
+    attn_f32x4_t sc[RB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) sc[rb] = (attn_f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int b = 0; b < KB; ++b)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) sc[rb] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[b][j], qf[rb][b][j], sc[rb], 0, 0, 0);
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      float top = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int pos = kv0 + 4 * s + i;
+        sc[rb][i] = pos <= last_key[rb] && pos >= first_key[rb] ? sc[rb][i] * p.scale : -INFINITY;
+        top = fmaxf(top, sc[rb][i]);
+      }
+      const float m_new = fmaxf(m[rb], cw_quad_max(top));
+      const float ref = m_new == -INFINITY ? 0.0f : m_new;  // no key of the row yet: every weight is exp(-inf)
+      const float alpha = expf(m[rb] - ref);
+      m[rb] = m_new;
+      float sum = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        sc[rb][i] = expf(sc[rb][i] - ref);
+        sum += sc[rb][i];
+      }
+      l[rb] = fmaf(l[rb], alpha, sum);  // of this lane's keys; the four lanes of a row are added at the end
+#pragma unroll
+      for (int e = 0; e < VG * VW; ++e)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[rb][e][i] *= alpha;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int g = 0; g < VG; ++g)
+#pragma unroll
+        for (int e = 0; e < VW; ++e)
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb)
+            acc[rb][g * VW + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[j][g][e], sc[rb][j], acc[rb][g * VW + e], 0, 0, 0);
+  };
+  // Two tiles take turns: one is on its way while the other is multiplied, and the places of the one after are
+  // looked up meanwhile. Past the last tile the last one is asked for again: no load hangs on a condition.
+  const int t_first = t_begin + wave;
+  if constexpr (HD > 192) {  // two tiles do not fit the registers
+    float ka[KB][4], va[4][VG][VW];
+    int64_t at[5], next[5];
+    if (t_first < t_end) places(t_first, at);
+    for (int t = t_first; t < t_end; t += WAVES) {
+      load(at, ka, va);
+      places(t + WAVES < t_end ? t + WAVES : t, next);
+      compute(t, at, ka, va);
+#pragma unroll
+      for (int i = 0; i < 5; ++i) at[i] = next[i];
+    }
+  } else if (t_first < t_end) {
+    const int t_last = t_first + (t_end - 1 - t_first) / WAVES * WAVES;
+    float ka[KB][4], va[4][VG][VW], kb[KB][4], vb[4][VG][VW];
+    int64_t at_a[5], at_b[5];
+    places(t_first, at_a);
+    load(at_a, ka, va);
+    places(min(t_first + WAVES, t_last), at_b);
+    for (int t = t_first; t < t_end; t += 2 * WAVES) {
+      load(at_b, kb, vb);
+      int64_t next[5];
+      places(min(t + 2 * WAVES, t_last), next);
+      compute(t, at_a, ka, va);
+#pragma unroll
+      for (int i = 0; i < 5; ++i) at_a[i] = next[i];
+      if (t + WAVES >= t_end) break;
+      load(at_a, ka, va);
+      places(min(t + 3 * WAVES, t_last), next);
+      compute(t + WAVES, at_b, kb, vb);
+#pragma unroll
+      for (int i = 0; i < 5; ++i) at_b[i] = next[i];
+    }
+  }
+
+  // ---- the waves' results meet, one block of rows after the other: final rows when there is one split, partial sums
+  // otherwise
+  const int64_t base = ((int64_t)item * gridDim.y + blockIdx.y) * p.n_splits + split;
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    if (rb > 0) __syncthreads();
+    const float total = cw_quad_sum(l[rb]);
+    float* mine = o_s + (wave * 16 + c) * OS + 4 * VW * s;
+    // lane (c, s) holds, of row c, elements 16 VW g + VW (4 s + i) + e
+#pragma unroll
+    for (int g = 0; g < VG; ++g)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < VW; ++e) mine[16 * VW * g + VW * i + e] = acc[rb][g * VW + e][i];
+    if (s == 0) {
+      ml_s[(wave * 16 + c) * 2] = m[rb];
+      ml_s[(wave * 16 + c) * 2 + 1] = total;
     }
     __syncthreads();
-    // ---- scores: thread = (key c, row group rg), rows rg + k * NRG
-    {
-      const int c = tid % BN, rg = tid / BN;
-      float s[RPT_S];
+    for (int idx = threadIdx.x; idx < 16 * HD; idx += WAVES * 64) {
+      const int rr = idx / HD, d = idx - rr * HD;
+      const int r = row0 + rb * 16 + rr, tok = r / gh, hig = chunk * gh + (r - tok * gh);
+      if (r >= rows || tok >= ntok || hig >= group) continue;
+      float M = -INFINITY;
 #pragma unroll
-      for (int k = 0; k < RPT_S; ++k) s[k] = 0.0f;
-      const float* kr = KVs + c * S::KS;
-      for (int d0 = 0; d0 < HD; d0 += 4) {
-        const float k0 = kr[d0], k1 = kr[d0 + 1], k2 = kr[d0 + 2], k3 = kr[d0 + 3];
+      for (int w = 0; w < WAVES; ++w) M = fmaxf(M, ml_s[(w * 16 + rr) * 2]);
+      float L = 0.0f, O = 0.0f;
 #pragma unroll
-        for (int k = 0; k < RPT_S; ++k) {
-          const float4 qv = *reinterpret_cast<const float4*>(&Qs[(rg + k * NRG) * S::QS + d0]);
-          s[k] = fmaf(qv.x, k0, s[k]);
-          s[k] = fmaf(qv.y, k1, s[k]);
-          s[k] = fmaf(qv.z, k2, s[k]);
-          s[k] = fmaf(qv.w, k3, s[k]);
-        }
+      for (int w = 0; w < WAVES; ++w) {
+        const float mw = ml_s[(w * 16 + rr) * 2];
+        const float f = mw == -INFINITY ? 0.0f : expf(mw - M);
+        L = fmaf(ml_s[(w * 16 + rr) * 2 + 1], f, L);
+        O = fmaf(o_s[(w * 16 + rr) * OS + d], f, O);
       }
-      const int pos_k = kv0 + c;
-#pragma unroll
-      for (int k = 0; k < RPT_S; ++k) {
-        const int r = rg + k * NRG;
-        const int tok = r / gh, hig = chunk * gh + (r - tok * gh);
-        const int prow = pos0 + tok;
-        const int lo = p.window > 0 ? prow - p.window + 1 : 0;
-        const bool ok = tok < ntok && hig < group && pos_k <= prow && pos_k >= lo;
-        Ss[r * S::SS + c] = ok ? s[k] * p.scale : -INFINITY;
-      }
-    }
-    __syncthreads();
-    // ---- values of the tile -> LDS (the key rows are no longer read)
-    for (int idx = tid; idx < BN * CPR; idx += 256) {
-      const int j = idx / CPR, ch = idx - j * CPR;
-      const int pos = kv0 + j;
-      float v[VEC];
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) v[e] = 0.0f;
-      if (pos >= kv_lo && pos < kv_end) {
-        const int page = table[pos / p.block_size];
-        if (page >= 0) {
-          const int64_t slot = (int64_t)page * p.block_size + pos % p.block_size;
-          Vec16<T>::load(vc + (slot * p.nkv + kvh) * HD + ch * VEC, v);
-        }
-      }
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) KVs[j * S::VS + ch * VEC + e] = v[e];
-    }
-    // ---- online softmax: TPR consecutive lanes share a row
-    {
-      const int r = tid / TPR, sub = tid % TPR;
-      float* srow = Ss + r * S::SS;
-      float tmax = -INFINITY;
-      for (int c = sub; c < BN; c += TPR) tmax = fmaxf(tmax, srow[c]);
-#pragma unroll
-      for (int off = TPR / 2; off > 0; off >>= 1) tmax = fmaxf(tmax, __shfl_xor(tmax, off, 64));
-      const float m_old = m_s[r];
-      const float m_new = fmaxf(m_old, tmax);
-      float alpha = 1.0f, sum = 0.0f;
-      if (m_new == -INFINITY) {
-        for (int c = sub; c < BN; c += TPR) srow[c] = 0.0f;
+      if (p.n_splits == 1) {
+        ((T*)p.out)[(int64_t)(q_begin + tok0 + tok) * p.out_stride + (kvh * group + hig) * HD + d] = cw_from_float<T>(O * (1.0f / L));
       } else {
-        alpha = expf(m_old - m_new);
-        for (int c = sub; c < BN; c += TPR) {
-          const float e = expf(srow[c] - m_new);
-          srow[c] = e;
-          sum += e;
+        p.part_o[(base * rows + r) * HD + d] = O;
+        if (d == 0) {
+          p.part_ml[(base * rows + r) * 2] = M;
+          p.part_ml[(base * rows + r) * 2 + 1] = L;
         }
-      }
-#pragma unroll
-      for (int off = TPR / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-      if (sub == 0) {
-        m_s[r] = m_new;
-        l_s[r] = l_s[r] * alpha + sum;
-        a_s[r] = alpha;
-      }
-    }
-    __syncthreads();
-    // ---- out += P * V
-    if (pv_active) {
-#pragma unroll
-      for (int k = 0; k < RPT; ++k) {
-        const int r = stripe + k * NSTRIPE;
-        const float a = r < ROWS ? a_s[r] : 1.0f;
-        acc[k][0] *= a; acc[k][1] *= a; acc[k][2] *= a; acc[k][3] *= a;
-      }
-      for (int c = 0; c < BN; ++c) {
-        const float4 v = *reinterpret_cast<const float4*>(&KVs[c * S::VS + dg * 4]);
-#pragma unroll
-        for (int k = 0; k < RPT; ++k) {
-          const int r = stripe + k * NSTRIPE;
-          const float pr = r < ROWS ? Ss[r * S::SS + c] : 0.0f;
-          acc[k][0] = fmaf(pr, v.x, acc[k][0]);
-          acc[k][1] = fmaf(pr, v.y, acc[k][1]);
-          acc[k][2] = fmaf(pr, v.z, acc[k][2]);
-          acc[k][3] = fmaf(pr, v.w, acc[k][3]);
-        }
-      }
-    }
-    __syncthreads();
-  }
-
-  // ---- write: final rows when there is one split, partial sums otherwise
-  if (!pv_active) return;
-  if (p.n_splits == 1) {
-    T* op = (T*)p.out;
-#pragma unroll
-    for (int k = 0; k < RPT; ++k) {
-      const int r = stripe + k * NSTRIPE;
-      if (r >= ROWS) continue;
-      const int tok = r / gh, hig = chunk * gh + (r - tok * gh);
-      if (tok >= ntok || hig >= group) continue;
-      const float inv = 1.0f / l_s[r];
-      T* o = op + (int64_t)(q_begin + tok0 + tok) * p.out_stride + (kvh * group + hig) * HD + dg * 4;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = cw_from_float<T>(acc[k][e] * inv);
-    }
-  } else {
-    const int64_t base = ((int64_t)item * gridDim.y + blockIdx.y) * p.n_splits + split;
-#pragma unroll
-    for (int k = 0; k < RPT; ++k) {
-      const int r = stripe + k * NSTRIPE;
-      if (r >= ROWS) continue;
-      float* o = p.part_o + (base * ROWS + r) * HD + dg * 4;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = acc[k][e];
-      if (dg == 0) {
-        p.part_ml[(base * ROWS + r) * 2] = m_s[r];
-        p.part_ml[(base * ROWS + r) * 2 + 1] = l_s[r];
       }
     }
   }
@@ -354,31 +391,44 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
   }
 }
 
-template <typename T, int ROWS, int BN>
-static int launch_attention(const AttnParams& p, int n_items, hipStream_t stream) {
+template <typename T, int RB, int WAVES>
+static int launch_attention_rows(const AttnParams& p, int rows, int n_items, hipStream_t stream) {
   constexpr int HD = CW_HD;
-  const size_t smem = sizeof(float) * TileShape<HD, ROWS, BN>::FLOATS;
-  static int limit = -1;
-  if (limit < 0) {
-    int dev = 0, v = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return CW_ERR_LAUNCH;
-    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
-      return CW_ERR_LAUNCH;
-    limit = v;
-  }
-  if ((size_t)limit < smem) return CW_ERR_SIZE;
+  constexpr size_t smem = sizeof(float) * WAVES * 16 * (HD + 4 + 2);
   static bool raised = false;
-  if (!raised) {
-    if (hipFuncSetAttribute((const void*)attn_tile_kernel<T, HD, ROWS, BN>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+  if (smem > 65536 && !raised) {
+    if (hipFuncSetAttribute((const void*)attn_f32_kernel<T, HD, RB, WAVES>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)smem) != hipSuccess)
       return CW_ERR_LAUNCH;
     raised = true;
   }
-  dim3 grid(n_items, p.nkv * p.n_chunks, p.n_splits), block(256);
-  hipLaunchKernelGGL((attn_tile_kernel<T, HD, ROWS, BN>), grid, block, smem, stream, p);
+  const int subs = rows / (16 * RB);
+  if ((int64_t)n_items * subs > 0x7fffffff) return CW_ERR_SIZE;
+  const dim3 grid(n_items * subs, p.nkv * p.n_chunks, p.n_splits);
+  hipLaunchKernelGGL((attn_f32_kernel<T, HD, RB, WAVES>), grid, dim3(WAVES * 64), smem, stream, p, rows, subs);
+  return cw_launch_status();
+}
+
+// 32 rows a workgroup (four waves) where that still gives every compute unit two workgroups, else 16 rows (eight waves).
+// Measured on an MI355X, float32, us a call, before (vector-unit tiles of 64 rows and 64 keys in LDS) and now: heads of
+// 64, 14 on 2: 17 tokens 24 -> 8.8, 300 97 -> 17.5, 1000 298 -> 58; heads of 128, 12 on 2: 300 tokens 174 -> 23, 2048
+// 1571 -> 229 (16 rows: 283); one token behind 300 keys 33 -> 10.3, 8 behind 2048 (8 parts) 62 -> 22.5.
+template <typename T, int ROWS>
+static int launch_attention(const AttnParams& p, int n_items, hipStream_t stream) {
+  constexpr int HD = CW_HD;
+  int rc;
+  if constexpr (HD > 128) {  // registers for four waves of 16 rows only
+    rc = launch_attention_rows<T, 1, 4>(p, ROWS, n_items, stream);
+  } else if constexpr (ROWS == 64) {
+    const int64_t pairs = (int64_t)n_items * p.nkv * p.n_chunks * p.n_splits * 2;  // workgroups of 32 rows
+    rc = pairs >= 512 ? launch_attention_rows<T, 2, 4>(p, ROWS, n_items, stream) : launch_attention_rows<T, 1, 8>(p, ROWS, n_items, stream);
+  } else {
+    rc = launch_attention_rows<T, 1, 8>(p, ROWS, n_items, stream);
+  }
+  if (rc != CW_OK) return rc;
   if (p.n_splits > 1) {
     dim3 mgrid(n_items, p.nkv * p.n_chunks, (ROWS * HD + 255) / 256);
-    hipLaunchKernelGGL((attn_merge_kernel<T, HD, ROWS>), mgrid, block, 0, stream, p);
+    hipLaunchKernelGGL((attn_merge_kernel<T, HD, ROWS>), mgrid, dim3(256), 0, stream, p);
   }
   return cw_launch_status();
 }
@@ -391,7 +441,7 @@ CW_EXPORT int64_t cw_attention_workspace_floats(int rows, int n_items, int nkv, 
   return (int64_t)n_items * nkv * n_chunks * n_splits * rows * (CW_HD + 2);
 }
 
-// rows: 64 (portions of prompts) or 16 (single tokens, few tokens). gh * tokens-per-item <= rows.
+// rows of an item: 64 (portions of prompts) or 16 (single tokens, few tokens). gh * tokens-per-item <= rows.
 CW_EXPORT int cw_attention(int rows, int dtype, const void* q, int64_t q_stride, void* out,
                            int64_t out_stride, const void* k_cache, const void* v_cache,
                            const int* block_tables, int table_stride, const int* ctx_lens,
@@ -417,13 +467,10 @@ CW_EXPORT int cw_attention(int rows, int dtype, const void* q, int64_t q_stride,
   p.part_o = workspace;
   p.part_ml = workspace ? workspace + n_o : nullptr;
   p.zeros = nullptr;
-  constexpr int BN = CW_HD <= 128 ? 64 : 32;
   if (dtype == CW_F32) {
-    return rows == 64 ? launch_attention<float, 64, BN>(p, n_items, stream)
-                      : launch_attention<float, 16, BN>(p, n_items, stream);
+    return rows == 64 ? launch_attention<float, 64>(p, n_items, stream) : launch_attention<float, 16>(p, n_items, stream);
   } else if (dtype == CW_BF16) {
-    return rows == 64 ? launch_attention<bf16_t, 64, BN>(p, n_items, stream)
-                      : launch_attention<bf16_t, 16, BN>(p, n_items, stream);
+    return rows == 64 ? launch_attention<bf16_t, 64>(p, n_items, stream) : launch_attention<bf16_t, 16>(p, n_items, stream);
   }
   return CW_ERR_DTYPE;
 }

@@ -67,10 +67,11 @@ def portions_have_short_ranges(q_lens, ctx_lens) -> bool:
 # is cut into at most this many parts
 MIN_PART_KEYS = 256
 MAX_PARTS = 64
-# keys of a tile of the float32 kernel for single tokens: a workgroup takes about 8 us for one and they follow
-# one another, while the kernel that merges the parts takes 5 us however many there are (one request of 300 keys
-# of the 0.5B shape: 34 + 5 us with parts of 256 keys, 14 + 5 with parts of 64)
-TILE_KEYS = 64
+# Parts of a single token's keys for the float32 kernel: a workgroup of eight waves takes 128 keys in one turn of some
+# 1.5 us, and the kernel that merges the parts takes 4 us however many there are. Up to 384 keys stay whole (one
+# request of the 0.5B shape, one part / parts of 128 keys: 300 keys 10.3 / 10.5 us, 510 keys 12.9 / 10.9).
+F32_PART_KEYS = 128
+F32_WHOLE_KEYS = 384
 
 
 def _share_long_key_ranges(items: np.ndarray, ctx, workgroups_per_item: int):
@@ -173,10 +174,11 @@ def _make_plan(ctx, nh: int, nkv: int, narrow_ok: bool, whole_keys: int = 0) -> 
         plan.wide_splits = int(max(1, min(spare, most_keys // MIN_PART_KEYS, MAX_PARTS)))
     plan.chunks_single = -(-group // gh_single)
     if plan.n_single:
-        groups_running = plan.n_single * nkv * plan.chunks_single
-        by_occupancy = -(-4 * ctx.num_compute_units // groups_running)
-        by_length = max(1, longest_single // TILE_KEYS)
-        plan.single_splits = max(1, min(by_occupancy, by_length, 64))
+        # as many parts as still give every workgroup a compute unit of its own (64 requests of 1500 keys, heads of
+        # 128 on 2 kv heads: 42 us with 2 parts, 47 with 4, 62 with 8)
+        by_occupancy = ctx.num_compute_units // (plan.n_single * nkv * plan.chunks_single)
+        plan.single_splits = 1 if longest_single <= min(F32_WHOLE_KEYS, whole_keys) else max(
+            1, min(by_occupancy, longest_single // F32_PART_KEYS, 64))
         # decode kernel: a workgroup per (request, kv head, split); a split is at least 128 keys
         # (one 32-key tile for each of its four waves). As many splits as still give every
         # workgroup a compute unit of its own: one more and some units run a second round (24

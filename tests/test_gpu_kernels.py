@@ -914,6 +914,29 @@ def test_attention_window(dtype, window):
         at += q_len
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("nh,nkv,hd,bs,q_len,ctx,window,key_parts", [
+    (16, 16, 16, 16, 1030, 1030, 0, 0),   # 32 rows a workgroup (512 of them or more), whole pages of 16
+    (14, 2, 64, 24, 1100, 1110, 0, 3),    # the same, pages that hold no whole tiles, parts, groups of 7
+    (14, 2, 64, 16, 47, 63, 0, 0),        # 16 rows a workgroup, fewer tiles than waves
+    (12, 2, 128, 32, 131, 700, 100, 2),   # a window that begins inside a tile, behind cached keys
+    (2, 1, 160, 16, 65, 129, 0, 0),       # four waves, two tiles in flight
+    (2, 1, 256, 4, 65, 129, 0, 2),        # four waves, one tile in flight
+])
+def test_attention_rows_on_the_matrix_cores(dtype, nh, nkv, hd, bs, q_len, ctx, window, key_parts):
+    """The workgroup shapes of the float32-accumulating kernel against float64. float32 rounds at 6e-8: a score
+    of ``hd`` products and a sum over ``ctx`` keys some sqrt(hd) + sqrt(ctx) times, 49 at most, so 3e-6 and a
+    third for the exponentials (2-norm); bfloat16 adds its results' own rounding, 2^-9."""
+    n_blocks = -(-ctx // bs)
+    table = torch.randperm(n_blocks + 3).tolist()[:n_blocks]
+    kc, vc, ks, vs = _paged_setup(dtype, nkv, hd, bs, n_blocks + 3, [table], [ctx], poison=float("nan"))
+    q = torch.randn(q_len, nh, hd, device=DEV).to(dtype)
+    out = _run_attention(dtype, nh, nkv, hd, bs, [table], [ctx], [q_len], kc, vc, [q], window=window, key_parts=key_parts)
+    want = plain.attention_dense(q.double().cpu(), ks[0].double().cpu(), vs[0].double().cpu(), hd ** -0.5, window=window or None)
+    error = (out.double().cpu() - want).norm() / want.norm()
+    assert error < (4e-6 if dtype == torch.float32 else 2.0 ** -9 + 4e-6)
+
+
 # sizes of the bfloat16 decode kernel: head sizes 32..256, groups of 1 to 20 heads, pages of 4 to 32
 DECODE_KERNEL_CASES = [
     (8, 2, 32, 4, [1, 7, 16, 3]),
