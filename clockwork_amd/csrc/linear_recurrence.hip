@@ -35,7 +35,7 @@ struct LinRecForm {
 __device__ __forceinline__ float lr_decay(float z, int kind, float inv_tau) {
   if (kind >= 1) return expf(-expf(z));
   // log(sigmoid(z)) without cancellation, then the 1/tau-th power
-  const float ls = z < 0.0f ? z - log1pf(expf(z)) : -log1pf(expf(-z));
+  const float ls = fminf(z, 0.0f) - log1pf(expf(-fabsf(z)));
   return expf(ls * inv_tau);
 }
 
@@ -402,7 +402,8 @@ CW_EXPORT int cw_linear_recurrence(int dtype, const void* proj, int64_t stride, 
 }
 
 // ======================================================================================
-// The same recurrence for long portions, cut into segments of tokens that run side by side.
+// The same recurrence for long portions, cut into segments of tokens that run side by side. (Sizes that the matrix
+// cores take run on the kernels behind these.)
 //
 //   prepare:   per token and key channel the decay a (float32, through log-sigmoid), the scaled
 //              query and the key as float32 rows [T, heads * dim]: the walks below read them
@@ -678,6 +679,401 @@ __global__ __launch_bounds__(256) void lrs_finish_kernel(SegParams p) {
   }
 }
 
+// ======================================================================================
+// The same on the matrix cores, for segments of up to 32 tokens, dim 16, 32, 64 or 128 and vdim a multiple of
+// 16 up to 256, all in float32 (v_mfma_f32_16x16x4_f32). Within a chunk of 16 tokens
+//   o_t = (q_t * A_t)^T S + sum over j <= t of P[t][j] v_j,   S' = diag(A_16) S + sum over j of (k_j * Z_j) v_j^T
+// with A_t the product of the chunk's decays up to t, Z_j that of those behind j and P[t][j] = sum over d of
+// q_t[d] k_j[d] (the product of the decays behind j up to t)[d]. Every factor is a product of decays, each at most 1,
+// as in the walk: nothing is divided, so a decay that vanishes makes zeros and no infinity.
+//
+//   added:    (segment, head): decays (kept for ``outputs``), keys times the decays behind them, added = K'^T V.
+//   carry:    as above.
+//   outputs:  (segment, head): P on the vector unit, one thread a key and a run of channels, walking the chunk's
+//             tokens; the products; norm over vdim, gate and cast.
+// The walk takes 192 vector instructions and 48 reads of LDS a token, channel and column of 64; what bounds these
+// two kernels is a chain of trips to memory and LDS a workgroup, with three workgroups a compute unit beside each other.
+// Measured on an MI355X, 2048 tokens, 12 heads of 64 x 128, rank 32, bfloat16: prepare 21, walks 64 + 72, finish 14 and carry
+// 17 us before, added 21, outputs 32 and carry 17 now; one call 188 -> 69 us, of 100 tokens (14 heads of 64 x 64) 133 -> 27.
+// A wave owns 16 * VT columns; lane (c, s) = (l % 16, l / 16) holds, of a tile of the state, channels 4 s .. 4 s + 3 of
+// column c, which is also what a product that contracts over channels wants of it.
+typedef __attribute__((ext_vector_type(4))) float lrs_f32x4_t;
+#define LRS_MFMA_SEG 32
+#define LRS_MAX_STAGED 128  // ranks whose decay inputs the first kernel brings to LDS
+
+// sum over the 16 lanes of a row of the wave; every lane gets it
+__device__ __forceinline__ float lrs_row_sum(float v) {
+#define LRS_ROR(n) v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + (n), 0xf, 0xf, true))
+  LRS_ROR(8);
+  LRS_ROR(4);
+  LRS_ROR(2);
+  LRS_ROR(1);
+#undef LRS_ROR
+  return v;
+}
+
+// Elements of the wave's columns as a product's operand or result: token 16 b + 4 s + j, column col0 + 16 vt + c, of the
+// head's columns from ``off`` on; zeros past the segment's tokens and past vdim (read from a place inside, so that no load
+// hangs on a condition: one trip to memory for all of them).
+template <typename T, int VT>
+__device__ __forceinline__ void lrs_load_columns(const SegParams& p, int off, int64_t row0, int nt, int h, int col0, int c, int s,
+                                                 float (&vf)[2][4][VT]) {
+  const T* v = (const T*)p.proj + off + h * p.vdim + c;
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt) {
+        const int t = 16 * b + 4 * s + j, col = col0 + 16 * vt;
+        vf[b][j][vt] = cw_to_float(v[(row0 + min(t, nt - 1)) * p.stride + (col < p.vdim ? col : 0)]);
+        vf[b][j][vt] = t < nt && col < p.vdim ? vf[b][j][vt] : 0.0f;
+      }
+}
+
+template <typename T, int D, int VT>
+__global__ __launch_bounds__(256) void lrs_added_kernel(SegParams p) {
+  constexpr int LD = D + 4, G = 256 / D, TPG = LRS_MFMA_SEG / G;  // a thread makes TPG tokens' decays of one channel
+  __shared__ __align__(16) float keys[LRS_MFMA_SEG * LD];
+  __shared__ float total[G * D];
+  const int seg = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, s = lane >> 4;
+  const int r = p.seg_items[4 * seg], tok0 = p.seg_items[4 * seg + 1], ntok = p.seg_items[4 * seg + 2];
+  const int begin = p.cu_q[r], q_len = p.cu_q[r + 1] - begin;
+  const int slot = p.state_slots[r];
+  if (tok0 >= q_len || slot < 0 || slot >= p.n_slots) return;
+  const int nt = min(ntok, q_len - tok0);
+  const int64_t row0 = begin + tok0;
+  const int col0 = wave * 16 * VT;
+  float vf[2][4][VT];
+  lrs_load_columns<T, VT>(p, p.v_off, row0, nt, h, col0, c, s, vf);
+
+  const int d = tid % D, g = tid / D, t0 = g * TPG, channel = h * D + d;
+  const T* proj = (const T*)p.proj;
+  const T* w = (const T*)p.a2 + (int64_t)channel * p.rank;
+  constexpr int N = LrVec<T>::N;
+  const bool vec = p.form.decay_kind != 2 && p.rank % N == 0 && p.rank <= LRS_MAX_STAGED && !((uintptr_t)p.a2 & 15) &&
+                   (p.form.u ? p.form.u_stride % N == 0 && !((uintptr_t)p.form.u & 15)
+                             : p.u_off % N == 0 && p.stride % N == 0 && !((uintptr_t)proj & 15));
+  const T* u = p.form.u ? (const T*)p.form.u : proj + p.u_off;
+  const int64_t u_stride = p.form.u ? p.form.u_stride : p.stride;
+  float z[TPG], k[TPG];
+  const float bias = p.a2b ? p.a2b[channel] : 0.0f;
+#pragma unroll
+  for (int i = 0; i < TPG; ++i) {
+    z[i] = bias;
+    k[i] = cw_to_float(proj[(row0 + min(t0 + i, nt - 1)) * p.stride + p.k_off + channel]);
+  }
+  if (vec) {  // 16 bytes of the channel's row and of each token's decay input at a time
+    // (the tokens' inputs through LDS, as they are: every wave wants all of them)
+    extern __shared__ __align__(16) unsigned char staged[];
+    T* us = (T*)staged;
+    const int pieces = p.rank / N;
+    float wv[N];
+    LrVec<T>::load(w, wv);
+    for (int i = tid; i < LRS_MFMA_SEG * pieces; i += 256)
+      reinterpret_cast<uint4*>(us)[i] = *reinterpret_cast<const uint4*>(u + (row0 + min(i / pieces, nt - 1)) * u_stride + i % pieces * N);
+    __syncthreads();
+    for (int e = 0; e < p.rank; e += N) {
+      float next[N];
+      LrVec<T>::load(w + min(e + N, p.rank - N), next);
+#pragma unroll
+      for (int i = 0; i < TPG; ++i) {
+        float uv[N];
+        LrVec<T>::load(us + (t0 + i) * p.rank + e, uv);
+#pragma unroll
+        for (int n = 0; n < N; ++n) z[i] += wv[n] * uv[n];
+      }
+#pragma unroll
+      for (int n = 0; n < N; ++n) wv[n] = next[n];
+    }
+  } else {
+    for (int e = 0; e < p.rank; ++e) {
+      const float we = cw_to_float(w[e]);
+#pragma unroll
+      for (int i = 0; i < TPG; ++i) {
+        const float ue = cw_to_float(u[(row0 + min(t0 + i, nt - 1)) * u_stride + e]);
+        z[i] += we * (p.form.decay_kind == 2 ? tanhf(ue) : ue);
+      }
+    }
+  }
+  float run = 1.0f;  // the decays behind token i, of this thread's tokens
+#pragma unroll
+  for (int i = TPG - 1; i >= 0; --i) {
+    const float a = lr_decay(z[i], p.form.decay_kind, p.inv_tau);
+    k[i] = t0 + i < nt ? k[i] * run : 0.0f;
+    if (t0 + i < nt) p.dec[(row0 + t0 + i) * (int64_t)(p.heads * D) + channel] = a;
+    run *= t0 + i < nt ? a : 1.0f;
+  }
+  total[tid] = run;
+  __syncthreads();
+  float behind = 1.0f;
+  for (int i = g + 1; i < G; ++i) behind *= total[i * D + d];
+#pragma unroll
+  for (int i = 0; i < TPG; ++i) keys[(t0 + i) * LD + d] = k[i] * behind;
+  if (g == 0) p.seg_decay[((int64_t)seg * p.heads + h) * D + d] = run * behind;
+  __syncthreads();
+  float* mine = p.added + (((int64_t)seg * p.heads + h) * D) * p.vdim + col0 + c;
+#pragma unroll
+  for (int dt = 0; dt < D / 16; ++dt) {
+    lrs_f32x4_t acc[VT];
+#pragma unroll
+    for (int vt = 0; vt < VT; ++vt) acc[vt] = (lrs_f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float a = keys[(16 * b + 4 * s + j) * LD + 16 * dt + c];
+#pragma unroll
+        for (int vt = 0; vt < VT; ++vt) acc[vt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, vf[b][j][vt], acc[vt], 0, 0, 0);
+      }
+#pragma unroll
+    for (int vt = 0; vt < VT; ++vt)
+      if (col0 + 16 * vt < p.vdim)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mine[(int64_t)(16 * dt + 4 * s + i) * p.vdim + 16 * vt] = acc[vt][i];
+  }
+}
+
+template <typename T, int D, int VT>
+__global__ __launch_bounds__(256, D * VT <= 128 ? 3 : 1) void lrs_outputs_kernel(SegParams p) {
+  constexpr int LD = D + 4, DT = D / 16, PER = D / 16;  // PER: channels of a thread while P is made
+  constexpr int UNITS = (4 * D + 255) / 256;            // runs of 8 tokens of a channel that a thread scales
+  __shared__ __align__(16) float As[LRS_MFMA_SEG * LD], Qs[LRS_MFMA_SEG * LD], Ks[LRS_MFMA_SEG * LD];
+  __shared__ __align__(16) float Ps[2 * 16 * 20], chunk_decay[2 * D];
+  __shared__ float squares[4 * LRS_MFMA_SEG];
+  const int seg = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, s = lane >> 4;
+  const int r = p.seg_items[4 * seg], tok0 = p.seg_items[4 * seg + 1], ntok = p.seg_items[4 * seg + 2];
+  const int begin = p.cu_q[r], q_len = p.cu_q[r + 1] - begin;
+  const int slot = p.state_slots[r];
+  if (tok0 >= q_len || slot < 0 || slot >= p.n_slots) return;
+  const int nt = min(ntok, q_len - tok0);
+  const int64_t row0 = begin + tok0;
+  const int V = p.vdim, col0 = wave * 16 * VT;
+  const bool before = p.form.bonus != nullptr;  // the output reads the state before the token joins it
+  const T* proj = (const T*)p.proj;
+
+  // decays, queries and keys of the segment; past its tokens decays of 1 and zeros
+  constexpr int PIECES = LRS_MFMA_SEG * D / 256;
+  {
+    float a[PIECES], q[PIECES], k[PIECES];
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const int idx = tid + 256 * i, t = idx / D, d = idx - t * D;
+      const bool ok = t < nt;
+      const int64_t row = row0 + (ok ? t : 0);
+      const int channel = h * D + d;
+      a[i] = p.dec[row * (int64_t)(p.heads * D) + channel];
+      q[i] = cw_to_float(proj[row * p.stride + p.q_off + channel]);
+      k[i] = cw_to_float(proj[row * p.stride + p.k_off + channel]);
+      a[i] = ok ? a[i] : 1.0f;
+      q[i] = ok ? q[i] * p.q_scale : 0.0f;
+      k[i] = ok ? k[i] : 0.0f;
+    }
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const int idx = tid + 256 * i, at = idx / D * LD + idx % D;
+      As[at] = a[i];
+      Qs[at] = q[i];
+      Ks[at] = k[i];
+    }
+  }
+  // what the products and the end need is asked for meanwhile
+  float vf[2][4][VT];
+  lrs_load_columns<T, VT>(p, p.v_off, row0, nt, h, col0, c, s, vf);
+  lrs_f32x4_t S[DT][VT];
+  const float* start = p.added + (((int64_t)seg * p.heads + h) * D) * V + col0 + c;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int vt = 0; vt < VT; ++vt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const bool live = col0 + 16 * vt < V;
+        const float v = start[(int64_t)(16 * dt + 4 * s + i) * V + (live ? 16 * vt : -col0)];
+        S[dt][vt][i] = live ? v : 0.0f;
+      }
+  float gate[2][4][VT], nw[VT];
+  if (p.g_off >= 0) lrs_load_columns<T, VT>(p, p.g_off, row0, nt, h, col0, c, s, gate);
+#pragma unroll
+  for (int vt = 0; vt < VT; ++vt) nw[vt] = p.norm_w && col0 + 16 * vt < V ? p.norm_w[h * p.form.norm_w_stride + col0 + 16 * vt + c] : 1.0f;
+  __syncthreads();
+
+  {  // P: thread = (key j of the chunk, run of PER channels), the 16 runs in neighbouring lanes
+    const int j = tid >> 4, run = tid & 15;
+    float bonus[PER];
+#pragma unroll
+    for (int e = 0; e < PER; ++e) bonus[e] = before ? p.form.bonus[h * D + run * PER + e] : 1.0f;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      if (16 * b >= nt) break;
+      float w[PER], mine = 0.0f;
+#pragma unroll
+      for (int e = 0; e < PER; ++e) w[e] = Ks[(16 * b + j) * LD + run * PER + e];
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        const float* a = As + (16 * b + t) * LD + run * PER;
+        const float* q = Qs + (16 * b + t) * LD + run * PER;
+        float sum = 0.0f;
+#pragma unroll
+        for (int e = 0; e < PER; ++e) {
+          const float decayed = t > j ? w[e] * a[e] : w[e];
+          sum += q[e] * (before ? (t == j ? bonus[e] * w[e] : w[e]) : decayed);
+          w[e] = decayed;
+        }
+        sum = lrs_row_sum(sum);
+        mine = t == run ? sum : mine;
+      }
+      Ps[(16 * b + run) * 20 + j] = run >= j ? mine : 0.0f;  // (a later key has no part in it, whatever it holds)
+    }
+  }
+  // queries times the decays up to them, keys times those behind them, chunk by chunk
+  float qn[UNITS][8], kn[UNITS][8], all[UNITS];
+#pragma unroll
+  for (int n = 0; n < UNITS; ++n) {
+    const int unit = tid + 256 * n;
+    const int d = unit % D, half = unit / D & 1, b = unit / (2 * D);
+    if (b > 1) break;
+    float other = 1.0f, a[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      a[i] = As[(16 * b + 8 * half + i) * LD + d];
+      other *= As[(16 * b + 8 * (1 - half) + i) * LD + d];
+    }
+    float up = half ? other : 1.0f, down = half ? 1.0f : other;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float with = up * a[i];
+      qn[n][i] = Qs[(16 * b + 8 * half + i) * LD + d] * (before ? up : with);
+      up = with;
+    }
+#pragma unroll
+    for (int i = 7; i >= 0; --i) {
+      kn[n][i] = Ks[(16 * b + 8 * half + i) * LD + d] * down;
+      down *= a[i];
+    }
+    all[n] = down;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int n = 0; n < UNITS; ++n) {
+    const int unit = tid + 256 * n;
+    const int d = unit % D, half = unit / D & 1, b = unit / (2 * D);
+    if (b > 1) break;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      Qs[(16 * b + 8 * half + i) * LD + d] = qn[n][i];
+      Ks[(16 * b + 8 * half + i) * LD + d] = kn[n][i];
+    }
+    if (!half) chunk_decay[b * D + d] = all[n];
+  }
+  __syncthreads();
+
+  lrs_f32x4_t o[2][VT];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+#pragma unroll
+    for (int vt = 0; vt < VT; ++vt) o[b][vt] = (lrs_f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
+    if (16 * b >= nt) continue;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      const lrs_f32x4_t q = *reinterpret_cast<const lrs_f32x4_t*>(Qs + (16 * b + c) * LD + 16 * dt + 4 * s);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int vt = 0; vt < VT; ++vt) o[b][vt] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i], S[dt][vt][i], o[b][vt], 0, 0, 0);
+    }
+    bool finite = true;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt) finite = finite && fabsf(vf[b][j][vt]) < INFINITY;
+    if (__builtin_amdgcn_ballot_w64(!finite) == 0) {
+      const lrs_f32x4_t w = *reinterpret_cast<const lrs_f32x4_t*>(Ps + (16 * b + c) * 20 + 4 * s);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int vt = 0; vt < VT; ++vt) o[b][vt] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j], vf[b][j][vt], o[b][vt], 0, 0, 0);
+    } else {  // an infinite value must not meet the zeros of the tokens before it
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+#pragma unroll
+        for (int vt = 0; vt < VT; ++vt) {
+          const float v = __shfl(vf[b][j % 4][vt], (j / 4) * 16 + c, 64);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (4 * s + i >= j) o[b][vt][i] = fmaf(Ps[(16 * b + 4 * s + i) * 20 + j], v, o[b][vt][i]);
+        }
+    }
+    if (b == 0 && nt > 16) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const lrs_f32x4_t a = *reinterpret_cast<const lrs_f32x4_t*>(chunk_decay + 16 * dt + 4 * s);
+#pragma unroll
+        for (int vt = 0; vt < VT; ++vt) S[dt][vt] *= a;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float k = Ks[(4 * s + j) * LD + 16 * dt + c];
+#pragma unroll
+          for (int vt = 0; vt < VT; ++vt) S[dt][vt] = __builtin_amdgcn_mfma_f32_16x16x4f32(k, vf[0][j][vt], S[dt][vt], 0, 0, 0);
+        }
+      }
+    }
+  }
+
+  if (p.norm_w) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int vt = 0; vt < VT; ++vt) ss += o[b][vt][i] * o[b][vt][i];
+        ss = lrs_row_sum(ss);
+        if (c == 0) squares[wave * LRS_MFMA_SEG + 16 * b + 4 * s + i] = ss;
+      }
+    __syncthreads();
+  }
+  T* out = (T*)p.out;
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t = 16 * b + 4 * s + i;
+      if (t >= nt) continue;
+      float inv = 1.0f;
+      if (p.norm_w) {
+        const float* sq = squares + t;
+        inv = 1.0f / sqrtf(((sq[0] + sq[LRS_MFMA_SEG]) + (sq[2 * LRS_MFMA_SEG] + sq[3 * LRS_MFMA_SEG])) / (float)V + p.eps);
+      }
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt) {
+        const int col = col0 + 16 * vt + c;
+        if (col0 + 16 * vt >= V) continue;
+        float val = o[b][vt][i] * inv * nw[vt];
+        if (p.g_off >= 0) val *= gate[b][i][vt] / (1.0f + expf(-gate[b][i][vt]));
+        out[(row0 + t) * (int64_t)(p.heads * V) + h * V + col] = cw_from_float<T>(val);
+      }
+    }
+}
+
+template <typename T, int D>
+static void lrs_launch_mfma(const SegParams& p, int n_segments, dim3 carry_grid, hipStream_t stream) {
+  const dim3 grid(n_segments, p.heads), block(256);
+  const size_t staged = p.rank <= LRS_MAX_STAGED ? (size_t)LRS_MFMA_SEG * p.rank * sizeof(T) : 0;
+#define LRS_VT(VT_)                                                                                  \
+  do {                                                                                               \
+    hipLaunchKernelGGL((lrs_added_kernel<T, D, VT_>), grid, block, staged, stream, p);                  \
+    hipLaunchKernelGGL(lrs_carry_kernel, carry_grid, block, 0, stream, p);                           \
+    hipLaunchKernelGGL((lrs_outputs_kernel<T, D, VT_>), grid, block, 0, stream, p);                  \
+  } while (0)
+  if (p.vdim <= 64) LRS_VT(1);
+  else if (p.vdim <= 128) LRS_VT(2);
+  else LRS_VT(4);
+#undef LRS_VT
+}
+
 // dim a multiple of 4 up to 128
 CW_EXPORT int cw_linear_recurrence_segments_supported(int dim, int vdim) {
   return dim > 0 && dim <= LRS_MAX_DIM && dim % 4 == 0 && vdim > 0 ? 1 : 0;
@@ -731,6 +1127,21 @@ CW_EXPORT int cw_linear_recurrence_segments(int dtype, const void* proj, int64_t
   const size_t walk_lds = (size_t)3 * seg_tokens * dim * sizeof(float);
   const dim3 carry_grid(n_requests, heads, (unsigned)(((int64_t)dim * vdim + 255) / 256));
   const unsigned finish_blocks = (unsigned)(((int64_t)n_tokens * heads + 3) / 4);
+  // segments that the matrix cores take whole
+  if (seg_tokens <= LRS_MFMA_SEG && (dim == 16 || dim == 32 || dim == 64 || dim == 128) && vdim % 16 == 0 && vdim <= 256) {
+#define CW_MFMA(T_)                                                                       \
+  do {                                                                                    \
+    if (dim == 16) lrs_launch_mfma<T_, 16>(p, n_segments, carry_grid, stream);            \
+    else if (dim == 32) lrs_launch_mfma<T_, 32>(p, n_segments, carry_grid, stream);       \
+    else if (dim == 64) lrs_launch_mfma<T_, 64>(p, n_segments, carry_grid, stream);       \
+    else lrs_launch_mfma<T_, 128>(p, n_segments, carry_grid, stream);                     \
+  } while (0)
+    if (dtype == CW_F32) CW_MFMA(float);
+    else if (dtype == CW_BF16) CW_MFMA(bf16_t);
+    else return CW_ERR_DTYPE;
+#undef CW_MFMA
+    return cw_launch_status();
+  }
 #define CW_WALK(T_, DIM_)                                                                          \
   do {                                                                                             \
     hipLaunchKernelGGL((lrs_walk_kernel<T_, DIM_, 0>), walk_grid, dim3(walk_threads), walk_lds, stream, p); \

@@ -7,7 +7,8 @@ of the step; one kernel walks each request's tokens in order from the request's 
 (sigmoid(z)^(1/tau) through log-sigmoid, float32), norms and gates the outputs; output product.
 A step with a portion of more than 64 tokens cuts every request's tokens into segments of 32 that
 are walked side by side: each from a zero state, then the start states are carried from segment
-to segment, then each segment is walked again for its outputs (the same sums, other parentheses).
+to segment, then each segment gives its outputs (the same sums, other parentheses; in chunks of 16
+tokens on the matrix cores for key sizes of 16, 32, 64 and 128).
 The state is all the mixer keeps: a ``StateSpec``.
 """
 

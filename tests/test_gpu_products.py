@@ -459,6 +459,76 @@ def test_recurrence_of_infinite_values(dim, vdim, with_bonus):
     assert bool((state[0, 0, :, 3] == float("inf")).all()) and bool((state[0, 0, :, 6] == -float("inf")).all())
 
 
+# the matrix-core kernels' sizes (one to eight tiles of 16 channels, columns for one wave to four of four tiles each, waves
+# without columns), and two that the walks take; requests of less than a chunk, of whole and of broken segments
+@pytest.mark.parametrize("dim,vdim,rank", [(64, 128, 32), (16, 16, 5), (32, 256, 16), (128, 64, 8), (128, 192, 24), (64, 48, 3), (100, 32, 5), (64, 40, 8)])
+@pytest.mark.parametrize("form", ["sigmoid_power", "bonus", "double_exp"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_recurrence_in_segments(dim, vdim, rank, form, dtype):
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(dim + vdim)
+    heads, lens, f64 = 2, [70, 0, 33, 5, 64], torch.float64
+    T, width = sum(lens), 2 * (2 * dim + 2 * vdim) + rank
+    width += -width % 8
+    proj = (torch.randn(T, width, device=DEV, generator=gen) * 0.7).to(dtype)
+    a2 = (torch.randn(heads * dim, rank, device=DEV, generator=gen) * 0.5).to(dtype)
+    a2b, bonus = (torch.randn(heads * dim, device=DEV, generator=gen) for _ in range(2))
+    if form == "double_exp":
+        a2b[::3] = 6.0   # decays that vanish (exp(-400)): zeros, not infinities
+    norm = torch.rand(vdim, device=DEV, generator=gen) + 0.5
+    start = torch.randn(6, heads, dim, vdim, device=DEV, generator=gen)
+    ints = lambda *t: torch.tensor(t, dtype=torch.int32, device=DEV)  # noqa: E731
+    slots, cu = [4, 0, 2, 5, 1], [0, 70, 70, 103, 108, 172]
+    items = [(r, t, min(32, n - t), t // 32) for r, n in enumerate(lens) for t in range(0, n, 32)]
+    first = [sum(-(-n // 32) for n in lens[:r]) for r in range(6)]
+    offs = (0, heads * dim, 2 * heads * dim, 2 * heads * dim + heads * vdim, 2 * heads * dim + 2 * heads * vdim)
+    state = start.clone()
+    got = ops.linear_recurrence_segments(proj, *offs, a2, a2b, norm, state, ints(*slots), ints(*cu), ints(*sum(items, ())), len(items), 32,
+                                         ints(*first), 5, heads, dim, vdim, dim ** -0.5, 16.0, 1e-5,
+                                         decay="double_exp" if form == "double_exp" else "sigmoid_power", bonus=bonus if form == "bonus" else None)
+    cols = lambda at, n: proj[:, at:at + heads * n].to(f64).view(T, heads, n)  # noqa: E731
+    q, k, v, g = cols(offs[0], dim) * dim ** -0.5, cols(offs[1], dim), cols(offs[2], vdim), cols(offs[3], vdim)
+    z = proj[:, offs[4]:offs[4] + rank].to(f64) @ a2.to(f64).t() + a2b.to(f64)
+    decay = (torch.exp(-torch.exp(z)) if form == "double_exp" else torch.sigmoid(z).pow(1 / 16.0)).view(T, heads, dim)
+    want, after = torch.zeros(T, heads, vdim, dtype=f64, device=DEV), start.to(f64)
+    for r, slot in enumerate(slots):
+        S = after[slot]
+        for t in range(cu[r], cu[r + 1]):
+            kv = k[t, :, :, None] * v[t, :, None, :]
+            if form == "bonus":
+                want[t] = (q[t, :, :, None] * (S + bonus.to(f64).view(heads, dim, 1) * kv)).sum(1)
+            S = decay[t, :, :, None] * S + kv
+            if form != "bonus":
+                want[t] = (q[t, :, :, None] * S).sum(1)
+        after[slot] = S
+    want = want * torch.rsqrt(want.square().mean(-1, keepdim=True) + 1e-5) * norm.to(f64) * torch.nn.functional.silu(g)
+    # sums of up to 128 float32 terms over some 16 steps that have not decayed yet; the result's own rounding
+    tol = dict(atol=0.02, rtol=0.01) if dtype == torch.bfloat16 else dict(atol=1e-4, rtol=1e-4)
+    torch.testing.assert_close(got.to(f64).view(T, heads, vdim), want, **tol)
+    torch.testing.assert_close(state.to(f64), after, atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize("at", [0, 5, 16, 31, 40])
+def test_recurrence_in_segments_with_an_infinite_value(at):
+    """An infinite value makes its column infinite from its token on: no token before it, no other column."""
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(at)
+    dim, vdim, T = 64, 128, 70
+    proj = torch.rand(T, 2 * dim + vdim + 16, device=DEV, generator=gen) + 0.5
+    proj[at, 2 * dim + 3] = float("inf")
+    ints = lambda *t: torch.tensor(t, dtype=torch.int32, device=DEV)  # noqa: E731
+    state = torch.zeros(1, 1, dim, vdim, device=DEV)
+    got = ops.linear_recurrence_segments(proj, 0, dim, 2 * dim, -1, 2 * dim + vdim, torch.rand(dim, 16, device=DEV, generator=gen), None, None,
+                                         state, ints(0), ints(0, T), ints(0, 0, 32, 0, 0, 32, 32, 1, 0, 64, 6, 2), 3, 32, ints(0, 3), 1, 1, dim, vdim,
+                                         1.0, 16.0, 1e-5)
+    assert bool((got[at:, 3] == float("inf")).all()) and bool(torch.isfinite(got[:at]).all())
+    rest = [c for c in range(vdim) if c != 3]
+    assert bool(torch.isfinite(got[:, rest]).all()) and bool(torch.isfinite(state[..., rest]).all())
+    assert bool((state[0, 0, :, 3] == float("inf")).all())
+
+
 # runs of 32, 50 and 128 keys; mixed heads over one, two (two kernels) and three key/value heads (three kernels), no
 # mixing over four; sizes that are read in pieces and one by one, more columns than threads, groups of more than 16 heads
 @pytest.mark.parametrize("heads,kv,dim,vdim,talk", [(12, 2, 128, 128, True), (6, 2, 20, 24, True), (3, 1, 40, 24, True), (6, 3, 64, 64, True),
