@@ -1260,15 +1260,39 @@ __global__ __launch_bounds__(256) void sink_prefill_mfma_kernel(SinkAttnParams p
 // registers (the value fragments are read with the keys in that order). Weights are float32 and
 // fed as two bfloat16 operands, as in the kernel above.
 // ======================================================================================
+typedef __attribute__((ext_vector_type(4))) short sa_s16x4_t;
+typedef __attribute__((address_space(3))) sa_s16x4_t sa_lds_s16x4_t;
+
+// Two sets of four waves share every stage's keys (32 each) where a wave's queries and accumulators leave room for two
+// waves a SIMD: one's products then run beside the other's exponentials. The sets' results meet in LDS at the end.
+// HEAVY: the registers of a wave's heads (queries; accumulators of both key/value heads).
+static constexpr int so_sets(int hpw, int d32, int nt, int gc) { return hpw * (gc * nt * 4 + d32 * 4) <= 160 ? 2 : 1; }
 template <int HPW, int D32, int V16, int VS, int GC>
-__global__ __launch_bounds__(256) void sink_prefill_onewalk_kernel(SinkAttnParams p) {
+struct OneWalk {
+  static constexpr int D = D32 * 32, V = V16 * 16, NT = V16 / VS, VW = NT * 16;
+  static constexpr int SETS = so_sets(HPW, D32, NT, GC), KT = SM_KT * SETS, THREADS = 256 * SETS;
+  static constexpr int VROW = VW + 16;                      // value rows: 32 bytes of padding for the transposing reads
+  static constexpr int STAGE = GC * KT * (D + VROW);        // elements: keys as [head][D / 32][key][32], then values as [head][key][VROW]
+  static constexpr int TILES = 2 * STAGE * 2;               // bytes of the two stages
+  static constexpr int EXCHANGE = (SETS - 1) * 4 * HPW * (GC * NT * 1024 + 512);
+  static int64_t lds_bytes(int H) {                         // without the pages' table
+    const int64_t finish = (int64_t)GC * H * 16 * VW * 4;   // finished outputs, laid over the tiles
+    int64_t most = TILES > EXCHANGE ? TILES : EXCHANGE;
+    if (finish > most) most = finish;
+    return most + (int64_t)H * GC * 16 * 4;                 // the mixing matrix behind all of them
+  }
+};
+
+template <int HPW, int D32, int V16, int VS, int GC>
+__global__ __launch_bounds__((OneWalk<HPW, D32, V16, VS, GC>::THREADS)) void sink_prefill_onewalk_kernel(SinkAttnParams p, int mix_at,
+                                                                                                         int bs_shift) {
+  using W = OneWalk<HPW, D32, V16, VS, GC>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  constexpr int D = D32 * 32, V = V16 * 16, NT = V16 / VS, VW = NT * 16;
+  constexpr int D = W::D, V = W::V, NT = W::NT, VW = W::VW, SETS = W::SETS, KT = W::KT, NTH = W::THREADS, VROW = W::VROW;
   const int v0 = blockIdx.y * VW;
-  constexpr int KROW = D + 8;
-  constexpr int VROW = SM_KT + 8;
-  const int H = p.heads, G = GC, Hg = H / G;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int H = p.heads, Hg = H / GC;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3, set = __builtin_amdgcn_readfirstlane(tid >> 8);
   const int l16 = lane & 15, slot = lane >> 4;
   const int r = p.items[4 * blockIdx.x], tok0 = p.items[4 * blockIdx.x + 1];
   const int q_len = p.cu_q[r + 1] - p.cu_q[r];
@@ -1280,134 +1304,124 @@ __global__ __launch_bounds__(256) void sink_prefill_onewalk_kernel(SinkAttnParam
   const int64_t row0 = p.cu_q[r] + tok0;
   const int* table = p.block_tables + (int64_t)r * p.table_width;
 
-  bf16_t* Ks = reinterpret_cast<bf16_t*>(smem_raw);              // [G][KT][KROW]
-  bf16_t* Vt = Ks + G * SM_KT * KROW;                            // [G][VW][VROW]
-  float* Ox = reinterpret_cast<float*>(smem_raw);                // at the end, over the tiles: [H][16][VW] finished outputs of one key/value head
-  const int tile_bytes = (G * SM_KT * KROW + G * VW * VROW) * 2, finish_bytes = H * 16 * VW * 4;
-  float* Tk = reinterpret_cast<float*>(smem_raw + max(tile_bytes, finish_bytes));  // [H][H], behind both
-  int* Tb = reinterpret_cast<int*>(Tk + H * H);                  // [tb_len]
+  bf16_t* const tiles = reinterpret_cast<bf16_t*>(smem_raw);
+  float* const mix = reinterpret_cast<float*>(smem_raw + mix_at);  // [g][key/value head][16]: talk of its heads, 16 to a row
+  int* const Tb = reinterpret_cast<int*>(mix + H * GC * 16);       // [tb_len]
 
   const bf16_t* q = (const bf16_t*)p.q;
   const bf16_t* kc = (const bf16_t*)p.k_cache;
   const bf16_t* vc = (const bf16_t*)p.v_cache;
-  for (int i = tid; i < H * H; i += 256) Tk[i] = p.talk ? p.talk[i] : (i / H == i % H ? 1.0f : 0.0f);
   const int tb0 = lo / p.block_size;
-  for (int i = tid; i < p.tb_len; i += 256) Tb[i] = tb0 + i < p.table_width ? table[tb0 + i] : -1;
+  for (int i = tid; i < p.tb_len; i += NTH) Tb[i] = tb0 + i < p.table_width ? table[tb0 + i] : -1;
+  for (int i = tid; i < H * GC * 16; i += NTH) {
+    const int hh = i & 15, cc = (i >> 4) % GC, g = (i >> 4) / GC, h = cc * Hg + hh;
+    mix[i] = hh >= Hg ? 0.0f : p.talk ? p.talk[h * H + g] : (h == g ? 1.0f : 0.0f);
+  }
   __syncthreads();
 
   // query fragments as the B operand: lane = query l16, 8 elements at slot
   sa_bf16x8_t qf[HPW][D32];
+  float r1[HPW], r2[HPW];
   const int qi = min(l16, nq - 1);
 #pragma unroll
   for (int a = 0; a < HPW; ++a) {
     const int g = min(wave + 4 * a, H - 1);
 #pragma unroll
     for (int ks = 0; ks < D32; ++ks) qf[a][ks] = sm_load8(q + (row0 + qi) * p.q_stride + g * D + ks * 32 + slot * 8);
+    r1[a] = p.r1 ? p.r1[g] : 0.0f;
+    r2[a] = p.r1 ? p.r2[g] : 0.0f;
   }
 
-  constexpr int PF = 4;
-  uint4 kreg[PF], vreg[PF];
-  auto row_of = [&](int j) -> int64_t {
-    const int slot_ = min(max(j / p.block_size - tb0, 0), p.tb_len - 1);
-    const int page = Tb[slot_];
-    const int64_t row = (int64_t)page * p.block_size + j % p.block_size;
-    return (j <= last && j / p.block_size - tb0 < p.tb_len && page >= 0 && row < p.cache_rows) ? row : -1;
+  // A stage's traffic: neighbouring threads take 16-byte pieces of one key's row, piece by piece of a row.
+  constexpr int KPR = D / 8, VPR = VW / 8, KPI = NTH / KPR, VPI = NTH / VPR;  // rows that all threads take at once
+  constexpr int KN = (GC * KT + KPI - 1) / KPI, VN = (GC * KT + VPI - 1) / VPI;
+  uint4 kreg[KN], vreg[VN];
+  auto row_of = [&](int j) __attribute__((always_inline)) -> int64_t {  // -1: zeros
+    const int n = bs_shift >= 0 ? j >> bs_shift : j / p.block_size;
+    const int page = Tb[min(max(n - tb0, 0), p.tb_len - 1)];
+    const int64_t row = (int64_t)page * p.block_size + (j - n * p.block_size);
+    return (j <= last && n - tb0 < p.tb_len && page >= 0 && row < p.cache_rows) ? row : -1;
   };
-  auto fetch = [&](int k0) {
-    constexpr int KPR = D / 8, VPR = VW / 8;
+  auto fetch = [&](int k0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int it = 0; it < PF; ++it) {
-      const int idx = tid + it * 256;
-      {
-        const int at = min(idx, G * SM_KT * KPR - 1);
-        const int e = at % KPR, jj = (at / KPR) % SM_KT, c = at / (KPR * SM_KT);
-        const int64_t row = row_of(k0 + jj);
-        const uint4 x = *reinterpret_cast<const uint4*>(kc + ((row >= 0 ? row : 0) * G + c) * D + e * 8);
-        kreg[it] = (row >= 0 && idx == at) ? x : make_uint4(0, 0, 0, 0);
-      }
-      {
-        const int at = min(idx, G * SM_KT * VPR - 1);
-        const int e = at % VPR, jj = (at / VPR) % SM_KT, c = at / (VPR * SM_KT);
-        const int64_t row = row_of(k0 + jj);
-        const uint4 x = *reinterpret_cast<const uint4*>(vc + ((row >= 0 ? row : 0) * G + c) * V + v0 + e * 8);
-        vreg[it] = (row >= 0 && idx == at) ? x : make_uint4(0, 0, 0, 0);
-      }
+    for (int it = 0; it < KN; ++it) {
+      const int n = tid / KPR + it * KPI;
+      const int64_t row = row_of(k0 + n % KT);
+      const uint4 x = *reinterpret_cast<const uint4*>(kc + ((row >= 0 ? row : 0) * GC + min(n / KT, GC - 1)) * D + tid % KPR * 8);
+      kreg[it] = row >= 0 ? x : make_uint4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int it = 0; it < VN; ++it) {
+      const int n = tid / VPR + it * VPI;
+      const int64_t row = row_of(k0 + n % KT);
+      const uint4 x = *reinterpret_cast<const uint4*>(vc + ((row >= 0 ? row : 0) * GC + min(n / KT, GC - 1)) * V + v0 + tid % VPR * 8);
+      vreg[it] = row >= 0 ? x : make_uint4(0, 0, 0, 0);
     }
   };
-  auto store = [&]() {
-    constexpr int KPR = D / 8, VPR = VW / 8;
+  auto store = [&](int buf) __attribute__((always_inline)) {
+    bf16_t* ks = tiles + buf * W::STAGE;
+    bf16_t* vs = ks + GC * KT * D;
 #pragma unroll
-    for (int it = 0; it < PF; ++it) {
-      const int idx = tid + it * 256;
-      if (idx < G * SM_KT * KPR) {
-        const int e = idx % KPR, jj = (idx / KPR) % SM_KT, c = idx / (KPR * SM_KT);
-        *reinterpret_cast<uint4*>(Ks + (c * SM_KT + jj) * KROW + e * 8) = kreg[it];
-      }
-      if (idx < G * SM_KT * VPR) {
-        const int e = idx % VPR, jj = (idx / VPR) % SM_KT, c = idx / (VPR * SM_KT);
-        const uint32_t w[4] = {vreg[it].x, vreg[it].y, vreg[it].z, vreg[it].w};
-        uint16_t* dst = reinterpret_cast<uint16_t*>(Vt) + (c * VW + e * 8) * VROW + jj;
+    for (int it = 0; it < KN; ++it) {
+      const int n = tid / KPR + it * KPI, e = tid % KPR;
+      if (GC * KT % KPI == 0 || n < GC * KT)
+        *reinterpret_cast<uint4*>(ks + ((n / KT * D32 + (e >> 2)) * KT + n % KT) * 32 + (e & 3) * 8) = kreg[it];
+    }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          dst[(2 * u) * VROW] = (uint16_t)(w[u] & 0xffffu);
-          dst[(2 * u + 1) * VROW] = (uint16_t)(w[u] >> 16);
-        }
-      }
+    for (int it = 0; it < VN; ++it) {
+      const int n = tid / VPR + it * VPI;
+      if (GC * KT % VPI == 0 || n < GC * KT) *reinterpret_cast<uint4*>(vs + n * VROW + tid % VPR * 8) = vreg[it];
     }
   };
 
   constexpr float LOG2E = 1.4426950408889634f;
   const float scale2 = p.scale * LOG2E;
-  // per head: the query's running maximum (the same in the 4 lanes of a query), this lane's part
-  // of its denominator, and the accumulators, one per key/value head
+  // Per head: the query's running maximum (the same in the 4 lanes of a query), this lane's part of the denominator, and
+  // the accumulators, one per key/value head: value columns 16 nt + 4 slot + e of query l16. (The maximum itself, not a
+  // reference that lags behind it: the largest weight is then 1, which its two bfloat16 parts hold exactly.)
   float m[HPW], l[HPW];
   sa_f32x4_t out[HPW][GC][NT];
 #pragma unroll
   for (int a = 0; a < HPW; ++a) {
     const int g = min(wave + 4 * a, H - 1);
     m[a] = p.sink ? p.sink[g] * LOG2E : -3.0e38f;
-    l[a] = (p.sink && slot == 0) ? 1.0f : 0.0f;
+    l[a] = (p.sink && slot == 0 && set == 0) ? 1.0f : 0.0f;
 #pragma unroll
     for (int c = 0; c < GC; ++c)
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) out[a][c][nt] = sa_f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
   }
 
-  fetch(lo);
-  for (int k0 = lo; k0 <= last; k0 += SM_KT) {
-    __syncthreads();
-    store();
-    if (k0 + SM_KT <= last) fetch(k0 + SM_KT);
-    __syncthreads();
+  auto compute = [&](int k0, int buf) __attribute__((always_inline)) {
+    if (k0 > last) return;
+    const bf16_t* ks = tiles + buf * W::STAGE + set * (SM_KT * 32);
+    const bf16_t* vs = tiles + buf * W::STAGE + GC * KT * D + set * SM_KT * VROW;
     const bool inside = nq == 16 && k0 + SM_KT - 1 <= pos0 && (p.window <= 0 || pos0 + 15 - k0 < p.window);
+    const int dist0 = pos0 + l16 - k0 - 4 * slot;  // to key 4 slot of the wave's keys
     sa_bf16x8_t ph[HPW], pl[HPW];
 #pragma unroll
     for (int a = 0; a < HPW; ++a) {
       const int g = wave + 4 * a;
       if (g < H) {
-        const int c = g / Hg;
         // S^T tiles: rows = keys 16 kt + 4 slot + e, column = this lane's query
         sa_f32x4_t acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = {0.0f, 0.0f, 0.0f, 0.0f};
-        const bf16_t* kb = Ks + (c * SM_KT + l16) * KROW + slot * 8;
+        const bf16_t* kb = ks + (g / Hg * D32 * KT + l16) * 32 + slot * 8;
 #pragma unroll
-        for (int ks = 0; ks < D32; ++ks) {
-          acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sm_load8(kb + ks * 32), qf[a][ks], acc0, 0, 0, 0);
-          acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sm_load8(kb + 16 * KROW + ks * 32), qf[a][ks], acc1, 0, 0, 0);
+        for (int n = 0; n < D32; ++n) {
+          acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sm_load8(kb + n * (KT * 32)), qf[a][n], acc0, 0, 0, 0);
+          acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sm_load8(kb + n * (KT * 32) + 16 * 32), qf[a][n], acc1, 0, 0, 0);
         }
-        const float r1 = p.r1 ? p.r1[g] : 0.0f, r2 = p.r1 ? p.r2[g] : 0.0f;
-        float s[8];
-        float top = -INFINITY;
+        float w[8], top = -INFINITY;
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-          const int j = k0 + (u >> 2) * 16 + slot * 4 + (u & 3);
-          const int dist = pos0 + l16 - j;
+          const int dist = dist0 - (u >> 2) * 16 - (u & 3);
           float v = (u < 4 ? acc0[u & 3] : acc1[u & 3]) * scale2;
-          if (p.r1) v -= r1 * __builtin_amdgcn_logf(1.0f + r2 * (float)max(dist, 0));
+          if (p.r1) v -= r1[a] * __builtin_amdgcn_logf(1.0f + r2[a] * (float)max(dist, 0));
           if (!inside) {
             const bool seen = l16 < nq && dist >= 0 && (p.window <= 0 || dist < p.window);
             v = seen ? v : -INFINITY;
           }
-          s[u] = v;
+          w[u] = v;
           top = fmaxf(top, v);
         }
         top = cw_quad_max(top);
@@ -1415,10 +1429,9 @@ __global__ __launch_bounds__(256) void sink_prefill_onewalk_kernel(SinkAttnParam
         const float alpha = __builtin_amdgcn_exp2f(m[a] - mn);
         m[a] = mn;
         float sum = 0.0f;
-        float w[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-          w[u] = __builtin_amdgcn_exp2f(s[u] - mn);
+          w[u] = __builtin_amdgcn_exp2f(w[u] - mn);
           sum += w[u];
         }
         l[a] = l[a] * alpha + sum;
@@ -1428,77 +1441,124 @@ __global__ __launch_bounds__(256) void sink_prefill_onewalk_kernel(SinkAttnParam
           ph[a][u] = t;
           pl[a][u] = (__bf16)(w[u] - (float)t);
         }
-        // the accumulators' rows are queries slot * 4 + e: each takes its own query's factor
         if (__ballot(alpha != 1.0f) != 0) {
-          float ar[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) ar[e] = __shfl(alpha, slot * 4 + e, 64);
 #pragma unroll
           for (int cc = 0; cc < GC; ++cc)
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-              for (int e = 0; e < 4; ++e) out[a][cc][nt][e] *= ar[e];
+            for (int nt = 0; nt < NT; ++nt) out[a][cc][nt] *= alpha;
         }
       }
     }
-    // values: a fragment (one key/value head, 16 value columns) serves all of the wave's heads
+    // O^T += V^T P^T: a fragment (one key/value head, 16 value columns) serves all of the wave's heads
+    const bf16_t* vlane = vs + (4 * slot + (l16 >> 2)) * VROW + 4 * (l16 & 3);
 #pragma unroll
-    for (int cc = 0; cc < GC; ++cc) {
+    for (int cc = 0; cc < GC; ++cc)
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
-        // column l16 of the tile, keys 4 slot .. + 4 and 16 + 4 slot .. + 4: the order the weights lie in
-        const bf16_t* vb = Vt + (cc * VW + nt * 16 + l16) * VROW + slot * 4;
-        const uint2 lo4 = *reinterpret_cast<const uint2*>(vb), hi4 = *reinterpret_cast<const uint2*>(vb + 16);
-        const uint4 both = make_uint4(lo4.x, lo4.y, hi4.x, hi4.y);
-        const sa_bf16x8_t vf = *reinterpret_cast<const sa_bf16x8_t*>(&both);
+        const bf16_t* vp = vlane + cc * KT * VROW + nt * 16;
+        const sa_s16x4_t x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((sa_lds_s16x4_t*)vp);
+        const sa_s16x4_t x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((sa_lds_s16x4_t*)(vp + 16 * VROW));
+        const sa_bf16x8_t vf = __builtin_bit_cast(sa_bf16x8_t, __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
         for (int a = 0; a < HPW; ++a) {
           if (wave + 4 * a < H) {
-            out[a][cc][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph[a], vf, out[a][cc][nt], 0, 0, 0);
-            out[a][cc][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl[a], vf, out[a][cc][nt], 0, 0, 0);
+            out[a][cc][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, ph[a], out[a][cc][nt], 0, 0, 0);
+            out[a][cc][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl[a], out[a][cc][nt], 0, 0, 0);
           }
         }
       }
-    }
+  };
+
+  fetch(lo);
+  store(0);
+  __syncthreads();
+  for (int k0 = lo, buf = 0; k0 <= last; k0 += KT, buf ^= 1) {
+    if (k0 + KT <= last) fetch(k0 + KT);  // on its way while this stage is computed
+    compute(k0 + set * SM_KT, buf);
+    if (k0 + KT <= last) store(buf ^ 1);
+    __syncthreads();
   }
 
-  // ---- finish: denominators, then the mixing across heads, one key/value head at a time through LDS
-  float inv_row[HPW][4];
+  // ---- finish: the second set's results join the first's, through LDS (the tiles are done with)
+  if constexpr (SETS == 2) {
+    sa_f32x4_t* xo = reinterpret_cast<sa_f32x4_t*>(smem_raw);                      // [wave][a][head][nt][lane]
+    float* xml = reinterpret_cast<float*>(smem_raw + 4 * HPW * GC * NT * 1024);    // [wave][a][m, l][lane]
+    if (set == 1) {
 #pragma unroll
-  for (int a = 0; a < HPW; ++a) {
-    const float total = cw_quad_sum(l[a]);
-    const float inv = total > 0.0f ? 1.0f / total : 0.0f;
+      for (int a = 0; a < HPW; ++a) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) inv_row[a][e] = __shfl(inv, slot * 4 + e, 64);
-  }
-  bf16_t* o = (bf16_t*)p.out;
-  for (int cc = 0; cc < GC; ++cc) {
-    __syncthreads();  // the tiles (and the round before) are done with LDS
+        for (int cc = 0; cc < GC; ++cc)
 #pragma unroll
-    for (int a = 0; a < HPW; ++a) {
-      const int g = wave + 4 * a;
-      if (g < H) {
-#pragma unroll
-        for (int c2 = 0; c2 < GC; ++c2) {
-          if (c2 == cc) {
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-              for (int e = 0; e < 4; ++e)
-                Ox[(g * 16 + slot * 4 + e) * VW + nt * 16 + l16] = out[a][c2][nt][e] * inv_row[a][e];
-          }
-        }
+          for (int nt = 0; nt < NT; ++nt) xo[(((wave * HPW + a) * GC + cc) * NT + nt) * 64 + lane] = out[a][cc][nt];
+        xml[(wave * HPW + a) * 128 + lane] = m[a];
+        xml[(wave * HPW + a) * 128 + 64 + lane] = l[a];
       }
     }
     __syncthreads();
-    // heads of this key/value head: h = cc * Hg .. ; every thread takes outputs (h, query, column)
-    const int n_out = Hg * 16 * VW;
-    for (int idx = tid; idx < n_out; idx += 256) {
-      const int col = idx % VW, i = (idx / VW) % 16, h = cc * Hg + idx / (VW * 16);
-      float v = 0.0f;
-      for (int g = 0; g < H; ++g) v += Tk[h * H + g] * Ox[(g * 16 + i) * VW + col];
-      if (i < nq) o[(row0 + i) * (int64_t)(H * V) + h * V + v0 + col] = __float2bfloat16(v);
+    if (set == 0) {
+#pragma unroll
+      for (int a = 0; a < HPW; ++a) {
+        const float m1 = xml[(wave * HPW + a) * 128 + lane], l1 = xml[(wave * HPW + a) * 128 + 64 + lane];
+        const float mn = fmaxf(m[a], m1);
+        const float f0 = __builtin_amdgcn_exp2f(m[a] - mn), f1 = __builtin_amdgcn_exp2f(m1 - mn);
+        l[a] = l[a] * f0 + l1 * f1;
+#pragma unroll
+        for (int cc = 0; cc < GC; ++cc)
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt)
+            out[a][cc][nt] = out[a][cc][nt] * f0 + xo[(((wave * HPW + a) * GC + cc) * NT + nt) * 64 + lane] * f1;
+      }
+    }
+    __syncthreads();
+  }
+  // ---- denominators, then the mixing across heads: a thread takes four columns of one query of all heads of one
+  // key/value head
+  float* const Ox = reinterpret_cast<float*>(smem_raw);  // [key/value head][H][16][VW]
+  if (set == 0) {
+#pragma unroll
+    for (int a = 0; a < HPW; ++a) {
+      const int g = wave + 4 * a;
+      const float total = cw_quad_sum(l[a]);
+      const float inv = total > 0.0f ? 1.0f / total : 0.0f;
+      if (g < H)
+#pragma unroll
+        for (int cc = 0; cc < GC; ++cc)
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt)
+            *reinterpret_cast<sa_f32x4_t*>(Ox + ((cc * H + g) * 16 + l16) * VW + nt * 16 + slot * 4) = out[a][cc][nt] * inv;
+    }
+  }
+  __syncthreads();
+  bf16_t* o = (bf16_t*)p.out;
+  const bool wide = !((uintptr_t)o & 7);
+  for (int idx = tid; idx < GC * 16 * (VW / 4); idx += NTH) {
+    const int col = idx % (VW / 4) * 4, i = idx / (VW / 4) % 16, cc = idx / (VW / 4 * 16);
+    sa_f32x4_t v[16];
+#pragma unroll
+    for (int hh = 0; hh < 16; ++hh) v[hh] = sa_f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int g = 0; g < H; ++g) {
+      const sa_f32x4_t x = *reinterpret_cast<const sa_f32x4_t*>(Ox + ((cc * H + g) * 16 + i) * VW + col);
+      const sa_f32x4_t* w = reinterpret_cast<const sa_f32x4_t*>(mix + (g * GC + cc) * 16);
+#pragma unroll
+      for (int h4 = 0; h4 < 4; ++h4)
+        if (4 * h4 < Hg) {
+          const sa_f32x4_t f = w[h4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[4 * h4 + e] += f[e] * x;
+        }
+    }
+    if (i >= nq) continue;
+    bf16_t* to = o + (row0 + i) * (int64_t)(H * V) + cc * Hg * V + v0 + col;
+#pragma unroll
+    for (int hh = 0; hh < 16; ++hh) {
+      if (hh >= Hg) break;
+      if (wide) {
+        const float f[4] = {v[hh][0], v[hh][1], v[hh][2], v[hh][3]};
+        CwVec<bf16_t, 4>::store(to + hh * V, f);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) to[hh * V + e] = __float2bfloat16(v[hh][e]);
+      }
     }
   }
 }
@@ -1516,12 +1576,6 @@ CW_EXPORT int cw_sink_prefill_mfma_supported(int heads, int kv_heads, int dim, i
   // a thread moves up to four 16-byte pieces of a chunk's keys, and of its values
   if (kv_heads * SM_KT * (dim / 8) > 4 * 256 || kv_heads * SM_KT * (vdim / 8) > 4 * 256) return 0;
   return sink_prefill_mfma_lds_bytes(heads, kv_heads, dim, vdim) + SM_MAX_TABLE * 4 <= 150 * 1024 ? 1 : 0;
-}
-
-static int64_t sink_prefill_onewalk_lds_bytes(int H, int G, int D, int VW) {  // without the pages' table
-  const int64_t tiles = (int64_t)G * SM_KT * (D + 8) * 2 + (int64_t)G * VW * (SM_KT + 8) * 2;
-  const int64_t finish = (int64_t)H * 16 * VW * 4;   // laid over the tiles; the mixing matrix and the pages lie behind both
-  return (tiles > finish ? tiles : finish) + (int64_t)H * H * 4;
 }
 
 // items: runs of up to 16 tokens. bfloat16 only. A launch of fewer than v_split_below runs gives
@@ -1553,15 +1607,22 @@ CW_EXPORT int cw_sink_prefill_mfma(const void* q, int64_t q_stride, void* out, c
   const int hpw = (heads + 3) / 4;
   // one or two key/value heads: the kernel that walks the keys once (two workgroups a run always:
   // its accumulators for all value columns would not fit the registers)
-  if (kv_heads <= 2 && sink_prefill_onewalk_lds_bytes(heads, kv_heads, dim, vdim / 2) + tb_len * 4 <= 150 * 1024) {
-    const size_t smem1 = (size_t)sink_prefill_onewalk_lds_bytes(heads, kv_heads, dim, vdim / 2) + (size_t)tb_len * 4;
+  if (kv_heads <= 2) {
     const dim3 grid1(n_items, 2);
+    int bs_shift = -1;
+    for (int i = 0; i < 31; ++i)
+      if (1 << i == block_size) bs_shift = i;
 #define CW_ONE(HPW_, D32_, V16_, GC_)                                                                                 \
   do {                                                                                                                \
+    using W_ = OneWalk<HPW_, D32_, V16_, 2, GC_>;                                                                     \
+    const int64_t mix_end = W_::lds_bytes(heads), smem1 = mix_end + tb_len * 4;                                       \
+    if (smem1 > 160 * 1024) break;                                                                                    \
     if (smem1 > 48 * 1024 && hipFuncSetAttribute((const void*)sink_prefill_onewalk_kernel<HPW_, D32_, V16_, 2, GC_>,  \
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem1) != hipSuccess) \
       return CW_ERR_LAUNCH;                                                                                           \
-    hipLaunchKernelGGL((sink_prefill_onewalk_kernel<HPW_, D32_, V16_, 2, GC_>), grid1, block, smem1, stream, p);      \
+    hipLaunchKernelGGL((sink_prefill_onewalk_kernel<HPW_, D32_, V16_, 2, GC_>), grid1, dim3(W_::THREADS), smem1, stream, p, \
+                       (int)(mix_end - (int64_t)heads * GC_ * 64), bs_shift);                                         \
+    return cw_launch_status();                                                                                        \
   } while (0)
 #define CW_ONE_HEADS(D32_, V16_, GC_)              \
   do {                                             \
@@ -1582,7 +1643,6 @@ CW_EXPORT int cw_sink_prefill_mfma(const void* q, int64_t q_stride, void* out, c
 #undef CW_ONE_SIZES
 #undef CW_ONE_HEADS
 #undef CW_ONE
-    return cw_launch_status();
   }
   const size_t smem = (size_t)sink_prefill_mfma_lds_bytes(heads, kv_heads, dim, vdim / vs) + (size_t)tb_len * 4;
 #define CW_LAUNCH_VS(HPW_, D32_, V16_, VS_)                                                                           \
