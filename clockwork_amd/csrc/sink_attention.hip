@@ -1257,15 +1257,19 @@ __global__ __launch_bounds__(256) void sink_prefill_mfma_kernel(SinkAttnParams p
 // usual running maximum), and the finished, normalised accumulators are mixed once at the end,
 // through LDS. Scores are made as K Q^T: a lane then holds, for ITS query (l16), the chunk's keys
 // 4 slot + e and 16 + 4 slot + e, which is the A operand of the value product as it lies in the
-// registers (the value fragments are read with the keys in that order). Weights are float32 and
-// fed as two bfloat16 operands, as in the kernel above.
+// registers (the value fragments are read with the keys in that order, by the LDS transposing read). Weights are float32
+// and fed as two bfloat16 operands, as in the kernel above.
+// What bounds it is the vector unit: distance bias, maximum, exponential and the two halves of every weight are some
+// 130 instructions a head and 32 keys, beside 24 matrix instructions. Measured on an MI355X, 2048 tokens of 12 heads of 128
+// over 2, a window of 1024: 199 us with one set of waves, two barriers every 32 keys and values transposed by 16-bit
+// stores; 109 with two sets and stages of 64; 99 with the heads' chains beside each other, no branch a head and score.
 // ======================================================================================
 typedef __attribute__((ext_vector_type(4))) short sa_s16x4_t;
 typedef __attribute__((address_space(3))) sa_s16x4_t sa_lds_s16x4_t;
 
 // Two sets of four waves share every stage's keys (32 each) where a wave's queries and accumulators leave room for two
 // waves a SIMD: one's products then run beside the other's exponentials. The sets' results meet in LDS at the end.
-// HEAVY: the registers of a wave's heads (queries; accumulators of both key/value heads).
+// (hpw * ...: the registers of a wave's queries and of its accumulators of both key/value heads.)
 static constexpr int so_sets(int hpw, int d32, int nt, int gc) { return hpw * (gc * nt * 4 + d32 * 4) <= 160 ? 2 : 1; }
 template <int HPW, int D32, int V16, int VS, int GC>
 struct OneWalk {
@@ -1398,56 +1402,70 @@ __global__ __launch_bounds__((OneWalk<HPW, D32, V16, VS, GC>::THREADS)) void sin
     const bf16_t* vs = tiles + buf * W::STAGE + GC * KT * D + set * SM_KT * VROW;
     const bool inside = nq == 16 && k0 + SM_KT - 1 <= pos0 && (p.window <= 0 || pos0 + 15 - k0 < p.window);
     const int dist0 = pos0 + l16 - k0 - 4 * slot;  // to key 4 slot of the wave's keys
-    sa_bf16x8_t ph[HPW], pl[HPW];
+    // S^T tiles of all the wave's heads: rows = keys 16 kt + 4 slot + e, column = this lane's query. (A wave short of a
+    // head makes its last one again, which nobody reads: a branch a head would keep the heads' chains from each other.)
+    sa_f32x4_t sc[HPW][2];
 #pragma unroll
     for (int a = 0; a < HPW; ++a) {
-      const int g = wave + 4 * a;
-      if (g < H) {
-        // S^T tiles: rows = keys 16 kt + 4 slot + e, column = this lane's query
-        sa_f32x4_t acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = {0.0f, 0.0f, 0.0f, 0.0f};
-        const bf16_t* kb = ks + (g / Hg * D32 * KT + l16) * 32 + slot * 8;
+      const bf16_t* kb = ks + (min(wave + 4 * a, H - 1) / Hg * D32 * KT + l16) * 32 + slot * 8;
+      sc[a][0] = sc[a][1] = sa_f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int n = 0; n < D32; ++n) {
-          acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sm_load8(kb + n * (KT * 32)), qf[a][n], acc0, 0, 0, 0);
-          acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sm_load8(kb + n * (KT * 32) + 16 * 32), qf[a][n], acc1, 0, 0, 0);
-        }
-        float w[8], top = -INFINITY;
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const int dist = dist0 - (u >> 2) * 16 - (u & 3);
-          float v = (u < 4 ? acc0[u & 3] : acc1[u & 3]) * scale2;
-          if (p.r1) v -= r1[a] * __builtin_amdgcn_logf(1.0f + r2[a] * (float)max(dist, 0));
-          if (!inside) {
-            const bool seen = l16 < nq && dist >= 0 && (p.window <= 0 || dist < p.window);
-            v = seen ? v : -INFINITY;
-          }
-          w[u] = v;
-          top = fmaxf(top, v);
-        }
-        top = cw_quad_max(top);
-        const float mn = fmaxf(m[a], top);
-        const float alpha = __builtin_amdgcn_exp2f(m[a] - mn);
-        m[a] = mn;
-        float sum = 0.0f;
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          w[u] = __builtin_amdgcn_exp2f(w[u] - mn);
-          sum += w[u];
-        }
-        l[a] = l[a] * alpha + sum;
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const __bf16 t = (__bf16)w[u];
-          ph[a][u] = t;
-          pl[a][u] = (__bf16)(w[u] - (float)t);
-        }
-        if (__ballot(alpha != 1.0f) != 0) {
-#pragma unroll
-          for (int cc = 0; cc < GC; ++cc)
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) out[a][cc][nt] *= alpha;
-        }
+      for (int n = 0; n < D32; ++n) {
+        sc[a][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sm_load8(kb + n * (KT * 32)), qf[a][n], sc[a][0], 0, 0, 0);
+        sc[a][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sm_load8(kb + n * (KT * 32) + 16 * 32), qf[a][n], sc[a][1], 0, 0, 0);
       }
+    }
+    if (p.r1) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float dist = (float)max(dist0 - (u >> 2) * 16 - (u & 3), 0);
+#pragma unroll
+        for (int a = 0; a < HPW; ++a)
+          sc[a][u >> 2][u & 3] = sc[a][u >> 2][u & 3] * scale2 - r1[a] * __builtin_amdgcn_logf(1.0f + r2[a] * dist);
+      }
+    } else {
+#pragma unroll
+      for (int a = 0; a < HPW; ++a) sc[a][0] *= scale2, sc[a][1] *= scale2;
+    }
+    if (!inside) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int dist = dist0 - (u >> 2) * 16 - (u & 3);
+        const bool seen = l16 < nq && dist >= 0 && (p.window <= 0 || dist < p.window);
+#pragma unroll
+        for (int a = 0; a < HPW; ++a) sc[a][u >> 2][u & 3] = seen ? sc[a][u >> 2][u & 3] : -INFINITY;
+      }
+    }
+    sa_bf16x8_t ph[HPW], pl[HPW];
+    float alpha[HPW];
+    bool moved = false;
+#pragma unroll
+    for (int a = 0; a < HPW; ++a) {
+      float top = fmaxf(fmaxf(fmaxf(sc[a][0][0], sc[a][0][1]), fmaxf(sc[a][0][2], sc[a][0][3])),
+                        fmaxf(fmaxf(sc[a][1][0], sc[a][1][1]), fmaxf(sc[a][1][2], sc[a][1][3])));
+      top = cw_quad_max(top);
+      const float mn = fmaxf(m[a], top);
+      alpha[a] = __builtin_amdgcn_exp2f(m[a] - mn);
+      moved = moved || alpha[a] != 1.0f;
+      m[a] = mn;
+      float sum = 0.0f;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float w = __builtin_amdgcn_exp2f(sc[a][u >> 2][u & 3] - mn);
+        sum += w;
+        const __bf16 t = (__bf16)w;
+        ph[a][u] = t;
+        pl[a][u] = (__bf16)(w - (float)t);
+      }
+      l[a] = l[a] * alpha[a] + sum;
+    }
+    if (__ballot(moved) != 0) {
+#pragma unroll
+      for (int a = 0; a < HPW; ++a)
+#pragma unroll
+        for (int cc = 0; cc < GC; ++cc)
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) out[a][cc][nt] *= alpha[a];
     }
     // O^T += V^T P^T: a fragment (one key/value head, 16 value columns) serves all of the wave's heads
     const bf16_t* vlane = vs + (4 * slot + (l16 >> 2)) * VROW + 4 * (l16 & 3);
@@ -1460,12 +1478,9 @@ __global__ __launch_bounds__((OneWalk<HPW, D32, V16, VS, GC>::THREADS)) void sin
         const sa_s16x4_t x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((sa_lds_s16x4_t*)(vp + 16 * VROW));
         const sa_bf16x8_t vf = __builtin_bit_cast(sa_bf16x8_t, __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
-        for (int a = 0; a < HPW; ++a) {
-          if (wave + 4 * a < H) {
-            out[a][cc][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, ph[a], out[a][cc][nt], 0, 0, 0);
-            out[a][cc][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl[a], out[a][cc][nt], 0, 0, 0);
-          }
-        }
+        for (int a = 0; a < HPW; ++a) out[a][cc][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, ph[a], out[a][cc][nt], 0, 0, 0);
+#pragma unroll
+        for (int a = 0; a < HPW; ++a) out[a][cc][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl[a], out[a][cc][nt], 0, 0, 0);
       }
   };
 
