@@ -13,6 +13,9 @@
 // dereferenced (their table entries may be stale or -1).
 #include "common.h"
 
+#include <limits.h>
+#include <type_traits>
+
 #ifndef CW_HD
 #error "compile with -DCW_HD=<head_dim>"
 #endif
@@ -900,20 +903,17 @@ CW_EXPORT int cw_attention_decode_bf16(const void* q, int64_t q_stride, void* ou
 // =====================================================================================
 // bfloat16 attention for portions of prompts on the matrix cores.
 //
-// A workgroup takes a run of query tokens of one request and one key/value head. Four waves own
-// 32 query rows each (row = token * gh + head of the group, so the group shares every key and
-// value); for head sizes up to 128 a second set of four waves owns the same rows and the two sets
-// split every stage's keys, so each SIMD holds two waves that hide each other's waits, and the
-// sets' running states are merged through LDS at the end. All waves walk the same stages of keys,
-// which are fetched once per workgroup into LDS, double buffered: the loads of stage t + 1 are in
-// flight while stage t is computed.
+// A workgroup takes a run of query tokens of one request and one key/value head. A wave owns 32 query
+// rows (row = token * gh + head of the group, so the group shares every key and value); NH sets of waves
+// own the same rows and each set takes its share of a stage's keys. The sets' running states are
+// put together through LDS at the end.
 //   S^T[key, row] = K * Q^T     v_mfma_f32_16x16x32_bf16; K fragments come from LDS in operand
 //                               layout (lane = key l%16, 8 consecutive head elements at slot l/16),
 //                               Q fragments are loaded once from global memory the same way;
-//   softmax per row in float32: a lane holds 8 keys of one row; the running maximum is shared by
-//                               the row's 4 lanes every tile, the running sum only at the end;
-//                               tiles that no row masks skip the position tests;
-//   O^T[d, row] += V^T * P^T    P^T is already in operand layout (the lane's 8 keys of its row).
+//   softmax per row in float32: a lane holds 8 or 16 keys of one row; the running maximum is shared by
+//                               the row's 4 lanes every stage, the running sum only at the end;
+//                               stages that no row masks skip the position tests;
+//   O^T[d, row] += V^T * P^T    P^T is already in operand layout (the lane's keys of its row).
 //                               V^T fragments come from the row-major V tile through the LDS
 //                               transposing read (ds_read_b64_tr_b16): in a group of 16 lanes, lane
 //                               i receives element i%4 of what lanes i/4, 4 + i/4, 8 + i/4 and
@@ -921,11 +921,19 @@ CW_EXPORT int cw_attention_decode_bf16(const void* q, int64_t q_stride, void* ou
 //                               elements hand every lane its column of 4 keys.
 // The element order inside an MFMA's k dimension is free as long as both operands agree; that
 // is what lets every fragment be filled by plain 8- and 16-byte reads.
+//
+// What bounds it: a SIMD's vector unit (an exponential, a fused multiply-add, an addition, a maximum and half a conversion a
+// score, some 450 cycles a wave and 32 x 32 scores) beside its matrix instructions (512 cycles); 128 bytes a cycle out of LDS
+// feed one such product, so operands of 32 rows a wave ask for as much as LDS gives. Hence: loads go straight into
+// LDS with addresses made by the scalar unit (addresses a lane, stores and page look-ups cost as much vector time as
+// half the softmax), the row's reference point is looked up in other lanes only when it moves, operand reads run
+// ahead of the products in a written order, and the two waves of a SIMD are half an interval apart. Measured on an MI355X, before
+// (tiles through registers, all waves in step) -> now: 2048 tokens of 12 heads of 128 on 2 behind 6144, 164 -> 117 us
+// (0.77 PFLOP/s on 206 compute units); of 28 on 4, 319 -> 233 (0.90); 2048 tokens without a prefix 43 -> 32.6; 137 tokens
+// 11.7 -> 9.1; 1000 tokens of 14 heads of 64 behind 7000, 69 -> 51; of 16 of 256 on 4 behind 4000, 218 -> 143.
 typedef __attribute__((ext_vector_type(4))) short s16x4_t;
-typedef __attribute__((ext_vector_type(8))) short s16x8_t;
 typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
-
-typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
+typedef __attribute__((address_space(3))) void lds_raw_t;
 
 // RB: row blocks (waves that own 32 query rows each) of a workgroup, 4 or 2. With 2 the same eight
 // waves cut a stage's keys four ways instead of two: half the rows per workgroup and half the
@@ -934,43 +942,55 @@ typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
 template <int HD, int RB>
 struct PrefillTile {
   static_assert(RB == 4 || (RB == 2 && HD <= 128), "two row blocks only with the eight-wave workgroup");
-  // The K tile lies in LDS as HD / 32 blocks of [key][32 elements]: the 64 lanes of a fragment
-  // read (16 keys x 4 slots of 8 elements) and of a stash store (16 keys x 4 chunks) then touch
-  // 1 KB without a gap, so no bank is hit twice and the rows need no padding.
-  static constexpr int VROW = HD + 16;  // V rows: 32 bytes of padding, for the 8-byte transposing reads
-  static constexpr int NH = HD <= 128 ? 8 / RB : 1;  // waves that share a row block and split its keys
-  static constexpr int KW = HD <= 128 ? 128 / NH : 32;  // keys a wave takes from a stage
-  static constexpr int KT = KW * NH;            // keys of one stage
-  static constexpr int NT = 64 * RB * NH;       // threads of a workgroup
-  static constexpr int STAGE = KT * (HD + VROW);  // elements of one stage: a K tile, then a V tile
-  static constexpr size_t BYTES = 2 * STAGE * sizeof(bf16_t);
-  static constexpr int TABLE = 2048;  // block-table entries held in LDS at a time
-  // what the sets of waves exchange at the end: accumulators, then maxima and sums
-  static constexpr size_t XO_BYTES = (size_t)(NH - 1) * RB * 2 * (HD / 16) * 64 * 16;
-  static constexpr size_t XCHG_BYTES = XO_BYTES + (size_t)(NH - 1) * RB * 2 * 2 * 64 * 4;
-  static_assert(XCHG_BYTES <= BYTES, "the exchange reuses the tiles' memory");
+  static constexpr int NH = HD <= 128 ? 8 / RB : 1;     // sets of waves: they share a row block and split its keys
+  static constexpr int KW = HD <= 128 && RB == 4 ? 64 : 32;  // keys a wave takes from a stage
+  static constexpr int KT = KW * NH;                    // keys of one stage
+  static constexpr int WAVES = RB * NH;
+  static constexpr int NT = 64 * WAVES;                 // threads of a workgroup
+  // A K or V tile lies in LDS as blocks of 16 keys x 32 elements (1 KB: what one load of a wave with the
+  // LDS target brings), [16-key group][32 elements]. Inside a block a key's four 16-byte granules are
+  // permuted (kv_granule) so that no bank is hit twice when operands are read.
+  static constexpr int TILE = KT * HD * 2;              // bytes of a tile
+  static constexpr size_t TILES = 4 * (size_t)TILE;     // two of K, two of V
+  // what the sets of waves exchange at the end: accumulators of all sets, then maxima and sums
+  static constexpr size_t XO_BYTES = NH > 1 ? (size_t)NH * RB * 2 * (HD / 16) * 64 * 16 : 0;
+  static constexpr size_t XCHG_BYTES = XO_BYTES + (NH > 1 ? (size_t)NH * RB * 2 * 2 * 64 * 4 : 0);
+  static constexpr size_t BYTES = TILES > XCHG_BYTES ? TILES : XCHG_BYTES;
 };
 
-template <int HD, bool POW2, int RB>
+// Where granule g of key k (0 to 15) lies in a block. K: eight neighbouring lanes of a ds_read_b128 take one
+// granule of eight keys, 64 bytes apart, and with these permutations every bank once; V: 16 lanes of a transposing read
+// take 32 bytes of four keys.
+__device__ __forceinline__ int k_granule(int k, int g) { return g ^ ((((k >> 1) ^ (k >> 3)) & 1) | (((k >> 2) & 1) << 1)); }
+__device__ __forceinline__ int v_granule(int k, int g) { return g ^ ((((k >> 1) ^ (k >> 2)) & 1) << 1); }
+
+// 16 bytes a lane from memory to LDS, to 1 KB at ``to`` (the same for all lanes), lane by lane; from an address a lane, or
+// from one address for all and an offset a lane. Written out, because behind the builtin the compiler puts a wait for all
+// such loads before the next transposing read, of whatever tile: what the kernel waits for and where is its own to say.
+// (No register is written.)
+__device__ __forceinline__ void load_to_lds(const void* from, void* to) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+               : : "v"(from), "s"((uint32_t)(uintptr_t)(lds_raw_t*)to) : "memory");
+}
+__device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, void* to) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               : : "v"(offset), "s"(base), "s"((uint32_t)(uintptr_t)(lds_raw_t*)to) : "memory");
+}
+
+// PAGES16: a page holds 2^n keys, 16 or more, so that 16 keys of a stage lie in one page
+template <int HD, bool PAGES16, int RB, bool CAP>
 __global__ __launch_bounds__((PrefillTile<HD, RB>::NT), (HD <= 128 ? 2 : 1)) void attn_prefill_bf16_kernel(AttnParams p) {
   using Tile = PrefillTile<HD, RB>;
-  constexpr int NF = HD / 32;     // k-steps of the score product
+  constexpr int NF = HD / 32;     // k-steps of the score product, blocks of 32 elements of a row
   constexpr int ND = HD / 16;     // 16-wide blocks of the head dimension
-  constexpr int VROW = Tile::VROW;
-  constexpr int CPR = HD / 8;     // 16-byte chunks of a row
-  constexpr int NH = Tile::NH, KW = Tile::KW, KT = Tile::KT, NT = Tile::NT;
-  constexpr int NKB = KW / 16;  // 16-key blocks of a wave's keys
-  // A wave that is at its products goes before the SIMD's other one at its softmax: heads of 128, four row blocks
-  // (2048 tokens behind 6144: 12 heads on 2 170 -> 164 us, 28 on 4 327 -> 316; smaller heads lose 3 %, with two row
-  // blocks it makes no difference)
-  constexpr bool PRIO = HD == 128 && RB == 4;
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  bf16_t* tiles = reinterpret_cast<bf16_t*>(smem_raw);  // [stage 2][K tile, V tile]
-  int* tbl = reinterpret_cast<int*>(smem_raw + Tile::BYTES);
+  constexpr int NH = Tile::NH, KW = Tile::KW, KT = Tile::KT;
+  constexpr int NKB = KW / 16;    // 16-key blocks of a wave's keys
+  extern __shared__ __align__(1024) unsigned char smem_raw[];  // K tiles 0 and 1, V tiles 0 and 1
 
   const int lane = threadIdx.x & 63;
-  const int wave = (threadIdx.x >> 6) % RB;  // the wave's row block
-  const int half = threadIdx.x / (64 * RB);  // its share of a stage's keys
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wid % RB;  // the wave's row block
+  const int half = wid / RB;  // its share of a stage's keys
   const int c = lane & 15, s = lane >> 4;
   const int item = blockIdx.x;
   const int kvh = blockIdx.y / p.n_chunks, chunk = blockIdx.y % p.n_chunks;
@@ -1001,29 +1021,68 @@ __global__ __launch_bounds__((PrefillTile<HD, RB>::NT), (HD <= 128 ? 2 : 1)) voi
     t_first += part * per;
     t_last = min(t_last, t_first + per - 1);
   }
-  // the pages of the keys this workgroup reads -> LDS, a window of Tile::TABLE entries at a time
-  // (32k keys with pages of 16): no tile waits for a table entry from memory
-  const int* table = p.block_tables + (int64_t)req * p.table_stride;
-  const int page_last = cw_page_index<POW2>(wg_last, bs, sh);
-  int page0 = cw_page_index<POW2>(min(max(t_first * KT, wg_lo), wg_last), bs, sh);  // the page of tbl[0]
-  auto load_table = [&]() __attribute__((always_inline)) {
-    const int n_pages = min(page_last - page0 + 1, Tile::TABLE);
-    for (int i = threadIdx.x; i < n_pages; i += NT) tbl[i] = table[page0 + i];
+
+  // ---- tile traffic. A wave brings 16 keys of a stage (all of their blocks, or every other one where the stage has
+  // fewer groups of keys than waves): lane l takes granule l % 4 of key l / 4, four lanes 64 bytes of one row.
+  // (constant memory for the kernel: a page's number that all lanes want comes by the scalar unit)
+  const __attribute__((address_space(4))) int* const table =
+      (const __attribute__((address_space(4))) int*)(p.block_tables + (int64_t)req * p.table_stride);
+  constexpr int KG = KT / 16, SHARE = Tile::WAVES / KG;  // groups of 16 keys of a stage, waves that share one
+  static_assert(Tile::WAVES % KG == 0, "a whole number of waves a group of keys");
+  const int kg = wid % KG, sub = wid / KG;
+  const int f_key = kg * 16 + (lane >> 2);
+  const int row_elems = p.nkv * HD;
+  const bf16_t* const kc = (const bf16_t*)p.k_cache + kvh * HD;
+  const bf16_t* const vc = (const bf16_t*)p.v_cache + kvh * HD;
+  const bf16_t* const zrow = (const bf16_t*)p.zeros;
+  const int k_piece = k_granule(lane >> 2, lane & 3) * 8, v_piece = v_granule(lane >> 2, lane & 3) * 8;
+  // A key that no row sees (past the last token, or before the window's first key) is brought as its neighbour that
+  // some row sees: it is masked by its position. With whole pages a wave's 16 keys have one page and one address, and a
+  // lane an offset; else every lane has an address of its own. No page: zeros.
+  auto group_of = [&](int t) __attribute__((always_inline)) { return min(max(t * KT + kg * 16, wg_lo & ~15), wg_last & ~15); };
+  auto key_of = [&](int t) __attribute__((always_inline)) { return min(max(t * KT + f_key, wg_lo), wg_last); };
+  auto page_of = [&](int t) __attribute__((always_inline)) {
+    return PAGES16 ? table[group_of(t) >> sh] : table[cw_page_index<false>(key_of(t), bs, sh)];
   };
-  load_table();
-  __syncthreads();
-  const bf16_t* kc = (const bf16_t*)p.k_cache;
-  const bf16_t* vc = (const bf16_t*)p.v_cache;
-  const bf16_t* zrow = (const bf16_t*)p.zeros;
+  int64_t at_row = 0;   // in elements from the head's first: PAGES16 the row of the group's first key, else of the lane's key
+  int at_key = 0;       // PAGES16: the lane's row in the group, in elements
+  bool at_page = false;
+  auto aim = [&](int t, int page) __attribute__((always_inline)) {
+    at_page = page >= 0;
+    if constexpr (PAGES16) {
+      const int g = group_of(t);
+      at_row = (int64_t)(((uint64_t)(uint32_t)page * (uint32_t)bs + (uint32_t)(g & (bs - 1))) * (uint32_t)row_elems);
+      at_key = min(max(lane >> 2, wg_lo - g), wg_last - g) * (at_page ? row_elems : 0);
+    } else {
+      const uint32_t slot = (uint32_t)page * (uint32_t)bs + (uint32_t)cw_page_offset<false>(key_of(t), bs, sh);
+      at_row = (int64_t)((uint64_t)slot * (uint32_t)row_elems);
+    }
+  };
+  auto bring = [&](const bf16_t* head, int piece, int tile) __attribute__((always_inline)) {  // the wave's blocks of a tile
+    const bf16_t* const from = at_page ? head + at_row : zrow;
+#pragma unroll
+    for (int j = 0; j < (NF + SHARE - 1) / SHARE; ++j) {
+      const int blk = j * SHARE + sub;
+      unsigned char* const to = smem_raw + tile * Tile::TILE + (kg * NF + blk) * 1024;
+      if (NF % SHARE == 0 || blk < NF) {
+        if constexpr (PAGES16) load_to_lds(from + blk * 32, (uint32_t)(at_key + piece) * 2, to);
+        else load_to_lds(from + blk * 32 + piece, to);
+      }
+    }
+  };
 
   // ---- the wave's rows: block b, column c -> row b * 16 + c
   const bool wave_on = wave * tpw < ntok;
   const int p_first = pos0 + wave * tpw;
   const int p_last = pos0 + min(ntok, (wave + 1) * tpw) - 1;
   const int lo = p.window > 0 ? max(0, p_first - p.window + 1) : 0;
-  int row_pos[2];      // position of the row's token, -1 for an unused row
-  int64_t row_off[2];  // offset of the row's head in q / out, in elements
+  int row_pos[2];  // position of the row's token, far below zero for an unused row
   bf16x8_t qf[2][NF];
+  int page_a = 0, page_b = 0;
+  if (t_first <= t_last) {
+    page_a = page_of(t_first);
+    page_b = page_of(t_first + 1);
+  }
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
     const int row = b * 16 + c;
@@ -1031,9 +1090,8 @@ __global__ __launch_bounds__((PrefillTile<HD, RB>::NT), (HD <= 128 ? 2 : 1)) voi
     const int tokw = wave * tpw + tl;
     const int hig = chunk * gh + g;
     const bool ok = wave_on && tl < tpw && tokw < ntok && hig < group;
-    row_pos[b] = ok ? pos0 + tokw : -1;
-    row_off[b] = ok ? (int64_t)(kvh * group + hig) * HD : 0;
-    const bf16_t* qrow = ok ? (const bf16_t*)p.q + (int64_t)(q_begin + tok0 + tokw) * p.q_stride + row_off[b] : zrow;
+    row_pos[b] = ok ? pos0 + tokw : INT_MIN / 2;
+    const bf16_t* qrow = ok ? (const bf16_t*)p.q + (int64_t)(q_begin + tok0 + tokw) * p.q_stride + (kvh * group + hig) * HD : zrow;
 #pragma unroll
     for (int j = 0; j < NF; ++j) qf[b][j] = *reinterpret_cast<const bf16x8_t*>(qrow + (j * 4 + s) * 8);
   }
@@ -1043,261 +1101,227 @@ __global__ __launch_bounds__((PrefillTile<HD, RB>::NT), (HD <= 128 ? 2 : 1)) voi
   for (int b = 0; b < 2; ++b)
 #pragma unroll
     for (int db = 0; db < ND; ++db) o[b][db] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
-  // running maximum in units of the raw score (the scale is positive) and the lane's share of the sum
-  float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.0f, 0.0f};
+  // The running maximum in units of the raw score (the scale is positive) and the lane's share of the sum; the
+  // exponentials' reference point (the maximum times the scale, 0 while no key has been seen); and the score beyond which it moves
+  float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.0f, 0.0f}, ref[2] = {0.0f, 0.0f}, limit[2] = {-INFINITY, -INFINITY};
   const float sl2 = p.scale * 1.4426950408889634f;  // exp(x * scale) = exp2(x * sl2)
   const float rescale_step = 8.0f / sl2;            // 8 in the exponent, in units of the raw score
 
-  // ---- tile traffic: TPK threads share a key of the stage; thread j of them takes the 16-byte
-  // chunks j, j + TPK, ... of its K row and of its V row, so a thread looks up one page and
-  // builds one address per stage, and neighbouring lanes read neighbouring chunks (lanes spread
-  // over 16 different rows, which would suit the LDS banks better, cost more in memory coalescing
-  // than they saved: measured)
-  constexpr int TPK = NT / KT;                  // threads per key
-  constexpr int NCK = (CPR + TPK - 1) / TPK;    // chunks per thread and matrix
-  const int f_key = threadIdx.x / TPK, f_ch = threadIdx.x % TPK;
-  const int64_t row_elems = (int64_t)p.nkv * HD;
-  // Two row blocks: the workgroups are short of work per stage, so a stage's loads get two stages
-  // to arrive (a second register set); with four row blocks the registers are full and one is enough
-  constexpr bool DEEP = RB == 2;
-  u32x4_t gk[NCK], gv[NCK], gk1[DEEP ? NCK : 1], gv1[DEEP ? NCK : 1];
-  auto fetch = [&](int t, u32x4_t* gk, u32x4_t* gv) __attribute__((always_inline)) {  // global -> registers; a masked key reads a row of zeros
-    const int kp = t * KT + f_key;
-    bool ok = kp >= wg_lo && kp <= wg_last;
-    const int page = tbl[ok ? cw_page_index<POW2>(kp, bs, sh) - page0 : 0];
-    ok = ok && page >= 0;
-    const int64_t off = ((int64_t)page * bs + cw_page_offset<POW2>(kp, bs, sh)) * row_elems + kvh * HD + f_ch * 8;
-    const bf16_t* kr = ok ? kc + off : zrow;
-    const bf16_t* vr = ok ? vc + off : zrow;
-    const int step = ok ? TPK * 8 : 0;  // the row of zeros is short: every chunk reads its start
+  // where a lane's operands lie in a block: of K granule s of key c; of V 8 bytes of key 4 s + c / 4, in the
+  // first or the second 16 elements
+  const int k_at = c * 64 + k_granule(c, s) * 16;
+  const int v_key = 4 * s + (c >> 2);
+  const int v_at0 = v_key * 64 + v_granule(v_key, 0) * 16 + (c & 3) * 8, v_at1 = v_at0 ^ 32;
+
+  // the stages in which the wave has rows that see keys of its share
+  const int own = half * KW;  // the share's first key in a stage
+  const int on_first = max(t_first, (max(0, lo - own - (KW - 1)) + KT - 1) / KT);
+  const int on_last = wave_on && p_last >= own ? min(t_last, (p_last - own) / KT) : -1;
+  const int all_see = p_first - own - KW + 1;                                         // a stage that begins up to here and
+  const int all_hold = p.window > 0 ? max(wg_lo, p_last - p.window + 1) - own : -KT;  // from here on has no masked pair
+  const unsigned reach = p.window > 0 ? p.window : 0x7fffffff;                       // a row sees this many keys, its own the last
+  f32x4_t sc[NKB][2];
+  bf16x8_t pf[2][NKB / 2];
+  // The matrix products of an interval: O^T += V^T P^T of stage t - 1, then S^T = K Q^T of stage t, four products at a
+  // time, whose two operands from LDS are read DEPTH times four products ahead. The order is the one written here: left to
+  // itself the compiler reads two operands, waits for them, multiplies, and so on.
+  constexpr int DEPTH = 4;
+  auto products = [&](int t, auto with_outputs, auto with_scores) __attribute__((always_inline)) {
+    constexpr int OUT = decltype(with_outputs)::value ? NKB / 2 * (ND / 2) : 0;
+    constexpr int ALL = OUT + (decltype(with_scores)::value ? NKB / 2 * NF : 0);
+    unsigned char* const vs = smem_raw + (2 + ((t - 1 - t_first) & 1)) * Tile::TILE + half * (NKB * NF * 1024);
+    const unsigned char* const ks = smem_raw + ((t - t_first) & 1) * Tile::TILE + half * (NKB * NF * 1024) + k_at;
+    bf16x8_t f[DEPTH + 1][2];
+    auto read = [&](int i) __attribute__((always_inline)) {
+      bf16x8_t(&to)[2] = f[i % (DEPTH + 1)];
+      if (i < OUT) {
 #pragma unroll
-    for (int i = 0; i < NCK; ++i) {
-      const bool in_row = CPR % TPK == 0 || f_ch + i * TPK < CPR;
-      gk[i] = *reinterpret_cast<const u32x4_t*>(kr + (in_row ? i * step : 0));
-      gv[i] = *reinterpret_cast<const u32x4_t*>(vr + (in_row ? i * step : 0));
-    }
-  };
-  auto stash = [&](int stage, const u32x4_t* gk, const u32x4_t* gv) __attribute__((always_inline)) {  // registers -> LDS
-    bf16_t* ks = tiles + stage * Tile::STAGE + f_key * 32;
-    bf16_t* vs = tiles + stage * Tile::STAGE + KT * HD + f_key * VROW + f_ch * 8;
+        for (int u = 0; u < 2; ++u) {  // 16-wide blocks 2 d and 2 d + 1 of the head dimension
+          unsigned char* vp = vs + (u ? v_at1 : v_at0) + (i / (ND / 2) * 2 * NF + i % (ND / 2)) * 1024;
+          const s16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)vp);
+          const s16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(vp + NF * 1024));
+          to[u] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+      } else {
 #pragma unroll
-    for (int i = 0; i < NCK; ++i) {
-      if (CPR % TPK == 0 || f_ch + i * TPK < CPR) {
-        const int ch = f_ch + i * TPK;  // 16-byte chunk of the row: block ch / 4, place ch % 4
-        *reinterpret_cast<u32x4_t*>(ks + (ch >> 2) * (KT * 32) + (ch & 3) * 8) = gk[i];
-        *reinterpret_cast<u32x4_t*>(vs + i * TPK * 8) = gv[i];
+        for (int u = 0; u < 2; ++u)  // 16-key blocks 2 k and 2 k + 1
+          to[u] = *reinterpret_cast<const bf16x8_t*>(ks + (((i - OUT) / NF * 2 + u) * NF + (i - OUT) % NF) * 1024);
       }
-    }
-  };
-  // the pages of stage tn must lie in the table window before it is fetched; every wave comes
-  // here between the same two barriers and nobody reads the window meanwhile
-  auto window_for = [&](int tn) __attribute__((always_inline)) {
-    const int need = cw_page_index<POW2>(min(tn * KT + KT - 1, wg_last), bs, sh);
-    if (need >= page0 + Tile::TABLE) {
-      page0 = cw_page_index<POW2>(max(tn * KT, wg_lo), bs, sh);
-      load_table();
-      __syncthreads();
-    }
-  };
-  auto compute = [&](int t, int stage) __attribute__((always_inline)) {
-    const int kv0 = t * KT + half * KW;  // the wave's keys of this stage
-    const bool active = wave_on && kv0 <= p_last && kv0 + KW - 1 >= lo;
-    if (active) {
-      const bf16_t* ks = tiles + stage * Tile::STAGE + half * KW * 32;
-      const bf16_t* vs = tiles + stage * Tile::STAGE + KT * HD + half * KW * VROW;
-      // ---- S^T = K Q^T
-      if (PRIO) __builtin_amdgcn_s_setprio(1);
-      f32x4_t sc[NKB][2];
+    };
 #pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) {
-        bf16x8_t kf[NF];
+    for (int i = 0; i < (DEPTH < ALL ? DEPTH : ALL); ++i) read(i);
 #pragma unroll
-        for (int j = 0; j < NF; ++j)
-          kf[j] = *reinterpret_cast<const bf16x8_t*>(ks + j * (KT * 32) + (kb * 16 + c) * 32 + s * 8);
+    for (int i = 0; i < ALL; ++i) {
+      if (i + DEPTH < ALL) read(i + DEPTH);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-          sc[kb][b] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-          for (int j = 0; j < NF; ++j)
-            sc[kb][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[j], qf[b][j], sc[kb][b], 0, 0, 0);
-        }
-      }
-      if (PRIO) __builtin_amdgcn_s_setprio(0);
-      if (p.softcap > 0.0f) {
-        // capped scores, kept in units of the raw score: s <- (cap / scale) * tanh(s * scale / cap)
-        const float up = p.softcap / p.scale, down = p.scale / p.softcap;
-#pragma unroll
-        for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-          for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sc[kb][b][i] = up * tanhf(sc[kb][b][i] * down);
-      }
-      // ---- softmax per row; P^T packed as the B operand of the output product.
-      // A tile needs the position tests only if some row of the wave masks some key of it.
-      const bool masked = kv0 + KW - 1 > p_first || kv0 < wg_lo || (p.window > 0 && kv0 < p_last - p.window + 1);
-      if (masked) {
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-          const int rp = row_pos[b];
-          const int rlo = p.window > 0 ? rp - p.window + 1 : 0;
-#pragma unroll
-          for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int kp = kv0 + kb * 16 + 4 * s + i;
-              if (!(kp <= rp && kp >= rlo)) sc[kb][b][i] = -INFINITY;
-            }
-        }
-      }
-      float tmax[2];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        tmax[b] = fmaxf(fmaxf(sc[0][b][0], sc[0][b][1]), fmaxf(sc[0][b][2], sc[0][b][3]));
-#pragma unroll
-        for (int kb = 1; kb < NKB; ++kb)
-          tmax[b] = fmaxf(tmax[b], fmaxf(fmaxf(sc[kb][b][0], sc[kb][b][1]), fmaxf(sc[kb][b][2], sc[kb][b][3])));
-      }
-#pragma unroll
-      for (int b = 0; b < 2; ++b) tmax[b] = cw_quad_max(tmax[b]);
-      bf16x8_t pf[2][NKB / 2];
-      float alpha[2];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        // The reference point of the exponentials moves only when the maximum has grown by more
-        // than 2^8 in the exponent (or is the row's first): probabilities then reach 256 at most,
-        // which float32 sums and bfloat16 products take without loss, and the accumulators are
-        // rescaled a few times per row instead of in most tiles. The result is the same quotient.
-        const float m_new = tmax[b] > m_run[b] + rescale_step ? tmax[b] : m_run[b];
-        // a row that has seen no key yet keeps m = -inf; its probabilities are zero
-        const float msc = m_new == -INFINITY ? 0.0f : m_new * sl2;
-        const float a = __builtin_amdgcn_exp2f(m_run[b] * sl2 - msc);
-        float psum = 0.0f;
-#pragma unroll
-        for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float pe = __builtin_amdgcn_exp2f(fmaf(sc[kb][b][i], sl2, -msc));
-            psum += pe;
-            pf[b][kb / 2][(kb & 1) * 4 + i] = (__bf16)pe;
+          const bf16x8_t x = f[i % (DEPTH + 1)][u];
+          if (i < OUT) {
+            f32x4_t& to = o[b][i % (ND / 2) * 2 + u];
+            to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, pf[b][i / (ND / 2)], to, 0, 0, 0);
+          } else {
+            const int j = (i - OUT) % NF;
+            f32x4_t& to = sc[(i - OUT) / NF * 2 + u][b];
+            to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, qf[b][j], j ? to : (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
           }
-        l_run[b] = l_run[b] * a + psum;
-        m_run[b] = m_new;
-        alpha[b] = a;
-      }
-      if (__any(alpha[0] != 1.0f || alpha[1] != 1.0f)) {
+        }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // ---- softmax per row; P^T packed as the B operand of the output product
+  auto softmax = [&](int t) __attribute__((always_inline)) {
+    if (CAP) {
+      // capped scores, kept in units of the raw score: s <- (cap / scale) * tanh(s * scale / cap)
+      const float up = p.softcap / p.scale, down = p.scale / p.softcap;
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
-          for (int db = 0; db < ND; ++db) o[b][db] *= alpha[b];
-      }
-      if (PRIO) __builtin_amdgcn_s_setprio(1);
-      // ---- O^T += V^T P^T, one 16-wide block of the head dimension at a time
-      const bf16_t* vlane = vs + (4 * s + (c >> 2)) * VROW + 4 * (c & 3);
+          for (int i = 0; i < 4; ++i) sc[kb][b][i] = up * tanhf(sc[kb][b][i] * down);
+    }
+    // a stage needs the position tests only if some row of the wave masks some key of it
+    if (t * KT > all_see || t * KT < all_hold) {
 #pragma unroll
-      for (int k2 = 0; k2 < NKB / 2; ++k2)
+      for (int b = 0; b < 2; ++b) {
+        const int behind = row_pos[b] - (t * KT + own + 4 * s);  // the row's distance from the lane's first key
 #pragma unroll
-        for (int db = 0; db < ND; ++db) {
-          const bf16_t* vp = vlane + k2 * 32 * VROW + db * 16;
-          const s16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)vp);
-          const s16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(vp + 16 * VROW));
-          const bf16x8_t vt = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+        for (int kb = 0; kb < NKB; ++kb) {
 #pragma unroll
-          for (int b = 0; b < 2; ++b) o[b][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, pf[b][k2], o[b][db], 0, 0, 0);
+          for (int i = 0; i < 4; ++i)
+            if ((unsigned)(behind - (kb * 16 + i)) >= reach) sc[kb][b][i] = -INFINITY;
+          __builtin_amdgcn_sched_barrier(0);  // (the compiler would make all comparisons first, and spill them)
         }
-      if (PRIO) __builtin_amdgcn_s_setprio(0);
+      }
+    }
+    // The reference point of the exponentials moves only when the maximum has grown by more
+    // than 2^8 in the exponent (or is the row's first): probabilities then reach 256 at most,
+    // which float32 sums and bfloat16 products take without loss, and the accumulators are
+    // rescaled a few times per row instead of in most stages. The result is the same quotient.
+    // (fmed3 with infinity is the maximum without fmaxf's care for signalling NaNs, an instruction a score)
+    float most[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      most[b] = sc[0][b][0];
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (kb + i > 0) most[b] = __builtin_amdgcn_fmed3f(most[b], sc[kb][b][i], INFINITY);
+    }
+    if (__any(most[0] > limit[0] || most[1] > limit[1])) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const float top = cw_quad_max(most[b]);
+        const bool moves = top > limit[b];
+        const float to = moves ? top * sl2 : ref[b];
+        // (a row that has seen no key yet has nothing to rescale)
+        const float a = !moves || m_run[b] == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(ref[b] - to);
+        ref[b] = to;
+        m_run[b] = moves ? top : m_run[b];
+        limit[b] = moves ? top + rescale_step : limit[b];
+        l_run[b] *= a;
+#pragma unroll
+        for (int db = 0; db < ND; ++db) o[b][db] *= a;
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      float psum = 0.0f;
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float pe = __builtin_amdgcn_exp2f(fmaf(sc[kb][b][i], sl2, -ref[b]));
+          psum += pe;
+          pf[b][kb / 2][(kb & 1) * 4 + i] = (__bf16)pe;
+        }
+      l_run[b] += psum;
     }
   };
 
-  fetch(t_first, gk, gv);
-  stash(0, gk, gv);
-  // Every load so far (the query fragments among them) has to be home before the loop starts:
-  // the loop's first use of a fragment would otherwise carry a wait for "all loads but the last
-  // few", and in every later round that wait would sit on the stage just requested, in order.
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-  if constexpr (DEEP) {
-    // set 0 holds stage t + 1 while an even round computes stage t, set 1 stage t + 2; each set is
-    // stashed at the end of the round before its stage is computed and filled again at once
-    if (t_first + 1 <= t_last) fetch(t_first + 1, gk, gv);
-    if (t_first + 2 <= t_last) fetch(t_first + 2, gk1, gv1);
-    __syncthreads();
-    // The two waves of a SIMD (sets h and h + NH / 2) would walk through a round in step, both in
-    // the score product, then both in the softmax, each waiting for the unit the other holds. The
-    // later sets move their tile traffic to the start of the round (the buffer it writes was last
-    // read before the barrier), so their phases fall beside other ones of the earlier sets:
-    // 2048 tokens of 12 heads on 2 key/value heads 44.5 -> 42.6 us.
-    const bool late = half >= NH / 2;
-    for (int t = t_first; t <= t_last; t += 2) {
-      if (!late) compute(t, 0);
-      if (t + 1 <= t_last) stash(1, gk, gv);
-      if (t + 3 <= t_last) {
-        window_for(t + 3);
-        fetch(t + 3, gk, gv);
-      }
-      if (late) compute(t, 0);
-      __syncthreads();
-      if (t + 1 > t_last) break;
-      if (!late) compute(t + 1, 1);
-      if (t + 2 <= t_last) stash(0, gk1, gv1);
-      if (t + 4 <= t_last) {
-        window_for(t + 4);
-        fetch(t + 4, gk1, gv1);
-      }
-      if (late) compute(t + 1, 1);
-      __syncthreads();
-    }
-  } else {
-    __syncthreads();
-    for (int t = t_first; t <= t_last; ++t) {
-      const int stage = (t - t_first) & 1;
-      if (t < t_last) {
-        window_for(t + 1);
-        fetch(t + 1, gk, gv);  // in flight while this tile is computed
-      }
-      compute(t, stage);
-      if (t < t_last) stash(stage ^ 1, gk, gv);  // tile t + 1, read in the next round; nobody reads that buffer now
-      __syncthreads();
+  // ---- the walk. An interval between two barriers makes the output product of stage t - 1 and the scores and softmax
+  // of stage t, while K of stage t + 1 and V of stage t come into the tiles that the interval before has read last.
+  // The two waves of a SIMD (sets h and h + NH / 2) would walk through it in step, both in the products, then both in the
+  // softmax, each waiting for the unit that the other holds. So the later sets pass the barrier between
+  // products and softmax instead of behind the softmax, and one's products run beside the other's softmax.
+  const bool late = NH > 1 && half >= NH / 2;
+  auto next_interval = [&](int t, int page) __attribute__((always_inline)) {  // the one of stage t begins; the page of stage t + 1
+    // vmcnt(0), lgkmcnt(0): this wave's share of K of stage t and of V of stage t - 1 is in LDS, and its reads are back
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();        // everyone's is, and the tiles that stage t + 1 comes into have been read
+    asm volatile("" ::: "memory");
+    if (t > t_last) return;
+    if (t > t_first) bring(vc, v_piece, 2 + ((t - t_first) & 1));
+    aim(t + 1, page);  // (behind the last stage: a tile that nobody reads)
+    bring(kc, k_piece, (t + 1 - t_first) & 1);
+  };
+  if (t_first <= t_last) {
+    aim(t_first, page_a);
+    bring(kc, k_piece, 0);
+    bring(vc, v_piece, 2);  // (later V comes one interval after K)
+    const bool active = on_first <= on_last;
+    const int until = active ? on_first : t_last + 1;
+    next_interval(t_first, page_b);
+    for (int t = t_first + 1; t <= until; ++t) next_interval(t, page_of(t + 1));
+    if (active) {
+      products(on_first, std::false_type{}, std::true_type{});
+      int page = page_of(on_first + 2);
+      for (int t = on_first; t <= on_last; ++t) {
+        if (late) next_interval(t + 1, page);
+        page = page_of(t + (late ? 3 : 2));  // (here no read of LDS is on its way: with one the wait for either is for both)
+        softmax(t);
+        if (!late) next_interval(t + 1, page);
+        products(t + 1, std::true_type{}, std::true_type{});  // (the last scores go nowhere: one copy of the products keeps
+      }                                                        // the accumulators in their registers)
+      for (int t = on_last + 2; t <= t_last + 1; ++t) next_interval(t, page_of(t + 1));
     }
   }
 
-  // ---- the other sets of waves hand their rows' state to the first set through LDS (the tiles
-  // are dead after the loop's last barrier): o, then m and l, lanes side by side; the first set
-  // merges them in a fixed order
+  // ---- the sets of waves put their rows' states together through LDS: everyone's accumulators, maxima and sums go
+  // there, and each set finishes its share of the head dimension
+  constexpr int DB = (ND + NH - 1) / NH;  // 16-wide blocks of the head dimension that a set finishes
+  const int db0 = NH > 1 ? half * DB : 0;
   if constexpr (NH > 1) {
-    constexpr int SET = RB * 2 * ND * 64;  // accumulator vectors of one set
     f32x4_t* xo = reinterpret_cast<f32x4_t*>(smem_raw);
     float* xml = reinterpret_cast<float*>(smem_raw + Tile::XO_BYTES);
-    if (half > 0) {
+    cw_lds_barrier();  // the tiles are dead
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
+    for (int b = 0; b < 2; ++b) {
 #pragma unroll
-        for (int db = 0; db < ND; ++db) xo[(half - 1) * SET + ((wave * 2 + b) * ND + db) * 64 + lane] = o[b][db];
-        xml[(((half - 1) * RB + wave) * 2 + b) * 128 + lane] = m_run[b];
-        xml[(((half - 1) * RB + wave) * 2 + b) * 128 + 64 + lane] = l_run[b];
-      }
+      for (int db = 0; db < ND; ++db) xo[(((half * RB + wave) * 2 + b) * ND + db) * 64 + lane] = o[b][db];
+      xml[((half * RB + wave) * 2 + b) * 128 + lane] = m_run[b];
+      xml[((half * RB + wave) * 2 + b) * 128 + 64 + lane] = l_run[b];
     }
-    __syncthreads();
-    if (half > 0) return;
-#pragma unroll 1
-    for (int h = 0; h < NH - 1; ++h) {
+    cw_lds_barrier();
+    if (db0 >= ND) return;
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const float m1 = xml[((h * RB + wave) * 2 + b) * 128 + lane];
-        const float l1 = xml[((h * RB + wave) * 2 + b) * 128 + 64 + lane];
-        const float m = fmaxf(m_run[b], m1);
-        const float msc = m == -INFINITY ? 0.0f : m * sl2;
-        const float a0 = __builtin_amdgcn_exp2f(m_run[b] * sl2 - msc);
-        const float a1 = __builtin_amdgcn_exp2f(m1 * sl2 - msc);
-        l_run[b] = l_run[b] * a0 + l1 * a1;
-        m_run[b] = m;
+    for (int b = 0; b < 2; ++b) {
+      float mh[NH], m = -INFINITY, l = 0.0f;
 #pragma unroll
-        for (int db = 0; db < ND; ++db) {
-          const f32x4_t o1 = xo[h * SET + ((wave * 2 + b) * ND + db) * 64 + lane];
-          o[b][db] = o[b][db] * a0 + o1 * a1;
-        }
+      for (int h = 0; h < NH; ++h) {
+        mh[h] = xml[((h * RB + wave) * 2 + b) * 128 + lane];
+        m = fmaxf(m, mh[h]);
       }
+      const float msc = m == -INFINITY ? 0.0f : m * sl2;
+#pragma unroll
+      for (int d = 0; d < DB; ++d) o[b][d] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int h = 0; h < NH; ++h) {
+        const float a = __builtin_amdgcn_exp2f(mh[h] * sl2 - msc);
+        l += xml[((h * RB + wave) * 2 + b) * 128 + 64 + lane] * a;
+#pragma unroll
+        for (int d = 0; d < DB; ++d) o[b][d] += xo[(((h * RB + wave) * 2 + b) * ND + db0 + d) * 64 + lane] * a;
+      }
+      m_run[b] = m;
+      l_run[b] = l;
     }
   }
+  constexpr int DF = NH > 1 ? DB : ND;  // blocks of the head dimension in o
 
   // ---- a part of the key range: unnormalised sums, maximum and sum of every row of the workgroup
   // (unused rows too: zeros) for the merge kernel
@@ -1308,8 +1332,8 @@ __global__ __launch_bounds__((PrefillTile<HD, RB>::NT), (HD <= 128 ? 2 : 1)) voi
       const float l = cw_quad_sum(l_run[b]);
       const int64_t row = slot + wave * 32 + b * 16 + c;
 #pragma unroll
-      for (int db = 0; db < ND; ++db) *reinterpret_cast<f32x4_t*>(p.part_o + row * HD + db * 16 + 4 * s) = o[b][db];
-      if (s == 0) {
+      for (int d = 0; d < DF; ++d) *reinterpret_cast<f32x4_t*>(p.part_o + row * HD + (db0 + d) * 16 + 4 * s) = o[b][d];
+      if (s == 0 && half == 0) {
         p.part_ml[row * 2] = m_run[b];
         p.part_ml[row * 2 + 1] = l;
       }
@@ -1323,23 +1347,25 @@ __global__ __launch_bounds__((PrefillTile<HD, RB>::NT), (HD <= 128 ? 2 : 1)) voi
     float l = l_run[b];
     l = cw_quad_sum(l);
     if (row_pos[b] < 0) continue;
-    const float inv = attn_head_gate(p, q_begin + (row_pos[b] - (ctx - qlen)), (int)(row_off[b] / HD)) / l;
-    bf16_t* orow = (bf16_t*)p.out + (int64_t)(q_begin + (row_pos[b] - (ctx - qlen))) * p.out_stride + row_off[b];
+    const int head = kvh * group + chunk * gh + (b * 16 + c) % gh;
+    const int64_t token = q_begin + (row_pos[b] - (ctx - qlen));
+    const float inv = attn_head_gate(p, token, head) / l;
+    bf16_t* orow = (bf16_t*)p.out + token * p.out_stride + head * HD;
 #pragma unroll
-    for (int db = 0; db < ND; ++db) {
+    for (int d = 0; d < DF; ++d) {
       uint2 packed;
-      packed.x = (uint32_t)cw_float_to_bf16_bits(o[b][db][0] * inv) | ((uint32_t)cw_float_to_bf16_bits(o[b][db][1] * inv) << 16);
-      packed.y = (uint32_t)cw_float_to_bf16_bits(o[b][db][2] * inv) | ((uint32_t)cw_float_to_bf16_bits(o[b][db][3] * inv) << 16);
-      *reinterpret_cast<uint2*>(orow + db * 16 + 4 * s) = packed;
+      packed.x = (uint32_t)cw_float_to_bf16_bits(o[b][d][0] * inv) | ((uint32_t)cw_float_to_bf16_bits(o[b][d][1] * inv) << 16);
+      packed.y = (uint32_t)cw_float_to_bf16_bits(o[b][d][2] * inv) | ((uint32_t)cw_float_to_bf16_bits(o[b][d][3] * inv) << 16);
+      *reinterpret_cast<uint2*>(orow + (db0 + d) * 16 + 4 * s) = packed;
     }
   }
 }
 
-// Puts together the parts of items whose key range was shared among workgroups. One workgroup per
-// (item, key/value head) as in the kernel above; the workgroups of an item's parts share its rows
-// (part z takes rows z * ceil(rows / parts) ...), each reading those rows of every part. With few
-// rows a workgroup its threads also share the parts: thread (row, 4 elements, slice) sums the parts
-// slice, slice + S, ..., and the slices meet in LDS in a fixed order.
+// Puts together the parts of items whose key range was shared among workgroups. Four workgroups per (item, key/value
+// head) of the kernel above (with one a thread had eight rounds of loads: 1000 tokens behind 7000, 14 -> 6 us). The
+// workgroups of an item's parts share its rows, each reading its rows of every part. With few rows a workgroup its threads
+// also share the parts: thread (row, 4 elements, slice) sums the parts slice, slice + S, ..., and the slices meet in LDS
+// in a fixed order.
 #define PREFILL_MAX_PARTS 255
 
 template <int HD, int RB>
@@ -1358,8 +1384,9 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(AttnParams p) {
   const int q_begin = p.cu_q[req];
   const int ntok = min(p.items[4 * item + 2], p.cu_q[req + 1] - q_begin - tok0);
   const float sl2 = p.scale * 1.4426950408889634f;
-  const int rpb = (ROWS + parts - 1) / parts;  // rows of this workgroup
-  const int row0 = part * rpb;
+  const int shares = parts * gridDim.z;
+  const int rpb = (ROWS + shares - 1) / shares;  // rows of this workgroup
+  const int row0 = (part * gridDim.z + blockIdx.z) * rpb;
   if (row0 >= ROWS) return;
   auto slot = [&](int z, int row) { return ((int64_t)(item + z) * gridDim.y + blockIdx.y) * ROWS + row; };
   for (int i = threadIdx.x; i < rpb * parts; i += 256) {
@@ -1422,25 +1449,22 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(AttnParams p) {
 CW_EXPORT int cw_attention_prefill_supported() { return CW_HAS_PREFILL; }
 
 #if CW_HAS_PREFILL
-template <bool POW2, int RB>
-static int launch_prefill(const AttnParams& p, int n_items, int table_stride, hipStream_t stream) {
+template <bool PAGES16, int RB, bool CAP>
+static int launch_prefill(const AttnParams& p, int n_items, hipStream_t stream) {
   using Tile = PrefillTile<CW_HD, RB>;
   dim3 grid(n_items, p.nkv * p.n_chunks), block(Tile::NT);
-  // two stages of K and V tiles, then the window of the block table
-  const size_t entries = (size_t)table_stride < (size_t)Tile::TABLE ? table_stride : Tile::TABLE;
-  if ((Tile::KT + p.block_size - 1) / p.block_size + 1 > Tile::TABLE) return CW_ERR_SIZE;
-  const size_t smem = Tile::BYTES + sizeof(int) * entries;
-  if (smem > 160 * 1024) return CW_ERR_SIZE;
-  static size_t raised = 0;
-  if (smem > raised && smem > 48 * 1024) {
-    if (hipFuncSetAttribute((const void*)attn_prefill_bf16_kernel<CW_HD, POW2, RB>,
+  constexpr size_t smem = Tile::BYTES;
+  static_assert(smem <= 160 * 1024, "the tiles of two stages fit a compute unit's LDS");
+  static bool raised = false;
+  if (!raised && smem > 48 * 1024) {
+    if (hipFuncSetAttribute((const void*)attn_prefill_bf16_kernel<CW_HD, PAGES16, RB, CAP>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
       return CW_ERR_LAUNCH;
-    raised = smem;
+    raised = true;
   }
-  hipLaunchKernelGGL((attn_prefill_bf16_kernel<CW_HD, POW2, RB>), grid, block, smem, stream, p);
+  hipLaunchKernelGGL((attn_prefill_bf16_kernel<CW_HD, PAGES16, RB, CAP>), grid, block, smem, stream, p);
   if (p.part_o != nullptr)
-    hipLaunchKernelGGL((attn_prefill_merge_kernel<CW_HD, RB>), grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((attn_prefill_merge_kernel<CW_HD, RB>), dim3(grid.x, grid.y, 4), dim3(256), 0, stream, p);
   return cw_launch_status();
 }
 #endif
@@ -1501,13 +1525,16 @@ CW_EXPORT int cw_attention_prefill_bf16(const void* q, int64_t q_stride, void* o
     p.part_o = workspace;
     p.part_ml = workspace + need / (CW_HD + 2) * CW_HD;
   }
+  const bool cap = softcap > 0.0f;
+  auto launch = [&](auto rb) {
+    constexpr int RB = decltype(rb)::value;
+    if (p.bs_shift >= 4) return cap ? launch_prefill<true, RB, true>(p, n_items, stream) : launch_prefill<true, RB, false>(p, n_items, stream);
+    return cap ? launch_prefill<false, RB, true>(p, n_items, stream) : launch_prefill<false, RB, false>(p, n_items, stream);
+  };
 #if CW_HD <= 128
-  if (row_blocks == 2)
-    return p.bs_shift >= 0 ? launch_prefill<true, 2>(p, n_items, table_stride, stream)
-                           : launch_prefill<false, 2>(p, n_items, table_stride, stream);
+  if (row_blocks == 2) return launch(std::integral_constant<int, 2>{});
 #endif
-  return p.bs_shift >= 0 ? launch_prefill<true, 4>(p, n_items, table_stride, stream)
-                         : launch_prefill<false, 4>(p, n_items, table_stride, stream);
+  return launch(std::integral_constant<int, 4>{});
 #else
   return CW_ERR_ARG;
 #endif

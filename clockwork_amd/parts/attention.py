@@ -132,12 +132,16 @@ def _make_plan(ctx, nh: int, nkv: int, narrow_ok: bool, whole_keys: int = 0) -> 
     wide: list = []   # one array of items per portion
     mfma: list = []
     # Workgroups of four row blocks share each key among the most rows, but a launch has to
-    # fill the compute units, and the workgroup with the longest key range decides its time:
-    # with fewer than 1.5 workgroups a compute unit, halve them (unless the key ranges are long).
+    # fill the compute units, and the workgroup with the longest key range decides its time: where
+    # they would leave a twentieth of the compute units or more idle, halve them, unless the key ranges are
+    # long (us, two row blocks / four: 206 workgroups of four, 2048 tokens of 12 heads on 2, 32.4 / 36.9; 240, 2400 tokens,
+    # 37.6 / 41.6; 252, 1000 tokens of 28 heads on 4, 29.9 / 24.4; 264, 1050 tokens, 32.8 / 25.9; 376, 1500 tokens, 48.8 / 42.5).
+    # Groups of more than 32 heads, whose last chunk leaves rows idle: from 1.5 workgroups a unit on (6 % either way).
     tokens_of_four = 4 * (32 // min(group, 32))
     workgroups = sum(-(-q // tokens_of_four) for q in ctx.h_q_lens if q > 1) * nkv * -(-group // 32)
     short_ranges = portions_have_short_ranges(ctx.h_q_lens, ctx.h_ctx_lens)
-    row_blocks = 2 if narrow_ok and short_ranges and 2 * workgroups < 3 * ctx.num_compute_units else 4
+    enough = 1.5 if group > 32 else 0.95
+    row_blocks = 2 if narrow_ok and short_ranges and workgroups < enough * ctx.num_compute_units else 4
     tokens_per_mfma_item = row_blocks * (32 // min(group, 32))
     single: list[int] = []
     longest_single = 0

@@ -1117,6 +1117,37 @@ def ops_decode_ok(hd):
     return ops.decode_attention_supported(hd, torch.bfloat16)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,bs", [(12, 2, 128, 16), (14, 2, 64, 64), (3, 1, 96, 24), (4, 2, 256, 32)])
+@pytest.mark.parametrize("window", [0, 130])
+@pytest.mark.parametrize("row_blocks", [4, 2])
+def test_prefill_attention_kernel_at_the_edges_of_its_stages(nh, nkv, hd, bs, window, row_blocks):
+    """Contexts one key around the shares (32 and 64 keys) and stages (128) of the kernel's waves, so that waves
+    begin and end their walks at different stages; pages of whole groups of 16 keys and pages that are none; NaN behind every
+    request's last key and in pages behind the window. Probabilities and results are rounded to bfloat16, by 2^-9 each
+    at most: their 2-norms add up to less than 2^-8."""
+    if row_blocks == 2 and hd > 128:
+        pytest.skip("head sizes beyond 128 have the kernel with four row blocks only")
+    ctx_lens = [2, 33, 64, 65, 127, 128, 129, 257, 513]
+    q_lens = [2, 33, 15, 64, 65, 3, 20, 130, 40]
+    tables, at = [], 0
+    perm = torch.randperm(sum(-(-c // bs) for c in ctx_lens) + 3).tolist()
+    for c in ctx_lens:
+        tables.append(perm[at : at + -(-c // bs)])
+        at += -(-c // bs)
+    kc, vc, ks, vs = _paged_setup(torch.bfloat16, nkv, hd, bs, len(perm), tables, ctx_lens, poison=float("nan"))
+    tables_dev = [[-1 if window and b < max(0, c - q - window + 1) // bs else page for b, page in enumerate(t)]
+                  for t, c, q in zip(tables, ctx_lens, q_lens)]
+    qs = [torch.randn(q, nh, hd, device=DEV).to(torch.bfloat16) for q in q_lens]
+    out = _run_attention(torch.bfloat16, nh, nkv, hd, bs, tables_dev, ctx_lens, q_lens, kc, vc, qs, window=window,
+                         prefill_kernel=row_blocks)
+    at = 0
+    for r, q_len in enumerate(q_lens):
+        want = plain.attention_dense(qs[r].double().cpu(), ks[r].double().cpu(), vs[r].double().cpu(), hd ** -0.5,
+                                     window=window or None)
+        assert (out[at : at + q_len].double().cpu() - want).norm() / want.norm() < 2.0 ** -8, (r, q_len)
+        at += q_len
+
+
 @pytest.mark.parametrize("row_blocks", [4, 2])
 def test_prefill_attention_kernel_sharp_scores(row_blocks):
     """Scores of very different size, so that the running maximum moves from tile to tile and one
