@@ -25,19 +25,15 @@ __device__ __forceinline__ float cw_to_float(bf16_t x) { return __bfloat162float
 
 template <typename T> __device__ __forceinline__ T cw_from_float(float x);
 template <> __device__ __forceinline__ float cw_from_float<float>(float x) { return x; }
-template <> __device__ __forceinline__ bf16_t cw_from_float<bf16_t>(float x) { return __float2bfloat16(x); }
+template <> __device__ __forceinline__ bf16_t cw_from_float<bf16_t>(float x) { return __builtin_bit_cast(bf16_t, (__bf16)x); }
 
 // bfloat16 bits <-> float without going through the class type (for packed 16-byte loads)
 __device__ __forceinline__ float cw_bf16_bits_to_float(uint16_t b) {
   return __uint_as_float(((uint32_t)b) << 16);
 }
-__device__ __forceinline__ uint16_t cw_float_to_bf16_bits(float f) {
-  // round to nearest even; NaN stays NaN
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
-}
+// round to nearest even, NaN stays NaN: the conversion instruction (by hand it is nine, and a kernel that runs for
+// microseconds waits for its own code)
+__device__ __forceinline__ uint16_t cw_float_to_bf16_bits(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
 // Maximum / sum over the four lanes l, l ^ 16, l ^ 32, l ^ 48 of a wave, on the vector unit: the
 // swaps of 16-lane rows and of the wave's halves (v_permlane16_swap, v_permlane32_swap) hand every
@@ -138,15 +134,25 @@ template <> struct CwVec<bf16_t, 4> {
   }
 };
 
+// Sum and maximum over a wave on the vector unit, every lane ending with the same result: neighbours, pairs, fours and eights
+// of a row of 16 lanes by data-parallel operands, rows and halves as above. (Six shuffles through the LDS unit, each
+// waiting for the one before, take half a microsecond.)
+template <int CTRL> __device__ __forceinline__ float cw_dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
 __device__ __forceinline__ float cw_wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+  v += cw_dpp<0xB1>(v);   // lane ^ 1
+  v += cw_dpp<0x4E>(v);   // lane ^ 2
+  v += cw_dpp<0x141>(v);  // mirrored halves of a row: the other four
+  v += cw_dpp<0x140>(v);  // mirrored row: the other eight
+  return cw_quad_sum(v);
 }
 __device__ __forceinline__ float cw_wave_max(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-  return v;
+  v = fmaxf(v, cw_dpp<0xB1>(v));
+  v = fmaxf(v, cw_dpp<0x4E>(v));
+  v = fmaxf(v, cw_dpp<0x141>(v));
+  v = fmaxf(v, cw_dpp<0x140>(v));
+  return cw_quad_max(v);
 }
 
 // A workgroup barrier for data that waves hand each other through LDS: LDS writes made before it

@@ -86,8 +86,8 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ resid, const T* __restric
   }
 }
 
-// The same for rows of up to 8192 elements with H % 4 == 0: every thread keeps its (at most eight)
-// 4-element chunks of the row in registers, so the row is read once, and all loads are in flight
+// The same for rows of up to 8192 elements with H % 4 == 0, in chunks of 4 elements: every thread keeps its
+// (at most eight) chunks of the row in registers, so the row is read once, and all loads are in flight
 // together. The order of the sum of squares depends on H alone here too.
 template <typename T> struct Chunk4;
 template <> struct Chunk4<float> {
@@ -113,10 +113,75 @@ template <> struct Chunk4<bf16_t> {
   }
 };
 
-// KC: chunks of 4 elements a thread holds (rows of up to 1024 * KC elements).
-// Bound, for few rows, by its trips to memory, about a microsecond each: the row, the weights, the pending output and
-// up to eight planes of partial sums are all asked for before any of them is used (asked for one after the other, the
-// norm of 8 rows of 1536 with an output and six planes pending took 5.75 us in a decode step, 5.0 so).
+// The same for rows of up to 4096 elements, one chunk a thread: H / 4 threads, rounded up to whole waves.
+// Bound, for few rows, by its trips to memory, about a microsecond each, and by its own code: the row, the weights, the
+// pending output and up to eight planes of partial sums are all asked for before any of them is used, and there is one copy of
+// everything (the kernel below, with two or four chunks a thread, is 6 to 9 KB of code, this one 3 KB). With it, with sums
+// over a wave on the vector unit and bfloat16 rounded by the conversion instruction a decode step of 8 requests of the
+// 1.5B shape took 1465 us instead of 1502, of 64 requests 2379 / 2423, of 8 of the 7B shape 3410 / 3510.
+template <typename T, typename WT, typename DT>
+__global__ __launch_bounds__(1024) void add_rmsnorm_row_kernel(float* __restrict__ resid, const T* __restrict__ delta0,
+                                                               const DT* __restrict__ delta, int parts, int64_t part_stride,
+                                                               const WT* __restrict__ weight, float eps, T* __restrict__ out,
+                                                               const int* __restrict__ rows, int H,
+                                                               const WT* __restrict__ weight2, T* __restrict__ out2) {
+  constexpr int PU = 8;  // planes on their way at a time
+  __shared__ float partial[16];
+  const int i = blockIdx.x;
+  const int64_t t = rows ? rows[i] : i;
+  const bool in = (int)threadIdx.x < H / 4;
+  const int at = in ? threadIdx.x * 4 : 0;
+  float* const x = resid + t * H + at;
+  float v[4], w[4], e0[4], d[PU][4];
+  Chunk4<float>::load(x, v);
+  if (delta0) Chunk4<T>::load(delta0 + t * H + at, e0);
+  auto load_planes = [&](int q0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < PU; ++u)
+      if (q0 + u < parts) Chunk4<DT>::load(delta + (q0 + u) * part_stride + t * H + at, d[u]);
+  };
+  if (delta) load_planes(0);
+  Chunk4<WT>::load(weight + at, w);
+  if (delta0)  // an earlier branch's output that was not added yet: it comes first, as it would have
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += e0[e];
+  if (delta) {  // the partial sums are added in order
+    float acc[4];
+    for (int q0 = 0; q0 < parts; q0 += PU) {
+      if (q0 > 0) load_planes(q0);
+#pragma unroll
+      for (int u = 0; u < PU; ++u)
+        if (q0 + u < parts)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[e] = q0 + u == 0 ? d[u][e] : acc[e] + d[u][e];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += acc[e];
+  }
+  if (in && rows == nullptr && (delta || delta0)) Chunk4<float>::store(x, v);
+  const float ss = cw_wave_sum(in ? (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]) : 0.0f);
+  if ((threadIdx.x & 63) == 0) partial[threadIdx.x >> 6] = ss;
+  cw_lds_barrier();
+  float total = 0.0f;
+  for (int k = 0; k < (int)(blockDim.x >> 6); ++k) total += partial[k];
+  const float inv = 1.0f / sqrtf(total / (float)H + eps);
+  if (!in) return;
+  float r[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    v[e] = cw_to_float(cw_from_float<T>(v[e] * inv));
+    r[e] = w[e] * v[e];
+  }
+  Chunk4<T>::store(out + (int64_t)i * H + at, r);
+  if (out2) {  // a second norm of the same row: its statistics are the first's
+    Chunk4<WT>::load(weight2 + at, w);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = w[e] * v[e];
+    Chunk4<T>::store(out2 + (int64_t)i * H + at, r);
+  }
+}
+
+// KC: chunks of 4 elements a thread holds (rows of up to 1024 * KC elements): rows of more than 4096 elements.
 template <typename T, typename WT, typename DT, int KC>
 __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict__ resid, const T* __restrict__ delta0,
                                                               const DT* __restrict__ delta,
@@ -238,16 +303,8 @@ CW_EXPORT int cw_add_rmsnorm(float* resid, const void* delta0, const void* delta
   const int64_t part_stride = (int64_t)T_rows * H;
 #define CW_LAUNCH(T, WT, DT)                                                                           \
   do {                                                                                                 \
-    if (vec && H <= 1024)                                                                              \
-      hipLaunchKernelGGL((add_rmsnorm_vec_kernel<T, WT, DT, 1>), grid, block, 0, stream, resid,        \
-                         (const T*)delta0, (const DT*)delta, parts, part_stride, (const WT*)weight, eps, \
-                         (T*)out, rows, H, (const WT*)weight2, (T*)out2);                                                            \
-    else if (vec && H <= 2048)                                                                         \
-      hipLaunchKernelGGL((add_rmsnorm_vec_kernel<T, WT, DT, 2>), grid, block, 0, stream, resid,        \
-                         (const T*)delta0, (const DT*)delta, parts, part_stride, (const WT*)weight, eps, \
-                         (T*)out, rows, H, (const WT*)weight2, (T*)out2);                                                            \
-    else if (vec && H <= 4096)                                                                         \
-      hipLaunchKernelGGL((add_rmsnorm_vec_kernel<T, WT, DT, 4>), grid, block, 0, stream, resid,        \
+    if (vec && H <= 4096)                                                                              \
+      hipLaunchKernelGGL((add_rmsnorm_row_kernel<T, WT, DT>), grid, dim3((H / 4 + 63) / 64 * 64), 0, stream, resid, \
                          (const T*)delta0, (const DT*)delta, parts, part_stride, (const WT*)weight, eps, \
                          (T*)out, rows, H, (const WT*)weight2, (T*)out2);                                                            \
     else if (vec)                                                                                      \

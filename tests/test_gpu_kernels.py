@@ -359,6 +359,31 @@ def test_gemm_f32_rows_do_not_depend_on_batch():
     assert torch.equal(ops.linear(x[250:267].contiguous(), w, b), whole[250:267])
 
 
+@pytest.mark.parametrize("N,K", [(16, 16), (17, 48), (1152, 896), (90, 1920), (90, 1936), (100, 4864), (65600, 64)])
+def test_gemm_f32_few_rows_by_blocks(N, K):
+    """Up to 16 rows with a K of whole blocks of 16: one block, fewer blocks than waves, one part, several parts
+    that meet in LDS, more blocks than a workgroup takes, an output that another kernel makes, and planes; the same
+    bits for a row alone, among 3, among 16 and among 40 (tiles)."""
+    from clockwork_amd import ops
+
+    x, w, b = (torch.randn(*s, device=DEV) for s in ((40, K), (N, K), (N,)))
+    whole = ops.linear(x, w, b)
+    want = x.double() @ w.double().t() + b.double()
+    # a block of 16 and up to 1 + K / 16 additions, each rounded at 2^-24 of a partial sum
+    assert (whole.double() - want).norm() / want.norm() < 2.0 ** -24 * (16 + K / 16) ** 0.5
+    for lo, hi in ((0, 1), (7, 10), (20, 36)):
+        assert torch.equal(ops.linear(x[lo:hi].contiguous(), w, b), whole[lo:hi])
+    whole = ops.linear(x, w)
+    for lo, hi in ((0, 1), (20, 36)):
+        got = ops.linear(x[lo:hi].contiguous(), w, partial_ok=True)
+        if isinstance(got, ops.PartialSums):
+            total = got.parts[0].clone()
+            for part in got.parts[1:]:
+                total += part
+            got = total
+        assert torch.equal(got, whole[lo:hi])
+
+
 @pytest.mark.parametrize("M", [1, 8, 16, 17, 33, 64])
 @pytest.mark.parametrize("N,K", [(100, 176), (2048, 1536), (48, 64), (5000, 200)])
 def test_skinny_bf16_product(M, N, K):
@@ -833,6 +858,33 @@ def _run_attention(dtype, nh, nkv, hd, bs, tables, ctx_lens, q_lens, kc, vc, qs,
     return out.view(T, nh, hd)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H", [4, 252, 256, 260, 1536, 4092, 4096, 4100])
+@pytest.mark.parametrize("planes", [0, 1, 8, 9])
+def test_add_rmsnorm_a_chunk_a_thread(dtype, H, planes):
+    """Rows around whole waves and around the longest that 1024 threads take, with planes of partial sums around
+    the eight that are asked for at once, an output pending before them and some rows only. Against float64: the
+    sum of up to 4100 squares by waves rounds a few times at 2^-24, bfloat16 outputs twice at 2^-9."""
+    from clockwork_amd import ops
+
+    T = 5
+    resid = torch.randn(T, H, device=DEV)
+    first = torch.randn(T, H, device=DEV).to(dtype)
+    delta = torch.randn(planes, T, H, device=DEV) if planes else torch.randn(T, H, device=DEV).to(dtype)
+    weight = (1.0 + 0.1 * torch.randn(H, device=DEV)).to(dtype)
+    total = resid.double() + first.double() + (delta.double().sum(0) if planes else delta.double())
+    for rows in (None, [3, 0]):
+        r, out = resid.clone(), torch.empty((len(rows) if rows else T, H), dtype=dtype, device=DEV)
+        ops.add_rmsnorm(r, ops.PendingPair(first, ops.PartialSums(delta) if planes else delta), weight, 1e-6, out=out,
+                        rows=torch.tensor(rows, dtype=torch.int32, device=DEV) if rows else None)
+        want = total[rows] if rows else total
+        want = want / torch.sqrt(want.square().mean(-1, keepdim=True) + 1e-6) * weight.double()
+        assert (out.double() - want).norm() / want.norm() < (2.0 ** -8 if dtype == torch.bfloat16 else 1e-6)
+        # the stream is written where all rows are normed: the planes' sum and two additions, each rounded once
+        kept = resid.double() if rows else total
+        assert (r.double() - kept).abs().max() <= 16 * 2.0 ** -24 * kept.abs().max() + (0 if rows else 1e-6)
+
+
 # the reference's decode cases (tests/test_triton_kernel.py:14-20) plus sizes of our own
 DECODE_CASES = [
     (4, 4, 16, 4, [5, 12, 9]),
@@ -975,6 +1027,26 @@ def test_decode_attention_kernel(nh, nkv, hd, bs, ctx_lens, splits, fixed_ranges
     for r in range(len(ctx_lens)):
         want = plain.attention_dense(qs[r].float().cpu(), ks[r].float().cpu(), vs[r].float().cpu(), hd ** -0.5)
         torch.testing.assert_close(out[r : r + 1].float().cpu(), want, **tol(dtype))
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(6, 2, 96), (4, 1, 32), (12, 2, 128), (40, 2, 64), (2, 2, 160), (2, 1, 256)])
+@pytest.mark.parametrize("splits", [2, 3, 8, 9, 16, 17, 63, 64, 65, 129])
+def test_decode_attention_merge(nh, nkv, hd, splits):
+    """Splits around what a wave of the merging kernel takes at once (whole heads, pieces of 32 elements, statistics of
+    more than 64),
+    with contexts that leave most splits empty. Probabilities and results are rounded to bfloat16: under 2^-8 together."""
+    bs, ctx_lens = 16, [1, 33, 700, 2100]
+    tables, at = [], 0
+    perm = torch.randperm(sum(-(-c // bs) for c in ctx_lens) + 2).tolist()
+    for c in ctx_lens:
+        tables.append(perm[at : at + -(-c // bs)])
+        at += -(-c // bs)
+    kc, vc, ks, vs = _paged_setup(torch.bfloat16, nkv, hd, bs, len(perm), tables, ctx_lens, poison=float("nan"))
+    qs = [torch.randn(1, nh, hd, device=DEV).to(torch.bfloat16) for _ in ctx_lens]
+    out = _run_attention(torch.bfloat16, nh, nkv, hd, bs, tables, ctx_lens, [1] * 4, kc, vc, qs, splits=splits, decode_kernel=True)
+    for r in range(len(ctx_lens)):
+        want = plain.attention_dense(qs[r].double().cpu(), ks[r].double().cpu(), vs[r].double().cpu(), hd ** -0.5)
+        assert (out[r : r + 1].double().cpu() - want).norm() / want.norm() < 2.0 ** -8
 
 
 @pytest.mark.parametrize("nh,nkv,hd,bs", [(4, 2, 32, 4), (6, 1, 32, 8), (3, 3, 64, 16), (12, 2, 128, 16), (2, 1, 256, 16),
