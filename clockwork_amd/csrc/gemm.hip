@@ -65,9 +65,8 @@ __device__ __forceinline__ f32x4_t gemm_f32_load4(const float* __restrict__ row,
 // projections, one trip to memory): eight blocks of 16 k-values are on their way while eight are multiplied.
 // With plane_stride > 0 a part's sum is written out as plane z of C (whoever reads y next adds the planes
 // in order); else the parts meet in LDS.
-// Measured on an MI355X with one row of x, the four products of a layer of the 0.5B shape: 42 us (q/k/v 9.5, output
-// 9.2, gate/up 13.6 for 35 MB, down 9.5), against 111 us of vector-unit tiles of 64 x 64 with partial sums in memory
-// and 20 us for the kernels that added them.
+// For rows of whole blocks there is a faster kernel below; this one serves other K, the widest outputs and long K
+// whose parts meet in LDS.
 template <bool VEC>
 __global__ __launch_bounds__(512) void gemm_f32_rows_kernel(const float* __restrict__ A, int64_t lda,
                                                             const float* __restrict__ W,
@@ -133,6 +132,73 @@ __global__ __launch_bounds__(512) void gemm_f32_rows_kernel(const float* __restr
     float total = p[0];
     for (int z = 1; z < parts; ++z) total += p[z * 256];
     if (m < M && n < N) C[(int64_t)m * ldc + n] = total + (bias ? bias[n] : 0.0f);
+  }
+}
+
+// The same sums for rows of whole blocks (K a multiple of 16): the waves of a workgroup share the blocks of 16 k-values of
+// its parts of a tile of 16 rows of W, not the parts, so a workgroup's whole share of W is asked for at once; the blocks'
+// sums meet in LDS, [block][token][row of W], and are added in their order there. What bounds it is one trip to memory
+// and, for the large matrices, the stream of W. Measured on an MI355X with one row of x against the kernel above (whose waves
+// make a part each, eight blocks at a time, and which is twice the code): 1152 x 896 8.0 -> 5.0 us, 9728 x 896 14.4 -> 12.0,
+// 2048 x 1536 9.9 -> 8.3; the sums are the same bit for bit.
+#define GT_BLOCK_WAVES 8
+#define GT_BLOCKS 120   // blocks a workgroup takes: 1 KB of LDS each with 16 rows of x
+__global__ __launch_bounds__(GT_BLOCK_WAVES * 64) void gemm_f32_blocks_kernel(const float* __restrict__ A, int64_t lda,
+                                                                              const float* __restrict__ W,
+                                                                              const float* __restrict__ bias, float* __restrict__ C,
+                                                                              int64_t ldc, int M, int N, int K, int parts, int part_blocks,
+                                                                              int parts_here, int64_t plane_stride) {
+  extern __shared__ __align__(16) float red[];
+  constexpr int U = 8;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, s = lane >> 4;
+  const int n0 = blockIdx.x * 16;
+  const int z0 = blockIdx.y * parts_here, z1 = min(parts, z0 + parts_here);
+  const int b0 = z0 * part_blocks, b1 = min(K / 16, z1 * part_blocks);
+  const float* const w = W + (int64_t)min(n0 + (lane >> 2), N - 1) * K + 4 * (lane & 3);
+  const float* const x = A + (int64_t)min(r, M - 1) * lda + 4 * s;
+  for (int b = b0 + wave; b < b1; b += U * GT_BLOCK_WAVES) {
+    f32x4_t wv[U], xv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (b + u * GT_BLOCK_WAVES < b1) {
+        wv[u] = *reinterpret_cast<const f32x4_t*>(w + (b + u * GT_BLOCK_WAVES) * 16);
+        xv[u] = *reinterpret_cast<const f32x4_t*>(x + (b + u * GT_BLOCK_WAVES) * 16);
+      }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (b + u * GT_BLOCK_WAVES < b1) {
+        // lane (r, s) holds rows 4 s .. 4 s + 3 of W for token r
+        const f32x4_t t = gemm_f32_block(__builtin_bit_cast(f32x4_t, cw_swap_to_operand(__builtin_bit_cast(cw_i32x4_t, wv[u]), lane)), xv[u]);
+        if (r < M) *reinterpret_cast<f32x4_t*>(&red[((b + u * GT_BLOCK_WAVES - b0) * M + r) * 16 + 4 * s]) = t;
+      }
+  }
+  cw_lds_barrier();
+  // a thread takes one output of one part; without planes the parts' sums meet in LDS again, behind the blocks'
+  float* const sums = red + (b1 - b0) * M * 16;
+  const int outputs = M * 16;
+  for (int i = threadIdx.x; i < outputs * (z1 - z0); i += GT_BLOCK_WAVES * 64) {
+    const int z = i / outputs, at = i - z * outputs;
+    const int from = z * part_blocks, to = min(b1 - b0, from + part_blocks);
+    float total = red[from * outputs + at];
+#pragma unroll 8
+    for (int b = from + 1; b < to; ++b) total += red[b * outputs + at];
+    const int n = n0 + (at & 15);
+    if (plane_stride > 0) {
+      if (n < N) C[(z0 + z) * plane_stride + (int64_t)(at >> 4) * ldc + n] = total;
+    } else if (parts == 1) {
+      if (n < N) C[(int64_t)(at >> 4) * ldc + n] = total + (bias ? bias[n] : 0.0f);
+    } else {
+      sums[i] = total;
+    }
+  }
+  if (plane_stride > 0 || parts == 1) return;
+  cw_lds_barrier();
+  for (int at = threadIdx.x; at < outputs; at += GT_BLOCK_WAVES * 64) {
+    const int n = n0 + (at & 15);
+    float total = sums[at];
+    for (int z = 1; z < parts; ++z) total += sums[z * outputs + at];
+    if (n < N) C[(int64_t)(at >> 4) * ldc + n] = total + (bias ? bias[n] : 0.0f);
   }
 }
 
@@ -465,6 +531,33 @@ static int launch_gemm_f32(const float* A, int64_t lda, const float* W, const fl
                            int N, int K, int splits, int per, bool planes, hipStream_t stream) {
   const bool vec = !(K & 3) && !(lda & 3);
   const int64_t stride = planes ? (int64_t)M * N : 0;
+  // Whole blocks of 16: the kernel whose waves share blocks. Without planes a workgroup takes all parts, with planes
+  // as many as make GT_BLOCKS blocks at most and leave a workgroup for every compute unit. (Not for outputs as wide as a
+  // vocabulary, which stream either way: 151936 x 896 with 16 rows 152 us the other way, 158 this.)
+  if (M <= GT_ROWS_MAX && !(K & 15) && !(lda & 3) && N <= 65536) {
+    const int part_blocks = per / 16, tiles = (N + 15) / 16;
+    int here = splits;
+    if (planes) {
+      const int most = GT_BLOCKS / part_blocks, spread = (int)((int64_t)splits * tiles / 256);
+      here = spread < most ? spread : most;
+      if (here < 1) here = 1;
+      if (here > splits) here = splits;
+    }
+    const int blocks = here * part_blocks < K / 16 ? here * part_blocks : K / 16;
+    if (blocks <= GT_BLOCKS) {
+      const size_t lds = (size_t)(blocks + (planes || splits == 1 ? 0 : splits)) * M * 16 * sizeof(float);
+      const dim3 grid(tiles, (splits + here - 1) / here);
+      static size_t raised = 48 * 1024;
+      if (lds > raised) {
+        if (hipFuncSetAttribute((const void*)gemm_f32_blocks_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+          return CW_ERR_LAUNCH;
+        raised = lds;
+      }
+      hipLaunchKernelGGL(gemm_f32_blocks_kernel, grid, dim3(GT_BLOCK_WAVES * 64), lds, stream, A, lda, W, bias, C, ldc, M, N, K, splits,
+                         part_blocks, here, stride);
+      return cw_launch_status();
+    }
+  }
   if (M <= GT_ROWS_MAX) {
     // as planes: four parts a block, each wave its own. Else all of a tile's parts in one block of up to
     // eight waves, and as many tiles as make it four waves or more.
