@@ -40,8 +40,9 @@ GRAPH_BATCH_SIZES = (1, 2, 4, 8, 16, 24, 32, 48, 64, 96, 128, 192, 256)
 GRAPH_KEY_BUCKET = 512
 # a step that is one request's portion replays a graph captured for the token budget or for the
 # next of these sizes (a step of 65 to 500 tokens is otherwise bound by the host's launches); what a
-# step is padded by is computed for nothing (137 tokens of the 1.5B shape: 2.62 ms as 256, 2.46 as 160)
-PORTION_GRAPH_SIZES = (16, 32, 64, 96, 128, 160, 192, 256, 384, 448, 512)
+# step is padded by is computed for nothing (137 tokens of the 1.5B shape: 2.62 ms as 256, 2.46 as 160; 300 beside 15
+# decoding requests: 3.55 ms as 384, 3.30 as 320). From 64 on the products' tiles are 64 rows high.
+PORTION_GRAPH_SIZES = (16, 32, 64, 96, 128, 160, 192, 256, 320, 384, 448, 512)
 # the rows that the narrow products take in one, two or four tiles of tokens: a step of single
 # tokens beside a short portion is padded to the next of these in all, if it fits one
 NARROW_STEP_ROWS = (16, 32, 64)
