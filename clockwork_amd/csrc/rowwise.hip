@@ -157,102 +157,88 @@ __global__ __launch_bounds__(256) void add_layernorm_kernel(float* __restrict__ 
   }
 }
 
-// The same for rows of a multiple of 4 elements, up to 1024 * KC: a thread holds its pieces of 4 in registers.
-// Bound for few rows by its trips to memory, which all start before any operand is used, and for many by the bytes,
-// which are read once (1536 elements, two gated branches pending: 8 rows 9.1 us -> 5.1, 2048 rows 20.4 -> 14.9).
-template <typename T, typename WT, typename BT, int KC>
-__global__ __launch_bounds__(256) void add_layernorm_vec_kernel(float* __restrict__ resid, GatedPair<T, BT> pend,
-                                                                const WT* __restrict__ weight, const WT* __restrict__ bias,
-                                                                float eps, T* __restrict__ out, const int* __restrict__ rows,
-                                                                int H) {
-  __shared__ float scratch[4];
-  const int i = blockIdx.x, n_chunks = H / 4;
+// The same for rows of a multiple of 4 elements, up to 4096: a thread holds one piece of 4 in registers, H / 4 threads,
+// rounded up to whole waves. Bound for few rows by its trips to memory, which all start before any operand is used,
+// and by its own code (two pieces a thread are 7.4 KB of it, one 4.5: 8 prompts of 200 and 16 steps of a four-layer model of
+// width 1536, 73 such norms, 8.47 -> 8.40 ms), and for many rows by the bytes, which are read once.
+template <typename T, typename WT, typename BT>
+__global__ __launch_bounds__(1024) void add_layernorm_row_kernel(float* __restrict__ resid, GatedPair<T, BT> pend,
+                                                                 const WT* __restrict__ weight, const WT* __restrict__ bias,
+                                                                 float eps, T* __restrict__ out, const int* __restrict__ rows,
+                                                                 int H) {
+  constexpr int PU = 4;  // planes on their way at a time
+  __shared__ float partial[2][16];
+  const int i = blockIdx.x, waves = blockDim.x >> 6;
   const int64_t t = rows ? rows[i] : i;
-  float* x = resid + t * H;
-  const bool has = pend.a != nullptr;
-  float v[KC][4], w[KC][4], c[KC][4], a[KC][4], b[KC][4], za[KC][4], zb[KC][4], ba[KC][4], bb[KC][4], planes[4][KC][4];
+  const bool in = (int)threadIdx.x < H / 4;
+  const int at = in ? threadIdx.x * 4 : 0;
+  float* const x = resid + t * H + at;
+  float v[4], w[4], c[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  CwVec<float, 4>::load(x, v);
+  if (pend.a) {
+    const int64_t from = t * H + at;
+    float a[4], b[4] = {0.0f, 0.0f, 0.0f, 0.0f}, z[2][4], zb[2][4], planes[PU][4];
+    CwVec<T, 4>::load(pend.a + from, a);
+    auto load_planes = [&](int q0) __attribute__((always_inline)) {
 #pragma unroll
-  for (int k = 0; k < KC; ++k) {
-    const int ch = threadIdx.x + k * 256;
+      for (int q = 0; q < PU; ++q)
+        if (q0 + q < pend.parts) CwVec<float, 4>::load((const float*)pend.b + (q0 + q) * pend.plane + from, planes[q]);
+    };
+    if (pend.parts > 0) load_planes(0);
+    else if (pend.b) CwVec<T, 4>::load((const T*)pend.b + from, b);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[k][e] = c[k][e] = b[k][e] = ba[k][e] = bb[k][e] = 0.0f;
-    if (ch < n_chunks) {
-      CwVec<float, 4>::load(x + ch * 4, v[k]);
-      CwVec<WT, 4>::load(weight + ch * 4, w[k]);
-      if (bias) CwVec<WT, 4>::load(bias + ch * 4, c[k]);
-      if (has) {
-        CwVec<T, 4>::load(pend.a + t * H + ch * 4, a[k]);
-        if (pend.b && pend.parts == 0) CwVec<T, 4>::load((const T*)pend.b + t * H + ch * 4, b[k]);
-        if (pend.parts > 0) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            if (q < pend.parts) CwVec<float, 4>::load((const float*)pend.b + q * pend.plane + t * H + ch * 4, planes[q][k]);
-        }
-        if (pend.z) {
-          CwVec<T, 4>::load(pend.z + t * pend.z_stride + ch * 4, za[k]);
-          if (pend.zb) CwVec<BT, 4>::load(pend.zb + ch * 4, ba[k]);
-          if (pend.b) {
-            CwVec<T, 4>::load(pend.z + t * pend.z_stride + H + ch * 4, zb[k]);
-            if (pend.zb) CwVec<BT, 4>::load(pend.zb + H + ch * 4, bb[k]);
-          }
-        }
+    for (int u = 0; u < 2; ++u)
+      if (pend.z && (u == 0 || pend.b)) {
+        CwVec<T, 4>::load(pend.z + t * pend.z_stride + u * H + at, z[u]);
+        if (pend.zb) CwVec<BT, 4>::load(pend.zb + u * H + at, zb[u]);
       }
-    }
-  }
-  for (int q0 = 0; q0 < pend.parts; q0 += 4) {  // in their order, four on their way at a time
+    CwVec<WT, 4>::load(weight + at, w);
+    if (bias) CwVec<WT, 4>::load(bias + at, c);
+    for (int q0 = 0; q0 < pend.parts; q0 += PU) {  // in their order
+      if (q0 > 0) load_planes(q0);
 #pragma unroll
-    for (int k = 0; k < KC; ++k) {
-      const int ch = threadIdx.x + k * 256;
-      if (ch >= n_chunks) continue;
-      if (q0 > 0) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (q0 + q < pend.parts) CwVec<float, 4>::load((const float*)pend.b + (q0 + q) * pend.plane + t * H + ch * 4, planes[q][k]);
-      }
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
+      for (int q = 0; q < PU; ++q)
         if (q0 + q < pend.parts)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) b[k][e] += planes[q][k][e];
+          for (int e = 0; e < 4; ++e) b[e] += planes[q][e];
     }
-  }
-  float s = 0.0f;
+    if (pend.z) {
 #pragma unroll
-  for (int k = 0; k < KC; ++k) {
-    const int ch = threadIdx.x + k * 256;
-    if (ch < n_chunks) {
-      if (has) {
+      for (int u = 0; u < 2; ++u)
+        if (u == 0 || pend.b)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if (pend.z) {
-            a[k][e] *= 1.0f / (1.0f + expf(-(za[k][e] + ba[k][e])));
-            if (pend.b) b[k][e] *= 1.0f / (1.0f + expf(-(zb[k][e] + bb[k][e])));
+          for (int e = 0; e < 4; ++e) {
+            float& of = u ? b[e] : a[e];
+            of *= 1.0f / (1.0f + expf(-(z[u][e] + (pend.zb ? zb[u][e] : 0.0f))));
           }
-          v[k][e] += a[k][e] + b[k][e];
-        }
-        if (!rows) CwVec<float, 4>::store(x + ch * 4, v[k]);
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s += v[k][e];
     }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += a[e] + b[e];
+    if (in && !rows) CwVec<float, 4>::store(x, v);
+  } else {
+    CwVec<WT, 4>::load(weight + at, w);
+    if (bias) CwVec<WT, 4>::load(bias + at, c);
   }
-  const float mean = block_sum_256(s, scratch) / (float)H;
+  auto row_sum = [&](float s, float* to) __attribute__((always_inline)) {
+    s = cw_wave_sum(in ? s : 0.0f);
+    if ((threadIdx.x & 63) == 0) to[threadIdx.x >> 6] = s;
+    cw_lds_barrier();
+    float total = 0.0f;
+    for (int k = 0; k < waves; ++k) total += to[k];
+    return total;
+  };
+  const float mean = row_sum((v[0] + v[1]) + (v[2] + v[3]), partial[0]) / (float)H;
   float ss = 0.0f;
 #pragma unroll
-  for (int k = 0; k < KC; ++k)
-    if ((int)threadIdx.x + k * 256 < n_chunks)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) ss += (v[k][e] - mean) * (v[k][e] - mean);
-  const float inv = 1.0f / sqrtf(block_sum_256(ss, scratch) / (float)H + eps);
-#pragma unroll
-  for (int k = 0; k < KC; ++k) {
-    const int ch = threadIdx.x + k * 256;
-    if (ch < n_chunks) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[k][e] = (v[k][e] - mean) * inv * w[k][e] + c[k][e];
-      CwVec<T, 4>::store(out + (int64_t)i * H + ch * 4, v[k]);
-    }
+  for (int e = 0; e < 4; ++e) {
+    v[e] -= mean;
+    ss += v[e] * v[e];
   }
+  const float inv = 1.0f / sqrtf(row_sum(ss, partial[1]) / (float)H + eps);
+  if (!in) return;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = v[e] * inv * w[e] + c[e];
+  CwVec<T, 4>::store(out + (int64_t)i * H + at, v);
 }
 
 // z/zb/a/b: the pending gated branches (all nullptr: none); z_cols: columns of z (H or 2H); b_parts > 0: b is that many
@@ -269,17 +255,14 @@ CW_EXPORT int cw_add_layernorm(float* resid, const void* z, const void* zb, int 
 #define CW_LAUNCH(T, WT, BT)                                                                               \
   do {                                                                                                     \
     GatedPair<T, BT> pend{(const T*)z, (const BT*)zb, (const T*)a, b, z_cols, b_parts, b_plane};           \
-    if (quads && H <= 2048)                                                                                \
-      hipLaunchKernelGGL((add_layernorm_vec_kernel<T, WT, BT, 2>), grid, block, 0, stream, resid, pend,    \
-                         (const WT*)weight, (const WT*)bias, eps, (T*)out, rows, H);                       \
-    else if (quads && H <= 4096)                                                                           \
-      hipLaunchKernelGGL((add_layernorm_vec_kernel<T, WT, BT, 4>), grid, block, 0, stream, resid, pend,    \
+    if (quads && H <= 4096)                                                                                \
+      hipLaunchKernelGGL((add_layernorm_row_kernel<T, WT, BT>), grid, dim3((H / 4 + 63) / 64 * 64), 0, stream, resid, pend, \
                          (const WT*)weight, (const WT*)bias, eps, (T*)out, rows, H);                       \
     else                                                                                                   \
       hipLaunchKernelGGL((add_layernorm_kernel<T, WT, BT>), grid, block, 0, stream, resid, pend,           \
                          (const WT*)weight, (const WT*)bias, eps, (T*)out, rows, H);                       \
   } while (0)
-  // rows of more than 4096 elements do not fit the registers of 256 threads with all that is pending
+  // (rows of more than 4096 elements are more than 1024 threads take a piece each of)
   const bool quads = rw_quads(H, resid, z, zb, a, b, weight, bias, out) && b_plane % 4 == 0;
   const int zbt = zb ? zb_dtype : w_dtype;
   if (dtype == CW_F32 && w_dtype == CW_F32 && zbt == CW_F32) CW_LAUNCH(float, float, float);

@@ -111,6 +111,13 @@ def test_layernorm_alone_and_with_gated_branches(dtype, width):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width", [4, 252, 256, 260, 1536, 4092, 4096, 4100])
+def test_layernorm_of_a_piece_a_thread(dtype, width):
+    """Rows around whole waves of pieces of 4 and around the longest row that 1024 threads take."""
+    test_layernorm_alone_and_with_gated_branches(dtype, width)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_embedding_with_scale_and_positions(dtype):
     part = build_part(PositionTableEmbeddingSpec(vocab_size=50, hidden_size=36, scale=2.5, max_positions=40))
     w = bind(part, dtype, matrix_std=1.0)
