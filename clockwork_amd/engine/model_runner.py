@@ -40,9 +40,11 @@ GRAPH_BATCH_SIZES = (1, 2, 4, 8, 16, 24, 32, 48, 64, 96, 128, 192, 256)
 GRAPH_KEY_BUCKET = 512
 # a step that is one request's portion replays a graph captured for the token budget or for the
 # next of these sizes (a step of 65 to 500 tokens is otherwise bound by the host's launches); what a
-# step is padded by is computed for nothing (137 tokens of the 1.5B shape: 2.62 ms as 256, 2.46 as 160; 300 beside 15
-# decoding requests: 3.55 ms as 384, 3.30 as 320). From 64 on the products' tiles are 64 rows high.
-PORTION_GRAPH_SIZES = (16, 32, 64, 96, 128, 160, 192, 256, 320, 384, 448, 512)
+# step is padded by is computed for nothing (137 tokens of the 1.5B shape: 2.62 ms as 256, 2.46 as 160)
+PORTION_GRAPH_SIZES = (16, 32, 64, 96, 128, 160, 192, 256, 384, 448, 512)
+# beside single tokens, where a step waits for a whole prompt's share of every product, one size more (300 tokens beside 15
+# decoding requests of the 1.5B shape: 3.55 ms as 384, 3.30 as 320)
+MIXED_PORTION_GRAPH_SIZES = (16, 32, 64, 96, 128, 160, 192, 256, 320, 384, 448, 512)
 # the rows that the narrow products take in one, two or four tiles of tokens: a step of single
 # tokens beside a short portion is padded to the next of these in all, if it fits one
 NARROW_STEP_ROWS = (16, 32, 64)
@@ -323,7 +325,7 @@ class ModelRunner:
         want = [int(w) for w in portion.want]
         decoders = next(b for b in GRAPH_BATCH_SIZES if b >= d)
         rows = next((t for t in NARROW_STEP_ROWS if decoders + n <= t), None)
-        size = rows - decoders if rows else next((b for b in PORTION_GRAPH_SIZES if b >= max(n, NARROW_STEP_ROWS[-1])), None)
+        size = rows - decoders if rows else next((b for b in MIXED_PORTION_GRAPH_SIZES if b >= max(n, NARROW_STEP_ROWS[-1])), None)
         limit = self._table_width * self.manager.block_size
         if size is None or want not in ([], [n - 1]) or portion.start + n > limit:
             return NotImplemented
