@@ -512,7 +512,7 @@ __device__ __forceinline__ bf16x8_t dec_to_operand(const bf16x8_t& v, int lane) 
 }
 
 template <int HD, bool POW2, int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void attn_decode_bf16_kernel(AttnParams p) {
+__device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int item, const int y, const int split) {
   constexpr int NF = HD / 32;  // 32-element steps over the head dimension
   constexpr int ND = HD / 16;  // 16-wide blocks of the head dimension
   extern __shared__ __align__(16) float dyn_s[];  // [waves][16 heads][HD] outputs, then this split's pages
@@ -523,9 +523,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_bf16_kernel(AttnParams
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane & 15, s = lane >> 4;
-  const int item = blockIdx.x;
-  const int kvh = blockIdx.y / p.n_chunks, chunk = blockIdx.y % p.n_chunks;
-  const int split = blockIdx.z;
+  const int kvh = y / p.n_chunks, chunk = y % p.n_chunks;
   // Every trip to memory that depends on an earlier one costs about a microsecond, which is what
   // a short context takes in all: with ``identity`` and fixed key ranges per split, the context
   // length, the table entries and the query are fetched side by side, then keys and values.
@@ -688,7 +686,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_bf16_kernel(AttnParams
   for (int db = 0; db < ND; ++db)
     *reinterpret_cast<f32x4_t*>(&o_s[(wave * 16 + c) * HD + db * 16 + 4 * s]) = o[db];
   __syncthreads();
-  const int64_t base = ((int64_t)item * gridDim.y + blockIdx.y) * p.n_splits + split;
+  const int64_t base = ((int64_t)item * (p.nkv * p.n_chunks) + y) * p.n_splits + split;
   for (int idx = threadIdx.x; idx < gh * HD; idx += WAVES * 64) {
     const int g = idx / HD, d = idx - g * HD;
     const int hg = chunk * gh + g;
@@ -715,6 +713,11 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_bf16_kernel(AttnParams
       }
     }
   }
+}
+
+template <int HD, bool POW2, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void attn_decode_bf16_kernel(AttnParams p) {
+  attn_decode_of<HD, POW2, WAVES>(p, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // Merge of the decode kernel's splits: one wave per (item, head, EL elements of the head). EL / 4 lanes take a split's
@@ -832,6 +835,19 @@ CW_EXPORT int64_t cw_attention_decode_workspace_floats(int n_items, int nh, int 
 }
 
 #if CW_HAS_DECODE
+static void launch_decode_merge(const AttnParams& p, int n_items, hipStream_t stream) {
+  constexpr int HD = CW_HD;
+  if (p.n_splits > 1) {
+    const dim3 heads(n_items, p.nkv * p.n_chunks, p.gh), pieces(heads.x, heads.y, heads.z * (HD / 32));
+    if (p.n_splits <= 8 * (256 / HD))  // whole heads while all splits come in one go
+      hipLaunchKernelGGL((attn_decode_merge_kernel<HD, HD, 1>), heads, dim3(64), 0, stream, p);
+    else if (p.n_splits <= 64)
+      hipLaunchKernelGGL((attn_decode_merge_kernel<HD, 32, 1>), pieces, dim3(64), 0, stream, p);
+    else
+      hipLaunchKernelGGL((attn_decode_merge_kernel<HD, 32, DEC_MAX_SPLITS / 64>), pieces, dim3(64), 0, stream, p);
+  }
+}
+
 template <bool POW2, int WAVES>
 static int launch_decode(AttnParams& p, int n_items, hipStream_t stream) {
   constexpr int HD = CW_HD;
@@ -850,16 +866,48 @@ static int launch_decode(AttnParams& p, int n_items, hipStream_t stream) {
   }
   dim3 grid(n_items, p.nkv * p.n_chunks, p.n_splits), block(WAVES * 64);
   hipLaunchKernelGGL((attn_decode_bf16_kernel<HD, POW2, WAVES>), grid, block, smem, stream, p);
-  if (p.n_splits > 1) {
-    const dim3 heads(n_items, p.nkv * p.n_chunks, p.gh), pieces(heads.x, heads.y, heads.z * (HD / 32));
-    if (p.n_splits <= 8 * (256 / HD))  // whole heads while all splits come in one go
-      hipLaunchKernelGGL((attn_decode_merge_kernel<HD, HD, 1>), heads, dim3(64), 0, stream, p);
-    else if (p.n_splits <= 64)
-      hipLaunchKernelGGL((attn_decode_merge_kernel<HD, 32, 1>), pieces, dim3(64), 0, stream, p);
-    else
-      hipLaunchKernelGGL((attn_decode_merge_kernel<HD, 32, DEC_MAX_SPLITS / 64>), pieces, dim3(64), 0, stream, p);
-  }
+  launch_decode_merge(p, n_items, stream);
   return cw_launch_status();
+}
+#endif
+
+#if CW_HAS_DECODE
+// The decode kernel's parameters from its entry points' arguments, checked.
+static int decode_params(AttnParams& p, const void* q, int64_t q_stride, void* out, int64_t out_stride,
+                                       const void* k_cache, const void* v_cache, const int* block_tables,
+                                       int table_stride, const int* ctx_lens, const int* cu_q,
+                                       const int* items, int n_items, int nh, int nkv, int block_size,
+                                       int n_splits, int window, float scale, float* workspace,
+                                       int64_t workspace_floats, const void* zeros, int identity,
+                                       int split_keys, int max_ctx, float softcap, const void* gate, int64_t gate_stride,
+                                       int gate_off) {
+  if (n_items < 0 || nh <= 0 || nkv <= 0 || nh % nkv != 0 || block_size <= 0 || table_stride <= 0)
+    return CW_ERR_ARG;
+  if (n_splits < 1 || n_splits > DEC_MAX_SPLITS || window < 0) return CW_ERR_ARG;
+  if (((uintptr_t)q & 15) || ((uintptr_t)k_cache & 15) || ((uintptr_t)v_cache & 15) || (q_stride & 7))
+    return CW_ERR_ARG;
+  if (zeros == nullptr || ((uintptr_t)zeros & 15)) return CW_ERR_ARG;
+  // fixed key ranges must cover the longest context the caller will run
+  if (split_keys < 0 || (split_keys & 31) || max_ctx < 0) return CW_ERR_ARG;
+  if (split_keys > 0 && (int64_t)split_keys * n_splits < max_ctx) return CW_ERR_ARG;
+  const int group = nh / nkv;
+  p.q = q; p.q_stride = q_stride; p.out = out; p.out_stride = out_stride;
+  p.k_cache = k_cache; p.v_cache = v_cache; p.block_tables = block_tables;
+  p.table_stride = table_stride; p.ctx_lens = ctx_lens; p.cu_q = cu_q; p.items = items;
+  p.nh = nh; p.nkv = nkv; p.block_size = block_size; p.bs_shift = cw_log2_or_minus1(block_size);
+  p.identity = identity ? 1 : 0; p.split_keys = split_keys;
+  if (gate && (gate_off < 0 || gate_off + nh > gate_stride)) return CW_ERR_ARG;
+  p.gate = gate; p.gate_stride = gate_stride; p.gate_off = gate_off;
+  p.gh = cw_attention_decode_gh(group);
+  p.n_chunks = (group + p.gh - 1) / p.gh; p.n_splits = n_splits; p.window = window; p.scale = scale; p.softcap = softcap;
+  if ((int64_t)nkv * p.n_chunks * p.gh > 65535) return CW_ERR_SIZE;
+  const int64_t need = cw_attention_decode_workspace_floats(n_items, nh, nkv, n_splits);
+  if (need > 0 && (workspace == nullptr || workspace_floats < need)) return CW_ERR_ARG;
+  if ((uintptr_t)workspace & 7) return CW_ERR_ARG;
+  p.part_o = workspace;
+  p.part_ml = workspace ? workspace + need / (CW_HD + 2) * CW_HD : nullptr;
+  p.zeros = zeros;
+  return CW_OK;
 }
 #endif
 
@@ -878,34 +926,9 @@ CW_EXPORT int cw_attention_decode_bf16(const void* q, int64_t q_stride, void* ou
                                        int split_keys, int max_ctx, float softcap, const void* gate, int64_t gate_stride,
                                        int gate_off, hipStream_t stream) {
 #if CW_HAS_DECODE
-  if (n_items < 0 || nh <= 0 || nkv <= 0 || nh % nkv != 0 || block_size <= 0 || table_stride <= 0)
-    return CW_ERR_ARG;
-  if (n_splits < 1 || n_splits > DEC_MAX_SPLITS || window < 0) return CW_ERR_ARG;
-  if (((uintptr_t)q & 15) || ((uintptr_t)k_cache & 15) || ((uintptr_t)v_cache & 15) || (q_stride & 7))
-    return CW_ERR_ARG;
-  if (zeros == nullptr || ((uintptr_t)zeros & 15)) return CW_ERR_ARG;
-  // fixed key ranges must cover the longest context the caller will run
-  if (split_keys < 0 || (split_keys & 31) || max_ctx < 0) return CW_ERR_ARG;
-  if (split_keys > 0 && (int64_t)split_keys * n_splits < max_ctx) return CW_ERR_ARG;
-  if (n_items == 0) return CW_OK;
-  const int group = nh / nkv;
   AttnParams p{};
-  p.q = q; p.q_stride = q_stride; p.out = out; p.out_stride = out_stride;
-  p.k_cache = k_cache; p.v_cache = v_cache; p.block_tables = block_tables;
-  p.table_stride = table_stride; p.ctx_lens = ctx_lens; p.cu_q = cu_q; p.items = items;
-  p.nh = nh; p.nkv = nkv; p.block_size = block_size; p.bs_shift = cw_log2_or_minus1(block_size);
-  p.identity = identity ? 1 : 0; p.split_keys = split_keys;
-  if (gate && (gate_off < 0 || gate_off + nh > gate_stride)) return CW_ERR_ARG;
-  p.gate = gate; p.gate_stride = gate_stride; p.gate_off = gate_off;
-  p.gh = cw_attention_decode_gh(group);
-  p.n_chunks = (group + p.gh - 1) / p.gh; p.n_splits = n_splits; p.window = window; p.scale = scale; p.softcap = softcap;
-  if ((int64_t)nkv * p.n_chunks * p.gh > 65535) return CW_ERR_SIZE;
-  const int64_t need = cw_attention_decode_workspace_floats(n_items, nh, nkv, n_splits);
-  if (need > 0 && (workspace == nullptr || workspace_floats < need)) return CW_ERR_ARG;
-  if ((uintptr_t)workspace & 7) return CW_ERR_ARG;
-  p.part_o = workspace;
-  p.part_ml = workspace ? workspace + need / (CW_HD + 2) * CW_HD : nullptr;
-  p.zeros = zeros;
+  const int status = decode_params(p, q, q_stride, out, out_stride, k_cache, v_cache, block_tables, table_stride, ctx_lens, cu_q, items, n_items, nh, nkv, block_size, n_splits, window, scale, workspace, workspace_floats, zeros, identity, split_keys, max_ctx, softcap, gate, gate_stride, gate_off);
+  if (status != CW_OK || n_items == 0) return status;
   // what a split's keys are shared among: the most keys a split may have, by the caller's fixed places or by its table
   const int64_t keys = split_keys > 0 ? split_keys : ((int64_t)table_stride * block_size + n_splits - 1) / n_splits;
   // more than four waves can have on their way at once: eight (2049 keys of 128 elements in one workgroup: 30 us
@@ -999,7 +1022,7 @@ __device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, v
 
 // PAGES16: a page holds 2^n keys, 16 or more, so that 16 keys of a stage lie in one page
 template <int HD, bool PAGES16, int RB, bool CAP>
-__global__ __launch_bounds__((PrefillTile<HD, RB>::NT), (HD <= 128 ? 2 : 1)) void attn_prefill_bf16_kernel(AttnParams p) {
+__device__ __forceinline__ void attn_prefill_of(const AttnParams& p, const int item, const int y) {
   using Tile = PrefillTile<HD, RB>;
   constexpr int NF = HD / 32;     // k-steps of the score product, blocks of 32 elements of a row
   constexpr int ND = HD / 16;     // 16-wide blocks of the head dimension
@@ -1012,8 +1035,7 @@ __global__ __launch_bounds__((PrefillTile<HD, RB>::NT), (HD <= 128 ? 2 : 1)) voi
   const int wave = wid % RB;  // the wave's row block
   const int half = wid / RB;  // its share of a stage's keys
   const int c = lane & 15, s = lane >> 4;
-  const int item = blockIdx.x;
-  const int kvh = blockIdx.y / p.n_chunks, chunk = blockIdx.y % p.n_chunks;
+  const int kvh = y / p.n_chunks, chunk = y % p.n_chunks;
   const int req = p.items[4 * item], tok0 = p.items[4 * item + 1];
   const int gh = p.gh;
   const int tpw = 32 / gh;  // tokens of a wave
@@ -1346,7 +1368,7 @@ __global__ __launch_bounds__((PrefillTile<HD, RB>::NT), (HD <= 128 ? 2 : 1)) voi
   // ---- a part of the key range: unnormalised sums, maximum and sum of every row of the workgroup
   // (unused rows too: zeros) for the merge kernel
   if (parts > 1) {
-    const int64_t slot = ((int64_t)item * gridDim.y + blockIdx.y) * (RB * 32);
+    const int64_t slot = ((int64_t)item * (p.nkv * p.n_chunks) + y) * (RB * 32);
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
       const float l = cw_quad_sum(l_run[b]);
@@ -1380,6 +1402,35 @@ __global__ __launch_bounds__((PrefillTile<HD, RB>::NT), (HD <= 128 ? 2 : 1)) voi
     }
   }
 }
+
+template <int HD, bool PAGES16, int RB, bool CAP>
+__global__ __launch_bounds__((PrefillTile<HD, RB>::NT), (HD <= 128 ? 2 : 1)) void attn_prefill_bf16_kernel(AttnParams p) {
+  attn_prefill_of<HD, PAGES16, RB, CAP>(p, blockIdx.x, blockIdx.y);
+}
+
+#if CW_HD % 32 == 0 && CW_HD <= 128
+// A step's portions and its single tokens in one launch: the first workgroups take the portions' items, the others the single
+// tokens' splits, eight waves each. One workgroup fits a compute unit, and each launch by itself is bound by its longest
+// workgroup's chain of trips to memory: 320 tokens beside 16 requests of 1500 (12 heads of 128 on 2) are 64 workgroups
+// and then 256 of some 10 us each; together, 64 and 192, they take little longer than the longer ones (28 layers: 3.30 -> 3.04 ms).
+struct AttnBoth {
+  AttnParams portions, singles;
+  int n_portions, n_singles;  // items of each
+};
+template <int HD, bool PAGES16, int RB>
+__global__ __launch_bounds__((PrefillTile<HD, RB>::NT), 2) void attn_together_bf16_kernel(AttnBoth a) {
+  static_assert(PrefillTile<HD, RB>::NT == 512, "both kinds of workgroups have eight waves");
+  const int first = a.n_portions * a.portions.nkv * a.portions.n_chunks;
+  int b = blockIdx.x;
+  if (b < first) {
+    attn_prefill_of<HD, PAGES16, RB, false>(a.portions, b % a.n_portions, b / a.n_portions);
+  } else {
+    b -= first;
+    const int of = b / a.n_singles, heads = a.singles.nkv * a.singles.n_chunks;
+    attn_decode_of<HD, PAGES16, 8>(a.singles, b - of * a.n_singles, of % heads, of / heads);
+  }
+}
+#endif
 
 // Puts together the parts of items whose key range was shared among workgroups. Four workgroups per (item, key/value
 // head) of the kernel above (with one a thread had eight rounds of loads: 1000 tokens behind 7000, 14 -> 6 us). The
@@ -1504,6 +1555,42 @@ CW_EXPORT int cw_attention_prefill_row_blocks_ok(int row_blocks) {
   return CW_HAS_PREFILL && (row_blocks == 4 || (row_blocks == 2 && CW_HD <= 128)) ? 1 : 0;
 }
 
+#if CW_HAS_PREFILL
+// The parameters of the kernel for portions from its entry points' arguments, checked.
+static int prefill_params(AttnParams& p, const void* q, int64_t q_stride, void* out, int64_t out_stride,
+                                        const void* k_cache, const void* v_cache, const int* block_tables,
+                                        int table_stride, const int* ctx_lens, const int* cu_q,
+                                        const int* items, int n_items, int nh, int nkv, int block_size,
+                                        int window, float scale, const void* zeros, int row_blocks,
+                                        int with_parts, float* workspace, int64_t workspace_floats,
+                                        float softcap, const void* gate, int64_t gate_stride, int gate_off) {
+  if (zeros == nullptr || ((uintptr_t)zeros & 15)) return CW_ERR_ARG;
+  if (n_items < 0 || nh <= 0 || nkv <= 0 || nh % nkv != 0 || block_size <= 0 || table_stride <= 0 || window < 0)
+    return CW_ERR_ARG;
+  if (!cw_attention_prefill_row_blocks_ok(row_blocks)) return CW_ERR_ARG;
+  if (((uintptr_t)q & 15) || ((uintptr_t)k_cache & 15) || ((uintptr_t)v_cache & 15) || ((uintptr_t)out & 7) ||
+      (q_stride & 7) || (out_stride & 3))
+    return CW_ERR_ARG;
+  const int group = nh / nkv;
+  p.q = q; p.q_stride = q_stride; p.out = out; p.out_stride = out_stride;
+  p.k_cache = k_cache; p.v_cache = v_cache; p.block_tables = block_tables;
+  p.table_stride = table_stride; p.ctx_lens = ctx_lens; p.cu_q = cu_q; p.items = items;
+  p.nh = nh; p.nkv = nkv; p.block_size = block_size; p.bs_shift = cw_log2_or_minus1(block_size); p.gh = group < 32 ? group : 32;
+  p.n_chunks = (group + p.gh - 1) / p.gh; p.n_splits = 1; p.window = window; p.scale = scale; p.softcap = softcap;
+  p.part_o = nullptr; p.part_ml = nullptr; p.zeros = zeros;
+  if (gate && (gate_off < 0 || gate_off + nh > gate_stride)) return CW_ERR_ARG;
+  p.gate = gate; p.gate_stride = gate_stride; p.gate_off = gate_off;
+  if ((int64_t)nkv * p.n_chunks > 65535) return CW_ERR_SIZE;
+  if (with_parts) {
+    const int64_t need = cw_attention_prefill_workspace_floats(n_items, nh, nkv, row_blocks);
+    if (workspace == nullptr || workspace_floats < need || ((uintptr_t)workspace & 15)) return CW_ERR_ARG;
+    p.part_o = workspace;
+    p.part_ml = workspace + need / (CW_HD + 2) * CW_HD;
+  }
+  return CW_OK;
+}
+#endif
+
 // Portions of prompts, bfloat16. items: (request, first token, tokens, part | parts << 8) with
 // tokens <= row_blocks * (32 / gh), gh = min(group, 32) heads of a group per workgroup; tokens of
 // an item beyond that are not computed. row_blocks: 4, or 2 (see PrefillTile). An item with
@@ -1520,31 +1607,9 @@ CW_EXPORT int cw_attention_prefill_bf16(const void* q, int64_t q_stride, void* o
                                         float softcap, const void* gate, int64_t gate_stride, int gate_off,
                                         hipStream_t stream) {
 #if CW_HAS_PREFILL
-  if (zeros == nullptr || ((uintptr_t)zeros & 15)) return CW_ERR_ARG;
-  if (n_items < 0 || nh <= 0 || nkv <= 0 || nh % nkv != 0 || block_size <= 0 || table_stride <= 0 || window < 0)
-    return CW_ERR_ARG;
-  if (!cw_attention_prefill_row_blocks_ok(row_blocks)) return CW_ERR_ARG;
-  if (((uintptr_t)q & 15) || ((uintptr_t)k_cache & 15) || ((uintptr_t)v_cache & 15) || ((uintptr_t)out & 7) ||
-      (q_stride & 7) || (out_stride & 3))
-    return CW_ERR_ARG;
-  if (n_items == 0) return CW_OK;
-  const int group = nh / nkv;
   AttnParams p{};
-  p.q = q; p.q_stride = q_stride; p.out = out; p.out_stride = out_stride;
-  p.k_cache = k_cache; p.v_cache = v_cache; p.block_tables = block_tables;
-  p.table_stride = table_stride; p.ctx_lens = ctx_lens; p.cu_q = cu_q; p.items = items;
-  p.nh = nh; p.nkv = nkv; p.block_size = block_size; p.bs_shift = cw_log2_or_minus1(block_size); p.gh = group < 32 ? group : 32;
-  p.n_chunks = (group + p.gh - 1) / p.gh; p.n_splits = 1; p.window = window; p.scale = scale; p.softcap = softcap;
-  p.part_o = nullptr; p.part_ml = nullptr; p.zeros = zeros;
-  if (gate && (gate_off < 0 || gate_off + nh > gate_stride)) return CW_ERR_ARG;
-  p.gate = gate; p.gate_stride = gate_stride; p.gate_off = gate_off;
-  if ((int64_t)nkv * p.n_chunks > 65535) return CW_ERR_SIZE;
-  if (with_parts) {
-    const int64_t need = cw_attention_prefill_workspace_floats(n_items, nh, nkv, row_blocks);
-    if (workspace == nullptr || workspace_floats < need || ((uintptr_t)workspace & 15)) return CW_ERR_ARG;
-    p.part_o = workspace;
-    p.part_ml = workspace + need / (CW_HD + 2) * CW_HD;
-  }
+  const int status = prefill_params(p, q, q_stride, out, out_stride, k_cache, v_cache, block_tables, table_stride, ctx_lens, cu_q, items, n_items, nh, nkv, block_size, window, scale, zeros, row_blocks, with_parts, workspace, workspace_floats, softcap, gate, gate_stride, gate_off);
+  if (status != CW_OK || n_items == 0) return status;
   const bool cap = softcap > 0.0f;
   auto launch = [&](auto rb) {
     constexpr int RB = decltype(rb)::value;
@@ -1555,6 +1620,62 @@ CW_EXPORT int cw_attention_prefill_bf16(const void* q, int64_t q_stride, void* o
   if (row_blocks == 2) return launch(std::integral_constant<int, 2>{});
 #endif
   return launch(std::integral_constant<int, 4>{});
+#else
+  return CW_ERR_ARG;
+#endif
+}
+
+// 1 if portions and single tokens of one step can run as one launch (see attn_together_bf16_kernel).
+CW_EXPORT int cw_attention_together_supported() { return CW_HAS_PREFILL && CW_HD <= 128 ? 1 : 0; }
+
+// cw_attention_prefill_bf16 of ``portions`` (whole items, no parts) and cw_attention_decode_bf16 of ``singles`` in one
+// launch, then the merge of the single tokens' splits; the arguments are theirs.
+CW_EXPORT int cw_attention_together_bf16(const void* q, int64_t q_stride, void* out, int64_t out_stride, const void* k_cache,
+                                         const void* v_cache, const int* block_tables, int table_stride, const int* ctx_lens,
+                                         const int* cu_q, const int* portions, int n_portions, int row_blocks, const int* singles,
+                                         int n_singles, int n_splits, int split_keys, int max_ctx, int nh, int nkv,
+                                         int block_size, int window, float scale, float* workspace, int64_t workspace_floats,
+                                         const void* zeros, hipStream_t stream) {
+#if CW_HAS_PREFILL && CW_HD <= 128
+  AttnBoth a{};
+  int status = prefill_params(a.portions, q, q_stride, out, out_stride, k_cache, v_cache, block_tables, table_stride, ctx_lens, cu_q,
+                              portions, n_portions, nh, nkv, block_size, window, scale, zeros, row_blocks, 0, nullptr, 0, 0.0f,
+                              nullptr, 0, 0);
+  if (status != CW_OK) return status;
+  status = decode_params(a.singles, q, q_stride, out, out_stride, k_cache, v_cache, block_tables, table_stride, ctx_lens, cu_q,
+                         singles, n_singles, nh, nkv, block_size, n_splits, window, scale, workspace, workspace_floats, zeros, 0,
+                         split_keys, max_ctx, 0.0f, nullptr, 0, 0);
+  if (status != CW_OK) return status;
+  if (n_portions == 0 || n_singles == 0) return CW_ERR_ARG;
+  a.n_portions = n_portions; a.n_singles = n_singles;
+  const int64_t groups = (int64_t)n_portions * nkv * a.portions.n_chunks + (int64_t)n_singles * nkv * a.singles.n_chunks * n_splits;
+  if (groups > 0x7fffffff) return CW_ERR_SIZE;
+  // LDS: the portions' tiles, or the single tokens' outputs and the pages of a split
+  const int64_t max_tiles = ((int64_t)table_stride * block_size + 31) / 32;
+  const int64_t tiles_per_split = split_keys > 0 ? split_keys / 32 : (max_tiles + n_splits - 1) / n_splits;
+  const int64_t pages = (tiles_per_split * 32 + block_size - 1) / block_size + 2;
+  const size_t for_singles = sizeof(float) * 8 * 16 * CW_HD + sizeof(int) * (size_t)pages;
+  auto launch = [&](auto rb, auto pages16) {
+    constexpr int RB = decltype(rb)::value;
+    constexpr bool P16 = decltype(pages16)::value;
+    const size_t smem = for_singles > PrefillTile<CW_HD, RB>::BYTES ? for_singles : PrefillTile<CW_HD, RB>::BYTES;
+    if (smem > 156 * 1024) return CW_ERR_SIZE;  // (beside the single tokens' statistics)
+    static size_t raised = 0;
+    if (smem > raised) {
+      if (hipFuncSetAttribute((const void*)attn_together_bf16_kernel<CW_HD, P16, RB>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)smem) != hipSuccess)
+        return CW_ERR_LAUNCH;
+      raised = smem;
+    }
+    hipLaunchKernelGGL((attn_together_bf16_kernel<CW_HD, P16, RB>), dim3((unsigned)groups), dim3(512), smem, stream, a);
+    launch_decode_merge(a.singles, n_singles, stream);
+    return cw_launch_status();
+  };
+  using Two = std::integral_constant<int, 2>;
+  using Four = std::integral_constant<int, 4>;
+  if (a.portions.bs_shift >= 4)
+    return row_blocks == 2 ? launch(Two{}, std::true_type{}) : launch(Four{}, std::true_type{});
+  return row_blocks == 2 ? launch(Two{}, std::false_type{}) : launch(Four{}, std::false_type{});
 #else
   return CW_ERR_ARG;
 #endif

@@ -239,6 +239,8 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_attention_prefill_supported": [],
             "cw_attention_prefill_bf16": [P, L, P, L, P, P, P, I, P, P, P, I, I, I, I, I, F, P, I, I, P, L, F, P, L, I, P],
             "cw_attention_prefill_workspace_floats": [I, I, I, I],
+            "cw_attention_together_supported": [],
+            "cw_attention_together_bf16": [P, L, P, L, P, P, P, I, P, P, P, I, I, P, I, I, I, I, I, I, I, I, F, P, L, P, P],
             "cw_attention_prefill_row_blocks_ok": [I],
             "cw_attention_decode_supported": [],
             "cw_attention_decode_gh": [I],
@@ -1357,6 +1359,55 @@ def attention_decode(q, q_stride: int, out, k_cache, v_cache, block_tables, ctx_
             window, float(scale), _ptr(workspace), ws_floats, _zero_row(out.device), int(bool(identity)),
             int(split_keys), int(max_ctx), float(softcap), *_head_gate(head_gate, n_tokens, nh), _stream()),
         "attention_decode_bf16",
+    )
+
+
+def together_attention_supported(hd: int, dtype: torch.dtype) -> bool:
+    return dtype == torch.bfloat16 and bool(_load("attention", hd).cw_attention_together_supported())
+
+
+def attention_together(q, q_stride: int, out, k_cache, v_cache, block_tables, ctx_lens, cu_q, portions, n_portions: int,
+                       row_blocks: int, singles, n_singles: int, n_splits: int, split_keys: int, max_ctx: int, nh: int, nkv: int,
+                       hd: int, block_size: int, window: int, scale: float, n_tokens: int, n_requests: int,
+                       workspace=None) -> None:
+    """``attention_prefill`` of the items ``portions`` (no parts) and ``attention_decode`` of ``singles`` in one launch;
+    arguments as for these."""
+    if not prefill_row_blocks_ok(hd, row_blocks):
+        raise KernelError(f"the kernel for head size {hd} does not take {row_blocks} row blocks")
+    _gpu(k_cache, v_cache, block_tables, ctx_lens, cu_q, portions, singles, workspace)
+    out_stride = _gpu_rows(out)
+    if not (q.is_cuda and q.dtype == out.dtype == k_cache.dtype == v_cache.dtype == torch.bfloat16):
+        raise KernelError("the kernel is bfloat16")
+    if not (out.dim() == 2 and out.shape[0] >= n_tokens and out.shape[1] == nh * hd):
+        raise KernelError("attention output must be [T, nh * hd]")
+    if not (q_stride >= nh * hd):
+        raise KernelError("query rows overlap")
+    if not (block_tables.dtype == torch.int32 and block_tables.dim() == 2 and block_tables.shape[0] >= n_requests):
+        raise KernelError("block_tables must be int32 [R, max_blocks]")
+    _i32(ctx_lens, n_requests, "ctx_lens")
+    _i32(cu_q, n_requests + 1, "cu_q")
+    for items, n in ((portions, n_portions), (singles, n_singles)):
+        if not (items.dtype == torch.int32 and items.numel() >= 4 * n > 0):
+            raise KernelError("items must be int32 [n_items, 4], of both kinds")
+    if not (tuple(k_cache.shape[-2:]) == (nkv, hd) and k_cache.shape == v_cache.shape):
+        raise KernelError("cache must be [..., nkv, hd]")
+    if split_keys:
+        if not (split_keys % 32 == 0 and split_keys * n_splits >= max_ctx > 0):
+            raise KernelError("fixed key ranges do not cover the longest context")
+    lib = _load("attention", hd)
+    need = lib.cw_attention_decode_workspace_floats(n_singles, nh, nkv, n_splits)
+    ws_floats = 0
+    if need > 0:
+        _need(workspace is not None and workspace.dtype == torch.float32 and workspace.numel() >= need,
+              f"decode attention needs a float32 workspace of {need} elements")
+        ws_floats = workspace.numel()
+    _check(
+        lib.cw_attention_together_bf16(
+            q.data_ptr(), int(q_stride), _ptr(out), out_stride, _ptr(k_cache), _ptr(v_cache), _ptr(block_tables),
+            block_tables.shape[1], _ptr(ctx_lens), _ptr(cu_q), _ptr(portions), n_portions, int(row_blocks), _ptr(singles),
+            n_singles, n_splits, int(split_keys), int(max_ctx), nh, nkv, block_size, window, float(scale), _ptr(workspace),
+            ws_floats, _zero_row(out.device), _stream()),
+        "attention_together_bf16",
     )
 
 

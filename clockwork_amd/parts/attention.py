@@ -46,6 +46,7 @@ class AttentionPlan:
     decode_split_keys: int = 0    # keys of each of those splits, at fixed places (a multiple of 32)
     decode_max_ctx: int = 0       # the longest context the fixed places were planned for
     single_identity: bool = False  # a batch of single tokens only: item i is request i, token row i
+    together: bool = False        # the matrix-core kernels' portions and single tokens go as one launch
 
 
 # a portion's key ranges count as long when its tokens see this many keys or more on average
@@ -103,18 +104,30 @@ def _share_long_key_ranges(items: np.ndarray, ctx, workgroups_per_item: int):
     return out.astype(np.int32).reshape(-1), most
 
 
-def attention_plan(ctx, nh: int, nkv: int, narrow_ok: bool = False, whole_keys: int = 0) -> AttentionPlan:
+def attention_plan(ctx, nh: int, nkv: int, narrow_ok: bool = False, whole_keys: int = 0, together_ok: bool = False) -> AttentionPlan:
     """The step's work items for heads of this geometry, made once a step and kept in
     ``ctx.plans``. ``narrow_ok``: the matrix-core kernel for portions also comes with two row
     blocks a workgroup (see ``ops.prefill_row_blocks_ok``). ``whole_keys``: up to this many keys of a single
-    token stay with one workgroup (see ``whole_single_keys``)."""
+    token stay with one workgroup (see ``whole_single_keys``). ``together_ok``: the caller can run portions and single
+    tokens as one launch (see ``_share_the_card``)."""
     # a batch of single tokens has no portions: one plan, whatever the kernel for portions offers
     narrow_ok = bool(narrow_ok) and any(q > 1 for q in ctx.h_q_lens)
-    key = ("attention", nh, nkv, narrow_ok, whole_keys)
+    key = ("attention", nh, nkv, narrow_ok, whole_keys, together_ok)
     plan = ctx.plans.get(key)
     if plan is None:
-        plan = ctx.plans[key] = _make_plan(ctx, nh, nkv, narrow_ok, whole_keys)
+        plan = ctx.plans[key] = _make_plan(ctx, nh, nkv, narrow_ok, whole_keys, together_ok)
     return plan
+
+
+def _share_the_card(plan: AttentionPlan, room: int, base: int) -> None:
+    """One launch for a step's portions and single tokens, where all workgroups of both are at work at once: ``room``
+    compute units are left beside the portions' workgroups, a split of every single token takes ``base`` of them. The splits
+    are then as many as fit, but not fewer than half of those that the single tokens alone would be cut into: where the
+    portions take nearly the whole card, a few long splits would outlast both launches (a step of 15
+    requests of 1500 keys beside 300 tokens, 1.5B shape: 3.30 ms with 8 splits behind the portions, 3.04 with 6 beside them)."""
+    splits = min(room // base, plan.decode_splits)
+    if splits >= 1 and 2 * splits >= plan.decode_splits:
+        plan.together, plan.decode_splits = True, splits
 
 
 def whole_single_keys(head_dim: int) -> int:
@@ -124,7 +137,7 @@ def whole_single_keys(head_dim: int) -> int:
     return 512 if head_dim <= 128 else 0
 
 
-def _make_plan(ctx, nh: int, nkv: int, narrow_ok: bool, whole_keys: int = 0) -> AttentionPlan:
+def _make_plan(ctx, nh: int, nkv: int, narrow_ok: bool, whole_keys: int = 0, together_ok: bool = False) -> AttentionPlan:
     group = nh // nkv
     gh_wide = min(group, 64)
     tokens_per_tile = 64 // gh_wide
@@ -192,6 +205,8 @@ def _make_plan(ctx, nh: int, nkv: int, narrow_ok: bool, whole_keys: int = 0) -> 
         base = plan.n_single * nkv * -(-group // min(group, 16))
         plan.decode_splits = 1 if longest_single <= whole_keys else max(
             1, min(ctx.num_compute_units // base, longest_single // 128, 64))
+        if together_ok and plan.n_mfma and plan.mfma_parts == 1:
+            _share_the_card(plan, ctx.num_compute_units - plan.n_mfma * nkv * -(-group // 32), base)
         # fixed places for the splits: a workgroup then knows its pages before it knows the
         # request's length, which saves it a trip to memory
         plan.decode_split_keys = 32 * -(-(-(-longest_single // plan.decode_splits)) // 32)
@@ -236,7 +251,7 @@ class PagedAttention(Part):
         hd = self.spec.head_dim
         narrow_ok = ops.prefill_attention_supported(hd, dtype) and ops.prefill_row_blocks_ok(hd, 2)
         return attention_plan(ctx, self.spec.num_heads, self.spec.num_kv_heads, narrow_ok=narrow_ok,
-                              whole_keys=whole_single_keys(hd))
+                              whole_keys=whole_single_keys(hd), together_ok=ops.together_attention_supported(hd, dtype))
 
     def prepare(self, ctx) -> None:
         """The step's work items, before ``forward`` (a captured step must not make them)."""
@@ -296,6 +311,15 @@ class PagedAttention(Part):
             nh=nh, nkv=nkv, hd=hd, block_size=cache.block_size, window=s.window or 0,
             scale=s.scale, n_tokens=T, n_requests=ctx.num_requests,
         )
+        if plan.together:
+            workspace = None
+            if plan.decode_splits > 1:
+                need = ops.decode_attention_workspace_floats(hd, plan.n_single, nh, nkv, plan.decode_splits)
+                workspace = torch.empty(need, dtype=torch.float32, device=q.device)
+            ops.attention_together(portions=plan.mfma_items, n_portions=plan.n_mfma, row_blocks=plan.mfma_row_blocks,
+                                   singles=plan.single_items, n_singles=plan.n_single, n_splits=plan.decode_splits,
+                                   split_keys=plan.decode_split_keys, max_ctx=plan.decode_max_ctx, workspace=workspace, **common)
+            return out
         if plan.n_wide and mfma:
             workspace = None
             if plan.mfma_parts > 1:

@@ -1125,6 +1125,81 @@ def test_prefill_attention_kernel_with_shared_key_ranges(nh, nkv, hd, bs, window
         at += q_len
 
 
+@pytest.mark.parametrize("nh,nkv,hd,bs", [(12, 2, 128, 16), (14, 2, 64, 8), (40, 1, 64, 16), (3, 3, 96, 24), (4, 2, 32, 1)])
+@pytest.mark.parametrize("window", [0, 70])
+@pytest.mark.parametrize("row_blocks", [4, 2])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_portions_and_single_tokens_in_one_launch(nh, nkv, hd, bs, window, row_blocks, splits):
+    """The same results as the two launches give, bit for bit, and nothing written past the batch: portions of 2 to 150
+    tokens and single tokens of 1 to 1100 keys, in any order, splits at fixed places and (a split of 0 keys) by length."""
+    from clockwork_amd import ops
+
+    ctx_lens = [21, 1, 150, 700, 2, 1100, 333]
+    q_lens = [6, 1, 150, 1, 2, 1, 40]
+    tables, at = [], 0
+    perm = torch.randperm(sum(-(-c // bs) for c in ctx_lens) + 3).tolist()
+    for c in ctx_lens:
+        tables.append(perm[at : at + -(-c // bs)])
+        at += -(-c // bs)
+    kc, vc, _, _ = _paged_setup(torch.bfloat16, nkv, hd, bs, len(perm), tables, ctx_lens, poison=float("nan"))
+    width = max(len(t) for t in tables)
+    bt = torch.tensor([t + [-1] * (width - len(t)) for t in tables], dtype=torch.int32, device=DEV)
+    cl = torch.tensor(ctx_lens, dtype=torch.int32, device=DEV)
+    cu = torch.tensor([0] + list(torch.tensor(q_lens).cumsum(0)), dtype=torch.int32, device=DEV)
+    T, step = sum(q_lens), ops.prefill_tokens_per_item(nh // nkv, row_blocks)
+    portions = [[r, t, min(step, q - t), 0] for r, q in enumerate(q_lens) if q > 1 for t in range(0, q, step)]
+    singles = [[r, 0, 1, 0] for r, q in enumerate(q_lens) if q == 1]
+    p_items, s_items = (torch.tensor(x, dtype=torch.int32, device=DEV).reshape(-1) for x in (portions, singles))
+    q = torch.randn(T, nh * hd, device=DEV).to(torch.bfloat16)
+    common = dict(q=q, q_stride=nh * hd, k_cache=kc, v_cache=vc, block_tables=bt, ctx_lens=cl, cu_q=cu, nh=nh, nkv=nkv, hd=hd,
+                  block_size=bs, window=window, scale=hd ** -0.5, n_tokens=T, n_requests=len(q_lens))
+    need = ops.decode_attention_workspace_floats(hd, len(singles), nh, nkv, splits)
+    for split_keys in (0, 32 * -(-1100 // (32 * splits))):
+        outs = []
+        for together in (False, True):
+            out = torch.full((T + 2, nh * hd), -77.0, dtype=torch.bfloat16, device=DEV)
+            ws = torch.full((need,), float("nan"), device=DEV) if need else None
+            how = dict(n_splits=splits, workspace=ws, split_keys=split_keys, max_ctx=1100 if split_keys else 0)
+            if together:
+                ops.attention_together(out=out, portions=p_items, n_portions=len(portions), row_blocks=row_blocks, singles=s_items,
+                                       n_singles=len(singles), **how, **common)
+            else:
+                ops.attention_prefill(out=out, items=p_items, n_items=len(portions), row_blocks=row_blocks, **common)
+                ops.attention_decode(out=out, items=s_items, n_items=len(singles), **how, **common)
+            outs.append(out)
+        assert not torch.isnan(outs[0].float()).any() and bool((outs[1][T:] == -77.0).all())
+        starts = cu.tolist()
+        for r, n in enumerate(q_lens):
+            a, b = (x[starts[r] : starts[r] + n].double() for x in outs)
+            if n > 1:
+                assert torch.equal(a, b)
+            else:  # the launch alone takes four waves a split for short splits, which share the keys otherwise
+                assert (a - b).norm() <= 2.0 ** -8 * a.norm()
+
+
+def test_the_plan_puts_portions_and_single_tokens_together():
+    """One launch where both kinds' workgroups fit the card side by side and the single tokens keep half of their splits;
+    two where the portions' key ranges are in parts, or fill the card."""
+    from clockwork_amd.engine.batch import StepContext
+    from clockwork_amd.parts.attention import attention_plan
+
+    def plan_of(q_lens, ctx_lens, **how):
+        ctx = StepContext()
+        ctx.device = torch.device(DEV)
+        ctx.h_q_lens, ctx.h_ctx_lens = list(q_lens), list(ctx_lens)
+        assert ctx.num_compute_units == 256
+        return attention_plan(ctx, 12, 2, narrow_ok=True, whole_keys=512, **how)
+
+    plan = plan_of([320] + [1] * 16, [320] + [1500] * 16, together_ok=True)
+    assert plan.together and plan.decode_splits == 6 and plan.decode_split_keys * 6 >= 1500
+    plan = plan_of([320] + [1] * 16, [320] + [1500] * 16)
+    assert not plan.together and plan.decode_splits == 8
+    assert plan_of([320] + [1] * 16, [320] + [300] * 16, together_ok=True).together
+    assert not plan_of([2048] + [1] * 8, [2048] + [1500] * 8, together_ok=True).together  # the portion fills the card
+    assert not plan_of([64] + [1] * 8, [8000] + [1500] * 8, together_ok=True).together    # its keys are in parts
+    assert not plan_of([320], [320], together_ok=True).together
+
+
 def test_the_plan_shares_long_key_ranges_among_workgroups():
     """A short portion behind a long cached prefix makes few workgroups with long walks: its items
     are cut into as many parts as there are idle compute units for. A launch that fills the card
