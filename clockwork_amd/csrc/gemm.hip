@@ -1292,6 +1292,7 @@ CW_EXPORT int cw_gemm_bf16_skinny(int mode, const void* X, int64_t ldx, const vo
 // every rotary pair (half-split pairing, full rotary dimension) end up in one workgroup. The
 // epilogue adds the bias, rotates by float32(pos) * inv_freq[i] and writes q to ``q_out``
 // [M, nh * hd], rotated k and plain v to their cache rows ``slots[m]`` ([rows, nkv, hd]).
+// blockIdx.y takes MT tiles of 16 tokens.
 template <int WAVES, int MT>
 __global__ __launch_bounds__(WAVES * 64) void gemm_qkv_rope_bf16_kernel(
     const bf16_t* __restrict__ X, int64_t ldx, const bf16_t* __restrict__ W, const void* __restrict__ bias,
@@ -1303,6 +1304,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_qkv_rope_bf16_kernel(
   const int r = lane & 15, s = lane >> 4;
   const int half = hd / 2;
   const int tiles_per_head = hd / 16;
+  const int m0 = blockIdx.y * (MT * 16);          // the workgroup's first token
+  M = min(M - m0, MT * 16);
+  X += m0 * ldx;
+  positions += m0;
+  slots += m0;
+  q_out += (int64_t)m0 * nh * hd;
   const int head = blockIdx.x / tiles_per_head;   // 0 .. nh + 2 nkv - 1
   const int tile = blockIdx.x % tiles_per_head;
   const bool is_v = head >= nh + nkv;
@@ -1357,7 +1364,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_qkv_rope_bf16_kernel(
 #pragma unroll
   for (int e = 0; e < 8; ++e) zero[e] = (__bf16)0.0f;
   const int k_steps = (K + 31) / 32;
-  constexpr int U = MT == 1 ? 4 : 2;
+  constexpr int U = MT <= 2 ? 4 : 2;
   for (int ks0 = wave * U; ks0 < k_steps; ks0 += WAVES * U) {
     bf16x8_t wf[U], xf[U][MT];
 #pragma unroll
@@ -1479,17 +1486,26 @@ CW_EXPORT int cw_gemm_qkv_rope_bf16(const void* X, int64_t ldx, const void* W, c
   hipLaunchKernelGGL((gemm_qkv_rope_bf16_kernel<WAVES_, MT_>), grid, dim3(WAVES_ * 64), 0, stream, x, ldx, \
                      w, bias, bias_f32, positions, slots, inv_freq, (bf16_t*)q_out, (bf16_t*)k_cache,    \
                      (bf16_t*)v_cache, cache_rows, M, K, nh, nkv, hd)
-  if (M > 32) {  // the reduction buffer is WAVES * MT KB
-    if (K >= 512) CW_QKV(8, 4);
-    else CW_QKV(4, 4);
-  } else if (M > 16) {
-    if (tiles <= 256 && K >= 1024) CW_QKV(16, 2);
-    else if (K >= 512) CW_QKV(8, 2);
-    else CW_QKV(4, 2);
-  } else {
+  if (M <= 16) {
     if (tiles <= 256 && K >= 1024) CW_QKV(16, 1);
     else if (K >= 512) CW_QKV(8, 1);
     else CW_QKV(4, 1);
+  } else {
+    // One tile of tokens a workgroup while there are few of them, else two: a workgroup takes in its rows of x beside its
+    // rows of W (four tiles: 196 KB beside 49 KB at a width of 1536), at some 30 GB/s. (us, four or two tiles and
+    // one workgroup a tile of W / one tile / two, widths of 1536 and 128 tiles of W: 17 rows 5.80 / 4.78 / 5.80, 32 rows 6.35 /
+    // 5.06 / 6.14, 48 rows 7.56 / 6.73 / 6.11, 64 rows 7.90 / 6.95 / 6.39; of 896 and 72 tiles, 64 rows 6.20 / 5.02 / 5.19; of
+    // 2048 and 160 tiles, 17 rows 8.11 / 7.32 / 7.59, 64 rows 11.7 / 11.2 / 10.6.)
+    const int groups = (M + 15) / 16;
+    if (tiles * groups <= 320) {
+      grid.y = groups;
+      if (K >= 512) CW_QKV(8, 1);
+      else CW_QKV(4, 1);
+    } else {
+      grid.y = (groups + 1) / 2;
+      if (K >= 512) CW_QKV(8, 2);
+      else CW_QKV(4, 2);
+    }
   }
 #undef CW_QKV
   return cw_launch_status();
