@@ -15,6 +15,7 @@
 
 #include <limits.h>
 #include <type_traits>
+#include <utility>
 
 #ifndef CW_HD
 #error "compile with -DCW_HD=<head_dim>"
@@ -50,6 +51,7 @@ struct AttnParams {
   // decode kernel only
   int identity;           // 1: item i is request i and its one token is row i of the batch (items, cu_q unread)
   int split_keys;         // > 0: split s takes keys [s * split_keys, (s + 1) * split_keys), a multiple of 32
+  int decode_pages;       // -1: a split's pages do not fit LDS, they are looked up in memory
 };
 
 // the factor of a head's output of the token in row ``token`` of the batch
@@ -479,6 +481,45 @@ CW_EXPORT int cw_attention(int rows, int dtype, const void* q, int64_t q_stride,
 }
 
 // =====================================================================================
+// What the bfloat16 kernels below share: tiles of keys and values in LDS, as blocks of 16 keys x 32 elements (1 KB: what one
+// load of a wave with the LDS target brings), a key's four 16-byte granules permuted.
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+typedef __attribute__((ext_vector_type(4))) short s16x4_t;
+typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
+typedef __attribute__((address_space(3))) void lds_raw_t;
+
+// Where granule g of key k (0 to 15) lies in a block. K: eight neighbouring lanes of a ds_read_b128 take one
+// granule of eight keys, 64 bytes apart, and with these permutations every bank once; V: 16 lanes of a transposing read
+// take 32 bytes of four keys.
+__device__ __forceinline__ int k_granule(int k, int g) { return g ^ ((((k >> 1) ^ (k >> 3)) & 1) | (((k >> 2) & 1) << 1)); }
+__device__ __forceinline__ int v_granule(int k, int g) { return g ^ ((((k >> 1) ^ (k >> 2)) & 1) << 1); }
+
+// 16 bytes a lane from memory to LDS, to 1 KB at ``to`` (the same for all lanes), lane by lane; from an address a lane, or
+// from one address for all and an offset a lane. Written out, because behind the builtin the compiler puts a wait for all
+// such loads before the next transposing read, of whatever tile: what the kernel waits for and where is its own to say.
+// (No register is written.)
+__device__ __forceinline__ void load_to_lds(const void* from, void* to) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+               : : "v"(from), "s"((uint32_t)(uintptr_t)(lds_raw_t*)to) : "memory");
+}
+// (``OFFSET`` bytes further on at both ends: the instruction's own offset counts for the address in LDS as well)
+template <int OFFSET>
+__device__ __forceinline__ void load_to_lds(const void* from, void* to) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off offset:%2"
+               : : "v"(from), "s"((uint32_t)(uintptr_t)(lds_raw_t*)to), "n"(OFFSET) : "memory");
+}
+// The blocks of 32 elements of 16 rows, 64 bytes apart in memory and 1 KB in LDS.
+template <int... J>
+__device__ __forceinline__ void row_to_lds(const void* from, unsigned char* to, std::integer_sequence<int, J...>) {
+  (load_to_lds<J * 64>(from, to + J * (1024 - 64)), ...);
+}
+__device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, void* to) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               : : "v"(offset), "s"(base), "s"((uint32_t)(uintptr_t)(lds_raw_t*)to) : "memory");
+}
+
+// =====================================================================================
 // bfloat16 decode attention: one query token per work item, keys and values streamed at memory
 // speed, all products on the matrix cores.
 //
@@ -487,41 +528,32 @@ CW_EXPORT int cw_attention(int rows, int dtype, const void* q, int64_t q_stride,
 //   S^T[key, head] = K * Q^T        v_mfma_f32_16x16x32_bf16; the up to 16 heads of the group are
 //                                   the columns, so every key is fetched once for the whole group;
 //   softmax per head in float32: a lane holds 8 keys of one head, two shuffles finish a head;
-//   V^T from V: V times a 0/1 selector matrix comes back with keys in the lane's registers
-//                                   (the layout the next product needs), values bit-exact;
 //   O^T[d, head] += V^T * P^T       P^T is the softmax output as it lies in the registers.
-// K and V fragments are loaded from the pages with 16-byte loads, four neighbouring lanes 64 bytes of a key,
-// and swapped into operand layout by lane exchanges when they are used (ds_bpermute: the LDS unit's crossbar,
-// no memory). Loaded in operand layout, where neighbouring lanes hold different keys, each load is 64 requests to a
-// compute unit's load path instead of 16, and a tile of 32 keys of 128 elements takes that path a thousand cycles:
-// 2049 keys in one workgroup of four waves take 34 us so and 30 with the exchange, with eight waves 33 and 22.
-// The next tile's loads are issued before the current tile is computed. Waves are merged through
-// LDS at the end; splits are merged by a second, small kernel.
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+// A wave's tile comes from the pages straight into LDS of its own, four neighbouring lanes 64 bytes of a key, and its operands
+// from there: K fragments by 16-byte reads, V^T fragments by the transposing read (see the kernel for portions). Once a tile's
+// operands are in registers the next one is asked for (room for two tiles of heads of 64 gained nothing). Through registers,
+// with a lane exchange of every fragment into operand layout and V^T by products with 0/1 selector matrices, a tile of 32
+// keys of 128 elements cost a wave some 700 instructions, 1.8 us. Waves are merged through LDS at the end; splits are merged
+// by a second, small kernel. Bound by the chain from the context's length over the table to the keys, for many requests by memory.
+// Measured on an MI355X (with the merge; us, that way -> this): one request of 120 keys, 14 heads of 64 on 2, 4.7 -> 3.9, of 400
+// keys 6.4 -> 5.2; 12 heads of 128 on 2, one request of 2048 10.3 -> 8.7, 8 of 2048 12.8 -> 10.9, 32 of 2048 21.6 -> 20.3, 64 of
+// 2048 34.1 -> 32.3; 8 of 2048, 16 heads of 256 on 4, 26.5 -> 21.2. A decode step of 8 requests (1.5B shape) 1445 -> 1414 us.
+template <int HD> struct DecodeTile {
+  static constexpr int BYTES = 32 * HD * 4;  // 32 keys and values: a wave's LDS; its 16 heads' outputs lie over it at the end
+};
 
-// lane (c, s) takes what lane 4 c + s loaded: row c, slot s of 16 rows by four slots of 16 bytes
-typedef __attribute__((ext_vector_type(4))) int i32x4_t;
-__device__ __forceinline__ bf16x8_t dec_to_operand(const bf16x8_t& v, int lane) {
-  const int from = ((lane & 15) * 4 + (lane >> 4)) * 4;  // byte address of that lane
-  const i32x4_t q = __builtin_bit_cast(i32x4_t, v);
-  i32x4_t t;
-#pragma unroll
-  for (int d = 0; d < 4; ++d) t[d] = __builtin_amdgcn_ds_bpermute(from, q[d]);
-  return __builtin_bit_cast(bf16x8_t, t);
-}
-
-template <int HD, bool POW2, int WAVES>
+template <int HD, bool POW2, int WAVES, bool CAP>
 __device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int item, const int y, const int split) {
   constexpr int NF = HD / 32;  // 32-element steps over the head dimension
   constexpr int ND = HD / 16;  // 16-wide blocks of the head dimension
-  extern __shared__ __align__(16) float dyn_s[];  // [waves][16 heads][HD] outputs, then this split's pages
-  float* o_s = dyn_s;
-  int* tbl = reinterpret_cast<int*>(dyn_s + WAVES * 16 * HD);
+  using Tile = DecodeTile<HD>;
+  extern __shared__ __align__(1024) unsigned char dec_smem[];  // [waves][a tile], then this split's pages if they fit
+  const bool in_lds = p.decode_pages >= 0;
+  int* const tbl = reinterpret_cast<int*>(dec_smem + WAVES * Tile::BYTES);
   __shared__ float M_s[WAVES][16];
   __shared__ float L_s[WAVES][16];
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, s = lane >> 4;
   const int kvh = y / p.n_chunks, chunk = y % p.n_chunks;
   // Every trip to memory that depends on an earlier one costs about a microsecond, which is what
@@ -547,7 +579,8 @@ __device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int it
     const int k_last = min(k_first + p.split_keys, p.table_stride * bs) - 1;
     page0 = cw_page_index<POW2>(k_first, bs, sh);
     const int n_pages = k_last >= k_first ? cw_page_index<POW2>(k_last, bs, sh) - page0 + 1 : 0;
-    for (int i = threadIdx.x; i < n_pages; i += WAVES * 64) tbl[i] = table[page0 + i];
+    if (in_lds)
+      for (int i = threadIdx.x; i < n_pages; i += WAVES * 64) tbl[i] = table[page0 + i];
   }
   const int pos = ctx - qlen + tok0;
   const int lo = p.window > 0 ? max(0, pos - p.window + 1) : 0;
@@ -565,7 +598,8 @@ __device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int it
     page0 = cw_page_index<POW2>(t_begin * 32, bs, sh);
     const int last_key = min(pos, t_end * 32 - 1);
     const int n_pages = t_end > t_begin ? cw_page_index<POW2>(last_key, bs, sh) - page0 + 1 : 0;
-    for (int i = threadIdx.x; i < n_pages; i += WAVES * 64) tbl[i] = table[page0 + i];
+    if (in_lds)
+      for (int i = threadIdx.x; i < n_pages; i += WAVES * 64) tbl[i] = table[page0 + i];
   }
   __syncthreads();
 
@@ -578,41 +612,56 @@ __device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int it
 #pragma unroll
     for (int j = 0; j < NF; ++j) qf[j] = *reinterpret_cast<const bf16x8_t*>(qrow + (j * 4 + s) * 8);
   }
-  // selectors (B operand) that pick elements 0..15 / 16..31 of a 32-element step: (k = 8s + e, n = c)
-  bf16x8_t sel_lo, sel_hi;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    sel_lo[e] = (8 * s + e == c) ? (__bf16)1.0f : (__bf16)0.0f;
-    sel_hi[e] = (8 * s + e == 16 + c) ? (__bf16)1.0f : (__bf16)0.0f;
-  }
-
-  // loads of one 32-key tile, always issued: a masked key is read from a row of zeros
-  auto load_tile = [&](int t, bf16x8_t (*kf)[NF], bf16x8_t (*vf)[NF]) {
+  // tile t into the wave's LDS; a masked key is read from a row of zeros
+  unsigned char* const region = dec_smem + wave * Tile::BYTES;
+  const int f_key = lane >> 2, k_piece = k_granule(f_key, lane & 3) * 8, v_piece = v_granule(f_key, lane & 3) * 8;
+  auto bring = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
-      const int kp = t * 32 + kb * 16 + (lane >> 2);
-      const bool ok = t < t_end && kp >= lo && kp <= pos;
-      const int page = tbl[ok ? cw_page_index<POW2>(kp, bs, sh) - page0 : 0];
+      const int kp = t * 32 + kb * 16 + f_key;
+      const bool ok = kp >= lo && kp <= pos;
+      const int at = ok ? cw_page_index<POW2>(kp, bs, sh) - page0 : 0;
+      const int page = in_lds ? tbl[at] : ok ? table[page0 + at] : -1;
       const bool have = ok && page >= 0;
       const int64_t off = (((int64_t)page * bs + cw_page_offset<POW2>(kp, bs, sh)) * p.nkv + kvh) * HD;
-      const bf16_t* kr = have ? kc + off : zrow;
-      const bf16_t* vr = have ? vc + off : zrow;
-#pragma unroll
-      for (int j = 0; j < NF; ++j) kf[kb][j] = *reinterpret_cast<const bf16x8_t*>(kr + (j * 4 + (lane & 3)) * 8);
-#pragma unroll
-      for (int j = 0; j < NF; ++j) vf[kb][j] = *reinterpret_cast<const bf16x8_t*>(vr + (j * 4 + (lane & 3)) * 8);
+      const bf16_t* kr = (have ? kc + off : zrow) + k_piece;
+      const bf16_t* vr = (have ? vc + off : zrow) + v_piece;
+      unsigned char* const to = region + kb * NF * 1024;
+      row_to_lds(kr, to, std::make_integer_sequence<int, NF>{});
+      row_to_lds(vr, to + Tile::BYTES / 2, std::make_integer_sequence<int, NF>{});
     }
   };
+  const int k_at = c * 64 + k_granule(c, s) * 16, v_key = 4 * s + (c >> 2);
+  const int v_at0 = v_key * 64 + v_granule(v_key, 0) * 16 + (c & 3) * 8, v_at1 = v_at0 ^ 32;
 
   f32x4_t o[ND];
 #pragma unroll
   for (int db = 0; db < ND; ++db) o[db] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
   float m_run = -INFINITY, l_run = 0.0f;  // of head c, the same in all four lane groups
-  bf16x8_t kf[2][NF], vf[2][NF], kf_n[2][NF], vf_n[2][NF];
-  load_tile(t_begin + wave, kf, vf);
+  if (t_begin + wave < t_end) bring(t_begin + wave);
+  // the query is home, too: a wait for it inside the loop would be one for the tile on its way
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   for (int t = t_begin + wave; t < t_end; t += WAVES) {
     const int kv0 = t * 32;
-    load_tile(t + WAVES, kf_n, vf_n);  // the wave's next tile is on its way meanwhile
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // the wave's own loads: its tile is in LDS
+    asm volatile("" ::: "memory");
+    bf16x8_t kf[2][NF], vt[ND];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int j = 0; j < NF; ++j) kf[kb][j] = *reinterpret_cast<const bf16x8_t*>(region + (kb * NF + j) * 1024 + k_at);
+#pragma unroll
+    for (int db = 0; db < ND; ++db) {
+      unsigned char* vp = region + Tile::BYTES / 2 + (db >> 1) * 1024 + (db & 1 ? v_at1 : v_at0);
+      const s16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)vp);
+      const s16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(vp + NF * 1024));
+      vt[db] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+    }
+    if (t + WAVES < t_end) {
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the tile has been read
+      asm volatile("" ::: "memory");
+      bring(t + WAVES);
+    }
     // ---- S^T = K Q^T, keys 4s..4s+3 of each 16-key block for head c
     float sv[8];
     float tmax = -INFINITY;
@@ -620,12 +669,12 @@ __device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int it
     for (int kb = 0; kb < 2; ++kb) {
       f32x4_t sc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int j = 0; j < NF; ++j) sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dec_to_operand(kf[kb][j], lane), qf[j], sc, 0, 0, 0);
+      for (int j = 0; j < NF; ++j) sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[kb][j], qf[j], sc, 0, 0, 0);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int kp = kv0 + kb * 16 + 4 * s + i;
         float v = sc[i] * p.scale;
-        if (p.softcap > 0.0f) v = p.softcap * tanhf(v / p.softcap);
+        if (CAP) v = p.softcap * tanhf(v / p.softcap);
         v = (kp >= lo && kp <= pos) ? v : -INFINITY;
         sv[kb * 4 + i] = v;
         tmax = fmaxf(tmax, v);
@@ -655,58 +704,48 @@ __device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int it
     }
     // ---- O^T += V^T P^T
 #pragma unroll
-    for (int j = 0; j < NF; ++j) {
-      bf16x8_t vt_lo, vt_hi;
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
-        const bf16x8_t vo = dec_to_operand(vf[kb][j], lane);
-        const f32x4_t tl = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vo, sel_lo, zero, 0, 0, 0);
-        const f32x4_t th = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vo, sel_hi, zero, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          vt_lo[kb * 4 + i] = (__bf16)tl[i];
-          vt_hi[kb * 4 + i] = (__bf16)th[i];
-        }
-      }
-      o[2 * j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt_lo, pf, o[2 * j], 0, 0, 0);
-      o[2 * j + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt_hi, pf, o[2 * j + 1], 0, 0, 0);
-    }
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int j = 0; j < NF; ++j) { kf[kb][j] = kf_n[kb][j]; vf[kb][j] = vf_n[kb][j]; }
+    for (int db = 0; db < ND; ++db) o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt[db], pf, o[db], 0, 0, 0);
   }
 
   // a context beyond the fixed key ranges (the caller promised there is none) must not pass for a result
   if (p.split_keys > 0 && pos >= p.n_splits * p.split_keys) l_run = NAN;
-  // ---- merge the waves: o_s[wave][head c][d], lane (c, s) holds d = db * 16 + 4s .. + 3
+  // ---- merge the waves: [head c][d] over the wave's tiles, lane (c, s) holds d = db * 16 + 4s .. + 3
   if (s == 0) { M_s[wave][c] = m_run; L_s[wave][c] = l_run; }
+  float* const mine = reinterpret_cast<float*>(region);
 #pragma unroll
-  for (int db = 0; db < ND; ++db)
-    *reinterpret_cast<f32x4_t*>(&o_s[(wave * 16 + c) * HD + db * 16 + 4 * s]) = o[db];
+  for (int db = 0; db < ND; ++db) *reinterpret_cast<f32x4_t*>(&mine[c * HD + db * 16 + 4 * s]) = o[db];
   __syncthreads();
   const int64_t base = ((int64_t)item * (p.nkv * p.n_chunks) + y) * p.n_splits + split;
-  for (int idx = threadIdx.x; idx < gh * HD; idx += WAVES * 64) {
-    const int g = idx / HD, d = idx - g * HD;
+  for (int idx = threadIdx.x; idx < gh * (HD / 4); idx += WAVES * 64) {
+    const int g = idx / (HD / 4), d = (idx - g * (HD / 4)) * 4;
     const int hg = chunk * gh + g;
     if (hg >= group) continue;
     float M = -INFINITY;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) M = fmaxf(M, M_s[w][g]);
-    float L = 0.0f, O = 0.0f;
+    float L = 0.0f;
+    f32x4_t O = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
       const float mw = M_s[w][g];
       const float wgt = mw == -INFINITY ? 0.0f : __expf(mw - M);
       L = fmaf(L_s[w][g], wgt, L);
-      O = fmaf(o_s[(w * 16 + g) * HD + d], wgt, O);
+      O += *reinterpret_cast<const f32x4_t*>(dec_smem + w * Tile::BYTES + (g * HD + d) * 4) * wgt;
     }
     if (p.n_splits == 1) {
-      ((bf16_t*)p.out)[(int64_t)(q_begin + tok0) * p.out_stride + (kvh * group + hg) * HD + d] =
-          __float2bfloat16(O / L * attn_head_gate(p, q_begin + tok0, kvh * group + hg));
+      const float scale = attn_head_gate(p, q_begin + tok0, kvh * group + hg) / L;
+      bf16_t* const out = (bf16_t*)p.out + (int64_t)(q_begin + tok0) * p.out_stride + (kvh * group + hg) * HD + d;
+      if (((uintptr_t)p.out & 7) == 0 && (p.out_stride & 3) == 0) {
+        *reinterpret_cast<uint2*>(out) = make_uint2((uint32_t)cw_float_to_bf16_bits(O[0] * scale) | ((uint32_t)cw_float_to_bf16_bits(O[1] * scale) << 16),
+                                                    (uint32_t)cw_float_to_bf16_bits(O[2] * scale) | ((uint32_t)cw_float_to_bf16_bits(O[3] * scale) << 16));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[e] = cw_from_float<bf16_t>(O[e] * scale);
+      }
     } else {
-      p.part_o[(base * gh + g) * HD + d] = O;
+      float* const out = p.part_o + (base * gh + g) * HD + d;  // (8 bytes aligned)
+      *reinterpret_cast<float2*>(out) = make_float2(O[0], O[1]);
+      *reinterpret_cast<float2*>(out + 2) = make_float2(O[2], O[3]);
       if (d == 0) {
         p.part_ml[(base * gh + g) * 2] = M;
         p.part_ml[(base * gh + g) * 2 + 1] = L;
@@ -715,9 +754,9 @@ __device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int it
   }
 }
 
-template <int HD, bool POW2, int WAVES>
+template <int HD, bool POW2, int WAVES, bool CAP>
 __global__ __launch_bounds__(WAVES * 64) void attn_decode_bf16_kernel(AttnParams p) {
-  attn_decode_of<HD, POW2, WAVES>(p, blockIdx.x, blockIdx.y, blockIdx.z);
+  attn_decode_of<HD, POW2, WAVES, CAP>(p, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // Merge of the decode kernel's splits: one wave per (item, head, EL elements of the head). EL / 4 lanes take a split's
@@ -835,6 +874,16 @@ CW_EXPORT int64_t cw_attention_decode_workspace_floats(int n_items, int nh, int 
 }
 
 #if CW_HAS_DECODE
+// The most pages of a split that are taken: what 160 KB hold beside the waves' outputs.
+static bool decode_pages_ok(int waves, int64_t pages) {
+  return sizeof(float) * waves * 16 * CW_HD + sizeof(int) * (size_t)pages <= 160 * 1024;
+}
+
+// Pages of a split that lie in LDS beside ``tiles`` bytes (and the waves' statistics): all of them, or -1.
+static int decode_pages_in_lds(size_t tiles, int64_t pages) {
+  return tiles + sizeof(int) * (size_t)pages <= 158 * 1024 ? (int)pages : -1;
+}
+
 static void launch_decode_merge(const AttnParams& p, int n_items, hipStream_t stream) {
   constexpr int HD = CW_HD;
   if (p.n_splits > 1) {
@@ -848,26 +897,34 @@ static void launch_decode_merge(const AttnParams& p, int n_items, hipStream_t st
   }
 }
 
-template <bool POW2, int WAVES>
-static int launch_decode(AttnParams& p, int n_items, hipStream_t stream) {
+template <bool POW2, int WAVES, bool CAP>
+static int launch_decode_of(AttnParams& p, int n_items, hipStream_t stream) {
   constexpr int HD = CW_HD;
   // keys of a split: at most ceil(tiles / splits) tiles of 32; their pages go to LDS
   const int64_t max_tiles = ((int64_t)p.table_stride * p.block_size + 31) / 32;
   const int64_t tiles_per_split = p.split_keys > 0 ? p.split_keys / 32 : (max_tiles + p.n_splits - 1) / p.n_splits;
   const int64_t pages = (tiles_per_split * 32 + p.block_size - 1) / p.block_size + 2;
-  const size_t smem = sizeof(float) * WAVES * 16 * HD + sizeof(int) * (size_t)pages;
-  if (smem > 160 * 1024) return CW_ERR_SIZE;
+  if (!decode_pages_ok(WAVES, pages)) return CW_ERR_SIZE;
+  constexpr size_t tiles = (size_t)WAVES * DecodeTile<HD>::BYTES;
+  p.decode_pages = decode_pages_in_lds(tiles, pages);
+  const size_t smem = tiles + (p.decode_pages > 0 ? sizeof(int) * (size_t)p.decode_pages : 0);
   static size_t raised = 0;
   if (smem > raised) {
-    if (hipFuncSetAttribute((const void*)attn_decode_bf16_kernel<HD, POW2, WAVES>,
+    if (hipFuncSetAttribute((const void*)attn_decode_bf16_kernel<HD, POW2, WAVES, CAP>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
       return CW_ERR_LAUNCH;
     raised = smem;
   }
   dim3 grid(n_items, p.nkv * p.n_chunks, p.n_splits), block(WAVES * 64);
-  hipLaunchKernelGGL((attn_decode_bf16_kernel<HD, POW2, WAVES>), grid, block, smem, stream, p);
+  hipLaunchKernelGGL((attn_decode_bf16_kernel<HD, POW2, WAVES, CAP>), grid, block, smem, stream, p);
   launch_decode_merge(p, n_items, stream);
   return cw_launch_status();
+}
+
+template <int WAVES>
+static int launch_decode(AttnParams& p, int n_items, hipStream_t stream) {
+  if (p.softcap > 0.0f) return p.bs_shift >= 0 ? launch_decode_of<true, WAVES, true>(p, n_items, stream) : launch_decode_of<false, WAVES, true>(p, n_items, stream);
+  return p.bs_shift >= 0 ? launch_decode_of<true, WAVES, false>(p, n_items, stream) : launch_decode_of<false, WAVES, false>(p, n_items, stream);
 }
 #endif
 
@@ -931,13 +988,10 @@ CW_EXPORT int cw_attention_decode_bf16(const void* q, int64_t q_stride, void* ou
   if (status != CW_OK || n_items == 0) return status;
   // what a split's keys are shared among: the most keys a split may have, by the caller's fixed places or by its table
   const int64_t keys = split_keys > 0 ? split_keys : ((int64_t)table_stride * block_size + n_splits - 1) / n_splits;
-  // more than four waves can have on their way at once: eight (2049 keys of 128 elements in one workgroup: 30 us
-  // with four waves, 22 with eight; larger heads have no registers for two tiles of eight waves), where their LDS leaves
-  // room for the pages (of a table of very many small ones)
+  // more than four waves can have on their way at once: eight (larger heads' tiles have no room for them)
   if constexpr (CW_HD <= 128)
-    if (keys > 128 && sizeof(float) * 8 * 16 * CW_HD + sizeof(int) * ((keys + 63) / block_size + 3) <= 160 * 1024)
-      return p.bs_shift >= 0 ? launch_decode<true, 8>(p, n_items, stream) : launch_decode<false, 8>(p, n_items, stream);
-  return p.bs_shift >= 0 ? launch_decode<true, 4>(p, n_items, stream) : launch_decode<false, 4>(p, n_items, stream);
+    if (keys > 128 && decode_pages_ok(8, (keys + 63) / block_size + 3)) return launch_decode<8>(p, n_items, stream);
+  return launch_decode<4>(p, n_items, stream);
 #else
   return CW_ERR_ARG;
 #endif
@@ -974,10 +1028,6 @@ CW_EXPORT int cw_attention_decode_bf16(const void* q, int64_t q_stride, void* ou
 // (tiles through registers, all waves in step) -> now: 2048 tokens of 12 heads of 128 on 2 behind 6144, 164 -> 117 us
 // (0.77 PFLOP/s on 206 compute units); of 28 on 4, 319 -> 233 (0.90); 2048 tokens without a prefix 43 -> 32.6; 137 tokens
 // 11.7 -> 9.1; 1000 tokens of 14 heads of 64 behind 7000, 69 -> 51; of 16 of 256 on 4 behind 4000, 218 -> 143.
-typedef __attribute__((ext_vector_type(4))) short s16x4_t;
-typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
-typedef __attribute__((address_space(3))) void lds_raw_t;
-
 // RB: row blocks (waves that own 32 query rows each) of a workgroup, 4 or 2. With 2 the same eight
 // waves cut a stage's keys four ways instead of two: half the rows per workgroup and half the
 // time per stage, for launches whose portions would otherwise leave compute units without work
@@ -1000,25 +1050,6 @@ struct PrefillTile {
   static constexpr size_t XCHG_BYTES = XO_BYTES + (NH > 1 ? (size_t)NH * RB * 2 * 2 * 64 * 4 : 0);
   static constexpr size_t BYTES = TILES > XCHG_BYTES ? TILES : XCHG_BYTES;
 };
-
-// Where granule g of key k (0 to 15) lies in a block. K: eight neighbouring lanes of a ds_read_b128 take one
-// granule of eight keys, 64 bytes apart, and with these permutations every bank once; V: 16 lanes of a transposing read
-// take 32 bytes of four keys.
-__device__ __forceinline__ int k_granule(int k, int g) { return g ^ ((((k >> 1) ^ (k >> 3)) & 1) | (((k >> 2) & 1) << 1)); }
-__device__ __forceinline__ int v_granule(int k, int g) { return g ^ ((((k >> 1) ^ (k >> 2)) & 1) << 1); }
-
-// 16 bytes a lane from memory to LDS, to 1 KB at ``to`` (the same for all lanes), lane by lane; from an address a lane, or
-// from one address for all and an offset a lane. Written out, because behind the builtin the compiler puts a wait for all
-// such loads before the next transposing read, of whatever tile: what the kernel waits for and where is its own to say.
-// (No register is written.)
-__device__ __forceinline__ void load_to_lds(const void* from, void* to) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-               : : "v"(from), "s"((uint32_t)(uintptr_t)(lds_raw_t*)to) : "memory");
-}
-__device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, void* to) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               : : "v"(offset), "s"(base), "s"((uint32_t)(uintptr_t)(lds_raw_t*)to) : "memory");
-}
 
 // PAGES16: a page holds 2^n keys, 16 or more, so that 16 keys of a stage lie in one page
 template <int HD, bool PAGES16, int RB, bool CAP>
@@ -1427,7 +1458,7 @@ __global__ __launch_bounds__((PrefillTile<HD, RB>::NT), 2) void attn_together_bf
   } else {
     b -= first;
     const int of = b / a.n_singles, heads = a.singles.nkv * a.singles.n_chunks;
-    attn_decode_of<HD, PAGES16, 8>(a.singles, b - of * a.n_singles, of % heads, of / heads);
+    attn_decode_of<HD, PAGES16, 8, false>(a.singles, b - of * a.n_singles, of % heads, of / heads);
   }
 }
 #endif
@@ -1654,12 +1685,15 @@ CW_EXPORT int cw_attention_together_bf16(const void* q, int64_t q_stride, void* 
   const int64_t max_tiles = ((int64_t)table_stride * block_size + 31) / 32;
   const int64_t tiles_per_split = split_keys > 0 ? split_keys / 32 : (max_tiles + n_splits - 1) / n_splits;
   const int64_t pages = (tiles_per_split * 32 + block_size - 1) / block_size + 2;
-  const size_t for_singles = sizeof(float) * 8 * 16 * CW_HD + sizeof(int) * (size_t)pages;
+  if (!decode_pages_ok(8, pages)) return CW_ERR_SIZE;
+  constexpr size_t tiles = 8 * (size_t)DecodeTile<CW_HD>::BYTES;
+  a.singles.decode_pages = decode_pages_in_lds(tiles, pages);
+  const size_t for_singles = tiles + (a.singles.decode_pages > 0 ? sizeof(int) * (size_t)a.singles.decode_pages : 0);
   auto launch = [&](auto rb, auto pages16) {
     constexpr int RB = decltype(rb)::value;
     constexpr bool P16 = decltype(pages16)::value;
     const size_t smem = for_singles > PrefillTile<CW_HD, RB>::BYTES ? for_singles : PrefillTile<CW_HD, RB>::BYTES;
-    if (smem > 156 * 1024) return CW_ERR_SIZE;  // (beside the single tokens' statistics)
+    static_assert(PrefillTile<CW_HD, RB>::BYTES <= 158 * 1024, "tiles and the single tokens' statistics fit LDS");
     static size_t raised = 0;
     if (smem > raised) {
       if (hipFuncSetAttribute((const void*)attn_together_bf16_kernel<CW_HD, P16, RB>, hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -1029,6 +1029,19 @@ def test_decode_attention_kernel(nh, nkv, hd, bs, ctx_lens, splits, fixed_ranges
         torch.testing.assert_close(out[r : r + 1].float().cpu(), want, **tol(dtype))
 
 
+@pytest.mark.parametrize("nh,nkv,hd,ctx", [(3, 1, 128, 20000), (2, 1, 256, 12000)])
+def test_decode_attention_of_a_table_that_does_not_fit_beside_the_tiles(nh, nkv, hd, ctx):
+    """Pages of one key: a split's page numbers are looked up in memory."""
+    table = torch.randperm(ctx + 5).tolist()[:ctx]
+    kc, vc, ks, vs = _paged_setup(torch.bfloat16, nkv, hd, 1, ctx + 5, [table], [ctx], poison=float("nan"))
+    q = 3.0 * torch.randn(1, nh, hd, device=DEV).to(torch.bfloat16)
+    for fixed_ranges in (False, True):
+        out = _run_attention(torch.bfloat16, nh, nkv, hd, 1, [table], [ctx], [1], kc, vc, [q], splits=1, decode_kernel=True,
+                             fixed_ranges=fixed_ranges)
+        want = plain.attention_dense(q.double().cpu(), ks[0].double().cpu(), vs[0].double().cpu(), hd ** -0.5)
+        assert (out.double().cpu() - want).norm() / want.norm() < 2.0 ** -8
+
+
 @pytest.mark.parametrize("nh,nkv,hd", [(6, 2, 96), (4, 1, 32), (12, 2, 128), (40, 2, 64), (2, 2, 160), (2, 1, 256)])
 @pytest.mark.parametrize("splits", [2, 3, 8, 9, 16, 17, 63, 64, 65, 129])
 def test_decode_attention_merge(nh, nkv, hd, splits):
