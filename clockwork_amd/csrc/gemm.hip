@@ -143,19 +143,23 @@ __global__ __launch_bounds__(512) void gemm_f32_rows_kernel(const float* __restr
 // 2048 x 1536 9.9 -> 8.3; the sums are the same bit for bit.
 #define GT_BLOCK_WAVES 8
 #define GT_BLOCKS 120   // blocks a workgroup takes: 1 KB of LDS each with 16 rows of x
+// GLU: W = [gate; up], a tile is 8 gate rows and the 8 up rows that belong to them, C the gated product [M, N / 2].
+template <bool GLU>
 __global__ __launch_bounds__(GT_BLOCK_WAVES * 64) void gemm_f32_blocks_kernel(const float* __restrict__ A, int64_t lda,
                                                                               const float* __restrict__ W,
                                                                               const float* __restrict__ bias, float* __restrict__ C,
                                                                               int64_t ldc, int M, int N, int K, int parts, int part_blocks,
-                                                                              int parts_here, int64_t plane_stride) {
+                                                                              int parts_here, int64_t plane_stride, float act) {
   extern __shared__ __align__(16) float red[];
   constexpr int U = 8;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, s = lane >> 4;
-  const int n0 = blockIdx.x * 16;
+  const int n0 = blockIdx.x * (GLU ? 8 : 16), cols = GLU ? N / 2 : N;
   const int z0 = blockIdx.y * parts_here, z1 = min(parts, z0 + parts_here);
   const int b0 = z0 * part_blocks, b1 = min(K / 16, z1 * part_blocks);
-  const float* const w = W + (int64_t)min(n0 + (lane >> 2), N - 1) * K + 4 * (lane & 3);
+  const int tile_row = lane >> 2;
+  const int row = GLU ? min(n0 + (tile_row & 7), cols - 1) + (tile_row >> 3) * cols : min(n0 + tile_row, N - 1);
+  const float* const w = W + (int64_t)row * K + 4 * (lane & 3);
   const float* const x = A + (int64_t)min(r, M - 1) * lda + 4 * s;
   for (int b = b0 + wave; b < b1; b += U * GT_BLOCK_WAVES) {
     f32x4_t wv[U], xv[U];
@@ -186,14 +190,26 @@ __global__ __launch_bounds__(GT_BLOCK_WAVES * 64) void gemm_f32_blocks_kernel(co
     const int n = n0 + (at & 15);
     if (plane_stride > 0) {
       if (n < N) C[(z0 + z) * plane_stride + (int64_t)(at >> 4) * ldc + n] = total;
-    } else if (parts == 1) {
+    } else if (parts == 1 && !GLU) {
       if (n < N) C[(int64_t)(at >> 4) * ldc + n] = total + (bias ? bias[n] : 0.0f);
     } else {
       sums[i] = total;
     }
   }
-  if (plane_stride > 0 || parts == 1) return;
+  if (plane_stride > 0 || (parts == 1 && !GLU)) return;
   cw_lds_barrier();
+  if constexpr (GLU) {
+    for (int i = threadIdx.x; i < M * 8; i += GT_BLOCK_WAVES * 64) {
+      const int at = (i >> 3) * 16 + (i & 7), n = n0 + (i & 7);
+      float gate = sums[at], up = sums[at + 8];
+      for (int z = 1; z < parts; ++z) {
+        gate += sums[z * outputs + at];
+        up += sums[z * outputs + at + 8];
+      }
+      if (n < cols) C[(int64_t)(i >> 3) * ldc + n] = cw_gated(gate, up, act);
+    }
+    return;
+  }
   for (int at = threadIdx.x; at < outputs; at += GT_BLOCK_WAVES * 64) {
     const int n = n0 + (at & 15);
     float total = sums[at];
@@ -549,12 +565,12 @@ static int launch_gemm_f32(const float* A, int64_t lda, const float* W, const fl
       const dim3 grid(tiles, (splits + here - 1) / here);
       static size_t raised = 48 * 1024;
       if (lds > raised) {
-        if (hipFuncSetAttribute((const void*)gemm_f32_blocks_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+        if (hipFuncSetAttribute((const void*)gemm_f32_blocks_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
           return CW_ERR_LAUNCH;
         raised = lds;
       }
-      hipLaunchKernelGGL(gemm_f32_blocks_kernel, grid, dim3(GT_BLOCK_WAVES * 64), lds, stream, A, lda, W, bias, C, ldc, M, N, K, splits,
-                         part_blocks, here, stride);
+      hipLaunchKernelGGL(gemm_f32_blocks_kernel<false>, grid, dim3(GT_BLOCK_WAVES * 64), lds, stream, A, lda, W, bias, C, ldc, M, N, K,
+                         splits, part_blocks, here, stride, 0.0f);
       return cw_launch_status();
     }
   }
@@ -616,6 +632,31 @@ CW_EXPORT int cw_gemm_f32(const float* A, int64_t lda, const float* W, const flo
   if (rc != CW_OK) return rc;
   hipLaunchKernelGGL(gemm_f32_sum_kernel, dim3((unsigned)((part_stride + 255) / 256)), dim3(256), 0, stream, workspace,
                      splits, part_stride, bias, C, ldc, M, N);
+  return cw_launch_status();
+}
+
+// Does cw_gemm_f32_swiglu take this product (few rows, whole blocks of K that one workgroup takes)?
+CW_EXPORT int cw_gemm_f32_swiglu_ok(int M, int N, int K, int64_t lda) {
+  return M > 0 && M <= GT_ROWS_MAX && N > 0 && !(N & 1) && N <= 65536 && K > 0 && !(K & 15) && !(lda & 3) && lda >= K && K / 16 <= GT_BLOCKS ? 1 : 0;
+}
+
+// The gated product of W = [gate; up] [N, K] as float32 [M, N / 2]: what cw_gemm_f32 and the gate kernel give, bit for bit,
+// without the [M, N] between them (``act`` as for the bfloat16 products).
+CW_EXPORT int cw_gemm_f32_swiglu(const float* A, int64_t lda, const float* W, float* C, int64_t ldc, int M, int N, int K, float act,
+                                 hipStream_t stream) {
+  if (M == 0) return CW_OK;
+  if (!cw_gemm_f32_swiglu_ok(M, N, K, lda) || ldc < N / 2 || !C || ((uintptr_t)A & 15) || ((uintptr_t)W & 15)) return CW_ERR_ARG;
+  int splits, per;
+  gemm_f32_plan(N, K, &splits, &per);
+  const size_t lds = (size_t)(K / 16 + splits) * M * 16 * sizeof(float);
+  static size_t raised = 48 * 1024;
+  if (lds > raised) {
+    if (hipFuncSetAttribute((const void*)gemm_f32_blocks_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+      return CW_ERR_LAUNCH;
+    raised = lds;
+  }
+  hipLaunchKernelGGL(gemm_f32_blocks_kernel<true>, dim3((N / 2 + 7) / 8), dim3(GT_BLOCK_WAVES * 64), lds, stream, A, lda, W, nullptr, C, ldc,
+                     M, N, K, splits, per / 16, splits, 0, act);
   return cw_launch_status();
 }
 

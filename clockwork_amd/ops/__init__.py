@@ -106,6 +106,8 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_gemm_f32_workspace_floats": [I, I, I],
             "cw_gemm_f32_partial_planes": [I, I, I],
             "cw_gemm_f32_partial": [P, L, P, P, I, I, I, P],
+            "cw_gemm_f32_swiglu_ok": [I, I, I, L],
+            "cw_gemm_f32_swiglu": [P, L, P, P, L, I, I, I, F, P],
             "cw_gemm_bf16_skinny": [I, P, L, P, P, L, I, I, I, I, F, P],
             "cw_gemm_bf16_skinny_ksplits": [I, I, I],
             "cw_gemm_bf16_skinny_fast": [I, I, I, I],
@@ -1187,6 +1189,11 @@ def linear_swiglu(x, gate_up_weight: torch.Tensor, policy: "ProductPolicy | None
     if not (gate_up_weight.shape[1] == K and two_i % 2 == 0):
         raise KernelError("gate_up weight must be [2 I, K]")
     out = torch.empty((M, two_i // 2), dtype=x.dtype, device=x.device)
+    if (x.dtype == torch.float32 and gate_up_weight.dtype == torch.float32 and limit != GELU_GATE and _aligned(x, gate_up_weight)
+            and _load("gemm").cw_gemm_f32_swiglu_ok(M, two_i, K, K)):
+        _check(_load("gemm").cw_gemm_f32_swiglu(_ptr(x), K, _ptr(gate_up_weight), _ptr(out), two_i // 2, M, two_i, K, float(limit), _stream()),
+               "gemm_f32_swiglu")
+        return out
     if (x.dtype == torch.bfloat16 and M <= STREAM_MAX_ROWS and K % 8 == 0
             and _load("gemm").cw_gemm_bf16_skinny_fast(2, M, two_i, K)):
         if not (gate_up_weight.dtype == torch.bfloat16):

@@ -384,6 +384,18 @@ def test_gemm_f32_few_rows_by_blocks(N, K):
         assert torch.equal(got, whole[lo:hi])
 
 
+@pytest.mark.parametrize("M", [1, 3, 16])
+@pytest.mark.parametrize("I,K", [(8, 16), (9, 48), (4864, 896), (100, 1920), (100, 1936)])
+@pytest.mark.parametrize("limit", [0.0, 7.0, -1.0, -2.0])
+def test_gated_gemm_f32_of_few_rows(M, I, K, limit):
+    """The gated product in one kernel is the product and the gate kernel, bit for bit (the last K is for two kernels)."""
+    from clockwork_amd import ops
+
+    x, w = torch.randn(M, K, device=DEV), torch.randn(2 * I, K, device=DEV)
+    want = ops._gate(ops.linear(x, w), torch.empty(M, I, device=DEV), limit)
+    assert torch.equal(ops.linear_swiglu(x, w, limit=limit), want)
+
+
 @pytest.mark.parametrize("M", [1, 8, 16, 17, 33, 64])
 @pytest.mark.parametrize("N,K", [(100, 176), (2048, 1536), (48, 64), (5000, 200)])
 def test_skinny_bf16_product(M, N, K):
