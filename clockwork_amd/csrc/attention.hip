@@ -1026,8 +1026,9 @@ CW_EXPORT int cw_attention_decode_bf16(const void* q, int64_t q_stride, void* ou
 // half the softmax), the row's reference point is looked up in other lanes only when it moves, operand reads run
 // ahead of the products in a written order, and the two waves of a SIMD are half an interval apart. Measured on an MI355X, before
 // (tiles through registers, all waves in step) -> now: 2048 tokens of 12 heads of 128 on 2 behind 6144, 164 -> 117 us
-// (0.77 PFLOP/s on 206 compute units); of 28 on 4, 319 -> 233 (0.90); 2048 tokens without a prefix 43 -> 32.6; 137 tokens
-// 11.7 -> 9.1; 1000 tokens of 14 heads of 64 behind 7000, 69 -> 51; of 16 of 256 on 4 behind 4000, 218 -> 143.
+// (0.77 PFLOP/s on 196 compute units); of 28 on 4, 319 -> 222 (0.95; 233 with every wave's rows in whole tokens, 28 of 32 for
+// groups of 7); 2048 tokens without a prefix 43 -> 31; 137 tokens 11.7 -> 9.0; 1000 tokens of 14 heads of 64 behind 7000, 69 -> 50;
+// of 16 of 256 on 4 behind 4000, 218 -> 143.
 // RB: row blocks (waves that own 32 query rows each) of a workgroup, 4 or 2. With 2 the same eight
 // waves cut a stage's keys four ways instead of two: half the rows per workgroup and half the
 // time per stage, for launches whose portions would otherwise leave compute units without work
@@ -1069,7 +1070,6 @@ __device__ __forceinline__ void attn_prefill_of(const AttnParams& p, const int i
   const int kvh = y / p.n_chunks, chunk = y % p.n_chunks;
   const int req = p.items[4 * item], tok0 = p.items[4 * item + 1];
   const int gh = p.gh;
-  const int tpw = 32 / gh;  // tokens of a wave
   const int ctx = p.ctx_lens[req];
   const int q_begin = p.cu_q[req];
   const int qlen = p.cu_q[req + 1] - q_begin;
@@ -1144,10 +1144,10 @@ __device__ __forceinline__ void attn_prefill_of(const AttnParams& p, const int i
     }
   };
 
-  // ---- the wave's rows: block b, column c -> row b * 16 + c
-  const bool wave_on = wave * tpw < ntok;
-  const int p_first = pos0 + wave * tpw;
-  const int p_last = pos0 + min(ntok, (wave + 1) * tpw) - 1;
+  // ---- the wave's rows: block b, column c -> row wave * 32 + b * 16 + c of the workgroup, token row / gh, head row % gh
+  const bool wave_on = wave * 32 < ntok * gh;
+  const int p_first = pos0 + wave * 32 / gh;
+  const int p_last = pos0 + min(ntok - 1, (wave * 32 + 31) / gh);
   const int lo = p.window > 0 ? max(0, p_first - p.window + 1) : 0;
   int row_pos[2];  // position of the row's token, far below zero for an unused row
   bf16x8_t qf[2][NF];
@@ -1158,11 +1158,9 @@ __device__ __forceinline__ void attn_prefill_of(const AttnParams& p, const int i
   }
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    const int row = b * 16 + c;
-    const int tl = row / gh, g = row - tl * gh;
-    const int tokw = wave * tpw + tl;
-    const int hig = chunk * gh + g;
-    const bool ok = wave_on && tl < tpw && tokw < ntok && hig < group;
+    const int row = wave * 32 + b * 16 + c;
+    const int tokw = row / gh, hig = chunk * gh + row - tokw * gh;
+    const bool ok = tokw < ntok && hig < group;
     row_pos[b] = ok ? pos0 + tokw : INT_MIN / 2;
     const bf16_t* qrow = ok ? (const bf16_t*)p.q + (int64_t)(q_begin + tok0 + tokw) * p.q_stride + (kvh * group + hig) * HD : zrow;
 #pragma unroll
@@ -1420,7 +1418,7 @@ __device__ __forceinline__ void attn_prefill_of(const AttnParams& p, const int i
     float l = l_run[b];
     l = cw_quad_sum(l);
     if (row_pos[b] < 0) continue;
-    const int head = kvh * group + chunk * gh + (b * 16 + c) % gh;
+    const int head = kvh * group + chunk * gh + (wave * 32 + b * 16 + c) % gh;
     const int64_t token = q_begin + (row_pos[b] - (ctx - qlen));
     const float inv = attn_head_gate(p, token, head) / l;
     bf16_t* orow = (bf16_t*)p.out + token * p.out_stride + head * HD;
@@ -1482,7 +1480,7 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(AttnParams p) {
   const int item = blockIdx.x - part;  // the item's part 0
   const int kvh = blockIdx.y / p.n_chunks, chunk = blockIdx.y % p.n_chunks;
   const int req = p.items[4 * item], tok0 = p.items[4 * item + 1];
-  const int gh = p.gh, tpw = 32 / gh, group = p.nh / p.nkv;
+  const int gh = p.gh, group = p.nh / p.nkv;
   const int q_begin = p.cu_q[req];
   const int ntok = min(p.items[4 * item + 2], p.cu_q[req + 1] - q_begin - tok0);
   const float sl2 = p.scale * 1.4426950408889634f;
@@ -1506,10 +1504,8 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(AttnParams p) {
     const int pair = has ? u % n_pairs : 0, slice = has ? u / n_pairs : 0;
     const int r = pair / VEC, d = (pair - r * VEC) * 4;
     const int row = row0 + r;
-    const int wave = row >> 5, rr = row & 31;
-    const int tl = rr / gh, g = rr - tl * gh;
-    const int tokw = wave * tpw + tl, hig = chunk * gh + g;
-    const bool valid = has && row < ROWS && tl < tpw && tokw < ntok && hig < group;
+    const int tokw = row / gh, hig = chunk * gh + row - tokw * gh;
+    const bool valid = has && row < ROWS && tokw < ntok && hig < group;
     float m = -INFINITY, l = 0.0f;
     f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
     if (valid) {
@@ -1623,7 +1619,7 @@ static int prefill_params(AttnParams& p, const void* q, int64_t q_stride, void* 
 #endif
 
 // Portions of prompts, bfloat16. items: (request, first token, tokens, part | parts << 8) with
-// tokens <= row_blocks * (32 / gh), gh = min(group, 32) heads of a group per workgroup; tokens of
+// tokens <= row_blocks * 32 / gh, gh = min(group, 32) heads of a group per workgroup; tokens of
 // an item beyond that are not computed. row_blocks: 4, or 2 (see PrefillTile). An item with
 // parts > 1 stands ``parts`` times in the list, one after the other, as part 0, 1, ...: each takes
 // a share of the keys that its tokens see, and a second kernel puts the shares together. Any item

@@ -1306,7 +1306,7 @@ def prefill_row_blocks_ok(hd: int, row_blocks: int) -> bool:
 def prefill_tokens_per_item(group: int, row_blocks: int = 4) -> int:
     """Tokens one work item of ``attention_prefill`` may hold: a row block is 32 rows, a row a
     (token, head of the group) pair."""
-    return row_blocks * (32 // min(group, 32))
+    return row_blocks * 32 // min(group, 32)
 
 
 def decode_attention_supported(hd: int, dtype: torch.dtype) -> bool:

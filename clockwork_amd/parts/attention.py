@@ -144,18 +144,22 @@ def _make_plan(ctx, nh: int, nkv: int, narrow_ok: bool, whole_keys: int = 0, tog
     gh_single = min(group, 16)
     wide: list = []   # one array of items per portion
     mfma: list = []
-    # Workgroups of four row blocks share each key among the most rows, but a launch has to
-    # fill the compute units, and the workgroup with the longest key range decides its time: where
-    # they would leave a twentieth of the compute units or more idle, halve them, unless the key ranges are
-    # long (us, two row blocks / four: 206 workgroups of four, 2048 tokens of 12 heads on 2, 32.4 / 36.9; 240, 2400 tokens,
-    # 37.6 / 41.6; 252, 1000 tokens of 28 heads on 4, 29.9 / 24.4; 264, 1050 tokens, 32.8 / 25.9; 376, 1500 tokens, 48.8 / 42.5).
-    # Groups of more than 32 heads, whose last chunk leaves rows idle: from 1.5 workgroups a unit on (6 % either way).
-    tokens_of_four = 4 * (32 // min(group, 32))
+    # Workgroups of four row blocks share each key among the most rows, but the one with the longest key range
+    # decides the launch's time. Unless the key ranges are long, two row blocks are the faster way where their workgroups
+    # are at most one for every compute unit (us, two row blocks / four: 1024 tokens of 16 heads of 64 on 8, 256
+    # workgroups of two, 12.8 / 17.0); beyond, a second round of them costs their chain of first loads again, which pays
+    # for key ranges of ten stages and more (1800 tokens of 12 heads of 128 on 2, 360 of two, 26.5 / 33.1; 2500 tokens, 500,
+    # 40.4 / 43.4; 1000 tokens of 28 on 4, 448, 28.7 / 24.2; 640 of 32 on 8, 320, 22.1 / 18.3), while four would leave a
+    # twentieth of the units idle. Groups of more than 32 heads, whose last chunk leaves rows idle: up to 1.5
+    # workgroups of four a unit (6 % either way).
+    tokens_of_four = 4 * 32 // min(group, 32)
     workgroups = sum(-(-q // tokens_of_four) for q in ctx.h_q_lens if q > 1) * nkv * -(-group // 32)
     short_ranges = portions_have_short_ranges(ctx.h_q_lens, ctx.h_ctx_lens)
-    enough = 1.5 if group > 32 else 0.95
-    row_blocks = 2 if narrow_ok and short_ranges and workgroups < enough * ctx.num_compute_units else 4
-    tokens_per_mfma_item = row_blocks * (32 // min(group, 32))
+    longest = max((c for q, c in zip(ctx.h_q_lens, ctx.h_ctx_lens) if q > 1), default=0)
+    units = ctx.num_compute_units
+    two = 2 * workgroups <= units or (workgroups < 1.5 * units if group > 32 else longest >= 1280 and workgroups < 0.95 * units)
+    row_blocks = 2 if narrow_ok and short_ranges and two else 4
+    tokens_per_mfma_item = row_blocks * 32 // min(group, 32)
     single: list[int] = []
     longest_single = 0
 
