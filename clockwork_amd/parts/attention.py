@@ -57,8 +57,9 @@ def portions_have_short_ranges(q_lens, ctx_lens) -> bool:
     """The rule by which a step's portions (entries of more than one token) choose the shape of
     the matrix-core kernel's workgroups: True while their tokens see fewer than 3072 keys on
     average. Behind a long cached prefix every workgroup's key range is long and about the same,
-    and sharing the keys among more rows wins (2048 tokens of the 1.5B shape: 46 against 52 us
-    with no prefix, 94 against 96 us behind 2048 tokens, 197 against 182 us behind 6144)."""
+    and sharing the keys among more rows wins (2048 tokens of 12 heads of 128 on 2, us, two row blocks / four: no
+    prefix 31.8 / 36.9, behind 1024 tokens 49.4 / 50.5, 2048 68.0 / 64.0, 6144 142.7 / 118.1; 1000 tokens, whose
+    workgroups of four are 96, behind 2500 41.5 / 56.5, the keys not cut into parts)."""
     tokens = sum(q for q in q_lens if q > 1)
     keys = sum(q * (c - q / 2.0) for q, c in zip(q_lens, ctx_lens) if q > 1)
     return tokens > 0 and keys / tokens < LONG_RANGE_KEYS
@@ -133,7 +134,8 @@ def _share_the_card(plan: AttentionPlan, room: int, base: int) -> None:
 def whole_single_keys(head_dim: int) -> int:
     """Heads of up to 128 elements come with eight waves a workgroup, which take 512 keys in two turns: as
     long as the kernel that merges the parts of a request would take alone (us for one request, one part
-    against four: heads of 64, 120 keys 4.8 / 7.8, 500 keys 6.7 / 8.0; of 128, 6.3 / 9.5 and 9.7 / 9.5)."""
+    against two for 300 keys and three for 500: heads of 64 4.8 / 6.7 and 5.6 / 6.8; of 128, 7.0 / 7.9 and
+    8.7 / 8.0)."""
     return 512 if head_dim <= 128 else 0
 
 
