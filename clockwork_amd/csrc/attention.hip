@@ -498,16 +498,16 @@ __device__ __forceinline__ int v_granule(int k, int g) { return g ^ ((((k >> 1) 
 // 16 bytes a lane from memory to LDS, to 1 KB at ``to`` (the same for all lanes), lane by lane; from an address a lane, or
 // from one address for all and an offset a lane. Written out, because behind the builtin the compiler puts a wait for all
 // such loads before the next transposing read, of whatever tile: what the kernel waits for and where is its own to say.
-// (No register is written.)
+// (No vector register is written; m0, where the instruction finds the address in LDS, is.)
 __device__ __forceinline__ void load_to_lds(const void* from, void* to) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-               : : "v"(from), "s"((uint32_t)(uintptr_t)(lds_raw_t*)to) : "memory");
+               : : "v"(from), "s"((uint32_t)(uintptr_t)(lds_raw_t*)to) : "memory", "m0");
 }
 // (``OFFSET`` bytes further on at both ends: the instruction's own offset counts for the address in LDS as well)
 template <int OFFSET>
 __device__ __forceinline__ void load_to_lds(const void* from, void* to) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off offset:%2"
-               : : "v"(from), "s"((uint32_t)(uintptr_t)(lds_raw_t*)to), "n"(OFFSET) : "memory");
+               : : "v"(from), "s"((uint32_t)(uintptr_t)(lds_raw_t*)to), "n"(OFFSET) : "memory", "m0");
 }
 // The blocks of 32 elements of 16 rows, 64 bytes apart in memory and 1 KB in LDS.
 template <int... J>
@@ -516,7 +516,7 @@ __device__ __forceinline__ void row_to_lds(const void* from, unsigned char* to, 
 }
 __device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, void* to) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               : : "v"(offset), "s"(base), "s"((uint32_t)(uintptr_t)(lds_raw_t*)to) : "memory");
+               : : "v"(offset), "s"(base), "s"((uint32_t)(uintptr_t)(lds_raw_t*)to) : "memory", "m0");
 }
 
 // =====================================================================================

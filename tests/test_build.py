@@ -1,5 +1,7 @@
 """The HIP libraries: no execution path without them, and clear errors on the way to them."""
 
+import re
+
 import pytest
 
 from clockwork_amd import ops
@@ -46,3 +48,28 @@ def test_the_target_rules_xnack_out_unless_told_otherwise(monkeypatch):
     monkeypatch.setenv("CLOCKWORK_AMD_ARCH", "gfx950")
     assert build.target_arch() == "gfx950"
     assert "--offload-arch" not in " ".join(build.FLAGS)  # the target is added per compile
+
+
+def _assembly_statements(text: str):
+    """The inline assembly of a source, statement by statement."""
+    for found in re.finditer(r"\basm\s+(?:volatile\s*)?\(", text):
+        depth, at, quoted = 1, found.end(), False
+        while depth:
+            c = text[at]
+            if c == "\\":
+                at += 1
+            elif c == '"':
+                quoted = not quoted
+            elif not quoted:
+                depth += (c == "(") - (c == ")")
+            at += 1
+        yield text[found.start() : at]
+
+
+def test_inline_assembly_names_the_scalar_register_that_it_writes():
+    """The compiler keeps values in m0 of its own (LDS loads, lane writes, registers chosen at run time): a statement
+    that writes it has to say so."""
+    statements = [a for path in sorted(build.CSRC.glob("*.h*")) for a in _assembly_statements(path.read_text())]
+    writers = [a for a in statements if re.search(r"\bs_\w+ m0\b", a)]
+    assert len(statements) > len(writers) >= 3
+    assert [a for a in writers if '"m0"' not in a] == []
