@@ -874,10 +874,11 @@ CW_EXPORT int64_t cw_attention_decode_workspace_floats(int n_items, int nh, int 
 }
 
 #if CW_HAS_DECODE
-// The most pages of a split that are taken: what 160 KB hold beside the waves' outputs.
-static bool decode_pages_ok(int waves, int64_t pages) {
-  return sizeof(float) * waves * 16 * CW_HD + sizeof(int) * (size_t)pages <= 160 * 1024;
-}
+// The most pages of a split that are taken by this many waves: 160 KB less 16 rows of float32 a wave. (Pages beyond
+// what LDS holds beside the tiles are looked up in memory, so the kernel itself would take any number; four waves' bound is
+// what the entries refuse beyond, eight waves' where four take over.)
+static constexpr int64_t decode_pages_most(int waves) { return (160 * 1024 - (int64_t)sizeof(float) * waves * 16 * CW_HD) / (int64_t)sizeof(int); }
+static bool decode_pages_ok(int waves, int64_t pages) { return pages <= decode_pages_most(waves); }
 
 // Pages of a split that lie in LDS beside ``tiles`` bytes (and the waves' statistics): all of them, or -1.
 static int decode_pages_in_lds(size_t tiles, int64_t pages) {
@@ -1655,6 +1656,18 @@ CW_EXPORT int cw_attention_prefill_bf16(const void* q, int64_t q_stride, void* o
 // 1 if portions and single tokens of one step can run as one launch (see attn_together_bf16_kernel).
 CW_EXPORT int cw_attention_together_supported() { return CW_HAS_PREFILL && CW_HD <= 128 ? 1 : 0; }
 
+// The most keys that a split of cw_attention_together_bf16 takes with pages of this size, a multiple of 32 (0: there is no
+// such launch): what cw_attention_decode_bf16 takes, whose splits may be shorter.
+CW_EXPORT int cw_attention_together_split_keys(int block_size) {
+#if CW_HAS_PREFILL && CW_HD <= 128
+  if (block_size <= 0) return 0;
+  const int64_t keys = (decode_pages_most(4) - 2) * (int64_t)block_size;
+  return (int)((keys < INT_MAX ? keys : INT_MAX) & ~31);
+#else
+  return 0;
+#endif
+}
+
 // cw_attention_prefill_bf16 of ``portions`` (whole items, no parts) and cw_attention_decode_bf16 of ``singles`` in one
 // launch, then the merge of the single tokens' splits; the arguments are theirs.
 CW_EXPORT int cw_attention_together_bf16(const void* q, int64_t q_stride, void* out, int64_t out_stride, const void* k_cache,
@@ -1681,7 +1694,7 @@ CW_EXPORT int cw_attention_together_bf16(const void* q, int64_t q_stride, void* 
   const int64_t max_tiles = ((int64_t)table_stride * block_size + 31) / 32;
   const int64_t tiles_per_split = split_keys > 0 ? split_keys / 32 : (max_tiles + n_splits - 1) / n_splits;
   const int64_t pages = (tiles_per_split * 32 + block_size - 1) / block_size + 2;
-  if (!decode_pages_ok(8, pages)) return CW_ERR_SIZE;
+  if (!decode_pages_ok(4, pages)) return CW_ERR_SIZE;  // (eight waves here, but as many pages as the launch alone takes)
   constexpr size_t tiles = 8 * (size_t)DecodeTile<CW_HD>::BYTES;
   a.singles.decode_pages = decode_pages_in_lds(tiles, pages);
   const size_t for_singles = tiles + (a.singles.decode_pages > 0 ? sizeof(int) * (size_t)a.singles.decode_pages : 0);

@@ -242,6 +242,7 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_attention_prefill_bf16": [P, L, P, L, P, P, P, I, P, P, P, I, I, I, I, I, F, P, I, I, P, L, F, P, L, I, P],
             "cw_attention_prefill_workspace_floats": [I, I, I, I],
             "cw_attention_together_supported": [],
+            "cw_attention_together_split_keys": [I],
             "cw_attention_together_bf16": [P, L, P, L, P, P, P, I, P, P, P, I, I, P, I, I, I, I, I, I, I, I, F, P, L, P, P],
             "cw_attention_prefill_row_blocks_ok": [I],
             "cw_attention_decode_supported": [],
@@ -1371,6 +1372,12 @@ def attention_decode(q, q_stride: int, out, k_cache, v_cache, block_tables, ctx_
 
 def together_attention_supported(hd: int, dtype: torch.dtype) -> bool:
     return dtype == torch.bfloat16 and bool(_load("attention", hd).cw_attention_together_supported())
+
+
+def together_attention_split_keys(hd: int, dtype: torch.dtype, block_size: int) -> int:
+    """The most keys that a split of a single token may have in ``attention_together`` with pages of this size (0: no such
+    launch for these heads)."""
+    return int(_load("attention", hd).cw_attention_together_split_keys(block_size)) if together_attention_supported(hd, dtype) else 0
 
 
 def attention_together(q, q_stride: int, out, k_cache, v_cache, block_tables, ctx_lens, cu_q, portions, n_portions: int,

@@ -105,29 +105,36 @@ def _share_long_key_ranges(items: np.ndarray, ctx, workgroups_per_item: int):
     return out.astype(np.int32).reshape(-1), most
 
 
-def attention_plan(ctx, nh: int, nkv: int, narrow_ok: bool = False, whole_keys: int = 0, together_ok: bool = False) -> AttentionPlan:
+def attention_plan(ctx, nh: int, nkv: int, narrow_ok: bool = False, whole_keys: int = 0, together_ok: bool = False,
+                   together_split_keys: int = 0) -> AttentionPlan:
     """The step's work items for heads of this geometry, made once a step and kept in
     ``ctx.plans``. ``narrow_ok``: the matrix-core kernel for portions also comes with two row
     blocks a workgroup (see ``ops.prefill_row_blocks_ok``). ``whole_keys``: up to this many keys of a single
     token stay with one workgroup (see ``whole_single_keys``). ``together_ok``: the caller can run portions and single
-    tokens as one launch (see ``_share_the_card``)."""
+    tokens as one launch (see ``_share_the_card``), whose splits take ``together_split_keys`` keys at most (0: any)."""
     # a batch of single tokens has no portions: one plan, whatever the kernel for portions offers
     narrow_ok = bool(narrow_ok) and any(q > 1 for q in ctx.h_q_lens)
-    key = ("attention", nh, nkv, narrow_ok, whole_keys, together_ok)
+    key = ("attention", nh, nkv, narrow_ok, whole_keys, together_ok, together_split_keys)
     plan = ctx.plans.get(key)
     if plan is None:
-        plan = ctx.plans[key] = _make_plan(ctx, nh, nkv, narrow_ok, whole_keys, together_ok)
+        plan = ctx.plans[key] = _make_plan(ctx, nh, nkv, narrow_ok, whole_keys, together_ok, together_split_keys)
     return plan
 
 
-def _share_the_card(plan: AttentionPlan, room: int, base: int) -> None:
+def _split_keys(longest: int, splits: int) -> int:
+    """Keys of each of ``splits`` fixed places that cover ``longest`` keys: a multiple of 32."""
+    return 32 * -(-(-(-longest // splits)) // 32)
+
+
+def _share_the_card(plan: AttentionPlan, room: int, base: int, longest: int, most_keys: int) -> None:
     """One launch for a step's portions and single tokens, where all workgroups of both are at work at once: ``room``
     compute units are left beside the portions' workgroups, a split of every single token takes ``base`` of them. The splits
     are then as many as fit, but not fewer than half of those that the single tokens alone would be cut into: where the
     portions take nearly the whole card, a few long splits would outlast both launches (a step of 15
-    requests of 1500 keys beside 300 tokens, 1.5B shape: 3.30 ms with 8 splits behind the portions, 3.04 with 6 beside them)."""
+    requests of 1500 keys beside 300 tokens, 1.5B shape: 3.30 ms with 8 splits behind the portions, 3.04 with 6 beside them). A split of more than ``most_keys`` keys
+    (of the ``longest`` context) has more pages than the launch takes: two launches then, whose splits are shorter."""
     splits = min(room // base, plan.decode_splits)
-    if splits >= 1 and 2 * splits >= plan.decode_splits:
+    if splits >= 1 and 2 * splits >= plan.decode_splits and not 0 < most_keys < _split_keys(longest, splits):
         plan.together, plan.decode_splits = True, splits
 
 
@@ -139,7 +146,8 @@ def whole_single_keys(head_dim: int) -> int:
     return 512 if head_dim <= 128 else 0
 
 
-def _make_plan(ctx, nh: int, nkv: int, narrow_ok: bool, whole_keys: int = 0, together_ok: bool = False) -> AttentionPlan:
+def _make_plan(ctx, nh: int, nkv: int, narrow_ok: bool, whole_keys: int = 0, together_ok: bool = False,
+               together_split_keys: int = 0) -> AttentionPlan:
     group = nh // nkv
     gh_wide = min(group, 64)
     tokens_per_tile = 64 // gh_wide
@@ -212,10 +220,10 @@ def _make_plan(ctx, nh: int, nkv: int, narrow_ok: bool, whole_keys: int = 0, tog
         plan.decode_splits = 1 if longest_single <= whole_keys else max(
             1, min(ctx.num_compute_units // base, longest_single // 128, 64))
         if together_ok and plan.n_mfma and plan.mfma_parts == 1:
-            _share_the_card(plan, ctx.num_compute_units - plan.n_mfma * nkv * -(-group // 32), base)
+            _share_the_card(plan, ctx.num_compute_units - plan.n_mfma * nkv * -(-group // 32), base, longest_single, together_split_keys)
         # fixed places for the splits: a workgroup then knows its pages before it knows the
         # request's length, which saves it a trip to memory
-        plan.decode_split_keys = 32 * -(-(-(-longest_single // plan.decode_splits)) // 32)
+        plan.decode_split_keys = _split_keys(longest_single, plan.decode_splits)
         plan.decode_max_ctx = longest_single
         plan.single_identity = plan.n_single == len(ctx.h_q_lens)
     plan.wide_items, plan.single_items, plan.mfma_items = ctx.upload([wide, single, mfma])
@@ -256,8 +264,9 @@ class PagedAttention(Part):
     def _plan(self, ctx, dtype) -> AttentionPlan:
         hd = self.spec.head_dim
         narrow_ok = ops.prefill_attention_supported(hd, dtype) and ops.prefill_row_blocks_ok(hd, 2)
+        together_keys = ops.together_attention_split_keys(hd, dtype, ctx.block_size)
         return attention_plan(ctx, self.spec.num_heads, self.spec.num_kv_heads, narrow_ok=narrow_ok,
-                              whole_keys=whole_single_keys(hd), together_ok=ops.together_attention_supported(hd, dtype))
+                              whole_keys=whole_single_keys(hd), together_ok=together_keys > 0, together_split_keys=together_keys)
 
     def prepare(self, ctx) -> None:
         """The step's work items, before ``forward`` (a captured step must not make them)."""

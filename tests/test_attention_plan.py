@@ -1,13 +1,17 @@
 """The attention part's planning of work items, on the CPU (no kernel runs)."""
 
 import numpy as np
+import pytest
+import torch
 
-from clockwork_amd.parts.attention import MAX_PARTS, MIN_PART_KEYS, _share_long_key_ranges, portions_have_short_ranges
+from clockwork_amd import ops
+from clockwork_amd.parts.attention import MAX_PARTS, MIN_PART_KEYS, _share_long_key_ranges, attention_plan, portions_have_short_ranges
 
 
 class _Step:
     def __init__(self, q_lens, ctx_lens, num_compute_units=256):
         self.h_q_lens, self.h_ctx_lens, self.num_compute_units = list(q_lens), list(ctx_lens), num_compute_units
+        self.plans, self.upload = {}, lambda arrays: [np.asarray(a, dtype=np.int32) for a in arrays]
 
 
 def _items(q_lens, tokens_per_item):
@@ -67,3 +71,27 @@ def test_short_and_long_key_ranges():
     assert portions_have_short_ranges([2048], [2048])
     assert not portions_have_short_ranges([2048], [8192])
     assert not portions_have_short_ranges([1, 1], [500, 600])  # no portion at all
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("block_size", [1, 3, 16])
+@pytest.mark.parametrize("requests,keys", [(60, 50000), (60, 32736), (60, 32737), (16, 300000), (15, 1500)])
+def test_one_launch_is_planned_only_where_it_takes_a_splits_pages(hd, block_size, requests, keys):
+    """60 requests of 50,000 keys in pages of one key beside a portion of 64 tokens: a split of the one launch would have more
+    pages than it takes, while two launches take the step (with splits of their own length)."""
+    most = ops.together_attention_split_keys(hd, torch.bfloat16, block_size)
+    assert most % 32 == 0 and most // block_size >= 32000
+    how = dict(narrow_ok=True, whole_keys=512)
+    plan = attention_plan(_Step([1] * requests + [64], [keys] * requests + [64]), 12, 2, together_ok=True, together_split_keys=most, **how)
+    apart = attention_plan(_Step([1] * requests + [64], [keys] * requests + [64]), 12, 2, **how)
+    free = attention_plan(_Step([1] * requests + [64], [keys] * requests + [64]), 12, 2, together_ok=True, **how)
+    if plan.together:
+        assert plan.decode_split_keys <= most and plan.decode_splits == free.decode_splits
+    else:
+        assert (plan.decode_splits, plan.decode_split_keys) == (apart.decode_splits, apart.decode_split_keys) and free.decode_split_keys > most
+    assert plan.together == (free.decode_split_keys <= most) and plan.decode_split_keys * plan.decode_splits >= keys
+
+
+def test_heads_without_the_one_launch_have_no_keys_for_it():
+    assert ops.together_attention_split_keys(256, torch.bfloat16, 16) == 0 == ops.together_attention_split_keys(48, torch.bfloat16, 16)
+    assert ops.together_attention_split_keys(128, torch.float32, 16) == 0 == ops.together_attention_split_keys(128, torch.bfloat16, 0)

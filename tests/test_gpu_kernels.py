@@ -1202,6 +1202,38 @@ def test_portions_and_single_tokens_in_one_launch(nh, nkv, hd, bs, window, row_b
                 assert (a - b).norm() <= 2.0 ** -8 * a.norm()
 
 
+@pytest.mark.parametrize("keys", [24640, 32736, 32768])
+def test_portions_and_single_tokens_in_one_launch_with_pages_of_one_key(keys):
+    """More pages in a split than the launch of eight waves alone takes (24,574) but not more than that of four does
+    (32,766): the one launch takes them as the two do, and refuses one more multiple of 32. Portions are the same bits; single
+    tokens add the same terms in another order (float32 sums, one rounding to bfloat16: 2^-8)."""
+    from clockwork_amd import ops
+
+    nh, nkv, hd = 12, 2, 128
+    kc, vc = (torch.randn(keys + 50, nkv, hd, device=DEV).to(torch.bfloat16) for _ in range(2))
+    bt = torch.full((2, keys), -1, dtype=torch.int32, device=DEV)
+    order = torch.randperm(keys + 50, device=DEV).int()
+    bt[0], bt[1, :40] = order[:keys], order[keys : keys + 40]
+    cl, cu = torch.tensor([keys, 40], dtype=torch.int32, device=DEV), torch.tensor([0, 1, 41], dtype=torch.int32, device=DEV)
+    p_items = torch.tensor([[1, t, min(20, 40 - t), 0] for t in (0, 20)], dtype=torch.int32, device=DEV).reshape(-1)
+    s_items = torch.tensor([0, 0, 1, 0], dtype=torch.int32, device=DEV)
+    q = torch.randn(41, nh * hd, device=DEV).to(torch.bfloat16)
+    common = dict(q=q, q_stride=nh * hd, k_cache=kc, v_cache=vc, block_tables=bt, ctx_lens=cl, cu_q=cu, nh=nh, nkv=nkv, hd=hd,
+                  block_size=1, window=0, scale=hd ** -0.5, n_tokens=41, n_requests=2)
+    split = dict(n_splits=1, split_keys=keys, max_ctx=keys)
+    one, two = (torch.full((41, nh * hd), -77.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    together = lambda: ops.attention_together(out=one, portions=p_items, n_portions=2, row_blocks=4, singles=s_items, n_singles=1, **split, **common)  # noqa: E731
+    if keys > ops.together_attention_split_keys(hd, torch.bfloat16, 1):
+        with pytest.raises(ops.KernelError):
+            together()
+        return
+    together()
+    ops.attention_prefill(out=two, items=p_items, n_items=2, row_blocks=4, **common)
+    ops.attention_decode(out=two, items=s_items, n_items=1, **split, **common)
+    assert torch.equal(one[1:], two[1:])
+    assert (one[0].double() - two[0].double()).norm() <= 2.0 ** -8 * two[0].double().norm() and bool(torch.isfinite(one.float()).all())
+
+
 def test_the_plan_puts_portions_and_single_tokens_together():
     """One launch where both kinds' workgroups fit the card side by side and the single tokens keep half of their splits;
     two where the portions' key ranges are in parts, or fill the card."""
