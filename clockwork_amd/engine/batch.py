@@ -80,6 +80,7 @@ class StepContext:
         self.plans: dict = {}     # what parts have planned for this step, under keys of their own
         self._pinned: list = []   # host buffers of the plans' uploads, alive as long as the step
         self.num_compute_units = 256
+        self.captured = False     # a captured step's batch: planned for all steps of its class
         self.products = None      # the engine's ops.ProductPolicy (None: the defaults)
 
     def upload(self, arrays) -> list:
@@ -357,6 +358,7 @@ class StaticPortionBatch:
         ctx.h_q_lens = [n]
         ctx.h_ctx_lens = [typical_start + n]
         ctx.h_starts = [typical_start]
+        ctx.captured = True
         ctx.h_state_slots = [manager.idle_state_slot]
         ctx.seq_ids = [""]
         ctx.num_compute_units = num_compute_units
@@ -468,6 +470,7 @@ class StaticMixedBatch:
         ctx.h_q_lens = [1] * decoders + [portion]
         ctx.h_ctx_lens = [key_capacity] * decoders + [typical_start + portion]
         ctx.h_starts = [0] * decoders + [typical_start]
+        ctx.captured = True
         ctx.h_state_slots = [manager.idle_state_slot] * requests
         ctx.seq_ids = [""] * requests
         ctx.num_compute_units = num_compute_units

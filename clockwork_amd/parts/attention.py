@@ -8,7 +8,10 @@ portions and single tokens in the same step; output product.
 
 from __future__ import annotations
 
+import math
 from dataclasses import dataclass
+from functools import lru_cache
+from types import SimpleNamespace
 from typing import Optional
 
 import numpy as np
@@ -105,19 +108,50 @@ def _share_long_key_ranges(items: np.ndarray, ctx, workgroups_per_item: int):
     return out.astype(np.int32).reshape(-1), most
 
 
+def typical_start(start: int) -> int:
+    """Where the portions that one captured step serves are taken to begin when it is planned: nowhere behind cached
+    keys, or behind the nearest power of two of them, from 512 on. (How many parts a portion's keys are cut into follows
+    their number, and a captured step for each number would be one for each request: with a power of two the parts are
+    at most 1.4 times too long or too short, and they stop growing where they fill the card.)"""
+    near = 1 << round(math.log2(start)) if start > 0 else 0
+    return near if near >= 512 else 0
+
+
+def _as_captured(step):
+    """``step`` as a captured step is planned: every portion where the portions of its kind begin."""
+    return SimpleNamespace(h_q_lens=step.h_q_lens, num_compute_units=step.num_compute_units, upload=step.upload,
+                           h_ctx_lens=[c if q == 1 else q + typical_start(c - q) for q, c in zip(step.h_q_lens, step.h_ctx_lens)])
+
+
+@lru_cache(maxsize=4096)
+def captured_choices(q_lens: tuple, ctx_lens: tuple, nh: int, nkv: int, units: int, mfma: bool, narrow_ok: bool, whole_keys: int,
+                     together_ok: bool) -> tuple:
+    """What the plan of a captured step decides by its portions' cached keys: steps of the same tokens and the same choices
+    have the same plan. ``mfma``: the portions run on the bfloat16 matrix-core kernel."""
+    step = SimpleNamespace(h_q_lens=q_lens, h_ctx_lens=ctx_lens, num_compute_units=units, upload=lambda arrays: arrays)
+    plan = _make_plan(_as_captured(step), nh, nkv, narrow_ok and any(q > 1 for q in q_lens), whole_keys, together_ok)
+    if not mfma:
+        return ("parts", plan.wide_splits)
+    parts = np.maximum(np.asarray(plan.mfma_items).reshape(-1, 4)[:, 3] >> 8, 1)
+    edges = np.flatnonzero(np.diff(parts, prepend=0))  # runs of items of the same number of parts
+    return (plan.mfma_row_blocks, plan.together, plan.decode_splits, tuple(zip(edges.tolist(), parts[edges].tolist())))
+
+
 def attention_plan(ctx, nh: int, nkv: int, narrow_ok: bool = False, whole_keys: int = 0, together_ok: bool = False,
-                   together_split_keys: int = 0) -> AttentionPlan:
+                   together_split_keys: int = 0, captured: bool = False) -> AttentionPlan:
     """The step's work items for heads of this geometry, made once a step and kept in
     ``ctx.plans``. ``narrow_ok``: the matrix-core kernel for portions also comes with two row
     blocks a workgroup (see ``ops.prefill_row_blocks_ok``). ``whole_keys``: up to this many keys of a single
     token stay with one workgroup (see ``whole_single_keys``). ``together_ok``: the caller can run portions and single
-    tokens as one launch (see ``_share_the_card``), whose splits take ``together_split_keys`` keys at most (0: any)."""
+    tokens as one launch (see ``_share_the_card``), whose splits take ``together_split_keys`` keys at most (0: any).
+    ``captured``: the plan is for all steps of the same ``captured_choices``, not for this one's portions alone."""
     # a batch of single tokens has no portions: one plan, whatever the kernel for portions offers
     narrow_ok = bool(narrow_ok) and any(q > 1 for q in ctx.h_q_lens)
-    key = ("attention", nh, nkv, narrow_ok, whole_keys, together_ok, together_split_keys)
+    key = ("attention", nh, nkv, narrow_ok, whole_keys, together_ok, together_split_keys, captured)
     plan = ctx.plans.get(key)
     if plan is None:
-        plan = ctx.plans[key] = _make_plan(ctx, nh, nkv, narrow_ok, whole_keys, together_ok, together_split_keys)
+        plan = ctx.plans[key] = _make_plan(_as_captured(ctx) if captured else ctx, nh, nkv, narrow_ok, whole_keys, together_ok,
+                                           together_split_keys)
     return plan
 
 
@@ -231,6 +265,9 @@ def _make_plan(ctx, nh: int, nkv: int, narrow_ok: bool, whole_keys: int = 0, tog
 
 
 class PagedAttention(Part):
+    compute_units = 256  # of the card that the part is bound to
+    _choices = None      # what ``captured_choices`` takes beside the step, the same for every step
+
     @property
     def graph_safe(self) -> bool:
         """A fixed sequence of launches if the position encoding is one too."""
@@ -265,18 +302,24 @@ class PagedAttention(Part):
         hd = self.spec.head_dim
         narrow_ok = ops.prefill_attention_supported(hd, dtype) and ops.prefill_row_blocks_ok(hd, 2)
         together_keys = ops.together_attention_split_keys(hd, dtype, ctx.block_size)
-        return attention_plan(ctx, self.spec.num_heads, self.spec.num_kv_heads, narrow_ok=narrow_ok,
-                              whole_keys=whole_single_keys(hd), together_ok=together_keys > 0, together_split_keys=together_keys)
+        return attention_plan(ctx, self.spec.num_heads, self.spec.num_kv_heads, narrow_ok=narrow_ok, whole_keys=whole_single_keys(hd),
+                              together_ok=together_keys > 0, together_split_keys=together_keys, captured=ctx.captured)
 
     def prepare(self, ctx) -> None:
         """The step's work items, before ``forward`` (a captured step must not make them)."""
         self._plan(ctx, self.dtype)
 
     def shape_class(self, q_lens, ctx_lens):
-        """Portions behind a long cached prefix run another workgroup shape than early ones."""
+        """Portions behind few and many cached keys run other workgroups, cut their keys into other numbers of parts and
+        leave the single tokens another share of the card: what of that the plan of a captured step decides."""
         if not any(q > 1 for q in q_lens):
             return "single tokens"
-        return "short key ranges" if portions_have_short_ranges(q_lens, ctx_lens) else "long key ranges"
+        if self._choices is None:
+            nh, nkv, hd = self.spec.num_heads, self.spec.num_kv_heads, self.spec.head_dim
+            mfma = ops.prefill_attention_supported(hd, self.dtype)
+            self._choices = (nh, nkv, self.compute_units, mfma, mfma and ops.prefill_row_blocks_ok(hd, 2), whole_single_keys(hd),
+                             ops.together_attention_supported(hd, self.dtype))
+        return captured_choices(tuple(q_lens), tuple(ctx_lens), *self._choices)
 
     def bind(self, params, device, dtype) -> None:
         self.qkv_weight = params["qkv_weight"]
@@ -284,6 +327,9 @@ class PagedAttention(Part):
         self.out_weight = params["out_weight"]
         self.out_bias = params.get("out_bias")
         self.dtype = dtype
+        self._choices = None
+        if torch.device(device).type == "cuda":
+            self.compute_units = ops._compute_units(device)
         self.position.bind({}, device, dtype)
 
     def forward(self, x: torch.Tensor, ctx, cache: EntryCache) -> torch.Tensor:

@@ -5,13 +5,14 @@ import pytest
 import torch
 
 from clockwork_amd import ops
-from clockwork_amd.parts.attention import MAX_PARTS, MIN_PART_KEYS, _share_long_key_ranges, attention_plan, portions_have_short_ranges
+from clockwork_amd.parts.attention import MAX_PARTS, MIN_PART_KEYS, PagedAttention, _share_long_key_ranges, attention_plan, portions_have_short_ranges, typical_start
+from clockwork_amd.parts.specs import AttentionSpec
 
 
 class _Step:
     def __init__(self, q_lens, ctx_lens, num_compute_units=256):
         self.h_q_lens, self.h_ctx_lens, self.num_compute_units = list(q_lens), list(ctx_lens), num_compute_units
-        self.plans, self.upload = {}, lambda arrays: [np.asarray(a, dtype=np.int32) for a in arrays]
+        self.block_size, self.captured, self.plans, self.upload = 16, False, {}, lambda arrays: [np.asarray(a, dtype=np.int32) for a in arrays]
 
 
 def _items(q_lens, tokens_per_item):
@@ -95,3 +96,38 @@ def test_one_launch_is_planned_only_where_it_takes_a_splits_pages(hd, block_size
 def test_heads_without_the_one_launch_have_no_keys_for_it():
     assert ops.together_attention_split_keys(256, torch.bfloat16, 16) == 0 == ops.together_attention_split_keys(48, torch.bfloat16, 16)
     assert ops.together_attention_split_keys(128, torch.float32, 16) == 0 == ops.together_attention_split_keys(128, torch.bfloat16, 0)
+
+
+def _captured_plan(part, q_lens, ctx_lens):
+    step = _Step(q_lens, ctx_lens)
+    step.captured = True
+    plan = part._plan(step, part.dtype)
+    if ops.prefill_attention_supported(part.spec.head_dim, part.dtype):  # the fields that this type's kernels read
+        return (plan.n_mfma, plan.mfma_row_blocks, plan.mfma_parts, plan.mfma_items.tobytes(), plan.n_single, plan.single_items.tobytes(),
+                plan.decode_splits, plan.decode_split_keys, plan.decode_max_ctx, plan.single_identity, plan.together)
+    return (plan.n_wide, plan.wide_splits, plan.wide_items.tobytes(), plan.n_single, plan.single_items.tobytes(), plan.single_splits)
+
+
+@pytest.mark.parametrize("nh,nkv,hd,dtype", [(12, 2, 128, torch.bfloat16), (14, 2, 64, torch.bfloat16), (28, 4, 128, torch.bfloat16),
+                                             (40, 1, 64, torch.bfloat16), (16, 4, 256, torch.bfloat16), (14, 2, 64, torch.float32)])
+def test_captured_steps_of_one_class_have_one_plan(nh, nkv, hd, dtype):
+    """A captured step is kept under its token counts, the decoding requests' context and its class, and serves whatever
+    portion comes under the same: where the first one began must not decide how the others run. Portions behind 0 to 12,000
+    cached keys, alone and beside single tokens: one plan for each class, and few classes."""
+    part = PagedAttention(AttentionSpec(hidden_size=nh * hd, num_heads=nh, num_kv_heads=nkv, head_dim=hd, qkv_bias=False, out_bias=False,
+                                        scale=hd ** -0.5))
+    part.dtype = dtype
+    starts = [*range(0, 1200, 40), *range(1200, 4000, 190), *range(4000, 12000, 900)]
+    for decoders, capacity in ((0, 0), (1, 512), (16, 2048), (64, 1024)):
+        for size in (12, 60, 160, 320, 512, 1000, 2048):
+            plans = {}
+            for start in starts:
+                q_lens, ctx_lens = [1] * decoders + [size], [capacity] * decoders + [start + size]
+                plans.setdefault(part.shape_class(q_lens, ctx_lens), set()).add(_captured_plan(part, q_lens, ctx_lens))
+            assert all(len(of) == 1 for of in plans.values()), (decoders, size, {k: len(v) for k, v in plans.items()})
+            assert len(plans) <= 6, (decoders, size, len(plans))
+
+
+def test_portions_of_a_captured_step_begin_near_those_that_it_serves():
+    assert [typical_start(s) for s in (0, 1, 300, 362, 363, 512, 724, 725, 7000, 10000)] == [0, 0, 0, 0, 512, 512, 512, 1024, 8192, 8192]
+    assert all(s / 1.42 < typical_start(s) < 1.42 * s for s in range(363, 40000, 77))
