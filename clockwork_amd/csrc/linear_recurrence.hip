@@ -434,7 +434,7 @@ struct SegParams {
   const int* seg_items;   // [n_segments, 4]: request, first token of the segment (in the portion), tokens, index of the segment in its request
   const int* req_first;   // [R + 1]: first segment of each request in seg_items
   float* dec;             // [T, heads * dim] decays
-  float* qf;              // [T, heads * dim]
+  float* qf;              // [T, heads * dim] (the walks only, as kf and raw)
   float* kf;              // [T, heads * dim]
   float* added;           // [n_segments, heads, dim, vdim]
   float* seg_decay;       // [n_segments, heads, dim]
@@ -1079,10 +1079,16 @@ CW_EXPORT int cw_linear_recurrence_segments_supported(int dim, int vdim) {
   return dim > 0 && dim <= LRS_MAX_DIM && dim % 4 == 0 && vdim > 0 ? 1 : 0;
 }
 
-// floats of workspace: dec, qf, kf [T, heads * dim] each, added [segments, heads, dim, vdim],
-// seg_decay [segments, heads, dim], raw [T, heads * vdim]
-CW_EXPORT int64_t cw_linear_recurrence_segments_workspace_floats(int n_tokens, int n_segments, int heads, int dim, int vdim) {
-  return 3 * (int64_t)n_tokens * heads * dim + (int64_t)n_segments * heads * dim * (vdim + 1) + (int64_t)n_tokens * heads * vdim;
+// Do the matrix cores take segments of up to seg_tokens tokens of these sizes whole?
+static bool lrs_takes_mfma(int seg_tokens, int dim, int vdim) {
+  return seg_tokens <= LRS_MFMA_SEG && (dim == 16 || dim == 32 || dim == 64 || dim == 128) && vdim % 16 == 0 && vdim <= 256;
+}
+
+// floats of workspace: dec [T, heads * dim], added [segments, heads, dim, vdim] and seg_decay [segments, heads, dim], and for
+// the walks qf, kf [T, heads * dim] each and raw [T, heads * vdim]
+CW_EXPORT int64_t cw_linear_recurrence_segments_workspace_floats(int n_tokens, int n_segments, int heads, int dim, int vdim, int seg_tokens) {
+  const int64_t both = (int64_t)n_tokens * heads * dim + (int64_t)n_segments * heads * dim * (vdim + 1);
+  return lrs_takes_mfma(seg_tokens, dim, vdim) ? both : both + (int64_t)n_tokens * heads * (2 * dim + vdim);
 }
 
 CW_EXPORT int cw_linear_recurrence_segments(int dtype, const void* proj, int64_t stride, int q_off, int k_off, int v_off,
@@ -1115,10 +1121,12 @@ CW_EXPORT int cw_linear_recurrence_segments(int dtype, const void* proj, int64_t
   p.q_scale = q_scale; p.inv_tau = inv_tau; p.eps = eps;
   p.form = LinRecForm{decay_kind, bonus, norm_w_stride, u, u_stride, (int)state_stride};
   const int64_t THD = (int64_t)n_tokens * heads * dim;
-  p.dec = workspace; p.qf = p.dec + THD; p.kf = p.qf + THD;
-  p.added = p.kf + THD;
+  const bool mfma = lrs_takes_mfma(seg_tokens, dim, vdim);
+  p.dec = workspace; p.added = p.dec + THD;
   p.seg_decay = p.added + (int64_t)n_segments * heads * dim * vdim;
-  p.raw = p.seg_decay + (int64_t)n_segments * heads * dim;
+  p.qf = mfma ? nullptr : p.seg_decay + (int64_t)n_segments * heads * dim;
+  p.kf = mfma ? nullptr : p.qf + THD;
+  p.raw = mfma ? nullptr : p.kf + THD;
   int64_t pb = (THD + 255) / 256;
   if (pb > 65536) pb = 65536;
   p.seg_tokens = seg_tokens;
@@ -1127,8 +1135,7 @@ CW_EXPORT int cw_linear_recurrence_segments(int dtype, const void* proj, int64_t
   const size_t walk_lds = (size_t)3 * seg_tokens * dim * sizeof(float);
   const dim3 carry_grid(n_requests, heads, (unsigned)(((int64_t)dim * vdim + 255) / 256));
   const unsigned finish_blocks = (unsigned)(((int64_t)n_tokens * heads + 3) / 4);
-  // segments that the matrix cores take whole
-  if (seg_tokens <= LRS_MFMA_SEG && (dim == 16 || dim == 32 || dim == 64 || dim == 128) && vdim % 16 == 0 && vdim <= 256) {
+  if (mfma) {
 #define CW_MFMA(T_)                                                                       \
   do {                                                                                    \
     if (dim == 16) lrs_launch_mfma<T_, 16>(p, n_segments, carry_grid, stream);            \

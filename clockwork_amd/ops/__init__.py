@@ -222,7 +222,7 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_linear_recurrence_supported": [I, I],
             "cw_linear_recurrence": [I, P, L, I, I, I, I, I, P, P, P, P, I, P, P, P, I, I, I, I, I, F, F, F, I, P, I, P, L, L, P],
             "cw_linear_recurrence_segments_supported": [I, I],
-            "cw_linear_recurrence_segments_workspace_floats": [I, I, I, I, I],
+            "cw_linear_recurrence_segments_workspace_floats": [I, I, I, I, I, I],
             "cw_linear_recurrence_segments": [I, P, L, I, I, I, I, I, P, P, P, P, I, P, P, P, I, I, P, P, P, I, I, I, I, I, I,
                                               F, F, F, I, P, I, P, L, L, P],
         },
@@ -1807,7 +1807,7 @@ def linear_recurrence_segments(proj, q_off: int, k_off: int, v_off: int, g_off: 
     _i32(seg_items, 4 * n_segments, "seg_items")
     _i32(req_first, n_requests + 1, "req_first")
     lib = _load("linear_recurrence")
-    need = lib.cw_linear_recurrence_segments_workspace_floats(T, n_segments, heads, dim, vdim)
+    need = lib.cw_linear_recurrence_segments_workspace_floats(T, n_segments, heads, dim, vdim, int(seg_tokens))
     workspace = torch.empty(max(int(need), 1), dtype=torch.float32, device=proj.device)
     out = torch.empty((T, heads * vdim), dtype=proj.dtype, device=proj.device)
     _check(lib.cw_linear_recurrence_segments(

@@ -236,3 +236,16 @@ def test_a_workspace_that_is_not_aligned_is_refused_before_any_launch():
         return lib.cw_sink_decode(0, 64, 128, 64, 64, 64, 32, 64, 2, 64, 64, 1, 32, 1, workspace, None, None, None, None, 4, 2, 32, 32, 16, 0, 1.0, None)
 
     assert call(4) == -1 and call(12) == -1
+
+
+@pytest.mark.parametrize("dim,vdim,seg_tokens,matrix_cores", [
+    (64, 128, 32, True), (16, 16, 32, True), (128, 256, 1, True),
+    (64, 128, 33, False), (48, 128, 32, False), (64, 120, 32, False), (128, 272, 32, False)])
+def test_long_portions_of_the_recurrence_ask_for_the_workspace_that_they_use(dim, vdim, seg_tokens, matrix_cores):
+    """Decays, what every segment adds and its decay; the walks keep float32 queries, keys and raw outputs beside them."""
+    from clockwork_amd import ops
+
+    T, segments, heads = 2048, 64, 12
+    floats = ops._load("linear_recurrence").cw_linear_recurrence_segments_workspace_floats(T, segments, heads, dim, vdim, seg_tokens)
+    used = T * heads * dim + segments * heads * dim * (vdim + 1)
+    assert floats == used + (0 if matrix_cores else T * heads * (2 * dim + vdim))
