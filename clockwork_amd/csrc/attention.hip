@@ -880,9 +880,12 @@ CW_EXPORT int64_t cw_attention_decode_workspace_floats(int n_items, int nh, int 
 static constexpr int64_t decode_pages_most(int waves) { return (160 * 1024 - (int64_t)sizeof(float) * waves * 16 * CW_HD) / (int64_t)sizeof(int); }
 static bool decode_pages_ok(int waves, int64_t pages) { return pages <= decode_pages_most(waves); }
 
-// Pages of a split that lie in LDS beside ``tiles`` bytes (and the waves' statistics): all of them, or -1.
+// Dynamic LDS of a workgroup of single tokens at most: 160 KB less the waves' statistics.
+#define DEC_MOST_LDS (158 * 1024)
+
+// Pages of a split that lie in LDS beside ``tiles`` bytes: all of them, or -1.
 static int decode_pages_in_lds(size_t tiles, int64_t pages) {
-  return tiles + sizeof(int) * (size_t)pages <= 158 * 1024 ? (int)pages : -1;
+  return tiles + sizeof(int) * (size_t)pages <= DEC_MOST_LDS ? (int)pages : -1;
 }
 
 static void launch_decode_merge(const AttnParams& p, int n_items, hipStream_t stream) {
@@ -907,15 +910,11 @@ static int launch_decode_of(AttnParams& p, int n_items, hipStream_t stream) {
   const int64_t pages = (tiles_per_split * 32 + p.block_size - 1) / p.block_size + 2;
   if (!decode_pages_ok(WAVES, pages)) return CW_ERR_SIZE;
   constexpr size_t tiles = (size_t)WAVES * DecodeTile<HD>::BYTES;
+  static_assert(tiles <= DEC_MOST_LDS, "the waves' tiles fit LDS");
   p.decode_pages = decode_pages_in_lds(tiles, pages);
   const size_t smem = tiles + (p.decode_pages > 0 ? sizeof(int) * (size_t)p.decode_pages : 0);
-  static size_t raised = 0;
-  if (smem > raised) {
-    if (hipFuncSetAttribute((const void*)attn_decode_bf16_kernel<HD, POW2, WAVES, CAP>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
-      return CW_ERR_LAUNCH;
-    raised = smem;
-  }
+  static std::atomic<bool> allowed{false};
+  if (cw_allow_lds(allowed, (const void*)attn_decode_bf16_kernel<HD, POW2, WAVES, CAP>, DEC_MOST_LDS) != CW_OK) return CW_ERR_LAUNCH;
   dim3 grid(n_items, p.nkv * p.n_chunks, p.n_splits), block(WAVES * 64);
   hipLaunchKernelGGL((attn_decode_bf16_kernel<HD, POW2, WAVES, CAP>), grid, block, smem, stream, p);
   launch_decode_merge(p, n_items, stream);
@@ -1702,14 +1701,9 @@ CW_EXPORT int cw_attention_together_bf16(const void* q, int64_t q_stride, void* 
     constexpr int RB = decltype(rb)::value;
     constexpr bool P16 = decltype(pages16)::value;
     const size_t smem = for_singles > PrefillTile<CW_HD, RB>::BYTES ? for_singles : PrefillTile<CW_HD, RB>::BYTES;
-    static_assert(PrefillTile<CW_HD, RB>::BYTES <= 158 * 1024, "tiles and the single tokens' statistics fit LDS");
-    static size_t raised = 0;
-    if (smem > raised) {
-      if (hipFuncSetAttribute((const void*)attn_together_bf16_kernel<CW_HD, P16, RB>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)smem) != hipSuccess)
-        return CW_ERR_LAUNCH;
-      raised = smem;
-    }
+    static_assert(PrefillTile<CW_HD, RB>::BYTES <= DEC_MOST_LDS, "tiles and the single tokens' statistics fit LDS");
+    static std::atomic<bool> allowed{false};
+    if (cw_allow_lds(allowed, (const void*)attn_together_bf16_kernel<CW_HD, P16, RB>, DEC_MOST_LDS) != CW_OK) return CW_ERR_LAUNCH;
     hipLaunchKernelGGL((attn_together_bf16_kernel<CW_HD, P16, RB>), dim3((unsigned)groups), dim3(512), smem, stream, a);
     launch_decode_merge(a.singles, n_singles, stream);
     return cw_launch_status();

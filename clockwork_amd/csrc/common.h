@@ -7,6 +7,8 @@
 #include <hip/hip_bf16.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #define CW_OK 0
 #define CW_ERR_ARG -1      // a size or pointer the kernel does not take
 #define CW_ERR_DTYPE -2    // unknown element type code
@@ -165,6 +167,16 @@ __device__ __forceinline__ void cw_lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Lets all launches of a kernel take up to ``most`` bytes of dynamic LDS, a constant of the kernel: a limit set to what one
+// launch takes could be lowered by another thread's smaller launch before the first one goes out. ``allowed``: of this kernel.
+static inline int cw_allow_lds(std::atomic<bool>& allowed, const void* kernel, int most) {
+  if (!allowed.load(std::memory_order_acquire)) {
+    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, most) != hipSuccess) return CW_ERR_LAUNCH;
+    allowed.store(true, std::memory_order_release);
+  }
+  return CW_OK;
 }
 
 static inline int cw_launch_status() {

@@ -143,6 +143,8 @@ __global__ __launch_bounds__(512) void gemm_f32_rows_kernel(const float* __restr
 // 2048 x 1536 9.9 -> 8.3; the sums are the same bit for bit.
 #define GT_BLOCK_WAVES 8
 #define GT_BLOCKS 120   // blocks a workgroup takes: 1 KB of LDS each with 16 rows of x
+// and of the parts that they make, of 256 k-values at least, where those meet in LDS as well
+#define GT_BLOCKS_LDS ((GT_BLOCKS + GT_BLOCKS / 16) * 1024)
 // GLU: W = [gate; up], a tile is 8 gate rows and the 8 up rows that belong to them, C the gated product [M, N / 2].
 template <bool GLU>
 __global__ __launch_bounds__(GT_BLOCK_WAVES * 64) void gemm_f32_blocks_kernel(const float* __restrict__ A, int64_t lda,
@@ -563,12 +565,8 @@ static int launch_gemm_f32(const float* A, int64_t lda, const float* W, const fl
     if (blocks <= GT_BLOCKS) {
       const size_t lds = (size_t)(blocks + (planes || splits == 1 ? 0 : splits)) * M * 16 * sizeof(float);
       const dim3 grid(tiles, (splits + here - 1) / here);
-      static size_t raised = 48 * 1024;
-      if (lds > raised) {
-        if (hipFuncSetAttribute((const void*)gemm_f32_blocks_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-          return CW_ERR_LAUNCH;
-        raised = lds;
-      }
+      static std::atomic<bool> allowed{false};
+      if (cw_allow_lds(allowed, (const void*)gemm_f32_blocks_kernel<false>, GT_BLOCKS_LDS) != CW_OK) return CW_ERR_LAUNCH;
       hipLaunchKernelGGL(gemm_f32_blocks_kernel<false>, grid, dim3(GT_BLOCK_WAVES * 64), lds, stream, A, lda, W, bias, C, ldc, M, N, K,
                          splits, part_blocks, here, stride, 0.0f);
       return cw_launch_status();
@@ -649,12 +647,8 @@ CW_EXPORT int cw_gemm_f32_swiglu(const float* A, int64_t lda, const float* W, fl
   int splits, per;
   gemm_f32_plan(N, K, &splits, &per);
   const size_t lds = (size_t)(K / 16 + splits) * M * 16 * sizeof(float);
-  static size_t raised = 48 * 1024;
-  if (lds > raised) {
-    if (hipFuncSetAttribute((const void*)gemm_f32_blocks_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-      return CW_ERR_LAUNCH;
-    raised = lds;
-  }
+  static std::atomic<bool> allowed{false};
+  if (cw_allow_lds(allowed, (const void*)gemm_f32_blocks_kernel<true>, GT_BLOCKS_LDS) != CW_OK) return CW_ERR_LAUNCH;
   hipLaunchKernelGGL(gemm_f32_blocks_kernel<true>, dim3((N / 2 + 7) / 8), dim3(GT_BLOCK_WAVES * 64), lds, stream, A, lda, W, nullptr, C, ldc,
                      M, N, K, splits, per / 16, splits, 0, act);
   return cw_launch_status();

@@ -73,3 +73,10 @@ def test_inline_assembly_names_the_scalar_register_that_it_writes():
     writers = [a for a in statements if re.search(r"\bs_\w+ m0\b", a)]
     assert len(statements) > len(writers) >= 3
     assert [a for a in writers if '"m0"' not in a] == []
+
+
+def test_no_limit_of_lds_follows_the_launches():
+    """A limit that is raised to what a launch takes, and remembered, may be lowered again by a thread that remembers an
+    older one: kernels whose launches differ in LDS are allowed their most at once."""
+    for path in sorted(build.CSRC.glob("*.h*")):
+        assert re.findall(r"\bstatic\s+(?!bool\b)\w+\s+raised\b.*", path.read_text()) == [], path.name
