@@ -162,9 +162,7 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_row_kernel(float* __restrict
   const float ss = cw_wave_sum(in ? (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]) : 0.0f);
   if ((threadIdx.x & 63) == 0) partial[threadIdx.x >> 6] = ss;
   cw_lds_barrier();
-  float total = 0.0f;
-  for (int k = 0; k < (int)(blockDim.x >> 6); ++k) total += partial[k];
-  const float inv = 1.0f / sqrtf(total / (float)H + eps);
+  const float inv = 1.0f / sqrtf(cw_block_total(partial, blockDim.x >> 6) / (float)H + eps);
   if (!in) return;
   float r[4];
 #pragma unroll

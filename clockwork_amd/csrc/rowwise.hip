@@ -223,9 +223,7 @@ __global__ __launch_bounds__(1024) void add_layernorm_row_kernel(float* __restri
     s = cw_wave_sum(in ? s : 0.0f);
     if ((threadIdx.x & 63) == 0) to[threadIdx.x >> 6] = s;
     cw_lds_barrier();
-    float total = 0.0f;
-    for (int k = 0; k < waves; ++k) total += to[k];
-    return total;
+    return cw_block_total(to, waves);
   };
   const float mean = row_sum((v[0] + v[1]) + (v[2] + v[3]), partial[0]) / (float)H;
   float ss = 0.0f;

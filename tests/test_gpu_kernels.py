@@ -897,6 +897,29 @@ def test_add_rmsnorm_a_chunk_a_thread(dtype, H, planes):
         assert (r.double() - kept).abs().max() <= 16 * 2.0 ** -24 * kept.abs().max() + (0 if rows else 1e-6)
 
 
+@pytest.mark.parametrize("norm", ["rms", "layer"])
+@pytest.mark.parametrize("large", [0, 7, 15])
+def test_a_row_s_waves_are_added_in_pairs(norm, large):
+    """Squares of 2^24 (twice that) in one wave's elements and of 1 (2) in each of the 15 others': one after the other behind the
+    large one each small sum would be lost whole, 7.5 units of 2^-24 in the factor; in pairs only the first addition
+    loses one, half a unit. Then the epsilon, a root, a quotient and a product, a unit each at most: 4.5 in all."""
+    from clockwork_amd import ops
+
+    H = 4096
+    x = torch.zeros(1, H, device=DEV)
+    x[0, 13 :: 256] = 1.0
+    x[0, 13 + 256 * large] = 4096.0
+    if norm == "layer":
+        x[0, 14 :: 256] = -x[0, 13 :: 256]
+    one, out = torch.ones(H, device=DEV), torch.empty(1, H, device=DEV)
+    if norm == "rms":
+        ops.add_rmsnorm(x.clone(), None, one, 1e-6, out)
+    else:
+        ops.add_layernorm(x.clone(), None, one, torch.zeros(H, device=DEV), 1e-6, out)
+    want = x.double() / torch.sqrt(x.double().square().mean() + 1e-6)
+    assert ((out.double() - want).abs() <= 4.5 * 2.0 ** -24 * want.abs()).all()
+
+
 # the reference's decode cases (tests/test_triton_kernel.py:14-20) plus sizes of our own
 DECODE_CASES = [
     (4, 4, 16, 4, [5, 12, 9]),
