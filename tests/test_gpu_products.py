@@ -529,6 +529,29 @@ def test_recurrence_in_segments_with_an_infinite_value(at):
     assert bool((state[0, 0, :, 3] == float("inf")).all())
 
 
+@pytest.mark.parametrize("dim,vdim,lost", [(16, 64, 3), (64, 64, 7), (64, 128, 7), (64, 256, 7), (128, 128, 7), (128, 256, 15)])
+def test_segments_of_the_recurrence_add_channels_in_several_chains(dim, vdim, lost):
+    """A state of 2^24 in the first channel and of 1 in one of every four: added behind the large one each 1 is lost, and so is
+    each channel of its chain of products (16 tiles of channels' steps over one, two or four chains), but none of the
+    others'."""
+    from clockwork_amd import ops
+
+    T, rank = 40, 16
+    ints = lambda *t: torch.tensor(t, dtype=torch.int32, device=DEV)  # noqa: E731
+    proj = torch.zeros(T, 2 * dim + vdim + rank, device=DEV)
+    proj[:, :dim] = 1.0                                  # queries; keys, values and decay inputs are zero
+    state = torch.zeros(1, 1, dim, vdim, device=DEV)
+    ones = [d for d in range(dim) if d % 16 < 4]
+    state[0, 0, ones] = 1.0
+    state[0, 0, 0] = 2.0 ** 24
+    got = ops.linear_recurrence_segments(proj, 0, dim, 2 * dim, -1, 2 * dim + vdim, torch.zeros(dim, rank, device=DEV),
+                                         torch.full((dim,), -60.0, device=DEV), None, state, ints(0), ints(0, T),
+                                         ints(0, 0, 32, 0, 0, 32, 8, 1), 2, 32, ints(0, 2), 1, 1, dim, vdim, 1.0, 16.0, 1e-5,
+                                         decay="double_exp")  # exp(-exp(-60)): decays of 1
+    want = 2.0 ** 24 + len(ones) - 1
+    assert bool(((want - got.double() >= 0) & (want - got.double() <= lost + 1)).all())
+
+
 # runs of 32, 50 and 128 keys; mixed heads over one, two (two kernels) and three key/value heads (three kernels), no
 # mixing over four; sizes that are read in pieces and one by one, more columns than threads, groups of more than 16 heads
 @pytest.mark.parametrize("heads,kv,dim,vdim,talk", [(12, 2, 128, 128, True), (6, 2, 20, 24, True), (3, 1, 40, 24, True), (6, 3, 64, 64, True),
