@@ -977,13 +977,14 @@ __global__ __launch_bounds__(256, D * VT <= 128 ? 3 : 1) void lrs_outputs_kernel
     for (int vt = 0; vt < VT; ++vt) o[b][vt] = (lrs_f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
     if (16 * b >= nt) continue;
     // Sums of every second or fourth tile of channels, and of the chunk's own keys, added at the end: one chain of additions
-    // for all of them rounds further. (Four tiles of columns a wave have registers for two chains,
-    // or one where three workgroups share a compute unit.)
-    constexpr int CHAINS = VT > 2 ? (D * VT <= 128 ? 1 : 2) : D == 128 ? 4 : 2, OWN = VT > 2 ? CHAINS - 1 : CHAINS;
-    lrs_f32x4_t apart[OWN > 0 ? OWN : 1][VT];
+    // for all of them rounds further. Four tiles of columns a wave have registers for one sum beside the total, which
+    // takes two tiles of channels at a time (none where three workgroups share a compute unit).
+    constexpr bool TURNS = VT > 2;
+    constexpr int SIDE = TURNS ? (D >= 64 ? 1 : 0) : D == 128 ? 4 : 2;
+    lrs_f32x4_t apart[SIDE > 0 ? SIDE : 1][VT];
     auto sum_of = [&](int k, int vt) __attribute__((always_inline)) -> lrs_f32x4_t& { return k ? apart[k - 1][vt] : o[b][vt]; };
 #pragma unroll
-    for (int k = 0; k < OWN; ++k)
+    for (int k = 0; k < SIDE; ++k)
 #pragma unroll
       for (int vt = 0; vt < VT; ++vt) apart[k][vt] = (lrs_f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -993,8 +994,14 @@ __global__ __launch_bounds__(256, D * VT <= 128 ? 3 : 1) void lrs_outputs_kernel
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int vt = 0; vt < VT; ++vt) {
-          lrs_f32x4_t& to = sum_of(dt % CHAINS, vt);
+          lrs_f32x4_t& to = sum_of(TURNS ? SIDE : dt % SIDE, vt);
           to = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i], S[dt][vt][i], to, 0, 0, 0);
+        }
+      if (TURNS && SIDE && dt & 1)
+#pragma unroll
+        for (int vt = 0; vt < VT; ++vt) {
+          o[b][vt] += apart[0][vt];
+          apart[0][vt] = (lrs_f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
         }
     }
     bool finite = true;
@@ -1007,7 +1014,7 @@ __global__ __launch_bounds__(256, D * VT <= 128 ? 3 : 1) void lrs_outputs_kernel
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int vt = 0; vt < VT; ++vt) sum_of(OWN, vt) = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j], vf[b][j][vt], sum_of(OWN, vt), 0, 0, 0);
+        for (int vt = 0; vt < VT; ++vt) sum_of(SIDE, vt) = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j], vf[b][j][vt], sum_of(SIDE, vt), 0, 0, 0);
     } else {  // an infinite value must not meet the zeros of the tokens before it
 #pragma unroll
       for (int j = 0; j < 16; ++j)
@@ -1016,17 +1023,17 @@ __global__ __launch_bounds__(256, D * VT <= 128 ? 3 : 1) void lrs_outputs_kernel
           const float v = __shfl(vf[b][j % 4][vt], (j / 4) * 16 + c, 64);
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            if (4 * s + i >= j) sum_of(OWN, vt)[i] = fmaf(Ps[(16 * b + 4 * s + i) * 20 + j], v, sum_of(OWN, vt)[i]);
+            if (4 * s + i >= j) sum_of(SIDE, vt)[i] = fmaf(Ps[(16 * b + 4 * s + i) * 20 + j], v, sum_of(SIDE, vt)[i]);
         }
     }
 #pragma unroll
     for (int vt = 0; vt < VT; ++vt) {
-      if constexpr (CHAINS == 4) {
+      if constexpr (SIDE == 4) {
         o[b][vt] += apart[0][vt];
         apart[0][vt] = apart[1][vt] + apart[2][vt];
       }
-      if (CHAINS > 1) o[b][vt] += apart[0][vt];
-      if (OWN == CHAINS) o[b][vt] += apart[OWN - 1][vt];
+      if (!TURNS) o[b][vt] += apart[0][vt];
+      if (SIDE) o[b][vt] += apart[SIDE - 1][vt];
     }
     if (b == 0 && nt > 16) {
 #pragma unroll
