@@ -216,18 +216,23 @@ __global__ __launch_bounds__(WAVES * 64) void attn_f32_kernel(AttnParams p, int 
   // one tile: ``at`` where it lay, ``k`` and ``v`` what lay there
   auto compute = [&](int t, const int64_t (&at)[5], float (&k)[KB][4], float (&v)[4][VG][VW]) __attribute__((always_inline)) {
     const int kv0 = 16 * t;
-    // no page: zeros
-    if (__builtin_amdgcn_ballot_w64(at[0] < 0 || at[1] < 0 || at[2] < 0 || at[3] < 0 || at[4] < 0)) {
+    // no page: zeros; and zeros for values outside the range (what lies there is another key's, and a weight of
+    // zero times an infinite value is no zero)
+    if (kv0 < kv_lo || kv0 + 16 > kv_end ||
+        __builtin_amdgcn_ballot_w64(at[0] < 0 || at[1] < 0 || at[2] < 0 || at[3] < 0 || at[4] < 0)) {
 #pragma unroll
       for (int b = 0; b < KB; ++b)
 #pragma unroll
         for (int j = 0; j < 4; ++j) k[b][j] = at[0] >= 0 ? k[b][j] : 0.0f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < 4; ++j) {
+        const int pos = kv0 + 4 * s + j;
+        const bool there = at[1 + j] >= 0 && pos >= kv_lo && pos < kv_end;
 #pragma unroll
         for (int g = 0; g < VG; ++g)
 #pragma unroll
-          for (int e = 0; e < VW; ++e) v[j][g][e] = at[1 + j] >= 0 ? v[j][g][e] : 0.0f;
+          for (int e = 0; e < VW; ++e) v[j][g][e] = there ? v[j][g][e] : 0.0f;
+      }
     }
     attn_f32x4_t sc[RB];
 #pragma unroll
@@ -1111,7 +1116,8 @@ __device__ __forceinline__ void attn_prefill_of(const AttnParams& p, const int i
   const int k_piece = k_granule(lane >> 2, lane & 3) * 8, v_piece = v_granule(lane >> 2, lane & 3) * 8;
   // A key that no row sees (past the last token, or before the window's first key) is brought as its neighbour that
   // some row sees: it is masked by its position. With whole pages a wave's 16 keys have one page and one address, and a
-  // lane an offset; else every lane has an address of its own. No page: zeros.
+  // lane an offset; else every lane has an address of its own. No page: zeros; and zeros for the values of a key that no
+  // row sees (a weight of zero times a neighbour's infinite value would be no zero).
   auto group_of = [&](int t) __attribute__((always_inline)) { return min(max(t * KT + kg * 16, wg_lo & ~15), wg_last & ~15); };
   auto key_of = [&](int t) __attribute__((always_inline)) { return min(max(t * KT + f_key, wg_lo), wg_last); };
   auto page_of = [&](int t) __attribute__((always_inline)) {
@@ -1120,8 +1126,10 @@ __device__ __forceinline__ void attn_prefill_of(const AttnParams& p, const int i
   int64_t at_row = 0;   // in elements from the head's first: PAGES16 the row of the group's first key, else of the lane's key
   int at_key = 0;       // PAGES16: the lane's row in the group, in elements
   bool at_page = false;
+  int at_first = 0;     // the group's first key, whoever sees it
   auto aim = [&](int t, int page) __attribute__((always_inline)) {
     at_page = page >= 0;
+    at_first = t * KT + kg * 16;
     if constexpr (PAGES16) {
       const int g = group_of(t);
       at_row = (int64_t)(((uint64_t)(uint32_t)page * (uint32_t)bs + (uint32_t)(g & (bs - 1))) * (uint32_t)row_elems);
@@ -1131,16 +1139,22 @@ __device__ __forceinline__ void attn_prefill_of(const AttnParams& p, const int i
       at_row = (int64_t)((uint64_t)slot * (uint32_t)row_elems);
     }
   };
-  auto bring = [&](const bf16_t* head, int piece, int tile) __attribute__((always_inline)) {  // the wave's blocks of a tile
-    const bf16_t* const from = at_page ? head + at_row : zrow;
+  auto bring = [&](const bf16_t* head, int piece, int tile, auto values) __attribute__((always_inline)) {  // the wave's blocks of a tile
+    auto blocks = [&](auto&& load) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < (NF + SHARE - 1) / SHARE; ++j) {
-      const int blk = j * SHARE + sub;
-      unsigned char* const to = smem_raw + tile * Tile::TILE + (kg * NF + blk) * 1024;
-      if (NF % SHARE == 0 || blk < NF) {
-        if constexpr (PAGES16) load_to_lds(from + blk * 32, (uint32_t)(at_key + piece) * 2, to);
-        else load_to_lds(from + blk * 32 + piece, to);
+      for (int j = 0; j < (NF + SHARE - 1) / SHARE; ++j) {
+        const int blk = j * SHARE + sub;
+        if (NF % SHARE == 0 || blk < NF) load(blk * 32, smem_raw + tile * Tile::TILE + (kg * NF + blk) * 1024);
       }
+    };
+    const int key = at_first + (lane >> 2);
+    const bool seen = !decltype(values)::value || (key >= wg_lo && key <= wg_last);
+    if (!PAGES16 || (decltype(values)::value && (at_first < wg_lo || at_first + 15 > wg_last))) {
+      const bf16_t* const from = (at_page && seen ? head + at_row + (PAGES16 ? at_key : 0) : zrow) + piece;
+      blocks([&](int at, unsigned char* to) { load_to_lds(from + at, to); });
+    } else {
+      const bf16_t* const from = at_page ? head + at_row : zrow;
+      blocks([&](int at, unsigned char* to) { load_to_lds(from + at, (uint32_t)(at_key + piece) * 2, to); });
     }
   };
 
@@ -1327,14 +1341,14 @@ __device__ __forceinline__ void attn_prefill_of(const AttnParams& p, const int i
     __builtin_amdgcn_s_barrier();        // everyone's is, and the tiles that stage t + 1 comes into have been read
     asm volatile("" ::: "memory");
     if (t > t_last) return;
-    if (t > t_first) bring(vc, v_piece, 2 + ((t - t_first) & 1));
+    if (t > t_first) bring(vc, v_piece, 2 + ((t - t_first) & 1), std::true_type{});
     aim(t + 1, page);  // (behind the last stage: a tile that nobody reads)
-    bring(kc, k_piece, (t + 1 - t_first) & 1);
+    bring(kc, k_piece, (t + 1 - t_first) & 1, std::false_type{});
   };
   if (t_first <= t_last) {
     aim(t_first, page_a);
-    bring(kc, k_piece, 0);
-    bring(vc, v_piece, 2);  // (later V comes one interval after K)
+    bring(kc, k_piece, 0, std::false_type{});
+    bring(vc, v_piece, 2, std::true_type{});  // (later V comes one interval after K)
     const bool active = on_first <= on_last;
     const int until = active ? on_first : t_last + 1;
     next_interval(t_first, page_b);

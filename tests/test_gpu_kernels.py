@@ -1375,6 +1375,36 @@ def test_prefill_attention_kernel_at_the_edges_of_its_stages(nh, nkv, hd, bs, wi
         at += q_len
 
 
+@pytest.mark.parametrize("window", [0, 37])
+@pytest.mark.parametrize("bs", [16, 24])
+@pytest.mark.parametrize("nh,nkv,hd,how", [(12, 2, 128, 4), (12, 2, 128, 2), (4, 2, 64, 4), (8, 2, 256, 4), (12, 2, 128, None), (4, 2, 64, None),
+                                           (8, 2, 256, None), (6, 3, 48, None)])
+def test_an_infinite_value_stays_infinite_where_it_is_seen(nh, nkv, hd, bs, window, how):
+    """Infinite values at the last key of each request and, with a window, at the first key that its first token sees: the
+    keys outside a workgroup's range have weights of zero, and nothing infinite may stand in for their values. (Float32
+    and the bfloat16 kernel for portions, by ``how`` row blocks.)"""
+    dtype = torch.float32 if how is None else torch.bfloat16
+    ctx_lens, q_lens = [90, 200, 133], [40, 1, 70]
+    tables, at = [], 0
+    for c in ctx_lens:
+        tables.append(list(range(at, at + -(-c // bs))))
+        at += len(tables[-1])
+    kc, vc, ks, vs = _paged_setup(dtype, nkv, hd, bs, at, tables, ctx_lens, poison=float("nan"))
+    sees = {}
+    for r, (c, n) in enumerate(zip(ctx_lens, q_lens)):
+        for channel, key, token in [(3, c - 1, n - 1)] + ([(5, c - n - window + 1, 0)] if window else []):
+            vc[tables[r][key // bs] * bs + key % bs, :, channel] = float("inf")
+            sees[r, channel] = token
+    qs = [torch.randn(n, nh, hd, device=DEV).to(dtype) for n in q_lens]
+    out = _run_attention(dtype, nh, nkv, hd, bs, tables, ctx_lens, q_lens, kc, vc, qs, window=window, prefill_kernel=how if how else False,
+                         decode_kernel=how is not None)
+    first = [0, 40, 41]
+    for (r, channel), token in sees.items():
+        row = out[first[r] + token]
+        assert bool((row[:, channel] == float("inf")).all()), (r, channel)
+        assert bool(torch.isfinite(row[:, [0, 1, 2, 4, *range(6, hd)]].float()).all()), (r, channel)
+
+
 @pytest.mark.parametrize("row_blocks", [4, 2])
 def test_prefill_attention_kernel_sharp_scores(row_blocks):
     """Scores of very different size, so that the running maximum moves from tile to tile and one
