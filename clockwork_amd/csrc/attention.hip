@@ -532,7 +532,7 @@ __device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, v
 // take turns on tiles of 32 keys. Per tile:
 //   S^T[key, head] = K * Q^T        v_mfma_f32_16x16x32_bf16; the up to 16 heads of the group are
 //                                   the columns, so every key is fetched once for the whole group;
-//   softmax per head in float32: a lane holds 8 keys of one head, two shuffles finish a head;
+//   softmax per head in float32: a lane holds 8 keys of one head, two swaps of lanes across the wave's rows finish a head;
 //   O^T[d, head] += V^T * P^T       P^T is the softmax output as it lies in the registers.
 // A wave's tile comes from the pages straight into LDS of its own, four neighbouring lanes 64 bytes of a key, and its operands
 // from there: K fragments by 16-byte reads, V^T fragments by the transposing read (see the kernel for portions). Once a tile's
@@ -1048,7 +1048,7 @@ struct PrefillTile {
   static constexpr int NT = 64 * WAVES;                 // threads of a workgroup
   // A K or V tile lies in LDS as blocks of 16 keys x 32 elements (1 KB: what one load of a wave with the
   // LDS target brings), [16-key group][32 elements]. Inside a block a key's four 16-byte granules are
-  // permuted (kv_granule) so that no bank is hit twice when operands are read.
+  // permuted (k_granule, v_granule) so that no bank is hit twice when operands are read.
   static constexpr int TILE = KT * HD * 2;              // bytes of a tile
   static constexpr size_t TILES = 4 * (size_t)TILE;     // two of K, two of V
   // what the sets of waves exchange at the end: accumulators of all sets, then maxima and sums

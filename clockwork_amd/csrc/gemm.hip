@@ -1399,7 +1399,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_qkv_rope_bf16_kernel(
 #pragma unroll
   for (int e = 0; e < 8; ++e) zero[e] = (__bf16)0.0f;
   const int k_steps = (K + 31) / 32;
-  constexpr int U = MT <= 2 ? 4 : 2;
+  constexpr int U = 4;  // k-steps in flight a wave
   for (int ks0 = wave * U; ks0 < k_steps; ks0 += WAVES * U) {
     bf16x8_t wf[U], xf[U][MT];
 #pragma unroll

@@ -42,8 +42,9 @@ GRAPH_KEY_BUCKET = 512
 # next of these sizes (a step of 65 to 500 tokens is otherwise bound by the host's launches); what a
 # step is padded by is computed for nothing (137 tokens of the 1.5B shape: 2.62 ms as 256, 2.46 as 160)
 PORTION_GRAPH_SIZES = (16, 32, 64, 96, 128, 160, 192, 256, 384, 448, 512)
-# beside single tokens, where a step waits for a whole prompt's share of every product, one size more (300 tokens beside 15
-# decoding requests of the 1.5B shape: 3.55 ms as 384, 3.30 as 320)
+# beside single tokens one size more (300 tokens beside 15 decoding requests of the 1.5B shape: 3.55 ms as 384, 3.30 as
+# 320). Lone portions of 257 to 320 tokens stay at 384, where the replay tests look for their captured step: a third of
+# padding at most (300 tokens: 3.03 ms, 2.90 as 320).
 MIXED_PORTION_GRAPH_SIZES = (16, 32, 64, 96, 128, 160, 192, 256, 320, 384, 448, 512)
 # the rows that the narrow products take in one, two or four tiles of tokens: a step of single
 # tokens beside a short portion is padded to the next of these in all, if it fits one

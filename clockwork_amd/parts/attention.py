@@ -74,7 +74,8 @@ MIN_PART_KEYS = 256
 MAX_PARTS = 64
 # Parts of a single token's keys for the float32 kernel: a workgroup of eight waves takes 128 keys in one turn of some
 # 1.5 us, and the kernel that merges the parts takes 4 us however many there are. Up to 384 keys stay whole (one
-# request of the 0.5B shape, one part / parts of 128 keys: 300 keys 10.3 / 10.5 us, 510 keys 12.9 / 10.9).
+# request of the 0.5B shape, one part / parts of 128 keys: 300 keys 10.3 / 10.5 us, 510 keys 12.9 / 10.9): a rule for steps
+# that are not captured. Captured ones are planned for a multiple of 512 keys and always have four parts or more.
 F32_PART_KEYS = 128
 F32_WHOLE_KEYS = 384
 
@@ -163,9 +164,13 @@ def _split_keys(longest: int, splits: int) -> int:
 def _share_the_card(plan: AttentionPlan, room: int, base: int, longest: int, most_keys: int) -> None:
     """One launch for a step's portions and single tokens, where all workgroups of both are at work at once: ``room``
     compute units are left beside the portions' workgroups, a split of every single token takes ``base`` of them. The splits
-    are then as many as fit, but not fewer than half of those that the single tokens alone would be cut into: where the
-    portions take nearly the whole card, a few long splits would outlast both launches (a step of 15
-    requests of 1500 keys beside 300 tokens, 1.5B shape: 3.30 ms with 8 splits behind the portions, 3.04 with 6 beside them). A split of more than ``most_keys`` keys
+    are then as many as fit, but not fewer than half of those that the single tokens alone would be cut into. Measured
+    on both sides of that line, us a layer's attention as two launches / as one with the splits that fit (12 heads of 128 on
+    2): 16 requests of 1500 keys (8 splits) beside 64 tokens 20.0 / 12.8 with 7, 320 tokens 22.6 / 16.0 with 6, 448 23.9 / 17.1
+    with 5; below it 760 tokens 27.1 / 19.2 with 3, 900 28.8 / 20.6 with 2; 32 of 1500 (4) beside 320 26.7 / 18.1 with 3, 760
+    30.8 / 17.0 with 1; 64 of 2000 (2) beside 320 42.7 / 33.6 with 1. So one launch is the faster one below the line as well:
+    the line is cautious, not where the two meet. (A step of 15 requests of 1500 beside 300 tokens, 1.5B shape: 3.30 ms with
+    8 splits behind the portions, 3.04 with 6 beside them.) A split of more than ``most_keys`` keys
     (of the ``longest`` context) has more pages than the launch takes: two launches then, whose splits are shorter."""
     splits = min(room // base, plan.decode_splits)
     if splits >= 1 and 2 * splits >= plan.decode_splits and not 0 < most_keys < _split_keys(longest, splits):
