@@ -640,6 +640,24 @@ def test_gate_up_of_a_long_portion_goes_through_the_wide_tile_kernel():
     torch.testing.assert_close(few.float(), want[:100], rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("M", [321, 336, 362, 363, 400])
+def test_gate_up_of_a_captured_step_beside_a_padded_portion_rounds_once(M):
+    """One to 48 decoding requests beside a portion padded to 320 or 384: gates and ups meet in float32 and the result is
+    rounded to bfloat16 once, by 2^-9 at most (rounded before the gate as well, the errors add up to 3.1e-3)."""
+    from clockwork_amd import ops
+
+    two_i, K = 17920, 1536
+    x, w = torch.randn(M, K, device=DEV).to(torch.bfloat16), (torch.randn(two_i, K, device=DEV) / K ** 0.5).to(torch.bfloat16)
+    ops.linear_swiglu(x, w)  # (whatever is loaded at a first call)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ops.linear_swiglu(x, w)
+    graph.replay()
+    gate, up = (x.double() @ w.double().t()).chunk(2, dim=1)
+    want = torch.nn.functional.silu(gate) * up
+    assert (out.double() - want).norm() <= 2.0 ** -9 * want.norm()
+
+
 def test_a_tuning_start_up_measures_which_gate_up_product_is_faster():
     """While the library tunes, the first long portion of a weight shape times both ways and the
     choice is kept by the engine's own policy: later products of that shape follow it, and a
