@@ -765,11 +765,7 @@ WIDE_MIN_TILES = 64
 # library leaves units idle there as well), 58 % in several (us, library and gate against this: 1.5B shape, 188 tiles, 304 rows
 # 34.8 / 36.4, 368 rows 37.4 / 36.0, 408 rows 38.9 / 36.7, 512 rows 44.5 / 37.3; 282 tiles, 640 rows 53.6 / 68.9; 376 tiles,
 # 1000 rows 88.3 / 71.8; 3B shape, 230 tiles, 304 rows 44.5 / 44.8, 385 rows 55.1 / 45.8; 345 tiles, 640 rows 77.8 / 84.9, 700 rows
-# 97.2 / 86.0; 7B shape, 400 rows 150 / 136, 640 rows 189 / 202: there reading W bounds both). In one round it is also taken with
-# a last row tile that is more than a quarter full: it is 1 to 3 % slower there (1.5B shape, 320 rows 34.8 / 35.9, 321 34.8 /
-# 35.8, 336 35.2 / 35.9, 360 36.0 / 36.1), but the library's product rounds gates and ups to bfloat16 before the gate reads them (errors
-# to 64 bits 3.1e-3 / 1.7e-3), and steps of 300 tokens beside others, which are padded to 320 of these rows, have had the finer
-# ones since they were padded to 384. Against the library's TUNED choice it wins for
+# 97.2 / 86.0; 7B shape, 400 rows 150 / 136, 640 rows 189 / 202: there reading W bounds both). Against the library's TUNED choice it wins for
 # the 0.5B, 1.5B, 3B, 14B and 32B shapes (the 1.5B shape's whole prefill step: 8.9 -> 7.9 ms) and
 # loses 3 % of the step for the 7B and 72B shapes, so a start-up that tunes (``library_tuning``)
 # times both ways on the model's own weights and keeps the faster (``ProductPolicy.swiglu_choices``).
@@ -790,8 +786,8 @@ def _compute_units(device) -> int:
 
 
 def wide_swiglu_pays(M: int, two_i: int, K: int, ldx: int) -> bool:
-    """Is the gate/up product of M rows faster (or as good as, and finer) through the wide-tile kernel, with the gate in its
-    epilogue, than through the library and the gate kernel?"""
+    """Is the gate/up product of M rows faster through the wide-tile kernel (with the gate in its
+    epilogue) than through the library and the gate kernel?"""
     if M < WIDE_SWIGLU_MIN_ROWS // 4:
         return False
     tiles = _load("gemm_tile").cw_gemm_bf16_wide_tiles(2, M, two_i, K, ldx)
@@ -802,8 +798,19 @@ def wide_swiglu_pays(M: int, two_i: int, K: int, ldx: int) -> bool:
     units, rows = _compute_units(torch.device("cuda", torch.cuda.current_device())), WIDE_SWIGLU_TILE_ROWS
     rounds = -(-tiles // units)
     work = tiles / (units * rounds) * M / (rows * -(-M // rows))
-    enough = work >= WIDE_SWIGLU_WORK if rounds > 1 else work >= WIDE_SWIGLU_WORK_ONE_ROUND or M % rows > rows // 4
-    return two_i * K <= WIDE_SWIGLU_SMALL_WEIGHTS and enough
+    return two_i * K <= WIDE_SWIGLU_SMALL_WEIGHTS and work >= (WIDE_SWIGLU_WORK if rounds > 1 else WIDE_SWIGLU_WORK_ONE_ROUND)
+
+
+def wide_swiglu_is_finer(M: int, two_i: int, K: int, ldx: int) -> bool:
+    """Is the wide-tile kernel, whose gate reads float32 sums, all but as fast as the library and the gate kernel, where gates and
+    ups are rounded to bfloat16 between them (errors to 64 bits 1.7e-3 / 3.1e-3)? Two row tiles in one round of few weights,
+    the second more than a quarter full: there it is 1 to 3 % slower (us, library and gate against this, 1.5B shape, 188 tiles: 321 rows 34.8 /
+    35.8, 336 rows 35.2 / 35.9, 360 rows 36.0 / 36.1), from 363 rows on it pays. Steps of 257 to 320 tokens beside others are of
+    these rows, and had float32 gates when they were padded to 384."""
+    tiles = _load("gemm_tile").cw_gemm_bf16_wide_tiles(2, M, two_i, K, ldx)
+    units, rows = _compute_units(torch.device("cuda", torch.cuda.current_device())), WIDE_SWIGLU_TILE_ROWS
+    return (WIDE_SWIGLU_MIN_TILES <= tiles <= units and rows + rows // 4 < M <= 2 * rows
+            and two_i * K <= WIDE_SWIGLU_SMALL_WEIGHTS)
 
 
 @contextlib.contextmanager
@@ -1216,8 +1223,9 @@ def linear_swiglu(x, gate_up_weight: torch.Tensor, policy: "ProductPolicy | None
         # fewer than 512 rows only inside a captured graph, where a shape's steps run from its second on. Run eagerly they
         # keep to the library's product, as the replay tests have it (450 tokens of the 1.5B shape, bound by the host's
         # launches: 3.9 ms, 3.65 with one launch instead of two)
-        if (_aligned(x, gate_up_weight) and wide_swiglu_pays(M, two_i, K, K)
-                and (M >= WIDE_SWIGLU_MIN_ROWS // 2 or torch.cuda.is_current_stream_capturing())):
+        captured = torch.cuda.is_current_stream_capturing()
+        if _aligned(x, gate_up_weight) and ((wide_swiglu_pays(M, two_i, K, K) and (M >= WIDE_SWIGLU_MIN_ROWS // 2 or captured))
+                                            or (captured and wide_swiglu_is_finer(M, two_i, K, K))):
             # with enough rows the shape of the weights decides, and a start-up that tunes the
             # library's products has measured it for this model's
             measured, key = M >= WIDE_SWIGLU_MIN_ROWS, _swiglu_key(two_i, K, limit)
