@@ -118,19 +118,25 @@ def typical_start(start: int) -> int:
     return near if near >= 512 else 0
 
 
-def _as_captured(step):
-    """``step`` as a captured step is planned: every portion where the portions of its kind begin."""
-    return SimpleNamespace(h_q_lens=step.h_q_lens, num_compute_units=step.num_compute_units, upload=step.upload,
-                           h_ctx_lens=[c if q == 1 else q + typical_start(c - q) for q, c in zip(step.h_q_lens, step.h_ctx_lens)])
+def _typical_lens(q_lens, ctx_lens) -> tuple:
+    """The contexts that a captured step is planned for: every portion where the portions of its kind begin."""
+    return tuple(c if q == 1 else q + typical_start(c - q) for q, c in zip(q_lens, ctx_lens))
 
 
 @lru_cache(maxsize=4096)
-def captured_choices(q_lens: tuple, ctx_lens: tuple, nh: int, nkv: int, units: int, mfma: bool, narrow_ok: bool, whole_keys: int,
-                     together_ok: bool) -> tuple:
+def captured_choices(q_lens: tuple, ctx_lens: tuple, *how) -> tuple:
     """What the plan of a captured step decides by its portions' cached keys: steps of the same tokens and the same choices
-    have the same plan. ``mfma``: the portions run on the bfloat16 matrix-core kernel."""
+    have the same plan. ``how``: (heads, kv heads, compute units, whether the portions run on the bfloat16 matrix-core kernel,
+    and ``attention_plan``'s ``narrow_ok``, ``whole_keys`` and ``together_ok``). (A portion's start is hardly ever one that was
+    there before, what it counts as nearly always is.)"""
+    return _choices_of(q_lens, _typical_lens(q_lens, ctx_lens), *how)
+
+
+@lru_cache(maxsize=1024)
+def _choices_of(q_lens: tuple, ctx_lens: tuple, nh: int, nkv: int, units: int, mfma: bool, narrow_ok: bool, whole_keys: int,
+                together_ok: bool) -> tuple:
     step = SimpleNamespace(h_q_lens=q_lens, h_ctx_lens=ctx_lens, num_compute_units=units, upload=lambda arrays: arrays)
-    plan = _make_plan(_as_captured(step), nh, nkv, narrow_ok and any(q > 1 for q in q_lens), whole_keys, together_ok)
+    plan = _make_plan(step, nh, nkv, narrow_ok and any(q > 1 for q in q_lens), whole_keys, together_ok)
     if not mfma:
         return ("parts", plan.wide_splits)
     parts = np.maximum(np.asarray(plan.mfma_items).reshape(-1, 4)[:, 3] >> 8, 1)
@@ -151,8 +157,11 @@ def attention_plan(ctx, nh: int, nkv: int, narrow_ok: bool = False, whole_keys: 
     key = ("attention", nh, nkv, narrow_ok, whole_keys, together_ok, together_split_keys, captured)
     plan = ctx.plans.get(key)
     if plan is None:
-        plan = ctx.plans[key] = _make_plan(_as_captured(ctx) if captured else ctx, nh, nkv, narrow_ok, whole_keys, together_ok,
-                                           together_split_keys)
+        step = ctx
+        if captured:
+            step = SimpleNamespace(h_q_lens=ctx.h_q_lens, h_ctx_lens=_typical_lens(ctx.h_q_lens, ctx.h_ctx_lens),
+                                   num_compute_units=ctx.num_compute_units, upload=ctx.upload)
+        plan = ctx.plans[key] = _make_plan(step, nh, nkv, narrow_ok, whole_keys, together_ok, together_split_keys)
     return plan
 
 
