@@ -21,11 +21,10 @@
 // Accumulation is float32; the K loop of an output runs in the same order whatever else is in
 // the batch.
 //
-// The second kernel of this file, gemm_wide_bf16_kernel, is the one the engine takes by itself
-// for the gate/up product of long portions (it is as fast as the library's kernels there, and the
-// gate costs no pass of its own): 256 x 192 tiles, K in stages of 32 that go from global memory
-// straight into LDS (buffer loads with the LDS target, no registers between), a ring of five
-// stages, and workgroups that stay and walk over their share of the tiles. It is described where
+// The second kernel of this file, gemm_wide_bf16_kernel, is the one the engine takes by itself for most products of
+// many rows: tiles of 96 x 96 to 256 x 288, K in stages of 64 that go from global memory
+// straight into LDS (buffer loads with the LDS target, no registers between), a ring of stages that fills the LDS,
+// and workgroups that stay and walk over their share of the tiles. It is described where
 // it stands.
 #include "common.h"
 #include <type_traits>
@@ -242,37 +241,44 @@ CW_EXPORT int cw_gemm_bf16_tiled(int mode, const void* X, int64_t ldx, const voi
 
 
 // ------------------------------------------------------------------------------------------------
-// Wide tiles. One workgroup of 4 waves per compute unit owns 256 rows of x by 192 rows of W; a
-// wave owns 128 x 96 of it in 8 x 6 accumulators of 16 x 16 (192 registers; with 512 registers a
-// wave a SIMD holds this one wave, so everything that has a latency is overlapped by hand).
+// Wide tiles. One workgroup of 4 waves per compute unit owns 32 MB rows of x by 32 NB rows of W; a
+// wave owns a quarter of it in MB x NB accumulators of 16 x 16 (up to 288 registers; with 512
+// registers a wave a SIMD holds this one wave, so everything that has a latency is overlapped by hand).
 //
-// K goes in stages of 32 elements: 16 KB of x and 12 KB of W, as 28 fragment blocks of 16 rows x
-// 64 bytes. A block comes in by ONE buffer load with the LDS target (buffer_load_dwordx4 ... lds):
-// lane l writes its 16 bytes at block + 16 l, no register and no LDS store instruction between.
-// Four lanes next to each other take the 64 bytes of one row, so the cache sees one request for
-// them (lanes that take 16 bytes of four different rows cost four; measured: 2.4 times the step
-// time), and the four granules of row r change places by w_swizzle(r), so that the 16 lanes that
-// later read one granule column of 16 rows with ds_read_b128 touch every bank once. The
-// descriptors end with the matrices, so rows past the end read as zeros.
+// K goes in stages of 64 elements: blocks of 8 rows x 128 bytes, whole lines of memory (half lines, as
+// stages of 32 need them, take a fifth to a third longer). A block comes in by ONE buffer load with
+// the LDS target (buffer_load_dwordx4 ... lds): lane l writes its 16 bytes at block + 16 l, no
+// register and no LDS store instruction between. The eight granules of row r change places by
+// (r >> 1) & 7, so that the 16 lanes that later read one granule column of 16 rows with ds_read_b128
+// touch every bank once. The descriptors end with the matrices, so rows past the end read as zeros.
 //
-// Five stages are in LDS (140 KB). In iteration t a wave multiplies stage t from registers (48
-// matrix instructions), reads the 14 fragments of stage t + 1 from LDS into the other register
-// set, one read after every 3 matrix instructions, and takes part in bringing stages t + 4 and
-// t + 5 in: two stages share their rows' 128-byte lines, so their loads are issued next to each
-// other (six matrix instructions apart), spread over both iterations of the pair (the texture
-// path takes a load every 16 cycles; eight of them in a row stall the wave). The loop is bound by
-// these loads as much as by the matrix cores: without any matrix instruction or fragment read
-// the kernel still takes 0.7 to 0.8 of its time, 50 to 78 GB/s into each compute unit. An even iteration ends when all loads but its own have
-// landed (stages t + 2, t + 3), then a barrier; the waits and barriers are bare instructions,
-// since a fence would wait for every load in flight. Measured on an MI355X: 0.52 us a stage
-// against 0.45 us for the matrix instructions alone.
+// SLOTS stages are in LDS. A stage is two phases of 32 elements of K: a phase multiplies one register
+// set of fragments, reads the next phase's from LDS into the other set and takes part in the loads, all in
+// the order written (sched_barrier). There is one wait and one barrier a stage, between its
+// phases: there every wave has read the whole stage, whose slot the loads of SLOTS stages on then take, and
+// stage t + 1 has landed, with SLOTS - 2 stages left in flight; the waits and barriers are bare
+// instructions, since a fence would wait for every load in flight. The lower half of the x fragments
+// has one register set: a row block's is read again when its products are issued.
+//
+// What bounds it. Inside a tile: with every load taken out the 1.5B shape's gate/up product of 2048
+// rows takes 0.85 of its time, of 160 rows 0.6. A compute unit takes in 43 GB/s from memory, 80 from L2, however
+// deep the ring is (its 32 KB L1 holds a line for every load in flight, and answers in order), so a tile's
+// loads go with (MB + NB) K, and its matrix instructions with MB NB K. Around it: a tile's first
+// loads, its gate and its stores, 5 us a
+// tile of 256 x 288, which only the next tile's first loads overlap. So few large tiles beat many small ones, in whole
+// rounds over the units. Gate/up of the 1.5B shape, us by 256 x 192 tiles in stages of 32 -> here (tiles): 2048 rows
+// 110 -> 99 (256 x 288, 504 in two rounds: 1.14 PFLOP/s), 1000 rows 70 -> 50 (256 x 288, 252 in one), 512 rows 37.3 -> 36.5
+// (256 x 192, 188), 336 rows 35.6 -> 25.7 (192 x 160, 224), 160 rows 26.9 (64 x 128 below) -> 21.9 (160 x 96, 187). Two workgroups a unit of
+// half the LDS each, to overlap one's gate with the other's products, gain nothing (2048 rows: 110).
 //
 // The workgroups of a launch are dealt to the 8 XCDs in turn; each XCD takes a run of consecutive
-// tiles (8 row tiles by 4 W tiles at a time: 176 KB a stage through one L2), each workgroup every
-// 32nd tile of the run. Before a workgroup stores a tile it asks for the first four stages of its
-// next one, which arrive while the results go out. A lane holds 4 columns of a row; two blocks
-// change places between lane rows (v_permlane16_swap) so that it stores 16 bytes and four lanes
-// 64 bytes of a row.
+// tiles (8 row tiles by 4 W tiles at a time), each workgroup every
+// 32nd tile of the run. Before a workgroup stores a tile it asks for the first stages of its
+// next one, which arrive while the results go out.
+//
+// The rows of W are dealt to the 16 rows of a wave's blocks so that a lane ends up with neighbouring columns
+// (wide_col). MODE 2: a block is 8 gate rows and the 8 up rows with the same indices, whose values a
+// v_permlane32_swap of two blocks brings into one lane; four blocks give a lane 8 neighbouring outputs.
 //
 // MODE as above (2 with ``act`` > 0: the clipped gated activation of that limit, -1: max(gate, 0) * up, -2: gelu_tanh(gate) * up), and 5: MODE 0 with
 // max(y, 0)^2, with ``act`` > 0 the tanh form of GELU, applied to the float32 sums (after the bias);
@@ -282,18 +288,12 @@ CW_EXPORT int cw_gemm_bf16_tiled(int mode, const void* X, int64_t ldx, const voi
 // [k_splits, M, N] that the next norm kernel adds up in their order.
 typedef __attribute__((ext_vector_type(2))) float f32x2_t;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
+typedef __attribute__((ext_vector_type(2))) unsigned int w_u32x2_t;
 typedef __attribute__((address_space(3))) void lds_void_t;
 
-#define W_NB 6                             // blocks of 16 W rows per wave
-#define W_BM 256
-#define W_BN (32 * W_NB)
-#define W_BK 32
-#define W_BLOCK 1024                       // bytes of a fragment block: 16 rows x 32 elements
-#define W_XHALF (16 * W_BLOCK)             // x of a stage: 256 rows x 32 elements
-#define W_WHALF (2 * W_NB * W_BLOCK)
-#define W_STAGE (W_XHALF + W_WHALF)
-#define W_SLOTS 5
-#define W_LOADS (4 + W_NB / 2)             // loads of a wave per stage
+#define W_BM 256                           // the tile of the grouped products and of cw_gemm_bf16_wide_tiles
+#define W_BN 192
+#define W_BLOCK 1024                       // bytes of a block: 8 rows x 64 elements
 #define W_GROUP_M 8                        // row tiles that run side by side
 
 struct WideArgs {
@@ -316,31 +316,43 @@ struct WideArgs {
   float act;                // MODE 2 and 5: which activation (see above)
 };
 
-// Row of W that row ``rb`` of W tile ``tn`` is. MODE 2: a wave's 96 rows are 48 gate rows followed
-// by the up rows with the same indices.
-template <int MODE>
-__device__ __forceinline__ int64_t w_row_of(int tn, int rb, int N) {
-  if (MODE == 2) {
-    const int I = N / 2;
-    const int wn = rb / (W_BN / 2), q = rb % (W_BN / 2);
-    const int64_t i = (int64_t)tn * (W_BN / 2) + wn * (W_BN / 4) + (q % (W_BN / 4));
-    return (q < W_BN / 4 ? i : I + i);
+// The column of a wave's part of the tile (MODE 2: the output) that row r of its W block ni belongs to. The
+// accumulator of a block holds rows 4 s .. 4 s + 3 in lane (c, s). Two blocks: 8 neighbouring columns a lane. MODE 2,
+// where s of 0 and 1 hold gates and s of 2 and 3 the ups to them: after the swap of two blocks lane s has 4 outputs, of four
+// blocks 8; what is left over keeps its order.
+template <int MODE, int NB>
+__host__ __device__ __forceinline__ int wide_col(int ni, int r) {
+  const int s = r >> 2, e = r & 3;
+  if (MODE == 2 || MODE == 4) {
+    const int s1 = s & 1;
+    if (ni < (NB & ~3)) return (ni >> 2) * 32 + ((ni & 1) * 2 + s1) * 8 + ((ni >> 1) & 1) * 4 + e;
+    if ((NB & 2) && ni < (NB & ~1)) return (NB & ~3) * 8 + ((ni & 1) * 2 + s1) * 4 + e;
+    return (NB - 1) * 8 + s1 * 4 + e;
   }
-  return (int64_t)tn * W_BN + rb;
+  return ni < (NB & ~1) ? (ni >> 1) * 32 + s * 8 + (ni & 1) * 4 + e : ni * 16 + r;
 }
-
-// Which of a row's four 16-byte granules changes places with which in LDS: rows that lie 128 or 256
-// bytes apart (r + 2, r + 4, ...) get different values, so that 8 or 16 lanes that read the same
-// granule of neighbouring rows touch every bank once.
-__device__ __forceinline__ int w_swizzle(int r) { return (((r >> 1) ^ (r >> 3)) & 1) | (((r >> 2) & 1) << 1); }
 
 __device__ __forceinline__ uint32_t w_pack_bf16(float lo, float hi) {
   const f32x2_t v = {lo, hi};
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));  // v_cvt_pk_bf16_f32
 }
 
+// cw_gated from the bare exp2 and reciprocal instructions
+__device__ __forceinline__ float w_gated(float g, float up, float act) {
+  if (act > 0.0f) {
+    const float gl = fminf(g, act), ul = fminf(fmaxf(up, -act), act);
+    return gl * __builtin_amdgcn_rcpf(1.0f + __expf(-1.702f * gl)) * (ul + 1.0f);
+  }
+  if (act < 0.0f) {
+    const float logistic = __builtin_amdgcn_rcpf(1.0f + __expf(-1.5957691216057308f * (g + 0.044715f * g * g * g)));
+    return (act < -1.5f ? g * logistic : fmaxf(g, 0.0f)) * up;
+  }
+  return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * up;
+}
+
 // s_waitcnt for "at most n vector-memory operations in flight" and nothing else
 #define W_WAIT_LOADS(n) __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | (((n) >> 4) << 14))
+#define W_WAIT_LDS() __builtin_amdgcn_s_waitcnt(0xC07F)  // every LDS read of this wave is back
 // a barrier without a fence: what it orders is said at each use
 #define W_BARRIER()                 \
   do {                              \
@@ -349,15 +361,20 @@ __device__ __forceinline__ uint32_t w_pack_bf16(float lo, float hi) {
     asm volatile("" ::: "memory"); \
   } while (0)
 
-template <int MODE, bool GROUPED = false>
+template <int MODE, int MB, int NB, int SLOTS, bool ANY_ROWS = true, bool GROUPED = false>
 __global__ __launch_bounds__(256) void gemm_wide_bf16_kernel(WideArgs a) {
   extern __shared__ __align__(1024) unsigned char w_smem[];
+  constexpr bool GATED = MODE == 2 || MODE == 4;
+  constexpr int BM = 32 * MB, BN = 32 * NB, PER = GATED ? BN / 2 : BN;  // PER: columns of the result
+  constexpr int LOADS = MB + NB;                                            // of a wave and stage: MB of x, NB of W
+  constexpr int STAGE = 4 * LOADS * W_BLOCK;
+  static_assert(SLOTS >= 2 && SLOTS * STAGE <= 160 * 1024 && SLOTS * LOADS <= 63, "the ring is the LDS of a compute unit");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   const int c = lane & 15, s = lane >> 4;
   // GROUPED: the number of row tiles is known on the device alone; x holds whole tiles
   const int tiles_m = GROUPED ? __builtin_amdgcn_readfirstlane(*a.n_row_tiles) : a.tiles_m;
-  const int M = GROUPED ? tiles_m * W_BM : a.M, N = a.N, K = a.K;
+  const int M = GROUPED ? tiles_m * BM : a.M, N = a.N, K = a.K, I = N / 2;
   const int per_split = tiles_m * a.tiles_n;
   const int total = per_split * (MODE == 3 ? a.k_splits : 1);
   const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3, per_xcd = gridDim.x >> 3;
@@ -374,24 +391,30 @@ __global__ __launch_bounds__(256) void gemm_wide_bf16_kernel(WideArgs a) {
     *tm = group * W_GROUP_M + (within - *tn * rows);
   };
 
-  uint32_t xo[4], wo[W_NB / 2];
-  const int lrow = lane >> 2, lsub = (lane & 3) ^ w_swizzle(lane >> 2);
-#pragma unroll
-  for (int j = 0; j < 4; ++j) xo[j] = (uint32_t)(((int64_t)(wave * 64 + j * 16 + lrow) * a.ldx + lsub * 8) * 2);
-#pragma unroll
-  for (int j = 0; j < W_NB / 2; ++j) {
-    const int64_t n = w_row_of<MODE>(0, wave * (W_BN / 4) + j * 16 + lrow, N);  // the same in every tile
-    wo[j] = (uint32_t)((n * K + lsub * 8) * 2);
-  }
-  const int k_run = MODE == 3 ? K / a.k_splits : K;  // elements of K that one work item sums
-  const int k_tiles = k_run / W_BK;
+  // Load i of a wave: MB blocks of x, every fourth, then the NB blocks of its half of W that hold the first or the last 8 rows
+  // of the fragments. Lane: granule (lane & 7) of row lane / 8 of a block. The rows of a wave's loads lie fixed numbers of rows
+  // apart, so few registers of addresses do (with 17 of them the widest tile's spilled, 5 us a tile).
+  const int parity = wave & 1, half = wave >> 1, r = parity * 8 + (lane >> 3);
+  const uint32_t granule_in = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+  const uint32_t x_at = (uint32_t)((int64_t)(half * 16 + r) * a.ldx * 2) + granule_in, x_step = (uint32_t)a.ldx * 64, w_row = (uint32_t)K * 2;
+  constexpr int REGULAR = GATED ? NB & ~3 : NB & ~1;  // blocks whose rows wide_col deals alike; the others one more register
+  auto w_first = [&](int ni) __attribute__((always_inline)) {
+    const int col = half * (PER / 2) + wide_col<MODE, NB>(ni, r) - wide_col<MODE, NB>(ni, 0);
+    return (uint32_t)((int64_t)(GATED && parity ? I + col : col) * K * 2) + granule_in;
+  };
+  const uint32_t w_at = w_first(0), w_at_rest = w_first(NB - 1);
+  // stages of K before work item id's run
+  auto stages_before = [&](int plane) __attribute__((always_inline)) { return MODE == 3 ? (int)((int64_t)(K / 64) * plane / a.k_splits) : 0; };
+  int stages;  // of the work item that comes in
   __amdgpu_buffer_rsrc_t xr, wr;
   auto aim = [&](int id) __attribute__((always_inline)) {
     int tm, tn;
     tile_of(id, &tm, &tn);
-    const int64_t k0 = MODE == 3 ? (int64_t)(id / per_split) * k_run : 0;
-    const int64_t x_row0 = (int64_t)tm * W_BM;
-    const int64_t w_row0 = w_row_of<MODE>(tn, 0, N);
+    const int plane = MODE == 3 ? id / per_split : 0;
+    const int64_t k0 = (int64_t)stages_before(plane) * 64;
+    stages = MODE == 3 ? stages_before(plane + 1) - stages_before(plane) : K / 64;
+    const int k_run = stages * 64;
+    const int64_t x_row0 = (int64_t)tm * BM, w_row0 = (int64_t)tn * PER;
     // the descriptors begin at the run's first element of the tile's first row and end with the
     // run's last element of the matrix's last row: rows past the end read as zeros
     xr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.X + x_row0 * a.ldx + k0), 0,
@@ -400,227 +423,294 @@ __global__ __launch_bounds__(256) void gemm_wide_bf16_kernel(WideArgs a) {
     wr = __builtin_amdgcn_make_buffer_rsrc((void*)(w_base + w_row0 * K + k0), 0,
                                            (int)(uint32_t)(((N - w_row0 - 1) * (int64_t)K + k_run) * 2), 0x00020000);
   };
-  // load i of a wave's W_LOADS for stage kt: its four x blocks, then its three W blocks
-  auto fetch_one = [&](int kt, int i) __attribute__((always_inline)) {
-    unsigned char* slot = w_smem + (kt % W_SLOTS) * W_STAGE;
-    if (i < 4)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t*)(slot + (wave * 4 + i) * W_BLOCK), 16, xo[i], kt * (W_BK * 2), 0, 0);
-    else
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void_t*)(slot + W_XHALF + (wave * (W_NB / 2) + i - 4) * W_BLOCK), 16,
-                                               wo[i - 4], kt * (W_BK * 2), 0, 0);
+  auto fetch_one = [&](int stage, int slot, int i) __attribute__((always_inline)) {
+    uint32_t apart = i < MB ? i * x_step : wide_col<MODE, NB>(i - MB, 0) * w_row;
+    asm volatile("" : "+s"(apart));  // added here and now: the sums of all loads would take as many registers
+    if (i < MB) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t*)(w_smem + slot + (i * 4 + wave) * W_BLOCK), 16, x_at + apart, stage * 128, 0, 0);
+    } else {
+      const int ni = i - MB;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void_t*)(w_smem + slot + (4 * MB + (half * NB + ni) * 2 + parity) * W_BLOCK), 16,
+                                               (ni < REGULAR ? w_at : w_at_rest) + apart, stage * 128, 0, 0);
+    }
   };
+  // (of fewer stages than slots the last comes in again: the number of loads in flight is what the waits count on)
   auto fetch_first_stages = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < W_LOADS; ++i) {
-      fetch_one(0, i);
-      fetch_one(1, i);
-    }
+    for (int j = 0; j < SLOTS; ++j)
 #pragma unroll
-    for (int i = 0; i < W_LOADS; ++i) {
-      fetch_one(2, i);
-      fetch_one(3, i);
-    }
+      for (int i = 0; i < LOADS; ++i) fetch_one(min(j, stages - 1), j * STAGE, i);
   };
 
-  f32x4_t acc[8][W_NB];
-  bf16x8_t xf[2][8], wf[2][W_NB];
-  // read i of the 8 + W_NB fragment reads of a stage: W first, in the order of their use
-  auto read_one = [&](int kt, int set, int i) __attribute__((always_inline)) {
-    const unsigned char* slot = w_smem + (kt % W_SLOTS) * W_STAGE + c * 64 + ((s ^ w_swizzle(c)) * 16);
-    if (i < W_NB) wf[set][i] = *reinterpret_cast<const bf16x8_t*>(slot + W_XHALF + (wn * W_NB + i) * W_BLOCK);
-    else xf[set][i - W_NB] = *reinterpret_cast<const bf16x8_t*>(slot + (wm * 8 + i - W_NB) * W_BLOCK);
+  constexpr int PRODUCTS = MB * NB, READS = MB + NB;
+  f32x4_t acc[MB][NB];
+  bf16x8_t xf[2][MB], wf[2][NB];
+  auto x_set = [](int set, int mi) __attribute__((always_inline)) { return mi < MB / 2 ? 0 : set; };
+  const unsigned char* x_base = w_smem + c * 128 + wm * MB * 2048;
+  const unsigned char* w_base = w_smem + c * 128 + (2 * MB + wn * NB) * 2048;
+  const int granule[2] = {((s) ^ ((c >> 1) & 7)) * 16, ((4 + s) ^ ((c >> 1) & 7)) * 16};
+  // read i of a phase's fragments: W first, x in the order of its use
+  auto read_one = [&](int slot, int half, int set, int i) __attribute__((always_inline)) {
+    if (i < NB) wf[set][i] = *reinterpret_cast<const bf16x8_t*>(w_base + slot + granule[half] + i * 2048);
+    else xf[x_set(set, i - NB)][i - NB] = *reinterpret_cast<const bf16x8_t*>(x_base + slot + granule[half] + (i - NB) * 2048);
   };
-  // Iteration t, as described above. ``set`` is t % 2: the register set of stage t's fragments.
-  auto iteration = [&](int t, auto set_c, auto fetch_c, auto read_c) __attribute__((always_inline)) {
-    constexpr int set = decltype(set_c)::value;
-    constexpr bool with_fetch = decltype(fetch_c)::value, with_read = decltype(read_c)::value;
+  // One phase: the products of register set ``set``; with_read: the next phase's fragments, of half ``half`` of the stage
+  // in ``read_slot``; loads from .. to of the wave's for stage ``stage`` into ``load_slot``.
+  auto phase = [&](auto set_c, auto read_c, int read_slot, int half, auto from_c, auto to_c, int stage, int load_slot) __attribute__((always_inline)) {
+    constexpr int set = decltype(set_c)::value, from = decltype(from_c)::value, count = decltype(to_c)::value - from;
+    constexpr bool with_read = decltype(read_c)::value;
 #pragma unroll
-    for (int g = 0; g < 16; ++g) {
-      const int mi = g >> 1;
+    for (int g = 0; g < PRODUCTS; ++g) {
+      const int mi = g / NB, ni = g % NB;
+      if constexpr (PRODUCTS <= 64) {
+        acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[set][ni], xf[x_set(set, mi)][mi], acc[mi][ni], 0, 0, 0);
+      } else {
+        // More accumulators than there are accumulation registers: 62 live there and the others with the operands. Left to
+        // itself the compiler keeps all in one kind and moves a hundred of them back and forth an iteration.
+        if (g < 62) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[mi][ni]) : "v"(wf[set][ni]), "v"(xf[x_set(set, mi)][mi]));
+        else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[mi][ni]) : "v"(wf[set][ni]), "v"(xf[x_set(set, mi)][mi]));
+      }
+      // reads and loads spread over the products (the texture path takes a load every 16 cycles; several in a row stall
+      // the wave), the reads done a little before the end
+      constexpr int SPAN = PRODUCTS - 3;
+      const int r0 = min(g * READS / SPAN, READS), r1 = min((g + 1) * READS / SPAN, READS);
+      const int l0 = (2 * g + 1) * count / (2 * PRODUCTS), l1 = (2 * g + 3) * count / (2 * PRODUCTS);
+      if ((with_read && r0 < r1) || l0 < l1) {
+        // the order of issue is the order written here: the scheduler may move nothing across
+        __builtin_amdgcn_sched_barrier(0);
+        if (with_read)
 #pragma unroll
-      for (int q = 0; q < W_NB / 2; ++q) {
-        const int ni = (g & 1) * (W_NB / 2) + q;
-        acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[set][ni], xf[set][mi], acc[mi][ni], 0, 0, 0);
+          for (int r = r0; r < r1; ++r) read_one(read_slot, half, set ^ 1, r);
+#pragma unroll
+        for (int l = l0; l < l1; ++l) fetch_one(stage, load_slot, from + l);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      // the order of issue is the order written here: the scheduler may move nothing across
-      __builtin_amdgcn_sched_barrier(0);
-      if (with_read && g < 8 + W_NB) read_one(t + 1, set ^ 1, g);
-      if (with_fetch && (g & 1) == 0) {
-        // a load after every second group: four pairs of loads in the even iteration, three in the
-        // odd one, the two halves of a line six matrix instructions apart
-        const int i = (g >> 2) + (set ? 4 : 0);
-        if (i < W_LOADS) fetch_one(t + 4 - set + ((g >> 1) & 1), i);
-      }
-      __builtin_amdgcn_sched_barrier(0);
     }
-    if (set == 0) {
-      if (with_fetch) W_WAIT_LOADS(8);  // all but the 8 loads just issued: stages t + 2 and t + 3 are in
-      else W_WAIT_LOADS(0);
-    } else {
-      // the next iteration asks for stage t + 6, which lands in the slot of stage t + 1: this wave's
-      // fragment reads of that stage (issued above) have to be back before any wave may do so
-      __builtin_amdgcn_s_waitcnt(0xC07F);
-    }
-    // every wave's loads of stage t + 2 are in LDS, and every wave has read stage t + 1
-    W_BARRIER();
+    // what the compiler does not know of products that it has not written: their results need this long before a move of
+    // accumulators (at the loop's ends) may read them
+    if constexpr (PRODUCTS > 64) asm volatile("s_nop 15" ::: "memory");
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
+  using Last = std::integral_constant<int, LOADS>;
+  // two slots: all loads in the phase behind the barrier, else half of them in the next one
+  using Split = std::integral_constant<int, SLOTS == 2 ? LOADS : (LOADS + 1) / 2>;
   using Yes = std::true_type;
   using No = std::false_type;
+  auto next_slot = [](int slot) __attribute__((always_inline)) { return slot == (SLOTS - 1) * STAGE ? 0 : slot + STAGE; };
 
   int id = run_begin + local;
   if (id >= run_end) return;
   aim(id);
   fetch_first_stages();
-  for (; id < run_end; id += per_xcd) {
+  for (bool first = true; id < run_end; id += per_xcd, first = false) {
     int tm, tn;
     tile_of(id, &tm, &tn);
 #pragma unroll
-    for (int mi = 0; mi < 8; ++mi)
+    for (int mi = 0; mi < MB; ++mi)
 #pragma unroll
-      for (int ni = 0; ni < W_NB; ++ni) acc[mi][ni] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
-    W_WAIT_LOADS(0);
-    W_BARRIER();  // the first four stages are in LDS
-#pragma unroll
-    for (int i = 0; i < 8 + W_NB; ++i) read_one(0, 0, i);
-    // the first iteration's loads go into stage 0's slot: every wave has to have read it
-    __builtin_amdgcn_s_waitcnt(0xC07F);
+      for (int ni = 0; ni < NB; ++ni) acc[mi][ni] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
+    // the first stage is in LDS (a tile's stores come after its successor's loads, and count as well)
+    if (first) W_WAIT_LOADS((SLOTS - 1) * LOADS);
+    else W_WAIT_LOADS(0);
     W_BARRIER();
-    int t = 0;
-    for (; t + 4 < k_tiles; t += 2) {
-      iteration(t, I0{}, Yes{}, Yes{});
-      iteration(t + 1, I1{}, Yes{}, Yes{});
+#pragma unroll
+    for (int i = 0; i < READS; ++i) read_one(0, 0, 0, i);
+    int slot = 0, t = 0;
+    phase(I0{}, Yes{}, slot, 1, I0{}, I0{}, 0, 0);
+    // every wave has read stage t and its loads of stage t + 1 have landed
+    W_WAIT_LOADS((SLOTS - 2) * LOADS);
+    W_WAIT_LDS();
+    W_BARRIER();
+    for (; t + SLOTS < stages; ++t) {
+      const int next = next_slot(slot);
+      phase(I1{}, Yes{}, next, 0, I0{}, Split{}, t + SLOTS, slot);
+      phase(I0{}, Yes{}, next, 1, Split{}, Last{}, t + SLOTS, slot);
+      W_WAIT_LOADS((SLOTS - 2) * LOADS);
+      W_WAIT_LDS();
+      W_BARRIER();
+      slot = next;
     }
-    iteration(t, I0{}, No{}, Yes{});
-    iteration(t + 1, I1{}, No{}, Yes{});
-    iteration(t + 2, I0{}, No{}, Yes{});
-    iteration(t + 3, I1{}, No{}, No{});
+    W_WAIT_LOADS(0);
+    W_BARRIER();  // the last stages are in
+    for (; t + 1 < stages; ++t) {
+      const int next = next_slot(slot);
+      phase(I1{}, Yes{}, next, 0, I0{}, I0{}, 0, 0);
+      phase(I0{}, Yes{}, next, 1, I0{}, I0{}, 0, 0);
+      slot = next;
+    }
+    phase(I1{}, No{}, 0, 0, I0{}, I0{}, 0, 0);
+    W_WAIT_LDS();
+    W_BARRIER();
     // every slot is free: the first stages of the next tile come in while this one's results go out
     if (id + per_xcd < run_end) {
       aim(id + per_xcd);
       fetch_first_stages();
     }
 
-    // ---- lane (c, s) holds y[m = .. + mi * 16 + c][4 s + e of W block ni], e = 0..3
-    const int I = N / 2;
-    const int out_cols = MODE == 2 ? I : N;
-    constexpr int OUT_BLOCKS = MODE == 2 ? W_NB / 2 : W_NB;
-    const int64_t col0 = MODE == 2 ? (int64_t)tn * (W_BN / 2) + wn * (W_BN / 4) : (int64_t)tn * W_BN + wn * (W_BN / 2);
-    float row_factor = 1.0f;  // GROUPED: of the row that is being stored
-    auto packed = [&](int mi, int ni, uint32_t* lo, uint32_t* hi) __attribute__((always_inline)) {
-      float v[4];
+    const int out_cols = GATED ? I : N;
+    constexpr int ELEMENT = MODE == 3 ? 4 : 2;
+    unsigned char* C = (unsigned char*)a.C + (MODE == 3 ? (int64_t)(id / per_split) * M * a.ldc * 4 : 0);
+    const int64_t row0 = (int64_t)tm * BM + wm * (16 * MB);
+    const int col0 = tn * PER + wn * (PER / 2);
+    // Rows of 16-byte multiples: buffer stores, whose descriptor ends with the last row and drops what is told to lie beyond, so
+    // nothing branches at a store. (With branches the last tile of a row, 32 of 96 columns, took the 1.5B shape's product of 512
+    // rows from 36 to 43 us.)
+    // ANY_ROWS: any other rows too, a value a store. (One kernel for both, with the activations besides, keeps so much alive that
+    // the widest tile's registers spill, 5 us a tile: it has neither.)
+    const bool whole = !ANY_ROWS || !(a.ldc & (16 / ELEMENT - 1)) && !((uintptr_t)a.C & 15) && !(out_cols & (16 / ELEMENT - 1)) && a.ldc < (1 << 20);
+    const __amdgpu_buffer_rsrc_t cr = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(C + ((int64_t)tm * BM * a.ldc + tn * PER) * ELEMENT), 0,
+        (int)(uint32_t)((min((int64_t)M - (int64_t)tm * BM - 1, (int64_t)BM) * a.ldc + min(PER, out_cols - tn * PER)) * ELEMENT), 0x00020000);
+    const uint32_t c_row = (uint32_t)(((wm * 16 * MB + c) * a.ldc + wn * (PER / 2)) * ELEMENT), c_step = (uint32_t)(16 * a.ldc * ELEMENT);
+    // count neighbouring columns from column n of the wave's part on, in row block mi
+    auto store_whole = [&](int mi, uint32_t more, int n, const float* v, auto count_c) __attribute__((always_inline)) {
+      constexpr int count = decltype(count_c)::value;
+      const uint32_t to = col0 + n < out_cols ? c_row + mi * c_step + more + n * ELEMENT : 0x80000000u;
+      if constexpr (MODE == 3) {
+        const f32x4_t v4 = {v[0], v[1], v[2], v[3]};
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v4), cr, to, 0, 0);
+      } else if constexpr (count == 8) {
+        const u32x4_t w4 = {w_pack_bf16(v[0], v[1]), w_pack_bf16(v[2], v[3]), w_pack_bf16(v[4], v[5]), w_pack_bf16(v[6], v[7])};
+        __builtin_amdgcn_raw_buffer_store_b128(w4, cr, to, 0, 0);
+      } else {
+        const w_u32x2_t w2 = {w_pack_bf16(v[0], v[1]), w_pack_bf16(v[2], v[3])};
+        __builtin_amdgcn_raw_buffer_store_b64(w2, cr, to, 0, 0);
+      }
+    };
+    // the same for any tile: row m of C
+    auto store = [&](int64_t m, bool live, int n, const float* v, auto count_c) __attribute__((always_inline)) {
+      constexpr int count = decltype(count_c)::value;
+      if (!live) return;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (MODE == 2) {
-          const float g = acc[mi][ni][e], up = acc[mi][ni + W_NB / 2][e];
-          if (a.act > 0.0f) {
-            const float gl = fminf(g, a.act), ul = fminf(fmaxf(up, -a.act), a.act);
-            v[e] = gl * __builtin_amdgcn_rcpf(1.0f + __expf(-1.702f * gl)) * (ul + 1.0f);
-          } else if (a.act < 0.0f) {
-            const float logistic = __builtin_amdgcn_rcpf(1.0f + __expf(-1.5957691216057308f * (g + 0.044715f * g * g * g)));
-            v[e] = (a.act < -1.5f ? g * logistic : fmaxf(g, 0.0f)) * up;
-          } else {
-            v[e] = g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * up;
+      for (int e = 0; e < count; ++e) {
+        if (col0 + n + e >= out_cols) continue;
+        if constexpr (MODE == 3) ((float*)C)[m * a.ldc + col0 + n + e] = v[e];
+        else ((uint16_t*)C)[m * a.ldc + col0 + n + e] = (uint16_t)w_pack_bf16(v[e], 0.0f);
+      }
+    };
+    using Four = std::integral_constant<int, 4>;
+    using Eight = std::integral_constant<int, 8>;
+    if constexpr (GATED) {
+      auto all = [&](auto whole_c) __attribute__((always_inline)) {
+        constexpr bool whole_tile = decltype(whole_c)::value;
+        // gates of two accumulators and the ups to them, each in one lane
+        auto gated = [&](const f32x4_t& p, const f32x4_t& q, float* v) __attribute__((always_inline)) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const cw_u32x2_t gu = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[e]), __float_as_uint(q[e]), false, false);
+            v[e] = w_gated(__uint_as_float(gu[0]), __uint_as_float(gu[1]), MODE == 2 ? 0.0f : a.act);
           }
-        } else {
-          v[e] = acc[mi][ni][e];
-          const int64_t n = col0 + ni * 16 + 4 * s + e;
-          if (a.bias != nullptr && n < N)
-            v[e] += a.bias_f32 ? ((const float*)a.bias)[n] : __bfloat162float(((const bf16_t*)a.bias)[n]);
-          if (GROUPED) v[e] *= row_factor;
-          if (MODE == 5) {
-            if (a.act > 0.0f) {
-              v[e] *= __builtin_amdgcn_rcpf(1.0f + __expf(-1.5957691216057308f * (v[e] + 0.044715f * v[e] * v[e] * v[e])));
+        };
+#pragma unroll
+        for (int mi = 0; mi < MB; ++mi) {
+          const int64_t m = row0 + mi * 16 + c;
+#pragma unroll
+          for (int q = 0; q + 3 < NB; q += 4) {
+            float v[8];
+            gated(acc[mi][q], acc[mi][q + 1], v);
+            gated(acc[mi][q + 2], acc[mi][q + 3], v + 4);
+            if (whole_tile) store_whole(mi, 0, q * 8 + s * 8, v, Eight{});
+            else store(m, m < M, q * 8 + s * 8, v, Eight{});
+          }
+          if constexpr ((NB & 2) != 0) {
+            float v[4];
+            gated(acc[mi][NB & ~3], acc[mi][(NB & ~3) + 1], v);
+            if (whole_tile) store_whole(mi, 0, (NB & ~3) * 8 + s * 4, v, Four{});
+            else store(m, m < M, (NB & ~3) * 8 + s * 4, v, Four{});
+          }
+          if ((NB & 1) && !(mi & 1)) {
+            // the last block alone: of this row block and of the next, if there is one
+            const int other = mi + 1 < MB ? mi + 1 : mi;
+            const int64_t m2 = m + (s >> 1) * 16;
+            float v[4];
+            gated(acc[mi][NB - 1], acc[other][NB - 1], v);
+            if (whole_tile) {
+              if (s < 2 || other != mi) store_whole(mi, (s >> 1) * c_step, (NB - 1) * 8 + (s & 1) * 4, v, Four{});
             } else {
-              const float r = fmaxf(v[e], 0.0f);
-              v[e] = r * r;
+              store(m2, m2 < M && (s < 2 || other != mi), (NB - 1) * 8 + (s & 1) * 4, v, Four{});
             }
           }
         }
-      }
-      *lo = w_pack_bf16(v[0], v[1]);
-      *hi = w_pack_bf16(v[2], v[3]);
-    };
-    if constexpr (MODE == 3) {
-      // the lane's four neighbouring columns of a row as they are: 16 bytes of the run's plane
-      float* plane = (float*)a.C + (int64_t)(id / per_split) * M * a.ldc;
-      const bool vec_ok = !(a.ldc & 3) && !((uintptr_t)a.C & 15);
+      };
+      if (whole) all(Yes{});
+      else if constexpr (ANY_ROWS) all(No{});
+    } else {
+      auto all = [&](auto whole_c) __attribute__((always_inline)) {
+        constexpr bool whole_tile = decltype(whole_c)::value;
 #pragma unroll
-      for (int mi = 0; mi < 8; ++mi) {
-        const int64_t m = (int64_t)tm * W_BM + wm * 128 + mi * 16 + c;
-        if (m >= M) continue;
+        for (int mi = 0; mi < MB; ++mi) {
+          int64_t m = row0 + mi * 16 + c;
+          bool live = m < M;
+          float row_factor = 1.0f;  // GROUPED: of the row that is being stored
+          if (GROUPED && a.row_target != nullptr) {
+            const int target = live ? a.row_target[m] : -1;
+            live = target >= 0;
+            row_factor = (live && a.row_factor != nullptr) ? a.row_factor[target] : 1.0f;
+            m = live ? target : 0;
+          }
+          auto value = [&](int ni, float* v) __attribute__((always_inline)) {
+            const int n0 = col0 + wide_col<MODE, NB>(ni, 4 * s);
 #pragma unroll
-        for (int ni = 0; ni < W_NB; ++ni) {
-          const int64_t n0 = col0 + ni * 16 + 4 * s;
-          if (n0 >= N) continue;
-          float* dst = plane + m * a.ldc + n0;
-          if (n0 + 4 <= N && vec_ok) {
-            *reinterpret_cast<f32x4_t*>(dst) = acc[mi][ni];
-          } else {
+            for (int e = 0; e < 4; ++e) {
+              v[e] = acc[mi][ni][e];
+              if (MODE == 3) continue;
+              if (a.bias != nullptr && n0 + e < N)
+                v[e] += a.bias_f32 ? ((const float*)a.bias)[n0 + e] : __bfloat162float(((const bf16_t*)a.bias)[n0 + e]);
+              if (GROUPED) v[e] *= row_factor;
+              if (MODE == 5) {
+                if (a.act > 0.0f) {
+                  v[e] *= __builtin_amdgcn_rcpf(1.0f + __expf(-1.5957691216057308f * (v[e] + 0.044715f * v[e] * v[e] * v[e])));
+                } else {
+                  const float r = fmaxf(v[e], 0.0f);
+                  v[e] = r * r;
+                }
+              }
+            }
+          };
+          // GROUPED with targets: the rows lie apart
+          auto put = [&](int n, const float* v, auto count_c) __attribute__((always_inline)) {
+            if constexpr (GROUPED) {
+              if (whole_tile) {
+                if (live && col0 + n < out_cols) {
+                  uint16_t* to = (uint16_t*)C + m * a.ldc + col0 + n;
+                  if constexpr (decltype(count_c)::value == 8)
+                    *reinterpret_cast<uint4*>(to) = make_uint4(w_pack_bf16(v[0], v[1]), w_pack_bf16(v[2], v[3]), w_pack_bf16(v[4], v[5]), w_pack_bf16(v[6], v[7]));
+                  else
+                    *reinterpret_cast<uint2*>(to) = make_uint2(w_pack_bf16(v[0], v[1]), w_pack_bf16(v[2], v[3]));
+                }
+              } else {
+                store(m, live, n, v, count_c);
+              }
+            } else {
+              if (whole_tile) store_whole(mi, 0, n, v, count_c);
+              else store(m, live, n, v, count_c);
+            }
+          };
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (n0 + e < N) dst[e] = acc[mi][ni][e];
+          for (int ni = 0; ni + 1 < NB; ni += 2) {
+            float v[8];
+            value(ni, v);
+            value(ni + 1, v + 4);
+            if constexpr (MODE == 3) {
+              put(ni * 16 + s * 8, v, Four{});
+              put(ni * 16 + s * 8 + 4, v + 4, Four{});
+            } else {
+              put(ni * 16 + s * 8, v, Eight{});
+            }
+          }
+          if constexpr ((NB & 1) != 0) {
+            float v[4];
+            value(NB - 1, v);
+            put((NB - 1) * 16 + s * 4, v, Four{});
           }
         }
-      }
-      continue;
-    }
-    const bool wide_ok = !(a.ldc & 7) && !((uintptr_t)a.C & 15);
-#pragma unroll
-    for (int mi = 0; mi < 8; ++mi) {
-      int64_t m = (int64_t)tm * W_BM + wm * 128 + mi * 16 + c;
-      bool live = m < M;
-      if (GROUPED && a.row_target != nullptr) {
-        // the permutes below exchange values between the lanes of one row, so a lane whose row is
-        // not stored still takes part in them
-        const int target = live ? a.row_target[m] : -1;
-        live = target >= 0;
-        row_factor = (live && a.row_factor != nullptr) ? a.row_factor[target] : 1.0f;
-        m = live ? target : 0;
-      }
-#pragma unroll
-      for (int ni = 0; ni + 1 < OUT_BLOCKS; ni += 2) {
-        uint32_t a_lo, a_hi, b_lo, b_hi;
-        packed(mi, ni, &a_lo, &a_hi);
-        packed(mi, ni + 1, &b_lo, &b_hi);
-        // lane rows 1 and 3 of the first take lane rows 0 and 2 of the second: the lane then holds
-        // columns 8 (s / 2) .. + 8 of block ni (s even) or of block ni + 1 (s odd)
-        const cw_u32x2_t lo = __builtin_amdgcn_permlane16_swap(a_lo, b_lo, false, false);
-        const cw_u32x2_t hi = __builtin_amdgcn_permlane16_swap(a_hi, b_hi, false, false);
-        const int64_t n0 = col0 + (ni + (s & 1)) * 16 + 8 * (s >> 1);
-        if (!live || n0 >= out_cols) continue;
-        uint16_t* dst = (uint16_t*)a.C + m * a.ldc + n0;
-        const uint32_t w4[4] = {lo[0], hi[0], lo[1], hi[1]};
-        if (n0 + 8 <= out_cols && wide_ok) {
-          *reinterpret_cast<uint4*>(dst) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (n0 + e < out_cols) dst[e] = (uint16_t)(w4[e >> 1] >> ((e & 1) * 16));
-        }
-      }
-      if (OUT_BLOCKS & 1) {
-        constexpr int ni = OUT_BLOCKS - 1;
-        uint32_t lo, hi;
-        packed(mi, ni, &lo, &hi);
-        const int64_t n0 = col0 + ni * 16 + 4 * s;
-        if (!live || n0 >= out_cols) continue;
-        uint16_t* dst = (uint16_t*)a.C + m * a.ldc + n0;
-        if (n0 + 4 <= out_cols && !(a.ldc & 3)) {
-          *reinterpret_cast<uint2*>(dst) = make_uint2(lo, hi);
-        } else {
-          const uint32_t w2[2] = {lo, hi};
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n0 + e < out_cols) dst[e] = (uint16_t)(w2[e >> 1] >> ((e & 1) * 16));
-        }
-      }
+      };
+      if (whole) all(Yes{});
+      else if constexpr (ANY_ROWS) all(No{});
     }
   }
 }
-
-static const size_t W_SMEM = (size_t)W_SLOTS * W_STAGE;
 
 static int w_tiles(int mode, int M, int N) {
   const int out_cols = mode == 2 ? N / 2 : N;
@@ -628,7 +718,7 @@ static int w_tiles(int mode, int M, int N) {
   return ((M + W_BM - 1) / W_BM) * ((out_cols + per_tile - 1) / per_tile);
 }
 
-// Does the wide-tile kernel take this product? Returns its number of tiles, or 0.
+// Does the wide-tile kernel take this product? Returns its number of tiles of 256 x 192, or 0.
 CW_EXPORT int cw_gemm_bf16_wide_tiles(int mode, int M, int N, int K, int64_t ldx) {
   if (M <= 0 || N <= 0 || (mode != 0 && mode != 2 && mode != 5) || (mode == 2 && (N & 1))) return 0;
   if ((K & 63) || K < 256 || (ldx & 7) || ldx < K) return 0;
@@ -642,25 +732,116 @@ CW_EXPORT int cw_gemm_bf16_wide_partial_ok(int M, int N, int K, int64_t ldx, int
   return cw_gemm_bf16_wide_tiles(0, M, N, K, ldx) > 0 ? 1 : 0;
 }
 
-template <int MODE>
-static int w_launch(WideArgs a, int workgroups, hipStream_t stream) {
-  static bool raised = false;
-  if (!raised) {
-    if (hipFuncSetAttribute((const void*)gemm_wide_bf16_kernel<MODE>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)W_SMEM) != hipSuccess)
-      return CW_ERR_LAUNCH;
-    raised = true;
-  }
-  const int out_cols = MODE == 2 ? a.N / 2 : a.N;
-  const int per_tile = MODE == 2 ? W_BN / 2 : W_BN;
+// ``row_tiles``: GROUPED: how many there are at most
+template <int MODE, int MB, int NB, int SLOTS, bool ANY_ROWS = true, bool GROUPED = false>
+static int w_launch(WideArgs a, int row_tiles, int workgroups, hipStream_t stream) {
+  constexpr int SMEM = SLOTS * 4 * (MB + NB) * W_BLOCK;
+  static std::atomic<bool> allowed{false};
+  const int status = cw_allow_lds(allowed, (const void*)gemm_wide_bf16_kernel<MODE, MB, NB, SLOTS, ANY_ROWS, GROUPED>, SMEM);
+  if (status != CW_OK) return status;
+  constexpr bool gated = MODE == 2 || MODE == 4;
+  const int out_cols = gated ? a.N / 2 : a.N, per_tile = gated ? 16 * NB : 32 * NB;
   a.tiles_n = (out_cols + per_tile - 1) / per_tile;
-  a.tiles_m = (a.M + W_BM - 1) / W_BM;
-  const int total = a.tiles_m * a.tiles_n * (MODE == 3 ? a.k_splits : 1);
+  a.tiles_m = GROUPED ? 0 : (a.M + 32 * MB - 1) / (32 * MB);  // GROUPED: read on the device
+  const int64_t total = (int64_t)(GROUPED ? row_tiles : a.tiles_m) * a.tiles_n * (MODE == 3 ? a.k_splits : 1);
+  if (total > 0x3fffffff) return CW_ERR_SIZE;
   // a multiple of 8 workgroups, so that every XCD gets the same number of them
-  int grid = total < workgroups ? total : workgroups;
+  int grid = total < workgroups ? (int)total : workgroups;
   grid = (grid + 7) & ~7;
-  hipLaunchKernelGGL((gemm_wide_bf16_kernel<MODE>), dim3(grid), dim3(256), W_SMEM, stream, a);
+  hipLaunchKernelGGL((gemm_wide_bf16_kernel<MODE, MB, NB, SLOTS, ANY_ROWS, GROUPED>), dim3(grid), dim3(256), SMEM, stream, a);
   return cw_launch_status();
+}
+
+// What a tile costs: ``fixed`` us of a work item and stage[q - 1] us a stage of 64 elements of K while q workgroups share a
+// compute unit (the smallest tiles; the others have one to themselves). Fits over 3600 timings with operands from memory, 72 to
+// 2048 rows of 26 shapes of the 0.5B to 14B models' layers and others (N 512 to 37888, K 512 to 18944), off by 9 % in the
+// mean; what the rule names by them takes 1.5 % more than the fastest tile and number of runs, 11 % at worst (192 rows of the
+// 1.5B shape's gate/up product 24.6 us, 21.5 by 160 x 160). A stage of the large tiles goes with BM + BN, 2.3 ns a row: its
+// loads; 256 x 192 and 256 x 288 have two stages of them in LDS and wait longer, and gain by their few rounds.
+struct TileRate {
+  int bm, bn, modes, per_unit;  // modes: a bit each of 0, 2 and 3 (1, 2, 4); 8: rows of any length
+  float fixed, stage[3];
+};
+static const TileRate TILE_RATES[] = {
+    {64, 64, 15, 3, -1.63f, {0.342f, 0.556f, 0.809f}}, {64, 128, 12, 2, -1.26f, {0.475f, 0.835f}}, {96, 96, 5, 1, 0.12f, {0.399f}},
+    {128, 96, 1, 1, 0.29f, {0.451f}},                  {128, 128, 12, 1, 0.34f, {0.592f}},        {160, 96, 2, 1, 0.53f, {0.507f}},
+    {160, 128, 7, 1, 0.79f, {0.594f}},                 {160, 160, 2, 1, 1.39f, {0.686f}},         {192, 160, 7, 1, 1.48f, {0.782f}},
+    {192, 192, 6, 1, 2.42f, {0.870f}},                 {256, 128, 4, 1, 1.62f, {0.803f}},         {256, 160, 1, 1, 3.59f, {0.898f}},
+    {256, 192, 11, 1, 1.37f, {1.295f}},                {256, 288, 2, 1, 2.63f, {1.704f}},
+};
+
+// Time of a product's work items in microseconds, without what every launch costs: whole rounds over the compute units, the
+// last one a little shorter for what it leaves idle, and the planes' way to memory and back.
+static float tile_time(const TileRate& t, int mode, int M, int N, int K, int planes, int cus) {
+  const int cols = mode == 2 ? N / 2 : N, per_tile = mode == 2 ? t.bn / 2 : t.bn;
+  const int64_t items = (int64_t)((M + t.bm - 1) / t.bm) * ((cols + per_tile - 1) / per_tile) * planes;
+  const int64_t rounds = items / ((int64_t)cus * t.per_unit), rest = items - rounds * cus * t.per_unit;
+  const float stages = (float)((K / 64 + planes - 1) / planes);
+  float time = (float)rounds * (t.fixed + stages * t.stage[t.per_unit - 1]);
+  if (rest > 0) {
+    const int share = (int)((rest + cus - 1) / cus);
+    time += (t.fixed + stages * t.stage[share - 1]) * (0.79f + 0.21f * ((float)rest / (float)cus - (float)(share - 1)));
+  }
+  return time + (mode == 3 ? 1.8e-6f * (float)planes * (float)M * (float)N : 0.0f);
+}
+
+// The tile and the number of runs of K that take the least time; ``wide_only``: of the wide-tile kernel's.
+static int tile_choice(int mode, int M, int N, int K, int most_planes, bool wide_only, bool whole, int cus) {
+  int best = 0;
+  float least = 0.0f;
+  for (const TileRate& t : TILE_RATES) {
+    if (!(t.modes & (mode == 0 ? 1 : mode == 2 ? 2 : 4)) || (wide_only && t.bm == 64) || !(whole || (t.modes & 8))) continue;
+    for (int planes = 1; planes <= most_planes && (planes == 1 || K / planes >= 256); ++planes) {
+      const float time = tile_time(t, mode, M, N, K, planes, cus);
+      if (best == 0 || time < least) {
+        least = time;
+        best = t.bm | t.bn << 10 | planes << 20;
+      }
+    }
+  }
+  return best;
+}
+
+// The product by the tile of bm x bn (128 x 128 and 256 x 192 for rows of any length, the others for whole ones: 16-byte
+// multiples), if there is such a tile for the mode.
+static int w_by_tile(int mode, int bm, int bn, bool whole, const WideArgs& a, int workgroups, hipStream_t stream) {
+  const int kind = mode == 2 && a.act != 0.0f ? 4 : mode;
+#define CW_WIDE(MODE_, MB_, NB_, SLOTS_, ANY_)                                     \
+  if (kind == MODE_ && bm == 32 * MB_ && bn == 32 * NB_ && (whole || ANY_)) return w_launch<MODE_, MB_, NB_, SLOTS_, ANY_>(a, 0, workgroups, stream)
+#define CW_WIDE_GATED(MB_, NB_, SLOTS_, ANY_) \
+  CW_WIDE(2, MB_, NB_, SLOTS_, ANY_);         \
+  CW_WIDE(4, MB_, NB_, SLOTS_, ANY_)
+  CW_WIDE(0, 3, 3, 6, false);
+  CW_WIDE(0, 4, 3, 5, false);
+  CW_WIDE(0, 4, 4, 5, true);
+  CW_WIDE(0, 5, 4, 4, false);
+  CW_WIDE(0, 6, 5, 3, false);
+  CW_WIDE(0, 8, 5, 3, false);
+  CW_WIDE(0, 8, 6, 2, true);
+  CW_WIDE_GATED(4, 4, 5, true);
+  CW_WIDE_GATED(5, 3, 5, false);
+  CW_WIDE_GATED(5, 4, 4, false);
+  CW_WIDE_GATED(5, 5, 4, false);
+  CW_WIDE_GATED(6, 5, 3, false);
+  CW_WIDE_GATED(6, 6, 3, false);
+  CW_WIDE_GATED(8, 6, 2, true);
+  CW_WIDE_GATED(8, 9, 2, false);
+  CW_WIDE(3, 3, 3, 6, false);
+  CW_WIDE(3, 4, 4, 5, true);
+  CW_WIDE(3, 5, 4, 4, false);
+  CW_WIDE(3, 6, 5, 3, false);
+  CW_WIDE(3, 6, 6, 3, false);
+  CW_WIDE(3, 8, 4, 3, false);
+  CW_WIDE(3, 8, 6, 2, true);
+#undef CW_WIDE_GATED
+#undef CW_WIDE
+  return CW_ERR_ARG;
+}
+
+// Rows of C that the tiles without ANY_ROWS take.
+static bool w_whole(int mode, const void* C, int64_t ldc, int out_cols) {
+  const int granule = mode == 3 ? 4 : 8;
+  return !(ldc & (granule - 1)) && !(out_cols & (granule - 1)) && !((uintptr_t)C & 15) && ldc < (1 << 20);
 }
 
 // The same product as cw_gemm_bf16_tiled through the wide-tile kernel, for the shapes that
@@ -676,8 +857,10 @@ CW_EXPORT int cw_gemm_bf16_wide(int mode, const void* X, int64_t ldx, const void
   if (cw_gemm_bf16_wide_tiles(mode, M, N, K, ldx) == 0) return CW_ERR_SIZE;
   WideArgs a{(const bf16_t*)X, ldx, (const bf16_t*)W, bias, bias_f32, C, ldc, M, N, K, 0, 0, 1};
   a.act = act;
-  return mode == 2 ? w_launch<2>(a, workgroups, stream)
-                   : mode == 5 ? w_launch<5>(a, workgroups, stream) : w_launch<0>(a, workgroups, stream);
+  if (mode == 5) return w_launch<5, 8, 6, 2>(a, 0, workgroups, stream);
+  const bool whole = w_whole(mode, C, ldc, mode == 2 ? N / 2 : N);
+  const int tile = tile_choice(mode, M, N, K, 1, true, whole, workgroups);
+  return w_by_tile(mode, tile & 1023, tile >> 10 & 1023, whole, a, workgroups, stream);
 }
 
 // parts[z] = x[:, run z of K] W[:, run z of K]^T for z < k_splits: float32 planes [k_splits, M, N]
@@ -690,27 +873,7 @@ CW_EXPORT int cw_gemm_bf16_wide_partial(const void* X, int64_t ldx, const void* 
   if (M == 0) return CW_OK;
   if (!cw_gemm_bf16_wide_partial_ok(M, N, K, ldx, k_splits)) return CW_ERR_SIZE;
   WideArgs a{(const bf16_t*)X, ldx, (const bf16_t*)W, nullptr, 0, parts, ldc, M, N, K, 0, 0, k_splits};
-  return w_launch<3>(a, workgroups, stream);
-}
-
-template <int MODE>
-static int w_launch_grouped(WideArgs a, int max_row_tiles, int workgroups, hipStream_t stream) {
-  static bool raised = false;
-  if (!raised) {
-    if (hipFuncSetAttribute((const void*)gemm_wide_bf16_kernel<MODE, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)W_SMEM) != hipSuccess)
-      return CW_ERR_LAUNCH;
-    raised = true;
-  }
-  const int out_cols = MODE == 2 ? a.N / 2 : a.N;
-  const int per_tile = MODE == 2 ? W_BN / 2 : W_BN;
-  a.tiles_n = (out_cols + per_tile - 1) / per_tile;
-  a.tiles_m = 0;  // read on the device
-  const int64_t most = (int64_t)max_row_tiles * a.tiles_n;
-  int grid = most < workgroups ? (int)most : workgroups;
-  grid = (grid + 7) & ~7;
-  hipLaunchKernelGGL((gemm_wide_bf16_kernel<MODE, true>), dim3(grid), dim3(256), W_SMEM, stream, a);
-  return cw_launch_status();
+  return w_launch<3, 8, 6, 2>(a, 0, workgroups, stream);
 }
 
 // Products of row tiles with matrices of their own through the wide-tile kernel: x holds
@@ -733,8 +896,9 @@ CW_EXPORT int cw_gemm_bf16_wide_grouped(int mode, const void* X, int64_t ldx, co
   if (cw_gemm_bf16_wide_tiles(mode, max_row_tiles * W_BM, N, K, ldx) == 0) return CW_ERR_SIZE;
   WideArgs a{(const bf16_t*)X, ldx, (const bf16_t*)W, nullptr, 0, C, ldc, 0, N, K, 0, 0, 1,
              tile_group, n_row_tiles, row_target, row_factor, w_group_stride, act};
-  return mode == 2 ? w_launch_grouped<2>(a, max_row_tiles, workgroups, stream)
-                   : w_launch_grouped<0>(a, max_row_tiles, workgroups, stream);
+  if (mode == 0) return w_launch<0, 8, 6, 2, true, true>(a, max_row_tiles, workgroups, stream);
+  return act == 0.0f ? w_launch<2, 8, 6, 2, true, true>(a, max_row_tiles, workgroups, stream)
+                     : w_launch<4, 8, 6, 2, true, true>(a, max_row_tiles, workgroups, stream);
 }
 
 // rows of a tile of cw_gemm_bf16_wide_grouped
@@ -910,15 +1074,14 @@ static int mid_launch(WideArgs a, hipStream_t stream) {
 
 // y = x W^T through the tiles between. mode 0: bfloat16 [M, N], + bias [N] when given; 2: W = [gate; up], the gated
 // product bfloat16 [M, N / 2] (``act`` as elsewhere); 3: float32 planes [k_splits, M, N] of partial sums over runs of K.
-// bm, bn: 64 or 128 each. K a multiple of 64 (of at least 64 elements a run), both matrices below 4 GiB.
+// bm, bn: 64 x 64, 64 x 128, 128 x 64, or a tile of the wide-tile kernel's (w_by_tile). K a multiple of 64 (of at least 64 elements a run), both matrices below 4 GiB.
 CW_EXPORT int cw_gemm_bf16_mid(int mode, const void* X, int64_t ldx, const void* W, const void* bias, int bias_f32, void* C,
-                               int64_t ldc, int M, int N, int K, float act, int k_splits, int bm, int bn, hipStream_t stream) {
-  if (M < 0 || N <= 0 || K <= 0 || (mode != 0 && mode != 2 && mode != 3) || !(act >= 0.0f || mode == 2)) return CW_ERR_ARG;
+                               int64_t ldc, int M, int N, int K, float act, int k_splits, int bm, int bn, int workgroups, hipStream_t stream) {
+  if (M < 0 || workgroups < 8 || N <= 0 || K <= 0 || (mode != 0 && mode != 2 && mode != 3) || !(act >= 0.0f || mode == 2)) return CW_ERR_ARG;
   if (((uintptr_t)X & 15) || ((uintptr_t)W & 15) || ((uintptr_t)C & (mode == 3 ? 15 : 7)) || !C) return CW_ERR_ARG;
   if ((mode == 2 && (N & 1)) || (mode != 0 && bias != nullptr)) return CW_ERR_ARG;
   if ((K & 63) || (ldx & 7) || ldx < K || ldc < (mode == 2 ? N / 2 : N)) return CW_ERR_ARG;
   if (mode == 3 ? (k_splits < 1 || k_splits > MID_MAX_PLANES || K / 64 < k_splits) : k_splits != 1) return CW_ERR_ARG;
-  if ((bm != 64 && bm != 128) || (bn != 64 && bn != 128)) return CW_ERR_ARG;
   if ((int64_t)N * K * 2 >= (1ll << 32) || ((int64_t)M * ldx + 128 * ldx) * 2 >= (1ll << 32)) return CW_ERR_SIZE;
   if (M == 0) return CW_OK;
   WideArgs a{(const bf16_t*)X, ldx, (const bf16_t*)W, bias, bias_f32, C, ldc, M, N, K, 0, 0, k_splits};
@@ -929,9 +1092,47 @@ CW_EXPORT int cw_gemm_bf16_mid(int mode, const void* X, int64_t ldx, const void*
   CW_MID(64, 64);
   CW_MID(64, 128);
   CW_MID(128, 64);
-  CW_MID(128, 128);
 #undef CW_MID
-  return CW_ERR_ARG;
+  return w_by_tile(mode, bm, bn, w_whole(mode, C, ldc, mode == 2 ? N / 2 : N), a, workgroups, stream);
+}
+
+// Which of this file's kernels a product of many rows should run on: 0 the library's, else bm | bn << 10 |
+// planes << 20 (cw_gemm_bf16_mid; mode as there), by the table of tiles above. For rows of 16-byte multiples; of others
+// cw_gemm_bf16_mid_choice is asked.
+// Where the lines lie, measured with operands from memory, 72 to 2048 rows (us, library -> here):
+//  * mode 3 (a sum that the next norm adds up; times with that norm): K of two and a half times N and more, everywhere (1.5B
+//    shape's down product, 72 rows 25.3 -> 15.3, 336 rows 40.3 -> 23.6, 1000 rows 55.8 -> 41.7, 2048 rows 83.3 -> 68.0; 7B
+//    shape, 512 rows 204 -> 78, 2048 rows 385 -> 265) until M N is 8 M (14B shape, 1500 rows 223 -> 201, 2048 rows 267 -> 304),
+//    2.1 M for outputs of more than 5120 columns (72B shape, 256 rows 293 -> 177, 640 rows 302 -> 370). A squarer matrix
+//    while M N is below 1.2 M, 1.03 M for more than 1536 columns (2048 x 2048, 500 rows 17.5 -> 16.9, 522 rows 18.8 ->
+//    20.2), and N at most 5120: beyond, mode 0 and a norm of its bfloat16 result are faster (1536 x 1536, 1000 rows 17.7,
+//    11.2 and 4.6).
+//  * mode 2: every shape measured up to the 7B one (72 rows of the 0.5B shape 15.1 -> 10.5, of the 1.5B shape 28.5 -> 20.1, of
+//    the 7B shape 74.6 -> 53.0; 640 rows 27.1 -> 16.3, 51.0 -> 44.0, 194 -> 177). The 14B shape's 141 M elements: 128 rows 72 ->
+//    66, 256 rows 100 -> 105, 384 rows 116 -> 125. A K of more than 1024 and half of N is a narrow output's (896 x 4864, 165 rows
+//    15.0 -> 20.6).
+//  * mode 0: a long K is summed faster by the library in parts (512 x 2048, 160 rows 8.4 -> 9.9), so K up to 512, up to 896
+//    for 896 columns and more (q/k/v of the 0.5B shape 7.9 -> 6.1 for 160 rows, 11.0 -> 9.4 for 2048; 512 columns 5.3 -> 6.1); up to 1536
+//    for 1536 columns and more from 0.5 M outputs on (q/k/v of the 1.5B shape, 160 rows 8.1 -> 8.4, 336 rows 9.4 -> 8.7, 2048 rows 18.3
+//    -> 17.8; its output product, 2048 rows 17.4 -> 14.3; 4640 columns, 100 rows 11.6 -> 11.7, 128 rows 16.8 -> 12.0, 2048 rows 38.5 -> 31.6); up to
+//    4096 for 2048 columns and more from 1.6 M on (4608 x 3584, 512 rows 34.4 -> 27.7, 1000 rows 47.0 -> 37.4; 3584 x 3584, 384 rows 23.1 -> 27.9).
+CW_EXPORT int cw_gemm_bf16_wide_choice(int mode, int M, int N, int K, int64_t ldx, int cus) {
+  if (M <= 64 || M > 2048 || N <= 0 || K < 256 || (K & 63) || (ldx & 7) || ldx < K || cus < 8) return 0;
+  if ((int64_t)N * K * 2 >= (1ll << 32) || ((int64_t)M * ldx + 128 * ldx) * 2 >= (1ll << 32)) return 0;
+  if (N & (mode == 2 ? 15 : mode == 3 ? 3 : 7)) return 0;
+  const int64_t elements = (int64_t)N * K, outputs = (int64_t)M * N;
+  if (mode == 0) {
+    const bool here = K <= 512 ? N >= 32 : K <= 896 ? N >= 896 : K <= 1536 ? N >= 1536 && outputs >= 500000 : K <= 4096 && N >= 2048 && outputs >= 1600000;
+    if (!here || N > 8192) return 0;
+  } else if (mode == 2) {
+    if ((N & 1) || (N < 2 * K && K > 1024) || elements > 136000000) return 0;
+  } else if (mode == 3) {
+    const int64_t most = 2 * (int64_t)K >= 5 * (int64_t)N ? (N <= 5120 ? 8000000 : 2100000) : N <= 1536 ? 1200000 : N <= 5120 ? 1030000 : 0;
+    if (outputs > most) return 0;
+  } else {
+    return 0;
+  }
+  return tile_choice(mode, M, N, K, mode == 3 ? MID_MAX_PLANES : 1, false, true, cus);
 }
 
 // Time of a product's work items in microseconds as the choice below weighs them, without what every launch costs:
@@ -949,8 +1150,8 @@ static float mid_time(int M, int N, int K, int bm, int bn, int planes, int cus) 
   return share * (float)(rounds * stages) * stage + (planes > 1 ? 2.2e-6f * (float)planes * (float)M * (float)N : 0.0f);
 }
 
-// Which of this file's kernels a product of many rows should run on: 0 the library's, else bm | bn << 10 |
-// planes << 20 (bm 256: cw_gemm_bf16_wide_partial, else cw_gemm_bf16_mid). mode as there.
+// Which tiles a product of many rows should run on whose rows of results are no multiples of 16 bytes: 0 the library's, else
+// bm | bn << 10 | planes << 20 (cw_gemm_bf16_mid). mode as there.
 // Where the lines lie, measured with operands from memory, 72 to 2048 rows, for the layers of the 0.5B to 72B shapes
 // and for outputs of 16 to 4096 columns with K of 256 to 16384 (us, library -> here):
 //  * mode 3 (a sum that the next norm adds up): K of three times N and more. The library's product of that kind leaves

@@ -122,7 +122,8 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_gemm_bf16_wide_partial_ok": [I, I, I, L, I],
             "cw_gemm_bf16_wide_partial": [P, L, P, P, L, I, I, I, I, I, P],
             "cw_gemm_bf16_mid_choice": [I, I, I, I, L, I],
-            "cw_gemm_bf16_mid": [I, P, L, P, P, I, P, L, I, I, I, F, I, I, I, P],
+            "cw_gemm_bf16_wide_choice": [I, I, I, I, L, I],
+            "cw_gemm_bf16_mid": [I, P, L, P, P, I, P, L, I, I, I, F, I, I, I, I, P],
             "cw_gemm_bf16_wide_grouped": [I, P, L, P, L, P, L, I, I, P, P, I, P, P, F, I, P],
         },
         "rowwise": {
@@ -528,8 +529,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias=None, out_dtype=None, par
     through this package's tiled kernels; float32 accumulation either way. With ``partial_ok``
     the result may come back as :class:`PartialSums` (a narrow output with a long K, few rows):
     only for a result that goes straight into ``add_rmsnorm``. ``portions_partial_ok``: the kernel that reads it adds
-    the planes, however many there are: with many rows as well, by the rule of ``cw_gemm_bf16_mid_choice``
-    (csrc/gemm_tile.hip), and in float32 (up to 64 planes)."""
+    the planes, however many there are: with many rows as well, by the rules of ``cw_gemm_bf16_wide_choice``
+    and ``cw_gemm_bf16_mid_choice`` (csrc/gemm_tile.hip), and in float32 (up to 64 planes)."""
     policy = policy if policy is not None else DEFAULT_POLICY
     _gpu(x, weight, bias)
     M, K = x.shape
@@ -580,15 +581,16 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias=None, out_dtype=None, par
             _check(lib.cw_gemm_bf16_skinny(1 if want_f32 else 0, _ptr(x), K, _ptr(weight), _ptr(out), N, M, N, K, 0, 0.0, _stream()),
                    "gemm_bf16_skinny")
             return out
+    plain = M > STREAM_MAX_ROWS and out_dtype is None and (bias is None or bias.dtype == torch.bfloat16 and tuple(bias.shape) == (N,))
+    if plain and portions_partial_ok and bias is None:
+        choice = _mid_choice(3, x, weight, policy)
+        if choice:
+            return linear_mid(x, weight, choice, partial=True)
     if partial_ok and out_dtype is None and bias is None and M >= WIDE_PRODUCT_MIN_ROWS and x.is_contiguous():
         splits = _wide_partial_chosen(x, weight, policy)
         if splits:
             return linear_wide_partial(x, weight, splits)
-    if M > STREAM_MAX_ROWS and out_dtype is None and (bias is None or bias.dtype == torch.bfloat16 and tuple(bias.shape) == (N,)):
-        if portions_partial_ok and bias is None and not (M >= WIDE_PRODUCT_MIN_ROWS and (N, K) in policy.wide_partial_choices):
-            choice = _mid_choice(3, x, weight, policy)
-            if choice:
-                return linear_mid(x, weight, choice, partial=True)
+    if plain:
         choice = _mid_choice(0, x, weight, policy, bias=bias)
         if choice:
             return linear_mid(x, weight, choice, bias=bias)
@@ -722,8 +724,8 @@ FUSED_QKV_MAX_WEIGHTS = 8 << 20
 def linear_tiled(x: torch.Tensor, weight: torch.Tensor, bias=None, swiglu: bool = False, wide=None, limit: float = 0.0) -> torch.Tensor:
     """y = x @ weight.T (+ bias), or with ``swiglu`` silu(x @ gate.T) * (x @ up.T) for weight =
     [gate; up], through the LDS-tiled matrix-core kernels for many bfloat16 rows (csrc/gemm_tile.hip):
-    the one with 256 x 192 tiles where it takes the shape and has tiles enough to fill the GPU, the
-    one with 128 x 128 tiles otherwise (``wide``: True or False to say which). The rows of x may
+    the one with wide tiles where it takes the shape and has tiles enough to fill the GPU, the
+    one with 128 x 128 tiles through registers otherwise (``wide``: True or False to say which). The rows of x may
     have a stride (a slice of a wider buffer). ``limit`` > 0 (with ``swiglu``): the clipped gated activation."""
     _gpu(weight, bias)
     if not (x.is_cuda and x.dim() == 2):
@@ -799,18 +801,6 @@ def wide_swiglu_pays(M: int, two_i: int, K: int, ldx: int) -> bool:
     rounds = -(-tiles // units)
     work = tiles / (units * rounds) * M / (rows * -(-M // rows))
     return two_i * K <= WIDE_SWIGLU_SMALL_WEIGHTS and work >= (WIDE_SWIGLU_WORK if rounds > 1 else WIDE_SWIGLU_WORK_ONE_ROUND)
-
-
-def wide_swiglu_is_finer(M: int, two_i: int, K: int, ldx: int) -> bool:
-    """Is the wide-tile kernel, whose gate reads float32 sums, all but as fast as the library and the gate kernel, where gates and
-    ups are rounded to bfloat16 between them (errors to 64 bits 1.7e-3 / 3.1e-3)? Two row tiles in one round of few weights,
-    the second more than a quarter full: there it is 1 to 3 % slower (us, library and gate against this, 1.5B shape, 188 tiles: 321 rows 34.8 /
-    35.8, 336 rows 35.2 / 35.9, 360 rows 36.0 / 36.1), from 363 rows on it pays. Steps of 257 to 320 tokens beside others are of
-    these rows, and had float32 gates when they were padded to 384."""
-    tiles = _load("gemm_tile").cw_gemm_bf16_wide_tiles(2, M, two_i, K, ldx)
-    units, rows = _compute_units(torch.device("cuda", torch.cuda.current_device())), WIDE_SWIGLU_TILE_ROWS
-    return (WIDE_SWIGLU_MIN_TILES <= tiles <= units and rows + rows // 4 < M <= 2 * rows
-            and two_i * K <= WIDE_SWIGLU_SMALL_WEIGHTS)
 
 
 @contextlib.contextmanager
@@ -978,13 +968,14 @@ def _aligned(*tensors) -> bool:
 
 
 def _mid_choice(mode: int, x: torch.Tensor, weight: torch.Tensor, policy: ProductPolicy, bias=None, limit: float = 0.0) -> int:
-    """What ``cw_gemm_bf16_mid_choice`` says of x @ weight.T; 0 for operands that its kernels do not take, and where a tuning
+    """What ``cw_gemm_bf16_wide_choice`` and, for rows of other lengths, ``cw_gemm_bf16_mid_choice`` say of x @ weight.T; 0 for operands that their kernels do not take, and where a tuning
     start-up has timed this very number of rows and found the library's tuned product the faster one."""
     if not _aligned(x, weight):
         return 0
     M, K = x.shape
     N = weight.shape[0]
-    choice = _load("gemm_tile").cw_gemm_bf16_mid_choice(mode, M, N, K, K, _compute_units(x.device))
+    lib, units = _load("gemm_tile"), _compute_units(x.device)
+    choice = lib.cw_gemm_bf16_wide_choice(mode, M, N, K, K, units) or lib.cw_gemm_bf16_mid_choice(mode, M, N, K, K, units)
     if choice and (policy.tuning or policy.mid_choices):
         key = (mode, M, *_swiglu_key(N, K, limit))
         if policy.tuning and key not in policy.mid_choices and policy.recall("mid_choices", key) is None:
@@ -1016,8 +1007,8 @@ def _measure_mid(mode: int, choice: int, x: torch.Tensor, weight: torch.Tensor, 
 
 def linear_mid(x: torch.Tensor, weight: torch.Tensor, choice: int, bias=None, swiglu: bool = False, partial: bool = False,
                limit: float = 0.0):
-    """x @ weight.T through the tiles for the steps between (csrc/gemm_tile.hip), of the sizes that ``choice`` names
-    (what ``cw_gemm_bf16_mid_choice`` returned): bfloat16 (+ bias), the gated product of [gate; up] with
+    """x @ weight.T through the tiles (csrc/gemm_tile.hip) of the sizes that ``choice`` names
+    (what ``cw_gemm_bf16_wide_choice`` or ``cw_gemm_bf16_mid_choice`` returned): bfloat16 (+ bias), the gated product of [gate; up] with
     ``swiglu``, or :class:`PartialSums` over runs of K with ``partial``."""
     _gpu(x, weight, bias)
     M, K = x.shape
@@ -1027,15 +1018,13 @@ def linear_mid(x: torch.Tensor, weight: torch.Tensor, choice: int, bias=None, sw
         raise KernelError("a tiled product is bfloat16, x [M, K] with weight [N, K]")
     if bias is not None and not (bias.numel() == N and bias.dtype in (torch.bfloat16, torch.float32) and not swiglu and not partial):
         raise KernelError("bias must be [N] bfloat16 or float32")
-    if partial and bm == 256:
-        return linear_wide_partial(x, weight, planes)
     if partial:
         out = torch.empty((planes, M, N), dtype=torch.float32, device=x.device)
     else:
         out = torch.empty((M, N // 2 if swiglu else N), dtype=torch.bfloat16, device=x.device)
     _check(_load("gemm_tile").cw_gemm_bf16_mid(3 if partial else 2 if swiglu else 0, _ptr(x), K, _ptr(weight), _ptr(bias),
                                                int(bias is not None and bias.dtype == torch.float32), _ptr(out), out.shape[-1],
-                                               M, N, K, float(limit), planes, bm, bn, _stream()), "gemm_bf16_mid")
+                                               M, N, K, float(limit), planes, bm, bn, _compute_units(x.device), _stream()), "gemm_bf16_mid")
     return PartialSums(out) if partial else out
 
 
@@ -1215,17 +1204,16 @@ def linear_swiglu(x, gate_up_weight: torch.Tensor, policy: "ProductPolicy | None
                                                   _stream()), "gemm_bf16_skinny(swiglu)")
         return out
     if x.dtype == torch.bfloat16 and gate_up_weight.dtype == torch.bfloat16 and K % 8 == 0 and x.is_contiguous():
-        choice = _mid_choice(2, x, gate_up_weight, policy, limit=limit)
-        if choice:
-            return linear_mid(x, gate_up_weight, choice, swiglu=True, limit=limit)
+        # fewer than 512 rows by the wide rule only inside a captured graph, where a shape's steps run from its second on
+        captured = torch.cuda.is_current_stream_capturing()
+        wide = _aligned(x, gate_up_weight) and wide_swiglu_pays(M, two_i, K, K) and (M >= WIDE_SWIGLU_MIN_ROWS // 2 or captured)
+        if not wide:
+            choice = _mid_choice(2, x, gate_up_weight, policy, limit=limit)
+            if choice:
+                return linear_mid(x, gate_up_weight, choice, swiglu=True, limit=limit)
         if policy.hip_products:
             return linear_tiled(x, gate_up_weight, swiglu=True, limit=limit)
-        # fewer than 512 rows only inside a captured graph, where a shape's steps run from its second on. Run eagerly they
-        # keep to the library's product, as the replay tests have it (450 tokens of the 1.5B shape, bound by the host's
-        # launches: 3.9 ms, 3.65 with one launch instead of two)
-        captured = torch.cuda.is_current_stream_capturing()
-        if _aligned(x, gate_up_weight) and ((wide_swiglu_pays(M, two_i, K, K) and (M >= WIDE_SWIGLU_MIN_ROWS // 2 or captured))
-                                            or (captured and wide_swiglu_is_finer(M, two_i, K, K))):
+        if wide:
             # with enough rows the shape of the weights decides, and a start-up that tunes the
             # library's products has measured it for this model's
             measured, key = M >= WIDE_SWIGLU_MIN_ROWS, _swiglu_key(two_i, K, limit)

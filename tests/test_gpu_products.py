@@ -206,6 +206,65 @@ def test_tiles_between_the_narrow_and_the_wide(M, N, K, bm, bn):
         torch.testing.assert_close(ops.linear_mid(x, w, one, swiglu=True, limit=limit).float(), ref, **bf16)
 
 
+# every tile of the wide-tile kernel that test_tiles_between_the_narrow_and_the_wide leaves out
+WIDE_TILES = {0: [(96, 96), (128, 96), (160, 128), (192, 160), (256, 160), (256, 192)],
+              2: [(160, 96), (160, 128), (160, 160), (192, 160), (192, 192), (256, 192), (256, 288)],
+              3: [(96, 96), (160, 128), (192, 160), (192, 192), (256, 128), (256, 192)]}
+
+
+# one row tile with few rows and fewer stages than slots; rows and columns that end inside a tile; several tiles a workgroup
+@pytest.mark.parametrize("mode,bm,bn", [(mode, *t) for mode, tiles in WIDE_TILES.items() for t in tiles])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 256), (65, 48, 64), (321, 1168, 640), (2048, 5168, 320)])
+def test_tiles_of_the_wide_kernel(mode, bm, bn, M, N, K):
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(M + N)
+    x = torch.randn(M, K, device=DEV, generator=gen).to(torch.bfloat16)
+    w = (torch.randn(N, K, device=DEV, generator=gen) / K ** 0.5).to(torch.bfloat16)
+    want = x.float() @ w.float().t()
+    # as above: float32 sums of K products of about 1 / sqrt(K), one rounding to bfloat16
+    f32, bf16 = dict(rtol=1e-4, atol=1e-4), dict(rtol=2.0 ** -8 + 1e-4, atol=1e-4)
+    one = bm | bn << 10 | 1 << 20
+    if mode == 0:
+        for bias in (None, torch.randn(N, device=DEV, generator=gen), torch.randn(N, device=DEV, generator=gen).to(torch.bfloat16)):
+            torch.testing.assert_close(ops.linear_mid(x, w, one, bias=bias).float(), want + (0 if bias is None else bias.float()), **bf16)
+    elif mode == 2:
+        g, u = want[:, : N // 2], want[:, N // 2:]
+        for limit, ref in {0.0: torch.nn.functional.silu(g) * u, ops.RELU_GATE: torch.relu(g) * u,
+                           ops.GELU_GATE: torch.nn.functional.gelu(g, approximate="tanh") * u}.items():
+            torch.testing.assert_close(ops.linear_mid(x, w, one, swiglu=True, limit=limit).float(), ref, **bf16)
+    else:
+        for planes in (p for p in (1, 3, 5) if p <= K // 64):
+            got = ops.linear_mid(x, w, bm | bn << 10 | planes << 20, partial=True)
+            torch.testing.assert_close(got.sum(), want, **f32)
+            first = (K // 64 // planes) * 64
+            torch.testing.assert_close(got.parts[0], x[:, :first].float() @ w[:, :first].float().t(), **f32)
+
+
+@pytest.mark.parametrize("mode,N", [(0, 1001), (2, 2 * 1004), (3, 1002)])
+def test_tiles_for_whole_rows_refuse_others(mode, N):
+    """Results whose rows are no multiples of 16 bytes: refused where a tile takes whole rows only, and served by another."""
+    from clockwork_amd import ops
+
+    M, K = 200, 512
+    gen = torch.Generator(device=DEV).manual_seed(N)
+    x = torch.randn(M, K, device=DEV, generator=gen).to(torch.bfloat16)
+    w = (torch.randn(N, K, device=DEV, generator=gen) / K ** 0.5).to(torch.bfloat16)
+    for bm, bn in WIDE_TILES[mode]:
+        if (bm, bn) != (256, 192):
+            with pytest.raises(ops.KernelError):
+                ops.linear_mid(x, w, bm | bn << 10 | 1 << 20, swiglu=mode == 2, partial=mode == 3)
+    want = x.float() @ w.float().t()
+    bf16 = dict(rtol=2.0 ** -8 + 1e-4, atol=1e-4)
+    if mode == 2:
+        ref = torch.nn.functional.silu(want[:, : N // 2]) * want[:, N // 2:]
+        torch.testing.assert_close(ops.linear_mid(x, w, 256 | 192 << 10 | 1 << 20, swiglu=True).float(), ref, **bf16)
+        torch.testing.assert_close(ops.linear_swiglu(x, w).float(), ref, rtol=4 * 2.0 ** -8, atol=2e-2)
+    else:
+        got = ops.linear(x, w, partial_ok=mode == 3, portions_partial_ok=mode == 3)
+        torch.testing.assert_close(got.sum() if mode == 3 else got.float(), want, **bf16)
+
+
 def test_products_of_a_portion_by_their_rule():
     """What the rule names runs and is the product, on every side of its lines."""
     from clockwork_amd import ops

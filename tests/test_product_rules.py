@@ -39,6 +39,40 @@ def test_products_on_the_tiles_between(mode, M, N, K, wide):
     assert (bm == 256) == wide and (planes == 1 or mode == 3)
 
 
+def _wide_choice(mode, M, N, K, ldx=None):
+    code = ops._load("gemm_tile").cw_gemm_bf16_wide_choice(mode, M, N, K, ldx or K, CUS)
+    return (code & 1023, code >> 10 & 1023, code >> 20) if code else None
+
+
+@pytest.mark.parametrize("mode,M,N,K,there", [
+    # few columns of a long K, few outputs; both sides of each line
+    (0, 144, 512, 896, False), (0, 144, 896, 896, True), (0, 300, 2048, 1536, True), (0, 200, 2048, 1536, False), (0, 1000, 1152, 1536, False),
+    (0, 500, 3584, 3584, True), (0, 400, 3584, 3584, False), (0, 1000, 512, 2048, False), (0, 1000, 4096, 4160, False), (0, 700, 8200, 512, False),
+    # gated: up to 136 M elements, no narrow output of a long K
+    (2, 72, 37888, 3584, True), (2, 512, 27648, 5120, False), (2, 165, 896, 4864, False), (2, 2048, 2048, 1024, True),
+    # sums for a norm
+    (3, 2048, 1536, 8960, True), (3, 1500, 5120, 13824, True), (3, 1600, 5120, 27648, False), (3, 250, 8192, 29568, True), (3, 640, 8192, 29568, False),
+    (3, 780, 1536, 1536, True), (3, 790, 1536, 1536, False), (3, 500, 2048, 2048, True), (3, 520, 2048, 2048, False), (3, 152, 7376, 2304, False),
+    # rows that are no multiples of 16 bytes, rows of x that are none, too few rows and too many
+    (0, 256, 1028, 512, False), (2, 256, 8200, 512, False), (3, 256, 514, 2048, False), (0, 64, 1152, 896, False), (0, 2049, 1152, 896, False)])
+def test_products_on_the_wide_kernels_tiles(mode, M, N, K, there):
+    choice = _wide_choice(mode, M, N, K)
+    assert (choice is not None) == there
+    if there:
+        bm, bn, planes = choice
+        assert planes == 1 or (mode == 3 and K // planes >= 256)
+        assert _wide_choice(mode, M, N, K, K + 4) is None   # rows of x at no 16 bytes
+
+
+def test_tiles_follow_the_rounds_that_they_need():
+    """Gate/up of the 1.5B shape: the tile whose rounds over the compute units are fullest for what they cost."""
+    tiles = {M: _wide_choice(2, M, 17920, 1536)[:2] for M in (100, 160, 336, 512, 1000, 2048)}
+    assert tiles[1000] == tiles[2048] == (256, 288)      # 252 and 504 tiles
+    assert tiles[336] == (192, 160)                      # 224
+    assert tiles[100] == tiles[160] == (160, 96)         # 187, the fewest columns that one round of a row tile takes
+    assert all(_wide_choice(3, M, 1536, 8960)[2] <= _wide_choice(3, 160, 1536, 8960)[2] for M in (336, 1000, 2048))
+
+
 def test_no_choice_outside_what_the_kernels_take():
     for mode in (0, 2, 3):
         for M, N, K in ((64, 1152, 896), (2049, 1152, 896), (144, 1152, 900), (144, 1152, 192), (144, 0, 896)):
