@@ -172,11 +172,11 @@ __device__ __forceinline__ uint32_t philox_first_word(uint64_t seed, uint64_t co
 //
 //   MAX      per chunk: the largest logit and its first index; and 64 logits of the row, one every V / 64;
 //   HIST     per chunk, over 512 bins of logit / T: how many tokens fall into each (rows with top-k) and what they
-//            weigh, the weights being exp(logit / T - mx) (rows with top-p); and what the chunk weighs. Greedy rows
-//            end here;
-//   PICK     per row: the bin that holds the k-th largest token, or the bin in which the weight from the top exceeds
-//            top_p * total;
-//   COLLECT  per chunk: what the tokens above that bin weigh (all of them stay), and a list of the tokens in it;
+//            weigh, the weights being exp(logit / T - mx) (rows with top-p), added to the row's bins; and what the chunk
+//            weighs. Greedy rows end here;
+//   COLLECT  per chunk: the bin that holds the k-th largest token, or the bin in which the weight from the top exceeds
+//            top_p * total, from the row's bins, by every workgroup for itself; what the tokens above that bin weigh (all of
+//            them stay), and a list of the tokens in it;
 //   DRAW     per row: the k-th largest token of the list (radix selection over the order-preserving keys, 8 bits a
 //            step; dividing by the temperature keeps the order, so the floor of what is kept is
 //            (k-th largest) / temperature: ties at the k-th value survive, also ties that the division makes) and
@@ -202,9 +202,13 @@ __device__ __forceinline__ uint32_t philox_first_word(uint64_t seed, uint64_t co
 // Weights are integers, exp(.) * 2^40 rounded down: their sums do not depend on the order of
 // addition, so every comparison above gives the same answer however the row is cut and however
 // the additions are scheduled (LDS atomics included), run after run.
-// Bound by the passes over the logits, which come from the memory-side cache after the first. 64 rows of 151,936
-// logits, a quarter each greedy, temperature, top-k and top-p: 119 us as twelve kernels (a radix step of 8 bits of the
-// key each, over the whole rows), 64 us as five (61 with bins of one width).
+// Bound by the passes over the logits, which come from the memory-side cache after the first, by the division and the
+// exponential of every token (a third of HIST) and, in DRAW, by a chain of trips and barriers. 64 rows of 151,936
+// logits, a quarter each greedy, temperature, top-k and top-p, us: 119 as twelve kernels (a radix step of 8 bits of the
+// key each, over the whole rows), 63 as five, the row's bin by a kernel of its own from every chunk's bins (MAX 8.6, HIST 20.4, PICK 6.0,
+// COLLECT 10.4, DRAW 14.2 in a trace), 50 as four with the chunks' bins added up by atomics (9.3, 16.0, 9.0, 12.2).
+// Tried: a token's first loads asked for before its row is known (no gain), the division by a reciprocal and two exact steps
+// (HIST 1.5 us less, finding out where that is exact as much more in MAX).
 #define SAMPLE_THREADS 256
 #define SAMPLE_WAVES (SAMPLE_THREADS / 64)
 #define SAMPLE_MAX_CHUNKS 64
@@ -219,9 +223,9 @@ typedef unsigned long long u64_t;
 
 struct SampleRow {     // what is known about a row between two kernels
   u64_t limit;         // top_p * total (rows with top-p)
-  uint32_t bin;        // the bin to collect
+  uint32_t bin;        // the bin that COLLECT's second run collects
   uint32_t rank;       // rows with top-k: which of the bin's tokens, from the largest, is the k-th
-  uint32_t collect;    // 1: COLLECT has to run, 2: its second run has to
+  uint32_t collect;    // 2: COLLECT's second run has to run
   uint32_t listed[2];  // tokens that COLLECT's two runs found in the bin
   uint32_t unused;     // (a whole number of 8 bytes)
   float2 segments[3];  // see SampleBins
@@ -239,11 +243,11 @@ struct SampleArgs {
   const int64_t* draws;
   int* out;
   // workspace
-  u64_t* hist_w;      // [n][chunks][SAMPLE_BINS]
+  u64_t* hist_w;      // [n][SAMPLE_BINS], zeroed by MAX as hist_n
   u64_t* sums;        // [n][chunks] weight of the chunk (of its bins above the collected one, after COLLECT)
   SampleRow* rows;    // [n], zeroed by MAX
   uint4* found;       // [n][chunks] smallest and largest key that COLLECT found in the bin, (~0, 0) for none, and how many
-  uint32_t* hist_n;   // [n][chunks][SAMPLE_BINS]
+  uint32_t* hist_n;   // [n][SAMPLE_BINS]
   uint2* list;        // [n][SAMPLE_LIST] (key, index)
   float* pmax;        // [n][chunks]
   int* pmax_i;        // [n][chunks]
@@ -251,7 +255,7 @@ struct SampleArgs {
 };
 
 // Chunks a row is cut into: at least 2048 tokens each; 64 for few rows, for many rows as few as still make two
-// thousand workgroups (what PICK adds up grows with them).
+// thousand workgroups (a row's bins take an addition from each).
 static int sample_chunks(int n, int V) {
   int c = (V + 2047) / 2048;
   const int most = n <= 32 ? SAMPLE_MAX_CHUNKS : n >= 512 ? 4 : 2048 / n;
@@ -261,7 +265,7 @@ static int sample_chunks(int n, int V) {
 
 CW_EXPORT int64_t cw_sample_workspace_bytes(int n, int V) {
   const int64_t rc = (int64_t)n * sample_chunks(n, V);
-  return rc * SAMPLE_BINS * 12 + rc * 32 + (int64_t)n * ((int64_t)sizeof(SampleRow) + SAMPLE_LIST * 8 + SAMPLE_POINTS * 4) + 64;
+  return rc * 32 + (int64_t)n * ((int64_t)sizeof(SampleRow) + SAMPLE_BINS * 12 + SAMPLE_LIST * 8 + SAMPLE_POINTS * 4) + 64;
 }
 
 __device__ __forceinline__ float key_to_float(uint32_t k) {
@@ -328,6 +332,16 @@ __device__ __forceinline__ void sample_segments(float point, float temp, float2*
 }
 __device__ __forceinline__ u64_t topp_limit(float p, u64_t total) { return (u64_t)((double)p * (double)total); }
 
+// The row and the chunk of a workgroup of a pass: rows next to each other go to different XCDs and compute units, and a unit's
+// workgroups are of rows that lie an odd number apart, so that rows that need more work (their options may repeat every few
+// rows) are dealt evenly. (A quarter each greedy, temperature, top-k and top-p, in turn: with row = blockIdx.y a unit had rows of
+// one kind, and HIST took 20.7 us, as long as for 64 rows of top-p.)
+__device__ __forceinline__ void row_and_chunk(const SampleArgs& a, int& row, int& chunk) {
+  const int id = blockIdx.y * gridDim.x + blockIdx.x;
+  chunk = id / a.n;
+  row = (id - chunk * a.n + chunk + chunk / 4) % a.n;
+}
+
 // Four neighbouring logits from token i on (i a multiple of 4); NaN from ``hi`` on.
 __device__ __forceinline__ void sample_load4(const float* x, int i, int hi, int vec, float (&o)[4]) {
   if (vec && i + 4 <= hi) {
@@ -341,17 +355,25 @@ __device__ __forceinline__ void sample_load4(const float* x, int i, int hi, int 
 // f(index, logit) for the tokens of [lo, hi) (lo a multiple of 4), by THREADS neighbouring threads (all of the workgroup, or
 // a wave), 4 U loads in flight a thread. Up to three tokens past hi come as NaN, which everything here takes for -inf: a
 // test for each token by itself would cost as much as what most tokens need.
+template <int U, int THREADS = SAMPLE_THREADS>
+__device__ __forceinline__ void sample_batch(const float* x, int i0, int hi, int vec, float (&t)[U][4]) {
+#pragma unroll
+  for (int u = 0; u < U; ++u) sample_load4(x, min(i0 + u * 4 * THREADS, (int)((unsigned)(hi - 1) & ~3u)), hi, vec, t[u]);
+}
+template <int U, int THREADS = SAMPLE_THREADS, typename F>
+__device__ __forceinline__ void sample_take(const float (&t)[U][4], int i0, int hi, F f) {
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (i0 + u * 4 * THREADS < hi)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f(i0 + u * 4 * THREADS + e, t[u][e]);
+}
 template <int U = 2, int THREADS = SAMPLE_THREADS, typename F>
 __device__ __forceinline__ void sample_walk(const float* x, int lo, int hi, int vec, F f) {
   for (int i0 = lo + (int)(threadIdx.x & (THREADS - 1)) * 4; i0 < hi; i0 += U * 4 * THREADS) {
-    float a[U][4];
-#pragma unroll
-    for (int u = 0; u < U; ++u) sample_load4(x, min(i0 + u * 4 * THREADS, (int)((unsigned)(hi - 1) & ~3u)), hi, vec, a[u]);
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (i0 + u * 4 * THREADS < hi)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) f(i0 + u * 4 * THREADS + e, a[u][e]);
+    float t[U][4];
+    sample_batch<U, THREADS>(x, i0, hi, vec, t);
+    sample_take<U, THREADS>(t, i0, hi, f);
   }
 }
 
@@ -415,8 +437,13 @@ __device__ __forceinline__ void row_max(const SampleArgs& a, int row, float& bv,
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_max_kernel(SampleArgs a) {
   __shared__ float sv[SAMPLE_WAVES];
   __shared__ int si[SAMPLE_WAVES];
-  const int row = blockIdx.y, chunk = blockIdx.x;
+  int row, chunk;
+  row_and_chunk(a, row, chunk);
   if (chunk == 0 && threadIdx.x < sizeof(SampleRow) / 4) reinterpret_cast<uint32_t*>(a.rows + row)[threadIdx.x] = 0u;
+  for (int b = chunk * SAMPLE_THREADS + (int)threadIdx.x; b < SAMPLE_BINS; b += a.chunks * SAMPLE_THREADS) {
+    a.hist_w[(int64_t)row * SAMPLE_BINS + b] = 0;
+    a.hist_n[(int64_t)row * SAMPLE_BINS + b] = 0u;
+  }
   const int lo = chunk * a.per, hi = min(a.V, lo + a.per);
   const float* x = a.logits + (int64_t)row * a.row_stride;
   if (threadIdx.x < SAMPLE_POINTS) {
@@ -477,19 +504,22 @@ __device__ __forceinline__ void sample_locate(const SampleArgs& a, int row, floa
     return;
   }
   const float* x = a.logits + (int64_t)row * a.row_stride;
-  auto weight = [&](int i) __attribute__((always_inline)) -> u64_t {
-    const float v = x[i] / temp;
+  auto weight = [&](float raw) __attribute__((always_inline)) -> u64_t {
+    const float v = raw / temp;
     return v == v && order_key(v) >= floor_key ? weight_of(v, mx) : 0;
   };
   // in the chunk: thread t weighs a run of consecutive tokens; then a lane of the first wave takes a token of
   // the run that the target falls into
   const int lo = sel_chunk * a.per, hi = min(a.V, lo + a.per);
   const u64_t target = sel_base;
-  const int run = (hi - lo + SAMPLE_THREADS - 1) / SAMPLE_THREADS;
+  const int run = ((hi - lo + SAMPLE_THREADS - 1) / SAMPLE_THREADS + 3) / 4 * 4;
   const int my_lo = min(hi, lo + (int)threadIdx.x * run), my_hi = min(hi, my_lo + run);
   u64_t w = 0;
-#pragma unroll 8
-  for (int i = my_lo; i < my_hi; ++i) w += weight(i);
+  for (int i = my_lo; i < my_hi; i += 20) {  // (all of a thread's loads of 64 rows' chunks in flight at once)
+    float t[5][4];
+    sample_batch<5, 1>(x, i, my_hi, a.vec, t);
+    sample_take<5, 1>(t, i, my_hi, [&](int, float raw) __attribute__((always_inline)) { w += weight(raw); });
+  }
   const u64_t incl = block_running_sum(w);
   if (w > 0 && incl - w <= target && target < incl) {
     sel_run = threadIdx.x;
@@ -501,7 +531,7 @@ __device__ __forceinline__ void sample_locate(const SampleArgs& a, int row, floa
     const int run_lo = min(hi, lo + sel_run * run), run_hi = min(hi, run_lo + run);
     for (int i0 = run_lo; i0 < run_hi; i0 += 64) {
       const int i = i0 + (int)threadIdx.x;
-      const u64_t q = i < run_hi ? weight(i) : 0;
+      const u64_t q = i < run_hi ? weight(x[i]) : 0;
       u64_t upto = q;
 #pragma unroll
       for (int off = 1; off < 64; off <<= 1) {
@@ -522,8 +552,11 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_hist_kernel(SampleArgs 
   __shared__ u64_t bins_w[SAMPLE_BINS];
   __shared__ uint32_t bins_n[SAMPLE_BINS];
   __shared__ float2 segments[3];
-  const int row = blockIdx.y, chunk = blockIdx.x;
+  int row, chunk;
+  row_and_chunk(a, row, chunk);
   const float temp = a.temperature[row];
+  const int lo = chunk * a.per, hi = min(a.V, lo + a.per);
+  const float* x = a.logits + (int64_t)row * a.row_stride;
   const bool with_k = row_has_top_k(a, row), with_p = row_has_top_p(a, row);
   // the second wave works the segments out while the first looks for the maximum
   const float point = a.points[(int64_t)row * SAMPLE_POINTS + (threadIdx.x & 63)];
@@ -553,9 +586,8 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_hist_kernel(SampleArgs 
       known.segments[2] = bins.s2;
     }
   }
-  const int lo = chunk * a.per, hi = min(a.V, lo + a.per);
   u64_t sum = 0;
-  sample_walk(a.logits + (int64_t)row * a.row_stride, lo, hi, a.vec, [&](int, float raw) __attribute__((always_inline)) {
+  sample_walk(x, lo, hi, a.vec, [&](int, float raw) __attribute__((always_inline)) {
     const float v = raw / temp;
     const uint32_t bin = with_k || with_p ? bin_of(bins, v) : 0u;
     if (with_k) atomicAdd(&bins_n[bin], 1u);
@@ -565,78 +597,77 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_hist_kernel(SampleArgs 
     if (with_p && w) atomicAdd(&bins_w[bin], w);
   });
   sum = block_sum(sum);  // (and a barrier behind the bins)
-  const int64_t rc = (int64_t)row * a.chunks + chunk;
-  if (threadIdx.x == 0) a.sums[rc] = sum;
+  if (threadIdx.x == 0) a.sums[(int64_t)row * a.chunks + chunk] = sum;
+  // the row's bins: integers, so the order in which its chunks come does not matter
   for (int b = threadIdx.x; b < SAMPLE_BINS; b += SAMPLE_THREADS) {
-    if (with_k) a.hist_n[rc * SAMPLE_BINS + b] = bins_n[b];
-    if (with_p) a.hist_w[rc * SAMPLE_BINS + b] = bins_w[b];
+    if (with_k && bins_n[b]) atomicAdd(a.hist_n + (int64_t)row * SAMPLE_BINS + b, bins_n[b]);
+    if (with_p && bins_w[b]) atomicAdd(a.hist_w + (int64_t)row * SAMPLE_BINS + b, bins_w[b]);
   }
 }
 
 // The weights of bins 2 t and 2 t + 1 of the whole row, for thread t.
 __device__ __forceinline__ void row_bins(const SampleArgs& a, int row, u64_t& w0, u64_t& w1) {
-#pragma unroll 8
-  for (int c = 0; c < a.chunks; ++c) {
-    const ulonglong2 h = *reinterpret_cast<const ulonglong2*>(a.hist_w + ((int64_t)row * a.chunks + c) * SAMPLE_BINS + 2 * threadIdx.x);
-    w0 += h.x;
-    w1 += h.y;
-  }
+  const ulonglong2 h = *reinterpret_cast<const ulonglong2*>(a.hist_w + (int64_t)row * SAMPLE_BINS + 2 * threadIdx.x);
+  w0 = h.x;
+  w1 = h.y;
 }
 
-// PICK
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(SampleArgs a) {
+// The bin to collect and, with top-k, which of its tokens is the k-th, with top-p what the tokens more likely than the nucleus's
+// last weigh at most: by every workgroup of a row for itself.
+__device__ __forceinline__ void sample_pick(const SampleArgs& a, int row, bool with_k, uint32_t& bin, uint32_t& rank, u64_t& limit) {
   __shared__ uint32_t picked_bin, picked_rank;
-  const int row = blockIdx.x;
-  if (!(a.temperature[row] > 0.0f)) return;
-  const bool with_k = row_has_top_k(a, row), with_p = row_has_top_p(a, row);
-  if (!with_k && !with_p) return;
-  SampleRow& known = a.rows[row];
+  __shared__ u64_t all;
   // thread t: bins 2 t and 2 t + 1 of the whole row
   if (threadIdx.x == 0) picked_bin = 0u, picked_rank = 1u;
-  __syncthreads();
+  limit = 0;
   if (with_k) {
-    uint32_t n0 = 0u, n1 = 0u;
-#pragma unroll 8
-    for (int c = 0; c < a.chunks; ++c) {
-      const uint2 h = *reinterpret_cast<const uint2*>(a.hist_n + ((int64_t)row * a.chunks + c) * SAMPLE_BINS + 2 * threadIdx.x);
-      n0 += h.x;
-      n1 += h.y;
-    }
-    const uint32_t upto = block_running_sum(n0 + n1), k = (uint32_t)a.top_k[row];
-    const uint32_t before = upto - n0 - n1;
+    const uint2 h = *reinterpret_cast<const uint2*>(a.hist_n + (int64_t)row * SAMPLE_BINS + 2 * threadIdx.x);
+    const uint32_t upto = block_running_sum(h.x + h.y), k = (uint32_t)a.top_k[row];
+    const uint32_t before = upto - h.x - h.y;
     if (before < k && k <= upto) {
-      picked_bin = 2 * threadIdx.x + (before + n0 < k ? 1 : 0);
-      picked_rank = k - (before + n0 < k ? before + n0 : before);
+      picked_bin = 2 * threadIdx.x + (before + h.x < k ? 1 : 0);
+      picked_rank = k - (before + h.x < k ? before + h.x : before);
     }
   } else {
-    const u64_t total = block_sum((int)threadIdx.x < a.chunks ? a.sums[(int64_t)row * a.chunks + threadIdx.x] : 0);
-    const u64_t limit = topp_limit(a.top_p[row], total);
-    u64_t w0 = 0, w1 = 0;
+    u64_t w0, w1;
     row_bins(a, row, w0, w1);
     const u64_t upto = block_running_sum(w0 + w1);
+    if (threadIdx.x == SAMPLE_THREADS - 1) all = upto;
+    __syncthreads();
+    limit = topp_limit(a.top_p[row], all);
     const u64_t before = upto - w0 - w1;
     if (before <= limit && limit < upto) picked_bin = 2 * threadIdx.x + (before + w0 <= limit ? 1 : 0);
-    if (threadIdx.x == 0) known.limit = limit;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    known.bin = picked_bin;
-    known.rank = picked_rank;
-    known.collect = 1u;
-  }
+  bin = picked_bin;
+  rank = picked_rank;
 }
 
 // COLLECT; ``again``: its second run
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(SampleArgs a, int again) {
   __shared__ uint2 mine[SAMPLE_BLOCK_LIST];
   __shared__ uint32_t n_mine, at_list, ends[2];
-  const int row = blockIdx.y, chunk = blockIdx.x;
+  int row, chunk;
+  row_and_chunk(a, row, chunk);
   SampleRow& known = a.rows[row];
   const float temp = a.temperature[row];
-  if (!(temp > 0.0f) || known.collect != 1u + again) return;
-  const uint32_t bin = known.bin;
+  if (!(temp > 0.0f)) return;
+  uint32_t bin = 0u;
+  const bool with_k = row_has_top_k(a, row);
+  if (again ? known.collect != 2u : !with_k && !row_has_top_p(a, row)) return;
   const int lo = chunk * a.per, hi = min(a.V, lo + a.per);
   const float* x = a.logits + (int64_t)row * a.row_stride;
+  if (again) {
+    bin = known.bin;
+  } else {
+    uint32_t rank;
+    u64_t limit;
+    sample_pick(a, row, with_k, bin, rank, limit);
+    if (chunk == 0 && threadIdx.x == 0) {
+      known.rank = rank;
+      known.limit = limit;
+    }
+  }
   if (threadIdx.x == 0) n_mine = ends[1] = 0u, ends[0] = 0xffffffffu;
   const SampleBins bins = sample_bins(known.segments);
   float mraw;
@@ -653,7 +684,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(SampleAr
   float end = segment == 0 ? s1.x : segment == 1 ? s2.x : -INFINITY;
   if (j < SAMPLE_SEGMENT_BINS - 1 && seg_y > 0.0f) end = fmaxf(end, seg_top - (float)(j + 1) / seg_y);
   const float surely_below = (end - 1e-5f * (fabsf(end) + fabsf(seg_top)) - 1e-30f) * temp;
-  sample_walk(x, lo, hi, a.vec, [&](int i, float raw) __attribute__((always_inline)) {
+  auto look = [&](int i, float raw) __attribute__((always_inline)) {
     if (raw < surely_below) return;
     const float v = raw / temp;
     const uint32_t b = bin_of(bins, v);
@@ -665,7 +696,8 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(SampleAr
       least = min(least, key);
       if (at < SAMPLE_BLOCK_LIST) mine[at] = make_uint2(key, (uint32_t)i);
     }
-  });
+  };
+  sample_walk(x, lo, hi, a.vec, look);
   if (__ballot(most >= least)) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -704,6 +736,8 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(SampleArgs 
   const float temp = a.temperature[row];
   if (!(temp > 0.0f) || (again && known.collect != 2u)) return;
   const bool with_k = row_has_top_k(a, row), with_p = row_has_top_p(a, row);
+  // (a token of the list a thread before the list's length is known: what lies past it is not looked at)
+  const uint2 first_listed = a.list[(int64_t)row * SAMPLE_LIST + threadIdx.x];
   float mraw;
   int mi;
   row_max(a, row, mraw, mi);
@@ -718,7 +752,8 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(SampleArgs 
   const float* x = a.logits + (int64_t)row * a.row_stride;
   const bool fits = listed <= SAMPLE_LIST;
   if (fits)
-    for (uint32_t i = threadIdx.x; i < listed; i += SAMPLE_THREADS) list[i] = a.list[(int64_t)row * SAMPLE_LIST + i];
+    for (uint32_t i = threadIdx.x; i < listed; i += SAMPLE_THREADS)
+      list[i] = i < SAMPLE_THREADS ? first_listed : a.list[(int64_t)row * SAMPLE_LIST + i];
   if (threadIdx.x < 64) {  // a chunk a lane (there are at most 64)
     uint4 e = make_uint4(0xffffffffu, 0u, 0u, 0u);
     if ((int)threadIdx.x < a.chunks) e = a.found[(int64_t)row * a.chunks + threadIdx.x];
@@ -802,7 +837,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(SampleArgs 
       }
       if (above > limit) {
         // the nucleus ends in a bin above this one, all of whose tokens are among the k
-        u64_t w0 = 0, w1 = 0;
+        u64_t w0, w1;
         row_bins(a, row, w0, w1);
         const u64_t upto = block_running_sum(w0 + w1);
         const u64_t before = upto - w0 - w1;
@@ -894,9 +929,9 @@ CW_EXPORT int cw_sample(const float* logits, int64_t row_stride, int n, int V,
   const int64_t rc = (int64_t)n * a.chunks;
   // 16-byte items first
   u64_t* p8 = (u64_t*)workspace;
-  a.hist_w = p8; p8 += rc * SAMPLE_BINS;
+  a.hist_w = p8; p8 += (int64_t)n * SAMPLE_BINS;
   a.list = (uint2*)p8; p8 += (int64_t)n * SAMPLE_LIST;
-  a.hist_n = (uint32_t*)p8; p8 += rc * SAMPLE_BINS / 2;
+  a.hist_n = (uint32_t*)p8; p8 += (int64_t)n * SAMPLE_BINS / 2;
   a.found = (uint4*)p8; p8 += 2 * rc;
   a.sums = p8; p8 += rc;
   a.rows = (SampleRow*)p8; p8 += (int64_t)n * sizeof(SampleRow) / 8;
@@ -907,10 +942,7 @@ CW_EXPORT int cw_sample(const float* logits, int64_t row_stride, int n, int V,
   const dim3 grid(a.chunks, n), block(SAMPLE_THREADS);
   hipLaunchKernelGGL(sample_max_kernel, grid, block, 0, stream, a);
   hipLaunchKernelGGL(sample_hist_kernel, grid, block, 0, stream, a);
-  if (flags & 3) {
-    hipLaunchKernelGGL(sample_pick_kernel, dim3(n), block, 0, stream, a);
-    hipLaunchKernelGGL(sample_collect_kernel, grid, block, 0, stream, a, 0);
-  }
+  if (flags & 3) hipLaunchKernelGGL(sample_collect_kernel, grid, block, 0, stream, a, 0);
   hipLaunchKernelGGL(sample_draw_kernel, dim3(n), block, 0, stream, a, 0);
   if ((flags & 7) == 3) {
     hipLaunchKernelGGL(sample_collect_kernel, grid, block, 0, stream, a, 1);
