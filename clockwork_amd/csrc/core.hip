@@ -517,6 +517,29 @@ CW_EXPORT int cw_rope_kv_write(void* qkv, int dtype, const void* bias, int bias_
   return cw_launch_status();
 }
 
+// Cosines and sines of every token's angles, as the kernels above make them: [T, 2, n] for n frequencies. For a product that
+// rotates its results (csrc/gemm_tile.hip); once a step for all layers.
+__global__ __launch_bounds__(256) void rope_angles_kernel(const int* __restrict__ positions, const float* __restrict__ inv_freq, int64_t total, int n,
+                                                          float* __restrict__ out) {
+  const int64_t at = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (at >= total) return;
+  const int64_t t = at / n;
+  const int i = (int)(at - t * n);
+  float s_, c_;
+  sincosf((float)positions[t] * inv_freq[i], &s_, &c_);
+  out[2 * t * n + i] = c_;
+  out[(2 * t + 1) * n + i] = s_;
+}
+
+CW_EXPORT int cw_rope_angles(const int* positions, const float* inv_freq, int T, int n, float* out, hipStream_t stream) {
+  if (T < 0 || n <= 0 || !positions || !inv_freq || !out) return CW_ERR_ARG;
+  const int64_t total = (int64_t)T * n;
+  if (total == 0) return CW_OK;
+  if (total > (1ll << 38)) return CW_ERR_SIZE;
+  hipLaunchKernelGGL(rope_angles_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, positions, inv_freq, total, n, out);
+  return cw_launch_status();
+}
+
 // ---------------------------------------------------------------- SiLU(gate) * up
 // gate_up: [T, 2*I] (gate columns first), out: [T, I]; silu(z) = z / (1 + exp(-z)) in float32.
 template <typename T>

@@ -296,6 +296,11 @@ typedef __attribute__((address_space(3))) void lds_void_t;
 #define W_BLOCK 1024                       // bytes of a block: 8 rows x 64 elements
 #define W_GROUP_M 8                        // row tiles that run side by side
 
+__device__ __forceinline__ uint32_t w_pack_bf16(float lo, float hi) {
+  const f32x2_t v = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));  // v_cvt_pk_bf16_f32
+}
+
 struct WideArgs {
   const bf16_t* X;
   int64_t ldx;
@@ -314,7 +319,24 @@ struct WideArgs {
   const float* row_factor;  // nullptr, or a factor for the results that go to row row_target[m]: row_factor[row_target[m]]
   int64_t w_group_stride;   // elements from one stacked matrix to the next
   float act;                // MODE 2 and 5: which activation (see above)
+  // MODE 6 (of gemm_mid_bf16_kernel): heads of queries, keys and values, rotated and stored where they belong
+  const float* angles;      // [rows][2][hd / 2] cosines and sines of a row's position
+  const int* slots;         // [rows] the row of the caches, beyond them: none
+  bf16_t* k_cache;          // [cache_rows][nkv][hd]
+  bf16_t* v_cache;
+  int64_t cache_rows;
+  int nh, nkv, hd;
 };
+
+// MODE 6: a column of the result is a pair of a head, elements d and d + hd / 2; the row of W of its first element.
+__device__ __forceinline__ int64_t pair_row(int pair, int hd) { return (int64_t)(pair / (hd / 2)) * hd + pair % (hd / 2); }
+
+// Where the pairs of head ``head`` of row m go: a query to its row of C, a key or value to its slot; nullptr: nowhere.
+__device__ __forceinline__ bf16_t* pair_target(const WideArgs& a, int64_t m, int head, int64_t slot) {
+  if (head < a.nh) return (bf16_t*)a.C + m * a.ldc + (int64_t)head * a.hd;
+  if (slot < 0 || slot >= a.cache_rows) return nullptr;
+  return (head < a.nh + a.nkv ? a.k_cache + (slot * a.nkv + head - a.nh) * a.hd : a.v_cache + (slot * a.nkv + head - a.nh - a.nkv) * a.hd);
+}
 
 // The column of a wave's part of the tile (MODE 2: the output) that row r of its W block ni belongs to. The
 // accumulator of a block holds rows 4 s .. 4 s + 3 in lane (c, s). Two blocks: 8 neighbouring columns a lane. MODE 2,
@@ -330,11 +352,6 @@ __host__ __device__ __forceinline__ int wide_col(int ni, int r) {
     return (NB - 1) * 8 + s1 * 4 + e;
   }
   return ni < (NB & ~1) ? (ni >> 1) * 32 + s * 8 + (ni & 1) * 4 + e : ni * 16 + r;
-}
-
-__device__ __forceinline__ uint32_t w_pack_bf16(float lo, float hi) {
-  const f32x2_t v = {lo, hi};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));  // v_cvt_pk_bf16_f32
 }
 
 // cw_gated from the bare exp2 and reciprocal instructions
@@ -937,7 +954,8 @@ __global__ __launch_bounds__(256, 2) void gemm_mid_bf16_kernel(WideArgs a) {
   const int run = gridDim.x >> 3, rest = gridDim.x & 7, xcd = blockIdx.x & 7;
   const int tile = xcd * run + min(xcd, rest) + (blockIdx.x >> 3);
   const int tm = tile % a.tiles_m, tn = tile / a.tiles_m % a.tiles_n, plane = tile / (a.tiles_m * a.tiles_n);
-  const int m0 = tm * BM, w0 = tn * (MODE == 2 ? BN / 2 : BN);
+  constexpr bool PAIRS = MODE == 2 || MODE == 6;  // two rows of W a column
+  const int m0 = tm * BM, w0 = tn * (PAIRS ? BN / 2 : BN);
   const int stages = K / 64;
   const int first = MODE == 3 ? (int)((int64_t)stages * plane / a.k_splits) : 0;
   const int last = (MODE == 3 ? (int)((int64_t)stages * (plane + 1) / a.k_splits) : stages) - 1;
@@ -945,8 +963,9 @@ __global__ __launch_bounds__(256, 2) void gemm_mid_bf16_kernel(WideArgs a) {
   __amdgpu_buffer_rsrc_t xr, wr;
   xr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.X + (int64_t)m0 * a.ldx), 0,
                                          (int)(uint32_t)(((int64_t)(M - m0 - 1) * a.ldx + K) * 2), 0x00020000);
-  wr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.W + (int64_t)w0 * K), 0,
-                                         (int)(uint32_t)((int64_t)(N - w0) * K * 2), 0x00020000);
+  const int w_from = MODE == 6 ? 0 : w0;
+  wr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.W + (int64_t)w_from * K), 0,
+                                         (int)(uint32_t)((int64_t)(N - w_from) * K * 2), 0x00020000);
   // load i of a wave: block wave * LOADS + i of a stage, the x blocks first. (Of a size that hangs on no template
   // parameter, so that the host pass takes the loads below.)
   uint32_t at[8];
@@ -958,8 +977,10 @@ __global__ __launch_bounds__(256, 2) void gemm_mid_bf16_kernel(WideArgs a) {
       from = (int64_t)(block * 8 + (lane >> 3)) * a.ldx;
     } else {
       const int rb = (block - XB) * 8 + (lane >> 3);
-      if (MODE == 2) {  // a wave's rows are gate rows followed by the up rows with the same indices
+      if (PAIRS) {  // a wave's rows are gate rows followed by the up rows with the same indices (MODE 6: first and second halves)
         const int q = rb % (BN / 2), i2 = rb / (BN / 2) * (BN / 4) + q % (BN / 4);
+        if (MODE == 6) from = min(pair_row(w0 + i2, a.hd) + (q < BN / 4 ? 0 : a.hd / 2), (int64_t)N) * K;
+        else
         from = (int64_t)(q < BN / 4 ? i2 : I + i2) * K;
       } else {
         from = (int64_t)rb * K;
@@ -981,6 +1002,33 @@ __global__ __launch_bounds__(256, 2) void gemm_mid_bf16_kernel(WideArgs a) {
   for (int mi = 0; mi < TM; ++mi)
 #pragma unroll
     for (int ni = 0; ni < TN; ++ni) acc[mi][ni] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
+  // MODE 6: what the rotation and the stores need, asked for ahead of the tiles (asked for at the end, its trips to memory are 2 us)
+  constexpr int PAIR_BLOCKS = MODE == 6 ? TN / 2 : 1;
+  float4 cosines[TM][PAIR_BLOCKS], sines[TM][PAIR_BLOCKS];
+  float bias_first[PAIR_BLOCKS][4], bias_second[PAIR_BLOCKS][4];
+  int slot_of[TM];
+  if constexpr (MODE == 6) {
+#pragma unroll
+    for (int ni = 0; ni < PAIR_BLOCKS; ++ni) {
+      const int pair = min(w0 + wn * (BN / 4) + ni * 16, I - 16), head = pair / (a.hd / 2), d = pair - head * (a.hd / 2) + 4 * s;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int64_t at_first = (int64_t)head * a.hd + d + e, at_second = at_first + a.hd / 2;
+        bias_first[ni][e] = a.bias == nullptr ? 0.0f : a.bias_f32 ? ((const float*)a.bias)[at_first] : __bfloat162float(((const bf16_t*)a.bias)[at_first]);
+        bias_second[ni][e] = a.bias == nullptr ? 0.0f : a.bias_f32 ? ((const float*)a.bias)[at_second] : __bfloat162float(((const bf16_t*)a.bias)[at_second]);
+      }
+#pragma unroll
+      for (int mi = 0; mi < TM; ++mi) {
+        const int64_t m = min(m0 + (wm * TM + mi) * 16 + c, M - 1);
+        if (ni == 0) slot_of[mi] = a.slots[m];
+        cosines[mi][ni] = make_float4(1.0f, 1.0f, 1.0f, 1.0f), sines[mi][ni] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (head < a.nh + a.nkv) {
+          cosines[mi][ni] = *reinterpret_cast<const float4*>(a.angles + m * a.hd + d);
+          sines[mi][ni] = *reinterpret_cast<const float4*>(a.angles + m * a.hd + a.hd / 2 + d);
+        }
+      }
+    }
+  }
 #pragma unroll
   for (int i = 0; i < MID_SLOTS - 1; ++i) fetch(min(first + i, last), i);
   int slot = 0;
@@ -1010,11 +1058,33 @@ __global__ __launch_bounds__(256, 2) void gemm_mid_bf16_kernel(WideArgs a) {
   W_WAIT_LOADS(0);  // no load may reach LDS after the workgroup has gone
 
   // lane (c, s) holds columns 4 s .. 4 s + 3 of W block ni for row c of x block mi
-  const int out_cols = MODE == 2 ? I : N;
+  const int out_cols = PAIRS ? I : N;
 #pragma unroll
   for (int mi = 0; mi < TM; ++mi) {
     const int m = m0 + (wm * TM + mi) * 16 + c;
     if (m >= M) continue;
+    if constexpr (MODE == 6) {
+#pragma unroll
+      for (int ni = 0; ni < TN / 2; ++ni) {
+        const int pair = w0 + wn * (BN / 4) + ni * 16, head = pair / (a.hd / 2), d = pair - head * (a.hd / 2) + 4 * s;  // 16 pairs of one head
+        bf16_t* to = pair < I ? pair_target(a, m, head, slot_of[mi]) : nullptr;
+        if (to == nullptr) continue;
+        const f32x4_t first4 = acc[mi][ni], second4 = acc[mi][ni + TN / 2];
+        const float co[4] = {cosines[mi][ni].x, cosines[mi][ni].y, cosines[mi][ni].z, cosines[mi][ni].w};
+        const float si[4] = {sines[mi][ni].x, sines[mi][ni].y, sines[mi][ni].z, sines[mi][ni].w};
+        float x[4], y[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float f = first4[e] + bias_first[ni][e], g = second4[e] + bias_second[ni][e];
+          const bool rotated = head < a.nh + a.nkv;   // (values pass as they are, infinities among them)
+          x[e] = rotated ? f * co[e] - g * si[e] : f;
+          y[e] = rotated ? g * co[e] + f * si[e] : g;
+        }
+        *reinterpret_cast<uint2*>(to + d) = make_uint2(w_pack_bf16(x[0], x[1]), w_pack_bf16(x[2], x[3]));
+        *reinterpret_cast<uint2*>(to + a.hd / 2 + d) = make_uint2(w_pack_bf16(y[0], y[1]), w_pack_bf16(y[2], y[3]));
+      }
+      continue;
+    }
 #pragma unroll
     for (int ni = 0; ni < (MODE == 2 ? TN / 2 : TN); ++ni) {
       const int n = w0 + (MODE == 2 ? wn * (BN / 4) : wn * (BN / 2)) + ni * 16 + 4 * s;
@@ -1062,8 +1132,8 @@ static int mid_launch(WideArgs a, hipStream_t stream) {
       return CW_ERR_LAUNCH;
     raised = true;
   }
-  const int out_cols = MODE == 2 ? a.N / 2 : a.N;
-  const int per_tile = MODE == 2 ? BN / 2 : BN;
+  const int out_cols = MODE == 2 || MODE == 6 ? a.N / 2 : a.N;
+  const int per_tile = MODE == 2 || MODE == 6 ? BN / 2 : BN;
   a.tiles_n = (out_cols + per_tile - 1) / per_tile;
   a.tiles_m = (a.M + BM - 1) / BM;
   const int64_t total = (int64_t)a.tiles_m * a.tiles_n * (MODE == 3 ? a.k_splits : 1);
@@ -1214,4 +1284,42 @@ CW_EXPORT int cw_gemm_bf16_mid_choice(int mode, int M, int N, int K, int64_t ldx
     if ((float)items < (items > cus ? 0.72f : M > 1024 ? 0.55f : 0.0f) * (float)(cus * ((items + cus - 1) / cus))) return 0;
   }
   return best;
+}
+
+// Does the product of the queries, keys and values of M tokens run with bias, rotation and cache write inside (cw_gemm_bf16_pairs)?
+// In 64 x 64 tiles, where they are the ones for the product or nearly so: up to 576 of them and K of 2048. Where the lines lie (us, in a
+// graph, operands from memory, the fastest product and the rotation kernel behind it -> here): 0.5B shape, 160 rows 9.5 -> 7.8, 1000 rows
+// 12.1 -> 10.1, 2048 rows (576 tiles) 15.4 -> 14.5; 1.5B shape, 72 rows 10.9 -> 9.8, 336 rows 12.5 -> 10.4, 1000 rows (512) 16.2 -> 14.8, 1500
+// rows (768) 21.4 -> 21.7; 3B shape (K 2048), 72 rows 12.4 -> 13.2, 160 rows 14.5 -> 12.5, 768 rows (480) 19.3 -> 17.9, 1000 rows (640)
+// 21.4 -> 23.1; 7B shape (K 3584), 336 rows 29.7 -> 32.3. In tiles of 128 x 128 the rotation's end costs more than its kernel.
+CW_EXPORT int cw_gemm_bf16_pairs_ok(int M, int N, int K, int64_t ldx, int hd) {
+  if (M <= 64 || N <= 0 || K < 256 || (K & 63) || (ldx & 7) || ldx < K) return 0;
+  if ((hd & 31) || hd < 32 || hd > 256 || N % hd || K > 2048 || (K > 1536 && M < 128)) return 0;
+  return (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= 576 ? 1 : 0;
+}
+
+// Rows of x W^T (+ bias) as heads of hd elements, nh of queries, then nkv of keys and nkv of values, queries and keys rotated by
+// ``angles`` [M, 2, hd / 2] (cw_rope_angles): queries to Q [M, nh hd], keys and values to rows ``slots`` of the caches (negative
+// or beyond cache_rows: nowhere). Heads of a multiple of 32 elements up to 256.
+CW_EXPORT int cw_gemm_bf16_pairs(const void* X, int64_t ldx, const void* W, const void* bias, int bias_f32, const float* angles, const int* slots,
+                                 void* Q, void* k_cache, void* v_cache, int64_t cache_rows, int M, int K, int nh, int nkv, int hd, hipStream_t stream) {
+  if (M < 0 || K <= 0 || nh <= 0 || nkv <= 0 || hd <= 0 || cache_rows < 0) return CW_ERR_ARG;
+  if (!X || !W || !angles || !slots || !Q || !k_cache || !v_cache) return CW_ERR_ARG;
+  if (((uintptr_t)X & 15) || ((uintptr_t)W & 15) || ((uintptr_t)Q & 15) || ((uintptr_t)k_cache & 15) || ((uintptr_t)v_cache & 15) || ((uintptr_t)angles & 15))
+    return CW_ERR_ARG;
+  const int64_t n = ((int64_t)nh + 2 * (int64_t)nkv) * hd;
+  if (n > 0x7fffffff || (hd & 31) || hd > 256 || (K & 63) || (ldx & 7) || ldx < K) return CW_ERR_ARG;
+  const int N = (int)n;
+  if ((int64_t)N * K * 2 >= (1ll << 32) || ((int64_t)M * ldx + 256 * ldx) * 2 >= (1ll << 32)) return CW_ERR_SIZE;
+  if (M == 0) return CW_OK;
+  WideArgs a{(const bf16_t*)X, ldx, (const bf16_t*)W, bias, bias_f32, Q, (int64_t)nh * hd, M, N, K, 0, 0, 1};
+  a.angles = angles;
+  a.slots = slots;
+  a.k_cache = (bf16_t*)k_cache;
+  a.v_cache = (bf16_t*)v_cache;
+  a.cache_rows = cache_rows;
+  a.nh = nh;
+  a.nkv = nkv;
+  a.hd = hd;
+  return mid_launch<6, 64, 64>(a, stream);
 }

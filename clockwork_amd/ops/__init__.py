@@ -95,6 +95,7 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
         "core": {
             "cw_embedding": [P, I, P, P, I, I, I, P],
             "cw_add_rmsnorm": [P, P, P, I, I, P, I, F, P, I, P, I, I, P, P, P],
+            "cw_rope_angles": [P, P, I, I, P, P],
             "cw_rope_kv_write": [P, I, P, I, P, P, P, I, I, I, I, I, P, P, L, P],
             "cw_silu_mul": [P, P, I, I, I, F, P],
             "cw_copy_pages": [P, I, L, L, P, I, P],
@@ -123,6 +124,8 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_gemm_bf16_wide_partial": [P, L, P, P, L, I, I, I, I, I, P],
             "cw_gemm_bf16_mid_choice": [I, I, I, I, L, I],
             "cw_gemm_bf16_wide_choice": [I, I, I, I, L, I],
+            "cw_gemm_bf16_pairs_ok": [I, I, I, L, I],
+            "cw_gemm_bf16_pairs": [P, L, P, P, I, P, P, P, P, P, L, I, I, I, I, I, P],
             "cw_gemm_bf16_mid": [I, P, L, P, P, I, P, L, I, I, I, F, I, I, I, I, P],
             "cw_gemm_bf16_wide_grouped": [I, P, L, P, L, P, L, I, I, P, P, I, P, P, F, I, P],
         },
@@ -1152,6 +1155,46 @@ def qkv_rope_fused(x, weight, bias, positions, slots, inv_freq, nh: int, nkv: in
             M, K, nh, nkv, hd, _stream()),
         "gemm_qkv_rope_bf16",
     )
+    return q
+
+
+def rope_angles(positions: torch.Tensor, inv_freq: torch.Tensor) -> torch.Tensor:
+    """Cosines and sines of the tokens' angles, float32 [T, 2, len(inv_freq)]: what ``qkv_rope_rows`` rotates by."""
+    _gpu(positions, inv_freq)
+    T, n = positions.numel(), inv_freq.numel()
+    _i32(positions, T, "positions")
+    _need(inv_freq.dtype == torch.float32, "inv_freq must be float32")
+    out = torch.empty((T, 2, n), dtype=torch.float32, device=positions.device)
+    _check(_load("core").cw_rope_angles(_ptr(positions), _ptr(inv_freq), T, n, _ptr(out), _stream()), "rope_angles")
+    return out
+
+
+def qkv_rope_rows_ok(x: torch.Tensor, weight: torch.Tensor, bias, rotary_dim: int, hd: int, k_cache, v_cache) -> bool:
+    """Is ``qkv_rope_rows`` the faster way for these operands, by the rule of ``cw_gemm_bf16_pairs_ok``?"""
+    if not (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and k_cache.dtype == torch.bfloat16 and rotary_dim == hd
+            and x.is_contiguous() and _aligned(x, weight, k_cache, v_cache) and (bias is None or bias.dtype in (torch.bfloat16, torch.float32))):
+        return False
+    M, K = x.shape
+    return bool(_load("gemm_tile").cw_gemm_bf16_pairs_ok(M, weight.shape[0], K, K, hd))
+
+
+def qkv_rope_rows(x, weight, bias, angles, slots, nh: int, nkv: int, hd: int, k_cache, v_cache) -> torch.Tensor:
+    """``qkv_rope_fused`` for many rows: queries [M, nh * hd], keys and values at rows ``slots`` of the caches, through the
+    64 x 64 tiles (csrc/gemm_tile.hip); rotated by ``rope_angles``' table. Sums are rounded once, after the rotation."""
+    _gpu(x, weight, bias, angles, slots, k_cache, v_cache)
+    M, K = x.shape
+    if not (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and tuple(weight.shape) == ((nh + 2 * nkv) * hd, K)):
+        raise KernelError("qkv weight must be bfloat16 [(nh + 2 nkv) hd, K]")
+    _i32(slots, M, "slots")
+    _need(angles.dtype == torch.float32 and tuple(angles.shape) == (M, 2, hd // 2), "angles must be float32 [M, 2, hd / 2]")
+    _need(k_cache.dtype == torch.bfloat16 and v_cache.dtype == torch.bfloat16 and tuple(k_cache.shape[-2:]) == (nkv, hd) and k_cache.shape == v_cache.shape,
+          "cache must be bfloat16 [..., nkv, hd]")
+    if bias is not None and not (bias.numel() == weight.shape[0] and bias.dtype in (torch.bfloat16, torch.float32)):
+        raise KernelError("qkv bias")
+    q = torch.empty((M, nh * hd), dtype=torch.bfloat16, device=x.device)
+    _check(_load("gemm_tile").cw_gemm_bf16_pairs(_ptr(x), K, _ptr(weight), _ptr(bias), int(bias is not None and bias.dtype == torch.float32),
+                                                 _ptr(angles), _ptr(slots), _ptr(q), _ptr(k_cache), _ptr(v_cache), k_cache.numel() // (nkv * hd),
+                                                 M, K, nh, nkv, hd, _stream()), "gemm_bf16_pairs")
     return q
 
 

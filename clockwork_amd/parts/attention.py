@@ -354,6 +354,9 @@ class PagedAttention(Part):
         qkv = None
         if fused is not None:
             qkv = fused(x, self.qkv_weight, self.qkv_bias, ctx.positions, ctx.slots[cache.group], nh, nkv, hd, cache.k, cache.v)
+        rows = getattr(self.position, "project_rotate_store_rows", None) if cache.writes and qkv is None else None
+        if rows is not None:
+            qkv = rows(x, self.qkv_weight, self.qkv_bias, ctx, ctx.slots[cache.group], nh, nkv, hd, cache.k, cache.v)
         if qkv is not None:
             pass  # q only, [T, nh * hd]: keys and values are in the cache already
         elif cache.writes:

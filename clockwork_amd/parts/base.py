@@ -32,7 +32,8 @@ Roles and their run methods:
                  ``rotate_and_store(qkv, bias, positions, slots, nh, nkv, hd, k, v)``, and
                  uses ``project_rotate_store(x, weight, bias, positions, slots, nh, nkv, hd,
                  k, v) -> q or None`` when the part offers it (product, encoding and cache
-                 write in one kernel).
+                 write in one kernel), and where that has nothing ``project_rotate_store_rows``,
+                 with the context in the place of the positions.
 * arrangement:   built by its factory from the block's parts as keyword arguments, under
                  the names the ``LayerSpec`` gives them (``mixer``, ``feed_forward``,
                  ``mixer_norm``, ``ffn_norm`` or any others). ``parts() -> {name: part}``;

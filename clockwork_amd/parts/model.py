@@ -161,6 +161,7 @@ class DecoderModel:
         positions_of = getattr(self.embedding, "positions", None)
         if positions_of is not None:
             ctx.positions = positions_of(ctx)
+        ctx.made = {}   # what this pass makes on the device for several layers, by keys of the parts' own
         # a part outside the blocks that keeps something has its cache behind those of the run entries
         own = bool(self.own_caches())
         resid = self.embedding.forward(ctx, caches[len(self.spec.run)]) if own else self.embedding.forward(ctx)

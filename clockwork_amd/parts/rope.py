@@ -63,6 +63,21 @@ class RopeNeox(Part):
         return ops.qkv_rope_fused(x, weight, bias, positions, slots, self.inv_freq, nh, nkv, hd, k_cache, v_cache)
 
 
+    def project_rotate_store_rows(self, x, weight, bias, ctx, slots, nh, nkv, hd, k_cache, v_cache):
+        """The same for a portion's rows: by a table of the step's angles, made by the first layer that asks in a pass
+        over the model (``ctx.made``; 1 MB for 2048 tokens, 2 us). None where a product and ``rotate_and_store`` are the faster way."""
+        if slots is None or not ops.qkv_rope_rows_ok(x, weight, bias, self.spec.rotary_dim, hd, k_cache, v_cache):
+            return None
+        made = getattr(ctx, "made", None)
+        key = ("angles", self.spec.theta, self.spec.rotary_dim)
+        angles = made.get(key) if made is not None else None
+        if angles is None:
+            angles = ops.rope_angles(ctx.positions, self.inv_freq)
+            if made is not None:
+                made[key] = angles
+        return ops.qkv_rope_rows(x, weight, bias, angles, slots, nh, nkv, hd, k_cache, v_cache)
+
+
 class NoPosition(Part):
     """Stands in when a mixer has no position encoding: bias and cache write only."""
 

@@ -265,6 +265,53 @@ def test_tiles_for_whole_rows_refuse_others(mode, N):
         torch.testing.assert_close(got.sum() if mode == 3 else got.float(), want, **bf16)
 
 
+# one row, rows and pairs that end inside a tile, heads of one, three and four blocks of 16 pairs, a head over several tiles, an odd number of heads
+@pytest.mark.parametrize("M", [1, 65, 130, 333])
+@pytest.mark.parametrize("nh,nkv,hd,K,bias_dtype", [(12, 2, 128, 1536, torch.bfloat16), (14, 2, 64, 896, torch.float32), (3, 1, 32, 256, None),
+                                                    (3, 3, 96, 320, torch.bfloat16), (2, 1, 256, 512, None)])
+def test_queries_keys_and_values_of_many_rows_in_one_kernel(M, nh, nkv, hd, K, bias_dtype):
+    """Product, bias, rotation and cache write against the same in float64, rows without a slot and slots that no row has
+    left as they are, and the table of angles against the rotation kernel's own."""
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(M + hd)
+    width = (nh + 2 * nkv) * hd
+    x = torch.randn(M, K, device=DEV, generator=gen).to(torch.bfloat16)
+    w = (torch.randn(width, K, device=DEV, generator=gen) / K ** 0.5).to(torch.bfloat16)
+    bias = None if bias_dtype is None else torch.randn(width, device=DEV, generator=gen).to(bias_dtype)
+    positions = torch.randint(0, 30000, (M,), dtype=torch.int32, device=DEV, generator=gen)
+    inv_freq = (1.0 / 1e6 ** (torch.arange(0, hd, 2, dtype=torch.float32) / hd)).to(DEV)
+    slots = torch.randperm(M + 9, device=DEV, generator=gen)[:M].to(torch.int32)
+    slots[::5] = -1
+    slots[3::11] = M + 9   # beyond the cache
+    kc = torch.full((M + 9, nkv, hd), 9.0, device=DEV, dtype=torch.bfloat16)
+    vc = kc.clone()
+    angles = ops.rope_angles(positions, inv_freq)
+    q = ops.qkv_rope_rows(x, w, bias, angles, slots, nh, nkv, hd, kc, vc)
+    # the table is what the rotation kernel turns a pair (1, 0) by
+    ones = torch.zeros(M, 1, 2, hd // 2, device=DEV)
+    ones[:, :, 0] = 1.0
+    turned = ones.view(M, hd).contiguous()
+    ops.rope_kv_write(turned, None, positions, None, inv_freq, hd, 1, 0, hd, None, None)
+    assert torch.equal(turned.view(M, 2, hd // 2), angles)
+    y = x.double() @ w.double().t()
+    y = (y if bias is None else y + bias.double()).view(M, nh + 2 * nkv, hd)
+    a, b = y.chunk(2, dim=2)
+    cos, sin = (angles[:, j].double()[:, None, :] for j in (0, 1))
+    want = torch.cat([a * cos - b * sin, b * cos + a * sin], dim=2)
+    want[:, nh + nkv:] = y[:, nh + nkv:]
+    # float32 sums of K products of about 1 / sqrt(K) and one rounding to bfloat16
+    t = dict(rtol=2.0 ** -8 + 1e-4, atol=1e-4)
+    torch.testing.assert_close(q.double().view(M, nh, hd), want[:, :nh], **t)
+    live = (slots >= 0) & (slots < M + 9)
+    rows = slots[live].long()
+    torch.testing.assert_close(kc[rows].double(), want[live, nh:nh + nkv], **t)
+    torch.testing.assert_close(vc[rows].double(), want[live, nh + nkv:], **t)
+    rest = torch.ones(M + 9, dtype=torch.bool, device=DEV)
+    rest[rows] = False
+    assert bool((kc[rest] == 9.0).all()) and bool((vc[rest] == 9.0).all())
+
+
 def test_products_of_a_portion_by_their_rule():
     """What the rule names runs and is the product, on every side of its lines."""
     from clockwork_amd import ops

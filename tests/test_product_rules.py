@@ -64,6 +64,14 @@ def test_products_on_the_wide_kernels_tiles(mode, M, N, K, there):
         assert _wide_choice(mode, M, N, K, K + 4) is None   # rows of x at no 16 bytes
 
 
+@pytest.mark.parametrize("M,N,K,hd,there", [(2048, 1152, 896, 64, True), (2049, 1152, 896, 64, False), (1024, 2048, 1536, 128, True),
+                                           (1152, 2048, 1536, 128, True), (1153, 2048, 1536, 128, False), (72, 2048, 1536, 128, True), (72, 2560, 2048, 128, False),
+                                           (128, 2560, 2048, 128, True), (336, 4608, 3584, 128, False), (64, 1152, 896, 64, False), (160, 1152, 896, 48, False),
+                                           (160, 1150, 896, 64, False), (160, 1152, 900, 64, False)])
+def test_queries_keys_and_values_rotated_by_their_product(M, N, K, hd, there):
+    assert bool(ops._load("gemm_tile").cw_gemm_bf16_pairs_ok(M, N, K, K, hd)) == there
+
+
 def test_tiles_follow_the_rounds_that_they_need():
     """Gate/up of the 1.5B shape: the tile whose rounds over the compute units are fullest for what they cost."""
     tiles = {M: _wide_choice(2, M, 17920, 1536)[:2] for M in (100, 160, 336, 512, 1000, 2048)}
