@@ -3,6 +3,9 @@
 //  * cw_gemm_f32: true float32 on the matrix cores (v_mfma_f32_16x16x4_f32: float32 operands, products
 //    and sums). The order in which the products of one output element are summed depends on N and K
 //    alone, never on M, so a row's result does not depend on what else is in the batch.
+#include <climits>
+#include <type_traits>
+
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
@@ -692,10 +695,8 @@ __device__ __forceinline__ float cw_relu_squared(float z) { const float r = fmax
 // is cut into more, smaller tiles so that every compute unit streams a share of the matrix (the
 // unused rows of the MFMA tile are zeros). MODE 2 needs ROWS == 16.
 template <int MT, int RT, int MODE, int WAVES, int ROWS>
-__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_bf16_kernel(const bf16_t* __restrict__ X, int64_t ldx,
-                                                               const bf16_t* __restrict__ W,
-                                                               void* __restrict__ C, int64_t ldc,
-                                                               int M, int N, int K, float act) {
+__device__ __forceinline__ void skinny_tiles(const bf16_t* __restrict__ X, int64_t ldx, const bf16_t* __restrict__ W,
+                                             void* __restrict__ C, int64_t ldc, int M, int N, int K, float act, const int block) {
   __shared__ float red[WAVES][RT * MT * 256];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, s = lane >> 4;
@@ -709,11 +710,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_bf16_kernel(const bf16
   for (int rt = 0; rt < RT; ++rt) {
     int64_t n;
     if (MODE == 2) {
-      const int64_t i = ((int64_t)blockIdx.x * RT + rt) * 8 + (lr & 7);
+      const int64_t i = ((int64_t)block * RT + rt) * 8 + (lr & 7);
       n = (lr < 8) ? i : I + i;
       wok[rt] = i < I;
     } else {
-      n = ((int64_t)blockIdx.x * RT + rt) * ROWS + lr;
+      n = ((int64_t)block * RT + rt) * ROWS + lr;
       wok[rt] = lr < ROWS && n < N;
     }
     wrow[rt] = W + (wok[rt] ? n : 0) * K;
@@ -795,7 +796,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_bf16_kernel(const bf16
     for (int idx = threadIdx.x; idx < RT * MT * 128; idx += WAVES * 64) {
       const int j = idx & 7, rt = (idx >> 3) % RT, m = idx / (8 * RT);
       const int mt = m >> 4, tok = m & 15;
-      const int64_t i = ((int64_t)blockIdx.x * RT + rt) * 8 + j;
+      const int64_t i = ((int64_t)block * RT + rt) * 8 + j;
       if (m >= M || i >= I) continue;
       const float g = red[0][(rt * MT + mt) * 256 + j * 16 + tok];
       const float u = red[0][(rt * MT + mt) * 256 + (j + 8) * 16 + tok];
@@ -805,7 +806,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_bf16_kernel(const bf16
     for (int idx = threadIdx.x; idx < RT * MT * 256; idx += WAVES * 64) {
       const int j = idx & 15, rt = (idx >> 4) % RT, m = idx / (16 * RT);
       const int mt = m >> 4, tok = m & 15;
-      const int64_t n = ((int64_t)blockIdx.x * RT + rt) * ROWS + j;
+      const int64_t n = ((int64_t)block * RT + rt) * ROWS + j;
       if (m >= M || n >= N || j >= ROWS) continue;
       const float v = red[0][(rt * MT + mt) * 256 + j * 16 + tok];
       if (MODE == 3) ((float*)C)[((int64_t)blockIdx.y * M + m) * ldc + n] = v;
@@ -815,6 +816,41 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_bf16_kernel(const bf16
       else ((bf16_t*)C)[(int64_t)m * ldc + n] = __float2bfloat16(v);
     }
   }
+}
+
+template <int MT, int RT, int MODE, int WAVES, int ROWS>
+__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_bf16_kernel(const bf16_t* __restrict__ X, int64_t ldx,
+                                                               const bf16_t* __restrict__ W,
+                                                               void* __restrict__ C, int64_t ldc,
+                                                               int M, int N, int K, float act) {
+  skinny_tiles<MT, RT, MODE, WAVES, ROWS>(X, ldx, W, C, ldc, M, N, K, act, blockIdx.x);
+}
+
+// Several products of the same rows and the same K as one launch, each with an x, a matrix and an output of its own: a layer that
+// multiplies one input by three matrices of 2 to 5 thousand rows, or two inputs by a matrix each. By itself such a product streams
+// 1 to 2.5 TB/s, for its 100 to 300 row tiles leave compute units idle and every launch pays its ramp of 2 to 3 us. Measured on an
+// MI355X, a width of 1536, apart and together (us): 8 rows, outputs of 2048, 4640 and 3072 16.6 and 7.6, two of 1536 9.2 and 5.1;
+// one row 13.7 and 7.5, 7.6 and 4.4; a width of 896, three outputs of 2048, 2000 and 1024, 8 rows 9.7 and 3.7.
+#define GROUP_MAX 4
+struct ProductGroup {
+  const bf16_t* x[GROUP_MAX];
+  const bf16_t* w[GROUP_MAX];
+  bf16_t* c[GROUP_MAX];
+  int n[GROUP_MAX];
+  int first[GROUP_MAX + 1];  // tiles of 16 rows of W before each product's, INT_MAX past the last
+};
+// the product that row tile ``tile`` belongs to (the same for a whole workgroup)
+__device__ __forceinline__ int group_of(const ProductGroup& group, int tile) {
+  int g = 0;
+#pragma unroll
+  for (int i = 1; i < GROUP_MAX; ++i) g += tile >= group.first[i];
+  return g;
+}
+
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_group_bf16_kernel(ProductGroup group, int M, int K) {
+  const int g = group_of(group, blockIdx.x);
+  skinny_tiles<1, 1, 0, WAVES, 16>(group.x[g], K, group.w[g], group.c[g], group.n[g], M, group.n[g], K, 0.0f, (int)blockIdx.x - group.first[g]);
 }
 
 // The same product with the x fragments of a wave's whole share of the K loop (up to 24 steps of
@@ -842,11 +878,14 @@ struct StreamNormIn {
 // fragments of all SPW steps stay in registers: a long K costs registers for x only.
 constexpr int cw_stream_chunk(int spw) { return spw <= 8 ? spw : (spw <= 12 ? spw / 2 : spw / 4); }
 
-template <int MODE, int WAVES, int SPW, int MT, bool NORM = false>
+// GROUP (MODE 0): row tiles of several products of the same x, ``in`` a ProductGroup (W, C, ldc and N are not used).
+template <int MODE, int WAVES, int SPW, int MT, bool NORM = false, bool GROUP = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16_t* __restrict__ X, int64_t ldx,
                                                                const bf16_t* __restrict__ W,
                                                                void* __restrict__ C, int64_t ldc,
-                                                               int M, int N, int K, int n_tiles, float act, StreamNormIn nin) {
+                                                               int M, int N, int K, int n_tiles, float act,
+                                                               std::conditional_t<GROUP, ProductGroup, StreamNormIn> in) {
+  static_assert(!GROUP || (MODE == 0 && !NORM), "grouped products are plain ones");
   constexpr int NBUF = MT <= 2 ? 2 : 1;
   constexpr int CH = cw_stream_chunk(SPW), NC = SPW / CH;
   static_assert(SPW % CH == 0, "the steps of a wave are whole chunks");
@@ -868,6 +907,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
   }
   auto wrow = [&](int tile) __attribute__((always_inline)) -> const bf16_t* {
     int64_t n;
+    if constexpr (GROUP) {
+      const int g = group_of(in, tile);
+      return in.w[g] + (int64_t)min((tile - in.first[g]) * 16 + lr, in.n[g] - 1) * K;
+    }
     if (MODE == 2) {  // gate and up rows alternate, so that a pair lies side by side in the tile
       const int64_t i = min((int64_t)tile * 8 + (lr >> 1), (int64_t)I - 1);
       n = (lr & 1) ? I + i : i;
@@ -896,18 +939,18 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[u][e] = wv[u][e] = 0.0f;
       if (k + 8 <= K && r < M) {
-        const float4 a = *reinterpret_cast<const float4*>(nin.resid + (int64_t)r * K + k);
-        const float4 b = *reinterpret_cast<const float4*>(nin.resid + (int64_t)r * K + k + 4);
-        const bf16x8_t d = *reinterpret_cast<const bf16x8_t*>(nin.delta + (int64_t)r * K + k);
+        const float4 a = *reinterpret_cast<const float4*>(in.resid + (int64_t)r * K + k);
+        const float4 b = *reinterpret_cast<const float4*>(in.resid + (int64_t)r * K + k + 4);
+        const bf16x8_t d = *reinterpret_cast<const bf16x8_t*>(in.delta + (int64_t)r * K + k);
         v[u][0] = a.x + (float)d[0]; v[u][1] = a.y + (float)d[1]; v[u][2] = a.z + (float)d[2]; v[u][3] = a.w + (float)d[3];
         v[u][4] = b.x + (float)d[4]; v[u][5] = b.y + (float)d[5]; v[u][6] = b.z + (float)d[6]; v[u][7] = b.w + (float)d[7];
-        if (nin.weight_f32) {
-          const float4 w0 = *reinterpret_cast<const float4*>((const float*)nin.weight + k);
-          const float4 w1 = *reinterpret_cast<const float4*>((const float*)nin.weight + k + 4);
+        if (in.weight_f32) {
+          const float4 w0 = *reinterpret_cast<const float4*>((const float*)in.weight + k);
+          const float4 w1 = *reinterpret_cast<const float4*>((const float*)in.weight + k + 4);
           wv[u][0] = w0.x; wv[u][1] = w0.y; wv[u][2] = w0.z; wv[u][3] = w0.w;
           wv[u][4] = w1.x; wv[u][5] = w1.y; wv[u][6] = w1.z; wv[u][7] = w1.w;
         } else {
-          const bf16x8_t w8 = *reinterpret_cast<const bf16x8_t*>((const bf16_t*)nin.weight + k);
+          const bf16x8_t w8 = *reinterpret_cast<const bf16x8_t*>((const bf16_t*)in.weight + k);
 #pragma unroll
           for (int e = 0; e < 8; ++e) wv[u][e] = (float)w8[e];
         }
@@ -921,7 +964,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
     float total = 0.0f;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) total += ssq[w][r];
-    const float inv = 1.0f / sqrtf(total / (float)K + nin.eps);
+    const float inv = 1.0f / sqrtf(total / (float)K + in.eps);
 #pragma unroll
     for (int u = 0; u < SPW; ++u)
 #pragma unroll
@@ -975,6 +1018,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
         float v = 0.0f;
 #pragma unroll
         for (int w = 0; w < WAVES; ++w) v += red[buf][w][idx];
+        if constexpr (GROUP) {
+          const int g = group_of(in, tile), n = (tile - in.first[g]) * 16 + j;
+          if (m < M && n < in.n[g]) in.c[g][(int64_t)m * in.n[g] + n] = __float2bfloat16(v);
+          continue;
+        }
         const int64_t n = (int64_t)tile * 16 + j;
         if (m < M && n < N) {
           if (MODE == 3) ((float*)C)[((int64_t)blockIdx.y * M + m) * ldc + n] = v;
@@ -1318,6 +1366,68 @@ CW_EXPORT int cw_gemm_bf16_skinny(int mode, const void* X, int64_t ldx, const vo
   if (tiles <= 256 && K >= 1024) return launch_skinny<4, 1, 8>(mode, x, ldx, w, C, ldc, M, N, K, 1, act, stream);
   return rows >= 4096 ? launch_skinny<4, 2, 4>(mode, x, ldx, w, C, ldc, M, N, K, 1, act, stream)
                       : launch_skinny<4, 1, 4>(mode, x, ldx, w, C, ldc, M, N, K, 1, act, stream);
+}
+
+// Are these products of ``M`` rows and K columns taken as one launch (``tiles``: their tiles of 16 rows of W)? Up to 16 rows
+// always; beyond, and up to 64, where all have the same x and the streaming kernel takes them (apart, those of fewer than 256
+// tiles are products of the library or of 64-row tiles).
+CW_EXPORT int cw_gemm_bf16_group_ok(int count, int same_x, int M, int64_t tiles, int K) {
+  if (count < 2 || count > GROUP_MAX || M < 1 || M > CW_SKINNY_MAX_M || K < 8 || (K & 7) || tiles < count || tiles > (1 << 20)) return 0;
+  if (M <= 16) return 1;
+  int mt, spw, n_tiles;
+  dim3 grid;
+  return same_x && plan_stream(0, M, (int)tiles * 16, K, 1, &mt, &spw, &grid, &n_tiles) && spw <= 8 ? 1 : 0;
+}
+
+// C[i] [M, N[i]] = X[i] W[i]^T for ``count`` products, all bfloat16, rows without gaps: X[i] [M, K], W[i] [N[i], K].
+CW_EXPORT int cw_gemm_bf16_group(int count, const void* const* X, const void* const* W, void* const* C, const int* N, int M, int K,
+                                 hipStream_t stream) {
+  if (count < 2 || count > GROUP_MAX || M < 0 || !X || !W || !C || !N) return CW_ERR_ARG;
+  ProductGroup group{};
+  int64_t tiles = 0;
+  bool same_x = true;
+  for (int i = 0; i < GROUP_MAX; ++i) {
+    group.first[i] = i < count ? (int)tiles : INT_MAX;
+    if (i >= count) continue;
+    if (N[i] <= 0 || N[i] > (1 << 24) || !X[i] || !W[i] || !C[i] || ((uintptr_t)X[i] & 15) || ((uintptr_t)W[i] & 15)) return CW_ERR_ARG;
+    group.x[i] = (const bf16_t*)X[i];
+    group.w[i] = (const bf16_t*)W[i];
+    group.c[i] = (bf16_t*)C[i];
+    group.n[i] = N[i];
+    tiles += (N[i] + 15) / 16;
+    same_x = same_x && X[i] == X[0];
+  }
+  group.first[GROUP_MAX] = INT_MAX;
+  if (M == 0) return CW_OK;
+  if (!cw_gemm_bf16_group_ok(count, same_x, M, tiles, K)) return CW_ERR_SIZE;
+  int mt, spw, n_tiles;
+  dim3 grid;
+  if (same_x && plan_stream(0, M, (int)tiles * 16, K, 1, &mt, &spw, &grid, &n_tiles) && spw <= 8) {
+#define CW_GROUP(SPW_, MT_)                                                                                                  \
+  if constexpr (cw_stream_fits(16, SPW_, MT_))                                                                               \
+    hipLaunchKernelGGL((gemm_stream_bf16_kernel<0, 16, SPW_, MT_, false, true>), grid, dim3(16 * 64), 0, stream, group.x[0], \
+                       (int64_t)K, (const bf16_t*)nullptr, (void*)nullptr, (int64_t)0, M, 0, K, n_tiles, 0.0f, group)
+#define CW_GROUP_STEPS(SPW_)             \
+  case SPW_:                             \
+    if (mt == 1) { CW_GROUP(SPW_, 1); }  \
+    else if (mt == 2) { CW_GROUP(SPW_, 2); } \
+    else { CW_GROUP(SPW_, 4); }          \
+    break
+    switch (spw) {
+      CW_GROUP_STEPS(1); CW_GROUP_STEPS(2); CW_GROUP_STEPS(3); CW_GROUP_STEPS(4); CW_GROUP_STEPS(5); CW_GROUP_STEPS(6);
+      CW_GROUP_STEPS(7); CW_GROUP_STEPS(8);
+      default: return CW_ERR_SIZE;
+    }
+#undef CW_GROUP_STEPS
+#undef CW_GROUP
+    return cw_launch_status();
+  }
+  // waves a tile as for one product of as many tiles
+  const dim3 blocks((unsigned)tiles);
+  if (tiles <= 256 && K >= 1024) hipLaunchKernelGGL(gemm_skinny_group_bf16_kernel<16>, blocks, dim3(16 * 64), 0, stream, group, M, K);
+  else if (K >= 512) hipLaunchKernelGGL(gemm_skinny_group_bf16_kernel<8>, blocks, dim3(8 * 64), 0, stream, group, M, K);
+  else hipLaunchKernelGGL(gemm_skinny_group_bf16_kernel<4>, blocks, dim3(4 * 64), 0, stream, group, M, K);
+  return cw_launch_status();
 }
 
 // =====================================================================================

@@ -114,6 +114,8 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_gemm_bf16_skinny_fast": [I, I, I, I],
             "cw_gemm_bf16_swiglu_normed_ok": [I, I, I],
             "cw_gemm_bf16_swiglu_normed": [P, P, P, I, F, P, P, L, I, I, I, P],
+            "cw_gemm_bf16_group_ok": [I, I, I, L, I],
+            "cw_gemm_bf16_group": [I, P, P, P, P, I, I, P],
             "cw_gemm_qkv_rope_bf16": [P, L, P, P, I, P, P, P, P, P, P, L, I, I, I, I, I, P],
         },
         "gemm_tile": {
@@ -608,6 +610,31 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias=None, out_dtype=None, par
         _check(_load("core").cw_bf16_to_f32(_ptr(y), _ptr(out), M * N, _stream()), "bf16_to_f32")
         return out
     return y
+
+
+def linear_several(xs, weights):
+    """[x @ w.T for x, w in zip(xs, weights)] as one launch, or None where they are not taken together (by the rule of
+    ``cw_gemm_bf16_group_ok``, csrc/gemm.hip: two to four bfloat16 products of the same few rows and the same K, none with
+    a bias). What ``linear`` gives, but for the order of the float32 sums."""
+    first = xs[0]
+    M, K = first.shape
+    if M > STREAM_MAX_ROWS or first.dtype != torch.bfloat16:
+        return None
+    if not all(tuple(x.shape) == (M, K) and x.dtype == torch.bfloat16 and x.is_contiguous() for x in xs):
+        return None
+    if not all(w.dtype == torch.bfloat16 and w.shape[1] == K and w.is_contiguous() for w in weights):
+        return None
+    lib = _load("gemm")
+    if not (_aligned(*xs, *weights) and lib.cw_gemm_bf16_group_ok(
+            len(weights), int(all(x is first for x in xs)), M, sum(-(-w.shape[0] // 16) for w in weights), K)):
+        return None
+    _gpu(*xs, *weights)
+    out = [torch.empty((M, w.shape[0]), dtype=torch.bfloat16, device=first.device) for w in weights]
+    pointers = ctypes.c_void_p * len(out)
+    _check(lib.cw_gemm_bf16_group(len(out), pointers(*(x.data_ptr() for x in xs)), pointers(*(w.data_ptr() for w in weights)),
+                                  pointers(*(y.data_ptr() for y in out)), (ctypes.c_int * len(out))(*(w.shape[0] for w in weights)),
+                                  M, K, _stream()), "gemm_bf16_group")
+    return out
 
 
 class ProductPolicy:

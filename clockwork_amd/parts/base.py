@@ -26,7 +26,11 @@ Roles and their run methods:
                  ``resid`` is left untouched.
 * mixer:         ``forward(x, ctx, cache) -> y`` with x, y [T, H] in the activation
                  type (y may be an ``ops.PartialSums``: it only ever goes to a norm); ``cache_need()`` returns a KVPagesSpec, a PagedRowsSpec, a StateSpec, a CacheNeeds of several, or None.
-                 ``cache`` is the run entry's :class:`EntryCache`.
+                 ``cache`` is the run entry's :class:`EntryCache`. Optional: ``input_weights()``,
+                 the matrices that x is multiplied with before anything else (no bias); ``forward``
+                 then takes their products as a fourth argument where the block has made them,
+                 in one launch with others of the same x (``ops.linear_several``). And
+                 ``before_output(x, ctx, cache, made=None)``: all but the product with ``out_weight``.
 * feed-forward:  ``forward(x, ctx) -> y``.
 * position enc.: used by a mixer, not by the block; the attention mixer expects
                  ``rotate_and_store(qkv, bias, positions, slots, nh, nkv, hd, k, v)``, and

@@ -81,6 +81,9 @@ class BranchGate:
     def bind(self, params, device, dtype) -> None:
         self.weight, self.bias = params["weight"], params["bias"]
 
+    def input_weights(self) -> list:
+        return [self.weight]
+
     def forward(self, x, ctx):
         """The gates' products [T, branches * hidden] (before bias and sigmoid)."""
         return ops.linear(x, self.weight, policy=getattr(ctx, "products", None))
@@ -115,9 +118,16 @@ class ParallelBlock:
 
     def forward(self, resid, delta, ctx, cache):
         x = self.mixer_norm.forward(resid, delta)
-        a = self.mixer.forward(x, ctx, cache)
+        # the products of x that the mixer begins with and the gates', as one launch where the rows are few
+        first = getattr(self.mixer, "input_weights", list)()
+        weights = first + (self.gate.input_weights() if first and self.gate is not None else [])
+        made = ops.linear_several([x] * len(weights), weights) if len(weights) > 1 else None
+        a = self.mixer.forward(x, ctx, cache) if made is None else self.mixer.forward(x, ctx, cache, made[: len(first)])
         b = self.feed_forward.forward(x, ctx) if self.feed_forward is not None else None
-        z = self.gate.forward(x, ctx) if self.gate is not None else None
+        if made is not None and self.gate is not None:
+            z = made[-1]
+        else:
+            z = self.gate.forward(x, ctx) if self.gate is not None else None
         pending = ops.GatedBranches(z, self.gate.bias if self.gate is not None else None, a, b)
         if getattr(ctx, "next_norm_accepts_gated", False):
             return pending

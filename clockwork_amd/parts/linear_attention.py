@@ -96,20 +96,23 @@ class DecayedLinearAttention(Part):
     def shape_class(self, q_lens, ctx_lens):
         return "segments" if max(q_lens, default=0) > SEGMENT_MIN_TOKENS and self.segments_ok else "token by token"
 
-    def forward(self, x: torch.Tensor, ctx, cache: EntryCache) -> torch.Tensor:
+    def input_weights(self) -> list:
+        return [self.in_weight]
+
+    def forward(self, x: torch.Tensor, ctx, cache: EntryCache, made=None) -> torch.Tensor:
+        return ops.linear(self.before_output(x, ctx, cache, made), self.out_weight, policy=getattr(ctx, "products", None))
+
+    def before_output(self, x: torch.Tensor, ctx, cache: EntryCache, made=None) -> torch.Tensor:
         s = self.spec
-        policy = getattr(ctx, "products", None)
-        proj = ops.linear(x, self.in_weight, policy=policy)
+        proj = made[0] if made is not None else ops.linear(x, self.in_weight, policy=getattr(ctx, "products", None))
         common = (proj, self.q_off, self.k_off, self.v_off, self.g_off, self.u_off, self.decay_weight, self.decay_bias,
                   self.norm_weight, cache.state, ctx.state_slots, ctx.cu_q)
         sizes = (ctx.num_requests, s.num_heads, s.key_dim, s.value_dim, s.key_dim ** -0.5, s.tau, s.norm_eps)
         plan = self._segments(ctx)
         if plan is not None:
             items, n_segments, first = plan
-            out = ops.linear_recurrence_segments(*common, items, n_segments, SEGMENT_TOKENS, first, *sizes)
-        else:
-            out = ops.linear_recurrence(*common, *sizes)
-        return ops.linear(out, self.out_weight, policy=policy)
+            return ops.linear_recurrence_segments(*common, items, n_segments, SEGMENT_TOKENS, first, *sizes)
+        return ops.linear_recurrence(*common, *sizes)
 
 
 class ShiftedRecurrence(Part):

@@ -107,11 +107,25 @@ class PairMixer(Part):
                 out.append(cache.members[members[0]] if len(members) else EntryCache(writes=False))
         return out
 
-    def forward(self, x: torch.Tensor, ctx, cache: EntryCache):
+    def input_weights(self) -> list:
+        """Both mixers', if they are not one matrix already and both state theirs."""
+        own = [getattr(m, "input_weights", list)() for m in (self.left, self.right)]
+        return [] if self.joint or not all(own) else own[0] + own[1]
+
+    def _outputs(self, x, ctx, left, right, made):
+        """The two mixers' outputs; the last product of each as one launch where they are of the same few rows and one K."""
+        mine = len(self.left.input_weights()) if made is not None else 0
+        each = ((self.left, left, made and made[:mine]), (self.right, right, made and made[mine:]))
+        if not all(hasattr(m, "before_output") for m, _, _ in each):
+            return [m.forward(x, ctx, own) if given is None else m.forward(x, ctx, own, given) for m, own, given in each]
+        outs = [m.before_output(x, ctx, own, given) for m, own, given in each]
+        weights = [m.out_weight for m, _, _ in each]
+        return ops.linear_several(outs, weights) or [ops.linear(o, w, policy=getattr(ctx, "products", None)) for o, w in zip(outs, weights)]
+
+    def forward(self, x: torch.Tensor, ctx, cache: EntryCache, made=None):
         left, right = self._caches(cache)
         if not self.joint:
-            return ops.rms_mean2(self.left.forward(x, ctx, left), self.right.forward(x, ctx, right), self.left_norm, self.right_norm,
-                                 self.spec.eps)
+            return ops.rms_mean2(*self._outputs(x, ctx, left, right, made), self.left_norm, self.right_norm, self.spec.eps)
         policy = getattr(ctx, "products", None)
         proj = ops.linear(x, self.in_weight, policy=policy)
         T, (l, r) = x.shape[0], self.spec.scales

@@ -138,13 +138,18 @@ class SinkAttention(Part):
     def shape_class(self, q_lens, ctx_lens):
         return "single tokens" if all(q == 1 for q in q_lens) else "portions"
 
-    def forward(self, x: torch.Tensor, ctx, cache: EntryCache) -> torch.Tensor:
+    def input_weights(self) -> list:
+        return [self.qkv_weight]
+
+    def forward(self, x: torch.Tensor, ctx, cache: EntryCache, made=None) -> torch.Tensor:
+        return ops.linear(self.before_output(x, ctx, cache, made), self.out_weight, policy=getattr(ctx, "products", None))
+
+    def before_output(self, x: torch.Tensor, ctx, cache: EntryCache, made=None) -> torch.Tensor:
         s = self.spec
-        policy = getattr(ctx, "products", None)
         if not cache.writes:
             raise NotImplementedError("this mixer writes its own keys and values: it cannot borrow another entry's cache")
         k_plane, v_plane = cache.planes["k"], cache.planes["v"]
-        qkv = ops.linear(x, self.qkv_weight, policy=policy)
+        qkv = made[0] if made is not None else ops.linear(x, self.qkv_weight, policy=getattr(ctx, "products", None))
         ops.qk_rownorm_store(qkv, 0, self.q_width, self.q_width + self.k_width, self.q_width, self.k_width, self.v_width,
                              self.q_norm, self.k_norm, s.qk_norm_eps, ctx.slots[cache.group], k_plane, v_plane)
         out = torch.empty((x.shape[0], s.num_heads * s.value_dim), dtype=x.dtype, device=x.device)
@@ -160,4 +165,4 @@ class SinkAttention(Part):
         if n_runs:
             ops.sink_attention_decode(qkv, qkv.shape[1], out, k_plane, v_plane, ctx.block_tables[cache.group], ctx.ctx_lens,
                                       ctx.cu_q, ctx.num_requests, run_keys, n_runs, *options)
-        return ops.linear(out, self.out_weight, policy=policy)
+        return out

@@ -757,3 +757,29 @@ def test_gate_up_products_with_gelu(M, K, I, dtype):
     off_g, off_u = half * g + 2.0 ** -19, half * u + 2.0 ** -19
     bound = 1.13 * (off_g * (u + off_u) + g * off_u) + (half + 2.0 ** -20) * want.abs()
     assert bool(((got - want).abs() <= bound).all())
+
+
+# both kernels of several products (tiles of their own with 4, 8 and 16 waves, and streamed), outputs that end inside a tile, the ends of
+# the rows that each takes; the last has more steps than the streaming kernel of several products is built for
+@pytest.mark.parametrize("K,widths", [(8, (1, 17)), (520, (16, 33, 1, 100)), (1032, (3000, 1000)), (1536, (2048, 4640, 3072)), (1536, (1536, 1535, 5120)),
+                                      (4096, (8000, 300)), (4360, (8000, 300))])
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
+@pytest.mark.parametrize("same", [True, False])
+def test_several_products_in_one_launch(M, K, widths, same):
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(M + K)
+    xs = [torch.randn(M, K, device=DEV, generator=gen).bfloat16()] * len(widths)
+    if not same:
+        xs = [(x * (i + 1)).contiguous() for i, x in enumerate(xs)]
+    ws = [(torch.randn(n, K, device=DEV, generator=gen) * K ** -0.5).bfloat16() for n in widths]
+    got = ops.linear_several(xs, ws)
+    tiles = sum(-(-n // 16) for n in widths)
+    if got is None:
+        assert M > 16 and (not same or tiles < 256 or K < 1024 or K >= 4096)
+        return
+    assert M <= 16 or same
+    for x, w, y in zip(xs, ws, got):
+        want = x.double() @ w.double().t()
+        # K terms that come to a unit, in float32 (2^-24 each step of sums of some 60 at most), then one rounding
+        assert bool(((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -17 * float(x.abs().max())).all())

@@ -161,3 +161,22 @@ def test_parts_over_k_do_not_come_to_more_workgroups_than_units(N, K, parts):
     tiles = -(-N // 16)
     assert -(-tiles // -(-tiles * parts // CUS)) * parts <= CUS
     assert all(ops._load("gemm").cw_gemm_bf16_skinny_ksplits(M, N, K) == parts for M in (1, 8, 16))
+
+
+def test_several_products_of_few_rows():
+    """Which are taken together, and that operands of other kinds are not."""
+    import torch
+
+    from clockwork_amd import ops
+
+    ok = ops._load("gemm").cw_gemm_bf16_group_ok
+    for M in (1, 16):
+        assert ok(2, 0, M, 2, 8) and ok(4, 1, M, 5000, 1536)
+    # beyond 16 rows: one x, and tiles and a K that the streaming kernel takes
+    assert ok(3, 1, 64, 610, 1536) and not ok(3, 0, 64, 610, 1536) and not ok(3, 1, 64, 200, 1536) and not ok(3, 1, 17, 610, 512)
+    # one product, five, no rows, more rows, columns that are not whole 16 bytes
+    assert not (ok(1, 1, 8, 96, 1536) or ok(5, 1, 8, 480, 1536) or ok(2, 1, 0, 96, 1536) or ok(2, 1, 65, 610, 1536) or ok(2, 1, 8, 96, 1532))
+    x, w = torch.zeros(4, 64, dtype=torch.bfloat16), torch.zeros(32, 64, dtype=torch.bfloat16)
+    for xs, ws in (([x, x], [w, w.float()]), ([x.float(), x.float()], [w, w]), ([x, x[:2]], [w, w]), ([x, x], [w, w[:, :32]]),
+                   ([x, x], [w, w.t().contiguous().t()]), ([x[:, :32], x[:, :32]], [w[:, :32].contiguous()] * 2), ([x], [w])):
+        assert ops.linear_several(xs, ws) is None
