@@ -149,12 +149,28 @@ __global__ __launch_bounds__(512) void gemm_f32_rows_kernel(const float* __restr
 // and of the parts that they make, of 256 k-values at least, where those meet in LDS as well
 #define GT_BLOCKS_LDS ((GT_BLOCKS + GT_BLOCKS / 16) * 1024)
 // GLU: W = [gate; up], a tile is 8 gate rows and the 8 up rows that belong to them, C the gated product [M, N / 2].
-template <bool GLU>
+// PAIRS: W = [queries; keys; values] of ``to``, a tile of a query or key head is 8 rows of its first half and the 8 of its second
+// that they are rotated with; C the rotated queries, keys and values go to their cache rows. The
+// rotation as a kernel of its own is a launch that moves a few KB: 3.7 us of a layer's decode step of the 0.5B shape.
+#define GT_PLAIN 0
+#define GT_GLU 1
+#define GT_PAIRS 2
+struct F32PairsOut {
+  const int* positions;
+  const int* slots;
+  const float* inv_freq;
+  float* k_cache;
+  float* v_cache;
+  int64_t cache_rows;
+  int nh, nkv, hd;
+};
+template <int KIND>
 __global__ __launch_bounds__(GT_BLOCK_WAVES * 64) void gemm_f32_blocks_kernel(const float* __restrict__ A, int64_t lda,
                                                                               const float* __restrict__ W,
                                                                               const float* __restrict__ bias, float* __restrict__ C,
                                                                               int64_t ldc, int M, int N, int K, int parts, int part_blocks,
-                                                                              int parts_here, int64_t plane_stride, float act) {
+                                                                              int parts_here, int64_t plane_stride, float act, F32PairsOut to) {
+  constexpr bool GLU = KIND == GT_GLU, PAIRS = KIND == GT_PAIRS;
   extern __shared__ __align__(16) float red[];
   constexpr int U = 8;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -163,7 +179,29 @@ __global__ __launch_bounds__(GT_BLOCK_WAVES * 64) void gemm_f32_blocks_kernel(co
   const int z0 = blockIdx.y * parts_here, z1 = min(parts, z0 + parts_here);
   const int b0 = z0 * part_blocks, b1 = min(K / 16, z1 * part_blocks);
   const int tile_row = lane >> 2;
-  const int row = GLU ? min(n0 + (tile_row & 7), cols - 1) + (tile_row >> 3) * cols : min(n0 + tile_row, N - 1);
+  int row = GLU ? min(n0 + (tile_row & 7), cols - 1) + (tile_row >> 3) * cols : min(n0 + tile_row, N - 1);
+  // what a thread's output takes besides its sum is asked for beside the weights
+  int head = 0, first = 0, pos = 0;
+  int64_t slot = -1;
+  float inv = 0.0f, bias_a = 0.0f, bias_b = 0.0f;
+  bool rotated = false;
+  if constexpr (PAIRS) {
+    head = n0 / to.hd;
+    rotated = head < to.nh + to.nkv;
+    const int half = to.hd / 2;
+    first = rotated ? (n0 - head * to.hd) / 2 : n0 - head * to.hd;
+    if (rotated) row = head * to.hd + first + (tile_row & 7) + (tile_row >> 3) * half;
+    const int at = threadIdx.x, m = rotated ? at >> 3 : at >> 4, d = first + (at & (rotated ? 7 : 15));
+    if (m < M) {
+      slot = to.slots[m];
+      if (bias) bias_a = bias[head * to.hd + d];
+      if (rotated) {
+        pos = to.positions[m];
+        inv = to.inv_freq[d];
+        if (bias) bias_b = bias[head * to.hd + d + half];
+      }
+    }
+  }
   const float* const w = W + (int64_t)row * K + 4 * (lane & 3);
   const float* const x = A + (int64_t)min(r, M - 1) * lda + 4 * s;
   for (int b = b0 + wave; b < b1; b += U * GT_BLOCK_WAVES) {
@@ -195,13 +233,13 @@ __global__ __launch_bounds__(GT_BLOCK_WAVES * 64) void gemm_f32_blocks_kernel(co
     const int n = n0 + (at & 15);
     if (plane_stride > 0) {
       if (n < N) C[(z0 + z) * plane_stride + (int64_t)(at >> 4) * ldc + n] = total;
-    } else if (parts == 1 && !GLU) {
+    } else if (parts == 1 && KIND == GT_PLAIN) {
       if (n < N) C[(int64_t)(at >> 4) * ldc + n] = total + (bias ? bias[n] : 0.0f);
     } else {
       sums[i] = total;
     }
   }
-  if (plane_stride > 0 || (parts == 1 && !GLU)) return;
+  if (plane_stride > 0 || (parts == 1 && KIND == GT_PLAIN)) return;
   cw_lds_barrier();
   if constexpr (GLU) {
     for (int i = threadIdx.x; i < M * 8; i += GT_BLOCK_WAVES * 64) {
@@ -212,6 +250,29 @@ __global__ __launch_bounds__(GT_BLOCK_WAVES * 64) void gemm_f32_blocks_kernel(co
         up += sums[z * outputs + at + 8];
       }
       if (n < cols) C[(int64_t)(i >> 3) * ldc + n] = cw_gated(gate, up, act);
+    }
+    return;
+  }
+  if constexpr (PAIRS) {
+    const int at = threadIdx.x, m = rotated ? at >> 3 : at >> 4, d = first + (at & (rotated ? 7 : 15)), half = to.hd / 2;
+    if (m >= M) return;  // up to 16 rows: an output or a pair of them a thread
+    auto summed = [&](int column) __attribute__((always_inline)) {
+      float total = sums[m * 16 + column];
+      for (int z = 1; z < parts; ++z) total += sums[z * outputs + m * 16 + column];
+      return total;
+    };
+    const bool kept = slot >= 0 && slot < to.cache_rows;
+    if (!rotated) {
+      if (kept) to.v_cache[(slot * to.nkv + (head - to.nh - to.nkv)) * to.hd + d] = summed(at & 15) + bias_a;
+      return;
+    }
+    const float a = summed(at & 7) + bias_a, b = summed((at & 7) + 8) + bias_b;
+    float sn, cs;
+    sincosf((float)pos * inv, &sn, &cs);
+    float* const out = head < to.nh ? C + (int64_t)m * ldc + head * to.hd : to.k_cache + (slot * to.nkv + (head - to.nh)) * to.hd;
+    if (head < to.nh || kept) {
+      out[d] = a * cs - b * sn;
+      out[d + half] = b * cs + a * sn;
     }
     return;
   }
@@ -569,9 +630,9 @@ static int launch_gemm_f32(const float* A, int64_t lda, const float* W, const fl
       const size_t lds = (size_t)(blocks + (planes || splits == 1 ? 0 : splits)) * M * 16 * sizeof(float);
       const dim3 grid(tiles, (splits + here - 1) / here);
       static std::atomic<bool> allowed{false};
-      if (cw_allow_lds(allowed, (const void*)gemm_f32_blocks_kernel<false>, GT_BLOCKS_LDS) != CW_OK) return CW_ERR_LAUNCH;
-      hipLaunchKernelGGL(gemm_f32_blocks_kernel<false>, grid, dim3(GT_BLOCK_WAVES * 64), lds, stream, A, lda, W, bias, C, ldc, M, N, K,
-                         splits, part_blocks, here, stride, 0.0f);
+      if (cw_allow_lds(allowed, (const void*)gemm_f32_blocks_kernel<GT_PLAIN>, GT_BLOCKS_LDS) != CW_OK) return CW_ERR_LAUNCH;
+      hipLaunchKernelGGL(gemm_f32_blocks_kernel<GT_PLAIN>, grid, dim3(GT_BLOCK_WAVES * 64), lds, stream, A, lda, W, bias, C, ldc, M, N, K,
+                         splits, part_blocks, here, stride, 0.0f, F32PairsOut{});
       return cw_launch_status();
     }
   }
@@ -651,9 +712,37 @@ CW_EXPORT int cw_gemm_f32_swiglu(const float* A, int64_t lda, const float* W, fl
   gemm_f32_plan(N, K, &splits, &per);
   const size_t lds = (size_t)(K / 16 + splits) * M * 16 * sizeof(float);
   static std::atomic<bool> allowed{false};
-  if (cw_allow_lds(allowed, (const void*)gemm_f32_blocks_kernel<true>, GT_BLOCKS_LDS) != CW_OK) return CW_ERR_LAUNCH;
-  hipLaunchKernelGGL(gemm_f32_blocks_kernel<true>, dim3((N / 2 + 7) / 8), dim3(GT_BLOCK_WAVES * 64), lds, stream, A, lda, W, nullptr, C, ldc,
-                     M, N, K, splits, per / 16, splits, 0, act);
+  if (cw_allow_lds(allowed, (const void*)gemm_f32_blocks_kernel<GT_GLU>, GT_BLOCKS_LDS) != CW_OK) return CW_ERR_LAUNCH;
+  hipLaunchKernelGGL(gemm_f32_blocks_kernel<GT_GLU>, dim3((N / 2 + 7) / 8), dim3(GT_BLOCK_WAVES * 64), lds, stream, A, lda, W, nullptr, C, ldc,
+                     M, N, K, splits, per / 16, splits, 0, act, F32PairsOut{});
+  return cw_launch_status();
+}
+
+// Does cw_gemm_f32_pairs take queries, keys and values of these heads (rotated whole) of few rows, whole blocks of K?
+CW_EXPORT int cw_gemm_f32_pairs_ok(int M, int K, int nh, int nkv, int hd) {
+  return nh > 0 && nkv > 0 && hd > 0 && !(hd & 15) && hd <= 1024 && nh + 2 * nkv <= 65536 / hd && M > 0 && M <= GT_ROWS_MAX && K > 0 && !(K & 15) &&
+                 K / 16 <= GT_BLOCKS
+             ? 1
+             : 0;
+}
+
+// A [M, K] W^T + bias for W [(nh + 2 nkv) hd, K]: rotated queries to Q [M, nh hd], rotated keys and the values to rows ``slots`` of
+// the caches (negative, or past cache_rows: none). What cw_gemm_f32 and cw_rope_kv_write give, in one kernel; bias or nullptr.
+CW_EXPORT int cw_gemm_f32_pairs(const float* A, const float* W, const float* bias, const int* positions, const int* slots,
+                                const float* inv_freq, float* Q, float* k_cache, float* v_cache, int64_t cache_rows, int M, int K,
+                                int nh, int nkv, int hd, hipStream_t stream) {
+  if (M == 0) return CW_OK;
+  if (!cw_gemm_f32_pairs_ok(M, K, nh, nkv, hd)) return CW_ERR_SIZE;
+  if (!A || !W || !positions || !slots || !inv_freq || !Q || !k_cache || !v_cache || ((uintptr_t)A & 15) || ((uintptr_t)W & 15)) return CW_ERR_ARG;
+  const int N = (nh + 2 * nkv) * hd;
+  int splits, per;
+  gemm_f32_plan(N, K, &splits, &per);
+  const size_t lds = (size_t)(K / 16 + splits) * M * 16 * sizeof(float);
+  static std::atomic<bool> allowed{false};
+  if (cw_allow_lds(allowed, (const void*)gemm_f32_blocks_kernel<GT_PAIRS>, GT_BLOCKS_LDS) != CW_OK) return CW_ERR_LAUNCH;
+  hipLaunchKernelGGL(gemm_f32_blocks_kernel<GT_PAIRS>, dim3(N / 16), dim3(GT_BLOCK_WAVES * 64), lds, stream, A, (int64_t)K, W, bias, Q,
+                     (int64_t)nh * hd, M, N, K, splits, per / 16, splits, 0, 0.0f,
+                     F32PairsOut{positions, slots, inv_freq, k_cache, v_cache, cache_rows, nh, nkv, hd});
   return cw_launch_status();
 }
 

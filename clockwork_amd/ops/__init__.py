@@ -109,6 +109,8 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_gemm_f32_partial": [P, L, P, P, I, I, I, P],
             "cw_gemm_f32_swiglu_ok": [I, I, I, L],
             "cw_gemm_f32_swiglu": [P, L, P, P, L, I, I, I, F, P],
+            "cw_gemm_f32_pairs_ok": [I, I, I, I, I],
+            "cw_gemm_f32_pairs": [P, P, P, P, P, P, P, P, P, L, I, I, I, I, I, P],
             "cw_gemm_bf16_skinny": [I, P, L, P, P, L, I, I, I, I, F, P],
             "cw_gemm_bf16_skinny_ksplits": [I, I, I],
             "cw_gemm_bf16_skinny_fast": [I, I, I, I],
@@ -1146,22 +1148,26 @@ def _measure_swiglu(x: torch.Tensor, gate_up_weight: torch.Tensor, out: torch.Te
     return own <= library
 
 
-def qkv_rope_fused_supported(x: torch.Tensor, weight: torch.Tensor, rotary_dim: int, hd: int) -> bool:
-    """The fused q/k/v product + rotary + cache write takes few bfloat16 rows and a full rotary
-    dimension. Beyond 16 rows it serves small weight matrices only: a large one is faster as a
-    product and a rotation kernel (measured: 33 MB at 24 rows and more)."""
-    rows = x.shape[0]
+def qkv_rope_fused_supported(x: torch.Tensor, weight: torch.Tensor, rotary_dim: int, hd: int, nh: int = 0, nkv: int = 0) -> bool:
+    """The fused q/k/v product + rotary + cache write takes few rows and a full rotary dimension: bfloat16, beyond 16 rows with small
+    weight matrices only (a large one is faster as a product and a rotation kernel, measured: 33 MB at 24 rows and more); or
+    float32, by the rule of ``cw_gemm_f32_pairs_ok`` (csrc/gemm.hip), which asks for the number of heads."""
+    rows, K = x.shape
+    if x.dtype == torch.float32 and weight.dtype == torch.float32:
+        return (rotary_dim == hd and x.is_contiguous() and weight.is_contiguous() and _aligned(x, weight)
+                and bool(_load("gemm").cw_gemm_f32_pairs_ok(rows, K, nh, nkv, hd)))
     return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
             and (rows <= SKINNY_MAX_ROWS or (rows <= STREAM_MAX_ROWS and weight.numel() <= FUSED_QKV_MAX_WEIGHTS))
-            and x.shape[1] % 8 == 0 and rotary_dim == hd and hd % 16 == 0)
+            and K % 8 == 0 and rotary_dim == hd and hd % 16 == 0)
 
 
 def qkv_rope_fused(x, weight, bias, positions, slots, inv_freq, nh: int, nkv: int, hd: int, k_cache, v_cache) -> torch.Tensor:
     """q = rope(x @ Wq.T + bq) returned as [M, nh * hd]; rope(x @ Wk.T + bk) and x @ Wv.T + bv written
-    to the cache rows ``slots``: one kernel for few bfloat16 rows (see csrc/gemm.hip)."""
+    to the cache rows ``slots``: one kernel for few rows, all operands of one type (a bias of bfloat16 rows may be float32; see
+    csrc/gemm.hip)."""
     _gpu(x, weight, bias, positions, slots, inv_freq, k_cache, v_cache)
     M, K = x.shape
-    if not (qkv_rope_fused_supported(x, weight, hd, hd)):
+    if not (qkv_rope_fused_supported(x, weight, hd, hd, nh, nkv)):
         raise KernelError("the fused q/k/v kernel does not take these operands")
     if not (tuple(weight.shape) == ((nh + 2 * nkv) * hd, K)):
         raise KernelError("qkv weight must be [(nh + 2 nkv) hd, K]")
@@ -1169,16 +1175,21 @@ def qkv_rope_fused(x, weight, bias, positions, slots, inv_freq, nh: int, nkv: in
     _i32(slots, M, "slots")
     if not (inv_freq.dtype == torch.float32 and inv_freq.numel() == hd // 2):
         raise KernelError("inv_freq must be float32 [hd / 2]")
-    _need(k_cache.dtype == torch.bfloat16 and tuple(k_cache.shape[-2:]) == (nkv, hd) and k_cache.shape == v_cache.shape,
-          "cache must be bfloat16 [..., nkv, hd]")
+    _need(k_cache.dtype == x.dtype and v_cache.dtype == x.dtype and tuple(k_cache.shape[-2:]) == (nkv, hd) and k_cache.shape == v_cache.shape,
+          "cache must be of the activation type, [..., nkv, hd]")
     if bias is not None:
-        if not (bias.numel() == weight.shape[0] and bias.dtype in (torch.bfloat16, torch.float32)):
+        if not (bias.numel() == weight.shape[0] and bias.dtype in (x.dtype, torch.float32)):
             raise KernelError("qkv bias")
-    q = torch.empty((M, nh * hd), dtype=torch.bfloat16, device=x.device)
+    q = torch.empty((M, nh * hd), dtype=x.dtype, device=x.device)
+    rows = k_cache.numel() // (nkv * hd)
+    if x.dtype == torch.float32:
+        _check(_load("gemm").cw_gemm_f32_pairs(_ptr(x), _ptr(weight), _ptr(bias), _ptr(positions), _ptr(slots), _ptr(inv_freq), _ptr(q),
+                                               _ptr(k_cache), _ptr(v_cache), rows, M, K, nh, nkv, hd, _stream()), "gemm_f32_pairs")
+        return q
     _check(
         _load("gemm").cw_gemm_qkv_rope_bf16(
             _ptr(x), K, _ptr(weight), _ptr(bias), int(bias is not None and bias.dtype == torch.float32), _ptr(positions),
-            _ptr(slots), _ptr(inv_freq), _ptr(q), _ptr(k_cache), _ptr(v_cache), k_cache.numel() // (nkv * hd),
+            _ptr(slots), _ptr(inv_freq), _ptr(q), _ptr(k_cache), _ptr(v_cache), rows,
             M, K, nh, nkv, hd, _stream()),
         "gemm_qkv_rope_bf16",
     )

@@ -58,7 +58,7 @@ class RopeNeox(Part):
         """Optional fast path of the attention mixer: the q/k/v product, this encoding and the cache
         write as one kernel. Returns q [T, nh * hd], or None when the shapes do not allow it (the
         mixer then runs the product and ``rotate_and_store`` apart)."""
-        if slots is None or not ops.qkv_rope_fused_supported(x, weight, self.spec.rotary_dim, hd):
+        if slots is None or not ops.qkv_rope_fused_supported(x, weight, self.spec.rotary_dim, hd, nh, nkv):
             return None
         return ops.qkv_rope_fused(x, weight, bias, positions, slots, self.inv_freq, nh, nkv, hd, k_cache, v_cache)
 

@@ -783,3 +783,32 @@ def test_several_products_in_one_launch(M, K, widths, same):
         want = x.double() @ w.double().t()
         # K terms that come to a unit, in float32 (2^-24 each step of sums of some 60 at most), then one rounding
         assert bool(((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -17 * float(x.abs().max())).all())
+
+
+# one part of K and several, a K of the most blocks, heads of one tile and of many, a step of one row and of the most
+@pytest.mark.parametrize("M", [1, 7, 16])
+@pytest.mark.parametrize("nh,nkv,hd,K", [(14, 2, 64, 896), (1, 1, 16, 16), (3, 1, 48, 560), (12, 2, 128, 1536), (2, 2, 32, 1920)])
+@pytest.mark.parametrize("with_bias", [True, False])
+def test_float32_queries_keys_and_values_rotated_by_their_product(M, nh, nkv, hd, K, with_bias):
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(M + K)
+    N, rows = (nh + 2 * nkv) * hd, 40
+    x, w = torch.randn(M, K, device=DEV, generator=gen), torch.randn(N, K, device=DEV, generator=gen) * K ** -0.5
+    b = torch.randn(N, device=DEV, generator=gen) if with_bias else None
+    slots = torch.randperm(rows, device=DEV, generator=gen)[:M].int()
+    if M > 3:
+        slots[1], slots[2] = -1, rows   # no row, and one past the cache
+    positions = torch.randint(0, 30000, (M,), device=DEV, generator=gen, dtype=torch.int32)
+    for freq in (torch.zeros(hd // 2, device=DEV), 1.0 / 10000.0 ** (torch.arange(0, hd, 2, device=DEV) / hd)):
+        caches = [torch.full((rows, nkv, hd), 7.0, device=DEV) for _ in range(4)]
+        assert ops.qkv_rope_fused_supported(x, w, hd, hd, nh, nkv)
+        q = ops.qkv_rope_fused(x, w, b, positions, slots, freq, nh, nkv, hd, caches[0], caches[1])
+        apart = ops.linear(x, w)
+        ops.rope_kv_write(apart, b, positions, slots, freq, hd, nh, nkv, hd, caches[2], caches[3])
+        for got, want in ((q, apart[:, : nh * hd]), (caches[0], caches[2]), (caches[1], caches[3])):
+            if not bool(freq.any()):
+                assert torch.equal(got, want)   # turned by nothing: the same sums
+            # two products and a sum of values of up to 6 units, contracted or not: a unit in the last place of each
+            assert bool(((got - want).abs() <= 3 * 6 * 2.0 ** -24).all())
+    assert not ops.qkv_rope_fused_supported(x, w, hd - 2, hd, nh, nkv) and not ops.qkv_rope_fused_supported(x[:, : K - 8], w[:, : K - 8], hd, hd, nh, nkv)

@@ -180,3 +180,13 @@ def test_several_products_of_few_rows():
     for xs, ws in (([x, x], [w, w.float()]), ([x.float(), x.float()], [w, w]), ([x, x[:2]], [w, w]), ([x, x], [w, w[:, :32]]),
                    ([x, x], [w, w.t().contiguous().t()]), ([x[:, :32], x[:, :32]], [w[:, :32].contiguous()] * 2), ([x], [w])):
         assert ops.linear_several(xs, ws) is None
+
+
+def test_float32_queries_keys_and_values_of_few_rows():
+    from clockwork_amd import ops
+
+    ok = ops._load("gemm").cw_gemm_f32_pairs_ok
+    assert ok(1, 896, 14, 2, 64) and ok(16, 1920, 2, 2, 32)
+    # rows, blocks of K, whole blocks, whole tiles of a head, heads
+    assert not (ok(0, 896, 14, 2, 64) or ok(17, 896, 14, 2, 64) or ok(1, 1936, 14, 2, 64) or ok(1, 888, 14, 2, 64) or ok(1, 896, 14, 2, 24)
+                or ok(1, 896, 0, 2, 64) or ok(1, 896, 2, 0, 64) or ok(1, 896, 1000, 20, 64))
