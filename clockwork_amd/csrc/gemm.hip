@@ -284,17 +284,17 @@ __global__ __launch_bounds__(GT_BLOCK_WAVES * 64) void gemm_f32_blocks_kernel(co
   }
 }
 
-// A wave's sums to C, 2 x TM tiles from row m0 of x and row n0 of W: lane (r, s) holds rows 4 s .. 4 s + 3 of
+// A wave's sums to C, TN x TM tiles from row m0 of x and row n0 of W: lane (r, s) holds rows 4 s .. 4 s + 3 of
 // W for token r of each.
-template <int TM>
-__device__ __forceinline__ void gemm_f32_store_tile(const f32x4_t (&total)[2][TM], float* __restrict__ C,
+template <int TN, int TM>
+__device__ __forceinline__ void gemm_f32_store_tile(const f32x4_t (&total)[TN][TM], float* __restrict__ C,
                                                     const float* __restrict__ bias, int plane, int64_t plane_stride,
                                                     int64_t ldc, int m0, int n0, int M, int N, int r, int s) {
   const bool planes = plane_stride > 0;
   float* out = C + (int64_t)plane * plane_stride;
   const bool vec_store = !(ldc & 3) && !((uintptr_t)out & 15);
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < TN; ++i)
 #pragma unroll
     for (int j = 0; j < TM; ++j) {
       const int m = m0 + 16 * j + r, n = n0 + 16 * i + 4 * s;
@@ -409,7 +409,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
     k_end = next_end;
   }
 
-  gemm_f32_store_tile<TM>(total, C, bias, blockIdx.z, plane_stride, ldc, m0 + wm, n0 + wn, M, N, r, s);
+  gemm_f32_store_tile(total, C, bias, blockIdx.z, plane_stride, ldc, m0 + wm, n0 + wn, M, N, r, s);
 }
 
 // The same product, rows of whole blocks of 16 k-values: tiles of BM rows of x by 64 rows of W, K in stages of
@@ -420,8 +420,13 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
 // granules of row R change places by (R >> 1) & 7, so that the 16 lanes that read one granule of 16 rows touch
 // every bank once. The descriptors end with the matrices: rows past the end read as zeros. What a stage holds past
 // the end of its part is not multiplied. BM is 32 where 64 would leave compute units without a tile.
-// Measured on an MI355X, the four products of a layer of the 0.5B shape with 384 rows: 919 us on 64 x 64 tiles of
-// the vector units, 163 us here (q/k/v 17, output 17, gate/up 83 at 81 TFLOP/s, down 46).
+// The operands of a block are read from LDS beside the products of the block before it, across the stages' barriers, and the
+// loop's two blocks have sums of their own: read at the head of a stage, and with the sums moved to other registers, the matrix cores
+// waited for a tenth of the time. The matrix cores bound it now where there are tiles enough: 124 TFLOP/s for 2048 rows of 4096 x
+// 4096 (114 before), and tiles of 128 x 128, which load half as much, reach the same. Measured on an MI355X, us, before and now:
+// 336 rows of 9728 x 896 78 and 68, 896 x 4864 45 and 40, 1152 x 896 16.4 and 16.1 (108 tiles); 1000 rows of 17920 x 1536 555 and
+// 497; 40 rows of 1536 x 8960 25.5 and 23.0. (The four products of a layer of the 0.5B shape with 384 rows, 919 us on 64 x 64
+// tiles of the vector units.)
 typedef __attribute__((address_space(3))) void lds_void_t;
 // s_waitcnt for "at most n vector-memory operations in flight" and nothing else
 #define GF_WAIT_LOADS(n) __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | (((n) >> 4) << 14))
@@ -439,7 +444,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_ring_kernel(const float* __re
                                                             const float* __restrict__ bias,
                                                             float* __restrict__ C, int64_t ldc, int M, int N, int K,
                                                             int parts, int k_per_part, int64_t plane_stride) {
-  constexpr int BN = 64, BK = 32, SLOTS = 4, TM = BM / 32;
+  constexpr int BN = 64, BK = 32, SLOTS = 4, TM = BM / 32, TN = 2;
   constexpr int XB = BM / 8, WB = BN / 8, LOADS = (XB + WB) / 4;  // 1 KB blocks of a stage; loads of a wave
   constexpr int STAGE = (XB + WB) * 1024;
   extern __shared__ __align__(1024) unsigned char ring[];  // SLOTS * STAGE bytes
@@ -486,62 +491,80 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_ring_kernel(const float* __re
     if (fk + BK < end) fk += BK;
     else if (fz < z_last) fk = ++fz * k_per_part;
   };
-  f32x4_t acc[2][TM], total[2][TM], t[2][TM];  // t: the sum of the last block, not added to acc yet
+  // even, odd: the sums of the last block of 16 with an even and with an odd number in its stage. A block's sums join
+  // the part's beside the products of the next one: added at once they would wait for the last product, with the matrix
+  // core idle, and so they did when they were moved to other registers first.
+  f32x4_t acc[TN][TM], total[TN][TM], even[TN][TM], odd[TN][TM];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < TN; ++i)
 #pragma unroll
-    for (int j = 0; j < TM; ++j) acc[i][j] = total[i][j] = t[i][j] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int i = 0; i < SLOTS - 1; ++i) fetch_next(i);
+    for (int j = 0; j < TM; ++j) acc[i][j] = total[i][j] = odd[i][j] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
   const unsigned char* mine = ring + r * 128;
   const int turn = (r >> 1) & 7;
+  auto read = [&](f32x4_t (&wf)[TN], f32x4_t (&xf)[TM], int slot, int b) __attribute__((always_inline)) {
+    const unsigned char* from = mine + slot * STAGE + ((b * 4 + s) ^ turn) * 16;
+#pragma unroll
+    for (int i = 0; i < TN; ++i) wf[i] = *reinterpret_cast<const f32x4_t*>(from + XB * 1024 + wn * 128 + i * 2048);
+#pragma unroll
+    for (int j = 0; j < TM; ++j) xf[j] = *reinterpret_cast<const f32x4_t*>(from + wm * 128 + j * 2048);
+  };
+  // gemm_f32_block for each pair, the pairs' products taking turns, and the sums of the block before to the part's
+  auto multiply = [&](const f32x4_t (&wf)[TN], const f32x4_t (&xf)[TM], f32x4_t (&sums)[TN][TM], const f32x4_t (&before)[TN][TM])
+      __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j)
+          sums[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][q], xf[j][q], q == 0 ? (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f} : sums[i][j], 0, 0, 0);
+      if (q == 1) {
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+          for (int j = 0; j < TM; ++j) acc[i][j] += before[i][j];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < SLOTS - 1; ++i) fetch_next(i);
+  GF_WAIT_LOADS((SLOTS - 2) * LOADS);
+  GF_BARRIER();
+  f32x4_t w0[TN], x0[TM], w1[TN], x1[TM];
+  read(w0, x0, 0, 0);
   for (int z = z_first, slot = 0; z <= z_last; ++z) {
     const int k_end = min(K, (z + 1) * k_per_part);
-    for (int k0 = z * k_per_part; k0 < k_end; k0 += BK, slot = (slot + 1) % SLOTS) {
-      // this wave's loads of the stage are in; behind the barrier every wave's are, and every wave has read the
-      // stage before it, whose slot the next loads take
-      GF_WAIT_LOADS((SLOTS - 2) * LOADS);
+    for (int k0 = z * k_per_part; k0 < k_end; k0 += BK) {
+      read(w1, x1, slot, 1);
+      multiply(w0, x0, even, odd);
+      // this wave's loads of the next stage are in; behind the barrier every wave's are, and every wave has read all
+      // of the stage before this one, whose slot the next loads take
+      GF_WAIT_LOADS((SLOTS - 3) * LOADS);
       GF_BARRIER();
       fetch_next((slot + SLOTS - 1) % SLOTS);
-      const unsigned char* xs = mine + slot * STAGE + wm * 128;
-      const unsigned char* ws = mine + slot * STAGE + XB * 1024 + wn * 128;
+      slot = (slot + 1) % SLOTS;
+      read(w0, x0, slot, 0);
+      if (k0 + 16 < k_end) {
+        multiply(w1, x1, odd, even);
+      } else {  // a part is a whole number of blocks, not of stages
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        if (b == 1 && k0 + 16 >= k_end) break;  // a part is a whole number of blocks, not of stages
-        f32x4_t wf[2], xf[TM], next[2][TM];
+        for (int i = 0; i < TN; ++i)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) wf[i] = *reinterpret_cast<const f32x4_t*>(ws + i * 2048 + ((b * 4 + s) ^ turn) * 16);
-#pragma unroll
-        for (int j = 0; j < TM; ++j) xf[j] = *reinterpret_cast<const f32x4_t*>(xs + j * 2048 + ((b * 4 + s) ^ turn) * 16);
-        // gemm_f32_block for each pair, the pairs' products taking turns; the sums of the block before join the
-        // totals meanwhile (added at once they would wait for the last product, with the matrix core idle)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < TM; ++j)
-              next[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][q], xf[j][q], q == 0 ? (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f} : next[i][j], 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < TM; ++j) {
-            acc[i][j] += t[i][j];
-            t[i][j] = next[i][j];
-          }
+          for (int j = 0; j < TM; ++j) odd[i][j] = even[i][j];
       }
     }
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < TN; ++i)
 #pragma unroll
       for (int j = 0; j < TM; ++j) {
-        acc[i][j] += t[i][j];
+        acc[i][j] += odd[i][j];
         total[i][j] = (ONE_PART || z == z_first) ? acc[i][j] : total[i][j] + acc[i][j];
-        acc[i][j] = t[i][j] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
+        acc[i][j] = odd[i][j] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
       }
   }
   GF_WAIT_LOADS(0);  // no load may reach LDS after the workgroup has gone
-  gemm_f32_store_tile<TM>(total, C, bias, plane, plane_stride, ldc, m0 + wm, n0 + wn, M, N, r, s);
+  gemm_f32_store_tile(total, C, bias, plane, plane_stride, ldc, m0 + wm, n0 + wn, M, N, r, s);
 }
 
 // C[m, n] = ((p_0 + p_1) + ... + p_{splits-1}) + bias[n] over the partial sums p_z[m, n] (rows of N
