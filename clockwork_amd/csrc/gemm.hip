@@ -1284,7 +1284,8 @@ static bool plan_stream(int mode, int M, int N, int K, int k_splits, int* mt, in
   // (up to 16 rows the one-tile kernels are as fast below two rounds; beyond, the alternative
   // is a library product that is slower as soon as every compute unit has a tile)
   const int slots = cw_num_compute_units();
-  if ((int64_t)*n_tiles * k_splits < (M <= 16 ? 2 * slots : slots)) return false;
+  // (partial sums of 17 rows and more go by cw_gemm_bf16_skinny_planes, down to a sixteenth of the units)
+  if ((int64_t)*n_tiles * k_splits < (M <= 16 ? 2 * slots : mode == 3 ? slots / 16 : slots)) return false;
   const int per = (*n_tiles * k_splits + slots - 1) / slots;
   *grid = dim3((*n_tiles + per - 1) / per, k_splits);
   return true;
@@ -1344,7 +1345,7 @@ CW_EXPORT int cw_gemm_bf16_skinny_ksplits(int M, int N, int K) {
     while (s > 1 && K / s < 256) --s;
     int mt_, spw, n_tiles;
     dim3 grid;
-    if (s <= 1 || !plan_stream(3, M, N, K, s, &mt_, &spw, &grid, &n_tiles)) return 1;
+    if (s <= 1 || tiles * s < cw_num_compute_units() || !plan_stream(3, M, N, K, s, &mt_, &spw, &grid, &n_tiles)) return 1;
     return s;
   }
   // up to 16 rows: a long K; or an output so wide that its norm does not run inside the next product (that kernel
@@ -1379,6 +1380,33 @@ CW_EXPORT int cw_gemm_bf16_skinny_ksplits(int M, int N, int K) {
   while (s > 1 && K / s < 1024) --s;
   if (s < 1) s = 1;
   return s;
+}
+
+// The same for 17 to 64 rows and a reader that adds the planes inside its own kernel (the residual-add + norm kernel does): from 2
+// planes on, 1 where none of these counts is taken. A workgroup's time is its row tiles of W times its steps, its x (every
+// workgroup takes in all rows of its part), a reduction a tile, and the planes' way to memory and back; a count that comes to more
+// workgroups than units has a second round for the few beyond. Without planes a narrow output's tiles leave units idle, and the
+// alternative is a library product that does the same. Product and the norm behind it, us, before (the library's, or as many
+// parts as fill the units) and by this rule, with 17 / 64 rows: 896 x 896 9.5 / 13.4, now 5.7 / 6.5; 1536 x 1536 6.5 / 8.0, now 6.2 / 7.3;
+// 2560 x 2560 12.8 / 17.0, now 8.2 / 10.8; 3584 x 3584 15.4 / 17.6, now 11.6 / 14.4; 4096 x 14336 48.7 / 51.8, now 29.0 / 33.6; 5120 x
+// 13824 43.4 / 45.7, now 36.9 / 41.3; 1536 x 8960 as before. (Over 30 shapes and 17, 32, 33 and 64 rows within 2 % of the best
+// count's time in the mean, 21 % at worst.)
+CW_EXPORT int cw_gemm_bf16_skinny_planes(int M, int N, int K) {
+  if (M <= 16 || M > 64 || N <= 0 || (N + 15) / 16 > 512) return 1;
+  int best = 1;
+  float least = 0.0f;
+  for (int s = 2; s <= 16 && K / s >= 256; ++s) {
+    int mt, spw, n_tiles;
+    dim3 grid;
+    if (!plan_stream(3, M, N, K, s, &mt, &spw, &grid, &n_tiles) || (int)(grid.x * grid.y) > cw_num_compute_units()) continue;
+    const int per = (n_tiles + (int)grid.x - 1) / (int)grid.x;
+    const float t = 0.22f * (float)(per * spw) + 0.11f * (float)(spw * mt) + 0.55f * (float)per + 2e-6f * (float)s * (float)M * (float)N;
+    if (best == 1 || t < least) {
+      least = t;
+      best = s;
+    }
+  }
+  return best;
 }
 
 // 1 if cw_gemm_bf16_skinny streams the weights once for this shape at full speed: every shape

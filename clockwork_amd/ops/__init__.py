@@ -113,6 +113,7 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_gemm_f32_pairs": [P, P, P, P, P, P, P, P, P, L, I, I, I, I, I, P],
             "cw_gemm_bf16_skinny": [I, P, L, P, P, L, I, I, I, I, F, P],
             "cw_gemm_bf16_skinny_ksplits": [I, I, I],
+            "cw_gemm_bf16_skinny_planes": [I, I, I],
             "cw_gemm_bf16_skinny_fast": [I, I, I, I],
             "cw_gemm_bf16_swiglu_normed_ok": [I, I, I],
             "cw_gemm_bf16_swiglu_normed": [P, P, P, I, F, P, P, L, I, I, I, P],
@@ -577,6 +578,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias=None, out_dtype=None, par
                     policy.k_split_choices[(N, K)] = _measure_k_splits(x, weight, splits)
                 chosen = policy.k_split_choices.get((N, K), 0)
                 splits = chosen or splits
+            elif M > SKINNY_MAX_ROWS and portions_partial_ok:
+                chosen = splits = lib.cw_gemm_bf16_skinny_planes(M, N, K)
             if splits > 1:
                 parts = torch.empty((splits, M, N), dtype=torch.float32, device=x.device)
                 _check(lib.cw_gemm_bf16_skinny(3, _ptr(x), K, _ptr(weight), _ptr(parts), N, M, N, K, chosen, 0.0, _stream()),

@@ -812,3 +812,22 @@ def test_float32_queries_keys_and_values_rotated_by_their_product(M, nh, nkv, hd
             # two products and a sum of values of up to 6 units, contracted or not: a unit in the last place of each
             assert bool(((got - want).abs() <= 3 * 6 * 2.0 ** -24).all())
     assert not ops.qkv_rope_fused_supported(x, w, hd - 2, hd, nh, nkv) and not ops.qkv_rope_fused_supported(x[:, : K - 8], w[:, : K - 8], hd, hd, nh, nkv)
+
+
+# few tiles and more than two a workgroup, an output and a K that end inside a tile and a step, the most planes
+@pytest.mark.parametrize("N,K", [(896, 896), (768, 512), (1544, 8968), (4096, 4096), (5128, 1000), (64, 8192)])
+@pytest.mark.parametrize("M", [17, 32, 33, 64])
+def test_planes_of_17_to_64_rows(M, N, K):
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(M + N)
+    x = torch.randn(M, K, device=DEV, generator=gen).bfloat16()
+    w = (torch.randn(N, K, device=DEV, generator=gen) * K ** -0.5).bfloat16()
+    planes = ops._load("gemm").cw_gemm_bf16_skinny_planes(M, N, K)
+    got = ops.linear(x, w, partial_ok=True, portions_partial_ok=True)
+    assert isinstance(got, ops.PartialSums) == (planes > 1) and (planes == 1 or got.parts.shape == (planes, M, N))
+    if planes > 1:
+        # float32 sums of K terms that come to a unit
+        torch.testing.assert_close(got.sum().double(), x.double() @ w.double().t(), rtol=0, atol=2.0 ** -17)
+    # a reader that adds no planes inside its kernel gets what it got
+    assert not isinstance(ops.linear(x, w, portions_partial_ok=True), ops.PartialSums)

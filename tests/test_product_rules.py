@@ -190,3 +190,16 @@ def test_float32_queries_keys_and_values_of_few_rows():
     # rows, blocks of K, whole blocks, whole tiles of a head, heads
     assert not (ok(0, 896, 14, 2, 64) or ok(17, 896, 14, 2, 64) or ok(1, 1936, 14, 2, 64) or ok(1, 888, 14, 2, 64) or ok(1, 896, 14, 2, 24)
                 or ok(1, 896, 0, 2, 64) or ok(1, 896, 2, 0, 64) or ok(1, 896, 1000, 20, 64))
+
+
+@pytest.mark.parametrize("N,K,planes", [(896, 896, 2), (1536, 1536, 2), (1536, 8960, 5), (3584, 3584, 2), (4096, 14336, 8), (8192, 28672, 16), (768, 512, 2)])
+def test_planes_of_17_to_64_rows(N, K, planes):
+    """A workgroup takes ceil(tiles * planes / 256) tiles of a part; no more workgroups than units."""
+    lib = ops._load("gemm")
+    assert lib.cw_gemm_bf16_skinny_planes(33, N, K) == planes
+    for M in (17, 32, 33, 64):
+        s = lib.cw_gemm_bf16_skinny_planes(M, N, K)
+        tiles = -(-N // 16)
+        assert 2 <= s <= 16 and K // s >= 256 and -(-tiles // -(-tiles * s // CUS)) * s <= CUS
+    # rows, an output of more than 512 tiles, K too short to cut, an output that leaves the units idle however K is cut
+    assert all(lib.cw_gemm_bf16_skinny_planes(*shape) == 1 for shape in ((16, N, K), (65, N, K), (33, 8193, K), (33, N, 511), (33, 64, 512)))
