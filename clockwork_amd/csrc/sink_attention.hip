@@ -10,7 +10,7 @@
 // first walk finds every row's maximum and denominator, the second recomputes the scores, normalises,
 // mixes across heads in LDS and multiplies with the values. Scores, weights and sums are float32.
 // Keys and values come in chunks of KT keys, one key/value head at a time, through LDS.
-#include "common.h"
+#include "recurrence.h"
 
 #define SA_KT 32       // keys a chunk
 #define SA_LANES 16    // lanes that share a (query, head) row of scores: 2 keys a lane and chunk
@@ -567,10 +567,10 @@ __global__ __launch_bounds__(256) void sink_decode_merge_kernel(SinkDecodeParams
 // HS, HV: heads a thread takes at a time with a key and with a value (of a group; of all, where they are mixed). What
 // fills the last turn up repeats its last head: a test for each head would wait for each one's LDS read by itself.
 template <typename T, int HS, int HV>
-__global__ __launch_bounds__(256) void sink_decode_runs_kernel(SinkDecodeParams p) {
+__device__ __forceinline__ void sink_decode_run(const SinkDecodeParams& p, const int r, const int run) {
   extern __shared__ __align__(16) float smem[];
   const int H = p.heads, G = p.kv_heads, D = p.dim, V = p.vdim, Hg = H / G, SK = p.sk, SP = (SK + 3) & ~3;
-  const int r = blockIdx.x, run = blockIdx.y, tid = threadIdx.x;
+  const int tid = threadIdx.x;
   int lo, pos;
   if (!sd_range(p, r, lo, pos)) return;
   const int k0 = lo + run * SK;
@@ -760,6 +760,24 @@ __global__ __launch_bounds__(256) void sink_decode_runs_kernel(SinkDecodeParams 
   }
 }
 
+template <typename T, int HS, int HV>
+__global__ __launch_bounds__(256) void sink_decode_runs_kernel(SinkDecodeParams p) {
+  sink_decode_run<T, HS, HV>(p, blockIdx.x, blockIdx.y);
+}
+
+// The runs, and behind them the workgroups of a recurrence over the same step (recurrence.h), which needs nothing of them: both are
+// bound by their trips to memory, one after another, and leave most units idle. 8 requests of 200 keys, 12 heads of 128 over 2, beside
+// 12 heads of 64 x 128: 15.2 and 9.2 us as launches of their own; as one, a layer takes 8.2 us less.
+template <int HS, int HV, int RPT>
+__global__ __launch_bounds__(256) void sink_decode_runs_beside_kernel(SinkDecodeParams p, int requests, int run_blocks, RecurrenceLaunch l) {
+  const int block = blockIdx.x;
+  if (block < run_blocks) {
+    sink_decode_run<bf16_t, HS, HV>(p, block % requests, block / requests);
+  } else {
+    recurrence_quads<bf16_t, RPT>(l.p, l.f, l.rank_quads != 0, (block - run_blocks) / l.p.heads, (block - run_blocks) % l.p.heads);
+  }
+}
+
 // grid: request, key/value head (mixed) or 1, 64 value columns; a wave per head, up to 16 waves
 template <typename T>
 __global__ __launch_bounds__(1024) void sink_decode_mix_kernel(SinkDecodeParams p) {
@@ -846,14 +864,24 @@ CW_EXPORT int cw_sink_decode_supported(int heads, int kv_heads, int dim, int vdi
   return a <= 150 * 1024 && b <= 150 * 1024 ? 1 : 0;
 }
 
+// Can a recurrence go beside these runs (``beside`` of cw_sink_decode)? bfloat16, two kernels, five to eight heads of a group and
+// up to 16 mixed ones.
+CW_EXPORT int cw_sink_decode_beside_ok(int dtype, int n_runs, int heads, int kv_heads, int mixed) {
+  if (dtype != CW_BF16 || heads <= 0 || kv_heads <= 0 || heads % kv_heads || !sd_two(n_runs, heads, kv_heads, mixed != 0)) return 0;
+  const int group = heads / kv_heads;
+  return mixed && group > 4 && group <= 8 && heads > 8 && heads <= 16 ? 1 : 0;
+}
+
 // Every request of the step has one token (requests with another count are left alone). The keys a
 // token sees ([max(0, pos - window + 1), pos]) are cut into runs of sk keys from their first;
-// n_runs is the most runs any request has (the host knows the longest context).
+// n_runs is the most runs any request has (the host knows the longest context). ``beside``: nullptr, or a recurrence of the same
+// step that cw_linear_recurrence_prepare has left, to run in the same launch (see cw_sink_decode_beside_ok).
 CW_EXPORT int cw_sink_decode(int dtype, const void* q, int64_t q_stride, void* out, const void* k_cache,
                              const void* v_cache, int64_t cache_rows, const int* block_tables, int table_width,
                              const int* ctx_lens, const int* cu_q, int n_requests, int sk, int n_runs, float* workspace,
                              const float* r1, const float* r2, const float* sink, const float* talk, int heads,
-                             int kv_heads, int dim, int vdim, int block_size, int window, float scale, hipStream_t stream) {
+                             int kv_heads, int dim, int vdim, int block_size, int window, float scale, const void* beside,
+                             hipStream_t stream) {
   if (n_requests < 0 || !q || !out || !k_cache || !v_cache || !block_tables || !ctx_lens || !cu_q || !workspace)
     return CW_ERR_ARG;
   if (block_size <= 0 || table_width <= 0 || window < 0 || (r1 && !r2) || sk < 1 || sk > SD_MAX_SK || n_runs < 1)
@@ -872,6 +900,7 @@ CW_EXPORT int cw_sink_decode(int dtype, const void* q, int64_t q_stride, void* o
   p.partial = p.stats + (int64_t)n_requests * n_runs * heads * 2;
   p.heads = heads; p.kv_heads = kv_heads; p.dim = dim; p.vdim = vdim; p.block_size = block_size; p.window = window;
   p.sk = sk; p.n_runs = n_runs; p.scale = scale; p.cache_rows = cache_rows;
+  if (beside && !cw_sink_decode_beside_ok(dtype, n_runs, heads, kv_heads, talk != nullptr)) return CW_ERR_SIZE;
   const size_t smem1 = ((size_t)heads * dim + (size_t)heads * sk) * sizeof(float);
   const size_t smem2 = (2 * (size_t)heads * sk + 2 * heads + sk + (size_t)heads * heads) * sizeof(float);
   const dim3 grid(n_requests, n_runs), block(256);
@@ -883,6 +912,28 @@ CW_EXPORT int cw_sink_decode(int dtype, const void* q, int64_t q_stride, void* o
     const dim3 mgrid(n_requests, talk ? kv_heads : 1, (vdim + 63) / 64), mblock(64 * (heads < 16 ? heads : 16));
     // heads a thread takes at a time: a whole group and all mixed heads in one turn, for up to 16
     const int hg = heads / kv_heads, hv = talk ? heads : hg;
+    if (beside) {
+      const RecurrenceLaunch& l = *(const RecurrenceLaunch*)beside;
+      const size_t both = lds > (size_t)l.lds ? lds : (size_t)l.lds;
+      const int64_t run_blocks = (int64_t)n_requests * n_runs, blocks = run_blocks + (int64_t)l.requests * l.p.heads;
+      if (blocks > 0x7fffffff) return CW_ERR_SIZE;
+#define CW_BESIDE(HS_, HV_, RPT_)                                                                                      \
+  do {                                                                                                                 \
+    if (both > 48 * 1024 && hipFuncSetAttribute((const void*)sink_decode_runs_beside_kernel<HS_, HV_, RPT_>,           \
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)both) != hipSuccess)  \
+      return CW_ERR_LAUNCH;                                                                                            \
+    if (mlds > 48 * 1024 && hipFuncSetAttribute((const void*)sink_decode_mix_kernel<bf16_t>,                           \
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)mlds) != hipSuccess)  \
+      return CW_ERR_LAUNCH;                                                                                            \
+    hipLaunchKernelGGL((sink_decode_runs_beside_kernel<HS_, HV_, RPT_>), dim3((unsigned)blocks), block, both, stream, p, n_requests, \
+                       (int)run_blocks, l);                                                                            \
+    hipLaunchKernelGGL((sink_decode_mix_kernel<bf16_t>), mgrid, mblock, mlds, stream, p);                              \
+    return cw_launch_status();                                                                                         \
+  } while (0)
+      if (l.rows == 4) CW_BESIDE(8, 16, 4);
+      CW_BESIDE(8, 16, 8);
+#undef CW_BESIDE
+    }
 #define CW_TWO(T_, HS_, HV_)                                                                                           \
   do {                                                                                                                 \
     if (lds > 48 * 1024 && hipFuncSetAttribute((const void*)sink_decode_runs_kernel<T_, HS_, HV_>,                     \

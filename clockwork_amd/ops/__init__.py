@@ -225,10 +225,13 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_sink_prefill_mfma_supported": [I, I, I, I],
             "cw_sink_prefill_mfma": [P, L, P, P, P, L, P, I, P, P, P, I, P, P, P, P, I, I, I, I, I, I, F, I, P],
             "cw_sink_decode_supported": [I, I, I, I],
-            "cw_sink_decode": [I, P, L, P, P, P, L, P, I, P, P, I, I, I, P, P, P, P, P, I, I, I, I, I, I, F, P],
+            "cw_sink_decode": [I, P, L, P, P, P, L, P, I, P, P, I, I, I, P, P, P, P, P, I, I, I, I, I, I, F, P, P],
+            "cw_sink_decode_beside_ok": [I, I, I, I, I],
         },
         "linear_recurrence": {
             "cw_linear_recurrence_supported": [I, I],
+            "cw_linear_recurrence_prepared_bytes": [],
+            "cw_linear_recurrence_prepare": [I, P, L, I, I, I, I, I, P, P, P, P, I, P, P, P, I, I, I, I, I, F, F, F, I, P, I, P, L, L, P],
             "cw_linear_recurrence": [I, P, L, I, I, I, I, I, P, P, P, P, I, P, P, P, I, I, I, I, I, F, F, F, I, P, I, P, L, L, P],
             "cw_linear_recurrence_segments_supported": [I, I],
             "cw_linear_recurrence_segments_workspace_floats": [I, I, I, I, I, I],
@@ -1841,9 +1844,22 @@ def _recurrence_operands(proj, q_off, k_off, v_off, g_off, u_off, a2, a2_bias, n
     return T, width, (int(q_off), int(k_off), int(v_off), int(g_off), int(u_off)), tail
 
 
+class PreparedRecurrence:
+    """A launch of ``linear_recurrence`` that another kernel makes; holds the tensors that it reads and writes until then."""
+
+    __slots__ = ("buffer", "operands")
+
+    def __init__(self, size: int, operands: tuple) -> None:
+        self.buffer, self.operands = ctypes.create_string_buffer(size), operands
+
+    @property
+    def address(self) -> int:
+        return ctypes.addressof(self.buffer)
+
+
 def linear_recurrence(proj, q_off: int, k_off: int, v_off: int, g_off: int, u_off: int, a2, a2_bias, norm_weight, state,
                       state_slots, cu_q, n_requests: int, heads: int, dim: int, vdim: int, q_scale: float, tau: float,
-                      eps: float, decay: str = "sigmoid_power", bonus=None, decay_input=None) -> torch.Tensor:
+                      eps: float, decay: str = "sigmoid_power", bonus=None, decay_input=None, prepare: bool = False):
     """The decayed recurrence S <- diag(a) S + k v^T, o = S^T (q_scale q) over the step's tokens,
     request by request from each request's slot of ``state`` (float32 [slots, ...]: a slot's
     first heads * dim * vdim floats are the matrices, updated in place). Rows of ``proj`` hold q,
@@ -1856,18 +1872,26 @@ def linear_recurrence(proj, q_off: int, k_off: int, v_off: int, g_off: int, u_of
     ``decay_input`` [T, rank]: the decay's input as a tensor of its own. ``decay`` "double_exp":
     a = exp(-exp(a2 input + bias)); "double_exp_tanh": a = exp(-exp(a2 tanh(input) + bias)). ``bonus`` float32 [heads, dim]: the output reads the
     state before the token joins it and the token itself through the bonus,
-    o = (S + diag(bonus) k v^T)^T q, then S <- diag(a) S + k v^T."""
+    o = (S + diag(bonus) k v^T)^T q, then S <- diag(a) S + k v^T.
+
+    ``prepare``: (the output, a launch) with nothing run yet, for a kernel that takes it beside its own work in this step
+    (``sink_attention_decode``); (the output, None) where it has run as ever, for sizes that have no such launch."""
     _gpu(proj, a2, a2_bias, norm_weight, state, state_slots, cu_q, bonus, decay_input)
     T, width, offs, tail = _recurrence_operands(proj, q_off, k_off, v_off, g_off, u_off, a2, a2_bias, norm_weight, state, heads,
                                                 dim, vdim, decay, bonus, decay_input)
     _i32(state_slots, n_requests, "state_slots")
     _i32(cu_q, n_requests + 1, "cu_q")
     out = torch.empty((T, heads * vdim), dtype=proj.dtype, device=proj.device)
-    _check(_load("linear_recurrence").cw_linear_recurrence(
-        dtype_code(proj.dtype), _ptr(proj), width, *offs, _ptr(a2), _ptr(a2_bias),
-        _ptr(norm_weight), _ptr(state), state.shape[0], _ptr(state_slots), _ptr(cu_q), _ptr(out), n_requests, heads, dim,
-        vdim, a2.shape[1], float(q_scale), 1.0 / float(tau), float(eps), *tail, _stream()), "linear_recurrence")
-    return out
+    args = (dtype_code(proj.dtype), _ptr(proj), width, *offs, _ptr(a2), _ptr(a2_bias), _ptr(norm_weight), _ptr(state), state.shape[0],
+            _ptr(state_slots), _ptr(cu_q), _ptr(out), n_requests, heads, dim, vdim, a2.shape[1], float(q_scale), 1.0 / float(tau),
+            float(eps), *tail)
+    lib = _load("linear_recurrence")
+    if prepare:
+        launch = PreparedRecurrence(lib.cw_linear_recurrence_prepared_bytes(), (proj, decay_input, out))
+        if n_requests > 0 and lib.cw_linear_recurrence_prepare(*args, launch.address) == 0:
+            return out, launch
+    _check(lib.cw_linear_recurrence(*args, _stream()), "linear_recurrence")
+    return (out, None) if prepare else out
 
 
 def linear_recurrence_segments_supported(dim: int, vdim: int) -> bool:
@@ -1973,10 +1997,11 @@ def sink_decode_supported(heads: int, kv_heads: int, dim: int, vdim: int) -> boo
 
 def sink_attention_decode(q, q_stride: int, out, k_cache, v_cache, block_tables, ctx_lens, cu_q, n_requests: int,
                           run_keys: int, n_runs: int, r1, r2, sink, talk, heads: int, kv_heads: int, dim: int, vdim: int,
-                          block_size: int, window: int, scale: float) -> None:
+                          block_size: int, window: int, scale: float, beside=None) -> None:
     """``sink_attention`` for the step's requests of one token each (others are left alone): the
     keys a token sees are cut into ``n_runs`` runs of ``run_keys`` keys (the most any request of
-    the step has), a workgroup each; the runs are merged by a kernel of its own."""
+    the step has), a workgroup each; the runs are merged by a kernel of its own. ``beside``: a launch that
+    ``linear_recurrence`` has prepared, to run beside the runs (where ``sink_decode_takes_beside``)."""
     _gpu(q, out, k_cache, v_cache, block_tables, ctx_lens, cu_q, r1, r2, sink, talk)
     T = q.shape[0]
     _need(q.dim() == 2 and q.shape[1] == q_stride and heads * dim <= q_stride, "q must be [T, q_stride] with the query heads first")
@@ -1999,8 +2024,14 @@ def sink_attention_decode(q, q_stride: int, out, k_cache, v_cache, block_tables,
     _check(lib.cw_sink_decode(
         dtype_code(q.dtype), _ptr(q), q_stride, _ptr(out), _ptr(k_cache), _ptr(v_cache), rows, _ptr(block_tables),
         block_tables.shape[1], _ptr(ctx_lens), _ptr(cu_q), n_requests, run_keys, n_runs, _ptr(workspace), _ptr(r1), _ptr(r2),
-        _ptr(sink), _ptr(talk), heads, kv_heads, dim, vdim, block_size, int(window), float(scale), _stream()),
+        _ptr(sink), _ptr(talk), heads, kv_heads, dim, vdim, block_size, int(window), float(scale),
+        beside.address if beside is not None else None, _stream()),
         "sink_attention_decode")
+
+
+def sink_decode_takes_beside(dtype, n_runs: int, heads: int, kv_heads: int, mixed: bool) -> bool:
+    """Can ``sink_attention_decode`` of this geometry run a prepared recurrence in its launch?"""
+    return bool(_load("sink_attention").cw_sink_decode_beside_ok(dtype_code(dtype), n_runs, heads, kv_heads, int(mixed)))
 
 
 def sink_prefill_mfma_supported(heads: int, kv_heads: int, dim: int, vdim: int, dtype) -> bool:

@@ -30,7 +30,9 @@ Roles and their run methods:
                  the matrices that x is multiplied with before anything else (no bias); ``forward``
                  then takes their products as a fourth argument where the block has made them,
                  in one launch with others of the same x (``ops.linear_several``). And
-                 ``before_output(x, ctx, cache, made=None)``: all but the product with ``out_weight``.
+                 ``before_output(x, ctx, cache, made=None)``: all but the product with ``out_weight``;
+                 ``prepared_output`` and ``takes_beside`` put the kernel of one mixer of a pair into
+                 the other's launch.
 * feed-forward:  ``forward(x, ctx) -> y``.
 * position enc.: used by a mixer, not by the block; the attention mixer expects
                  ``rotate_and_store(qkv, bias, positions, slots, nh, nkv, hd, k, v)``, and

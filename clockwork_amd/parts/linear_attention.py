@@ -103,6 +103,15 @@ class DecayedLinearAttention(Part):
         return ops.linear(self.before_output(x, ctx, cache, made), self.out_weight, policy=getattr(ctx, "products", None))
 
     def before_output(self, x: torch.Tensor, ctx, cache: EntryCache, made=None) -> torch.Tensor:
+        return self._output(x, ctx, cache, made, False)
+
+    def prepared_output(self, x: torch.Tensor, ctx, cache: EntryCache, made=None) -> tuple:
+        """(``before_output``'s tensor, the launch that is still to make it or None): for a mixer beside this one whose
+        kernel takes the launch into its own (``takes_beside``)."""
+        out = self._output(x, ctx, cache, made, True)
+        return out if isinstance(out, tuple) else (out, None)
+
+    def _output(self, x, ctx, cache: EntryCache, made, prepare: bool):
         s = self.spec
         proj = made[0] if made is not None else ops.linear(x, self.in_weight, policy=getattr(ctx, "products", None))
         common = (proj, self.q_off, self.k_off, self.v_off, self.g_off, self.u_off, self.decay_weight, self.decay_bias,
@@ -112,7 +121,7 @@ class DecayedLinearAttention(Part):
         if plan is not None:
             items, n_segments, first = plan
             return ops.linear_recurrence_segments(*common, items, n_segments, SEGMENT_TOKENS, first, *sizes)
-        return ops.linear_recurrence(*common, *sizes)
+        return ops.linear_recurrence(*common, *sizes, prepare=prepare)
 
 
 class ShiftedRecurrence(Part):

@@ -118,7 +118,11 @@ class PairMixer(Part):
         each = ((self.left, left, made and made[:mine]), (self.right, right, made and made[mine:]))
         if not all(hasattr(m, "before_output") for m, _, _ in each):
             return [m.forward(x, ctx, own) if given is None else m.forward(x, ctx, own, given) for m, own, given in each]
-        outs = [m.before_output(x, ctx, own, given) for m, own, given in each]
+        if hasattr(self.right, "prepared_output") and getattr(self.left, "takes_beside", lambda *a: False)(x, ctx):
+            b, launch = self.right.prepared_output(x, ctx, *each[1][1:])
+            outs = [self.left.before_output(x, ctx, *each[0][1:], beside=launch), b]
+        else:
+            outs = [m.before_output(x, ctx, own, given) for m, own, given in each]
         weights = [m.out_weight for m, _, _ in each]
         return ops.linear_several(outs, weights) or [ops.linear(o, w, policy=getattr(ctx, "products", None)) for o, w in zip(outs, weights)]
 

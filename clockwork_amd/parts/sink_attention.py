@@ -144,7 +144,12 @@ class SinkAttention(Part):
     def forward(self, x: torch.Tensor, ctx, cache: EntryCache, made=None) -> torch.Tensor:
         return ops.linear(self.before_output(x, ctx, cache, made), self.out_weight, policy=getattr(ctx, "products", None))
 
-    def before_output(self, x: torch.Tensor, ctx, cache: EntryCache, made=None) -> torch.Tensor:
+    def takes_beside(self, x: torch.Tensor, ctx) -> bool:
+        """Does ``before_output`` run another mixer's prepared recurrence in the launch of its single tokens' runs?"""
+        s, n_runs = self.spec, self._plan(ctx)[3]
+        return n_runs > 0 and ops.sink_decode_takes_beside(x.dtype, n_runs, s.num_heads, s.num_kv_heads, self.talk is not None)
+
+    def before_output(self, x: torch.Tensor, ctx, cache: EntryCache, made=None, beside=None) -> torch.Tensor:
         s = self.spec
         if not cache.writes:
             raise NotImplementedError("this mixer writes its own keys and values: it cannot borrow another entry's cache")
@@ -164,5 +169,5 @@ class SinkAttention(Part):
                                ctx.cu_q, items, n_items, self.run, *options)
         if n_runs:
             ops.sink_attention_decode(qkv, qkv.shape[1], out, k_plane, v_plane, ctx.block_tables[cache.group], ctx.ctx_lens,
-                                      ctx.cu_q, ctx.num_requests, run_keys, n_runs, *options)
+                                      ctx.cu_q, ctx.num_requests, run_keys, n_runs, *options, beside=beside)
         return out

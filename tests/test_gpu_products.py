@@ -831,3 +831,41 @@ def test_planes_of_17_to_64_rows(M, N, K):
         torch.testing.assert_close(got.sum().double(), x.double() @ w.double().t(), rtol=0, atol=2.0 ** -17)
     # a reader that adds no planes inside its kernel gets what it got
     assert not isinstance(ops.linear(x, w, portions_partial_ok=True), ops.PartialSums)
+
+
+# four and eight rows of the state a thread; requests of one token and of several, a request without a slot, keys of one run and of many
+@pytest.mark.parametrize("heads,dim,r_vdim,rank", [(14, 64, 64, 16), (12, 128, 128, 32), (10, 64, 64, 5)])
+@pytest.mark.parametrize("q_lens", [(1,), (1, 1, 1, 1, 1), (1, 7, 1)])
+def test_a_recurrence_beside_the_runs_of_single_tokens(heads, dim, r_vdim, rank, q_lens):
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(heads + len(q_lens))
+    rand = lambda *s: torch.randn(*s, device=DEV, generator=gen)  # noqa: E731
+    ints = lambda t: torch.as_tensor(t, dtype=torch.int32, device=DEV)  # noqa: E731
+    R, T, kv, bs, pages, sk = len(q_lens), sum(q_lens), 2, 16, 20, 32
+    ctx = [300 - 70 * r for r in range(R)]
+    k, v = (rand(R * pages, bs, kv, dim).bfloat16() for _ in range(2))
+    tables, cu = torch.arange(R * pages, device=DEV, dtype=torch.int32).view(R, pages), ints([0, *torch.tensor(q_lens).cumsum(0).tolist()])
+    q = rand(T, heads * dim).bfloat16()
+    sink = (rand(heads).abs(), rand(heads).abs(), rand(heads), torch.eye(heads, device=DEV) + 0.2 * rand(heads, heads))
+    runs = -(-max(ctx) // sk)
+    assert ops.sink_decode_takes_beside(torch.bfloat16, runs, heads, kv, True)
+    assert not ops.sink_decode_takes_beside(torch.float32, runs, heads, kv, True) and not ops.sink_decode_takes_beside(torch.bfloat16, runs, heads, kv, False)
+    qk, vv = heads * 64, heads * r_vdim
+    proj = rand(T, 2 * qk + 2 * vv + rank).bfloat16()
+    a2, bias, norm = rand(qk, rank).bfloat16(), rand(qk), rand(r_vdim)
+    first = rand(R + 1, heads, 64, r_vdim)
+    slots = ints([R - r if r != 1 else -1 for r in range(R)])
+
+    def both(beside):
+        state, out = first.clone(), torch.zeros(T, heads * dim, device=DEV, dtype=torch.bfloat16)
+        args = (proj, 0, qk, 2 * qk, 2 * qk + vv, 2 * qk + 2 * vv, a2, bias, norm, state, slots, cu, R, heads, 64, r_vdim, 0.125, 16.0, 1e-6)
+        y, launch = ops.linear_recurrence(*args, prepare=True) if beside else (ops.linear_recurrence(*args), None)
+        assert (launch is not None) == beside
+        ops.sink_attention_decode(q, heads * dim, out, k, v, tables, ints(ctx), cu, R, sk, runs, *sink, heads, kv, dim, dim, bs, 200, dim ** -0.5,
+                                  beside=launch)
+        return y, state, out
+
+    apart, together = both(False), both(True)
+    rows = torch.cat([torch.arange(int(cu[r]), int(cu[r + 1]), device=DEV) for r in range(R) if r != 1])   # a request without a slot has no outputs
+    assert torch.equal(apart[0][rows], together[0][rows]) and torch.equal(apart[1], together[1]) and torch.equal(apart[2], together[2])
