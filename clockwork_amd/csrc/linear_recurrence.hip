@@ -186,7 +186,7 @@ static int recurrence_launch(RecurrenceLaunch& l, int dtype, const void* proj, i
 CW_EXPORT int cw_linear_recurrence_prepared_bytes() { return sizeof(RecurrenceLaunch); }
 
 // The launch of cw_linear_recurrence as ``prepared`` (cw_linear_recurrence_prepared_bytes()), for a kernel that runs it beside other
-// work (cw_sink_decode); CW_ERR_SIZE where there is none for these sizes: bfloat16, four columns and four or eight rows a thread.
+// work (cw_sink_decode_beside); CW_ERR_SIZE where there is none for these sizes: bfloat16, four columns and four or eight rows a thread.
 CW_EXPORT int cw_linear_recurrence_prepare(int dtype, const void* proj, int64_t stride, int q_off, int k_off, int v_off, int g_off,
                                            int u_off, const void* a2, const float* a2b, const float* norm_w, float* state,
                                            int n_slots, const int* state_slots, const int* cu_q, void* out, int n_requests,

@@ -864,7 +864,7 @@ CW_EXPORT int cw_sink_decode_supported(int heads, int kv_heads, int dim, int vdi
   return a <= 150 * 1024 && b <= 150 * 1024 ? 1 : 0;
 }
 
-// Can a recurrence go beside these runs (``beside`` of cw_sink_decode)? bfloat16, two kernels, five to eight heads of a group and
+// Can a recurrence go beside these runs (cw_sink_decode_beside)? bfloat16, two kernels, five to eight heads of a group and
 // up to 16 mixed ones.
 CW_EXPORT int cw_sink_decode_beside_ok(int dtype, int n_runs, int heads, int kv_heads, int mixed) {
   if (dtype != CW_BF16 || heads <= 0 || kv_heads <= 0 || heads % kv_heads || !sd_two(n_runs, heads, kv_heads, mixed != 0)) return 0;
@@ -876,7 +876,7 @@ CW_EXPORT int cw_sink_decode_beside_ok(int dtype, int n_runs, int heads, int kv_
 // token sees ([max(0, pos - window + 1), pos]) are cut into runs of sk keys from their first;
 // n_runs is the most runs any request has (the host knows the longest context). ``beside``: nullptr, or a recurrence of the same
 // step that cw_linear_recurrence_prepare has left, to run in the same launch (see cw_sink_decode_beside_ok).
-CW_EXPORT int cw_sink_decode(int dtype, const void* q, int64_t q_stride, void* out, const void* k_cache,
+CW_EXPORT int cw_sink_decode_beside(int dtype, const void* q, int64_t q_stride, void* out, const void* k_cache,
                              const void* v_cache, int64_t cache_rows, const int* block_tables, int table_width,
                              const int* ctx_lens, const int* cu_q, int n_requests, int sk, int n_runs, float* workspace,
                              const float* r1, const float* r2, const float* sink, const float* talk, int heads,
@@ -979,6 +979,16 @@ CW_EXPORT int cw_sink_decode(int dtype, const void* q, int64_t q_stride, void* o
   else return CW_ERR_DTYPE;
 #undef CW_LAUNCH
   return cw_launch_status();
+}
+
+CW_EXPORT int cw_sink_decode(int dtype, const void* q, int64_t q_stride, void* out, const void* k_cache,
+                             const void* v_cache, int64_t cache_rows, const int* block_tables, int table_width,
+                             const int* ctx_lens, const int* cu_q, int n_requests, int sk, int n_runs, float* workspace,
+                             const float* r1, const float* r2, const float* sink, const float* talk, int heads,
+                             int kv_heads, int dim, int vdim, int block_size, int window, float scale, hipStream_t stream) {
+  return cw_sink_decode_beside(dtype, q, q_stride, out, k_cache, v_cache, cache_rows, block_tables, table_width, ctx_lens, cu_q, n_requests,
+                               sk, n_runs, workspace, r1, r2, sink, talk, heads, kv_heads, dim, vdim, block_size, window, scale, nullptr,
+                               stream);
 }
 
 // ======================================================================================

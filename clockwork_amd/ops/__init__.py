@@ -225,7 +225,8 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_sink_prefill_mfma_supported": [I, I, I, I],
             "cw_sink_prefill_mfma": [P, L, P, P, P, L, P, I, P, P, P, I, P, P, P, P, I, I, I, I, I, I, F, I, P],
             "cw_sink_decode_supported": [I, I, I, I],
-            "cw_sink_decode": [I, P, L, P, P, P, L, P, I, P, P, I, I, I, P, P, P, P, P, I, I, I, I, I, I, F, P, P],
+            "cw_sink_decode": [I, P, L, P, P, P, L, P, I, P, P, I, I, I, P, P, P, P, P, I, I, I, I, I, I, F, P],
+            "cw_sink_decode_beside": [I, P, L, P, P, P, L, P, I, P, P, I, I, I, P, P, P, P, P, I, I, I, I, I, I, F, P, P],
             "cw_sink_decode_beside_ok": [I, I, I, I, I],
         },
         "linear_recurrence": {
@@ -2021,7 +2022,7 @@ def sink_attention_decode(q, q_stride: int, out, k_cache, v_cache, block_tables,
     lib = _load("sink_attention")
     need = lib.cw_sink_decode_workspace_floats(n_requests, n_runs, run_keys, heads, kv_heads, vdim, int(talk is not None))
     workspace = torch.empty(max(int(need), 1), dtype=torch.float32, device=q.device)
-    _check(lib.cw_sink_decode(
+    _check(lib.cw_sink_decode_beside(
         dtype_code(q.dtype), _ptr(q), q_stride, _ptr(out), _ptr(k_cache), _ptr(v_cache), rows, _ptr(block_tables),
         block_tables.shape[1], _ptr(ctx_lens), _ptr(cu_q), n_requests, run_keys, n_runs, _ptr(workspace), _ptr(r1), _ptr(r2),
         _ptr(sink), _ptr(talk), heads, kv_heads, dim, vdim, block_size, int(window), float(scale),
