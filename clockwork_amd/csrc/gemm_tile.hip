@@ -261,8 +261,8 @@ CW_EXPORT int cw_gemm_bf16_tiled(int mode, const void* X, int64_t ldx, const voi
 // has one register set: a row block's is read again when its products are issued.
 //
 // What bounds it. Inside a tile: with every load taken out the 1.5B shape's gate/up product of 2048
-// rows takes 0.85 of its time, of 160 rows 0.6. A compute unit takes in 43 GB/s from memory, 80 from L2, however
-// deep the ring is (its 32 KB L1 holds a line for every load in flight, and answers in order), so a tile's
+// rows takes 0.85 of its time, of 160 rows 0.6. A compute unit was seen to take in 43 GB/s from memory and 80 from
+// L2 however deep the ring is (why is not known; a bound on its loads in flight would do that), so a tile's
 // loads go with (MB + NB) K, and its matrix instructions with MB NB K. Around it: a tile's first
 // loads, its gate and its stores, 5 us a
 // tile of 256 x 288, which only the next tile's first loads overlap. So few large tiles beat many small ones, in whole
@@ -483,9 +483,11 @@ __global__ __launch_bounds__(256) void gemm_wide_bf16_kernel(WideArgs a) {
         acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[set][ni], xf[x_set(set, mi)][mi], acc[mi][ni], 0, 0, 0);
       } else {
         // More accumulators than there are accumulation registers: 62 live there and the others with the operands. Left to
-        // itself the compiler keeps all in one kind and moves a hundred of them back and forth an iteration.
+        // itself the compiler keeps all in one kind and moves a hundred of them back and forth an iteration. It does not know
+        // either that these are products, which may read what it has written two states before at the earliest: it writes
+        // the others' zeros right before their first one.
         if (g < 62) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[mi][ni]) : "v"(wf[set][ni]), "v"(xf[x_set(set, mi)][mi]));
-        else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[mi][ni]) : "v"(wf[set][ni]), "v"(xf[x_set(set, mi)][mi]));
+        else asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[mi][ni]) : "v"(wf[set][ni]), "v"(xf[x_set(set, mi)][mi]));
       }
       // reads and loads spread over the products (the texture path takes a load every 16 cycles; several in a row stall
       // the wave), the reads done a little before the end

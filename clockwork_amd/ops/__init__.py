@@ -809,7 +809,9 @@ WIDE_MIN_TILES = 64
 # 97.2 / 86.0; 7B shape, 400 rows 150 / 136, 640 rows 189 / 202: there reading W bounds both). Against the library's TUNED choice it wins for
 # the 0.5B, 1.5B, 3B, 14B and 32B shapes (the 1.5B shape's whole prefill step: 8.9 -> 7.9 ms) and
 # loses 3 % of the step for the 7B and 72B shapes, so a start-up that tunes (``library_tuning``)
-# times both ways on the model's own weights and keeps the faster (``ProductPolicy.swiglu_choices``).
+# times both ways on the model's own weights and keeps the faster (``ProductPolicy.swiglu_choices``). These figures are of tiles
+# of 256 x 192; by the tiles it chooses from now (csrc/gemm_tile.hip) the kernel takes 1 to 30 % less, so the line is cautious: what
+# lies below it goes by ``cw_gemm_bf16_wide_choice``, from 65 rows on.
 WIDE_SWIGLU_MIN_TILES = 180
 WIDE_SWIGLU_MIN_ROWS = 1024
 WIDE_SWIGLU_WORK, WIDE_SWIGLU_WORK_ONE_ROUND = 0.58, 0.52
