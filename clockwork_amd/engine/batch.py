@@ -78,7 +78,7 @@ class StepContext:
         self.h_state_slots: list[int] = []
         self.seq_ids: list[str] = []
         self.plans: dict = {}     # what parts have planned for this step, under keys of their own
-        self.made: dict = {}      # what a pass over the model makes for several layers (begun anew by every pass)
+        self.made: dict | None = None   # what a pass over the model makes for several layers; None outside of one
         self._pinned: list = []   # host buffers of the plans' uploads, alive as long as the step
         self.num_compute_units = 256
         self.captured = False     # a captured step's batch: planned for all steps of its class

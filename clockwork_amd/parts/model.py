@@ -156,12 +156,20 @@ class DecoderModel:
         """Run the step's tokens; returns float32 logits [len(ctx.logit_rows), vocab] or None
         when no logits are wanted. ``caches[i]`` is the EntryCache of run entry i; those of
         ``own_caches`` follow."""
+        # what this pass makes on the device for several layers, by keys of the parts' own: of this pass alone, since the
+        # step's tensors may hold other numbers by the next (and a layer run by itself finds nothing kept)
+        ctx.made = {}
+        try:
+            return self._pass(ctx, caches)
+        finally:
+            ctx.made = None
+
+    def _pass(self, ctx, caches) -> Optional[torch.Tensor]:
         # what ``ctx.positions`` holds is the embedding part's to say: without its word every token
         # carries its index in its request (``ctx.sequence_positions``, which stays what it is)
         positions_of = getattr(self.embedding, "positions", None)
         if positions_of is not None:
             ctx.positions = positions_of(ctx)
-        ctx.made = {}   # what this pass makes on the device for several layers, by keys of the parts' own
         # a part outside the blocks that keeps something has its cache behind those of the run entries
         own = bool(self.own_caches())
         resid = self.embedding.forward(ctx, caches[len(self.spec.run)]) if own else self.embedding.forward(ctx)

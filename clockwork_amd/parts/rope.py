@@ -65,7 +65,8 @@ class RopeNeox(Part):
 
     def project_rotate_store_rows(self, x, weight, bias, ctx, slots, nh, nkv, hd, k_cache, v_cache):
         """The same for a portion's rows: by a table of the step's angles, made by the first layer that asks in a pass
-        over the model (``ctx.made``; 1 MB for 2048 tokens, 2 us). None where a product and ``rotate_and_store`` are the faster way."""
+        over the model (``ctx.made``; 1 MB for 2048 tokens, 2 us), by every call
+        outside of one. None where a product and ``rotate_and_store`` are the faster way."""
         if slots is None or not ops.qkv_rope_rows_ok(x, weight, bias, self.spec.rotary_dim, hd, k_cache, v_cache):
             return None
         made = getattr(ctx, "made", None)

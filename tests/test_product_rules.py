@@ -203,3 +203,42 @@ def test_planes_of_17_to_64_rows(N, K, planes):
         assert 2 <= s <= 16 and K // s >= 256 and -(-tiles // -(-tiles * s // CUS)) * s <= CUS
     # rows, an output of more than 512 tiles, K too short to cut, an output that leaves the units idle however K is cut
     assert all(lib.cw_gemm_bf16_skinny_planes(*shape) == 1 for shape in ((16, N, K), (65, N, K), (33, 8193, K), (33, N, 511), (33, 64, 512)))
+
+
+def test_a_table_of_angles_is_kept_for_a_pass_over_the_model_only(monkeypatch):
+    """Layers of one pass share a table; a layer that is called by itself, with a context whose positions have been
+    written again since, makes its own, also after a pass."""
+    import types
+
+    import torch
+
+    from clockwork_amd.engine.batch import StepContext
+    from clockwork_amd.parts import rope
+    from clockwork_amd.parts.model import DecoderModel
+    from clockwork_amd.parts.specs import RopeNeoxSpec
+
+    made = []
+    monkeypatch.setattr(rope.ops, "qkv_rope_rows_ok", lambda *a: True)
+    monkeypatch.setattr(rope.ops, "rope_angles", lambda positions, inv_freq: made.append(positions.clone()) or made[-1])
+    monkeypatch.setattr(rope.ops, "qkv_rope_rows", lambda x, w, b, angles, *a: angles)
+    part = rope.RopeNeox(RopeNeoxSpec(rotary_dim=64, theta=1e6))
+    part.bind({}, "cpu", torch.bfloat16)
+    ctx = StepContext()
+    ctx.positions = torch.arange(100, dtype=torch.int32)
+
+    def layer():
+        return part.project_rotate_store_rows(None, None, None, ctx, torch.zeros(100), 2, 1, 64, None, None)
+
+    assert torch.equal(layer(), ctx.positions)
+    ctx.positions += 100
+    assert torch.equal(layer(), ctx.positions) and len(made) == 2
+    # a model of two layers: one table, and nothing left of it
+    block = types.SimpleNamespace(forward=lambda *a: layer())
+    entries = [types.SimpleNamespace(layer=i, add_input=False, reenter=None) for i in range(2)]
+    model = types.SimpleNamespace(embedding=types.SimpleNamespace(forward=lambda ctx: None), own_caches=lambda: [], layers=[block, block],
+                                  spec=types.SimpleNamespace(run=entries), final_norm=None)
+    model._pass = types.MethodType(DecoderModel._pass, model)
+    DecoderModel.forward(model, ctx, [None, None])
+    assert len(made) == 3
+    ctx.positions += 100
+    assert torch.equal(layer(), ctx.positions) and len(made) == 4
