@@ -1,6 +1,9 @@
 """The HIP libraries: no execution path without them, and clear errors on the way to them."""
 
 import re
+import struct
+import subprocess
+from pathlib import Path
 
 import pytest
 
@@ -80,3 +83,77 @@ def test_no_limit_of_lds_follows_the_launches():
     older one: kernels whose launches differ in LDS are allowed their most at once."""
     for path in sorted(build.CSRC.glob("*.h*")):
         assert re.findall(r"\bstatic\s+(?!bool\b)\w+\s+raised\b.*", path.read_text()) == [], path.name
+
+
+LLVM = Path("/opt/rocm/llvm/bin")
+
+
+def _code_objects(path: Path):
+    """The ELF files for the GPU inside a built library."""
+    data, mark = path.read_bytes(), b"__CLANG_OFFLOAD_BUNDLE__"
+    at = data.find(mark)
+    while at >= 0:
+        (count,), entry = struct.unpack_from("<Q", data, at + len(mark)), at + len(mark) + 8
+        for _ in range(count):
+            offset, size, length = struct.unpack_from("<QQQ", data, entry)
+            if b"amdgcn" in data[entry + 24 : entry + 24 + length] and size:
+                yield data[at + offset : at + offset + size]
+            entry += 24 + length
+        at = data.find(mark, at + 1)
+
+
+def _llvm(tool: str, library: str, tmp_path, *options) -> str:
+    out = []
+    for i, code in enumerate(_code_objects(build.ensure_built(library))):
+        file = tmp_path / f"{library}{i}.co"
+        file.write_bytes(code)
+        out.append(subprocess.run([LLVM / tool, *options, file], capture_output=True, text=True, check=True).stdout)
+    assert out
+    return "\n".join(out)
+
+
+def _instructions(library: str, tmp_path, pattern: str) -> dict:
+    """Kernels whose names match -> their instructions in order."""
+    found = {}
+    for part in re.split(r"\n(?=[0-9a-f]+ <)", _llvm("llvm-objdump", library, tmp_path, "-d", "--no-show-raw-insn")):
+        head = re.match(r"[0-9a-f]+ <(\S+)>:", part)
+        if head and re.search(pattern, head.group(1)):
+            found[head.group(1)] = [line.split("//")[0].strip() for line in part.split("\n")[1:] if line.strip()]
+    return found
+
+
+def _registers(operands: str) -> set:
+    out = {(kind, n) for kind, first, last in re.findall(r"\b([av])\[(\d+):(\d+)\]", operands) for n in range(int(first), int(last) + 1)}
+    return out | {(kind, int(n)) for kind, n in re.findall(r"\b([av])(\d+)\b", operands)}
+
+
+def test_products_written_in_assembly_wait_for_their_operands(tmp_path):
+    """The compiler does not see that they are products. In the code as built: a tile's first ones begin with a zero of
+    their own; no vector instruction writes an operand less than two states before the product that reads it, and none
+    looks at a result less than twelve states behind the product that writes it (8 passes of 16 x 16 x 32)."""
+    kernels = _instructions("gemm_tile", tmp_path, r"gemm_wide_bf16_kernelILi\d+ELi8ELi9E")
+    assert len(kernels) >= 2
+    for name, code in kernels.items():
+        products = [i for i, x in enumerate(code) if x.startswith("v_mfma")]
+        assert sum(code[i].endswith(", 0") for i in products) == 72, name
+        for i in products:
+            result, *operands = code[i].split(None, 1)[1].split(", ")
+            written, read = _registers(result), set().union(*map(_registers, operands))
+            states = 0
+            for x in reversed(code[max(0, i - 4) : i]):
+                if states >= 2:
+                    break
+                if x.startswith("s_nop"):
+                    states += int(x.split()[1]) + 1
+                    continue
+                assert not (x.startswith("v_") and not x.startswith("v_mfma") and _registers(x.split(None, 1)[1].split(", ")[0]) & read), (name, x, code[i])
+                states += 1
+            states = 0
+            for x in code[i + 1 : i + 13]:
+                if states >= 12:
+                    break
+                if x.startswith("s_nop"):
+                    states += int(x.split()[1]) + 1
+                    continue
+                assert x.startswith(("s_", "v_mfma")) or not _registers(x) & written, (name, code[i], x)
+                states += 1
