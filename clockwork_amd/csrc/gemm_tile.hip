@@ -345,7 +345,7 @@ __device__ __forceinline__ bf16_t* pair_target(const WideArgs& a, int64_t m, int
 template <int MODE, int NB>
 __host__ __device__ __forceinline__ int wide_col(int ni, int r) {
   const int s = r >> 2, e = r & 3;
-  if (MODE == 2 || MODE == 4) {
+  if (MODE == 2) {
     const int s1 = s & 1;
     if (ni < (NB & ~3)) return (ni >> 2) * 32 + ((ni & 1) * 2 + s1) * 8 + ((ni >> 1) & 1) * 4 + e;
     if ((NB & 2) && ni < (NB & ~1)) return (NB & ~3) * 8 + ((ni & 1) * 2 + s1) * 4 + e;
@@ -354,24 +354,25 @@ __host__ __device__ __forceinline__ int wide_col(int ni, int r) {
   return ni < (NB & ~1) ? (ni >> 1) * 32 + s * 8 + (ni & 1) * 4 + e : ni * 16 + r;
 }
 
-// cw_gated from the bare exp2 and reciprocal instructions; KIND: which of them, W_GATE_ANY by ``act``
+// cw_gated from the bare exp2 and reciprocal instructions. A build of the kernel for each: asked for at every value the activation
+// took a fifth of 1600 rows' time with relu, asked for once a tile it took a copy of the tile's end for each, whose addresses
+// went to scratch in the widest tile. 17920 x 1536 with silu / relu / GELU / clipped, us: 2048 rows 92.5 / 99.7 / 106.5 / 107.7 with
+// three copies, 92.5 / 92.2 / 94.1 / 95.3 now; 1000 rows 49.4 / 52.0 / 56.2 / 56.6, now 49.3 / 48.2 / 49.6 / 50.0; 160 rows 22 throughout.
 #define W_GATE_SILU 0
 #define W_GATE_CLIPPED 1
 #define W_GATE_RELU 2
 #define W_GATE_GELU 3
-#define W_GATE_ANY 4
-__device__ __forceinline__ int w_gate_kind(float act) {
+static int w_gate(float act) {
   return act > 0.0f ? W_GATE_CLIPPED : act < -1.5f ? W_GATE_GELU : act < 0.0f ? W_GATE_RELU : W_GATE_SILU;
 }
-template <int KIND>
+template <int GATE>
 __device__ __forceinline__ float w_gated(float g, float up, float act) {
-  const int kind = KIND == W_GATE_ANY ? w_gate_kind(act) : KIND;
-  if (kind == W_GATE_CLIPPED) {
+  if (GATE == W_GATE_CLIPPED) {
     const float gl = fminf(g, act), ul = fminf(fmaxf(up, -act), act);
     return gl * __builtin_amdgcn_rcpf(1.0f + __expf(-1.702f * gl)) * (ul + 1.0f);
   }
-  if (kind == W_GATE_RELU) return fmaxf(g, 0.0f) * up;
-  if (kind == W_GATE_GELU) return g * __builtin_amdgcn_rcpf(1.0f + __expf(-1.5957691216057308f * (g + 0.044715f * g * g * g))) * up;
+  if (GATE == W_GATE_RELU) return fmaxf(g, 0.0f) * up;
+  if (GATE == W_GATE_GELU) return g * __builtin_amdgcn_rcpf(1.0f + __expf(-1.5957691216057308f * (g + 0.044715f * g * g * g))) * up;
   return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * up;
 }
 
@@ -386,10 +387,10 @@ __device__ __forceinline__ float w_gated(float g, float up, float act) {
     asm volatile("" ::: "memory"); \
   } while (0)
 
-template <int MODE, int MB, int NB, int SLOTS, bool ANY_ROWS = true, bool GROUPED = false>
+template <int MODE, int MB, int NB, int SLOTS, bool ANY_ROWS = true, bool GROUPED = false, int GATE = W_GATE_SILU>
 __global__ __launch_bounds__(256) void gemm_wide_bf16_kernel(WideArgs a) {
   extern __shared__ __align__(1024) unsigned char w_smem[];
-  constexpr bool GATED = MODE == 2 || MODE == 4;
+  constexpr bool GATED = MODE == 2;
   constexpr int BM = 32 * MB, BN = 32 * NB, PER = GATED ? BN / 2 : BN;  // PER: columns of the result
   constexpr int LOADS = MB + NB;                                            // of a wave and stage: MB of x, NB of W
   constexpr int STAGE = 4 * LOADS * W_BLOCK;
@@ -582,8 +583,9 @@ __global__ __launch_bounds__(256) void gemm_wide_bf16_kernel(WideArgs a) {
     // Rows of 16-byte multiples: buffer stores, whose descriptor ends with the last row and drops what is told to lie beyond, so
     // nothing branches at a store. (With branches the last tile of a row, 32 of 96 columns, took the 1.5B shape's product of 512
     // rows from 36 to 43 us.)
-    // ANY_ROWS: any other rows too, a value a store. (One kernel for both, with the activations besides, keeps so much alive that
-    // the widest tile's registers spill, 5 us a tile: it has neither.)
+    // ANY_ROWS: any other rows too, a value a store. (Two ends of a tile in one kernel keep so much alive that the widest tile's
+    // registers spill, and what comes back from scratch waits for the next tile's first loads, 5 us a tile: that tile takes whole
+    // rows only.)
     const bool whole = !ANY_ROWS || !(a.ldc & (16 / ELEMENT - 1)) && !((uintptr_t)a.C & 15) && !(out_cols & (16 / ELEMENT - 1)) && a.ldc < (1 << 20);
     const __amdgpu_buffer_rsrc_t cr = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(C + ((int64_t)tm * BM * a.ldc + tn * PER) * ELEMENT), 0,
@@ -618,15 +620,14 @@ __global__ __launch_bounds__(256) void gemm_wide_bf16_kernel(WideArgs a) {
     using Four = std::integral_constant<int, 4>;
     using Eight = std::integral_constant<int, 8>;
     if constexpr (GATED) {
-      auto all = [&](auto whole_c, auto kind_c) __attribute__((always_inline)) {
+      auto all = [&](auto whole_c) __attribute__((always_inline)) {
         constexpr bool whole_tile = decltype(whole_c)::value;
-        constexpr int KIND = decltype(kind_c)::value;
         // gates of two accumulators and the ups to them, each in one lane
         auto gated = [&](const f32x4_t& p, const f32x4_t& q, float* v) __attribute__((always_inline)) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const cw_u32x2_t gu = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[e]), __float_as_uint(q[e]), false, false);
-            v[e] = w_gated<KIND>(__uint_as_float(gu[0]), __uint_as_float(gu[1]), a.act);
+            v[e] = w_gated<GATE>(__uint_as_float(gu[0]), __uint_as_float(gu[1]), a.act);
           }
         };
 #pragma unroll
@@ -660,24 +661,8 @@ __global__ __launch_bounds__(256) void gemm_wide_bf16_kernel(WideArgs a) {
           }
         }
       };
-      using Silu = std::integral_constant<int, W_GATE_SILU>;
-      if constexpr (MODE == 2) {
-        if (whole) all(Yes{}, Silu{});
-        else if constexpr (ANY_ROWS) all(No{}, Silu{});
-      } else {
-        // which activation is asked once a tile, not for every value, and relu takes no exponential. 17920 x 1536 with relu / GELU, us,
-        // before and now: 1600 rows 106 / 110 and 93 / 95 (silu 93), 2048 rows 111 / 117 and 107 / 110, 160 rows 23.6 / 24.6 and 22.3 / 22.2
-        const int kind = w_gate_kind(a.act);
-        if (!whole) {
-          if constexpr (ANY_ROWS) all(No{}, std::integral_constant<int, W_GATE_ANY>{});
-        } else if (kind == W_GATE_RELU) {
-          all(Yes{}, std::integral_constant<int, W_GATE_RELU>{});
-        } else if (kind == W_GATE_GELU) {
-          all(Yes{}, std::integral_constant<int, W_GATE_GELU>{});
-        } else {
-          all(Yes{}, std::integral_constant<int, W_GATE_CLIPPED>{});
-        }
-      }
+      if (whole) all(Yes{});
+      else if constexpr (ANY_ROWS) all(No{});
     } else {
       auto all = [&](auto whole_c) __attribute__((always_inline)) {
         constexpr bool whole_tile = decltype(whole_c)::value;
@@ -776,13 +761,13 @@ CW_EXPORT int cw_gemm_bf16_wide_partial_ok(int M, int N, int K, int64_t ldx, int
 }
 
 // ``row_tiles``: GROUPED: how many there are at most
-template <int MODE, int MB, int NB, int SLOTS, bool ANY_ROWS = true, bool GROUPED = false>
+template <int MODE, int MB, int NB, int SLOTS, bool ANY_ROWS = true, bool GROUPED = false, int GATE = W_GATE_SILU>
 static int w_launch(WideArgs a, int row_tiles, int workgroups, hipStream_t stream) {
   constexpr int SMEM = SLOTS * 4 * (MB + NB) * W_BLOCK;
   static std::atomic<bool> allowed{false};
-  const int status = cw_allow_lds(allowed, (const void*)gemm_wide_bf16_kernel<MODE, MB, NB, SLOTS, ANY_ROWS, GROUPED>, SMEM);
+  const int status = cw_allow_lds(allowed, (const void*)gemm_wide_bf16_kernel<MODE, MB, NB, SLOTS, ANY_ROWS, GROUPED, GATE>, SMEM);
   if (status != CW_OK) return status;
-  constexpr bool gated = MODE == 2 || MODE == 4;
+  constexpr bool gated = MODE == 2;
   const int out_cols = gated ? a.N / 2 : a.N, per_tile = gated ? 16 * NB : 32 * NB;
   a.tiles_n = (out_cols + per_tile - 1) / per_tile;
   a.tiles_m = GROUPED ? 0 : (a.M + 32 * MB - 1) / (32 * MB);  // GROUPED: read on the device
@@ -791,7 +776,7 @@ static int w_launch(WideArgs a, int row_tiles, int workgroups, hipStream_t strea
   // a multiple of 8 workgroups, so that every XCD gets the same number of them
   int grid = total < workgroups ? (int)total : workgroups;
   grid = (grid + 7) & ~7;
-  hipLaunchKernelGGL((gemm_wide_bf16_kernel<MODE, MB, NB, SLOTS, ANY_ROWS, GROUPED>), dim3(grid), dim3(256), SMEM, stream, a);
+  hipLaunchKernelGGL((gemm_wide_bf16_kernel<MODE, MB, NB, SLOTS, ANY_ROWS, GROUPED, GATE>), dim3(grid), dim3(256), SMEM, stream, a);
   return cw_launch_status();
 }
 
@@ -848,12 +833,16 @@ static int tile_choice(int mode, int M, int N, int K, int most_planes, bool wide
 // The product by the tile of bm x bn (128 x 128 and 256 x 192 for rows of any length, the others for whole ones: 16-byte
 // multiples), if there is such a tile for the mode.
 static int w_by_tile(int mode, int bm, int bn, bool whole, const WideArgs& a, int workgroups, hipStream_t stream) {
-  const int kind = mode == 2 && a.act != 0.0f ? 4 : mode;
-#define CW_WIDE(MODE_, MB_, NB_, SLOTS_, ANY_)                                     \
-  if (kind == MODE_ && bm == 32 * MB_ && bn == 32 * NB_ && (whole || ANY_)) return w_launch<MODE_, MB_, NB_, SLOTS_, ANY_>(a, 0, workgroups, stream)
-#define CW_WIDE_GATED(MB_, NB_, SLOTS_, ANY_) \
-  CW_WIDE(2, MB_, NB_, SLOTS_, ANY_);         \
-  CW_WIDE(4, MB_, NB_, SLOTS_, ANY_)
+  const int gate = mode == 2 ? w_gate(a.act) : W_GATE_SILU;
+#define CW_WIDE_GATE(MODE_, MB_, NB_, SLOTS_, ANY_, GATE_)                                                 \
+  if (mode == MODE_ && gate == GATE_ && bm == 32 * MB_ && bn == 32 * NB_ && (whole || ANY_))               \
+  return w_launch<MODE_, MB_, NB_, SLOTS_, ANY_, false, GATE_>(a, 0, workgroups, stream)
+#define CW_WIDE(MODE_, MB_, NB_, SLOTS_, ANY_) CW_WIDE_GATE(MODE_, MB_, NB_, SLOTS_, ANY_, W_GATE_SILU)
+#define CW_WIDE_GATED(MB_, NB_, SLOTS_, ANY_)               \
+  CW_WIDE(2, MB_, NB_, SLOTS_, ANY_);                       \
+  CW_WIDE_GATE(2, MB_, NB_, SLOTS_, ANY_, W_GATE_CLIPPED);  \
+  CW_WIDE_GATE(2, MB_, NB_, SLOTS_, ANY_, W_GATE_RELU);     \
+  CW_WIDE_GATE(2, MB_, NB_, SLOTS_, ANY_, W_GATE_GELU)
   CW_WIDE(0, 3, 3, 6, false);
   CW_WIDE(0, 4, 3, 5, false);
   CW_WIDE(0, 4, 4, 5, true);
@@ -878,6 +867,7 @@ static int w_by_tile(int mode, int bm, int bn, bool whole, const WideArgs& a, in
   CW_WIDE(3, 8, 6, 2, true);
 #undef CW_WIDE_GATED
 #undef CW_WIDE
+#undef CW_WIDE_GATE
   return CW_ERR_ARG;
 }
 
@@ -941,7 +931,7 @@ CW_EXPORT int cw_gemm_bf16_wide_grouped(int mode, const void* X, int64_t ldx, co
              tile_group, n_row_tiles, row_target, row_factor, w_group_stride, act};
   if (mode == 0) return w_launch<0, 8, 6, 2, true, true>(a, max_row_tiles, workgroups, stream);
   return act == 0.0f ? w_launch<2, 8, 6, 2, true, true>(a, max_row_tiles, workgroups, stream)
-                     : w_launch<4, 8, 6, 2, true, true>(a, max_row_tiles, workgroups, stream);
+                     : w_launch<2, 8, 6, 2, true, true, W_GATE_CLIPPED>(a, max_row_tiles, workgroups, stream);
 }
 
 // rows of a tile of cw_gemm_bf16_wide_grouped

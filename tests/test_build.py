@@ -157,3 +157,13 @@ def test_products_written_in_assembly_wait_for_their_operands(tmp_path):
                     continue
                 assert x.startswith(("s_", "v_mfma")) or not _registers(x) & written, (name, code[i], x)
                 states += 1
+
+
+def test_the_wide_tiles_keep_everything_in_registers(tmp_path):
+    """What a tile's end fetches back from scratch waits for the loads of the next tile that are in flight."""
+    kernels = re.split(r"\n\s+- \.agpr_count", _llvm("llvm-readelf", "gemm_tile", tmp_path, "--notes"))[1:]
+    wide = [k for k in kernels if "gemm_wide_bf16_kernel" in k]
+    assert len(wide) > 30
+    for kernel in wide:
+        found = dict(re.findall(r"\.(name|vgpr_spill_count|private_segment_fixed_size):\s+(\S+)", kernel))
+        assert found["vgpr_spill_count"] == found["private_segment_fixed_size"] == "0", found
