@@ -212,9 +212,10 @@ WIDE_TILES = {0: [(96, 96), (128, 96), (160, 128), (192, 160), (256, 160), (256,
               3: [(96, 96), (160, 128), (192, 160), (192, 192), (256, 128), (256, 192)]}
 
 
-# one row tile with few rows and fewer stages than slots; rows and columns that end inside a tile; several tiles a workgroup
+# one row tile with few rows and fewer stages than slots; rows and columns that end inside a tile; more tiles than one for each of 256
+# workgroups, 264 of the widest: the next tile's first loads beside this one's end
 @pytest.mark.parametrize("mode,bm,bn", [(mode, *t) for mode, tiles in WIDE_TILES.items() for t in tiles])
-@pytest.mark.parametrize("M,N,K", [(1, 16, 256), (65, 48, 64), (321, 1168, 640), (2048, 5168, 320)])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 256), (65, 48, 64), (321, 1168, 640), (2048, 5168, 320), (2048, 9504, 256)])
 def test_tiles_of_the_wide_kernel(mode, bm, bn, M, N, K):
     from clockwork_amd import ops
 
@@ -231,7 +232,8 @@ def test_tiles_of_the_wide_kernel(mode, bm, bn, M, N, K):
     elif mode == 2:
         g, u = want[:, : N // 2], want[:, N // 2:]
         for limit, ref in {0.0: torch.nn.functional.silu(g) * u, ops.RELU_GATE: torch.relu(g) * u,
-                           ops.GELU_GATE: torch.nn.functional.gelu(g, approximate="tanh") * u}.items():
+                           ops.GELU_GATE: torch.nn.functional.gelu(g, approximate="tanh") * u,
+                           0.5: torch.clamp(g, max=0.5) * torch.sigmoid(1.702 * torch.clamp(g, max=0.5)) * (torch.clamp(u, -0.5, 0.5) + 1.0)}.items():
             torch.testing.assert_close(ops.linear_mid(x, w, one, swiglu=True, limit=limit).float(), ref, **bf16)
     else:
         for planes in (p for p in (1, 3, 5) if p <= K // 64):
