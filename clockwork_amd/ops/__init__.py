@@ -596,14 +596,14 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias=None, out_dtype=None, par
                    "gemm_bf16_skinny")
             return out
     plain = M > STREAM_MAX_ROWS and out_dtype is None and (bias is None or bias.dtype == torch.bfloat16 and tuple(bias.shape) == (N,))
+    if partial_ok and out_dtype is None and bias is None and M >= WIDE_PRODUCT_MIN_ROWS and x.is_contiguous():
+        splits = _wide_partial_chosen(x, weight, policy, portions_partial_ok)
+        if splits:
+            return linear_wide_partial(x, weight, splits)
     if plain and portions_partial_ok and bias is None:
         choice = _mid_choice(3, x, weight, policy)
         if choice:
             return linear_mid(x, weight, choice, partial=True)
-    if partial_ok and out_dtype is None and bias is None and M >= WIDE_PRODUCT_MIN_ROWS and x.is_contiguous():
-        splits = _wide_partial_chosen(x, weight, policy)
-        if splits:
-            return linear_wide_partial(x, weight, splits)
     if plain:
         choice = _mid_choice(0, x, weight, policy, bias=bias)
         if choice:
@@ -659,7 +659,7 @@ class ProductPolicy:
     (N, K) whose product of few rows is summed in parts over K (a narrow output with a long K),
     the number of parts that start-up found the fastest, the same for every step of up to 16 rows.
     ``wide_partial_choices``: for an (N, K) of a long portion's product with a narrow output and a
-    long K, into how many runs of K the wide-tile kernel sums it (0: the library's product stays).
+    long K, into how many runs of K tiles of 256 x 192 sum it (0: the rule's tiles, or the library's product, were faster).
     ``mid_choices``: for a product of so many rows that the tiles between would serve by their rule ((mode, rows, N, K), the
     activation behind it as in ``swiglu_choices``), whether they were as fast as the library's tuned product.
     ``tuning``: such a start-up is under way (``library_tuning``)."""
@@ -1008,15 +1008,23 @@ def _aligned(*tensors) -> bool:
     return all(t.data_ptr() % 16 == 0 for t in tensors)
 
 
-def _mid_choice(mode: int, x: torch.Tensor, weight: torch.Tensor, policy: ProductPolicy, bias=None, limit: float = 0.0) -> int:
-    """What ``cw_gemm_bf16_wide_choice`` and, for rows of other lengths, ``cw_gemm_bf16_mid_choice`` say of x @ weight.T; 0 for operands that their kernels do not take, and where a tuning
-    start-up has timed this very number of rows and found the library's tuned product the faster one."""
+def _tile_rule(mode: int, x: torch.Tensor, weight: torch.Tensor) -> int:
+    """What ``cw_gemm_bf16_wide_choice`` and, for rows of other lengths, ``cw_gemm_bf16_mid_choice`` say of x @ weight.T; 0 for
+    operands that their kernels do not take."""
     if not _aligned(x, weight):
         return 0
     M, K = x.shape
     N = weight.shape[0]
     lib, units = _load("gemm_tile"), _compute_units(x.device)
-    choice = lib.cw_gemm_bf16_wide_choice(mode, M, N, K, K, units) or lib.cw_gemm_bf16_mid_choice(mode, M, N, K, K, units)
+    return lib.cw_gemm_bf16_wide_choice(mode, M, N, K, K, units) or lib.cw_gemm_bf16_mid_choice(mode, M, N, K, K, units)
+
+
+def _mid_choice(mode: int, x: torch.Tensor, weight: torch.Tensor, policy: ProductPolicy, bias=None, limit: float = 0.0) -> int:
+    """What ``_tile_rule`` says of x @ weight.T; 0 where a tuning start-up has timed this very number of rows and found the
+    library's tuned product the faster one."""
+    choice = _tile_rule(mode, x, weight)
+    M, K = x.shape
+    N = weight.shape[0]
     if choice and (policy.tuning or policy.mid_choices):
         key = (mode, M, *_swiglu_key(N, K, limit))
         if policy.tuning and key not in policy.mid_choices and policy.recall("mid_choices", key) is None:
@@ -1075,11 +1083,11 @@ WIDE_PARTIAL_MAX_TILES = 128
 WIDE_PARTIAL_MIN_K = 1024
 
 
-def _wide_partial_chosen(x: torch.Tensor, weight: torch.Tensor, policy: ProductPolicy) -> int:
-    """Into how many runs of K does the wide-tile kernel sum this product of many rows (0: it
-    does not, the library's product runs)? Only what a tuning start-up has measured on these very
-    shapes: the kernel's partial sums and the norm that adds them against the library's product and
-    the norm of its bfloat16 result."""
+def _wide_partial_chosen(x: torch.Tensor, weight: torch.Tensor, policy: ProductPolicy, rule_allowed: bool = False) -> int:
+    """Into how many runs of K do tiles of 256 x 192 sum this product of many rows (0: they do not)? Only what a tuning
+    start-up has measured on these very shapes: the kernel's partial sums and the norm that adds them against the library's
+    product and the norm of its bfloat16 result and, where the reader takes them (``rule_allowed``), against the tiles and
+    runs that the rule names."""
     M, K = x.shape
     N = weight.shape[0]
     key = (N, K)
@@ -1095,6 +1103,9 @@ def _wide_partial_chosen(x: torch.Tensor, weight: torch.Tensor, policy: ProductP
             norm_weight = torch.ones(N, dtype=torch.bfloat16, device=x.device)
             out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
             best = _timed_us(lambda: add_rmsnorm(resid, _library_product(x, weight, None), norm_weight, 1e-6, out, write_back=False))
+            rule = _tile_rule(3, x, weight) if rule_allowed else 0
+            if rule:
+                best = min(best, _timed_us(lambda: add_rmsnorm(resid, linear_mid(x, weight, rule, partial=True), norm_weight, 1e-6, out, write_back=False)))
             for splits in (2, 3, 4, 5, 6, 7, 8):
                 if not lib.cw_gemm_bf16_wide_partial_ok(M, N, K, K, splits):
                     continue

@@ -125,3 +125,32 @@ def test_the_tiles_between_leave_a_product_that_was_timed_to_the_library(monkeyp
     assert later.read_choices(path) == 2 and ops._mid_choice(0, rows[128], weight, later) == by_rule   # (not in use before it asks)
     later.tuning = True
     assert ops._mid_choice(0, rows[128], weight, later) == 0 and len(timed) == 2
+
+
+def test_runs_of_k_that_a_start_up_timed_come_before_the_rules_tiles(monkeypatch):
+    """A long portion's product with a timed (N, K): the timed runs, or what the rule names where they were not the fastest;
+    and they are timed against that as well as against the library."""
+    M, N, K = 1024, 1536, 8960
+    x, w = torch.zeros(M, K, dtype=torch.bfloat16), torch.zeros(N, K, dtype=torch.bfloat16)
+    costs = {"library": 50.0, "tiles": 40.0}
+    monkeypatch.setattr(ops, "_gpu", lambda *a: None)
+    monkeypatch.setattr(ops, "_compute_units", lambda device: 256)
+    monkeypatch.setattr(ops, "_library_product", lambda *a: "library")
+    monkeypatch.setattr(ops, "linear_mid", lambda *a, **k: "tiles")
+    monkeypatch.setattr(ops, "linear_wide_partial", lambda x, w, runs: runs)
+    monkeypatch.setattr(ops, "add_rmsnorm", lambda resid, y, *a, **k: y)
+    monkeypatch.setattr(ops, "_timed_us", lambda fn: costs.get(fn(), 45.0))
+    run = lambda policy: ops.linear(x, w, partial_ok=True, portions_partial_ok=True, policy=policy)  # noqa: E731
+    policy = ops.ProductPolicy()
+    assert run(policy) == "tiles"
+    policy.wide_partial_choices[(N, K)] = 3
+    assert run(policy) == 3
+    policy.wide_partial_choices[(N, K)] = 0
+    assert run(policy) == "tiles"
+    for four, want in ((45.0, "tiles"), (39.5, "tiles"), (30.0, 4)):
+        costs[4] = four
+        policy = ops.ProductPolicy()
+        policy.tuning = True
+        assert run(policy) == want
+        policy.tuning = False
+        assert run(policy) == want and policy.wide_partial_choices[(N, K)] == (4 if want == 4 else 0)
