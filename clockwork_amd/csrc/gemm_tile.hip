@@ -1183,8 +1183,8 @@ CW_EXPORT int cw_gemm_bf16_mid(int mode, const void* X, int64_t ldx, const void*
 }
 
 // Which of this file's kernels a product of many rows should run on: 0 the library's, else bm | bn << 10 |
-// planes << 20 (cw_gemm_bf16_mid; mode as there), by the table of tiles above. For rows of 16-byte multiples; of others
-// cw_gemm_bf16_mid_choice is asked.
+// planes << 20 (cw_gemm_bf16_mid; mode as there), by the table of tiles above. For results in rows of 16-byte multiples; for
+// others, of which nothing is named here, cw_gemm_bf16_mid_choice is there.
 // Where the lines lie, measured with operands from memory, 72 to 2048 rows (us, library -> here):
 //  * mode 3 (a sum that the next norm adds up; times with that norm): K of two and a half times N and more, everywhere (1.5B
 //    shape's down product, 72 rows 25.3 -> 15.3, 336 rows 40.3 -> 23.6, 1000 rows 55.8 -> 41.7, 2048 rows 83.3 -> 68.0; 7B
@@ -1202,6 +1202,12 @@ CW_EXPORT int cw_gemm_bf16_mid(int mode, const void* X, int64_t ldx, const void*
 //    for 1536 columns and more from 0.5 M outputs on (q/k/v of the 1.5B shape, 160 rows 8.1 -> 8.4, 336 rows 9.4 -> 8.7, 2048 rows 18.3
 //    -> 17.8; its output product, 2048 rows 17.4 -> 14.3; 4640 columns, 100 rows 11.6 -> 11.7, 128 rows 16.8 -> 12.0, 2048 rows 38.5 -> 31.6); up to
 //    4096 for 2048 columns and more from 1.6 M on (4608 x 3584, 512 rows 34.4 -> 27.7, 1000 rows 47.0 -> 37.4; 3584 x 3584, 384 rows 23.1 -> 27.9).
+//    Beyond 8192 columns, and for the few outputs of 320 rows and more with a K of 1536 that are no 0.5 M, the 64 x 64 tiles by
+//    their own lines (whole_sums_in_small_tiles): 8704 x 512, 72 rows 8.0 -> 5.9, 400 rows 12.4 -> 10.9; 16384 x 512, 160 rows 12.5 -> 10.8;
+//    9728 x 896, 72 rows 11.9 -> 9.8, 160 rows 13.1 -> 11.1; 1536 x 1536, 325 rows 8.9 -> 8.3. From 512 tiles on with a K of more than
+//    512 they lose as often as they win (9728 x 896, 256 rows 15.5 -> 16.3, 12288 x 896, 160 rows 13.3 -> 15.4; 9728 x 640, 256 rows
+//    15.0 -> 13.3, 320 rows 14.3 -> 13.1); which, the number of tiles does not tell.
+static int whole_sums_in_small_tiles(int M, int N, int K);
 CW_EXPORT int cw_gemm_bf16_wide_choice(int mode, int M, int N, int K, int64_t ldx, int cus) {
   if (M <= 64 || M > 2048 || N <= 0 || K < 256 || (K & 63) || (ldx & 7) || ldx < K || cus < 8) return 0;
   if ((int64_t)N * K * 2 >= (1ll << 32) || ((int64_t)M * ldx + 128 * ldx) * 2 >= (1ll << 32)) return 0;
@@ -1209,7 +1215,7 @@ CW_EXPORT int cw_gemm_bf16_wide_choice(int mode, int M, int N, int K, int64_t ld
   const int64_t elements = (int64_t)N * K, outputs = (int64_t)M * N;
   if (mode == 0) {
     const bool here = K <= 512 ? N >= 32 : K <= 896 ? N >= 896 : K <= 1536 ? N >= 1536 && outputs >= 500000 : K <= 4096 && N >= 2048 && outputs >= 1600000;
-    if (!here || N > 8192) return 0;
+    if (!here || N > 8192) return whole_sums_in_small_tiles(M, N, K);
   } else if (mode == 2) {
     if ((N & 1) || (N < 2 * K && K > 1024) || elements > 136000000) return 0;
   } else if (mode == 3) {
@@ -1257,16 +1263,18 @@ static float mid_time(int M, int N, int K, int bm, int bn, int planes, int cus) 
 //    6.4 for 144 rows; 512 columns 5.3 -> 6.1), while a compute unit has three tiles or so (4096 x 896, 400 rows 10.6 ->
 //    8.4, 700 rows 11.3 -> 12.1); and K up to 1536 for 1536 columns and more, 320 to 1024 rows (q/k/v of the 1.5B shape
 //    14.0 -> 12.7 for 1000, 8.6 -> 8.8 for 144).
+static int whole_sums_in_small_tiles(int M, int N, int K) {
+  const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
+  const bool short_k = M <= 1536 && N >= 32 && (K <= 512 || (K <= 896 && N >= 1024)) && tiles <= 1000 && tiles * K <= 600000;
+  const bool qkv = K > 896 && K <= 1536 && N >= 1536 && (int64_t)N * K <= 4 << 20 && M >= 320 && M <= 1024;
+  return short_k || qkv ? 64 | 64 << 10 | 1 << 20 : 0;
+}
+
 CW_EXPORT int cw_gemm_bf16_mid_choice(int mode, int M, int N, int K, int64_t ldx, int cus) {
   if (M <= 64 || M > 2048 || N <= 0 || K < 256 || (K & 63) || (ldx & 7) || ldx < K || cus < 8) return 0;
   if ((int64_t)N * K * 2 >= (1ll << 32) || ((int64_t)M * ldx + 128 * ldx) * 2 >= (1ll << 32)) return 0;
   const int64_t elements = (int64_t)N * K, outputs = (int64_t)M * N;
-  if (mode == 0) {
-    const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
-    const bool short_k = M <= 1536 && N >= 32 && (K <= 512 || (K <= 896 && N >= 1024)) && tiles <= 1000 && tiles * K <= 600000;
-    const bool qkv = K > 896 && K <= 1536 && N >= 1536 && elements <= 4 << 20 && M >= 320 && M <= 1024;
-    return short_k || qkv ? 64 | 64 << 10 | 1 << 20 : 0;
-  }
+  if (mode == 0) return whole_sums_in_small_tiles(M, N, K);
   if (mode == 2) {
     if ((N & 1) || (N < 2 * K && K > 1024) || !((int64_t)M * elements <= 4500000000ll || (elements <= 9 << 20 && M <= 640))) return 0;
   } else if (mode == 3) {

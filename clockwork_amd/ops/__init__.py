@@ -1009,14 +1009,15 @@ def _aligned(*tensors) -> bool:
 
 
 def _tile_rule(mode: int, x: torch.Tensor, weight: torch.Tensor) -> int:
-    """What ``cw_gemm_bf16_wide_choice`` and, for rows of other lengths, ``cw_gemm_bf16_mid_choice`` say of x @ weight.T; 0 for
-    operands that their kernels do not take."""
+    """What ``cw_gemm_bf16_wide_choice`` says of x @ weight.T or, if the results' rows are no multiples of 16 bytes,
+    ``cw_gemm_bf16_mid_choice``; 0 for operands that their kernels do not take."""
     if not _aligned(x, weight):
         return 0
     M, K = x.shape
     N = weight.shape[0]
     lib, units = _load("gemm_tile"), _compute_units(x.device)
-    return lib.cw_gemm_bf16_wide_choice(mode, M, N, K, K, units) or lib.cw_gemm_bf16_mid_choice(mode, M, N, K, K, units)
+    whole = N % {0: 8, 2: 16, 3: 4}[mode] == 0
+    return (lib.cw_gemm_bf16_wide_choice if whole else lib.cw_gemm_bf16_mid_choice)(mode, M, N, K, K, units)
 
 
 def _mid_choice(mode: int, x: torch.Tensor, weight: torch.Tensor, policy: ProductPolicy, bias=None, limit: float = 0.0) -> int:

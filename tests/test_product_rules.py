@@ -242,3 +242,22 @@ def test_a_table_of_angles_is_kept_for_a_pass_over_the_model_only(monkeypatch):
     assert len(made) == 3
     ctx.positions += 100
     assert torch.equal(layer(), ctx.positions) and len(made) == 4
+
+
+@pytest.mark.parametrize("mode,M,N,K,there", [
+    # whole rows: many columns and few outputs of a middling K are the narrow tiles' by lines of their own
+    (0, 72, 8704, 512, True), (0, 400, 8704, 512, True), (0, 512, 8704, 512, False), (0, 160, 9728, 896, True), (0, 320, 9728, 896, False),
+    (0, 322, 1536, 1536, True), (0, 319, 1536, 1536, False), (0, 2048, 2048, 1536, True),
+    # rows that end inside 16 bytes
+    (0, 300, 4097, 896, True), (2, 160, 8008, 640, True), (3, 144, 1538, 8960, True), (0, 300, 9729, 1536, False)])
+def test_one_rule_names_the_tiles_of_a_product(monkeypatch, mode, M, N, K, there):
+    """What the engine asks: for whole rows ``cw_gemm_bf16_wide_choice`` alone, for others ``cw_gemm_bf16_mid_choice`` alone."""
+    import torch
+
+    monkeypatch.setattr(ops, "_compute_units", lambda device: CUS)
+    code = ops._tile_rule(mode, torch.empty(M, K, dtype=torch.bfloat16), torch.empty(N, K, dtype=torch.bfloat16))
+    whole = N % {0: 8, 2: 16, 3: 4}[mode] == 0
+    assert ((code & 1023, code >> 10 & 1023, code >> 20) if code else None) == (_wide_choice if whole else _choice)(mode, M, N, K)
+    assert (code != 0) == there
+    if whole and there and not (N <= 8192 and M * N >= 500000):
+        assert code == 64 | 64 << 10 | 1 << 20
