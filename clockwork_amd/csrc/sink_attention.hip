@@ -274,6 +274,7 @@ CW_EXPORT int cw_sink_attention(int dtype, const void* q, int64_t q_stride, void
 //   merge:   the runs' partial outputs are added in order.
 // ======================================================================================
 #define SD_MAX_SK 128
+#define SD_BESIDE_LDS (158 * 1024)  // of a launch of runs beside a recurrence, the most (150 KB and 88 KB are the most of either)
 #define SD_HG 16      // query heads of a group that a thread handles at a time
 
 struct SinkDecodeParams {
@@ -864,8 +865,9 @@ CW_EXPORT int cw_sink_decode_supported(int heads, int kv_heads, int dim, int vdi
   return a <= 150 * 1024 && b <= 150 * 1024 ? 1 : 0;
 }
 
-// Can a recurrence go beside these runs (cw_sink_decode_beside)? bfloat16, two kernels, five to eight heads of a group and
-// up to 16 mixed ones.
+// Can a recurrence go beside these runs (cw_sink_decode_beside)? bfloat16, two kernels, five to eight heads of a group and nine to
+// 16 mixed ones: what the runs' build for 8 and 16 heads at a time serves, the only one that there is with a recurrence behind it
+// (each takes the compiler two kernels more; no other number of heads has been measured). Others go as launches of their own.
 CW_EXPORT int cw_sink_decode_beside_ok(int dtype, int n_runs, int heads, int kv_heads, int mixed) {
   if (dtype != CW_BF16 || heads <= 0 || kv_heads <= 0 || heads % kv_heads || !sd_two(n_runs, heads, kv_heads, mixed != 0)) return 0;
   const int group = heads / kv_heads;
@@ -916,12 +918,12 @@ CW_EXPORT int cw_sink_decode_beside(int dtype, const void* q, int64_t q_stride, 
       const RecurrenceLaunch& l = *(const RecurrenceLaunch*)beside;
       const size_t both = lds > (size_t)l.lds ? lds : (size_t)l.lds;
       const int64_t run_blocks = (int64_t)n_requests * n_runs, blocks = run_blocks + (int64_t)l.requests * l.p.heads;
-      if (blocks > 0x7fffffff) return CW_ERR_SIZE;
+      if (blocks > 0x7fffffff || both > SD_BESIDE_LDS) return CW_ERR_SIZE;
 #define CW_BESIDE(HS_, HV_, RPT_)                                                                                      \
   do {                                                                                                                 \
-    if (both > 48 * 1024 && hipFuncSetAttribute((const void*)sink_decode_runs_beside_kernel<HS_, HV_, RPT_>,           \
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)both) != hipSuccess)  \
-      return CW_ERR_LAUNCH;                                                                                            \
+    static std::atomic<bool> allowed{false};                                                                           \
+    const int status = cw_allow_lds(allowed, (const void*)sink_decode_runs_beside_kernel<HS_, HV_, RPT_>, SD_BESIDE_LDS); \
+    if (status != CW_OK) return status;                                                                                \
     if (mlds > 48 * 1024 && hipFuncSetAttribute((const void*)sink_decode_mix_kernel<bf16_t>,                           \
                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)mlds) != hipSuccess)  \
       return CW_ERR_LAUNCH;                                                                                            \
