@@ -813,13 +813,17 @@ static float tile_time(const TileRate& t, int mode, int M, int N, int K, int pla
   return time + (mode == 3 ? 1.8e-6f * (float)planes * (float)M * (float)N : 0.0f);
 }
 
-// The tile and the number of runs of K that take the least time; ``wide_only``: of the wide-tile kernel's.
+// The tile and the number of runs of K that take the least time; ``wide_only``: of the wide-tile kernel's. A long K of many rows is
+// summed whole by tiles of 192 x 160 and more only: smaller ones have all units ask L2 for more than the 12 TB/s that it gives
+// them, which a tile's cost does not know (7B shape's down product and norm, us: 1280 rows 199 by 160 x 128, 173 by 192 x 160 in three runs;
+// 2048 rows 236 by 192 x 160, 251 in two runs).
 static int tile_choice(int mode, int M, int N, int K, int most_planes, bool wide_only, bool whole, int cus) {
   int best = 0;
   float least = 0.0f;
   for (const TileRate& t : TILE_RATES) {
     if (!(t.modes & (mode == 0 ? 1 : mode == 2 ? 2 : 4)) || (wide_only && t.bm == 64) || !(whole || (t.modes & 8))) continue;
     for (int planes = 1; planes <= most_planes && (planes == 1 || K / planes >= 256); ++planes) {
+      if (mode == 3 && planes == 1 && M > 640 && N >= 512 && K >= 3 * N && t.bm + t.bn < 352) continue;
       const float time = tile_time(t, mode, M, N, K, planes, cus);
       if (best == 0 || time < least) {
         least = time;

@@ -261,3 +261,12 @@ def test_one_rule_names_the_tiles_of_a_product(monkeypatch, mode, M, N, K, there
     assert (code != 0) == there
     if whole and there and not (N <= 8192 and M * N >= 500000):
         assert code == 64 | 64 << 10 | 1 << 20
+
+
+def test_long_sums_of_many_rows_are_whole_on_large_tiles_only():
+    """Smaller ones ask L2 for more than it gives (7B shape's down product, 1280 rows 199 us by 160 x 128, 173 in runs)."""
+    for M in range(641, 2049, 7):
+        for N, K in ((3584, 18944), (2048, 11008), (4096, 14336), (5120, 27648)):
+            choice = _wide_choice(3, M, N, K)
+            assert choice is None or choice[2] > 1 or choice[0] + choice[1] >= 352
+    assert _wide_choice(3, 1280, 3584, 18944) == (192, 160, 3) and _wide_choice(3, 2048, 3584, 18944) == (192, 160, 1)
