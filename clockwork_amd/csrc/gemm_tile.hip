@@ -781,17 +781,18 @@ static int w_launch(WideArgs a, int row_tiles, int workgroups, hipStream_t strea
 }
 
 // What a tile costs: ``fixed`` us of a work item and stage[q - 1] us a stage of 64 elements of K while q workgroups share a
-// compute unit (the smallest tiles; the others have one to themselves). Fits over 3600 timings with operands from memory, 72 to
-// 2048 rows of 26 shapes of the 0.5B to 14B models' layers and others (N 512 to 37888, K 512 to 18944), off by 9 % in the
-// mean; what the rule names by them takes 1.5 % more than the fastest tile and number of runs, 11 % at worst (192 rows of the
-// 1.5B shape's gate/up product 24.6 us, 21.5 by 160 x 160). A stage of the large tiles goes with BM + BN, 2.3 ns a row: its
+// compute unit (the smallest tiles; the others have one to themselves). Fits over timings with operands from memory, 72 to
+// 2048 rows of 26 shapes of the 0.5B to 14B models' layers and others (N 512 to 37888, K 512 to 18944); the fixed cost of 64 x 128
+// after another 22000, 65 to 2048 rows of 38 shapes. Over those a tile's time (and a launch's beside) is off by 7 % in the mean;
+// a tile that the rule names takes 1 to 1.6 % more than the fastest, the library among them, 24 % at worst (272 rows of 6144 x 1536 with
+// a gate 18.4 by 160 x 96, 14.9 by 128 x 128; 704 rows of 1024 x 4096 and a norm 20.9, 17.9 by 96 x 96). A stage of the large tiles goes with BM + BN, 2.3 ns a row: its
 // loads; 256 x 192 and 256 x 288 have two stages of them in LDS and wait longer, and gain by their few rounds.
 struct TileRate {
   int bm, bn, modes, per_unit;  // modes: a bit each of 0, 2 and 3 (1, 2, 4); 8: rows of any length
   float fixed, stage[3];
 };
 static const TileRate TILE_RATES[] = {
-    {64, 64, 15, 3, -1.63f, {0.342f, 0.556f, 0.809f}}, {64, 128, 12, 2, -1.26f, {0.475f, 0.835f}}, {96, 96, 5, 1, 0.12f, {0.399f}},
+    {64, 64, 15, 3, -1.63f, {0.342f, 0.556f, 0.809f}}, {64, 128, 12, 2, -0.9f, {0.475f, 0.835f}}, {96, 96, 5, 1, 0.12f, {0.399f}},
     {128, 96, 1, 1, 0.29f, {0.451f}},                  {128, 128, 12, 1, 0.34f, {0.592f}},        {160, 96, 2, 1, 0.53f, {0.507f}},
     {160, 128, 7, 1, 0.79f, {0.594f}},                 {160, 160, 2, 1, 1.39f, {0.686f}},         {192, 160, 7, 1, 1.48f, {0.782f}},
     {192, 192, 6, 1, 2.42f, {0.870f}},                 {256, 128, 4, 1, 1.62f, {0.803f}},         {256, 160, 1, 1, 3.59f, {0.898f}},
