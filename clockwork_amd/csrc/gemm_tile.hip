@@ -1206,7 +1206,8 @@ CW_EXPORT int cw_gemm_bf16_mid(int mode, const void* X, int64_t ldx, const void*
 //    for 896 columns and more (q/k/v of the 0.5B shape 7.9 -> 6.1 for 160 rows, 11.0 -> 9.4 for 2048; 512 columns 5.3 -> 6.1); up to 1536
 //    for 1536 columns and more from 0.5 M outputs on (q/k/v of the 1.5B shape, 160 rows 8.1 -> 8.4, 336 rows 9.4 -> 8.7, 2048 rows 18.3
 //    -> 17.8; its output product, 2048 rows 17.4 -> 14.3; 4640 columns, 100 rows 11.6 -> 11.7, 128 rows 16.8 -> 12.0, 2048 rows 38.5 -> 31.6); up to
-//    4096 for 2048 columns and more from 1.6 M on (4608 x 3584, 512 rows 34.4 -> 27.7, 1000 rows 47.0 -> 37.4; 3584 x 3584, 384 rows 23.1 -> 27.9).
+//    4096 for 2048 columns and more from 1.6 M on (4608 x 3584, 512 rows 34.4 -> 27.7, 1000 rows 47.0 -> 37.4; 3584 x 3584, 384 rows 23.1 -> 27.9),
+//    with a K of more than 2048 up to 9.5 M (6144 x 3072, 1500 rows 59.3 -> 49.6, 1600 rows 53.1 -> 70.3, 2048 rows 62.8 -> 65.6; 5120 x 2048, 2048 rows 42.2 -> 36.9).
 //    Beyond 8192 columns, and for the few outputs of 320 rows and more with a K of 1536 that are no 0.5 M, the 64 x 64 tiles by
 //    their own lines (whole_sums_in_small_tiles): 8704 x 512, 72 rows 8.0 -> 5.9, 400 rows 12.4 -> 10.9; 16384 x 512, 160 rows 12.5 -> 10.8;
 //    9728 x 896, 72 rows 11.9 -> 9.8, 160 rows 13.1 -> 11.1; 1536 x 1536, 325 rows 8.9 -> 8.3. From 512 tiles on with a K of more than
@@ -1219,7 +1220,7 @@ CW_EXPORT int cw_gemm_bf16_wide_choice(int mode, int M, int N, int K, int64_t ld
   if (N & (mode == 2 ? 15 : mode == 3 ? 3 : 7)) return 0;
   const int64_t elements = (int64_t)N * K, outputs = (int64_t)M * N;
   if (mode == 0) {
-    const bool here = K <= 512 ? N >= 32 : K <= 896 ? N >= 896 : K <= 1536 ? N >= 1536 && outputs >= 500000 : K <= 4096 && N >= 2048 && outputs >= 1600000;
+    const bool here = K <= 512 ? N >= 32 : K <= 896 ? N >= 896 : K <= 1536 ? N >= 1536 && outputs >= 500000 : K <= 4096 && N >= 2048 && outputs >= 1600000 && (K <= 2048 || outputs <= 9500000);
     if (!here || N > 8192) return whole_sums_in_small_tiles(M, N, K);
   } else if (mode == 2) {
     if ((N & 1) || (N < 2 * K && K > 1024) || elements > 136000000) return 0;

@@ -276,3 +276,8 @@ def test_long_sums_of_many_rows_are_whole_on_large_tiles_only():
 def test_few_small_tiles_rather_than_many_runs(M, N, K, want):
     """Sums that tiles of 64 x 128 in more runs were named for, 6 to 13 % slower (11.8 / 13.3, 13.1 / 14.5, 11.0 / 12.0, 14.2 / 15.2 us with the norm)."""
     assert _wide_choice(3, M, N, K) == want
+
+
+@pytest.mark.parametrize("M,N,K,there", [(1500, 6144, 3072, True), (1600, 6144, 3072, False), (2048, 6144, 3072, False), (2048, 5120, 2048, True), (2048, 4608, 3584, True)])
+def test_large_outputs_of_a_long_k_are_the_librarys(M, N, K, there):
+    assert (_wide_choice(0, M, N, K) is not None) == there
