@@ -354,7 +354,8 @@ __host__ __device__ __forceinline__ int wide_col(int ni, int r) {
   return ni < (NB & ~1) ? (ni >> 1) * 32 + s * 8 + (ni & 1) * 4 + e : ni * 16 + r;
 }
 
-// cw_gated from the bare exp2 and reciprocal instructions. A build of the kernel for each: asked for at every value the activation
+// cw_gated from the bare exp2 and reciprocal instructions (by expf and a division, as the smaller tiles do it, the bfloat16 results
+// are as far from 64 bits to seven digits; 5 to 11 in a million are others). A build of the kernel for each: asked for at every value the activation
 // took a fifth of 1600 rows' time with relu, asked for once a tile it took a copy of the tile's end for each, whose addresses
 // went to scratch in the widest tile. 17920 x 1536 with silu / relu / GELU / clipped, us: 2048 rows 92.5 / 99.7 / 106.5 / 107.7 with
 // three copies, 92.5 / 92.2 / 94.1 / 95.3 now; 1000 rows 49.4 / 52.0 / 56.2 / 56.6, now 49.3 / 48.2 / 49.6 / 50.0; 160 rows 22 throughout.
@@ -783,7 +784,7 @@ static int w_launch(WideArgs a, int row_tiles, int workgroups, hipStream_t strea
 // What a tile costs: ``fixed`` us of a work item and stage[q - 1] us a stage of 64 elements of K while q workgroups share a
 // compute unit (the smallest tiles; the others have one to themselves). Fits over timings with operands from memory, 72 to
 // 2048 rows of 26 shapes of the 0.5B to 14B models' layers and others (N 512 to 37888, K 512 to 18944); the fixed cost of 64 x 128
-// after another 22000, 65 to 2048 rows of 38 shapes. Over those a tile's time (and a launch's beside) is off by 7 % in the mean;
+// after another 22000, 65 to 2048 rows of 38 shapes. Over those a tile's time (and a launch's beside) is off by 7.5 % in the mean;
 // a tile that the rule names takes 1 to 1.6 % more than the fastest, the library among them, 24 % at worst (272 rows of 6144 x 1536 with
 // a gate 18.4 by 160 x 96, 14.9 by 128 x 128; 704 rows of 1024 x 4096 and a norm 20.9, 17.9 by 96 x 96). A stage of the large tiles goes with BM + BN, 2.3 ns a row: its
 // loads; 256 x 192 and 256 x 288 have two stages of them in LDS and wait longer, and gain by their few rounds.
@@ -836,7 +837,7 @@ static int tile_choice(int mode, int M, int N, int K, int most_planes, bool wide
 }
 
 // The product by the tile of bm x bn (128 x 128 and 256 x 192 for rows of any length, the others for whole ones: 16-byte
-// multiples), if there is such a tile for the mode.
+// multiples), if there is such a tile for the mode. (No rule names 128 x 128 for mode 0; whoever asks for it by its size gets it.)
 static int w_by_tile(int mode, int bm, int bn, bool whole, const WideArgs& a, int workgroups, hipStream_t stream) {
   const int gate = mode == 2 ? w_gate(a.act) : W_GATE_SILU;
 #define CW_WIDE_GATE(MODE_, MB_, NB_, SLOTS_, ANY_, GATE_)                                                 \

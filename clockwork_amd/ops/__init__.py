@@ -798,20 +798,17 @@ def linear_tiled(x: torch.Tensor, weight: torch.Tensor, bias=None, swiglu: bool 
 # the wide-tile kernel runs one workgroup per compute unit: with fewer tiles than this the
 # 128 x 128 kernel, whose tiles are a quarter of the size, fills the GPU better
 WIDE_MIN_TILES = 64
-# The engine takes the wide-tile kernel for the gate/up product by itself (no ``hip_products``)
-# where it beats the library product followed by the gate kernel. Measured on an MI355X over the
-# Qwen2.5 layer shapes from 0.5B to 72B with 256 to 4096 rows: with 180 tiles or more and 1024 rows or
-# more it is 5 to 25 % faster. With fewer rows it is for weights of at most 64 M elements where enough of its work is
-# not padding, of the rows to whole tiles and of the tiles to whole rounds over the compute units: 52 % in one round (the
-# library leaves units idle there as well), 58 % in several (us, library and gate against this: 1.5B shape, 188 tiles, 304 rows
-# 34.8 / 36.4, 368 rows 37.4 / 36.0, 408 rows 38.9 / 36.7, 512 rows 44.5 / 37.3; 282 tiles, 640 rows 53.6 / 68.9; 376 tiles,
-# 1000 rows 88.3 / 71.8; 3B shape, 230 tiles, 304 rows 44.5 / 44.8, 385 rows 55.1 / 45.8; 345 tiles, 640 rows 77.8 / 84.9, 700 rows
-# 97.2 / 86.0; 7B shape, 400 rows 150 / 136, 640 rows 189 / 202: there reading W bounds both). Against the library's TUNED choice it wins for
-# the 0.5B, 1.5B, 3B, 14B and 32B shapes (the 1.5B shape's whole prefill step: 8.9 -> 7.9 ms) and
-# loses 3 % of the step for the 7B and 72B shapes, so a start-up that tunes (``library_tuning``)
-# times both ways on the model's own weights and keeps the faster (``ProductPolicy.swiglu_choices``). These figures are of tiles
-# of 256 x 192; by the tiles it chooses from now (csrc/gemm_tile.hip) the kernel takes 1 to 30 % less, so the line is cautious: what
-# lies below it goes by ``cw_gemm_bf16_wide_choice``, from 65 rows on.
+# The engine takes the wide tiles for the gate/up product by itself (no ``hip_products``) with 1024 rows or more and 180 tiles of
+# 256 x 192 or more (a measure of the product's size: which tiles it runs on, csrc/gemm_tile.hip says by what they cost). Library
+# product and gate kernel / here, us, operands from memory, MI355X: 1024 rows of the 0.5B shape 35.8 / 22.5, 1.5B 81 / 48, 3B 105 / 88, 7B
+# 321 / 261, 14B 281 / 258, 32B 556 / 438, 72B 782 / 815; 1500 rows of the 7B shape 356 / 367, of the others 37.5 / 30.8, 94 / 78, 140 / 112, 404 /
+# 367, 801 / 688, 1116 / 1056; 2048 rows 63 / 45, 139 / 96, 193 / 164, 556 / 484, 528 / 420, 1071 / 847, 1530 / 1473. Against the library's TUNED
+# choice it loses for some shapes, so a start-up that tunes (``library_tuning``) times both ways on the model's own weights and
+# keeps the faster (``ProductPolicy.swiglu_choices``). Fewer rows go by ``cw_gemm_bf16_wide_choice``, up to 136 M elements of weights,
+# and run on the same tiles. Where 58 % of the work of 256 x 192 tiles is not padding, of rows to tiles and of tiles to rounds over
+# the units (52 % in one round), and the weights are at most 64 M elements, they do so without being timed at each number of
+# rows by a start-up that tunes: there nothing comes near (368 rows of the 1.5B shape 36.8 / 26.4, 512 rows 45.3 / 36.4, 1000 rows 84 / 48; 3B
+# shape, 408 rows 57 / 47, 700 rows 91 / 58).
 WIDE_SWIGLU_MIN_TILES = 180
 WIDE_SWIGLU_MIN_ROWS = 1024
 WIDE_SWIGLU_WORK, WIDE_SWIGLU_WORK_ONE_ROUND = 0.58, 0.52
