@@ -978,6 +978,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_group_bf16_kernel(Prod
 // NORM (MT = 1, no k-split): x is not read but made here, x = rmsnorm(resid + delta) * weight over
 // the K elements of a row, with the rounding steps of the stand-alone norm kernel; every
 // workgroup does so for itself (the rows are few and come from L2), nothing is written back.
+static __device__ uint4 cw_zeros[1];  // 8 elements (never written; not const, or loads from it or a matrix would be flat ones)
+
 struct StreamNormIn {
   const float* resid;    // [M, K] float32
   const bf16_t* delta;   // [M, K] bfloat16
@@ -1011,12 +1013,18 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
   auto to_operand = [&](const bf16x8_t& v) __attribute__((always_inline)) -> bf16x8_t {
     return cw_to_operand_layout(v, lane);
   };
-  int koff[SPW];  // the loading lane's 8 k-values of each step; a step outside K reads k = 0 and meets zeros in x
+  // The loading lane's 8 k-values of each step. A step outside of K meets zeros in x; it reads zeros, so that an infinite weight stays
+  // one, or in the products with a long K, whose loads the choice of address would slow by 4 %, k = 0.
+  constexpr bool ZEROS = MODE != 3 && NC == 1;
+  int koff[SPW];
 #pragma unroll
   for (int u = 0; u < SPW; ++u) {
     const int k = ((blockIdx.y * WAVES + wave) * SPW + u) * 32 + ls * 8;
-    koff[u] = k + 8 <= K ? k : 0;
+    koff[u] = k + 8 <= K ? k : ZEROS ? -1 : 0;
   }
+  auto weights = [&](const bf16_t* row, int k) __attribute__((always_inline)) -> bf16x8_t {
+    return *reinterpret_cast<const bf16x8_t*>(!ZEROS || k >= 0 ? row + k : reinterpret_cast<const bf16_t*>(cw_zeros));
+  };
   auto wrow = [&](int tile) __attribute__((always_inline)) -> const bf16_t* {
     int64_t n;
     if constexpr (GROUP) {
@@ -1037,7 +1045,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
   bf16x8_t cur[CH], nxt[CH];
   const bf16_t* w_tile = wrow(tile);
 #pragma unroll
-  for (int u = 0; u < CH; ++u) cur[u] = *reinterpret_cast<const bf16x8_t*>(w_tile + koff[u]);
+  for (int u = 0; u < CH; ++u) cur[u] = weights(w_tile, koff[u]);
 
   bf16x8_t xf[SPW][MT];
   if constexpr (NORM) {
@@ -1092,7 +1100,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
 #pragma unroll
       for (int u = 0; u < SPW; ++u) {
         const bool ok = ((blockIdx.y * WAVES + wave) * SPW + u) * 32 + ls * 8 + 8 <= K && m < M;
-        bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(xrow + koff[u]);
+        bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(xrow + (ZEROS ? max(koff[u], 0) : koff[u]));
         if (!ok) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] = (__bf16)0.0f;
@@ -1157,7 +1165,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
     auto load_set = [&](bf16x8_t (&dst)[CH], int t) __attribute__((always_inline)) {
       const bf16_t* w = wrow(min(t, n_tiles - 1));
 #pragma unroll
-      for (int u = 0; u < CH; ++u) dst[u] = *reinterpret_cast<const bf16x8_t*>(w + koff[u]);
+      for (int u = 0; u < CH; ++u) dst[u] = weights(w, koff[u]);
     };
     auto products = [&](const bf16x8_t (&w)[CH], f32x4_t (&acc)[MT]) __attribute__((always_inline)) {
 #pragma unroll
@@ -1198,7 +1206,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
         // the chunk after this one: of this tile, or the first of the workgroup's next tile
 #pragma unroll
         for (int u = 0; u < CH; ++u)
-          nxt[u] = *reinterpret_cast<const bf16x8_t*>((c + 1 < NC ? w_tile + koff[(c + 1) * CH + u] : w_next + koff[u]));
+          nxt[u] = c + 1 < NC ? weights(w_tile, koff[(c + 1) * CH + u]) : weights(w_next, koff[u]);
 #pragma unroll
         for (int u = 0; u < CH; ++u) {
           const bf16x8_t wu = to_operand(cur[u]);
@@ -1278,7 +1286,13 @@ static bool plan_stream(int mode, int M, int N, int K, int k_splits, int* mt, in
   const int waves = mode == 3 ? 8 : 16;
   *mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
   *spw = cw_stream_round_spw((k_steps + k_splits * waves - 1) / (k_splits * waves));
-  if (M > 64 || *spw > 24 || !cw_stream_fits(waves, *spw, *mt) || (mode != 3 && k_steps < 2 * waves)) return false;
+  // A K of less than two steps a wave leaves waves idle and still is the faster way from 16 steps on beyond 16 rows, where the other
+  // way is a library product, and from 24 on for fewer, where it is a workgroup a tile or four (us, that way / this one: [gate;
+  // up] of 9728 x 896 with 1, 8, 16 rows 6.0 / 6.0, 6.7 / 5.9, 7.7 / 5.9, with 17, 32, 64 14.1 / 6.7, 14.2 / 6.7, 14.7 / 9.4; 151936 x 896 53.5 / 49.1,
+  // 61.5 / 55.9, 65.9 / 58.0, 71.3 / 59.7, 74.9 / 62.9, 85.9 / 71.9; [gate; up] of 6144 x 768 3.8 / 3.7 to 4.3 / 4.3, 9.9 / 4.8 to 10.3 / 6.9; 16384 x 512
+  // with 1 and 8 rows 5.5 / 6.1, 5.9 / 5.8, with 17 to 64 12.5 / 6.6 to 12.7 / 9.8, its head of 151936 31.7 / 40.4, 35.4 / 41.1, 66.6 / 43.4, 66.0 / 59.2).
+  const int least_steps = M > 16 ? waves : waves + waves / 2;
+  if (M > 64 || *spw > 24 || !cw_stream_fits(waves, *spw, *mt) || (mode != 3 && k_steps < least_steps)) return false;
   // tiles per workgroup: one workgroup on every compute unit (a second round of these large
   // workgroups costs more than it brings), each with the same share
   // (up to 16 rows the one-tile kernels are as fast below two rounds; beyond, the alternative
@@ -1425,7 +1439,7 @@ CW_EXPORT int cw_gemm_bf16_swiglu_normed_ok(int M, int N, int K) {
   int mt, spw, n_tiles;
   dim3 grid;
   // rows of up to 2048 elements: a lane holds its share of a row in registers over the statistics
-  return M >= 1 && M <= 16 && !(N & 1) && !(K & 7) && plan_stream(2, M, N, K, 1, &mt, &spw, &grid, &n_tiles) &&
+  return M >= 1 && M <= 16 && K >= 1024 && !(N & 1) && !(K & 7) && plan_stream(2, M, N, K, 1, &mt, &spw, &grid, &n_tiles) &&
                  spw <= 4
              ? 1
              : 0;

@@ -871,3 +871,31 @@ def test_a_recurrence_beside_the_runs_of_single_tokens(heads, dim, r_vdim, rank,
     apart, together = both(False), both(True)
     rows = torch.cat([torch.arange(int(cu[r]), int(cu[r + 1]), device=DEV) for r in range(R) if r != 1])   # a request without a slot has no outputs
     assert torch.equal(apart[0][rows], together[0][rows]) and torch.equal(apart[1], together[1]) and torch.equal(apart[2], together[2])
+
+
+# K: 16, 23.25, 24 and 28 steps of 32 for 16 waves (idle waves, a step that K ends in); N: 512 tiles of gates and ups, or of 16
+# outputs, and just more
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
+@pytest.mark.parametrize("K", [512, 744, 768, 896])
+@pytest.mark.parametrize("N", [8192, 8208])
+def test_streamed_products_of_fewer_steps_than_two_a_wave(M, K, N):
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(M + K + N)
+    x = torch.randn(M, K, device=DEV, generator=gen).to(torch.bfloat16)
+    w = (torch.randn(N, K, device=DEV, generator=gen) / K ** 0.5).to(torch.bfloat16)
+    w[3, 0] = w[N - 1, K - 1] = float("inf")   # stay in their outputs, as infinities where x is not zero
+    x[:, 0] = x[:, K - 1] = 1.0
+    assert ops._load("gemm").cw_gemm_bf16_skinny_fast(1, M, N, K) == 1
+    y = x.double() @ w.double().t()
+    # float32 sums of K products of about 1 / sqrt(K): 2^-24 sqrt(K) of the result's spread at most, ten times that
+    got = ops.linear(x, w, out_dtype=torch.float32)
+    assert bool((got[:, [3, N - 1]] == float("inf")).all())
+    rest = [i for i in range(N) if i not in (3, N - 1)]
+    assert float((got.double() - y)[:, rest].abs().max()) < 10 * 2.0 ** -24 * K ** 0.5
+    # and rounded once to bfloat16: 2^-9 of a value
+    gated = ops.linear_swiglu(x, torch.cat([w, w.flip(0)]))
+    assert ops._load("gemm").cw_gemm_bf16_skinny_fast(2, M, 2 * N, K) == 1
+    want = torch.nn.functional.silu(y) * y.flip(1)
+    keep = [i for i in rest if N - 1 - i in rest]
+    torch.testing.assert_close(gated.double()[:, keep], want[:, keep], rtol=2.0 ** -8, atol=1e-5)
