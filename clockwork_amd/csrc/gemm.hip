@@ -1523,14 +1523,15 @@ CW_EXPORT int cw_gemm_bf16_skinny(int mode, const void* X, int64_t ldx, const vo
 }
 
 // Are these products of ``M`` rows and K columns taken as one launch (``tiles``: their tiles of 16 rows of W)? Up to 16 rows
-// always; beyond, and up to 64, where all have the same x and the streaming kernel takes them (apart, those of fewer than 256
-// tiles are products of the library or of 64-row tiles).
+// always; beyond, and up to 64, where all have the same x of 768 columns and more and the streaming kernel takes them (apart, those of
+// fewer than 256 tiles are products of the library or of 64-row tiles). 17 / 64 rows of 896, outputs of 1152, 3600 and 1792, us apart and
+// together: 26.7 and 5.4, 30.9 and 6.9; of 768, outputs of 2304, 3072 and 4096: 22.7 and 6.6, 24.4 and 8.7.
 CW_EXPORT int cw_gemm_bf16_group_ok(int count, int same_x, int M, int64_t tiles, int K) {
   if (count < 2 || count > GROUP_MAX || M < 1 || M > CW_SKINNY_MAX_M || K < 8 || (K & 7) || tiles < count || tiles > (1 << 20)) return 0;
   if (M <= 16) return 1;
   int mt, spw, n_tiles;
   dim3 grid;
-  return same_x && plan_stream(0, M, (int)tiles * 16, K, 1, &mt, &spw, &grid, &n_tiles) && spw <= 8 ? 1 : 0;
+  return same_x && K >= 768 && plan_stream(0, M, (int)tiles * 16, K, 1, &mt, &spw, &grid, &n_tiles) && spw <= 8 ? 1 : 0;
 }
 
 // C[i] [M, N[i]] = X[i] W[i]^T for ``count`` products, all bfloat16, rows without gaps: X[i] [M, K], W[i] [N[i], K].
