@@ -803,13 +803,49 @@ CW_EXPORT int cw_gemm_f32_partial(const float* A, int64_t lda, const float* W, f
 __device__ __forceinline__ float cw_gelu_erf(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752440f)); }
 __device__ __forceinline__ float cw_relu_squared(float z) { const float r = fmaxf(z, 0.0f); return r * r; }
 
+// A norm that the product before has begun (gemm_join_bf16_kernel): x holds the rows times the norm's weights, ``squares``
+// [M, parts] the sums of squares of each row's pieces (parts: a multiple of 4, at most 256). A row's factor 1 / sqrt(mean + eps)
+// multiplies the finished sums instead of the elements, so no product waits for it: the pieces are asked for ahead of the
+// weights, and a wave adds up those of its rows (wave, wave + WAVES, ...) while or after the weights come in.
+struct RowFactors {
+  const float* squares;
+  int parts;
+  float of_width, eps;  // 1 / elements of a row
+};
+template <int WAVES> struct RowPieces {
+  static constexpr int ROWS = 16 / WAVES;
+  float4 v[ROWS];
+  __device__ __forceinline__ void load(const RowFactors& in, int M) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+      const int m = wave + i * WAVES;
+      v[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (m < M && lane * 4 < in.parts) v[i] = *reinterpret_cast<const float4*>(in.squares + m * in.parts + lane * 4);
+    }
+  }
+  // visible behind the next barrier
+  __device__ __forceinline__ void factors(const RowFactors& in, float* to) const {
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+      const float total = cw_wave_sum((v[i].x + v[i].y) + (v[i].z + v[i].w));
+      if ((threadIdx.x & 63) == 0) to[(threadIdx.x >> 6) + i * WAVES] = __builtin_amdgcn_rsqf(fmaf(total, in.of_width, in.eps));
+    }
+  }
+};
+
 // ROWS (16, 8 or 4) is the number of weight rows a tile really holds: a narrow output with a long K
 // is cut into more, smaller tiles so that every compute unit streams a share of the matrix (the
 // unused rows of the MFMA tile are zeros). MODE 2 needs ROWS == 16.
-template <int MT, int RT, int MODE, int WAVES, int ROWS>
+template <int MT, int RT, int MODE, int WAVES, int ROWS, bool BEGUN = false>
 __device__ __forceinline__ void skinny_tiles(const bf16_t* __restrict__ X, int64_t ldx, const bf16_t* __restrict__ W,
-                                             void* __restrict__ C, int64_t ldc, int M, int N, int K, float act, const int block) {
+                                             void* __restrict__ C, int64_t ldc, int M, int N, int K, float act, const int block,
+                                             const RowFactors& begun = RowFactors{}) {
+  static_assert(!BEGUN || (MT == 1 && MODE == 2), "begun norms are gate/up products' of up to 16 rows");
   __shared__ float red[WAVES][RT * MT * 256];
+  __shared__ float factors[16];
+  [[maybe_unused]] RowPieces<WAVES> pieces;
+  if constexpr (BEGUN) pieces.load(begun, M);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, s = lane >> 4;
   const int lr = lane >> 2, ls = lane & 3;  // the row of a tile and the slot of a k-step that this lane loads
@@ -857,7 +893,10 @@ __device__ __forceinline__ void skinny_tiles(const bf16_t* __restrict__ X, int64
   const int k_steps = (K + 31) / 32;
   constexpr int U = 4;  // k-steps in flight per wave
   const int n_ksplit = MODE == 3 ? gridDim.y : 1;
-  for (int ks0 = ((MODE == 3 ? blockIdx.y : 0) * WAVES + wave) * U; ks0 < k_steps; ks0 += n_ksplit * WAVES * U) {
+  int ks0 = ((MODE == 3 ? blockIdx.y : 0) * WAVES + wave) * U;
+  [[maybe_unused]] bool first = true;
+  // (BEGUN: also a wave without a step adds up its rows' pieces)
+  for (; BEGUN && first || ks0 < k_steps; ks0 += n_ksplit * WAVES * U) {
     bf16x8_t wf[U][RT], xf[U][MT];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -871,6 +910,10 @@ __device__ __forceinline__ void skinny_tiles(const bf16_t* __restrict__ X, int64
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
         xf[u][mt] = (kxok && xok[mt]) ? *reinterpret_cast<const bf16x8_t*>(xrow[mt] + kx) : zero;
+    }
+    if constexpr (BEGUN) {
+      if (first) pieces.factors(begun, factors);
+      first = false;
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -910,8 +953,9 @@ __device__ __forceinline__ void skinny_tiles(const bf16_t* __restrict__ X, int64
       const int mt = m >> 4, tok = m & 15;
       const int64_t i = ((int64_t)block * RT + rt) * 8 + j;
       if (m >= M || i >= I) continue;
-      const float g = red[0][(rt * MT + mt) * 256 + j * 16 + tok];
-      const float u = red[0][(rt * MT + mt) * 256 + (j + 8) * 16 + tok];
+      const float factor = BEGUN ? factors[m] : 1.0f;
+      const float g = red[0][(rt * MT + mt) * 256 + j * 16 + tok] * factor;
+      const float u = red[0][(rt * MT + mt) * 256 + (j + 8) * 16 + tok] * factor;
       ((bf16_t*)C)[(int64_t)m * ldc + i] = __float2bfloat16(act > 0.0f ? cw_clipped_glu(g, u, act) : act < 0.0f ? cw_gated_below(g, u, act) : g / (1.0f + __expf(-g)) * u);
     }
   } else {
@@ -936,6 +980,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_bf16_kernel(const bf16
                                                                void* __restrict__ C, int64_t ldc,
                                                                int M, int N, int K, float act) {
   skinny_tiles<MT, RT, MODE, WAVES, ROWS>(X, ldx, W, C, ldc, M, N, K, act, blockIdx.x);
+}
+
+template <int RT, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_begun_bf16_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
+                                                                            bf16_t* __restrict__ C, int64_t ldc, int M, int N, int K,
+                                                                            float act, RowFactors begun) {
+  skinny_tiles<1, RT, 2, WAVES, 16, true>(X, K, W, C, ldc, M, N, K, act, blockIdx.x, begun);
 }
 
 // Several products of the same rows and the same K as one launch, each with an x, a matrix and an output of its own: a layer that
@@ -993,12 +1044,14 @@ struct StreamNormIn {
 constexpr int cw_stream_chunk(int spw) { return spw <= 8 ? spw : (spw <= 12 ? spw / 2 : spw / 4); }
 
 // GROUP (MODE 0): row tiles of several products of the same x, ``in`` a ProductGroup (W, C, ldc and N are not used).
-template <int MODE, int WAVES, int SPW, int MT, bool NORM = false, bool GROUP = false>
+// BEGUN (MODE 2, MT = 1): x comes with its norm begun, ``in`` a RowFactors.
+template <int MODE, int WAVES, int SPW, int MT, bool NORM = false, bool GROUP = false, bool BEGUN = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16_t* __restrict__ X, int64_t ldx,
                                                                const bf16_t* __restrict__ W,
                                                                void* __restrict__ C, int64_t ldc,
                                                                int M, int N, int K, int n_tiles, float act,
-                                                               std::conditional_t<GROUP, ProductGroup, StreamNormIn> in) {
+                                                               std::conditional_t<GROUP, ProductGroup, std::conditional_t<BEGUN, RowFactors, StreamNormIn>> in) {
+  static_assert(!BEGUN || (MODE == 2 && MT == 1 && !NORM), "begun norms are gate/up products' of up to 16 rows");
   static_assert(!GROUP || (MODE == 0 && !NORM), "grouped products are plain ones");
   constexpr int NBUF = MT <= 2 ? 2 : 1;
   constexpr int CH = cw_stream_chunk(SPW), NC = SPW / CH;
@@ -1007,6 +1060,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, s = lane >> 4;
   const int I = N / 2;  // MODE 2 only
+  __shared__ float factors[16];
+  [[maybe_unused]] RowPieces<WAVES> pieces;
+  if constexpr (BEGUN) pieces.load(in, M);
 
   // Loads as cw_to_operand_layout describes: this lane loads row lr of a tile, slot ls of a k-step.
   const int lr = lane >> 2, ls = lane & 3;
@@ -1109,6 +1165,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
       }
     }
   }
+  if constexpr (BEGUN) pieces.factors(in, factors);
   // what the waves' partial tiles of ``tile`` (in red[buf]) become: summed over the waves, then
   // stored as the mode says. One barrier before; a second after, when the buffer is not doubled.
   auto finish_tile = [&](const f32x4_t (&acc)[MT], int tile, int buf) __attribute__((always_inline)) {
@@ -1127,6 +1184,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
           const float2 gu = *reinterpret_cast<const float2*>(&red[buf][w][m * 16 + 2 * j]);
           g += gu.x;
           up += gu.y;
+        }
+        if constexpr (BEGUN) {
+          g *= factors[m];
+          up *= factors[m];
         }
         const int64_t i = (int64_t)tile * 8 + j;
         if (m < M && i < I) ((bf16_t*)C)[(int64_t)m * ldc + i] =
@@ -1593,13 +1654,18 @@ CW_EXPORT int cw_gemm_bf16_group(int count, const void* const* X, const void* co
 // epilogue adds the bias, rotates by float32(pos) * inv_freq[i] and writes q to ``q_out``
 // [M, nh * hd], rotated k and plain v to their cache rows ``slots[m]`` ([rows, nkv, hd]).
 // blockIdx.y takes MT tiles of 16 tokens.
-template <int WAVES, int MT>
+// BEGUN (MT = 1, at most 16 rows): x comes with its norm begun.
+template <int WAVES, int MT, bool BEGUN = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm_qkv_rope_bf16_kernel(
     const bf16_t* __restrict__ X, int64_t ldx, const bf16_t* __restrict__ W, const void* __restrict__ bias,
     int bias_f32, const int* __restrict__ positions, const int* __restrict__ slots,
     const float* __restrict__ inv_freq, bf16_t* __restrict__ q_out, bf16_t* __restrict__ k_cache,
-    bf16_t* __restrict__ v_cache, int64_t cache_rows, int M, int K, int nh, int nkv, int hd) {
+    bf16_t* __restrict__ v_cache, int64_t cache_rows, int M, int K, int nh, int nkv, int hd, RowFactors begun) {
+  static_assert(!BEGUN || MT == 1, "begun norms are products' of up to 16 rows");
   __shared__ __align__(16) float red[WAVES][MT * 256];  // [wave][token tile][token][tile row]
+  __shared__ float factors[16];
+  [[maybe_unused]] RowPieces<WAVES> pieces;
+  if constexpr (BEGUN) pieces.load(begun, M);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, s = lane >> 4;
   const int half = hd / 2;
@@ -1665,7 +1731,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_qkv_rope_bf16_kernel(
   for (int e = 0; e < 8; ++e) zero[e] = (__bf16)0.0f;
   const int k_steps = (K + 31) / 32;
   constexpr int U = 4;  // k-steps in flight a wave
-  for (int ks0 = wave * U; ks0 < k_steps; ks0 += WAVES * U) {
+  [[maybe_unused]] bool first = true;
+  // (BEGUN: also a wave without a step adds up its rows' pieces)
+  for (int ks0 = wave * U; BEGUN && first || ks0 < k_steps; ks0 += WAVES * U) {
     bf16x8_t wf[U], xf[U][MT];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -1677,6 +1745,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_qkv_rope_bf16_kernel(
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
         xf[u][mt] = (kxok && xok[mt]) ? *reinterpret_cast<const bf16x8_t*>(xrow[mt] + kx) : zero;
+    }
+    if constexpr (BEGUN) {
+      if (first) pieces.factors(begun, factors);
+      first = false;
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -1699,7 +1771,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_qkv_rope_bf16_kernel(
     red[0][idx] = sum;
   }
   __syncthreads();
-  auto summed = [&](int row, int m) -> float { return red[0][m * 16 + row]; };
+  auto summed = [&](int row, int m) -> float { return BEGUN ? red[0][m * 16 + row] * factors[m] : red[0][m * 16 + row]; };
   if constexpr (MT == 1) {
     // every thread has at most one output (v: 256 of them, q and k: 128 pairs)
     if (is_v) {
@@ -1785,7 +1857,7 @@ CW_EXPORT int cw_gemm_qkv_rope_bf16(const void* X, int64_t ldx, const void* W, c
 #define CW_QKV(WAVES_, MT_)                                                                              \
   hipLaunchKernelGGL((gemm_qkv_rope_bf16_kernel<WAVES_, MT_>), grid, dim3(WAVES_ * 64), 0, stream, x, ldx, \
                      w, bias, bias_f32, positions, slots, inv_freq, (bf16_t*)q_out, (bf16_t*)k_cache,    \
-                     (bf16_t*)v_cache, cache_rows, M, K, nh, nkv, hd)
+                     (bf16_t*)v_cache, cache_rows, M, K, nh, nkv, hd, RowFactors{})
   if (M <= 16) {
     if (tiles <= 256 && K >= 1024) CW_QKV(16, 1);
     else if (K >= 512) CW_QKV(8, 1);
@@ -1808,5 +1880,199 @@ CW_EXPORT int cw_gemm_qkv_rope_bf16(const void* X, int64_t ldx, const void* W, c
     }
   }
 #undef CW_QKV
+  return cw_launch_status();
+}
+
+// The same for at most 16 rows that come with their norm begun: X [M, K] and squares [M, parts] as cw_gemm_bf16_join writes them.
+CW_EXPORT int cw_gemm_qkv_rope_begun_bf16(const void* X, const float* squares, int parts, float eps, const void* W, const void* bias,
+                                          int bias_f32, const int* positions, const int* slots, const float* inv_freq, void* q_out,
+                                          void* k_cache, void* v_cache, int64_t cache_rows, int M, int K, int nh, int nkv, int hd,
+                                          hipStream_t stream) {
+  if (M < 1 || M > 16 || K <= 0 || nh <= 0 || nkv <= 0 || hd <= 0 || (hd & 15) || parts < 4 || parts > 256 || (parts & 3) || ((uintptr_t)squares & 15)) return CW_ERR_ARG;
+  if ((K & 7) || ((uintptr_t)X & 15) || ((uintptr_t)W & 15)) return CW_ERR_ARG;
+  if (!X || !squares || !W || !positions || !slots || !inv_freq || !q_out || !k_cache || !v_cache) return CW_ERR_ARG;
+  const RowFactors begun{squares, parts, 1.0f / (float)K, eps};
+  const int tiles = (nh + 2 * nkv) * (hd / 16);
+#define CW_QKV(WAVES_)                                                                                                             \
+  hipLaunchKernelGGL((gemm_qkv_rope_bf16_kernel<WAVES_, 1, true>), dim3(tiles), dim3(WAVES_ * 64), 0, stream, (const bf16_t*)X,      \
+                     (int64_t)K, (const bf16_t*)W, bias, bias_f32, positions, slots, inv_freq, (bf16_t*)q_out, (bf16_t*)k_cache,    \
+                     (bf16_t*)v_cache, cache_rows, M, K, nh, nkv, hd, begun)
+  if (tiles <= 256 && K >= 1024) CW_QKV(16);
+  else if (K >= 512) CW_QKV(8);
+  else CW_QKV(4);
+#undef CW_QKV
+  return cw_launch_status();
+}
+
+// =====================================================================================
+// A product of few rows that joins the residual stream and begins the norm behind it (decode: 1 to 16 tokens):
+//   resid += x W^T;  y = resid * norm_weight (bfloat16);  squares[m, tile] = sum of resid[m, n]^2 over a tile's columns.
+// The product that reads y multiplies its finished sums by 1 / sqrt(mean + eps) (RowFactors), so the residual add and the norm
+// are no launch of their own.
+// A workgroup owns up to R outputs (``rows`` of them) and all of K: the 16 rows of its matrix operand are R rows of W times 16 / R
+// neighbouring pieces of 32 k-values, each multiplied with its own piece of x into sums of its own, of which the other pieces' rows are
+// dropped. So a narrow output (N of 896 to 3584) makes enough workgroups for the card without planes of partial sums.
+// Bound by the launch and its first trip to memory, then by what a workgroup takes in: its rows of W and all of x. Product and norm as two
+// launches -> this one, us in a graph over 24 to 28 layers' matrices, 1 / 4 / 8 / 16 rows: 896 x 896 4.7 / 5.0 / 5.2 / 5.4 -> 3.1 / 3.2 / 3.2 /
+// 3.5; 896 x 4864 6.4 / 6.7 / 6.7 / 7.1 -> 4.3 / 4.9 / 5.6 / 7.2; 1536 x 1536 5.2 / 5.6 / 5.8 / 6.3 -> 3.4 / 3.5 / 3.7 / 4.2; 1536 x 8960 9.6 / 9.8 /
+// 10.0 / 10.4 -> 8.7 / 8.7 / 9.8 / 13.2; 3584 x 3584 9.9 / 10.0 / 10.0 / 10.3 -> 7.2 / 7.5 / 7.7 / 8.9; 3584 x 18944 28.7 / 29.5 / 30.8 / 32.1 -> 27.6 /
+// 30.5 / 33.1 / 41.2. (Two sets of operands a wave in turns, rows of x swapped into operand layout: slower, both are more code.)
+template <int WAVES, int R>
+__global__ __launch_bounds__(WAVES * 64) void gemm_join_bf16_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
+                                                                    float* __restrict__ resid, const void* __restrict__ norm_weight,
+                                                                    bf16_t* __restrict__ Y, float* __restrict__ squares, int M, int N,
+                                                                    int K, int rows, int norm_weight_f32) {
+  constexpr int P = 16 / R;                       // pieces of K side by side in an operand
+  constexpr int U = P == 4 ? 3 : P == 2 ? 5 : 8;  // operands of W on their way a wave
+  __shared__ __align__(16) float red[WAVES][256];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, s = lane >> 4;
+  const int lr = lane >> 2, ls = lane & 3;
+  const int n0 = blockIdx.x * rows;
+  const bool w_ok = lr % R < rows && n0 + lr % R < N;  // a row that is not there counts as zeros
+  const int w_k = (lr / R) * 32 + ls * 8;
+  const bf16_t* const wrow = W + (int64_t)(w_ok ? n0 + lr % R : 0) * K + w_k;
+  const bool x_ok = r < M;
+  const bf16_t* const xrow = X + (int64_t)(x_ok ? r : 0) * K + s * 8;
+  // what the last threads need of the stream and of the norm, asked for beside the weights
+  const int e_m = threadIdx.x >> 4, e_j = threadIdx.x & 15;
+  const bool e_ok = threadIdx.x < 256 && e_m < M && e_j < rows && n0 + e_j < N;
+  const int64_t e_at = (int64_t)e_m * N + n0 + e_j;
+  float e_resid = 0.0f, e_weight = 0.0f;
+  if (e_ok) {
+    e_resid = resid[e_at];
+    e_weight = norm_weight_f32 ? ((const float*)norm_weight)[n0 + e_j] : __bfloat162float(((const bf16_t*)norm_weight)[n0 + e_j]);
+  }
+  bf16x8_t zero;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) zero[e] = (__bf16)0.0f;
+  f32x4_t acc[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) acc[p] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
+  const int steps = (K + 32 * P - 1) / (32 * P);
+  for (int at = wave; at < steps; at += WAVES * U) {
+    bf16x8_t wf[U], xf[U][P];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int step = at + u * WAVES, k = step * (32 * P);
+      const bool on = step < steps;
+      wf[u] = on && w_ok && k + w_k + 8 <= K ? *reinterpret_cast<const bf16x8_t*>(wrow + k) : zero;
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+        xf[u][p] = on && x_ok && k + p * 32 + s * 8 + 8 <= K ? *reinterpret_cast<const bf16x8_t*>(xrow + k + p * 32) : zero;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bf16x8_t wo = cw_to_operand_layout(wf[u], lane);
+#pragma unroll
+      for (int p = 0; p < P; ++p) acc[p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wo, xf[u][p], acc[p], 0, 0, 0);
+    }
+  }
+  // lane (r, s) holds operand rows 4s..4s+3 of token r, which are rows of piece 4s / R: of that piece's sums
+  f32x4_t mine = acc[0];
+#pragma unroll
+  for (int p = 1; p < P; ++p)
+    if (s / (R / 4) == p) mine = acc[p];
+  *reinterpret_cast<f32x4_t*>(&red[wave][r * 16 + 4 * s]) = mine;
+  cw_lds_barrier();
+  if (threadIdx.x >= 256) return;
+  float v = 0.0f;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) v += red[w][threadIdx.x];
+  if constexpr (R == 4) v += cw_dpp<0x124>(v);  // rotated by 4 of a row's 16 lanes: the pieces of an output lie R lanes apart
+  if constexpr (R <= 8) v += cw_dpp<0x128>(v);  // by 8
+  v += e_resid;
+  if (e_ok) {
+    resid[e_at] = v;
+    Y[e_at] = __float2bfloat16(v * e_weight);
+  }
+  float q = e_ok ? v * v : 0.0f;  // of the token's R neighbours, in pairs
+  q += cw_dpp<0xB1>(q);
+  q += cw_dpp<0x4E>(q);
+  if constexpr (R >= 8) q += cw_dpp<0x141>(q);
+  if constexpr (R >= 16) q += cw_dpp<0x140>(q);
+  const int parts = ((int)gridDim.x + 3) & ~3;
+  if (e_m < M && e_j == 0) squares[e_m * parts + blockIdx.x] = q;
+  // (a row of pieces ends on a multiple of four: zeros)
+  if (blockIdx.x == gridDim.x - 1 && e_m < M && e_j > 0 && (int)blockIdx.x + e_j < parts) squares[e_m * parts + blockIdx.x + e_j] = 0.0f;
+}
+
+// How cw_gemm_bf16_join cuts a product: outputs a workgroup, of ``*slots`` that its kernel has room for, and waves. 0: it does not take
+// the product. Few rows of x beside the weights only: every workgroup takes in all of x, and from about 72 K elements on the planes and
+// the norm that adds them are the faster way (see the kernel: 8 rows of 8960 are even, 16 lose). Up to 16 outputs a compute unit in one
+// round, so that all units stream; a K of up to 2048 is one trip to memory for eight waves.
+static int join_plan(int M, int N, int K, int* slots, int* waves) {
+  if (M < 1 || M > 16 || N < 64 || N > 16 * cw_num_compute_units() || K < 256 || (K & 7) || (int64_t)M * K > 72 * 1024) return 0;
+  const int rows = (N + cw_num_compute_units() - 1) / cw_num_compute_units();
+  *waves = N <= 2048 && K <= 2048 ? 8 : 16;
+  *slots = rows > 8 ? 16 : rows > 4 || *waves == 8 ? 8 : 4;
+  const int taken = *waves == 8 ? *slots : rows;
+  return (N + taken - 1) / taken <= 256 ? taken : 0;  // pieces of a row that its reader takes
+}
+
+// The number of sums of squares that cw_gemm_bf16_join leaves of a row (zeros up to a multiple of 4 at the end), 0 where it does not take these sizes.
+CW_EXPORT int cw_gemm_bf16_join_parts(int M, int N, int K) {
+  int slots, waves;
+  const int rows = join_plan(M, N, K, &slots, &waves);
+  return rows ? ((N + rows - 1) / rows + 3) & ~3 : 0;
+}
+
+// resid [M, N] float32 += x W^T; Y [M, N] bfloat16 = resid * norm_weight [N]; squares [M, parts] float32. x [M, K] and W [N, K]
+// bfloat16, rows without gaps.
+CW_EXPORT int cw_gemm_bf16_join(const void* X, const void* W, float* resid, const void* norm_weight, int norm_weight_f32, void* Y,
+                                float* squares, int M, int N, int K, hipStream_t stream) {
+  int slots, waves;
+  const int rows = join_plan(M, N, K, &slots, &waves);
+  if (!rows) return CW_ERR_SIZE;
+  if (!X || !W || !resid || !norm_weight || !Y || !squares || ((uintptr_t)X & 15) || ((uintptr_t)W & 15)) return CW_ERR_ARG;
+  const dim3 grid((N + rows - 1) / rows);
+#define CW_JOIN(WAVES_, R_)                                                                                                  \
+  hipLaunchKernelGGL((gemm_join_bf16_kernel<WAVES_, R_>), grid, dim3(WAVES_ * 64), 0, stream, (const bf16_t*)X, (const bf16_t*)W, \
+                     resid, norm_weight, (bf16_t*)Y, squares, M, N, K, rows, norm_weight_f32)
+  if (waves == 8) CW_JOIN(8, 8);
+  else if (slots == 4) CW_JOIN(16, 4);
+  else if (slots == 8) CW_JOIN(16, 8);
+  else CW_JOIN(16, 16);
+#undef CW_JOIN
+  return cw_launch_status();
+}
+
+// y[m, i] = silu(gate_i . x_m) * (up_i . x_m) as cw_gemm_bf16_skinny's mode 2, for rows that come with their norm begun: X [M, K]
+// and squares [M, parts] as cw_gemm_bf16_join writes them.
+CW_EXPORT int cw_gemm_bf16_swiglu_begun(const void* X, const float* squares, int parts, float eps, const void* W, void* C, int64_t ldc,
+                                        int M, int N, int K, hipStream_t stream) {
+  if (M < 1 || M > 16 || N < 2 || (N & 1) || K < 8 || (K & 7) || parts < 4 || parts > 256 || (parts & 3)) return CW_ERR_SIZE;
+  if (!X || !squares || ((uintptr_t)squares & 15) || !W || !C || ldc < N / 2 || ((uintptr_t)X & 15) || ((uintptr_t)W & 15)) return CW_ERR_ARG;
+  const RowFactors begun{squares, parts, 1.0f / (float)K, eps};
+  const bf16_t *x = (const bf16_t*)X, *w = (const bf16_t*)W;
+  int mt, spw, n_tiles;
+  dim3 grid;
+  if (plan_stream(2, M, N, K, 1, &mt, &spw, &grid, &n_tiles)) {
+#define CW_BEGUN(SPW_)                                                                                                               \
+  case SPW_:                                                                                                                         \
+    if constexpr (cw_stream_fits(16, SPW_, 1)) {                                                                                     \
+      hipLaunchKernelGGL((gemm_stream_bf16_kernel<2, 16, SPW_, 1, false, false, true>), grid, dim3(16 * 64), 0, stream, x, (int64_t)K, \
+                         w, C, ldc, M, N, K, n_tiles, 0.0f, begun);                                                                  \
+      return cw_launch_status();                                                                                                     \
+    }                                                                                                                                \
+    break
+    switch (spw) {
+      CW_BEGUN(1); CW_BEGUN(2); CW_BEGUN(3); CW_BEGUN(4); CW_BEGUN(5); CW_BEGUN(6); CW_BEGUN(7); CW_BEGUN(8);
+      CW_BEGUN(10); CW_BEGUN(12); CW_BEGUN(16); CW_BEGUN(20); CW_BEGUN(24);
+      default: break;
+    }
+#undef CW_BEGUN
+    return CW_ERR_SIZE;
+  }
+  // waves and tiles as cw_gemm_bf16_skinny takes them
+  const int tiles = (N / 2 + 7) / 8;
+#define CW_SKINNY_BEGUN(RT_, WAVES_)                                                                                                \
+  hipLaunchKernelGGL((gemm_skinny_begun_bf16_kernel<RT_, WAVES_>), dim3((tiles + RT_ - 1) / RT_), dim3(WAVES_ * 64), 0, stream, x, w, \
+                     (bf16_t*)C, ldc, M, N, K, 0.0f, begun)
+  if (tiles <= 256 && K >= 1024) CW_SKINNY_BEGUN(1, 16);
+  else if (tiles >= 4096) CW_SKINNY_BEGUN(4, 4);
+  else if (tiles <= 1024 && K >= 512) CW_SKINNY_BEGUN(1, 8);
+  else CW_SKINNY_BEGUN(1, 4);
+#undef CW_SKINNY_BEGUN
   return cw_launch_status();
 }

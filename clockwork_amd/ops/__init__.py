@@ -119,7 +119,11 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_gemm_bf16_swiglu_normed": [P, P, P, I, F, P, P, L, I, I, I, P],
             "cw_gemm_bf16_group_ok": [I, I, I, L, I],
             "cw_gemm_bf16_group": [I, P, P, P, P, I, I, P],
+            "cw_gemm_bf16_join_parts": [I, I, I],
+            "cw_gemm_bf16_join": [P, P, P, P, I, P, P, I, I, I, P],
+            "cw_gemm_bf16_swiglu_begun": [P, P, I, F, P, P, L, I, I, I, P],
             "cw_gemm_qkv_rope_bf16": [P, L, P, P, I, P, P, P, P, P, P, L, I, I, I, I, I, P],
+            "cw_gemm_qkv_rope_begun_bf16": [P, P, I, F, P, P, I, P, P, P, P, P, P, L, I, I, I, I, I, P],
         },
         "gemm_tile": {
             "cw_gemm_bf16_tiled": [I, P, L, P, P, I, P, L, I, I, I, F, P],
@@ -395,6 +399,51 @@ class LazyAddNorm:
     def value(self) -> torch.Tensor:
         out = torch.empty(tuple(self.resid.shape), dtype=self.dtype, device=self.resid.device)
         return add_rmsnorm(self.resid, self.delta, self.weight, self.eps, out, write_back=False)
+
+
+class BegunNorm:
+    """rmsnorm(resid) * weight but for each row's factor 1 / sqrt(mean + eps): ``x`` [T, H] is the stream times the norm's
+    weights, ``squares`` [T, parts] the float32 sums of squares of each row's pieces. What a product that has added its
+    output to the stream hands to the next one (``linear_join``), which multiplies its sums by the factor. Nothing is
+    pending: the stream is up to date."""
+
+    __slots__ = ("x", "squares", "eps")
+
+    def __init__(self, x: torch.Tensor, squares: torch.Tensor, eps: float) -> None:
+        self.x, self.squares, self.eps = x, squares, eps
+
+    @property
+    def shape(self):
+        return self.x.shape
+
+    @property
+    def dtype(self):
+        return self.x.dtype
+
+
+def linear_join_ok(M: int, weight: torch.Tensor, norm_weight: torch.Tensor) -> bool:
+    """Does ``linear_join`` take a product of ``M`` rows with ``weight``? By the rule of ``cw_gemm_bf16_join_parts``
+    (csrc/gemm.hip): few rows, an output that fills the card once."""
+    return (weight.dtype == torch.bfloat16 and weight.is_contiguous() and _aligned(weight) and norm_weight.numel() == weight.shape[0]
+            and norm_weight.dtype in (torch.bfloat16, torch.float32)
+            and _load("gemm").cw_gemm_bf16_join_parts(M, weight.shape[0], weight.shape[1]) > 0)
+
+
+def linear_join(x: torch.Tensor, weight: torch.Tensor, resid: torch.Tensor, norm_weight: torch.Tensor, eps: float) -> BegunNorm:
+    """resid += x @ weight.T and the norm of the result begun, in one kernel. The sums join the float32 stream as they are."""
+    _gpu(x, weight, resid, norm_weight)
+    M, K = x.shape
+    N = weight.shape[0]
+    if not (x.dtype == torch.bfloat16 and weight.shape[1] == K and linear_join_ok(M, weight, norm_weight) and _aligned(x)):
+        raise KernelError("the joining product does not take these operands")
+    if not (resid.dtype == torch.float32 and tuple(resid.shape) == (M, N)):
+        raise KernelError(f"the residual stream is float32 [{M}, {N}]")
+    lib = _load("gemm")
+    y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    squares = torch.empty((M, lib.cw_gemm_bf16_join_parts(M, N, K)), dtype=torch.float32, device=x.device)
+    _check(lib.cw_gemm_bf16_join(_ptr(x), _ptr(weight), _ptr(resid), _ptr(norm_weight), int(norm_weight.dtype == torch.float32), _ptr(y),
+                                 _ptr(squares), M, N, K, _stream()), "gemm_bf16_join")
+    return BegunNorm(y, squares, eps)
 
 
 def add_rmsnorm(resid, delta, weight, eps: float, out, rows=None, write_back: bool = True, weight2=None, out2=None) -> torch.Tensor:
@@ -1179,10 +1228,21 @@ def qkv_rope_fused_supported(x: torch.Tensor, weight: torch.Tensor, rotary_dim: 
             and K % 8 == 0 and rotary_dim == hd and hd % 16 == 0)
 
 
+def qkv_rope_begun_ok(M: int, weight: torch.Tensor, rotary_dim: int, hd: int) -> bool:
+    """Does ``qkv_rope_fused`` take a :class:`BegunNorm` of ``M`` rows?"""
+    return (1 <= M <= SKINNY_MAX_ROWS and weight.dtype == torch.bfloat16 and weight.is_contiguous() and weight.shape[1] % 8 == 0
+            and rotary_dim == hd and hd % 16 == 0 and _aligned(weight))
+
+
 def qkv_rope_fused(x, weight, bias, positions, slots, inv_freq, nh: int, nkv: int, hd: int, k_cache, v_cache) -> torch.Tensor:
     """q = rope(x @ Wq.T + bq) returned as [M, nh * hd]; rope(x @ Wk.T + bk) and x @ Wv.T + bv written
     to the cache rows ``slots``: one kernel for few rows, all operands of one type (a bias of bfloat16 rows may be float32; see
-    csrc/gemm.hip)."""
+    csrc/gemm.hip). ``x`` may be a :class:`BegunNorm` of up to 16 rows."""
+    begun = x if isinstance(x, BegunNorm) else None
+    if begun is not None:
+        x = begun.x
+        if x.shape[0] > SKINNY_MAX_ROWS:
+            raise KernelError("a begun norm has at most 16 rows")
     _gpu(x, weight, bias, positions, slots, inv_freq, k_cache, v_cache)
     M, K = x.shape
     if not (qkv_rope_fused_supported(x, weight, hd, hd, nh, nkv)):
@@ -1203,6 +1263,12 @@ def qkv_rope_fused(x, weight, bias, positions, slots, inv_freq, nh: int, nkv: in
     if x.dtype == torch.float32:
         _check(_load("gemm").cw_gemm_f32_pairs(_ptr(x), _ptr(weight), _ptr(bias), _ptr(positions), _ptr(slots), _ptr(inv_freq), _ptr(q),
                                                _ptr(k_cache), _ptr(v_cache), rows, M, K, nh, nkv, hd, _stream()), "gemm_f32_pairs")
+        return q
+    if begun is not None:
+        _check(_load("gemm").cw_gemm_qkv_rope_begun_bf16(
+            _ptr(x), _ptr(begun.squares), begun.squares.shape[1], float(begun.eps), _ptr(weight), _ptr(bias),
+            int(bias is not None and bias.dtype == torch.float32), _ptr(positions), _ptr(slots), _ptr(inv_freq), _ptr(q), _ptr(k_cache),
+            _ptr(v_cache), rows, M, K, nh, nkv, hd, _stream()), "gemm_qkv_rope_begun_bf16")
         return q
     _check(
         _load("gemm").cw_gemm_qkv_rope_bf16(
@@ -1262,6 +1328,12 @@ def swiglu_norm_fusable(M: int, two_i: int, K: int, dtype, gate_up_weight, delta
             and bool(_load("gemm").cw_gemm_bf16_swiglu_normed_ok(M, two_i, K)))
 
 
+def swiglu_begun_ok(M: int, gate_up_weight: torch.Tensor) -> bool:
+    """Does the gate/up product take a :class:`BegunNorm` of ``M`` rows?"""
+    return (1 <= M <= SKINNY_MAX_ROWS and gate_up_weight.dtype == torch.bfloat16 and gate_up_weight.is_contiguous()
+            and gate_up_weight.shape[0] % 2 == 0 and gate_up_weight.shape[1] % 8 == 0 and _aligned(gate_up_weight))
+
+
 def linear_swiglu(x, gate_up_weight: torch.Tensor, policy: "ProductPolicy | None" = None, limit: float = 0.0) -> torch.Tensor:
     """silu(x @ gate.T) * (x @ up.T) for gate_up_weight = [gate; up] stacked along dim 0; ``limit`` > 0 or
     ``RELU_GATE`` or ``GELU_GATE``: the other activations of the two products that ``silu_mul`` knows.
@@ -1284,6 +1356,16 @@ def linear_swiglu(x, gate_up_weight: torch.Tensor, policy: "ProductPolicy | None
             )
             return out
         x = x.value()
+    if isinstance(x, BegunNorm):
+        _gpu(x.x, x.squares, gate_up_weight)
+        M, K = x.shape
+        two_i = gate_up_weight.shape[0]
+        if not (limit == 0.0 and swiglu_begun_ok(M, gate_up_weight) and gate_up_weight.shape[1] == K):
+            raise KernelError("the gate/up product does not take a begun norm of these sizes")
+        out = torch.empty((M, two_i // 2), dtype=x.dtype, device=x.x.device)
+        _check(_load("gemm").cw_gemm_bf16_swiglu_begun(_ptr(x.x), _ptr(x.squares), x.squares.shape[1], float(x.eps), _ptr(gate_up_weight),
+                                                       _ptr(out), two_i // 2, M, two_i, K, _stream()), "gemm_bf16_swiglu_begun")
+        return out
     _gpu(x, gate_up_weight)
     M, K = x.shape
     two_i = gate_up_weight.shape[0]

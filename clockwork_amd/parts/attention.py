@@ -346,7 +346,25 @@ class PagedAttention(Part):
             self.compute_units = ops._compute_units(device)
         self.position.bind({}, device, dtype)
 
+    def takes_begun_norm(self, n_tokens: int, cache: EntryCache) -> bool:
+        """May ``forward``'s input be an ``ops.BegunNorm`` of that many rows?"""
+        takes = getattr(self.position, "takes_begun_norm", None)
+        return takes is not None and cache.writes and takes(n_tokens, self.qkv_weight, self.spec.head_dim)
+
+    def joins(self, n_tokens: int, norm) -> bool:
+        """Can ``forward_joined`` add that many rows to the stream and begin ``norm``?"""
+        return self.out_bias is None and ops.linear_join_ok(n_tokens, self.out_weight, norm.weight)
+
+    def forward_joined(self, x, ctx, cache: EntryCache, resid, norm) -> "ops.BegunNorm":
+        """``forward``, its output added to ``resid`` and ``norm`` of that begun."""
+        return ops.linear_join(self._before_output(x, ctx, cache), self.out_weight, resid, norm.weight, norm.spec.eps)
+
     def forward(self, x: torch.Tensor, ctx, cache: EntryCache) -> torch.Tensor:
+        return ops.linear(self._before_output(x, ctx, cache), self.out_weight, self.out_bias, partial_ok=True,
+                          policy=getattr(ctx, "products", None), portions_partial_ok=getattr(ctx, "reader_adds_sums", False))
+
+    def _before_output(self, x, ctx, cache: EntryCache) -> torch.Tensor:
+        """All but the product with ``out_weight``, [T, heads * head_dim]."""
         s = self.spec
         nh, nkv, hd = s.num_heads, s.num_kv_heads, s.head_dim
         policy = getattr(ctx, "products", None)
@@ -369,9 +387,7 @@ class PagedAttention(Part):
             qkv = ops.linear(x, self.qkv_weight[: self.q_width], policy=policy)
             bias = self.qkv_bias[: self.q_width] if self.qkv_bias is not None else None
             self.position.rotate_and_store(qkv, bias, ctx.positions, None, nh, 0, hd, None, None)
-        out = self.attend(qkv, ctx, cache)
-        return ops.linear(out, self.out_weight, self.out_bias, partial_ok=True, policy=policy,
-                          portions_partial_ok=getattr(ctx, "reader_adds_sums", False))
+        return self.attend(qkv, ctx, cache)
 
     def attend(self, q: torch.Tensor, ctx, cache: EntryCache) -> torch.Tensor:
         """Attention of the step's rotated queries (the first ``num_heads * head_dim`` columns of

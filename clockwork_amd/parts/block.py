@@ -35,10 +35,26 @@ class PreNormBlock:
         """The norm that takes what the block before hands on (may it be two pending outputs?)."""
         return self.mixer_norm
 
+    def norm_to_begin(self, n_tokens: int, cache):
+        """The norm that the block before may begin (``ops.linear_join``), handing on an ``ops.BegunNorm``; None if this
+        block's mixer does not take one of that many rows."""
+        takes = getattr(self.mixer, "takes_begun_norm", None)
+        if takes is not None and getattr(self.mixer_norm, "can_be_begun", False) and takes(n_tokens, cache):
+            return self.mixer_norm
+        return None
+
     def forward(self, resid, delta, ctx, cache):
-        x = self.mixer_norm.forward(resid, delta)
+        x = delta if isinstance(delta, ops.BegunNorm) else self.mixer_norm.forward(resid, delta)
         next_adds = getattr(ctx, "next_norm_adds_sums", False)
         ctx.reader_adds_sums = next_adds if self.feed_forward is None else getattr(self.ffn_norm, "adds_partial_sums", False)
+        # Few rows, with another block to follow (the final norm takes pending outputs, of the chosen rows alone): the mixer's
+        # output joins the stream and begins the second norm in the kernel of its last product, and so does the
+        # feed-forward's with the next block's first norm. Neither the residual adds nor the norms are launches then.
+        T = resid.shape[0]
+        joins = getattr(self.mixer, "joins", None) if getattr(ctx, "block_follows", False) else None
+        takes = getattr(self.feed_forward, "takes_begun_norm", None)
+        if joins is not None and takes is not None and getattr(self.ffn_norm, "can_be_begun", False) and takes(T) and joins(T, self.ffn_norm):
+            return self._feed(self.mixer.forward_joined(x, ctx, cache, resid, self.ffn_norm), resid, ctx, next_adds)
         a = self.mixer.forward(x, ctx, cache)
         if self.feed_forward is None:
             return a
@@ -51,7 +67,14 @@ class PreNormBlock:
         if (fuses is not None and lazy is not None and getattr(ctx, "next_norm_accepts_pending", False)
                 and fuses(resid.shape[0], x.dtype, a)):
             return ops.PendingPair(a, self.feed_forward.forward(lazy(resid, a), ctx))
-        x = self.ffn_norm.forward(resid, a)
+        return self._feed(self.ffn_norm.forward(resid, a), resid, ctx, next_adds)
+
+    def _feed(self, x, resid, ctx, next_adds: bool):
+        """The feed-forward of ``x``, the stream being up to date: its output, or the next block's norm begun."""
+        ctx.reader_adds_sums = next_adds
+        norm, joins = getattr(ctx, "norm_to_begin", None), getattr(self.feed_forward, "joins", None)
+        if norm is not None and joins is not None and joins(resid.shape[0], norm):
+            return self.feed_forward.forward_joined(x, ctx, resid, norm)
         return self.feed_forward.forward(x, ctx)
 
 

@@ -32,6 +32,19 @@ class SwiGLU(Part):
         H, I = self.spec.hidden_size, self.spec.intermediate_size
         return ops.swiglu_norm_fusable(n_tokens, 2 * I, H, dtype, self.gate_up, delta)
 
+    def takes_begun_norm(self, n_tokens: int) -> bool:
+        """May ``forward``'s input be an ``ops.BegunNorm`` of that many rows?"""
+        return ops.swiglu_begun_ok(n_tokens, self.gate_up)
+
+    def joins(self, n_tokens: int, norm) -> bool:
+        """Can ``forward_joined`` add that many rows to the stream and begin ``norm``?"""
+        return ops.linear_join_ok(n_tokens, self.down, norm.weight)
+
+    def forward_joined(self, x, ctx, resid, norm) -> "ops.BegunNorm":
+        """``forward``, its output added to ``resid`` and ``norm`` of that begun."""
+        inner = ops.linear_swiglu(x, self.gate_up, policy=getattr(ctx, "products", None))
+        return ops.linear_join(inner, self.down, resid, norm.weight, norm.spec.eps)
+
     def forward(self, x, ctx) -> torch.Tensor:
         policy = getattr(ctx, "products", None)
         return ops.linear(ops.linear_swiglu(x, self.gate_up, policy=policy), self.down, partial_ok=True, policy=policy,

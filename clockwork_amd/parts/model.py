@@ -204,6 +204,11 @@ class DecoderModel:
             # and may its output be the planes of a product of many rows? (a re-entry comes ahead of the next norm)
             reenters = i + 1 < len(run) and run[i + 1].reenter is not None
             ctx.next_norm_adds_sums = bool(getattr(nxt, "adds_partial_sums", False)) and not reenters
+            # few rows of bfloat16 may also join the stream where they are made, and begin the next block's first norm
+            ctx.block_follows = i + 1 < len(run)
+            plain = ctx.block_follows and not reenters and not run[i + 1].add_input and getattr(self, "dtype", None) == torch.bfloat16
+            begin = getattr(self.layers[run[i + 1].layer], "norm_to_begin", None) if plain else None
+            ctx.norm_to_begin = begin(resid.shape[0], caches[i + 1]) if begin is not None else None
             ctx.reader_adds_sums = False   # for a part of the block: does whoever reads its output add them? The block says so
             delta = self.layers[entry.layer].forward(resid, delta, ctx, caches[i])
         if ctx.num_logit_rows == 0:

@@ -43,6 +43,9 @@ class RMSNorm(Part):
         ops.add_rmsnorm(resid, delta, self.weight, self.spec.eps, out, weight2=other.weight, out2=out2)
         return out, out2
 
+    # a product that has added its output to the stream may begin this norm of it (``ops.linear_join``)
+    can_be_begun = True
+
     def lazy(self, resid: torch.Tensor, delta) -> "ops.LazyAddNorm":
         """The norm of resid + delta for a consumer that computes it inside its own kernel; the
         residual is not updated, so ``delta`` has to reach the next norm as well."""

@@ -63,6 +63,10 @@ class RopeNeox(Part):
         return ops.qkv_rope_fused(x, weight, bias, positions, slots, self.inv_freq, nh, nkv, hd, k_cache, v_cache)
 
 
+    def takes_begun_norm(self, n_tokens: int, weight, hd: int) -> bool:
+        """May the x of ``project_rotate_store`` be an ``ops.BegunNorm`` of that many rows?"""
+        return ops.qkv_rope_begun_ok(n_tokens, weight, self.spec.rotary_dim, hd)
+
     def project_rotate_store_rows(self, x, weight, bias, ctx, slots, nh, nkv, hd, k_cache, v_cache):
         """The same for a portion's rows: by a table of the step's angles, made by the first layer that asks in a pass
         over the model (``ctx.made``; 1 MB for 2048 tokens, 2 us), by every call

@@ -899,3 +899,53 @@ def test_streamed_products_of_fewer_steps_than_two_a_wave(M, K, N):
     want = torch.nn.functional.silu(y) * y.flip(1)
     keep = [i for i in rest if N - 1 - i in rest]
     torch.testing.assert_close(gated.double()[:, keep], want[:, keep], rtol=2.0 ** -8, atol=1e-5)
+
+
+# N, K: workgroups of 8 outputs by 8 waves (K up to 2048, the last one short), of 4, of up to 8 and up to 16 outputs by 16 waves, pieces
+# of a row no multiple of four, a K that ends inside an operand's pieces
+@pytest.mark.parametrize("N,K,most", [(900, 264, 16), (1536, 1536, 16), (896, 4864, 15), (1000, 2504, 16), (1537, 8960, 8), (2052, 600, 16), (3584, 3584, 16)])
+@pytest.mark.parametrize("norm_dtype", [torch.bfloat16, torch.float32])
+def test_products_that_join_the_stream_and_begin_a_norm(N, K, most, norm_dtype):
+    """The stream, the rows times the norm's weights and the sums of squares against float64, and the two products that
+    take such rows against themselves on rows that were normed before."""
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(N + K)
+    w = (torch.randn(N, K, device=DEV, generator=gen) / K ** 0.5).to(torch.bfloat16)
+    norm = (1 + 0.1 * torch.randn(N, device=DEV, generator=gen)).to(norm_dtype)
+    assert not ops.linear_join_ok(17, w, norm) and not ops.linear_join_ok(1, w[:, :200].contiguous(), norm)
+    width = N // 8 * 8   # the readers take rows in pieces of 16 bytes
+    hd, nh, nkv = 32, 5, 2
+    gate_up = (torch.randn(2 * 4104, width, device=DEV, generator=gen) / width ** 0.5).to(torch.bfloat16)
+    qkv = (torch.randn((nh + 2 * nkv) * hd, width, device=DEV, generator=gen) / width ** 0.5).to(torch.bfloat16)
+    inv_freq = 1.0 / 1e4 ** (torch.arange(0, hd, 2, device=DEV, dtype=torch.float32) / hd)
+    for M in (1, 2, most):
+        x = torch.randn(M, K, device=DEV, generator=gen).to(torch.bfloat16)
+        before = torch.randn(M, N, device=DEV, generator=gen)
+        resid = before.clone()
+        assert ops.linear_join_ok(M, w, norm)
+        begun = ops.linear_join(x, w, resid, norm, 1e-6)
+        want = before.double() + x.double() @ w.double().t()
+        # float32 sums of K products of about 1 / sqrt(K): sqrt(K) roundings of 2^-24 at most, ten times that
+        assert float((resid.double() - want).abs().max()) < 10 * 2.0 ** -24 * K ** 0.5
+        torch.testing.assert_close(begun.x.double(), want * norm.double(), rtol=2.0 ** -8, atol=1e-5)
+        torch.testing.assert_close(begun.squares.double().sum(1), want.square().sum(1), rtol=1e-5, atol=0)
+        if N != width:
+            continue
+        # x by its norm in float64, rounded once: what the readers differ by is where the factor joins, 2^-9 of each of
+        # ``width`` products of about 1 / sqrt(width) on either side, and the rounding of the result
+        normed = want * torch.rsqrt(want.square().mean(-1, keepdim=True) + 1e-6) * norm.double()
+        y = normed @ gate_up.double().t()
+        inner = torch.nn.functional.silu(y[:, :4104]) * y[:, 4104:]
+        got = ops.linear_swiglu(begun, gate_up).double()
+        assert float((got - inner).norm() / inner.norm()) < 4 * 2.0 ** -9
+        positions = torch.arange(M, dtype=torch.int32, device=DEV) * 7
+        slots = torch.arange(M, dtype=torch.int32, device=DEV) * 2 + 1
+        caches = [torch.zeros(2 * M + 2, nkv, hd, dtype=torch.bfloat16, device=DEV) for _ in range(4)]
+        q = ops.qkv_rope_fused(begun, qkv, None, positions, slots, inv_freq, nh, nkv, hd, *caches[:2])
+        q2 = ops.qkv_rope_fused(normed.to(torch.bfloat16), qkv, None, positions, slots, inv_freq, nh, nkv, hd, *caches[2:])
+        for a, b in ((q, q2), (caches[0], caches[2]), (caches[1], caches[3])):
+            assert float((a.double() - b.double()).norm() / b.double().norm()) < 6 * 2.0 ** -9
+    with pytest.raises(ops.KernelError):
+        ops.linear_swiglu(ops.BegunNorm(torch.zeros(17, 1024, dtype=torch.bfloat16, device=DEV), torch.zeros(17, 4, device=DEV), 1e-6),
+                          torch.zeros(64, 1024, dtype=torch.bfloat16, device=DEV))

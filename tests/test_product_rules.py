@@ -281,3 +281,51 @@ def test_few_small_tiles_rather_than_many_runs(M, N, K, want):
 @pytest.mark.parametrize("M,N,K,there", [(1500, 6144, 3072, True), (1600, 6144, 3072, False), (2048, 6144, 3072, False), (2048, 5120, 2048, True), (2048, 4608, 3584, True)])
 def test_large_outputs_of_a_long_k_are_the_librarys(M, N, K, there):
     assert (_wide_choice(0, M, N, K) is not None) == there
+
+
+def test_few_rows_join_the_stream_between_blocks_only():
+    """The mixer's output begins the second norm and the feed-forward's the next block's first one, where the parts take such
+    rows and another block follows; the last block leaves its outputs to the final norm."""
+    import torch
+
+    from clockwork_amd.parts.block import PreNormBlock
+
+    calls = []
+
+    class Piece:
+        def __init__(self, name, most):
+            self.name, self.most = name, most
+
+        def takes_begun_norm(self, n, *cache):
+            return n <= self.most
+
+        def joins(self, n, norm):
+            return n <= self.most
+
+        def forward(self, x, *rest):
+            calls.append((self.name, type(x).__name__))
+            return torch.zeros(1)
+
+        def forward_joined(self, x, *rest):
+            calls.append((self.name + " joins", type(x).__name__, rest[-1].name))
+            return ops.BegunNorm(torch.zeros(1), torch.zeros(1), 1e-6)
+
+    def norm(name, begun=True):
+        return SimpleNamespace(name=name, can_be_begun=begun, forward=lambda resid, delta: calls.append(name) or torch.zeros(1))
+
+    def run(rows, follows, nxt, delta=None, begun=True):
+        calls.clear()
+        block = PreNormBlock(Piece("mixer", 16), norm("n1", begun), Piece("ffn", 16), norm("n2", begun))
+        ctx = SimpleNamespace(block_follows=follows, norm_to_begin=nxt)
+        out = block.forward(SimpleNamespace(shape=(rows, 8)), delta, ctx, None)
+        return list(calls), isinstance(out, ops.BegunNorm), block.norm_to_begin(rows, None)
+
+    nxt, begun = norm("next"), ops.BegunNorm(torch.zeros(1), torch.zeros(1), 1e-6)
+    got, joined, first = run(4, True, nxt)
+    assert got == ["n1", ("mixer joins", "Tensor", "n2"), ("ffn joins", "BegunNorm", "next")] and joined and first.name == "n1"
+    got, joined, _ = run(4, True, nxt, begun)
+    assert got == [("mixer joins", "BegunNorm", "n2"), ("ffn joins", "BegunNorm", "next")] and joined
+    assert run(4, True, None)[:2] == (["n1", ("mixer joins", "Tensor", "n2"), ("ffn", "BegunNorm")], False)
+    assert run(4, False, None, begun)[:2] == ([("mixer", "BegunNorm"), "n2", ("ffn", "Tensor")], False)
+    assert run(17, True, None) == (["n1", ("mixer", "Tensor"), "n2", ("ffn", "Tensor")], False, None)
+    assert run(4, True, None, begun=False) == (["n1", ("mixer", "Tensor"), "n2", ("ffn", "Tensor")], False, None)
