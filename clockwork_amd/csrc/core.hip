@@ -286,6 +286,44 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict_
   }
 }
 
+// Chosen rows of up to four matrices, one after the other: a workgroup a row and matrix. What a model's last block keeps of a
+// portion once its mixer has seen every token: bound by its launch (1 row of 4 KB and one of 6: 2.2 us inside a graph).
+#define TAKE_MAX 4
+struct TakeRows {
+  const unsigned char* src[TAKE_MAX];
+  unsigned char* dst[TAKE_MAX];
+  int64_t bytes[TAKE_MAX];  // of a row
+};
+template <typename V>
+__global__ __launch_bounds__(256) void take_rows_kernel(TakeRows t, const int* __restrict__ rows, int n_rows) {
+  const int i = blockIdx.x, at = rows[i];
+  if (at < 0 || at >= n_rows) return;
+  const int64_t n = t.bytes[blockIdx.y] / (int64_t)sizeof(V);
+  const V* from = reinterpret_cast<const V*>(t.src[blockIdx.y] + at * t.bytes[blockIdx.y]);
+  V* to = reinterpret_cast<V*>(t.dst[blockIdx.y] + i * t.bytes[blockIdx.y]);
+  for (int64_t j = threadIdx.x; j < n; j += 256) to[j] = from[j];
+}
+// dst[i] row r = src[i] row rows[r] for ``count`` matrices of ``n_rows`` rows without gaps, ``bytes[i]`` (even) a row. A row index
+// outside the matrix writes nothing.
+CW_EXPORT int cw_take_rows(int count, const void* const* src, void* const* dst, const int64_t* bytes, const int* rows, int n, int n_rows,
+                           hipStream_t stream) {
+  if (count < 1 || count > TAKE_MAX || n < 0 || n_rows <= 0 || !src || !dst || !bytes || !rows) return CW_ERR_ARG;
+  TakeRows t{};
+  uintptr_t bits = 0;
+  for (int i = 0; i < count; ++i) {
+    if (!src[i] || !dst[i] || bytes[i] <= 0 || (bytes[i] & 1)) return CW_ERR_ARG;
+    t.src[i] = (const unsigned char*)src[i];
+    t.dst[i] = (unsigned char*)dst[i];
+    t.bytes[i] = bytes[i];
+    bits |= (uintptr_t)src[i] | (uintptr_t)dst[i] | (uintptr_t)bytes[i];
+  }
+  if (n == 0) return CW_OK;
+  if ((bits & 15) == 0) hipLaunchKernelGGL(take_rows_kernel<uint4>, dim3(n, count), dim3(256), 0, stream, t, rows, n_rows);
+  else if ((bits & 1) == 0) hipLaunchKernelGGL(take_rows_kernel<uint16_t>, dim3(n, count), dim3(256), 0, stream, t, rows, n_rows);
+  else return CW_ERR_ARG;
+  return cw_launch_status();
+}
+
 // delta: nullptr, or [T, H] in the activation type (delta_parts == 0), or float32 [delta_parts, T, H].
 // delta0: nullptr, or [T, H] in the activation type, added to the residual before delta.
 CW_EXPORT int cw_add_rmsnorm(float* resid, const void* delta0, const void* delta, int delta_parts, int T_rows,

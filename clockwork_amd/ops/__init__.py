@@ -101,6 +101,7 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_copy_pages": [P, I, L, L, P, I, P],
             "cw_fresh_state_rows": [P, I, I, I, I, L, P, P, I, P],
             "cw_bf16_to_f32": [P, P, L, P],
+            "cw_take_rows": [I, P, P, P, P, I, I, P],
         },
         "gemm": {
             "cw_gemm_f32": [P, L, P, P, P, L, I, I, I, P, L, P],
@@ -336,6 +337,20 @@ def embedding(table: torch.Tensor, ids: torch.Tensor, out_resid: torch.Tensor) -
         "embedding",
     )
     return out_resid
+
+
+def take_rows(rows: torch.Tensor, *matrices) -> list:
+    """[m[rows] for m in matrices] for up to four matrices of the same number of rows, in one launch."""
+    T, n = matrices[0].shape[0], rows.numel()
+    _gpu(rows, *matrices)
+    _i32(rows, n, "rows")
+    if not all(m.dim() == 2 and m.shape[0] == T and m.element_size() % 2 == 0 for m in matrices):
+        raise KernelError("rows are taken of matrices of one number of rows")
+    out = [torch.empty((n, m.shape[1]), dtype=m.dtype, device=m.device) for m in matrices]
+    pointers, sizes = ctypes.c_void_p * len(out), ctypes.c_int64 * len(out)
+    _check(_load("core").cw_take_rows(len(out), pointers(*(m.data_ptr() for m in matrices)), pointers(*(o.data_ptr() for o in out)),
+                                      sizes(*(m.shape[1] * m.element_size() for m in matrices)), _ptr(rows), n, T, _stream()), "take_rows")
+    return out
 
 
 class PartialSums:

@@ -360,8 +360,16 @@ class PagedAttention(Part):
         return ops.linear_join(self._before_output(x, ctx, cache), self.out_weight, resid, norm.weight, norm.spec.eps)
 
     def forward(self, x: torch.Tensor, ctx, cache: EntryCache) -> torch.Tensor:
-        return ops.linear(self._before_output(x, ctx, cache), self.out_weight, self.out_bias, partial_ok=True,
-                          policy=getattr(ctx, "products", None), portions_partial_ok=getattr(ctx, "reader_adds_sums", False))
+        return self.output(self._before_output(x, ctx, cache), ctx)
+
+    def forward_rows(self, x, ctx, cache: EntryCache, rows, *others) -> tuple:
+        """``forward``'s ``rows``, the cache being left as by all of them, and the same rows of ``others``."""
+        out, *others = ops.take_rows(rows, self._before_output(x, ctx, cache), *others)
+        return self.output(out, ctx), others
+
+    def output(self, out: torch.Tensor, ctx):
+        return ops.linear(out, self.out_weight, self.out_bias, partial_ok=True, policy=getattr(ctx, "products", None),
+                          portions_partial_ok=getattr(ctx, "reader_adds_sums", False))
 
     def _before_output(self, x, ctx, cache: EntryCache) -> torch.Tensor:
         """All but the product with ``out_weight``, [T, heads * head_dim]."""

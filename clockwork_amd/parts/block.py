@@ -55,7 +55,23 @@ class PreNormBlock:
         takes = getattr(self.feed_forward, "takes_begun_norm", None)
         if joins is not None and takes is not None and getattr(self.ffn_norm, "can_be_begun", False) and takes(T) and joins(T, self.ffn_norm):
             return self._feed(self.mixer.forward_joined(x, ctx, cache, resid, self.ffn_norm), resid, ctx, next_adds)
-        a = self.mixer.forward(x, ctx, cache)
+        return self._after(self.mixer.forward(x, ctx, cache), resid, x.dtype, ctx, next_adds)
+
+    def takes_rows(self) -> bool:
+        """Can the block make chosen rows of its output alone (``forward_rows``)?"""
+        return hasattr(self.mixer, "forward_rows") and (self.feed_forward is None or getattr(self.feed_forward, "by_rows", False))
+
+    def forward_rows(self, resid, delta, ctx, cache, rows):
+        """``forward`` of the last block of a step: (the stream's ``rows``, what is still to be added to these). The cache
+        is left as by all rows; what follows the mixer is made of the chosen ones."""
+        x = delta if isinstance(delta, ops.BegunNorm) else self.mixer_norm.forward(resid, delta)
+        next_adds = getattr(ctx, "next_norm_adds_sums", False)
+        ctx.reader_adds_sums = next_adds if self.feed_forward is None else getattr(self.ffn_norm, "adds_partial_sums", False)
+        a, (resid,) = self.mixer.forward_rows(x, ctx, cache, rows, resid)
+        return resid, self._after(a, resid, x.dtype, ctx, next_adds)
+
+    def _after(self, a, resid, dtype, ctx, next_adds: bool):
+        """What the block hands on once its mixer's output ``a`` is there."""
         if self.feed_forward is None:
             return a
         ctx.reader_adds_sums = next_adds
@@ -65,7 +81,7 @@ class PreNormBlock:
         fuses = getattr(self.feed_forward, "fuses_input_norm", None)
         lazy = getattr(self.ffn_norm, "lazy", None)
         if (fuses is not None and lazy is not None and getattr(ctx, "next_norm_accepts_pending", False)
-                and fuses(resid.shape[0], x.dtype, a)):
+                and fuses(resid.shape[0], dtype, a)):
             return ops.PendingPair(a, self.feed_forward.forward(lazy(resid, a), ctx))
         return self._feed(self.ffn_norm.forward(resid, a), resid, ctx, next_adds)
 
@@ -146,6 +162,21 @@ class ParallelBlock:
         weights = first + (self.gate.input_weights() if first and self.gate is not None else [])
         made = ops.linear_several([x] * len(weights), weights) if len(weights) > 1 else None
         a = self.mixer.forward(x, ctx, cache) if made is None else self.mixer.forward(x, ctx, cache, made[: len(first)])
+        return self._after(x, a, resid, ctx, made)
+
+    def takes_rows(self) -> bool:
+        """Can the block make chosen rows of its output alone (``forward_rows``)?"""
+        return getattr(self.mixer, "takes_rows", lambda: False)() and (self.feed_forward is None or getattr(self.feed_forward, "by_rows", False))
+
+    def forward_rows(self, resid, delta, ctx, cache, rows):
+        """``forward`` of the last block of a step: (the stream's ``rows``, what is still to be added to these). The cache
+        is left as by all rows; what follows the mixer, and the feed-forward and the gates, are made of the chosen ones."""
+        x = self.mixer_norm.forward(resid, delta)
+        a, (x, resid) = self.mixer.forward_rows(x, ctx, cache, rows, x, resid)
+        return resid, self._after(x, a, resid, ctx, None)
+
+    def _after(self, x, a, resid, ctx, made):
+        """What the block hands on once its mixer's output ``a`` of its input ``x`` is there."""
         b = self.feed_forward.forward(x, ctx) if self.feed_forward is not None else None
         if made is not None and self.gate is not None:
             z = made[-1]

@@ -15,6 +15,7 @@ from clockwork_amd.parts.specs import SwiGLUSpec
 
 class SwiGLU(Part):
     graph_safe = True
+    by_rows = True   # a row of the output depends on that row of the input and on nothing else of the step
     def __init__(self, spec: SwiGLUSpec) -> None:
         self.spec = spec
 
@@ -56,6 +57,7 @@ class GatedMLP(Part):
     kernels of :class:`SwiGLU`."""
 
     graph_safe = True
+    by_rows = True
     partial_ok = False   # may the output come as ``ops.PartialSums``? A block whose next norm adds them up sets it
 
     def __init__(self, spec) -> None:

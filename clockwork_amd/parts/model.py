@@ -210,7 +210,15 @@ class DecoderModel:
             begin = getattr(self.layers[run[i + 1].layer], "norm_to_begin", None) if plain else None
             ctx.norm_to_begin = begin(resid.shape[0], caches[i + 1]) if begin is not None else None
             ctx.reader_adds_sums = False   # for a part of the block: does whoever reads its output add them? The block says so
-            delta = self.layers[entry.layer].forward(resid, delta, ctx, caches[i])
+            layer = self.layers[entry.layer]
+            # Only the rows that logits are asked of go on behind the last mixer, which every token's cache needs: of a prompt
+            # one. Above half of the rows taking them apart costs what it saves; a model of a single block makes all rows (it is
+            # run to look at that block's kernels).
+            if (i > 0 and not ctx.block_follows and 0 < 2 * ctx.num_logit_rows <= resid.shape[0] and getattr(self.final_norm, "takes_all_rows", False)
+                    and getattr(layer, "takes_rows", lambda: False)()):
+                resid, delta = layer.forward_rows(resid, delta, ctx, caches[i], ctx.logit_rows)
+                return self.head.forward(self.final_norm.forward(resid, delta), ctx)
+            delta = layer.forward(resid, delta, ctx, caches[i])
         if ctx.num_logit_rows == 0:
             return None
         rows = self.final_norm.forward(resid, delta, rows=ctx.logit_rows)

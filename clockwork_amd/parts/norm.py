@@ -12,6 +12,8 @@ from clockwork_amd.parts.specs import RMSNormSpec
 
 class RMSNorm(Part):
     graph_safe = True
+    # as a final norm: without ``rows`` it norms the whole of a stream that holds the chosen rows alone
+    takes_all_rows = True
     # takes a delta that is an ops.PendingPair (two branch outputs not yet added to the residual)
     accepts_pending = True
     # adds a delta that is an ops.PartialSums in its kernel, however many planes there are
@@ -58,6 +60,7 @@ class LayerNorm(Part):
     block's gated branches (``ops.GatedBranches``): the gates' sigmoids are made inside the kernel."""
 
     graph_safe = True
+    takes_all_rows = True
     accepts_gated = True
 
     def __init__(self, spec) -> None:

@@ -112,18 +112,35 @@ class PairMixer(Part):
         own = [getattr(m, "input_weights", list)() for m in (self.left, self.right)]
         return [] if self.joint or not all(own) else own[0] + own[1]
 
+    def takes_rows(self) -> bool:
+        """Can ``forward_rows`` make chosen rows of the output alone?"""
+        return not self.joint and all(hasattr(m, "before_output") for m in (self.left, self.right))
+
+    def forward_rows(self, x, ctx, cache: EntryCache, rows, *others) -> tuple:
+        """``forward``'s ``rows``, the caches being left as by all of them, and the same rows of ``others``."""
+        a, b, *others = ops.take_rows(rows, *self._before_outputs(x, ctx, *self._caches(cache), None), *others)
+        return ops.rms_mean2(*self._last_products([a, b], ctx), self.left_norm, self.right_norm, self.spec.eps), others
+
     def _outputs(self, x, ctx, left, right, made):
-        """The two mixers' outputs; the last product of each as one launch where they are of the same few rows and one K."""
+        """The two mixers' outputs."""
+        if not all(hasattr(m, "before_output") for m in (self.left, self.right)):
+            mine = len(self.left.input_weights()) if made is not None else 0
+            return [m.forward(x, ctx, own) if given is None else m.forward(x, ctx, own, given)
+                    for m, own, given in ((self.left, left, made and made[:mine]), (self.right, right, made and made[mine:]))]
+        return self._last_products(self._before_outputs(x, ctx, left, right, made), ctx)
+
+    def _before_outputs(self, x, ctx, left, right, made) -> list:
+        """All but the two mixers' last products."""
         mine = len(self.left.input_weights()) if made is not None else 0
         each = ((self.left, left, made and made[:mine]), (self.right, right, made and made[mine:]))
-        if not all(hasattr(m, "before_output") for m, _, _ in each):
-            return [m.forward(x, ctx, own) if given is None else m.forward(x, ctx, own, given) for m, own, given in each]
         if hasattr(self.right, "prepared_output") and getattr(self.left, "takes_beside", lambda *a: False)(x, ctx):
             b, launch = self.right.prepared_output(x, ctx, *each[1][1:])
-            outs = [self.left.before_output(x, ctx, *each[0][1:], beside=launch), b]
-        else:
-            outs = [m.before_output(x, ctx, own, given) for m, own, given in each]
-        weights = [m.out_weight for m, _, _ in each]
+            return [self.left.before_output(x, ctx, *each[0][1:], beside=launch), b]
+        return [m.before_output(x, ctx, own, given) for m, own, given in each]
+
+    def _last_products(self, outs: list, ctx) -> list:
+        """The two mixers' last products, as one launch where they are of the same few rows and one K."""
+        weights = [m.out_weight for m in (self.left, self.right)]
         return ops.linear_several(outs, weights) or [ops.linear(o, w, policy=getattr(ctx, "products", None)) for o, w in zip(outs, weights)]
 
     def forward(self, x: torch.Tensor, ctx, cache: EntryCache, made=None):

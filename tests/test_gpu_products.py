@@ -949,3 +949,44 @@ def test_products_that_join_the_stream_and_begin_a_norm(N, K, most, norm_dtype):
     with pytest.raises(ops.KernelError):
         ops.linear_swiglu(ops.BegunNorm(torch.zeros(17, 1024, dtype=torch.bfloat16, device=DEV), torch.zeros(17, 4, device=DEV), 1e-6),
                           torch.zeros(64, 1024, dtype=torch.bfloat16, device=DEV))
+
+
+@pytest.mark.parametrize("widths,T,chosen", [((1536,), 1, [0]), ((1536, 1024, 896, 8), 300, [299, 0, 0, 17]), ((7, 3), 40, [39]), ((4097, 2), 5, [4, 3])])
+def test_chosen_rows_of_several_matrices(widths, T, chosen):
+    from clockwork_amd import ops
+
+    rows = torch.tensor(chosen, dtype=torch.int32, device=DEV)
+    matrices = [torch.randn(T, n, device=DEV).to(torch.float32 if i % 2 == 0 else torch.bfloat16) for i, n in enumerate(widths)]
+    for got, m in zip(ops.take_rows(rows, *matrices), matrices):
+        assert torch.equal(got, m[rows.long()])
+    with pytest.raises(ops.KernelError):
+        ops.take_rows(rows, matrices[0], torch.zeros(T + 1, 8, device=DEV))
+    with pytest.raises(ops.KernelError):
+        ops.take_rows(rows.long(), matrices[0])
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("wanted", [[4], [0, 9], list(range(5)), list(range(6))])
+def test_the_last_block_makes_the_rows_that_are_asked_for(tmp_path, dtype, wanted):
+    """Logits of one, two and half of a portion's rows, which the last block makes alone, and of more, which come with all,
+    against those of all rows; and the token after them, which reads the last block's cache."""
+    from clockwork_amd.engine.batch import StepEntry
+    from clockwork_amd.weights.random_init import write_random_model
+    from tests import replay
+    from tests.configs import TINY_B
+
+    model_dir = write_random_model(tmp_path / "model", TINY_B, 5)
+    tokens = torch.randint(0, TINY_B["vocab_size"], (11,), generator=torch.Generator().manual_seed(2)).tolist()
+
+    def logits(rows):
+        runner = replay.make_runner(model_dir, dtype, 8, 16)
+        runner.reserve("r", 0, 10)
+        first = runner.step([StepEntry("r", 0, tokens[:10], rows)]).clone()
+        runner.reserve("r", 10, 1)
+        return first, runner.step([StepEntry("r", 10, tokens[10:], [0])]).clone()
+
+    all_rows, after = logits(list(range(10)))
+    got, then = logits(wanted)
+    bound = dict(rtol=1e-5, atol=1e-5) if dtype == "float32" else dict(rtol=2e-2, atol=2e-2)   # roundings of bfloat16 in another kernel
+    torch.testing.assert_close(got, all_rows[wanted], **bound)
+    torch.testing.assert_close(then, after, **bound)
