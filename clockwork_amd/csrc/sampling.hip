@@ -240,7 +240,7 @@ struct SampleArgs {
   const int* top_k;
   const float* top_p;
   const int64_t* seeds;
-  const int64_t* draws;
+  const int64_t* draws;   // nullptr: they come with the launch (DrawCounts)
   int* out;
   // workspace
   u64_t* hist_w;      // [n][SAMPLE_BINS], zeroed by MAX as hist_n
@@ -252,6 +252,13 @@ struct SampleArgs {
   float* pmax;        // [n][chunks]
   int* pmax_i;        // [n][chunks]
   float* points;      // [n][SAMPLE_POINTS]
+};
+
+// How many draws each of up to 64 rows has made, in the kernel's arguments: what changes from one step of a batch to the next is
+// then no copy to the device (a launch of its own, and twice as long on the host as the kernels' four: 38 -> 21 us a call of few rows).
+#define SAMPLE_COUNTED_ROWS 64
+struct DrawCounts {
+  uint32_t of_row[SAMPLE_COUNTED_ROWS];
 };
 
 // Chunks a row is cut into: at least 2048 tokens each; 64 for few rows, for many rows as few as still make two
@@ -474,12 +481,12 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_max_kernel(SampleArgs a
 // Draws the row's token among those whose scaled key is floor_key or more; ``chunk_w`` (LDS): what each chunk's
 // such tokens weigh. All threads of one workgroup.
 __device__ __forceinline__ void sample_locate(const SampleArgs& a, int row, float temp, float mx, int mi, uint32_t floor_key,
-                                              const u64_t* chunk_w) {
+                                              const u64_t* chunk_w, const DrawCounts& counts) {
   __shared__ int sel_chunk, sel_run, found;
   __shared__ u64_t sel_base, sel_total;
   if (threadIdx.x == 0) sel_chunk = sel_run = 0, found = -1, sel_base = 0;
   __syncthreads();
-  const uint32_t r = philox_first_word((uint64_t)a.seeds[row], (uint64_t)a.draws[row]);
+  const uint32_t r = philox_first_word((uint64_t)a.seeds[row], a.draws ? (uint64_t)a.draws[row] : (uint64_t)counts.of_row[row]);
   if (threadIdx.x < 64) {  // the chunk the target falls into: a running sum over the chunks
     const u64_t v = (int)threadIdx.x < a.chunks ? chunk_w[threadIdx.x] : 0;
     u64_t incl = v;
@@ -724,7 +731,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(SampleAr
 }
 
 // DRAW; ``again``: behind COLLECT's second run
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(SampleArgs a, int again) {
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(SampleArgs a, int again, DrawCounts counts) {
   __shared__ u64_t chunk_w[SAMPLE_MAX_CHUNKS];
   __shared__ u64_t bins_w[256];
   __shared__ uint32_t bins_n[256];
@@ -745,7 +752,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(SampleArgs 
   if ((int)threadIdx.x < a.chunks) chunk_w[threadIdx.x] = a.sums[(int64_t)row * a.chunks + threadIdx.x];
   __syncthreads();
   if (!with_k && !with_p) {
-    sample_locate(a, row, temp, mx, mi, 0u, chunk_w);
+    sample_locate(a, row, temp, mx, mi, 0u, chunk_w, counts);
     return;
   }
   const uint32_t listed = known.listed[again];
@@ -905,16 +912,16 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(SampleArgs 
     }
   }
   __syncthreads();
-  sample_locate(a, row, temp, mx, mi, floor_key, chunk_w);
+  sample_locate(a, row, temp, mx, mi, floor_key, chunk_w, counts);
 }
 
 // flags: bit 0 some row may have top-k, bit 1 some row may have top-p (3 when unknown), bit 2 no row has both: the steps
 // no row needs are not launched. workspace: cw_sample_workspace_bytes(n, V) bytes, 16-byte
 // aligned.
-CW_EXPORT int cw_sample(const float* logits, int64_t row_stride, int n, int V,
-                        const float* temperature, const int* top_k, const float* top_p,
-                        const int64_t* seeds, const int64_t* draws, int* out, void* workspace,
-                        int64_t workspace_bytes, int flags, hipStream_t stream) {
+static int launch_sample(const float* logits, int64_t row_stride, int n, int V,
+                         const float* temperature, const int* top_k, const float* top_p,
+                         const int64_t* seeds, const int64_t* draws, const DrawCounts& counts, int* out, void* workspace,
+                         int64_t workspace_bytes, int flags, hipStream_t stream) {
   if (n < 0 || V <= 0 || row_stride < V) return CW_ERR_ARG;
   if (n == 0) return CW_OK;
   if (n > 65535) return CW_ERR_SIZE;
@@ -943,11 +950,33 @@ CW_EXPORT int cw_sample(const float* logits, int64_t row_stride, int n, int V,
   hipLaunchKernelGGL(sample_max_kernel, grid, block, 0, stream, a);
   hipLaunchKernelGGL(sample_hist_kernel, grid, block, 0, stream, a);
   if (flags & 3) hipLaunchKernelGGL(sample_collect_kernel, grid, block, 0, stream, a, 0);
-  hipLaunchKernelGGL(sample_draw_kernel, dim3(n), block, 0, stream, a, 0);
+  hipLaunchKernelGGL(sample_draw_kernel, dim3(n), block, 0, stream, a, 0, counts);
   if ((flags & 7) == 3) {
     hipLaunchKernelGGL(sample_collect_kernel, grid, block, 0, stream, a, 1);
-    hipLaunchKernelGGL(sample_draw_kernel, dim3(n), block, 0, stream, a, 1);
+    hipLaunchKernelGGL(sample_draw_kernel, dim3(n), block, 0, stream, a, 1, counts);
   }
   return cw_launch_status();
+}
+CW_EXPORT int cw_sample(const float* logits, int64_t row_stride, int n, int V,
+                        const float* temperature, const int* top_k, const float* top_p,
+                        const int64_t* seeds, const int64_t* draws, int* out, void* workspace,
+                        int64_t workspace_bytes, int flags, hipStream_t stream) {
+  if (n > 0 && !draws) return CW_ERR_ARG;
+  return launch_sample(logits, row_stride, n, V, temperature, top_k, top_p, seeds, draws, DrawCounts{}, out, workspace, workspace_bytes, flags,
+                       stream);
+}
+// The same for up to 64 rows whose draw counts [n] (0 to 2^32 - 1) lie in host memory and are read before the call returns.
+CW_EXPORT int cw_sample_counted(const float* logits, int64_t row_stride, int n, int V,
+                                const float* temperature, const int* top_k, const float* top_p,
+                                const int64_t* seeds, const int64_t* host_draws, int* out, void* workspace,
+                                int64_t workspace_bytes, int flags, hipStream_t stream) {
+  if (n > SAMPLE_COUNTED_ROWS) return CW_ERR_SIZE;
+  if (n > 0 && !host_draws) return CW_ERR_ARG;
+  DrawCounts counts{};
+  for (int i = 0; i < n; ++i) {
+    if (host_draws[i] < 0 || host_draws[i] > (int64_t)UINT32_MAX) return CW_ERR_ARG;
+    counts.of_row[i] = (uint32_t)host_draws[i];
+  }
+  return launch_sample(logits, row_stride, n, V, temperature, top_k, top_p, seeds, nullptr, counts, out, workspace, workspace_bytes, flags, stream);
 }
 static_assert(sizeof(SampleRow) % 8 == 0 && sizeof(SampleRow) / 4 <= SAMPLE_THREADS, "MAX zeroes a row's record, a word a thread");

@@ -250,6 +250,7 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_argmax_static_init": [],
             "cw_argmax_static": [P, L, I, I, P, P],
             "cw_sample": [P, L, I, I, P, P, P, P, P, P, P, L, I, P],
+            "cw_sample_counted": [P, L, I, I, P, P, P, P, P, P, P, L, I, P],
             "cw_sample_workspace_bytes": [I, I],
         },
         "attention": {
@@ -1685,10 +1686,12 @@ def argmax(logits: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tenso
 
 def sample(logits, temperature, top_k, top_p, seeds, draws, out=None, any_top_k: bool = True,
            any_top_p: bool = True, any_both: bool = True) -> torch.Tensor:
-    """One token per row: rows with temperature 0 take the arg-max, the others are drawn.
+    """One token per row: rows with temperature 0 take the arg-max, the others are drawn. ``draws``, how many draws each row
+    has made: int64 [n] on the device or, of up to ``SAMPLE_COUNTED_ROWS`` rows, a list of ints, which go with the launch.
     ``any_top_k`` / ``any_top_p`` / ``any_both`` off: the caller knows that no row has that option
     (or both of them), and its kernels are not launched."""
-    _gpu(logits, temperature, top_k, top_p, seeds, draws, out)
+    counted = not isinstance(draws, torch.Tensor)
+    _gpu(logits, temperature, top_k, top_p, seeds, None if counted else draws, out)
     if not (logits.dtype == torch.float32 and logits.dim() == 2):
         raise KernelError("logits must be float32 [n, V]")
     n, V = logits.shape
@@ -1699,19 +1702,27 @@ def sample(logits, temperature, top_k, top_p, seeds, draws, out=None, any_top_k:
     _i32(top_k, n, "top_k")
     if not (seeds.dtype == torch.int64 and seeds.numel() == n):
         raise KernelError("seeds must be int64 [n]")
-    if not (draws.dtype == torch.int64 and draws.numel() == n):
+    if counted:
+        if not (len(draws) == n <= SAMPLE_COUNTED_ROWS and (n == 0 or 0 <= min(draws) <= max(draws) < 1 << 32)):
+            raise KernelError(f"draw counts on the host are [n], for up to {SAMPLE_COUNTED_ROWS} rows")
+    elif not (draws.dtype == torch.int64 and draws.numel() == n):
         raise KernelError("draws must be int64 [n]")
     if out is None:
         out = torch.empty(n, dtype=torch.int32, device=logits.device)
     _i32(out, n, "out")
     lib = _load("sampling")
     ws = torch.empty(int(lib.cw_sample_workspace_bytes(n, V)), dtype=torch.uint8, device=logits.device)
+    call, made = (lib.cw_sample_counted, (ctypes.c_int64 * n)(*draws)) if counted else (lib.cw_sample, _ptr(draws))
     _check(
-        lib.cw_sample(_ptr(logits), V, n, V, _ptr(temperature), _ptr(top_k), _ptr(top_p), _ptr(seeds), _ptr(draws),
-                      _ptr(out), _ptr(ws), ws.numel(), int(bool(any_top_k)) | (int(bool(any_top_p)) << 1) | (int(not any_both) << 2), _stream()),
+        call(_ptr(logits), V, n, V, _ptr(temperature), _ptr(top_k), _ptr(top_p), _ptr(seeds), made,
+             _ptr(out), _ptr(ws), ws.numel(), int(bool(any_top_k)) | (int(bool(any_top_p)) << 1) | (int(not any_both) << 2), _stream()),
         "sample",
     )
     return out
+
+
+# rows whose draw counts ``sample`` takes from the host (SAMPLE_COUNTED_ROWS in csrc/sampling.hip)
+SAMPLE_COUNTED_ROWS = 64
 
 
 # ---------------------------------------------------------------------------------------------

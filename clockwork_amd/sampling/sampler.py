@@ -73,7 +73,7 @@ class Sampler:
         if fixed is None:
             params = [s.sampling_params for s in seqs]
             if all(p.greedy for p in params):
-                fixed = None, False, False, list(seqs), False
+                fixed = None, False, False, list(seqs), False, None
             else:
                 vocab = logits.shape[1]
                 top_k = np.array([p.top_k if 0 < p.top_k < vocab else -1 for p in params], dtype=np.int32)
@@ -84,26 +84,36 @@ class Sampler:
                 packed = np.concatenate([seeds.view(np.int32), np.zeros(2 * n, dtype=np.int32),
                                          temperature.view(np.int32), top_p.view(np.int32), top_k])
                 any_both = bool(((top_k > 0) & (top_p < 1.0) & (temperature > 0)).any())
-                fixed = packed, bool((top_k > 0).any()), bool((top_p < 1.0).any()), list(seqs), any_both
+                fixed = packed, bool((top_k > 0).any()), bool((top_p < 1.0).any()), list(seqs), any_both, {}
             self._fixed.pop(key, None)
             while len(self._fixed) >= self._KEPT:
                 self._fixed.pop(next(iter(self._fixed)))
         else:
             self._fixed.pop(key)
         self._fixed[key] = fixed   # the newest entry last
-        packed, any_top_k, any_top_p, _, any_both = fixed
+        packed, any_top_k, any_top_p, _, any_both, sent = fixed
         if packed is None:
             return ops.argmax(logits)
-        slot = self._pinned(7 * n)
-        host = slot[0].numpy()
-        host[: 7 * n] = packed
-        host[2 * n : 4 * n].view(np.int64)[:] = [len(s.output_token_ids) + pending for s in seqs]
-        dev = torch.empty(7 * n, dtype=torch.int32, device=self.device)
-        dev.copy_(slot[0][: 7 * n], non_blocking=True)
-        slot[1] = torch.cuda.Event()
-        slot[1].record()
-        return ops.sample(
-            logits, dev[4 * n : 5 * n].view(torch.float32), dev[6 * n : 7 * n], dev[5 * n : 6 * n].view(torch.float32),
-            dev[0 : 2 * n].view(torch.int64), dev[2 * n : 4 * n].view(torch.int64),
-            any_top_k=any_top_k, any_top_p=any_top_p, any_both=any_both,
-        )
+        draws = [len(s.output_token_ids) + pending for s in seqs]
+        # Of a batch that comes again the options are on the device already, and the counts, which alone change, go with the
+        # launch: no copy, no buffer to wait for (a call of few rows 38 -> 21 us, the host's time). They are kept for the stream that they
+        # were sent on, where what reads them comes behind the copy (and a capture sends its own, into its own memory).
+        stream = None if n > ops.SAMPLE_COUNTED_ROWS or torch.cuda.is_current_stream_capturing() else ops._stream()
+        options = sent.get(stream) if stream is not None else None
+        if options is None:
+            slot = self._pinned(7 * n)
+            host = slot[0].numpy()
+            host[: 7 * n] = packed
+            host[2 * n : 4 * n].view(np.int64)[:] = draws
+            dev = torch.empty(7 * n, dtype=torch.int32, device=self.device)
+            dev.copy_(slot[0][: 7 * n], non_blocking=True)
+            slot[1] = torch.cuda.Event()
+            slot[1].record()
+            options = (dev[4 * n : 5 * n].view(torch.float32), dev[6 * n : 7 * n], dev[5 * n : 6 * n].view(torch.float32),
+                       dev[0 : 2 * n].view(torch.int64))
+            if stream is None:
+                draws = dev[2 * n : 4 * n].view(torch.int64)
+            else:
+                sent.clear()   # of one stream, the last one that the batch came on
+                sent[stream] = options
+        return ops.sample(logits, *options, draws, any_top_k=any_top_k, any_top_p=any_top_p, any_both=any_both)

@@ -990,3 +990,44 @@ def test_the_last_block_makes_the_rows_that_are_asked_for(tmp_path, dtype, wante
     bound = dict(rtol=1e-5, atol=1e-5) if dtype == "float32" else dict(rtol=2e-2, atol=2e-2)   # roundings of bfloat16 in another kernel
     torch.testing.assert_close(got, all_rows[wanted], **bound)
     torch.testing.assert_close(then, after, **bound)
+
+
+@pytest.mark.parametrize("n", [1, 5, 64])
+def test_draw_counts_that_come_with_the_launch(n):
+    """Counts as a list of ints and as a device tensor draw the same tokens; a sampler whose batch comes again draws what a new
+    one does, on the same stream and on another; more rows than go with a launch."""
+    from types import SimpleNamespace
+
+    from clockwork_amd import ops
+    from clockwork_amd.engine.sequence import SamplingParams
+    from clockwork_amd.sampling.sampler import Sampler
+
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    logits = torch.randn(n, 5003, device=DEV, generator=gen)
+    temperature = torch.full((n,), 0.9, device=DEV)
+    top_k = torch.arange(n, dtype=torch.int32, device=DEV) * 7 - 1
+    top_p = torch.full((n,), 0.95, device=DEV)
+    seeds = torch.arange(n, dtype=torch.int64, device=DEV) + 3
+    counts = [(i * 977 + 5) % 100000 for i in range(n)]
+    want = ops.sample(logits, temperature, top_k, top_p, seeds, torch.tensor(counts, device=DEV))
+    assert torch.equal(ops.sample(logits, temperature, top_k, top_p, seeds, counts), want)
+    for bad in (counts + [1], [-1] * n, [1 << 32] * n):
+        with pytest.raises(ops.KernelError):
+            ops.sample(logits, temperature, top_k, top_p, seeds, bad)
+    more = ops.SAMPLE_COUNTED_ROWS + 1
+    with pytest.raises(ops.KernelError):
+        ops.sample(logits[:1].expand(more, -1).contiguous(), torch.ones(more, device=DEV), torch.zeros(more, dtype=torch.int32, device=DEV),
+                   torch.ones(more, device=DEV), torch.zeros(more, dtype=torch.int64, device=DEV), [0] * more)
+
+    seqs = [SimpleNamespace(seq_id=str(i), sampling_params=SamplingParams(temperature=0.8, top_k=40, seed=i), output_token_ids=[]) for i in range(n)]
+    kept, other = Sampler(torch.device(DEV)), torch.cuda.Stream()
+    for turn in range(4):
+        fresh = Sampler(torch.device(DEV)).launch(logits, seqs, pending=turn % 2)
+        assert torch.equal(kept.launch(logits, seqs, pending=turn % 2), fresh)
+        other.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(other):
+            again = kept.launch(logits, seqs, pending=turn % 2)
+        other.synchronize()
+        assert torch.equal(again, fresh)
+        for s in seqs:
+            s.output_token_ids.append(turn)
