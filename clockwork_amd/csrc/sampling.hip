@@ -202,13 +202,14 @@ __device__ __forceinline__ uint32_t philox_first_word(uint64_t seed, uint64_t co
 // Weights are integers, exp(.) * 2^40 rounded down: their sums do not depend on the order of
 // addition, so every comparison above gives the same answer however the row is cut and however
 // the additions are scheduled (LDS atomics included), run after run.
-// Bound by the passes over the logits, which come from the memory-side cache after the first, by the division and the
-// exponential of every token (a third of HIST) and, in DRAW, by a chain of trips and barriers. 64 rows of 151,936
+// Bound by the passes over the logits, which come from the memory-side cache after the first, by the exponential, the quotient and
+// the sums of every token and, in DRAW and for few rows, by a chain of trips, barriers and sums over a wave. 64 rows of 151,936
 // logits, a quarter each greedy, temperature, top-k and top-p, us: 119 as twelve kernels (a radix step of 8 bits of the
-// key each, over the whole rows), 63 as five, the row's bin by a kernel of its own from every chunk's bins (MAX 8.6, HIST 20.4, PICK 6.0,
-// COLLECT 10.4, DRAW 14.2 in a trace), 50 as four with the chunks' bins added up by atomics (9.3, 16.0, 9.0, 12.2).
-// Tried: a token's first loads asked for before its row is known (no gain), the division by a reciprocal and two exact steps
-// (HIST 1.5 us less, finding out where that is exact as much more in MAX).
+// key each, over the whole rows), 63 as five, the row's bin by a kernel of its own from every chunk's bins, 50 as four with the
+// chunks' bins added up by atomics (in a trace MAX 9.3, HIST 16.0, COLLECT 9.0, DRAW 12.2), 46 without the copy of the counts, 39 with
+// quotients of five instructions, float64 sums and sums over a wave without shuffles (8.3, 14.2, 7.6, 10.3); 64 rows of
+// temperature 33 -> 26, one row of top-p 30 -> 25.
+// Tried: a token's first loads asked for before its row is known (no gain).
 #define SAMPLE_THREADS 256
 #define SAMPLE_WAVES (SAMPLE_THREADS / 64)
 #define SAMPLE_MAX_CHUNKS 64
@@ -267,6 +268,9 @@ static int sample_chunks(int n, int V) {
   int c = (V + 2047) / 2048;
   const int most = n <= 32 ? SAMPLE_MAX_CHUNKS : n >= 512 ? 4 : 2048 / n;
   if (c > most) c = most;
+  // (of at most 2^21 tokens: what a thread adds up of one stays below 2^53)
+  const int least = (int)(((int64_t)V + (1 << 21) - 1) >> 21);
+  if (c < least) c = least < SAMPLE_MAX_CHUNKS ? least : SAMPLE_MAX_CHUNKS;
   return c < 1 ? 1 : c;
 }
 
@@ -287,6 +291,20 @@ __device__ __forceinline__ u64_t weight_of(float v, float mx) {
   const float e = expf(v - mx);  // NaN for inf - inf: no weight
   return e == e ? (u64_t)(e * SAMPLE_WEIGHT_SCALE) : 0;
 }
+// A row's temperature and what divides by it. ``of(a)`` is a / T, rounded once: a product with the reciprocal, then twice the remainder
+// times the reciprocal, each remainder exact by a fused multiply-add; the first step leaves a quotient that is off by less than one
+// unit of its last place, and of such a one the second makes the correctly rounded quotient (Markstein). Five instructions for the
+// division's eleven, one of them at a quarter of the rate. Infinite quotients come out as NaN, which everything here takes for -inf (a row whose
+// largest logit is +inf has no weight at all, and its first maximum is taken).
+struct Quotient {
+  float t, y;
+  __device__ __forceinline__ explicit Quotient(float temp) : t(temp), y(1.0f / temp) {}
+  __device__ __forceinline__ float of(float a) const {
+    float q = a * y;
+    q = fmaf(fmaf(-t, q, a), y, q);
+    return fmaf(fmaf(-t, q, a), y, q);
+  }
+};
 // The three segments of a row's bins: x is the largest logit / T of one, y how many bins go into a unit below that (0
 // where the segment has no width: it is one bin then).
 struct SampleBins {
@@ -384,11 +402,40 @@ __device__ __forceinline__ void sample_walk(const float* x, int lo, int hi, int 
   }
 }
 
+// Sums over a wave, every lane ending with the total, and running sums (of a lane and those before it), by data-parallel operands:
+// a shuffle through the LDS unit takes ten times as long, and a sum has six of them one after the other.
+template <int CTRL, int ROWS = 0xf> __device__ __forceinline__ uint32_t sample_dpp(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, true);
+}
+template <int CTRL, int ROWS = 0xf> __device__ __forceinline__ u64_t sample_dpp(u64_t v) {
+  return ((u64_t)sample_dpp<CTRL, ROWS>((uint32_t)(v >> 32)) << 32) | sample_dpp<CTRL, ROWS>((uint32_t)v);
+}
+template <typename T> __device__ __forceinline__ T wave_running_sum(T v) {
+  v += sample_dpp<0x111>(v);       // the lane before, of the same row of 16
+  v += sample_dpp<0x112>(v);       // two before
+  v += sample_dpp<0x114>(v);
+  v += sample_dpp<0x118>(v);
+  v += sample_dpp<0x142, 0xa>(v);  // the last lane of rows 0 and 2 to rows 1 and 3
+  v += sample_dpp<0x143, 0xc>(v);  // lane 31 to rows 2 and 3
+  return v;
+}
+__device__ __forceinline__ uint32_t last_lane(uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, 63); }
+__device__ __forceinline__ u64_t last_lane(u64_t v) { return ((u64_t)last_lane((uint32_t)(v >> 32)) << 32) | last_lane((uint32_t)v); }
+__device__ __forceinline__ u64_t wave_sum(u64_t v) { return last_lane(wave_running_sum(v)); }
+__device__ __forceinline__ uint32_t wave_min(uint32_t v) {
+  v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x111, 0xf, 0xf, false));
+  v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x112, 0xf, 0xf, false));
+  v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x114, 0xf, 0xf, false));
+  v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x118, 0xf, 0xf, false));
+  v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x142, 0xa, 0xf, false));
+  v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x143, 0xc, 0xf, false));
+  return last_lane(v);
+}
+
 // Sum over the workgroup; every thread gets it.
 __device__ __forceinline__ u64_t block_sum(u64_t v) {
   __shared__ u64_t part[SAMPLE_WAVES];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  v = wave_sum(v);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
   __syncthreads();
   u64_t t = 0;
@@ -402,16 +449,19 @@ template <typename T>
 __device__ __forceinline__ T block_running_sum(T v) {
   __shared__ T part[SAMPLE_WAVES];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const T up = __shfl_up(v, off, 64);
-    if (lane >= off) v += up;
-  }
+  v = wave_running_sum(v);
   if (lane == 63) part[wave] = v;
   __syncthreads();
   for (int w = 0; w < wave; ++w) v += part[w];
   __syncthreads();
   return v;
+}
+
+// The largest value of a wave and the least index that goes with it.
+__device__ __forceinline__ void wave_argmax(float& v, int& i) {
+  const float best = cw_wave_max(v);
+  i = (int)wave_min(v == best ? (uint32_t)i : 0x7fffffffu);
+  v = best;
 }
 
 // The row's largest logit (NaN counts as -inf) and its first index, from the chunk maxima: the
@@ -426,12 +476,7 @@ __device__ __forceinline__ void row_max(const SampleArgs& a, int row, float& bv,
       v = a.pmax[row * a.chunks + threadIdx.x];
       i = a.pmax_i[row * a.chunks + threadIdx.x];
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const float ov = __shfl_xor(v, off, 64);
-      const int oi = __shfl_xor(i, off, 64);
-      argmax_merge(v, i, ov, oi);
-    }
+    wave_argmax(v, i);
     if (threadIdx.x == 0) { best_v = v; best_i = i; }
   }
   __syncthreads();
@@ -463,12 +508,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_max_kernel(SampleArgs a
     if (v != v) v = -INFINITY;
     argmax_merge(bv, bi, v, i);
   });
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const float ov = __shfl_xor(bv, off, 64);
-    const int oi = __shfl_xor(bi, off, 64);
-    argmax_merge(bv, bi, ov, oi);
-  }
+  wave_argmax(bv, bi);
   if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = bv; si[threadIdx.x >> 6] = bi; }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -489,13 +529,8 @@ __device__ __forceinline__ void sample_locate(const SampleArgs& a, int row, floa
   const uint32_t r = philox_first_word((uint64_t)a.seeds[row], a.draws ? (uint64_t)a.draws[row] : (uint64_t)counts.of_row[row]);
   if (threadIdx.x < 64) {  // the chunk the target falls into: a running sum over the chunks
     const u64_t v = (int)threadIdx.x < a.chunks ? chunk_w[threadIdx.x] : 0;
-    u64_t incl = v;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const u64_t up = __shfl_up(incl, off, 64);
-      if ((int)threadIdx.x >= off) incl += up;
-    }
-    const u64_t total = __shfl(incl, 63, 64);
+    const u64_t incl = wave_running_sum(v);
+    const u64_t total = last_lane(incl);
     // u = (r >> 8) / 2^24; the drawn token is the first whose running weight exceeds u * total
     u64_t target = (u64_t)((double)(r >> 8) * (1.0 / 16777216.0) * (double)total);
     if (total > 0 && target >= total) target = total - 1;  // (total >= 2^40: the largest logit weighs that much)
@@ -511,8 +546,9 @@ __device__ __forceinline__ void sample_locate(const SampleArgs& a, int row, floa
     return;
   }
   const float* x = a.logits + (int64_t)row * a.row_stride;
+  const Quotient over_t(temp);
   auto weight = [&](float raw) __attribute__((always_inline)) -> u64_t {
-    const float v = raw / temp;
+    const float v = over_t.of(raw);
     return v == v && order_key(v) >= floor_key ? weight_of(v, mx) : 0;
   };
   // in the chunk: thread t weighs a run of consecutive tokens; then a lane of the first wave takes a token of
@@ -539,15 +575,9 @@ __device__ __forceinline__ void sample_locate(const SampleArgs& a, int row, floa
     for (int i0 = run_lo; i0 < run_hi; i0 += 64) {
       const int i = i0 + (int)threadIdx.x;
       const u64_t q = i < run_hi ? weight(x[i]) : 0;
-      u64_t upto = q;
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const u64_t up = __shfl_up(upto, off, 64);
-        if ((int)threadIdx.x >= off) upto += up;
-      }
-      upto += before;
+      const u64_t upto = before + wave_running_sum(q);
       if (q > 0 && upto - q <= target && target < upto) found = i;
-      before = __shfl(upto, 63, 64);
+      before = last_lane(upto);
     }
   }
   __syncthreads();
@@ -593,18 +623,31 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_hist_kernel(SampleArgs 
       known.segments[2] = bins.s2;
     }
   }
-  u64_t sum = 0;
-  sample_walk(x, lo, hi, a.vec, [&](int, float raw) __attribute__((always_inline)) {
-    const float v = raw / temp;
-    const uint32_t bin = with_k || with_p ? bin_of(bins, v) : 0u;
-    if (with_k) atomicAdd(&bins_n[bin], 1u);
-    if (with_k && !with_p) return;  // (COLLECT weighs what top-k leaves)
-    const u64_t w = v == v ? weight_of(v, mx) : 0;
-    sum += w;
-    if (with_p && w) atomicAdd(&bins_w[bin], w);
-  });
-  sum = block_sum(sum);  // (and a barrier behind the bins)
-  if (threadIdx.x == 0) a.sums[(int64_t)row * a.chunks + chunk] = sum;
+  const Quotient over_t(temp);
+  if (!with_k && !with_p) {
+    // a thread's sum of whole numbers below 2^53 as float64, exact: one conversion a token instead of a 64-bit integer's six instructions
+    double sum = 0.0;
+    sample_walk(x, lo, hi, a.vec, [&](int, float raw) __attribute__((always_inline)) {
+      const float e = expf(over_t.of(raw) - mx);  // NaN: no weight
+      sum += e == e ? (double)truncf(e * SAMPLE_WEIGHT_SCALE) : 0.0;
+    });
+    const u64_t total = block_sum((u64_t)sum);
+    if (threadIdx.x == 0) a.sums[(int64_t)row * a.chunks + chunk] = total;
+    return;
+  }
+  // (COLLECT weighs what it leaves above the bin)
+  if (!with_p) {
+    sample_walk(x, lo, hi, a.vec, [&](int, float raw) __attribute__((always_inline)) { atomicAdd(&bins_n[bin_of(bins, over_t.of(raw))], 1u); });
+  } else {
+    sample_walk(x, lo, hi, a.vec, [&](int, float raw) __attribute__((always_inline)) {
+      const float v = over_t.of(raw);
+      const uint32_t bin = bin_of(bins, v);
+      if (with_k) atomicAdd(&bins_n[bin], 1u);
+      const u64_t w = v == v ? weight_of(v, mx) : 0;
+      if (w) atomicAdd(&bins_w[bin], w);
+    });
+  }
+  __syncthreads();
   // the row's bins: integers, so the order in which its chunks come does not matter
   for (int b = threadIdx.x; b < SAMPLE_BINS; b += SAMPLE_THREADS) {
     if (with_k && bins_n[b]) atomicAdd(a.hist_n + (int64_t)row * SAMPLE_BINS + b, bins_n[b]);
@@ -691,9 +734,10 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(SampleAr
   float end = segment == 0 ? s1.x : segment == 1 ? s2.x : -INFINITY;
   if (j < SAMPLE_SEGMENT_BINS - 1 && seg_y > 0.0f) end = fmaxf(end, seg_top - (float)(j + 1) / seg_y);
   const float surely_below = (end - 1e-5f * (fabsf(end) + fabsf(seg_top)) - 1e-30f) * temp;
+  const Quotient over_t(temp);
   auto look = [&](int i, float raw) __attribute__((always_inline)) {
     if (raw < surely_below) return;
-    const float v = raw / temp;
+    const float v = over_t.of(raw);
     const uint32_t b = bin_of(bins, v);
     if (b < bin) {
       sum += weight_of(v, mx);
@@ -706,11 +750,8 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(SampleAr
   };
   sample_walk(x, lo, hi, a.vec, look);
   if (__ballot(most >= least)) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      least = min(least, (uint32_t)__shfl_xor((int)least, off, 64));
-      most = max(most, (uint32_t)__shfl_xor((int)most, off, 64));
-    }
+    least = wave_min(least);
+    most = ~wave_min(~most);
     if ((threadIdx.x & 63) == 0) {
       atomicMin(&ends[0], least);
       atomicMax(&ends[1], most);
@@ -765,11 +806,8 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(SampleArgs 
     uint4 e = make_uint4(0xffffffffu, 0u, 0u, 0u);
     if ((int)threadIdx.x < a.chunks) e = a.found[(int64_t)row * a.chunks + threadIdx.x];
     chunk_n[threadIdx.x] = e.z;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      e.x = min(e.x, (uint32_t)__shfl_xor((int)e.x, off, 64));
-      e.y = max(e.y, (uint32_t)__shfl_xor((int)e.y, off, 64));
-    }
+    e.x = wave_min(e.x);
+    e.y = ~wave_min(~e.y);
     if (threadIdx.x == 0) ends[0] = e.x, ends[1] = e.y;
   }
   __syncthreads();
@@ -790,7 +828,8 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(SampleArgs 
   const int differing = least < most ? 32 - __clz(least ^ most) : 0;  // low bits that are not the same in all
   const uint32_t common = differing == 32 ? 0u : (most >> differing) << differing;
   // (a NaN's key is that of -inf: neither weighs anything)
-  auto scaled = [&](uint32_t key) __attribute__((always_inline)) -> float { return key_to_float(key) / temp; };
+  const Quotient over_t(temp);
+  auto scaled = [&](uint32_t key) __attribute__((always_inline)) -> float { return over_t.of(key_to_float(key)); };
   const u64_t above = block_sum((int)threadIdx.x < a.chunks ? chunk_w[threadIdx.x] : 0);
   uint32_t floor_key = 0u;
   // a bin whose largest token has no weight (masked tokens; at low temperatures most of a row): whichever of its
@@ -903,11 +942,10 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(SampleArgs 
       sample_walk<8, 64>(x, lo, hi, a.vec, [&](int, float raw) __attribute__((always_inline)) {
         const uint32_t key = order_key(raw);
         if (key < least || key > most) return;
-        const float v = raw / temp;
+        const float v = over_t.of(raw);
         if (order_key(v) >= floor_key) sum += weight_of(v, mx);
       });
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+      sum = wave_sum(sum);
       if ((threadIdx.x & 63) == 0) chunk_w[c] += sum;
     }
   }

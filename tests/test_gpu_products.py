@@ -1031,3 +1031,28 @@ def test_draw_counts_that_come_with_the_launch(n):
         assert torch.equal(again, fresh)
         for s in seqs:
             s.output_token_ids.append(turn)
+
+
+@pytest.mark.parametrize("temp", [1.3, 1.7, 1.9999999, 2.5, 3.0, 0.7, 0.3])
+def test_ties_that_dividing_by_the_temperature_makes(temp):
+    """Top-k of 1 keeps every token whose logit / T, rounded once to float32, is the largest's: of neighbouring floats some are
+    tied so and some are not, and which, the drawn tokens say."""
+    from clockwork_amd import ops
+
+    t = torch.tensor(temp, dtype=torch.float32)
+    near = torch.from_numpy((torch.tensor(7.3).view(torch.int32) + torch.arange(4000)).to(torch.int32).numpy()).view(torch.float32)
+    equal = (near[1:] / t) == (near[:-1] / t)
+    pairs = [i for kind in (True, False) for i in (equal == kind).nonzero().flatten()[:32].tolist()]
+    n, V, tries = len(pairs), 4099, 24
+    logits = torch.full((n, V), torch.finfo(torch.float32).min)
+    logits[:, ::7] = float("-inf")
+    logits[:, 11], logits[:, 4001] = near[pairs], near[[i + 1 for i in pairs]]
+    logits = logits.to(DEV)
+    seen = torch.zeros(n, V, dtype=torch.bool)
+    for i in range(tries):
+        got = ops.sample(logits, torch.full((n,), temp, device=DEV), torch.ones(n, dtype=torch.int32, device=DEV), torch.ones(n, device=DEV),
+                         torch.arange(n, dtype=torch.int64, device=DEV), [i] * n).cpu()
+        seen[torch.arange(n), got.long()] = True
+    assert bool(seen[:, 4001].all()) and int(seen.sum()) == int(seen[:, [11, 4001]].sum())
+    # a tied pair weighs the same: 24 draws miss one of the two once in 2^23
+    assert torch.equal(seen[:, 11], equal[pairs])
