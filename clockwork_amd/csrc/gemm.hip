@@ -31,6 +31,20 @@ __device__ __forceinline__ bf16x8_t cw_to_operand_layout(const bf16x8_t& v, int 
   return __builtin_bit_cast(bf16x8_t, cw_swap_to_operand(__builtin_bit_cast(cw_i32x4_t, v), lane));
 }
 
+// Two steps of K at once: lane l loads slot l % 8 of the 128 bytes that hold both, of row 2 (l / 8) into a and of the row after it
+// into b, so that a load asks for whole lines. Then lanes 4 to 7 of eight hold the second step: they change places with the
+// other row's first, and a and b are the two steps as a load of one each would have left them.
+__device__ __forceinline__ void cw_lines_to_steps(bf16x8_t& a, bf16x8_t& b) {
+  cw_i32x4_t p = __builtin_bit_cast(cw_i32x4_t, a), q = __builtin_bit_cast(cw_i32x4_t, b);
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const int first = p[d], second = q[d];
+    p[d] = __builtin_amdgcn_update_dpp(first, second, 0x114, 0xf, 0xa, false);   // row_shr:4 into lanes 4 .. 7 and 12 .. 15 of 16
+    q[d] = __builtin_amdgcn_update_dpp(second, first, 0x104, 0xf, 0x5, false);   // row_shl:4 into the others
+  }
+  a = __builtin_bit_cast(bf16x8_t, p), b = __builtin_bit_cast(bf16x8_t, q);
+}
+
 // =====================================================================================
 // float32. What a product of one output element is, whichever kernel makes it: K is cut into parts
 // (gemm_f32_plan), a part into blocks of 16 k-values. Lane (row, s) of an operand holds k-values
@@ -1045,7 +1059,14 @@ constexpr int cw_stream_chunk(int spw) { return spw <= 8 ? spw : (spw <= 12 ? sp
 
 // GROUP (MODE 0): row tiles of several products of the same x, ``in`` a ProductGroup (W, C, ldc and N are not used).
 // BEGUN (MODE 2, MT = 1): x comes with its norm begun, ``in`` a RowFactors.
-template <int MODE, int WAVES, int SPW, int MT, bool NORM = false, bool GROUP = false, bool BEGUN = false>
+// LINES: whole lines a load, which the caches need not keep: a stream of 110 MB comes in at 5.8 TB/s so and at 5.2 otherwise (half lines a
+// load that the caches need not keep: each comes twice), and what the step reads beside it has the caches for itself. us, without / with: [gate;
+// up] of 37888 x 3584 with 1, 8, 16 rows 48.8 / 43.0, 49.3 / 43.3, 51.0 / 44.5; 152064 x 3584 184 / 163, 190 / 170, 202 / 178; 151936 x 1536 with 1, 16, 64
+// rows 79 / 73, 89 / 80, 107 / 97; 17920 x 1536 12.0 / 11.9 to 14.3 / 13.8 (32 rows). In a wave's one pair (K up to 1024) of more than 16 rows
+// nothing is left of that (151936 x 896 with 32, 64 rows 60.2 / 60.7, 69.9 / 70.3), nor in partial sums of fewer than 64 MB (MODE 3; 1536 x 8960 6.7
+// to 10.8 / 7.6 to 10.1, the first row's wait for memory is the longer one; 3584 x 18944 with 1, 8, 16, 32 rows 25.0 / 24.3, 26.9 / 25.8, 28.3 / 28.3, 29.5 / 29.1;
+// 5120 x 13824 25.8 / 24.0, 27.5 / 24.6, 28.4 / 25.7, 29.3 / 27.3). A step of one request, us: 0.5B shape 714 / 703, 7B shape 3212 / 3085.
+template <int MODE, int WAVES, int SPW, int MT, bool NORM = false, bool GROUP = false, bool BEGUN = false, bool LINES = MODE != 3 && (MT == 1 || SPW > 2)>
 __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16_t* __restrict__ X, int64_t ldx,
                                                                const bf16_t* __restrict__ W,
                                                                void* __restrict__ C, int64_t ldc,
@@ -1057,7 +1078,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
   constexpr int CH = cw_stream_chunk(SPW), NC = SPW / CH;
   static_assert(SPW % CH == 0, "the steps of a wave are whole chunks");
   __shared__ __align__(16) float red[NBUF][WAVES][MT * 256];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = LINES ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
   const int r = lane & 15, s = lane >> 4;
   const int I = N / 2;  // MODE 2 only
   __shared__ float factors[16];
@@ -1069,39 +1090,80 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
   auto to_operand = [&](const bf16x8_t& v) __attribute__((always_inline)) -> bf16x8_t {
     return cw_to_operand_layout(v, lane);
   };
-  // The loading lane's 8 k-values of each step. A step outside of K meets zeros in x; it reads zeros, so that an infinite weight stays
-  // one, or in the products with a long K, whose loads the choice of address would slow by 4 %, k = 0.
+  // LINES: weights come in two steps of K a pair of loads (cw_lines_to_steps), which begin at even steps; of an odd number of steps the
+  // wave's first or last is left over and loaded alone, as x is.
+  constexpr int PAIRED = LINES ? CH & ~1 : 0;  // fragments of a set that come in pairs
+  const int step0 = (blockIdx.y * WAVES + wave) * SPW;
+  auto step_of = [&](int u) __attribute__((always_inline)) -> int {  // that set of fragments u of the wave holds
+    const int begin = step0 + u / CH * CH, i = u % CH;
+    if (!LINES || (CH & 1) == 0) return begin + i;
+    const int late = begin & 1;
+    return i < CH - 1 ? begin + late + i : begin + (late ? 0 : CH - 1);
+  };
+  // Where the loading lane finds its 8 k-values of a step or, with 8 slots, of a pair. What lies outside of K meets zeros in x; it reads zeros, so
+  // that an infinite weight stays one, or in the products with a long K, whose loads the choice of address would slow by 4 %, k = 0;
+  // there a pair outside of K as a whole reads the row's last one, which is on its way, and becomes zeros (k = 0, not kept by the caches, came from
+  // memory each time: 18944 columns of 3584 rows, where a wave in thirteen lies outside, 26.8 -> 24.3 us with 1 row, 27.7 -> 25.8 with 8).
   constexpr bool ZEROS = MODE != 3 && NC == 1;
-  int koff[SPW];
+  int koff[SPW];  // one load at a time
 #pragma unroll
   for (int u = 0; u < SPW; ++u) {
-    const int k = ((blockIdx.y * WAVES + wave) * SPW + u) * 32 + ls * 8;
+    const int k = (step0 + u) * 32 + ls * 8;
     koff[u] = k + 8 <= K ? k : ZEROS ? -1 : 0;
   }
-  auto weights = [&](const bf16_t* row, int k) __attribute__((always_inline)) -> bf16x8_t {
-    return *reinterpret_cast<const bf16x8_t*>(!ZEROS || k >= 0 ? row + k : reinterpret_cast<const bf16_t*>(cw_zeros));
+  auto at = [&](const bf16_t* row, int u, int slot, bool pair) __attribute__((always_inline)) -> const bf16x8_t* {
+    const int begin = step_of(u) * 32, k = (!ZEROS && pair && begin >= K ? max(K - 64, 0) : begin) + slot * 8;
+    return reinterpret_cast<const bf16x8_t*>(k + 8 <= K ? row + k : ZEROS ? reinterpret_cast<const bf16_t*>(cw_zeros) : row);
   };
-  auto wrow = [&](int tile) __attribute__((always_inline)) -> const bf16_t* {
+  auto wrow = [&](int tile, int tile_row) __attribute__((always_inline)) -> const bf16_t* {
     int64_t n;
     if constexpr (GROUP) {
       const int g = group_of(in, tile);
-      return in.w[g] + (int64_t)min((tile - in.first[g]) * 16 + lr, in.n[g] - 1) * K;
+      return in.w[g] + (int64_t)min((tile - in.first[g]) * 16 + tile_row, in.n[g] - 1) * K;
     }
     if (MODE == 2) {  // gate and up rows alternate, so that a pair lies side by side in the tile
-      const int64_t i = min((int64_t)tile * 8 + (lr >> 1), (int64_t)I - 1);
-      n = (lr & 1) ? I + i : i;
+      const int64_t i = min((int64_t)tile * 8 + (tile_row >> 1), (int64_t)I - 1);
+      n = (tile_row & 1) ? I + i : i;
     } else {
-      n = min((int64_t)tile * 16 + lr, (int64_t)N - 1);
+      n = min((int64_t)tile * 16 + tile_row, (int64_t)N - 1);
     }
     return W + n * K;
+  };
+  struct Rows {
+    const bf16_t *even, *odd, *alone;
+  };
+  auto rows_of = [&](int tile) __attribute__((always_inline)) -> Rows {
+    const int first = (lane >> 3) * 2;
+    return {PAIRED ? wrow(tile, first) : nullptr, PAIRED ? wrow(tile, first + 1) : nullptr, PAIRED < CH ? wrow(tile, lr) : nullptr};
+  };
+  // (whole lines that nobody reads again: they leave the caches to the others)
+  auto weights = [&](bf16x8_t (&dst)[CH], const Rows& rows, int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < PAIRED; u += 2) {
+      dst[u] = __builtin_nontemporal_load(at(rows.even, c * CH + u, lane & 7, true));
+      dst[u + 1] = __builtin_nontemporal_load(at(rows.odd, c * CH + u, lane & 7, true));
+    }
+#pragma unroll
+    for (int u = PAIRED; u < CH; ++u) dst[u] = LINES ? *at(rows.alone, c * CH + u, ls, false) : *reinterpret_cast<const bf16x8_t*>(!ZEROS || koff[c * CH + u] >= 0 ? rows.alone + koff[c * CH + u] : reinterpret_cast<const bf16_t*>(cw_zeros));
+  };
+  auto products = [&](bf16x8_t (&w)[CH], const auto& x, int c, f32x4_t (&acc)[MT]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      if (u % 2 == 0 && u < PAIRED) {
+        if (!ZEROS && step_of(c * CH + u) * 32 >= K) w[u] = w[u + 1] = bf16x8_t{};
+        cw_lines_to_steps(w[u], w[u + 1]);
+      }
+      const bf16x8_t wu = to_operand(w[u]);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wu, x[c * CH + u][mt], acc[mt], 0, 0, 0);
+    }
   };
   // the first tile's weights are requested before anything else: x, and with NORM the norm's
   // statistics, are fetched in their shadow
   int tile = blockIdx.x;
   bf16x8_t cur[CH], nxt[CH];
-  const bf16_t* w_tile = wrow(tile);
-#pragma unroll
-  for (int u = 0; u < CH; ++u) cur[u] = weights(w_tile, koff[u]);
+  Rows w_tile = rows_of(tile);
+  weights(cur, w_tile, 0);
 
   bf16x8_t xf[SPW][MT];
   if constexpr (NORM) {
@@ -1111,7 +1173,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
     float ss = 0.0f;
 #pragma unroll
     for (int u = 0; u < SPW; ++u) {
-      const int k = (wave * SPW + u) * 32 + s * 8;
+      const int k = step_of(u) * 32 + s * 8;
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[u][e] = wv[u][e] = 0.0f;
       if (k + 8 <= K && r < M) {
@@ -1155,8 +1217,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
       const bf16_t* xrow = X + (int64_t)min(m, M - 1) * ldx;
 #pragma unroll
       for (int u = 0; u < SPW; ++u) {
-        const bool ok = ((blockIdx.y * WAVES + wave) * SPW + u) * 32 + ls * 8 + 8 <= K && m < M;
-        bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(xrow + (ZEROS ? max(koff[u], 0) : koff[u]));
+        const int k = LINES ? step_of(u) * 32 + ls * 8 : koff[u];
+        const bool ok = step_of(u) * 32 + ls * 8 + 8 <= K && m < M;
+        bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(xrow + (LINES ? (k + 8 <= K ? k : 0) : ZEROS ? max(k, 0) : k));
         if (!ok) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] = (__bf16)0.0f;
@@ -1223,58 +1286,42 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_bf16_kernel(const bf16
     // after this one are issued before this tile's products and are waited for only when their
     // own products begin, so they are in flight during the whole of this tile's products,
     // reduction and stores. Past the last tile a valid address is read and dropped.
-    auto load_set = [&](bf16x8_t (&dst)[CH], int t) __attribute__((always_inline)) {
-      const bf16_t* w = wrow(min(t, n_tiles - 1));
-#pragma unroll
-      for (int u = 0; u < CH; ++u) dst[u] = weights(w, koff[u]);
-    };
-    auto products = [&](const bf16x8_t (&w)[CH], f32x4_t (&acc)[MT]) __attribute__((always_inline)) {
+    auto load_set = [&](bf16x8_t (&dst)[CH], int t) __attribute__((always_inline)) { weights(dst, rows_of(min(t, n_tiles - 1)), 0); };
+    auto zero = [&](f32x4_t (&acc)[MT]) __attribute__((always_inline)) {
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) acc[mt] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int u = 0; u < CH; ++u) {
-        const bf16x8_t wu = to_operand(w[u]);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-          acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wu, xf[u][mt], acc[mt], 0, 0, 0);
-      }
     };
     const int stride = (int)gridDim.x;
     while (tile < n_tiles) {
       f32x4_t acc[MT];
       load_set(nxt, tile + stride);
       __builtin_amdgcn_sched_barrier(0);  // the loads stay in front of the products
-      products(cur, acc);
+      zero(acc);
+      products(cur, xf, 0, acc);
       finish_tile(acc, tile, buf);
       buf = (buf + 1) % NBUF;
       tile += stride;
       if (tile >= n_tiles) break;
       load_set(cur, tile + stride);
       __builtin_amdgcn_sched_barrier(0);
-      products(nxt, acc);
+      zero(acc);
+      products(nxt, xf, 0, acc);
       finish_tile(acc, tile, buf);
       buf = (buf + 1) % NBUF;
       tile += stride;
     }
   } else {
     for (; tile < n_tiles; tile += gridDim.x) {
-      const bf16_t* w_next = wrow(min(tile + (int)gridDim.x, n_tiles - 1));
+      const Rows w_next = rows_of(min(tile + (int)gridDim.x, n_tiles - 1));
       f32x4_t acc[MT];
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) acc[mt] = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
         // the chunk after this one: of this tile, or the first of the workgroup's next tile
-#pragma unroll
-        for (int u = 0; u < CH; ++u)
-          nxt[u] = c + 1 < NC ? weights(w_tile, koff[(c + 1) * CH + u]) : weights(w_next, koff[u]);
-#pragma unroll
-        for (int u = 0; u < CH; ++u) {
-          const bf16x8_t wu = to_operand(cur[u]);
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt)
-            acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wu, xf[c * CH + u][mt], acc[mt], 0, 0, 0);
-        }
+        if (c + 1 < NC) weights(nxt, w_tile, c + 1);
+        else weights(nxt, w_next, 0);
+        products(cur, xf, c, acc);
 #pragma unroll
         for (int u = 0; u < CH; ++u) cur[u] = nxt[u];
       }
@@ -1310,6 +1357,13 @@ template <int MODE, int WAVES, int SPW, int MT>
 static int launch_stream_one(dim3 grid, const bf16_t* X, int64_t ldx, const bf16_t* W, void* C, int64_t ldc,
                              int M, int N, int K, int n_tiles, float act, hipStream_t stream) {
   if constexpr (cw_stream_fits(WAVES, SPW, MT)) {
+    if constexpr (MODE == 3 && SPW >= 4) {
+      if ((int64_t)N * K >= (1 << 25)) {
+        hipLaunchKernelGGL((gemm_stream_bf16_kernel<MODE, WAVES, SPW, MT, false, false, false, true>), grid, dim3(WAVES * 64), 0, stream, X, ldx,
+                           W, C, ldc, M, N, K, n_tiles, act, StreamNormIn{});
+        return cw_launch_status();
+      }
+    }
     hipLaunchKernelGGL((gemm_stream_bf16_kernel<MODE, WAVES, SPW, MT>), grid, dim3(WAVES * 64), 0, stream, X, ldx,
                        W, C, ldc, M, N, K, n_tiles, act, StreamNormIn{});
     return cw_launch_status();

@@ -901,6 +901,37 @@ def test_streamed_products_of_fewer_steps_than_two_a_wave(M, K, N):
     torch.testing.assert_close(gated.double()[:, keep], want[:, keep], rtol=2.0 ** -8, atol=1e-5)
 
 
+# K of 16 waves: an odd number of steps a wave and waves outside of K; 7 steps; 8, the last wave's cut; chunks of 5 and of 6 steps with
+# a K that ends inside a pair. Partial sums of 64 MB and more: chunks of 4 and 5 steps, waves outside of K, a K that ends inside a pair
+@pytest.mark.parametrize("M", [1, 16, 17, 40])
+@pytest.mark.parametrize("N,K,partial", [(8208, 1408, False), (8192, 3592, False), (8192, 4056, False), (8192, 5016, False), (8192, 5912, False),
+                                         (5120, 6560, True), (3584, 9384, True), (1536, 22016, True)])
+def test_streams_of_whole_lines(M, N, K, partial):
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(M + K + N)
+    x = torch.randn(M, K, device=DEV, generator=gen).to(torch.bfloat16)
+    w = (torch.randn(N, K, device=DEV, generator=gen) / K ** 0.5).to(torch.bfloat16)
+    y = x.double() @ w.double().t()
+    if partial:
+        got = ops.linear(x, w, partial_ok=True)
+        got = got.parts.sum(0) if isinstance(got, ops.PartialSums) else got
+    else:
+        got = ops.linear(x, w, out_dtype=torch.float32)
+    # float32 sums of K products of about 1 / sqrt(K): 2^-24 sqrt(K) of the result's spread at most, ten times that; a library product, where the
+    # kernels decline more than 16 rows, is rounded to bfloat16 once
+    ours = got.dtype == torch.float32 if partial else M <= 16 or ops._load("gemm").cw_gemm_bf16_skinny_fast(1, M, N, K)
+    bound = 10 * 2.0 ** -24 * K ** 0.5 if ours else 2.0 ** -8 * float(y.abs().max())
+    assert float((got.double() - y).abs().max()) < bound
+    # an infinite weight stays one, the outputs beside it finite (K in one set of fragments a wave; or in the last columns, which the waves outside of K read)
+    if partial or K <= 4096:
+        w[3, K - 1] = float("inf")
+        x[:, K - 1] = 1.0
+        again = ops.linear(x, w, partial_ok=True) if partial else ops.linear(x, w, out_dtype=torch.float32)
+        again = again.parts.sum(0) if isinstance(again, ops.PartialSums) else again
+        assert bool((again[:, 3] == float("inf")).all()) and bool(torch.isfinite(again[:, [2, 4]]).all())
+
+
 # N, K: workgroups of 8 outputs by 8 waves (K up to 2048, the last one short), of 4, of up to 8 and up to 16 outputs by 16 waves, pieces
 # of a row no multiple of four, a K that ends inside an operand's pieces
 @pytest.mark.parametrize("N,K,most", [(900, 264, 16), (1536, 1536, 16), (896, 4864, 15), (1000, 2504, 16), (1537, 8960, 8), (2052, 600, 16), (3584, 3584, 16)])
