@@ -388,15 +388,23 @@ __device__ __forceinline__ float w_gated(float g, float up, float act) {
     asm volatile("" ::: "memory"); \
   } while (0)
 
-template <int MODE, int MB, int NB, int SLOTS, bool ANY_ROWS = true, bool GROUPED = false, int GATE = W_GATE_SILU>
-__global__ __launch_bounds__(256) void gemm_wide_bf16_kernel(WideArgs a) {
+// APART: four waves of their own load a tile, where its products leave them registers (256 a thread beside the four that multiply; 192 x
+// 192 spilled 18). A wave that loads and multiplies stands still at each load that the load path does not take in yet, and its
+// products with it: loads alone took 20.8 of 21.9 us of 160 rows of 17920 x 1536 (x alone 8.1, W alone 13.8: they add up, one queue of about 64 KB a
+// compute unit in the order of issue; rings of their own, W eight stages deep, changed nothing). us, then / now: 160 and 352 rows of
+// that 22.0 / 21.3, 26.1 / 25.3, 1000 of it by 192 x 160 62.5 / 54.9; 2048 rows of 1536 x 1536 13.9 / 13.1, of 2048 x 1536 17.0 / 16.0; 160 and 352 rows of 1536 x 8960 in
+// planes 14.5 / 14.1, 19.7 / 19.2; over 26 shapes and the tiles in question 5 % in the mean.
+static constexpr bool w_loads_apart(int mb, int nb) { return mb * nb <= 32; }
+
+template <int MODE, int MB, int NB, int SLOTS, bool ANY_ROWS = true, bool GROUPED = false, int GATE = W_GATE_SILU, bool APART = w_loads_apart(MB, NB)>
+__global__ __launch_bounds__(APART ? 512 : 256) void gemm_wide_bf16_kernel(WideArgs a) {
   extern __shared__ __align__(1024) unsigned char w_smem[];
   constexpr bool GATED = MODE == 2;
   constexpr int BM = 32 * MB, BN = 32 * NB, PER = GATED ? BN / 2 : BN;  // PER: columns of the result
   constexpr int LOADS = MB + NB;                                            // of a wave and stage: MB of x, NB of W
   constexpr int STAGE = 4 * LOADS * W_BLOCK;
-  static_assert(SLOTS >= 2 && SLOTS * STAGE <= 160 * 1024 && SLOTS * LOADS <= 63, "the ring is the LDS of a compute unit");
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  static_assert(SLOTS >= 2 && SLOTS * STAGE <= 160 * 1024 && SLOTS * LOADS <= 63 && SLOTS <= 6, "the ring is the LDS of a compute unit");
+  const int tid = threadIdx.x, lane = tid & 63, wave8 = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave8 & 3;
   const int wm = wave >> 1, wn = wave & 1;
   const int c = lane & 15, s = lane >> 4;
   // GROUPED: the number of row tiles is known on the device alone; x holds whole tiles
@@ -450,17 +458,20 @@ __global__ __launch_bounds__(256) void gemm_wide_bf16_kernel(WideArgs a) {
     wr = __builtin_amdgcn_make_buffer_rsrc((void*)(w_base + w_row0 * K + k0), 0,
                                            (int)(uint32_t)(((N - w_row0 - 1) * (int64_t)K + k_run) * 2), 0x00020000);
   };
-  auto fetch_one = [&](int stage, int slot, int i) __attribute__((always_inline)) {
+  auto fetch_as = [&](bool once, int stage, int slot, int i) __attribute__((always_inline)) {
     uint32_t apart = i < MB ? i * x_step : wide_col<MODE, NB>(i - MB, 0) * w_row;
     asm volatile("" : "+s"(apart));  // added here and now: the sums of all loads would take as many registers
     if (i < MB) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t*)(w_smem + slot + (i * 4 + wave) * W_BLOCK), 16, x_at + apart, stage * 128, 0, 0);
     } else {
       const int ni = i - MB;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void_t*)(w_smem + slot + (4 * MB + (half * NB + ni) * 2 + parity) * W_BLOCK), 16,
-                                               (ni < REGULAR ? w_at : w_at_rest) + apart, stage * 128, 0, 0);
+      lds_void_t* to = (lds_void_t*)(w_smem + slot + (4 * MB + (half * NB + ni) * 2 + parity) * W_BLOCK);
+      const uint32_t from = (ni < REGULAR ? w_at : w_at_rest) + apart;
+      if (once) __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, to, 16, from, stage * 128, 0, 2);  // 2: nontemporal
+      else __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, to, 16, from, stage * 128, 0, 0);
     }
   };
+  auto fetch_one = [&](int stage, int slot, int i) __attribute__((always_inline)) { fetch_as(false, stage, slot, i); };
   // (of fewer stages than slots the last comes in again: the number of loads in flight is what the waits count on)
   auto fetch_first_stages = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -533,47 +544,112 @@ __global__ __launch_bounds__(256) void gemm_wide_bf16_kernel(WideArgs a) {
 
   int id = run_begin + local;
   if (id >= run_end) return;
-  aim(id);
-  fetch_first_stages();
+  if constexpr (APART) {
+    if (wave8 >= 4) {
+      // Barrier n of the workgroup: stage n is in LDS, and the waves that multiply have read stage n - 1, whose slot
+      // the next loads take. The stages of all its tiles are one row, so a tile's first come in while the last one's results go out.
+      int ahead = 0, to = 0;
+      // One or two row tiles, side by side on one XCD, read a matrix once: its lines need not stay in the caches, which are then x's and the
+      // next kernels' (160 and 352 rows of 17920 x 1536 21.3 -> 20.4 us, 25.3 -> 24.6; with 7 row tiles 32 -> 39). From 32 MB on: smaller ones gain nothing and
+      // partly wait longer (a step of 137 tokens of the 1.5B shape 2074 us with none so, 2082 with all, 2067 so; 100 tokens of the 7B shape 4611, 4400, 4283).
+      const bool once = tiles_m <= 2 && (int64_t)N * K >= (1 << 24);
+      for (; id < run_end; id += per_xcd) {
+        aim(id);
+        for (int t = 0; t < stages; ++t) {
+          if (ahead == SLOTS - 1) {
+            W_WAIT_LOADS((SLOTS - 2) * LOADS);
+            W_BARRIER();
+          } else {
+            ++ahead;
+          }
+          if (once) {
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) fetch_as(true, t, to, i);
+          } else {
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) fetch_one(t, to, i);
+          }
+          to = next_slot(to);
+        }
+      }
+      // the last ones, each as it comes in
+      auto last = [&](auto behind_c) __attribute__((always_inline)) {
+        constexpr int behind = decltype(behind_c)::value;
+        if (behind < SLOTS - 1 && ahead > behind) {
+          W_WAIT_LOADS((behind < SLOTS - 1 ? behind : 0) * LOADS);
+          W_BARRIER();
+        }
+      };
+      last(std::integral_constant<int, 4>{});
+      last(std::integral_constant<int, 3>{});
+      last(std::integral_constant<int, 2>{});
+      last(std::integral_constant<int, 1>{});
+      last(std::integral_constant<int, 0>{});
+      return;
+    }
+  } else {
+    aim(id);
+    fetch_first_stages();
+  }
+  int slot = 0;
   for (bool first = true; id < run_end; id += per_xcd, first = false) {
     int tm, tn;
     tile_of(id, &tm, &tn);
-    // the first stage is in LDS (a tile's stores come after its successor's loads, and count as well)
-    if (first) W_WAIT_LOADS((SLOTS - 1) * LOADS);
-    else W_WAIT_LOADS(0);
-    W_BARRIER();
+    if constexpr (APART) {
+      aim(id);  // (for its number of stages)
+      W_BARRIER();
 #pragma unroll
-    for (int i = 0; i < READS; ++i) read_one(0, 0, 0, i);
-    int slot = 0, t = 0;
-    phase(Yes{}, I0{}, Yes{}, slot, 1, I0{}, I0{}, 0, 0);
-    // every wave has read stage t and its loads of stage t + 1 have landed
-    W_WAIT_LOADS((SLOTS - 2) * LOADS);
-    W_WAIT_LDS();
-    W_BARRIER();
-    for (; t + SLOTS < stages; ++t) {
-      const int next = next_slot(slot);
-      phase(No{}, I1{}, Yes{}, next, 0, I0{}, Split{}, t + SLOTS, slot);
-      phase(No{}, I0{}, Yes{}, next, 1, Split{}, Last{}, t + SLOTS, slot);
+      for (int i = 0; i < READS; ++i) read_one(slot, 0, 0, i);
+      phase(Yes{}, I0{}, Yes{}, slot, 1, I0{}, I0{}, 0, 0);
+      for (int t = 1; t < stages; ++t) {
+        W_WAIT_LDS();
+        W_BARRIER();
+        slot = next_slot(slot);
+        phase(No{}, I1{}, Yes{}, slot, 0, I0{}, I0{}, 0, 0);
+        phase(No{}, I0{}, Yes{}, slot, 1, I0{}, I0{}, 0, 0);
+      }
+      phase(No{}, I1{}, No{}, 0, 0, I0{}, I0{}, 0, 0);
+      W_WAIT_LDS();
+      slot = next_slot(slot);
+    } else {
+      // the first stage is in LDS (a tile's stores come after its successor's loads, and count as well)
+      if (first) W_WAIT_LOADS((SLOTS - 1) * LOADS);
+      else W_WAIT_LOADS(0);
+      W_BARRIER();
+#pragma unroll
+      for (int i = 0; i < READS; ++i) read_one(0, 0, 0, i);
+      slot = 0;
+      int t = 0;
+      phase(Yes{}, I0{}, Yes{}, slot, 1, I0{}, I0{}, 0, 0);
+      // every wave has read stage t and its loads of stage t + 1 have landed
       W_WAIT_LOADS((SLOTS - 2) * LOADS);
       W_WAIT_LDS();
       W_BARRIER();
-      slot = next;
-    }
-    W_WAIT_LOADS(0);
-    W_BARRIER();  // the last stages are in
-    for (; t + 1 < stages; ++t) {
-      const int next = next_slot(slot);
-      phase(No{}, I1{}, Yes{}, next, 0, I0{}, I0{}, 0, 0);
-      phase(No{}, I0{}, Yes{}, next, 1, I0{}, I0{}, 0, 0);
-      slot = next;
-    }
-    phase(No{}, I1{}, No{}, 0, 0, I0{}, I0{}, 0, 0);
-    W_WAIT_LDS();
-    W_BARRIER();
-    // every slot is free: the first stages of the next tile come in while this one's results go out
-    if (id + per_xcd < run_end) {
-      aim(id + per_xcd);
-      fetch_first_stages();
+      for (; t + SLOTS < stages; ++t) {
+        const int next = next_slot(slot);
+        phase(No{}, I1{}, Yes{}, next, 0, I0{}, Split{}, t + SLOTS, slot);
+        phase(No{}, I0{}, Yes{}, next, 1, Split{}, Last{}, t + SLOTS, slot);
+        W_WAIT_LOADS((SLOTS - 2) * LOADS);
+        W_WAIT_LDS();
+        W_BARRIER();
+        slot = next;
+      }
+      W_WAIT_LOADS(0);
+      W_BARRIER();  // the last stages are in
+      for (; t + 1 < stages; ++t) {
+        const int next = next_slot(slot);
+        phase(No{}, I1{}, Yes{}, next, 0, I0{}, I0{}, 0, 0);
+        phase(No{}, I0{}, Yes{}, next, 1, I0{}, I0{}, 0, 0);
+        slot = next;
+      }
+      phase(No{}, I1{}, No{}, 0, 0, I0{}, I0{}, 0, 0);
+      W_WAIT_LDS();
+      W_BARRIER();
+      // every slot is free: the first stages of the next tile come in while this one's results go out
+      if (id + per_xcd < run_end) {
+        aim(id + per_xcd);
+        fetch_first_stages();
+      }
     }
 
     const int out_cols = GATED ? I : N;
@@ -765,9 +841,6 @@ CW_EXPORT int cw_gemm_bf16_wide_partial_ok(int M, int N, int K, int64_t ldx, int
 template <int MODE, int MB, int NB, int SLOTS, bool ANY_ROWS = true, bool GROUPED = false, int GATE = W_GATE_SILU>
 static int w_launch(WideArgs a, int row_tiles, int workgroups, hipStream_t stream) {
   constexpr int SMEM = SLOTS * 4 * (MB + NB) * W_BLOCK;
-  static std::atomic<bool> allowed{false};
-  const int status = cw_allow_lds(allowed, (const void*)gemm_wide_bf16_kernel<MODE, MB, NB, SLOTS, ANY_ROWS, GROUPED, GATE>, SMEM);
-  if (status != CW_OK) return status;
   constexpr bool gated = MODE == 2;
   const int out_cols = gated ? a.N / 2 : a.N, per_tile = gated ? 16 * NB : 32 * NB;
   a.tiles_n = (out_cols + per_tile - 1) / per_tile;
@@ -777,8 +850,21 @@ static int w_launch(WideArgs a, int row_tiles, int workgroups, hipStream_t strea
   // a multiple of 8 workgroups, so that every XCD gets the same number of them
   int grid = total < workgroups ? (int)total : workgroups;
   grid = (grid + 7) & ~7;
-  hipLaunchKernelGGL((gemm_wide_bf16_kernel<MODE, MB, NB, SLOTS, ANY_ROWS, GROUPED, GATE>), dim3(grid), dim3(256), SMEM, stream, a);
-  return cw_launch_status();
+  auto launch = [&](auto apart_c) -> int {
+    constexpr bool APART = decltype(apart_c)::value;
+    const auto kernel = gemm_wide_bf16_kernel<MODE, MB, NB, SLOTS, ANY_ROWS, GROUPED, GATE, APART>;
+    static std::atomic<bool> allowed{false};
+    const int status = cw_allow_lds(allowed, (const void*)kernel, SMEM);
+    if (status != CW_OK) return status;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(APART ? 512 : 256), SMEM, stream, a);
+    return cw_launch_status();
+  };
+  constexpr bool APART = w_loads_apart(MB, NB);
+  // Planes of many row tiles, which ask L2 for more than it gives in any case: alone they gain too (1000 rows of 1536 x 8960 32.3 / 31.0), behind a gate/up product and
+  // on a card whose clock is low they lose (1000 tokens behind 7000, 1.5B shape: 5800 / 5885 us on such a one, 5614 / 5593 on another).
+  if constexpr (MODE == 3 && APART)
+    if (a.tiles_m > 4) return launch(std::false_type{});
+  return launch(std::integral_constant<bool, APART>{});
 }
 
 // What a tile costs: ``fixed`` us of a work item and stage[q - 1] us a stage of 64 elements of K while q workgroups share a
@@ -788,6 +874,8 @@ static int w_launch(WideArgs a, int row_tiles, int workgroups, hipStream_t strea
 // a tile that the rule names takes 1 to 1.6 % more than the fastest, the library among them, 24 % at worst (272 rows of 6144 x 1536 with
 // a gate 18.4 by 160 x 96, 14.9 by 128 x 128; 704 rows of 1024 x 4096 and a norm 20.9, 17.9 by 96 x 96). A stage of the large tiles goes with BM + BN, 2.3 ns a row: its
 // loads; 256 x 192 and 256 x 288 have two stages of them in LDS and wait longer, and gain by their few rounds.
+// (Timed before tiles up to 192 x 160 had waves of their own for their loads, which took 5 % off them. Of 42 products of 100 to 2048 rows timed by
+// every tile since, the rule's is the fastest for 38, and 1.6, 1.6, 4 and 9 % behind for four.)
 struct TileRate {
   int bm, bn, modes, per_unit;  // modes: a bit each of 0, 2 and 3 (1, 2, 4); 8: rows of any length
   float fixed, stage[3];
