@@ -519,6 +519,16 @@ template <int... J>
 __device__ __forceinline__ void row_to_lds(const void* from, unsigned char* to, std::integer_sequence<int, J...>) {
   (load_to_lds<J * 64>(from, to + J * (1024 - 64)), ...);
 }
+// Two of them at once of 8 rows: 128 bytes apart in memory, 2 KB in LDS; lines that nobody reads again, for the caches not to keep.
+template <int OFFSET>
+__device__ __forceinline__ void load_lines_to_lds(const void* from, void* to) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off offset:%2 nt"
+               : : "v"(from), "s"((uint32_t)(uintptr_t)(lds_raw_t*)to), "n"(OFFSET) : "memory", "m0");
+}
+template <int... J>
+__device__ __forceinline__ void lines_to_lds(const void* from, unsigned char* to, std::integer_sequence<int, J...>) {
+  (load_lines_to_lds<J * 128>(from, to + J * (2048 - 128)), ...);
+}
 __device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, void* to) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                : : "v"(offset), "s"(base), "s"((uint32_t)(uintptr_t)(lds_raw_t*)to) : "memory", "m0");
@@ -547,7 +557,13 @@ template <int HD> struct DecodeTile {
   static constexpr int BYTES = 32 * HD * 4;  // 32 keys and values: a wave's LDS; its 16 heads' outputs lie over it at the end
 };
 
-template <int HD, bool POW2, int WAVES, bool CAP>
+// LINES (heads of whole lines): a load takes 128 bytes of 8 keys, whole lines that the caches need not keep, and a tile lies in LDS as blocks of
+// 16 keys x 64 elements, a key's eight granules permuted so that 16 lanes' operands (K: a granule of 16 keys; V: 32 bytes of four) take every
+// bank once. It costs a second table entry and address a key and pays where keys and values come at memory's speed. us, without / with, 2 heads of 128:
+// 32 requests of 1000 keys 13.1 / 11.5, 32 of 2048 18.3 / 15.6, 64 of 2048 27.2 / 23.7 (a decode step of those, 1.5B shape: 2255 / 2173); 8 of 2048,
+// in 256 workgroups of 160 keys, 10.7 / 10.0 alone and 1309 / 1324 a step; with few workgroups, whose time is trips to memory, 8 of 300 7.1 /
+// 8.3, one of 2048 9.2 / 9.8: these load half lines.
+template <int HD, bool POW2, int WAVES, bool CAP, bool LINES = false>
 __device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int item, const int y, const int split) {
   constexpr int NF = HD / 32;  // 32-element steps over the head dimension
   constexpr int ND = HD / 16;  // 16-wide blocks of the head dimension
@@ -619,25 +635,37 @@ __device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int it
   }
   // tile t into the wave's LDS; a masked key is read from a row of zeros
   unsigned char* const region = dec_smem + wave * Tile::BYTES;
-  const int f_key = lane >> 2, k_piece = k_granule(f_key, lane & 3) * 8, v_piece = v_granule(f_key, lane & 3) * 8;
+  // LINES: granule g of key k lies in slot g ^ (k >> 1 & 7) of its 128 bytes, of a value pair g / 2 of granules in pair g / 2 ^ (k >> 1 & 3)
+  const int f_key = lane >> 2;
+  const int k_piece = (LINES ? (lane & 7) ^ (lane >> 4) : k_granule(f_key, lane & 3)) * 8;
+  const int v_piece = (LINES ? ((((lane >> 1) ^ (lane >> 4)) & 3) << 1 | (lane & 1)) : v_granule(f_key, lane & 3)) * 8;
   auto bring = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      const int kp = t * 32 + kb * 16 + f_key;
+    for (int part = 0; part < (LINES ? 4 : 2); ++part) {  // of 8 keys or 16
+      const int kb = LINES ? part >> 1 : part, h = LINES ? part & 1 : 0;
+      const int kp = t * 32 + (LINES ? part * 8 + (lane >> 3) : part * 16 + f_key);
       const bool ok = kp >= lo && kp <= pos;
       const int at = ok ? cw_page_index<POW2>(kp, bs, sh) - page0 : 0;
       const int page = in_lds ? tbl[at] : ok ? table[page0 + at] : -1;
       const bool have = ok && page >= 0;
       const int64_t off = (((int64_t)page * bs + cw_page_offset<POW2>(kp, bs, sh)) * p.nkv + kvh) * HD;
-      const bf16_t* kr = (have ? kc + off : zrow) + k_piece;
+      const bf16_t* kr = (have ? kc + off : zrow) + (LINES ? k_piece ^ (h * 32) : k_piece);
       const bf16_t* vr = (have ? vc + off : zrow) + v_piece;
-      unsigned char* const to = region + kb * NF * 1024;
-      row_to_lds(kr, to, std::make_integer_sequence<int, NF>{});
-      row_to_lds(vr, to + Tile::BYTES / 2, std::make_integer_sequence<int, NF>{});
+      unsigned char* const to = region + kb * NF * 1024 + h * 1024;
+      if constexpr (LINES) {
+        lines_to_lds(kr, to, std::make_integer_sequence<int, NF / 2>{});
+        lines_to_lds(vr, to + Tile::BYTES / 2, std::make_integer_sequence<int, NF / 2>{});
+      } else {
+        row_to_lds(kr, to, std::make_integer_sequence<int, NF>{});
+        row_to_lds(vr, to + Tile::BYTES / 2, std::make_integer_sequence<int, NF>{});
+      }
     }
   };
-  const int k_at = c * 64 + k_granule(c, s) * 16, v_key = 4 * s + (c >> 2);
-  const int v_at0 = v_key * 64 + v_granule(v_key, 0) * 16 + (c & 3) * 8, v_at1 = v_at0 ^ 32;
+  const int v_key = 4 * s + (c >> 2);
+  const int k_at = LINES ? c * 128 + (s ^ (c >> 1)) * 16 : c * 64 + k_granule(c, s) * 16;
+  const int v_at = (LINES ? v_key * 128 + ((v_key >> 1) & 3) * 32 : v_key * 64 + v_granule(v_key, 0) * 16) + (c & 3) * 8;
+  auto k_in = [&](int j) __attribute__((always_inline)) { return LINES ? (j >> 1) * 2048 + (k_at ^ ((j & 1) * 64)) : j * 1024 + k_at; };  // step j of the head
+  auto v_in = [&](int db) __attribute__((always_inline)) { return LINES ? (db >> 2) * 2048 + (v_at ^ ((db & 3) * 32)) : (db >> 1) * 1024 + (v_at ^ ((db & 1) * 32)); };
 
   f32x4_t o[ND];
 #pragma unroll
@@ -654,10 +682,10 @@ __device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int it
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int j = 0; j < NF; ++j) kf[kb][j] = *reinterpret_cast<const bf16x8_t*>(region + (kb * NF + j) * 1024 + k_at);
+      for (int j = 0; j < NF; ++j) kf[kb][j] = *reinterpret_cast<const bf16x8_t*>(region + kb * NF * 1024 + k_in(j));
 #pragma unroll
     for (int db = 0; db < ND; ++db) {
-      unsigned char* vp = region + Tile::BYTES / 2 + (db >> 1) * 1024 + (db & 1 ? v_at1 : v_at0);
+      unsigned char* vp = region + Tile::BYTES / 2 + v_in(db);
       const s16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)vp);
       const s16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(vp + NF * 1024));
       vt[db] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
@@ -759,9 +787,9 @@ __device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int it
   }
 }
 
-template <int HD, bool POW2, int WAVES, bool CAP>
+template <int HD, bool POW2, int WAVES, bool CAP, bool LINES>
 __global__ __launch_bounds__(WAVES * 64) void attn_decode_bf16_kernel(AttnParams p) {
-  attn_decode_of<HD, POW2, WAVES, CAP>(p, blockIdx.x, blockIdx.y, blockIdx.z);
+  attn_decode_of<HD, POW2, WAVES, CAP, LINES>(p, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // Merge of the decode kernel's splits: one wave per (item, head, EL elements of the head). EL / 4 lanes take a split's
@@ -918,10 +946,22 @@ static int launch_decode_of(AttnParams& p, int n_items, hipStream_t stream) {
   static_assert(tiles <= DEC_MOST_LDS, "the waves' tiles fit LDS");
   p.decode_pages = decode_pages_in_lds(tiles, pages);
   const size_t smem = tiles + (p.decode_pages > 0 ? sizeof(int) * (size_t)p.decode_pages : 0);
-  static std::atomic<bool> allowed{false};
-  if (cw_allow_lds(allowed, (const void*)attn_decode_bf16_kernel<HD, POW2, WAVES, CAP>, DEC_MOST_LDS) != CW_OK) return CW_ERR_LAUNCH;
   dim3 grid(n_items, p.nkv * p.n_chunks, p.n_splits), block(WAVES * 64);
-  hipLaunchKernelGGL((attn_decode_bf16_kernel<HD, POW2, WAVES, CAP>), grid, block, smem, stream, p);
+  auto launch = [&](auto kernel, std::atomic<bool>& allowed) -> int {
+    if (cw_allow_lds(allowed, (const void*)kernel, DEC_MOST_LDS) != CW_OK) return CW_ERR_LAUNCH;
+    hipLaunchKernelGGL(kernel, grid, block, smem, stream, p);
+    return CW_OK;
+  };
+  static std::atomic<bool> allowed[2];
+  // whole lines where the card is as good as full of workgroups of 256 keys and more each: see attn_decode_of
+  int status = CW_OK;
+  if constexpr (HD % 64 == 0 && WAVES == 8) {
+    const bool lines = (int64_t)n_items * p.nkv * p.n_chunks * p.n_splits >= 192 && tiles_per_split >= 8;
+    status = lines ? launch(attn_decode_bf16_kernel<HD, POW2, WAVES, CAP, true>, allowed[1]) : launch(attn_decode_bf16_kernel<HD, POW2, WAVES, CAP, false>, allowed[0]);
+  } else {
+    status = launch(attn_decode_bf16_kernel<HD, POW2, WAVES, CAP, false>, allowed[0]);
+  }
+  if (status != CW_OK) return status;
   launch_decode_merge(p, n_items, stream);
   return cw_launch_status();
 }

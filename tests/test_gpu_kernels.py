@@ -1082,6 +1082,32 @@ def test_decode_attention_kernel(nh, nkv, hd, bs, ctx_lens, splits, fixed_ranges
         torch.testing.assert_close(out[r : r + 1].float().cpu(), want, **tol(dtype))
 
 
+# 24 requests of 1 to 700 keys in 2 splits: 192 workgroups of 8 waves and more, whose loads take whole lines; pages of a power of two and
+# not, a window that begins inside a tile, one key that holds all weight
+@pytest.mark.parametrize("nh,nkv,hd,bs", [(24, 4, 128, 16), (28, 4, 64, 16), (12, 4, 128, 24), (8, 4, 64, 4)])
+@pytest.mark.parametrize("window", [0, 75])
+@pytest.mark.parametrize("fixed_ranges", [False, True])
+def test_decode_attention_of_many_workgroups(nh, nkv, hd, bs, window, fixed_ranges):
+    gen = torch.Generator().manual_seed(nh + bs)
+    ctx_lens = [1, 700, 8, 9, 16, 17, 33, 177] + [int(c) for c in torch.randint(1, 700, (16,), generator=gen)]
+    num_blocks = sum(-(-c // bs) for c in ctx_lens) + 5
+    perm = torch.randperm(num_blocks, generator=gen).tolist()
+    tables, at = [], 0
+    for c in ctx_lens:
+        n = -(-c // bs)
+        tables.append(perm[at : at + n])
+        at += n
+    kc, vc, ks, vs = _paged_setup(torch.bfloat16, nkv, hd, bs, num_blocks, tables, ctx_lens, poison=float("nan"))
+    qs = [torch.randn(1, nh, hd, device=DEV).to(torch.bfloat16) for _ in ctx_lens]
+    for r, c in enumerate(ctx_lens):  # a key like the query that the first head of each group attends to
+        qs[r][0, :: nh // nkv] = 4.0 * ks[r][max(0, c - 5)]
+    out = _run_attention(torch.bfloat16, nh, nkv, hd, bs, tables, ctx_lens, [1] * len(ctx_lens), kc, vc, qs, splits=2, window=window,
+                         decode_kernel=True, fixed_ranges=fixed_ranges)
+    for r in range(len(ctx_lens)):
+        want = plain.attention_dense(qs[r].float().cpu(), ks[r].float().cpu(), vs[r].float().cpu(), hd ** -0.5, window=window or None)
+        torch.testing.assert_close(out[r : r + 1].float().cpu(), want, **tol(torch.bfloat16))
+
+
 @pytest.mark.parametrize("nh,nkv,hd,ctx", [(3, 1, 128, 20000), (2, 1, 256, 12000)])
 def test_decode_attention_of_a_table_that_does_not_fit_beside_the_tiles(nh, nkv, hd, ctx):
     """Pages of one key: a split's page numbers are looked up in memory."""
