@@ -241,7 +241,7 @@ CW_EXPORT int cw_gemm_bf16_tiled(int mode, const void* X, int64_t ldx, const voi
 
 
 // ------------------------------------------------------------------------------------------------
-// Wide tiles. One workgroup of 4 waves per compute unit owns 32 MB rows of x by 32 NB rows of W; a
+// Wide tiles. One workgroup of 4 waves, or of 8 of which four load (APART below), per compute unit owns 32 MB rows of x by 32 NB rows of W; a
 // wave owns a quarter of it in MB x NB accumulators of 16 x 16 (up to 288 registers; with 512
 // registers a wave a SIMD holds this one wave, so everything that has a latency is overlapped by hand).
 //
@@ -253,7 +253,7 @@ CW_EXPORT int cw_gemm_bf16_tiled(int mode, const void* X, int64_t ldx, const voi
 // touch every bank once. The descriptors end with the matrices, so rows past the end read as zeros.
 //
 // SLOTS stages are in LDS. A stage is two phases of 32 elements of K: a phase multiplies one register
-// set of fragments, reads the next phase's from LDS into the other set and takes part in the loads, all in
+// set of fragments, reads the next phase's from LDS into the other set and, of 4 waves, takes part in the loads, all in
 // the order written (sched_barrier). There is one wait and one barrier a stage, between its
 // phases: there every wave has read the whole stage, whose slot the loads of SLOTS stages on then take, and
 // stage t + 1 has landed, with SLOTS - 2 stages left in flight; the waits and barriers are bare
@@ -262,13 +262,13 @@ CW_EXPORT int cw_gemm_bf16_tiled(int mode, const void* X, int64_t ldx, const voi
 //
 // What bounds it. Inside a tile: with every load taken out the 1.5B shape's gate/up product of 2048
 // rows takes 0.85 of its time, of 160 rows 0.6. A compute unit was seen to take in 43 GB/s from memory and 80 from
-// L2 however deep the ring is (why is not known; a bound on its loads in flight would do that), so a tile's
+// L2 however deep the ring is, and x and W take the sum of what each takes alone (a queue of about 64 KB in the order of issue would do that), so a tile's
 // loads go with (MB + NB) K, and its matrix instructions with MB NB K. Around it: a tile's first
 // loads, its gate and its stores, 5 us a
 // tile of 256 x 288, which only the next tile's first loads overlap. So few large tiles beat many small ones, in whole
 // rounds over the units. Gate/up of the 1.5B shape, us by 256 x 192 tiles in stages of 32 -> here (tiles): 2048 rows
 // 110 -> 99 (256 x 288, 504 in two rounds: 1.14 PFLOP/s), 1000 rows 70 -> 50 (256 x 288, 252 in one), 512 rows 37.3 -> 36.5
-// (256 x 192, 188), 336 rows 35.6 -> 25.7 (192 x 160, 224), 160 rows 26.9 (64 x 128 below) -> 21.9 (160 x 96, 187). Two workgroups a unit of
+// (256 x 192, 188), 336 rows 35.6 -> 24.4 (192 x 160, 224), 160 rows 26.9 (64 x 128 below) -> 20.2 (160 x 96, 187). Two workgroups a unit of
 // half the LDS each, to overlap one's gate with the other's products, gain nothing (2048 rows: 110).
 //
 // The workgroups of a launch are dealt to the 8 XCDs in turn; each XCD takes a run of consecutive
