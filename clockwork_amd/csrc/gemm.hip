@@ -2051,23 +2051,30 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_join_bf16_kernel(const bf16_t
   if (blockIdx.x == gridDim.x - 1 && e_m < M && e_j > 0 && (int)blockIdx.x + e_j < parts) squares[e_m * parts + blockIdx.x + e_j] = 0.0f;
 }
 
-// How cw_gemm_bf16_join cuts a product: outputs a workgroup, of ``*slots`` that its kernel has room for, and waves. 0: it does not take
-// the product. Few rows of x beside the weights only: every workgroup takes in all of x, and from about 72 K elements on the planes and
-// the norm that adds them are the faster way (see the kernel: 8 rows of 8960 are even, 16 lose). Up to 16 outputs a compute unit in one
-// round, so that all units stream; a K of up to 2048 is one trip to memory for eight waves.
-static int join_plan(int M, int N, int K, int* slots, int* waves) {
-  if (M < 1 || M > 16 || N < 64 || N > 16 * cw_num_compute_units() || K < 256 || (K & 7) || (int64_t)M * K > 72 * 1024) return 0;
-  const int rows = (N + cw_num_compute_units() - 1) / cw_num_compute_units();
-  *waves = N <= 2048 && K <= 2048 ? 8 : 16;
+// How cw_gemm_bf16_join cuts a product on a card of ``units`` compute units: outputs a workgroup, of ``*slots`` that its kernel has
+// room for, and waves. 0: it does not take the product. Few rows of x beside the weights only: every workgroup takes in all of x, and from
+// about 72 K elements on the planes and the norm that adds them are the faster way (see the kernel: 8 rows of 8960 are even, 16 lose). Up to 16
+// outputs a compute unit in one round, so that all units stream; a K of up to 2048 is one trip to memory for eight waves, whose
+// workgroup has room for 8 outputs: on a card of fewer units, where more come to one, it has sixteen.
+static int join_plan(int M, int N, int K, int units, int* slots, int* waves) {
+  if (M < 1 || M > 16 || N < 64 || N > 16 * units || K < 256 || (K & 7) || (int64_t)M * K > 72 * 1024) return 0;
+  const int rows = (N + units - 1) / units;
+  *waves = N <= 2048 && K <= 2048 && rows <= 8 ? 8 : 16;
   *slots = rows > 8 ? 16 : rows > 4 || *waves == 8 ? 8 : 4;
   const int taken = *waves == 8 ? *slots : rows;
   return (N + taken - 1) / taken <= 256 ? taken : 0;  // pieces of a row that its reader takes
+}
+// The same as one number for a check of the rule: outputs + 256 slots + 65536 waves.
+CW_EXPORT int cw_gemm_bf16_join_rule(int M, int N, int K, int units) {
+  int slots = 0, waves = 0;
+  const int rows = units > 0 ? join_plan(M, N, K, units, &slots, &waves) : 0;
+  return rows ? rows | slots << 8 | waves << 16 : 0;
 }
 
 // The number of sums of squares that cw_gemm_bf16_join leaves of a row (zeros up to a multiple of 4 at the end), 0 where it does not take these sizes.
 CW_EXPORT int cw_gemm_bf16_join_parts(int M, int N, int K) {
   int slots, waves;
-  const int rows = join_plan(M, N, K, &slots, &waves);
+  const int rows = join_plan(M, N, K, cw_num_compute_units(), &slots, &waves);
   return rows ? ((N + rows - 1) / rows + 3) & ~3 : 0;
 }
 
@@ -2076,8 +2083,8 @@ CW_EXPORT int cw_gemm_bf16_join_parts(int M, int N, int K) {
 CW_EXPORT int cw_gemm_bf16_join(const void* X, const void* W, float* resid, const void* norm_weight, int norm_weight_f32, void* Y,
                                 float* squares, int M, int N, int K, hipStream_t stream) {
   int slots, waves;
-  const int rows = join_plan(M, N, K, &slots, &waves);
-  if (!rows) return CW_ERR_SIZE;
+  const int rows = join_plan(M, N, K, cw_num_compute_units(), &slots, &waves);
+  if (!rows || rows > slots) return CW_ERR_SIZE;
   if (!X || !W || !resid || !norm_weight || !Y || !squares || ((uintptr_t)X & 15) || ((uintptr_t)W & 15)) return CW_ERR_ARG;
   const dim3 grid((N + rows - 1) / rows);
 #define CW_JOIN(WAVES_, R_)                                                                                                  \

@@ -121,6 +121,7 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_gemm_bf16_group_ok": [I, I, I, L, I],
             "cw_gemm_bf16_group": [I, P, P, P, P, I, I, P],
             "cw_gemm_bf16_join_parts": [I, I, I],
+            "cw_gemm_bf16_join_rule": [I, I, I, I],
             "cw_gemm_bf16_join": [P, P, P, P, I, P, P, I, I, I, P],
             "cw_gemm_bf16_swiglu_begun": [P, P, I, F, P, P, L, I, I, I, P],
             "cw_gemm_qkv_rope_bf16": [P, L, P, P, I, P, P, P, P, P, P, L, I, I, I, I, I, P],

@@ -283,6 +283,24 @@ def test_large_outputs_of_a_long_k_are_the_librarys(M, N, K, there):
     assert (_wide_choice(0, M, N, K) is not None) == there
 
 
+# cards of 304 compute units down to 64, and a part of one
+@pytest.mark.parametrize("units", [304, 256, 128, 64, 32])
+def test_a_joining_product_has_room_for_its_outputs(units):
+    """A workgroup owns no more outputs than its kernel has room for (eight waves: 8), and the workgroups all of them."""
+    rule, taken = ops._load("gemm").cw_gemm_bf16_join_rule, 0
+    for N in (64, 72, 512, 896, 1000, 1024, 1536, 2048, 2056, 3584, 4096):
+        for K in (256, 896, 1536, 2048, 2056, 4864, 8960):
+            code = rule(1, N, K, units)
+            rows, slots, waves = code & 255, code >> 8 & 255, code >> 16
+            assert rows <= slots and (not code or (waves, slots) in ((8, 8), (16, 4), (16, 8), (16, 16)))
+            assert not code or -(-N // rows) <= min(units, 256)
+            taken += code != 0
+    assert taken
+    if units == 256:   # as its kernels were timed
+        assert [rule(8, N, K, units) for N, K in ((896, 896), (896, 4864), (1536, 1536), (1536, 8960), (3584, 3584))] == [
+            8 | 8 << 8 | 8 << 16, 4 | 4 << 8 | 16 << 16, 8 | 8 << 8 | 8 << 16, 6 | 8 << 8 | 16 << 16, 14 | 16 << 8 | 16 << 16]
+
+
 def test_few_rows_join_the_stream_between_blocks_only():
     """The mixer's output begins the second norm and the feed-forward's the next block's first one, where the parts take such
     rows and another block follows; the last block leaves its outputs to the final norm."""
