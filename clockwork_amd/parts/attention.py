@@ -351,7 +351,7 @@ class PagedAttention(Part):
         takes = getattr(self.position, "takes_begun_norm", None)
         return takes is not None and cache.writes and takes(n_tokens, self.qkv_weight, self.spec.head_dim)
 
-    def joins(self, n_tokens: int, norm) -> bool:
+    def joins_stream(self, n_tokens: int, norm) -> bool:
         """Can ``forward_joined`` add that many rows to the stream and begin ``norm``?"""
         return self.out_bias is None and ops.linear_join_ok(n_tokens, self.out_weight, norm.weight)
 

@@ -32,8 +32,14 @@ Roles and their run methods:
                  in one launch with others of the same x (``ops.linear_several``). And
                  ``before_output(x, ctx, cache, made=None)``: all but the product with ``out_weight``;
                  ``prepared_output`` and ``takes_beside`` put the kernel of one mixer of a pair into
-                 the other's launch.
+                 the other's launch. ``joins() -> bool`` with ``mix``: a scaled pair may make this
+                 mixer's products together with the other's.
 * feed-forward:  ``forward(x, ctx) -> y``.
+* mixer and feed-forward, of few rows: ``takes_begun_norm(rows, [the mixer's cache]) -> bool``: x may
+                 be an ``ops.BegunNorm``. ``joins_stream(rows, norm) -> bool`` with
+                 ``forward_joined(x, ctx, [cache,] resid, norm) -> ops.BegunNorm``: the output is added
+                 to ``resid`` and ``norm`` of that begun. A norm that this may be done to says
+                 ``can_be_begun``.
 * position enc.: used by a mixer, not by the block; the attention mixer expects
                  ``rotate_and_store(qkv, bias, positions, slots, nh, nkv, hd, k, v)``, and
                  uses ``project_rotate_store(x, weight, bias, positions, slots, nh, nkv, hd,

@@ -51,7 +51,7 @@ class PreNormBlock:
         # output joins the stream and begins the second norm in the kernel of its last product, and so does the
         # feed-forward's with the next block's first norm. Neither the residual adds nor the norms are launches then.
         T = resid.shape[0]
-        joins = getattr(self.mixer, "joins", None) if getattr(ctx, "block_follows", False) else None
+        joins = getattr(self.mixer, "joins_stream", None) if getattr(ctx, "block_follows", False) else None
         takes = getattr(self.feed_forward, "takes_begun_norm", None)
         if joins is not None and takes is not None and getattr(self.ffn_norm, "can_be_begun", False) and takes(T) and joins(T, self.ffn_norm):
             return self._feed(self.mixer.forward_joined(x, ctx, cache, resid, self.ffn_norm), resid, ctx, next_adds)
@@ -88,7 +88,7 @@ class PreNormBlock:
     def _feed(self, x, resid, ctx, next_adds: bool):
         """The feed-forward of ``x``, the stream being up to date: its output, or the next block's norm begun."""
         ctx.reader_adds_sums = next_adds
-        norm, joins = getattr(ctx, "norm_to_begin", None), getattr(self.feed_forward, "joins", None)
+        norm, joins = getattr(ctx, "norm_to_begin", None), getattr(self.feed_forward, "joins_stream", None)
         if norm is not None and joins is not None and joins(resid.shape[0], norm):
             return self.feed_forward.forward_joined(x, ctx, resid, norm)
         return self.feed_forward.forward(x, ctx)

@@ -37,7 +37,7 @@ class SwiGLU(Part):
         """May ``forward``'s input be an ``ops.BegunNorm`` of that many rows?"""
         return ops.swiglu_begun_ok(n_tokens, self.gate_up)
 
-    def joins(self, n_tokens: int, norm) -> bool:
+    def joins_stream(self, n_tokens: int, norm) -> bool:
         """Can ``forward_joined`` add that many rows to the stream and begin ``norm``?"""
         return ops.linear_join_ok(n_tokens, self.down, norm.weight)
 

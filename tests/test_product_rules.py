@@ -317,7 +317,7 @@ def test_few_rows_join_the_stream_between_blocks_only():
         def takes_begun_norm(self, n, *cache):
             return n <= self.most
 
-        def joins(self, n, norm):
+        def joins_stream(self, n, norm):
             return n <= self.most
 
         def forward(self, x, *rest):
@@ -347,3 +347,42 @@ def test_few_rows_join_the_stream_between_blocks_only():
     assert run(4, False, None, begun)[:2] == ([("mixer", "BegunNorm"), "n2", ("ffn", "Tensor")], False)
     assert run(17, True, None) == (["n1", ("mixer", "Tensor"), "n2", ("ffn", "Tensor")], False, None)
     assert run(4, True, None, begun=False) == (["n1", ("mixer", "Tensor"), "n2", ("ffn", "Tensor")], False, None)
+
+
+def _mixer_kinds():
+    import importlib
+    import inspect
+
+    from clockwork_amd import registry
+
+    kinds = []
+    for module, name in registry._BUILTIN_PARTS.values():
+        cls = getattr(importlib.import_module(module), name)
+        if list(inspect.signature(getattr(cls, "forward", lambda: None)).parameters)[:4] == ["self", "x", "ctx", "cache"]:
+            kinds.append(cls)
+    return kinds
+
+
+@pytest.mark.parametrize("cls", _mixer_kinds(), ids=lambda cls: cls.__name__)
+def test_every_mixer_in_a_block_whose_parts_join_the_stream(cls, monkeypatch):
+    """Few rows of bfloat16 in a block whose feed-forward and norms take part: a mixer that does not is run by ``forward``."""
+    import torch
+
+    from clockwork_amd.parts.block import PreNormBlock
+
+    mixer, out = cls.__new__(cls), torch.zeros(4, 8)
+    mixer.out_bias = torch.zeros(8)   # (plain attention with a bias behind its last product leaves the add to the norm)
+    monkeypatch.setattr(cls, "forward", lambda self, x, ctx, cache: out)
+    ffn = SimpleNamespace(takes_begun_norm=lambda n: True, joins_stream=lambda n, norm: False, forward=lambda x, ctx: x)
+    norm = SimpleNamespace(can_be_begun=True, forward=lambda resid, delta: torch.zeros(4, 8) if delta is None else delta)
+    got = PreNormBlock(mixer, norm, ffn, norm).forward(SimpleNamespace(shape=(4, 8)), None, SimpleNamespace(block_follows=True), None)
+    assert got is out
+
+
+def test_a_scaled_pair_refuses_mixers_without_a_place_between_products():
+    from clockwork_amd.parts.pair import PairMixer
+    from clockwork_amd.parts.specs import AttentionSpec, PairMixerSpec
+
+    side = AttentionSpec(hidden_size=64, num_heads=2, num_kv_heads=1, head_dim=32, qkv_bias=False, out_bias=False, scale=1.0)
+    with pytest.raises(NotImplementedError):
+        PairMixer(PairMixerSpec(hidden_size=64, left=side, right=side, scales=(0.5, 0.5)))
