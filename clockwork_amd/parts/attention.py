@@ -362,6 +362,10 @@ class PagedAttention(Part):
     def forward(self, x: torch.Tensor, ctx, cache: EntryCache) -> torch.Tensor:
         return self.output(self._before_output(x, ctx, cache), ctx)
 
+    def takes_rows(self) -> bool:
+        """Can ``forward_rows`` make chosen rows of the output alone?"""
+        return True
+
     def forward_rows(self, x, ctx, cache: EntryCache, rows, *others) -> tuple:
         """``forward``'s ``rows``, the cache being left as by all of them, and the same rows of ``others``."""
         out, *others = ops.take_rows(rows, self._before_output(x, ctx, cache), *others)

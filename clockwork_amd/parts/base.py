@@ -35,6 +35,13 @@ Roles and their run methods:
                  the other's launch. ``joins() -> bool`` with ``mix``: a scaled pair may make this
                  mixer's products together with the other's.
 * feed-forward:  ``forward(x, ctx) -> y``.
+* mixer and feed-forward, of a step's last block: a mixer with ``takes_rows() -> bool`` has, where that is
+                 true, ``forward_rows(x, ctx, cache, rows, *others) -> (y, others)``: ``forward``'s rows
+                 ``rows`` (int32), the cache being left as by all of them, and the same rows of the other
+                 matrices. A feed-forward whose rows depend on nothing else of the step says ``by_rows``, a
+                 final norm that norms a stream of chosen rows without ``rows`` ``takes_all_rows``; an
+                 arrangement of such parts offers ``takes_rows()`` and ``forward_rows(resid, delta, ctx,
+                 cache, rows) -> (resid, delta)``.
 * mixer and feed-forward, of few rows: ``takes_begun_norm(rows, [the mixer's cache]) -> bool``: x may
                  be an ``ops.BegunNorm``. ``joins_stream(rows, norm) -> bool`` with
                  ``forward_joined(x, ctx, [cache,] resid, norm) -> ops.BegunNorm``: the output is added

@@ -59,7 +59,7 @@ class PreNormBlock:
 
     def takes_rows(self) -> bool:
         """Can the block make chosen rows of its output alone (``forward_rows``)?"""
-        return hasattr(self.mixer, "forward_rows") and (self.feed_forward is None or getattr(self.feed_forward, "by_rows", False))
+        return getattr(self.mixer, "takes_rows", lambda: False)() and (self.feed_forward is None or getattr(self.feed_forward, "by_rows", False))
 
     def forward_rows(self, resid, delta, ctx, cache, rows):
         """``forward`` of the last block of a step: (the stream's ``rows``, what is still to be added to these). The cache
@@ -173,6 +173,8 @@ class ParallelBlock:
         is left as by all rows; what follows the mixer, and the feed-forward and the gates, are made of the chosen ones."""
         x = self.mixer_norm.forward(resid, delta)
         a, (x, resid) = self.mixer.forward_rows(x, ctx, cache, rows, x, resid)
+        if isinstance(a, ops.PartialSums):
+            a = a.sum(x.dtype)
         return resid, self._after(x, a, resid, ctx, None)
 
     def _after(self, x, a, resid, ctx, made):

@@ -386,3 +386,20 @@ def test_a_scaled_pair_refuses_mixers_without_a_place_between_products():
     side = AttentionSpec(hidden_size=64, num_heads=2, num_kv_heads=1, head_dim=32, qkv_bias=False, out_bias=False, scale=1.0)
     with pytest.raises(NotImplementedError):
         PairMixer(PairMixerSpec(hidden_size=64, left=side, right=side, scales=(0.5, 0.5)))
+
+
+@pytest.mark.parametrize("joint", [False, True])
+def test_blocks_take_chosen_rows_of_mixers_that_make_them(joint):
+    """A scaled pair whose mixers share one output product makes all rows, in either block; two mixers with outputs of their own make
+    the chosen ones; a mixer that does not know of it makes all."""
+    from clockwork_amd.parts.attention import PagedAttention
+    from clockwork_amd.parts.block import ParallelBlock, PreNormBlock
+    from clockwork_amd.parts.pair import PairMixer
+
+    pair = PairMixer.__new__(PairMixer)
+    pair.joint = joint
+    pair.left = pair.right = SimpleNamespace(before_output=None)
+    ffn, norm = SimpleNamespace(by_rows=True), SimpleNamespace()
+    for mixer, takes in ((pair, not joint), (PagedAttention.__new__(PagedAttention), True), (SimpleNamespace(), False)):
+        assert PreNormBlock(mixer, norm, ffn, norm).takes_rows() == ParallelBlock(mixer, norm, ffn).takes_rows() == takes
+        assert not PreNormBlock(mixer, norm, SimpleNamespace(), norm).takes_rows()
