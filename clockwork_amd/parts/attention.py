@@ -19,7 +19,7 @@ import torch
 
 from clockwork_amd import ops
 from clockwork_amd.config.spec import KVPagesSpec, ParamSpec
-from clockwork_amd.parts.base import EntryCache, Part
+from clockwork_amd.parts.base import EntryCache, Part, own_method
 from clockwork_amd.parts.rope import NoPosition
 from clockwork_amd.parts.specs import AttentionSpec
 from clockwork_amd.registry import build_part
@@ -349,11 +349,11 @@ class PagedAttention(Part):
     def takes_begun_norm(self, n_tokens: int, cache: EntryCache) -> bool:
         """May ``forward``'s input be an ``ops.BegunNorm`` of that many rows?"""
         takes = getattr(self.position, "takes_begun_norm", None)
-        return takes is not None and cache.writes and takes(n_tokens, self.qkv_weight, self.spec.head_dim)
+        return takes is not None and own_method(self, PagedAttention) and cache.writes and takes(n_tokens, self.qkv_weight, self.spec.head_dim)
 
     def joins_stream(self, n_tokens: int, norm) -> bool:
         """Can ``forward_joined`` add that many rows to the stream and begin ``norm``?"""
-        return self.out_bias is None and ops.linear_join_ok(n_tokens, self.out_weight, norm.weight)
+        return own_method(self, PagedAttention) and self.out_bias is None and ops.linear_join_ok(n_tokens, self.out_weight, norm.weight)
 
     def forward_joined(self, x, ctx, cache: EntryCache, resid, norm) -> "ops.BegunNorm":
         """``forward``, its output added to ``resid`` and ``norm`` of that begun."""
@@ -364,7 +364,7 @@ class PagedAttention(Part):
 
     def takes_rows(self) -> bool:
         """Can ``forward_rows`` make chosen rows of the output alone?"""
-        return True
+        return own_method(self, PagedAttention)
 
     def forward_rows(self, x, ctx, cache: EntryCache, rows, *others) -> tuple:
         """``forward``'s ``rows``, the cache being left as by all of them, and the same rows of ``others``."""

@@ -46,13 +46,15 @@ Roles and their run methods:
                  be an ``ops.BegunNorm``. ``joins_stream(rows, norm) -> bool`` with
                  ``forward_joined(x, ctx, [cache,] resid, norm) -> ops.BegunNorm``: the output is added
                  to ``resid`` and ``norm`` of that begun. A norm that this may be done to says
-                 ``can_be_begun``.
+                 ``can_be_begun``. These hooks go past ``forward``: a built-in part's say no for a part
+                 derived from it with a ``forward`` of its own (``own_method``).
 * position enc.: used by a mixer, not by the block; the attention mixer expects
                  ``rotate_and_store(qkv, bias, positions, slots, nh, nkv, hd, k, v)``, and
                  uses ``project_rotate_store(x, weight, bias, positions, slots, nh, nkv, hd,
                  k, v) -> q or None`` when the part offers it (product, encoding and cache
                  write in one kernel), and where that has nothing ``project_rotate_store_rows``,
-                 with the context in the place of the positions.
+                 with the context in the place of the positions. ``takes_begun_norm(rows, weight, hd) ->
+                 bool``: x of ``project_rotate_store`` may be an ``ops.BegunNorm``.
 * arrangement:   built by its factory from the block's parts as keyword arguments, under
                  the names the ``LayerSpec`` gives them (``mixer``, ``feed_forward``,
                  ``mixer_norm``, ``ffn_norm`` or any others). ``parts() -> {name: part}``;
@@ -102,6 +104,12 @@ class Part:
 
     def cache_need(self) -> Optional[Any]:
         return None
+
+
+def own_method(part, cls, name: str = "forward") -> bool:
+    """Is ``part``'s method still the one that ``cls`` defines? A hook of ``cls`` that does by another way what the method
+    does holds for no part that has a method of its own: derived from ``cls``, or given to the object."""
+    return getattr(getattr(part, name, None), "__func__", None) is getattr(cls, name)
 
 
 @dataclass

@@ -3,6 +3,7 @@
 from __future__ import annotations
 
 from clockwork_amd import ops
+from clockwork_amd.parts.base import own_method
 
 
 class PreNormBlock:
@@ -39,7 +40,7 @@ class PreNormBlock:
         """The norm that the block before may begin (``ops.linear_join``), handing on an ``ops.BegunNorm``; None if this
         block's mixer does not take one of that many rows."""
         takes = getattr(self.mixer, "takes_begun_norm", None)
-        if takes is not None and getattr(self.mixer_norm, "can_be_begun", False) and takes(n_tokens, cache):
+        if own_method(self, PreNormBlock) and takes is not None and getattr(self.mixer_norm, "can_be_begun", False) and takes(n_tokens, cache):
             return self.mixer_norm
         return None
 
@@ -59,7 +60,8 @@ class PreNormBlock:
 
     def takes_rows(self) -> bool:
         """Can the block make chosen rows of its output alone (``forward_rows``)?"""
-        return getattr(self.mixer, "takes_rows", lambda: False)() and (self.feed_forward is None or getattr(self.feed_forward, "by_rows", False))
+        return (own_method(self, PreNormBlock) and getattr(self.mixer, "takes_rows", lambda: False)()
+                and (self.feed_forward is None or getattr(self.feed_forward, "by_rows", False)))
 
     def forward_rows(self, resid, delta, ctx, cache, rows):
         """``forward`` of the last block of a step: (the stream's ``rows``, what is still to be added to these). The cache
@@ -166,7 +168,8 @@ class ParallelBlock:
 
     def takes_rows(self) -> bool:
         """Can the block make chosen rows of its output alone (``forward_rows``)?"""
-        return getattr(self.mixer, "takes_rows", lambda: False)() and (self.feed_forward is None or getattr(self.feed_forward, "by_rows", False))
+        return (own_method(self, ParallelBlock) and getattr(self.mixer, "takes_rows", lambda: False)()
+                and (self.feed_forward is None or getattr(self.feed_forward, "by_rows", False)))
 
     def forward_rows(self, resid, delta, ctx, cache, rows):
         """``forward`` of the last block of a step: (the stream's ``rows``, what is still to be added to these). The cache

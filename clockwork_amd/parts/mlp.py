@@ -9,15 +9,20 @@ import torch
 
 from clockwork_amd import ops
 from clockwork_amd.config.spec import ParamSpec
-from clockwork_amd.parts.base import Part
+from clockwork_amd.parts.base import Part, own_method
 from clockwork_amd.parts.specs import SwiGLUSpec
 
 
 class SwiGLU(Part):
     graph_safe = True
-    by_rows = True   # a row of the output depends on that row of the input and on nothing else of the step
+
     def __init__(self, spec: SwiGLUSpec) -> None:
         self.spec = spec
+
+    @property
+    def by_rows(self) -> bool:
+        """A row of the output depends on that row of the input and on nothing else of the step."""
+        return own_method(self, SwiGLU)
 
     def param_specs(self):
         H, I = self.spec.hidden_size, self.spec.intermediate_size
@@ -35,11 +40,11 @@ class SwiGLU(Part):
 
     def takes_begun_norm(self, n_tokens: int) -> bool:
         """May ``forward``'s input be an ``ops.BegunNorm`` of that many rows?"""
-        return ops.swiglu_begun_ok(n_tokens, self.gate_up)
+        return own_method(self, SwiGLU) and ops.swiglu_begun_ok(n_tokens, self.gate_up)
 
     def joins_stream(self, n_tokens: int, norm) -> bool:
         """Can ``forward_joined`` add that many rows to the stream and begin ``norm``?"""
-        return ops.linear_join_ok(n_tokens, self.down, norm.weight)
+        return own_method(self, SwiGLU) and ops.linear_join_ok(n_tokens, self.down, norm.weight)
 
     def forward_joined(self, x, ctx, resid, norm) -> "ops.BegunNorm":
         """``forward``, its output added to ``resid`` and ``norm`` of that begun."""
@@ -57,11 +62,14 @@ class GatedMLP(Part):
     kernels of :class:`SwiGLU`."""
 
     graph_safe = True
-    by_rows = True
     partial_ok = False   # may the output come as ``ops.PartialSums``? A block whose next norm adds them up sets it
 
     def __init__(self, spec) -> None:
         self.spec = spec
+
+    @property
+    def by_rows(self) -> bool:
+        return own_method(self, GatedMLP)
 
     def param_specs(self):
         H, I = self.spec.hidden_size, self.spec.intermediate_size

@@ -6,14 +6,12 @@ import torch
 
 from clockwork_amd import ops
 from clockwork_amd.config.spec import ParamSpec
-from clockwork_amd.parts.base import Part
+from clockwork_amd.parts.base import Part, own_method
 from clockwork_amd.parts.specs import RMSNormSpec
 
 
 class RMSNorm(Part):
     graph_safe = True
-    # as a final norm: without ``rows`` it norms the whole of a stream that holds the chosen rows alone
-    takes_all_rows = True
     # takes a delta that is an ops.PendingPair (two branch outputs not yet added to the residual)
     accepts_pending = True
     # adds a delta that is an ops.PartialSums in its kernel, however many planes there are
@@ -45,8 +43,15 @@ class RMSNorm(Part):
         ops.add_rmsnorm(resid, delta, self.weight, self.spec.eps, out, weight2=other.weight, out2=out2)
         return out, out2
 
-    # a product that has added its output to the stream may begin this norm of it (``ops.linear_join``)
-    can_be_begun = True
+    @property
+    def takes_all_rows(self) -> bool:
+        """As a final norm: without ``rows`` it norms the whole of a stream that holds the chosen rows alone."""
+        return own_method(self, RMSNorm)
+
+    @property
+    def can_be_begun(self) -> bool:
+        """A product that has added its output to the stream may begin this norm of it (``ops.linear_join``)."""
+        return own_method(self, RMSNorm)
 
     def lazy(self, resid: torch.Tensor, delta) -> "ops.LazyAddNorm":
         """The norm of resid + delta for a consumer that computes it inside its own kernel; the
@@ -60,11 +65,14 @@ class LayerNorm(Part):
     block's gated branches (``ops.GatedBranches``): the gates' sigmoids are made inside the kernel."""
 
     graph_safe = True
-    takes_all_rows = True
     accepts_gated = True
 
     def __init__(self, spec) -> None:
         self.spec = spec
+
+    @property
+    def takes_all_rows(self) -> bool:
+        return own_method(self, LayerNorm)
 
     def param_specs(self):
         specs = {"weight": ParamSpec((self.spec.size,), precision="stored", init=("one_plus_uniform", 0.1))}

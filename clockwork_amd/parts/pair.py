@@ -13,7 +13,7 @@ import torch
 
 from clockwork_amd import ops
 from clockwork_amd.config.spec import CacheNeeds, ParamSpec
-from clockwork_amd.parts.base import EntryCache, Part
+from clockwork_amd.parts.base import EntryCache, Part, own_method
 from clockwork_amd.parts.specs import PairMixerSpec
 from clockwork_amd.registry import build_part
 
@@ -114,7 +114,7 @@ class PairMixer(Part):
 
     def takes_rows(self) -> bool:
         """Can ``forward_rows`` make chosen rows of the output alone?"""
-        return not self.joint and all(hasattr(m, "before_output") for m in (self.left, self.right))
+        return own_method(self, PairMixer) and not self.joint and all(hasattr(m, "before_output") for m in (self.left, self.right))
 
     def forward_rows(self, x, ctx, cache: EntryCache, rows, *others) -> tuple:
         """``forward``'s ``rows``, the caches being left as by all of them, and the same rows of ``others``."""

@@ -12,7 +12,7 @@ import math
 import torch
 
 from clockwork_amd import ops
-from clockwork_amd.parts.base import Part
+from clockwork_amd.parts.base import Part, own_method
 from clockwork_amd.parts.specs import RopeNeoxSpec
 
 
@@ -65,7 +65,7 @@ class RopeNeox(Part):
 
     def takes_begun_norm(self, n_tokens: int, weight, hd: int) -> bool:
         """May the x of ``project_rotate_store`` be an ``ops.BegunNorm`` of that many rows?"""
-        return ops.qkv_rope_begun_ok(n_tokens, weight, self.spec.rotary_dim, hd)
+        return own_method(self, RopeNeox, "project_rotate_store") and ops.qkv_rope_begun_ok(n_tokens, weight, self.spec.rotary_dim, hd)
 
     def project_rotate_store_rows(self, x, weight, bias, ctx, slots, nh, nkv, hd, k_cache, v_cache):
         """The same for a portion's rows: by a table of the step's angles, made by the first layer that asks in a pass

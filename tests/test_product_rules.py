@@ -403,3 +403,59 @@ def test_blocks_take_chosen_rows_of_mixers_that_make_them(joint):
     for mixer, takes in ((pair, not joint), (PagedAttention.__new__(PagedAttention), True), (SimpleNamespace(), False)):
         assert PreNormBlock(mixer, norm, ffn, norm).takes_rows() == ParallelBlock(mixer, norm, ffn).takes_rows() == takes
         assert not PreNormBlock(mixer, norm, SimpleNamespace(), norm).takes_rows()
+
+
+def test_parts_with_a_forward_of_their_own_are_not_passed_by():
+    """A part derived from a built-in one, or an object given a method, is run by that method: the hooks that go past it say no."""
+    import torch
+
+    from clockwork_amd.parts import attention, block, mlp, norm, pair, rope
+    from clockwork_amd.parts.base import EntryCache
+    from clockwork_amd.parts.specs import AttentionSpec, GatedMLPSpec, LayerNormSpec, RMSNormSpec, RopeNeoxSpec, SwiGLUSpec
+
+    cpu, H, I, hd = "cpu", 512, 1024, 64
+    begun = norm.RMSNorm(RMSNormSpec(H, 1e-6))
+    begun.weight = torch.ones(H)
+
+    def attn(cls, position=rope.RopeNeox):
+        part = cls(AttentionSpec(H, 8, 2, hd, False, False, 0.1, position=RopeNeoxSpec(hd, 1e4)))
+        part.position = position(part.spec.position)
+        part.bind({"qkv_weight": torch.zeros(12 * hd, H, dtype=torch.bfloat16), "out_weight": torch.zeros(H, H, dtype=torch.bfloat16)}, cpu, torch.bfloat16)
+        return part
+
+    def ffn(cls, spec=SwiGLUSpec(H, I)):
+        part = cls(spec)
+        part.bind({"gate_up_weight": torch.zeros(2 * I, H, dtype=torch.bfloat16), "down_weight": torch.zeros(H, I, dtype=torch.bfloat16)}, cpu, torch.bfloat16)
+        return part
+
+    def two(cls):
+        part = cls.__new__(cls)
+        part.joint, part.left, part.right = False, SimpleNamespace(before_output=None), SimpleNamespace(before_output=None)
+        return part
+
+    def pre(cls):
+        return cls(attn(attention.PagedAttention), begun, ffn(mlp.SwiGLU), begun)
+
+    def par(cls):
+        return cls(two(pair.PairMixer), begun, ffn(mlp.SwiGLU))
+
+    cache = EntryCache()
+    kinds = [(attention.PagedAttention, attn, "forward", [lambda p: p.takes_begun_norm(4, cache), lambda p: p.joins_stream(4, begun), lambda p: p.takes_rows()]),
+             (rope.RopeNeox, lambda cls: attn(attention.PagedAttention, cls), "project_rotate_store", [lambda p: p.takes_begun_norm(4, cache)]),
+             (mlp.SwiGLU, ffn, "forward", [lambda p: p.takes_begun_norm(4), lambda p: p.joins_stream(4, begun), lambda p: p.by_rows]),
+             (mlp.GatedMLP, lambda cls: ffn(cls, GatedMLPSpec(H, I)), "forward", [lambda p: p.by_rows]),
+             (norm.RMSNorm, lambda cls: cls(RMSNormSpec(H, 1e-6)), "forward", [lambda p: p.can_be_begun, lambda p: p.takes_all_rows]),
+             (norm.LayerNorm, lambda cls: cls(LayerNormSpec(H, 1e-6)), "forward", [lambda p: p.takes_all_rows]),
+             (pair.PairMixer, two, "forward", [lambda p: p.takes_rows()]),
+             (block.PreNormBlock, pre, "forward", [lambda p: p.takes_rows(), lambda p: p.norm_to_begin(4, cache) is begun]),
+             (block.ParallelBlock, par, "forward", [lambda p: p.takes_rows()])]
+    for cls, build, method, hooks in kinds:
+        same = type("Same", (cls,), {})
+        own = type("Own", (cls,), {method: lambda self, *args: None})
+        for hook in hooks:
+            assert hook(build(cls)) and hook(build(same)), cls
+            assert not hook(build(own)), cls
+        if cls is not rope.RopeNeox:
+            given = build(cls)
+            setattr(given, method, lambda *args: None)
+            assert not any(hook(given) for hook in hooks), cls
