@@ -175,7 +175,9 @@ class ParallelBlock:
         """``forward`` of the last block of a step: (the stream's ``rows``, what is still to be added to these). The cache
         is left as by all rows; what follows the mixer, and the feed-forward and the gates, are made of the chosen ones."""
         x = self.mixer_norm.forward(resid, delta)
-        a, (x, resid) = self.mixer.forward_rows(x, ctx, cache, rows, x, resid)
+        first = getattr(self.mixer, "input_weights", list)()
+        made = ops.linear_several([x] * len(first), first) if len(first) > 1 else None
+        a, (x, resid) = self.mixer.forward_rows(x, ctx, cache, rows, x, resid, **({} if made is None else {"made": made}))
         if isinstance(a, ops.PartialSums):
             a = a.sum(x.dtype)
         return resid, self._after(x, a, resid, ctx, None)

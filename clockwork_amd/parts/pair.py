@@ -116,9 +116,9 @@ class PairMixer(Part):
         """Can ``forward_rows`` make chosen rows of the output alone?"""
         return own_method(self, PairMixer) and not self.joint and all(hasattr(m, "before_output") for m in (self.left, self.right))
 
-    def forward_rows(self, x, ctx, cache: EntryCache, rows, *others) -> tuple:
+    def forward_rows(self, x, ctx, cache: EntryCache, rows, *others, made=None) -> tuple:
         """``forward``'s ``rows``, the caches being left as by all of them, and the same rows of ``others``."""
-        a, b, *others = ops.take_rows(rows, *self._before_outputs(x, ctx, *self._caches(cache), None), *others)
+        a, b, *others = ops.take_rows(rows, *self._before_outputs(x, ctx, *self._caches(cache), made), *others)
         return ops.rms_mean2(*self._last_products([a, b], ctx), self.left_norm, self.right_norm, self.spec.eps), others
 
     def _outputs(self, x, ctx, left, right, made):

@@ -459,3 +459,29 @@ def test_parts_with_a_forward_of_their_own_are_not_passed_by():
             given = build(cls)
             setattr(given, method, lambda *args: None)
             assert not any(hook(given) for hook in hooks), cls
+
+
+@pytest.mark.parametrize("taken", [False, True])
+def test_chosen_rows_keep_the_first_products_of_a_pair_in_one_launch(taken, monkeypatch):
+    """The last block of a portion of few rows makes its mixers' first products as every other block does."""
+    import torch
+
+    from clockwork_amd.parts.block import ParallelBlock
+
+    weights, asked, got = [torch.zeros(2, 8), torch.ones(3, 8)], [], {}
+
+    def several(xs, ws):
+        asked.append((len(xs), [w is v for w, v in zip(ws, weights)]))
+        return ["left", "right"] if taken else None
+
+    def forward_rows(x, ctx, cache, rows, *others, made=None):
+        got["made"] = made
+        return x[rows], [o[rows] for o in others]
+
+    monkeypatch.setattr(ops, "linear_several", several)
+    x = torch.randn(40, 8)
+    mixer = SimpleNamespace(input_weights=lambda: list(weights), forward_rows=forward_rows)
+    block = ParallelBlock(mixer, SimpleNamespace(forward=lambda resid, delta: x))
+    resid, pending = block.forward_rows(torch.zeros(40, 8), None, SimpleNamespace(next_norm_accepts_gated=True), None, torch.tensor([39]))
+    assert asked == [(2, [True, True])] and got["made"] == (["left", "right"] if taken else None)
+    assert resid.shape == (1, 8) and torch.equal(pending.a, x[39:])
