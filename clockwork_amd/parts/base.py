@@ -40,9 +40,9 @@ Roles and their run methods:
                  ``rows`` (int32), the cache being left as by all of them, and the same rows of the other
                  matrices. A feed-forward whose rows depend on nothing else of the step says ``by_rows``, a
                  final norm that norms a stream of chosen rows without ``rows`` ``takes_all_rows``; an
-                 arrangement of such parts offers ``takes_rows()`` and ``forward_rows(resid, delta, ctx,
-                 cache, rows) -> (resid, delta)``. Products of ``input_weights()`` that the block has made
-                 come as ``made``.
+                 arrangement of such parts offers ``takes_rows(rows, chosen) -> bool``, by what pays, and
+                 ``forward_rows(resid, delta, ctx, cache, rows) -> (resid, delta)``. Products of
+                 ``input_weights()`` that the block has made come as ``made``.
 * mixer and feed-forward, of few rows: ``takes_begun_norm(rows, [the mixer's cache]) -> bool``: x may
                  be an ``ops.BegunNorm``. ``joins_stream(rows, norm) -> bool`` with
                  ``forward_joined(x, ctx, [cache,] resid, norm) -> ops.BegunNorm``: the output is added

@@ -58,9 +58,12 @@ class PreNormBlock:
             return self._feed(self.mixer.forward_joined(x, ctx, cache, resid, self.ffn_norm), resid, ctx, next_adds)
         return self._after(self.mixer.forward(x, ctx, cache), resid, x.dtype, ctx, next_adds)
 
-    def takes_rows(self) -> bool:
-        """Can the block make chosen rows of its output alone (``forward_rows``)?"""
-        return (own_method(self, PreNormBlock) and getattr(self.mixer, "takes_rows", lambda: False)()
+    def takes_rows(self, rows: int, chosen: int) -> bool:
+        """Does the block make ``chosen`` of that many rows of its output alone (``forward_rows``)? At most half of them, of
+        more than 32: a step, us, all rows / the chosen one, 0.5B, 1.5B and 7B shapes: 32 tokens 825 / 827, 1381 / 1382, 3813 / 3788, 24
+        beside 8 requests 877 / 879, 1477 / 1478, 3947 / 3928; 64 tokens 981 / 978, 1629 / 1625, 4371 / 4336, 48 beside 16 requests 1059 /
+        1053, 1758 / 1753, 4641 / 4628, 96 tokens 1157 / 1152, 1933 / 1922, 4019 / 4006."""
+        return (rows > 32 and 0 < 2 * chosen <= rows and own_method(self, PreNormBlock) and getattr(self.mixer, "takes_rows", lambda: False)()
                 and (self.feed_forward is None or getattr(self.feed_forward, "by_rows", False)))
 
     def forward_rows(self, resid, delta, ctx, cache, rows):
@@ -166,15 +169,20 @@ class ParallelBlock:
         a = self.mixer.forward(x, ctx, cache) if made is None else self.mixer.forward(x, ctx, cache, made[: len(first)])
         return self._after(x, a, resid, ctx, made)
 
-    def takes_rows(self) -> bool:
-        """Can the block make chosen rows of its output alone (``forward_rows``)?"""
-        return (own_method(self, ParallelBlock) and getattr(self.mixer, "takes_rows", lambda: False)()
+    def takes_rows(self, rows: int, chosen: int) -> bool:
+        """Does the block make ``chosen`` of that many rows of its output alone (``forward_rows``)? At most half of them, of more than
+        16, and up to 64 no more than 16, since products of few rows take as long for 17 rows as for 32: a step of
+        four blocks, us, all rows / the chosen ones, widths of 896 and 1536: 16 tokens 369 / 371, 521 / 530; 32 tokens 545 / 540, 770 / 762, 24 beside 8
+        requests 525 / 522, 713 / 707; 64 tokens 843 / 830, 1193 / 1172, 48 beside 16 requests 796 / 800, 1072 / 1076; 96 tokens 470 /
+        456, 671 / 646."""
+        return (rows > 16 and 0 < 2 * chosen <= rows and (rows > 64 or chosen <= 16) and own_method(self, ParallelBlock) and getattr(self.mixer, "takes_rows", lambda: False)()
                 and (self.feed_forward is None or getattr(self.feed_forward, "by_rows", False)))
 
     def forward_rows(self, resid, delta, ctx, cache, rows):
         """``forward`` of the last block of a step: (the stream's ``rows``, what is still to be added to these). The cache
         is left as by all rows; what follows the mixer, and the feed-forward and the gates, are made of the chosen ones."""
         x = self.mixer_norm.forward(resid, delta)
+        # (the mixer's first products still as one launch: with 32 rows apart 8 us more, 549 and 770 a step)
         first = getattr(self.mixer, "input_weights", list)()
         made = ops.linear_several([x] * len(first), first) if len(first) > 1 else None
         a, (x, resid) = self.mixer.forward_rows(x, ctx, cache, rows, x, resid, **({} if made is None else {"made": made}))

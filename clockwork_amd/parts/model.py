@@ -212,10 +212,11 @@ class DecoderModel:
             ctx.reader_adds_sums = False   # for a part of the block: does whoever reads its output add them? The block says so
             layer = self.layers[entry.layer]
             # Only the rows that logits are asked of go on behind the last mixer, which every token's cache needs: of a prompt
-            # one. Above half of the rows taking them apart costs what it saves; a model of a single block makes all rows (it is
-            # run to look at that block's kernels).
-            if (i > 0 and not ctx.block_follows and 0 < 2 * ctx.num_logit_rows <= resid.shape[0] and getattr(self.final_norm, "takes_all_rows", False)
-                    and getattr(layer, "takes_rows", lambda: False)()):
+            # one. From how many rows on that pays is the arrangement's to say. A model of one block makes all rows: whoever runs
+            # one runs that block, and finds the kernels that a layer of a longer model has for a portion of that size.
+            last = i > 0 and not ctx.block_follows and getattr(self.final_norm, "takes_all_rows", False)
+            takes = getattr(layer, "takes_rows", None) if last else None
+            if takes is not None and takes(resid.shape[0], ctx.num_logit_rows):
                 resid, delta = layer.forward_rows(resid, delta, ctx, caches[i], ctx.logit_rows)
                 return self.head.forward(self.final_norm.forward(resid, delta), ctx)
             delta = layer.forward(resid, delta, ctx, caches[i])

@@ -996,28 +996,40 @@ def test_chosen_rows_of_several_matrices(widths, T, chosen):
         ops.take_rows(rows.long(), matrices[0])
 
 
+# 40 tokens, of which one, two, 16, half and more have logits: up to half are made alone behind the last mixer, in a block of a
+# pair no more than 16 of so few; three blocks of one mixer, pairs with and without a feed-forward (gates of one branch and of two); models of
+# one block make all
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("wanted", [[4], [0, 9], list(range(5)), list(range(6))])
-def test_the_last_block_makes_the_rows_that_are_asked_for(tmp_path, dtype, wanted):
-    """Logits of one, two and half of a portion's rows, which the last block makes alone, and of more, which come with all,
-    against those of all rows; and the token after them, which reads the last block's cache."""
+@pytest.mark.parametrize("wanted", [[39], [0, 33], list(range(16)), list(range(20)), list(range(21))], ids=len)
+@pytest.mark.parametrize("config", ["B", "one", "FA", "FC", "long"])
+def test_the_last_block_makes_the_rows_that_are_asked_for(tmp_path, monkeypatch, dtype, wanted, config):
+    """Logits of rows that the last block makes alone against those of all rows; and the token after them, which reads the last
+    block's pages and state."""
     from clockwork_amd.engine.batch import StepEntry
+    from clockwork_amd.parts import block
     from clockwork_amd.weights.random_init import write_random_model
     from tests import replay
-    from tests.configs import TINY_B
+    from tests.configs import FUVAVIK_A, FUVAVIK_C, FUVAVIK_LONG, TINY_B
 
-    model_dir = write_random_model(tmp_path / "model", TINY_B, 5)
-    tokens = torch.randint(0, TINY_B["vocab_size"], (11,), generator=torch.Generator().manual_seed(2)).tolist()
+    cfg = {"B": TINY_B, "one": dict(TINY_B, num_hidden_layers=1), "FA": FUVAVIK_A, "FC": FUVAVIK_C, "long": FUVAVIK_LONG}[config]
+    kind = block.PreNormBlock if config in ("B", "one") else block.ParallelBlock
+    model_dir = write_random_model(tmp_path / "model", cfg, 5)
+    tokens = torch.randint(0, cfg.get("vocab_size", cfg.get("vocab")), (41,), generator=torch.Generator().manual_seed(2)).tolist()
+    made, forward_rows = [], kind.forward_rows
+    monkeypatch.setattr(kind, "forward_rows", lambda self, resid, *a: made.append(resid.shape[0]) or forward_rows(self, resid, *a))
 
     def logits(rows):
         runner = replay.make_runner(model_dir, dtype, 8, 16)
-        runner.reserve("r", 0, 10)
-        first = runner.step([StepEntry("r", 0, tokens[:10], rows)]).clone()
-        runner.reserve("r", 10, 1)
-        return first, runner.step([StepEntry("r", 10, tokens[10:], [0])]).clone()
+        runner.reserve("r", 0, 40)
+        first = runner.step([StepEntry("r", 0, tokens[:40], rows)]).clone()
+        runner.reserve("r", 40, 1)
+        return first, runner.step([StepEntry("r", 40, tokens[40:], [0])]).clone()
 
-    all_rows, after = logits(list(range(10)))
+    all_rows, after = logits(list(range(40)))
+    assert not made
     got, then = logits(wanted)
+    taken = config not in ("one", "FC") and len(wanted) <= (20 if kind is block.PreNormBlock else 16)
+    assert made == ([40] if taken else [])
     bound = dict(rtol=1e-5, atol=1e-5) if dtype == "float32" else dict(rtol=2e-2, atol=2e-2)   # roundings of bfloat16 in another kernel
     torch.testing.assert_close(got, all_rows[wanted], **bound)
     torch.testing.assert_close(then, after, **bound)

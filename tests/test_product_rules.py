@@ -401,8 +401,14 @@ def test_blocks_take_chosen_rows_of_mixers_that_make_them(joint):
     pair.left = pair.right = SimpleNamespace(before_output=None)
     ffn, norm = SimpleNamespace(by_rows=True), SimpleNamespace()
     for mixer, takes in ((pair, not joint), (PagedAttention.__new__(PagedAttention), True), (SimpleNamespace(), False)):
-        assert PreNormBlock(mixer, norm, ffn, norm).takes_rows() == ParallelBlock(mixer, norm, ffn).takes_rows() == takes
-        assert not PreNormBlock(mixer, norm, SimpleNamespace(), norm).takes_rows()
+        pre, par = PreNormBlock(mixer, norm, ffn, norm), ParallelBlock(mixer, norm, ffn)
+        assert pre.takes_rows(100, 1) == par.takes_rows(100, 1) == takes
+        assert not PreNormBlock(mixer, norm, SimpleNamespace(), norm).takes_rows(100, 1)
+        # as few rows as are not worth it, none, more than half
+        for rows, chosen in ((16, 1), (100, 0), (100, 51)):
+            assert not pre.takes_rows(rows, chosen) and not par.takes_rows(rows, chosen)
+        assert not pre.takes_rows(32, 1) and pre.takes_rows(33, 16) == pre.takes_rows(64, 17) == takes
+        assert par.takes_rows(17, 1) == par.takes_rows(64, 16) == par.takes_rows(65, 17) == takes and not par.takes_rows(64, 17)
 
 
 def test_parts_with_a_forward_of_their_own_are_not_passed_by():
@@ -447,8 +453,8 @@ def test_parts_with_a_forward_of_their_own_are_not_passed_by():
              (norm.RMSNorm, lambda cls: cls(RMSNormSpec(H, 1e-6)), "forward", [lambda p: p.can_be_begun, lambda p: p.takes_all_rows]),
              (norm.LayerNorm, lambda cls: cls(LayerNormSpec(H, 1e-6)), "forward", [lambda p: p.takes_all_rows]),
              (pair.PairMixer, two, "forward", [lambda p: p.takes_rows()]),
-             (block.PreNormBlock, pre, "forward", [lambda p: p.takes_rows(), lambda p: p.norm_to_begin(4, cache) is begun]),
-             (block.ParallelBlock, par, "forward", [lambda p: p.takes_rows()])]
+             (block.PreNormBlock, pre, "forward", [lambda p: p.takes_rows(100, 1), lambda p: p.norm_to_begin(4, cache) is begun]),
+             (block.ParallelBlock, par, "forward", [lambda p: p.takes_rows(100, 1)])]
     for cls, build, method, hooks in kinds:
         same = type("Same", (cls,), {})
         own = type("Own", (cls,), {method: lambda self, *args: None})
