@@ -557,12 +557,17 @@ template <int HD> struct DecodeTile {
   static constexpr int BYTES = 32 * HD * 4;  // 32 keys and values: a wave's LDS; its 16 heads' outputs lie over it at the end
 };
 
-// LINES (heads of whole lines): a load takes 128 bytes of 8 keys, whole lines that the caches need not keep, and a tile lies in LDS as blocks of
+// LINES (heads of 128): a load takes 128 bytes of 8 keys, whole lines that the caches need not keep, and a tile lies in LDS as blocks of
 // 16 keys x 64 elements, a key's eight granules permuted so that 16 lanes' operands (K: a granule of 16 keys; V: 32 bytes of four) take every
-// bank once. It costs a second table entry and address a key and pays where keys and values come at memory's speed. us, without / with, 2 heads of 128:
-// 32 requests of 1000 keys 13.1 / 11.5, 32 of 2048 18.3 / 15.6, 64 of 2048 27.2 / 23.7 (a decode step of those, 1.5B shape: 2255 / 2173); 8 of 2048,
-// in 256 workgroups of 160 keys, 10.7 / 10.0 alone and 1309 / 1324 a step; with few workgroups, whose time is trips to memory, 8 of 300 7.1 /
-// 8.3, one of 2048 9.2 / 9.8: these load half lines.
+// bank once. It costs a second table entry and address a key and pays where keys and values come at memory's speed and nobody else reads them. Where
+// another request has the same pages (a prefix, a fork), whole lines past the caches come from memory each time: such a split, which looks
+// for one at its first page, loads half lines as a kernel without LINES. Same bits either way. us, half lines only / whole lines only / this, heads of 128,
+// nothing shared: 12 on 2, 64 requests of 2048 keys 31.7 / 29.3 / 29.9, 32 of 2048 20.4 / 19.3 / 19.7, 32 of 1000 14.4 / 13.8 / 14.1; 28 on 4, 64 of
+// 1500 42.4 / 36.3 / 36.6. The first 1024 keys of 32 of 64 requests of 2048 the same 26.9 / 28.8 / 25.6, of all 22.6 / 25.3 / 22.0, the first
+// 1900 16.7 / 21.9 / 17.3; 28 on 4, 1024 of 32 of 64 of 1500 33.2 / 33.5 / 29.4, of all 64 of 1200 17.6 / 22.0 / 17.9. 8 of 2048, in 256 workgroups of 160 keys,
+// 10.7 / 10.0 alone and 1309 / 1324 a step; with few workgroups, whose time is trips to memory, 8 of 300 7.1 / 8.3, one of 2048 9.2 / 9.8: half lines. So,
+// too, where a group's heads are cut into several workgroups, which read the same keys (66 heads on 1, 64 of 1000: 25.1 / 31.8), and heads of
+// 64, whose keys are one line each (14 on 2, 64 of 2048: 19.5 / 20.5).
 template <int HD, bool POW2, int WAVES, bool CAP, bool LINES = false>
 __device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int item, const int y, const int split) {
   constexpr int NF = HD / 32;  // 32-element steps over the head dimension
@@ -573,6 +578,7 @@ __device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int it
   int* const tbl = reinterpret_cast<int*>(dec_smem + WAVES * Tile::BYTES);
   __shared__ float M_s[WAVES][16];
   __shared__ float L_s[WAVES][16];
+  __shared__ int shared_s;
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, s = lane >> 4;
@@ -602,6 +608,18 @@ __device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int it
     const int n_pages = k_last >= k_first ? cw_page_index<POW2>(k_last, bs, sh) - page0 + 1 : 0;
     if (in_lds)
       for (int i = threadIdx.x; i < n_pages; i += WAVES * 64) tbl[i] = table[page0 + i];
+    // LINES (item i is request i): does one of the 64 requests after this one have the same page where this split begins? Asked for beside
+    // the entries above. (A row of the batch without a request may hold anything: its context ends inside its first page.)
+    if (LINES && wave == WAVES - 1) {
+      const int n = (int)gridDim.x, other = req + 1 + lane - (req + 1 + lane < n ? 0 : n);
+      bool same = lane + 1 < n && n_pages > 0;  // (so other is one of n)
+      if (same) {
+        const int mine = table[page0];
+        same = p.block_tables[(int64_t)other * p.table_stride + page0] == mine && mine >= 0 && p.ctx_lens[other] > k_first + bs;
+      }
+      const bool any = __any(same);
+      if (lane == 0) shared_s = any;
+    }
   }
   const int pos = ctx - qlen + tok0;
   const int lo = p.window > 0 ? max(0, pos - p.window + 1) : 0;
@@ -635,24 +653,26 @@ __device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int it
   }
   // tile t into the wave's LDS; a masked key is read from a row of zeros
   unsigned char* const region = dec_smem + wave * Tile::BYTES;
-  // LINES: granule g of key k lies in slot g ^ (k >> 1 & 7) of its 128 bytes, of a value pair g / 2 of granules in pair g / 2 ^ (k >> 1 & 3)
+  // lines: granule g of key k lies in slot g ^ (k >> 1 & 7) of its 128 bytes, of a value pair g / 2 of granules in pair g / 2 ^ (k >> 1 & 3)
+  const bool lines = LINES && __builtin_amdgcn_readfirstlane(shared_s) == 0;
   const int f_key = lane >> 2;
-  const int k_piece = (LINES ? (lane & 7) ^ (lane >> 4) : k_granule(f_key, lane & 3)) * 8;
-  const int v_piece = (LINES ? ((((lane >> 1) ^ (lane >> 4)) & 3) << 1 | (lane & 1)) : v_granule(f_key, lane & 3)) * 8;
-  auto bring = [&](int t) __attribute__((always_inline)) {
+  const int k_piece = (lines ? (lane & 7) ^ (lane >> 4) : k_granule(f_key, lane & 3)) * 8;
+  const int v_piece = (lines ? ((((lane >> 1) ^ (lane >> 4)) & 3) << 1 | (lane & 1)) : v_granule(f_key, lane & 3)) * 8;
+  auto bring_by = [&](auto whole, int t) __attribute__((always_inline)) {
+    constexpr bool WHOLE = decltype(whole)::value;
 #pragma unroll
-    for (int part = 0; part < (LINES ? 4 : 2); ++part) {  // of 8 keys or 16
-      const int kb = LINES ? part >> 1 : part, h = LINES ? part & 1 : 0;
-      const int kp = t * 32 + (LINES ? part * 8 + (lane >> 3) : part * 16 + f_key);
+    for (int part = 0; part < (WHOLE ? 4 : 2); ++part) {  // of 8 keys or 16
+      const int kb = WHOLE ? part >> 1 : part, h = WHOLE ? part & 1 : 0;
+      const int kp = t * 32 + (WHOLE ? part * 8 + (lane >> 3) : part * 16 + f_key);
       const bool ok = kp >= lo && kp <= pos;
       const int at = ok ? cw_page_index<POW2>(kp, bs, sh) - page0 : 0;
       const int page = in_lds ? tbl[at] : ok ? table[page0 + at] : -1;
       const bool have = ok && page >= 0;
       const int64_t off = (((int64_t)page * bs + cw_page_offset<POW2>(kp, bs, sh)) * p.nkv + kvh) * HD;
-      const bf16_t* kr = (have ? kc + off : zrow) + (LINES ? k_piece ^ (h * 32) : k_piece);
+      const bf16_t* kr = (have ? kc + off : zrow) + (WHOLE ? k_piece ^ (h * 32) : k_piece);
       const bf16_t* vr = (have ? vc + off : zrow) + v_piece;
       unsigned char* const to = region + kb * NF * 1024 + h * 1024;
-      if constexpr (LINES) {
+      if constexpr (WHOLE) {
         lines_to_lds(kr, to, std::make_integer_sequence<int, NF / 2>{});
         lines_to_lds(vr, to + Tile::BYTES / 2, std::make_integer_sequence<int, NF / 2>{});
       } else {
@@ -661,11 +681,18 @@ __device__ __forceinline__ void attn_decode_of(const AttnParams& p, const int it
       }
     }
   };
+  auto bring = [&](int t) __attribute__((always_inline)) {
+    if constexpr (LINES)
+      if (lines) return bring_by(std::true_type{}, t);
+    bring_by(std::false_type{}, t);
+  };
+  // where a lane finds its operands: of two steps of the head, or of four blocks of 16 elements, 2 KB each
   const int v_key = 4 * s + (c >> 2);
-  const int k_at = LINES ? c * 128 + (s ^ (c >> 1)) * 16 : c * 64 + k_granule(c, s) * 16;
-  const int v_at = (LINES ? v_key * 128 + ((v_key >> 1) & 3) * 32 : v_key * 64 + v_granule(v_key, 0) * 16) + (c & 3) * 8;
-  auto k_in = [&](int j) __attribute__((always_inline)) { return LINES ? (j >> 1) * 2048 + (k_at ^ ((j & 1) * 64)) : j * 1024 + k_at; };  // step j of the head
-  auto v_in = [&](int db) __attribute__((always_inline)) { return LINES ? (db >> 2) * 2048 + (v_at ^ ((db & 3) * 32)) : (db >> 1) * 1024 + (v_at ^ ((db & 1) * 32)); };
+  const int k0 = lines ? c * 128 + (s ^ (c >> 1)) * 16 : c * 64 + k_granule(c, s) * 16, k1 = lines ? k0 ^ 64 : k0 + 1024;
+  const int v_base = (lines ? v_key * 128 + ((v_key >> 1) & 3) * 32 : v_key * 64 + v_granule(v_key, 0) * 16) + (c & 3) * 8;
+  const int v_at[4] = {v_base, v_base ^ 32, lines ? v_base ^ 64 : v_base + 1024, lines ? v_base ^ 96 : (v_base ^ 32) + 1024};
+  auto k_in = [&](int j) __attribute__((always_inline)) { return (j >> 1) * 2048 + (j & 1 ? k1 : k0); };  // step j of the head
+  auto v_in = [&](int db) __attribute__((always_inline)) { return (db >> 2) * 2048 + v_at[db & 3]; };
 
   f32x4_t o[ND];
 #pragma unroll
@@ -953,10 +980,11 @@ static int launch_decode_of(AttnParams& p, int n_items, hipStream_t stream) {
     return CW_OK;
   };
   static std::atomic<bool> allowed[2];
-  // whole lines where the card is as good as full of workgroups of 256 keys and more each: see attn_decode_of
+  // whole lines where the card is as good as full of workgroups of 256 keys and more each, at places that they know before the context's
+  // length (the look for the same page elsewhere costs no trip of its own then): see attn_decode_of
   int status = CW_OK;
-  if constexpr (HD % 64 == 0 && WAVES == 8) {
-    const bool lines = (int64_t)n_items * p.nkv * p.n_chunks * p.n_splits >= 192 && tiles_per_split >= 8;
+  if constexpr (HD == 128 && WAVES == 8) {
+    const bool lines = p.identity && p.split_keys >= 256 && p.n_chunks == 1 && (int64_t)n_items * p.nkv * p.n_splits >= 192;
     status = lines ? launch(attn_decode_bf16_kernel<HD, POW2, WAVES, CAP, true>, allowed[1]) : launch(attn_decode_bf16_kernel<HD, POW2, WAVES, CAP, false>, allowed[0]);
   } else {
     status = launch(attn_decode_bf16_kernel<HD, POW2, WAVES, CAP, false>, allowed[0]);

@@ -1082,8 +1082,8 @@ def test_decode_attention_kernel(nh, nkv, hd, bs, ctx_lens, splits, fixed_ranges
         torch.testing.assert_close(out[r : r + 1].float().cpu(), want, **tol(dtype))
 
 
-# 24 requests of 1 to 700 keys in 2 splits: 192 workgroups of 8 waves and more, whose loads take whole lines; pages of a power of two and
-# not, a window that begins inside a tile, one key that holds all weight
+# 24 requests of 1 to 700 keys in 2 splits: 192 workgroups of 8 waves and more, whose loads take whole lines where their places are fixed and
+# heads are of 128; pages of a power of two and not, a window that begins inside a tile, one key that holds all weight
 @pytest.mark.parametrize("nh,nkv,hd,bs", [(24, 4, 128, 16), (28, 4, 64, 16), (12, 4, 128, 24), (8, 4, 64, 4)])
 @pytest.mark.parametrize("window", [0, 75])
 @pytest.mark.parametrize("fixed_ranges", [False, True])
@@ -1106,6 +1106,48 @@ def test_decode_attention_of_many_workgroups(nh, nkv, hd, bs, window, fixed_rang
     for r in range(len(ctx_lens)):
         want = plain.attention_dense(qs[r].float().cpu(), ks[r].float().cpu(), vs[r].float().cpu(), hd ** -0.5, window=window or None)
         torch.testing.assert_close(out[r : r + 1].float().cpu(), want, **tol(torch.bfloat16))
+
+
+# splits of 352 keys: the first one's keys the same for some requests, all of two requests' the same, pages of a power of two and not; the
+# shared requests side by side or not, and one whose context ends inside the shared part
+@pytest.mark.parametrize("bs,shared", [(16, list(range(2, 14))), (16, [0, 5, 23]), (24, [1, 4, 9, 16, 20]), (32, [])])
+@pytest.mark.parametrize("window", [0, 75])
+def test_decode_attention_of_pages_that_several_requests_have(bs, shared, window):
+    """The outputs are those of requests that have copies of the pages, bit for bit, and those are attention."""
+    nh, nkv, hd, prefix = 24, 4, 128, 384
+    gen = torch.Generator().manual_seed(bs + len(shared))
+    ctx_lens = [int(c) for c in torch.randint(prefix + 1, 700, (24,), generator=gen)]
+    ctx_lens[11], ctx_lens[17] = 700, 9
+    if shared:
+        ctx_lens[shared[-1]] = prefix - 40
+    num_blocks = sum(-(-c // bs) for c in ctx_lens) + 5
+    perm = torch.randperm(num_blocks, generator=gen).tolist()
+    tables, at = [], 0
+    for c in ctx_lens:
+        n = -(-c // bs)
+        tables.append(perm[at : at + n])
+        at += n
+    kc, vc, ks, vs = _paged_setup(torch.bfloat16, nkv, hd, bs, num_blocks, tables, ctx_lens, poison=float("nan"))
+    with_shared = [list(t) for t in tables]
+    pairs = [(shared[0], r, min(prefix, ctx_lens[r]) // bs) for r in shared[1:]]
+    twin = next(r for r in range(24) if r not in shared and r != 17)
+    other = next(r for r in range(23, 0, -1) if r not in shared and r not in (17, twin))
+    n = min(len(tables[twin]), len(tables[other])) - 1
+    for a, b, pages in pairs + [(twin, other, n)]:
+        for i in range(pages):
+            for c, own in ((kc, ks), (vc, vs)):
+                src = c[tables[a][i] * bs : (tables[a][i] + 1) * bs]
+                c[tables[b][i] * bs : (tables[b][i] + 1) * bs] = src
+                own[b][i * bs : (i + 1) * bs] = src
+            with_shared[b][i] = tables[a][i]
+    qs = [torch.randn(1, nh, hd, device=DEV).to(torch.bfloat16) for _ in ctx_lens]
+    run = lambda t: _run_attention(torch.bfloat16, nh, nkv, hd, bs, t, ctx_lens, [1] * 24, kc, vc, qs, splits=2, window=window,
+                                   decode_kernel=True, fixed_ranges=True)
+    apart, together = run(tables), run(with_shared)
+    assert torch.equal(apart, together)
+    for r in range(24):
+        want = plain.attention_dense(qs[r].float().cpu(), ks[r].float().cpu(), vs[r].float().cpu(), hd ** -0.5, window=window or None)
+        torch.testing.assert_close(together[r : r + 1].float().cpu(), want, **tol(torch.bfloat16))
 
 
 @pytest.mark.parametrize("nh,nkv,hd,ctx", [(3, 1, 128, 20000), (2, 1, 256, 12000)])
