@@ -264,12 +264,15 @@ struct DrawCounts {
 
 // Chunks a row is cut into: at least 2048 tokens each; 64 for few rows, for many rows as few as still make two
 // thousand workgroups (a row's bins take an addition from each).
+// The most tokens of a chunk whose weights (2^40 at most) a thread may add up in float64: of 2^21 it takes 4 of every 1024, 2^13, and
+// every sum of these is a whole number of at most 2^53, which float64 holds.
+#define SAMPLE_FLOAT64_TOKENS (1 << 21)
+static_assert(4ll * (SAMPLE_FLOAT64_TOKENS / (4 * SAMPLE_THREADS)) << 40 <= 1ll << 53, "a thread's sums are exact");
 static int sample_chunks(int n, int V) {
   int c = (V + 2047) / 2048;
   const int most = n <= 32 ? SAMPLE_MAX_CHUNKS : n >= 512 ? 4 : 2048 / n;
   if (c > most) c = most;
-  // (of at most 2^21 tokens: what a thread adds up of one stays below 2^53)
-  const int least = (int)(((int64_t)V + (1 << 21) - 1) >> 21);
+  const int least = (int)(((int64_t)V + SAMPLE_FLOAT64_TOKENS - 1) / SAMPLE_FLOAT64_TOKENS);
   if (c < least) c = least < SAMPLE_MAX_CHUNKS ? least : SAMPLE_MAX_CHUNKS;
   return c < 1 ? 1 : c;
 }
@@ -625,13 +628,20 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_hist_kernel(SampleArgs 
   }
   const Quotient over_t(temp);
   if (!with_k && !with_p) {
-    // a thread's sum of whole numbers below 2^53 as float64, exact: one conversion a token instead of a 64-bit integer's six instructions
-    double sum = 0.0;
-    sample_walk(x, lo, hi, a.vec, [&](int, float raw) __attribute__((always_inline)) {
-      const float e = expf(over_t.of(raw) - mx);  // NaN: no weight
-      sum += e == e ? (double)truncf(e * SAMPLE_WEIGHT_SCALE) : 0.0;
-    });
-    const u64_t total = block_sum((u64_t)sum);
+    // a thread's sum of whole numbers as float64, exact: one conversion a token instead of a 64-bit integer's six instructions. (Of
+    // more than 64 chunks' tokens, 2^27 logits, a chunk has more than such a sum may: those are added up as integers.)
+    u64_t mine = 0;
+    if (a.per <= SAMPLE_FLOAT64_TOKENS) {
+      double sum = 0.0;
+      sample_walk(x, lo, hi, a.vec, [&](int, float raw) __attribute__((always_inline)) {
+        const float e = expf(over_t.of(raw) - mx);  // NaN: no weight
+        sum += e == e ? (double)truncf(e * SAMPLE_WEIGHT_SCALE) : 0.0;
+      });
+      mine = (u64_t)sum;
+    } else {
+      sample_walk(x, lo, hi, a.vec, [&](int, float raw) __attribute__((always_inline)) { mine += weight_of(over_t.of(raw), mx); });
+    }
+    const u64_t total = block_sum(mine);
     if (threadIdx.x == 0) a.sums[(int64_t)row * a.chunks + chunk] = total;
     return;
   }

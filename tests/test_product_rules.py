@@ -301,6 +301,17 @@ def test_a_joining_product_has_room_for_its_outputs(units):
             8 | 8 << 8 | 8 << 16, 4 | 4 << 8 | 16 << 16, 8 | 8 << 8 | 8 << 16, 6 | 8 << 8 | 16 << 16, 14 | 16 << 8 | 16 << 16]
 
 
+@pytest.mark.parametrize("n", [1, 32, 33, 64, 512, 65535])
+@pytest.mark.parametrize("V", [1, 2048, 151936, (1 << 21) + 1, (1 << 24) + 5, (1 << 26) - 3, 1 << 27])
+def test_chunks_of_a_row_of_logits_have_few_enough_tokens_for_float64_sums(n, V):
+    """4 tokens of every 1024 a thread, each a weight of up to 2^40: at most 2^53 in all (2^27 logits are 64 chunks of 2^21)."""
+    need = ops._load("sampling").cw_sample_workspace_bytes
+    one = need(1, 1) - 64 - 32   # what a row of one chunk needs beside the chunk's
+    chunks = ((need(n, V) - 64) // n - one) // 32
+    per = -(-(-(-V // chunks)) // 4) * 4
+    assert 1 <= chunks <= 64 and 4 * -(-per // 1024) * 2 ** 40 <= 2 ** 53
+
+
 def test_few_rows_join_the_stream_between_blocks_only():
     """The mixer's output begins the second norm and the feed-forward's the next block's first one, where the parts take such
     rows and another block follows; the last block leaves its outputs to the final norm."""
