@@ -297,8 +297,10 @@ __device__ __forceinline__ u64_t weight_of(float v, float mx) {
 // A row's temperature and what divides by it. ``of(a)`` is a / T, rounded once: a product with the reciprocal, then twice the remainder
 // times the reciprocal, each remainder exact by a fused multiply-add; the first step leaves a quotient that is off by less than one
 // unit of its last place, and of such a one the second makes the correctly rounded quotient (Markstein). Five instructions for the
-// division's eleven, one of them at a quarter of the rate. Infinite quotients come out as NaN, which everything here takes for -inf (a row whose
-// largest logit is +inf has no weight at all, and its first maximum is taken).
+// division's eleven, one of them at a quarter of the rate. The same bits as the division's where 1 / T is a normal number (T from 3e-39 to 8.5e37) and
+// the remainders are exact (a from 2^-100 in size, or 0; -0 / T comes out as 0): of smaller a, and larger T, a quotient may be off by a unit of its last
+// place, next to 0, where every weight is the same. Infinite quotients come out as NaN, which everything here takes for -inf (a row whose
+// largest logit is +inf, or a T below 3e-39, leaves no weight at all, and its first maximum is taken, as with the division).
 struct Quotient {
   float t, y;
   __device__ __forceinline__ explicit Quotient(float temp) : t(temp), y(1.0f / temp) {}
