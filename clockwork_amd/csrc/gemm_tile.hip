@@ -860,10 +860,13 @@ static int w_launch(WideArgs a, int row_tiles, int workgroups, hipStream_t strea
     return cw_launch_status();
   };
   constexpr bool APART = w_loads_apart(MB, NB);
-  // Planes of many row tiles, which ask L2 for more than it gives in any case: alone they gain too (1000 rows of 1536 x 8960 32.3 / 31.0), behind a gate/up product and
-  // on a card whose clock is low they lose (1000 tokens behind 7000, 1.5B shape: 5800 / 5885 us on such a one, 5614 / 5593 on another).
+  // Of planes of more than four row tiles, which ask L2 for more than it gives in any case, only K whole or in two runs. Steps, us, loads by all waves / by waves
+  // of their own: two planes, 2048 tokens of the 1.5B shape 6950 / 6917 and 6902 / 6874 (two cards), behind 4000 8754 / 8732, 2000 beside 15 requests
+  // 7164 / 7140, of the 0.5B shape 3330 / 3313, 3318 / 3304, one or two, of the 7B shape 25339 / 25119, 25436 / 25211, 800 tokens 12229 / 11997; three
+  // planes, 1000 tokens of the 1.5B shape behind 7000 5885 / 5975, 5800 / 5885, 5614 / 5593 (three cards; the product alone 32.3 / 31.0), behind none 4129 /
+  // 4157; four, 700 and 800 tokens 3537 / 3530, 4373 / 4348.
   if constexpr (MODE == 3 && APART)
-    if (a.tiles_m > 4) return launch(std::false_type{});
+    if (a.tiles_m > 4 && a.k_splits > 2) return launch(std::false_type{});
   return launch(std::integral_constant<bool, APART>{});
 }
 
