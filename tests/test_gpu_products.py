@@ -243,6 +243,29 @@ def test_tiles_of_the_wide_kernel(mode, bm, bn, M, N, K):
             torch.testing.assert_close(got.parts[0], x[:, :first].float() @ w[:, :first].float().t(), **f32)
 
 
+# 32 MB and more of W beside one or two row tiles: whole lines past the caches; few stages and several tiles a workgroup, many stages and one
+@pytest.mark.parametrize("mode,bm,bn", [(mode, *t) for mode, tiles in WIDE_TILES.items() for t in tiles if t[0] * t[1] <= 32 * 1024])
+@pytest.mark.parametrize("N,K", [(30016, 576), (8208, 2112)])
+def test_tiles_of_a_matrix_that_is_read_once(mode, bm, bn, N, K):
+    from clockwork_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(N + bm)
+    w = (torch.randn(N, K, device=DEV, generator=gen) / K ** 0.5).to(torch.bfloat16)
+    # as above: float32 sums of K products of about 1 / sqrt(K), one rounding to bfloat16
+    f32, bf16 = dict(rtol=1e-4, atol=1e-4), dict(rtol=2.0 ** -8 + 1e-4, atol=1e-4)
+    for M in (bm - 7, bm + 1, 2 * bm):
+        x = torch.randn(M, K, device=DEV, generator=gen).to(torch.bfloat16)
+        want = x.float() @ w.float().t()
+        if mode == 0:
+            torch.testing.assert_close(ops.linear_mid(x, w, bm | bn << 10 | 1 << 20).float(), want, **bf16)
+        elif mode == 2:
+            ref = torch.nn.functional.silu(want[:, : N // 2]) * want[:, N // 2:]
+            torch.testing.assert_close(ops.linear_mid(x, w, bm | bn << 10 | 1 << 20, swiglu=True).float(), ref, **bf16)
+        else:
+            for planes in (1, 3):
+                torch.testing.assert_close(ops.linear_mid(x, w, bm | bn << 10 | planes << 20, partial=True).sum(), want, **f32)
+
+
 @pytest.mark.parametrize("mode,N", [(0, 1001), (2, 2 * 1004), (3, 1002)])
 def test_tiles_for_whole_rows_refuse_others(mode, N):
     """Results whose rows are no multiples of 16 bytes: refused where a tile takes whole rows only, and served by another."""
