@@ -211,7 +211,9 @@ class ModelRunner:
         counts = {int(c) for c in token_counts}
         if any(c <= ops.SKINNY_MAX_ROWS for c in counts):
             counts.add(self.FEW_ROWS_SAMPLE)
-        for n in sorted(counts, reverse=True):
+        # the step of few rows first: a long portion's last block multiplies the one row that logits are asked of, and would time
+        # the choices for few rows on that
+        for n in sorted(counts, key=lambda n: (n != self.FEW_ROWS_SAMPLE, -n)):
             if (n <= ops.SKINNY_MAX_ROWS and n != self.FEW_ROWS_SAMPLE) or n > limit:
                 continue
             seq_id = "__tune_products__"
@@ -225,7 +227,7 @@ class ModelRunner:
                 done.append(n)
             finally:
                 self.release(seq_id)
-        return done
+        return sorted(done, reverse=True)
 
     # ------------------------------------------------------------------ decode steps as graphs
     def _graph_step(self, entries: Sequence[StepEntry]):

@@ -502,3 +502,24 @@ def test_chosen_rows_keep_the_first_products_of_a_pair_in_one_launch(taken, monk
     resid, pending = block.forward_rows(torch.zeros(40, 8), None, SimpleNamespace(next_norm_accepts_gated=True), None, torch.tensor([39]))
     assert asked == [(2, [True, True])] and got["made"] == (["left", "right"] if taken else None)
     assert resid.shape == (1, 8) and torch.equal(pending.a, x[39:])
+
+
+@pytest.mark.parametrize("counts", [[2048, 1, 2, 64], [300, 8], [48, 24]])
+def test_choices_for_few_rows_are_timed_on_the_step_of_few_rows(counts, monkeypatch):
+    """A tuning start-up runs it ahead of the long portions, whose last block multiplies one row."""
+    import contextlib
+
+    import torch
+
+    from clockwork_amd.engine.model_runner import ModelRunner
+
+    ran = []
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: None)
+    monkeypatch.setattr(ops, "library_tuning", lambda policy: contextlib.nullcontext())
+    runner = SimpleNamespace(dtype=torch.bfloat16, cfg=SimpleNamespace(model=SimpleNamespace(max_model_len=4096)), _table_width=256, products=None,
+                             manager=SimpleNamespace(block_size=16, can_admit=lambda *a: True), FEW_ROWS_SAMPLE=ModelRunner.FEW_ROWS_SAMPLE,
+                             reserve=lambda *a, **k: None, release=lambda s: None, step=lambda entries: ran.append(len(entries[0].tokens)))
+    few = min(counts) <= ops.SKINNY_MAX_ROWS
+    large = sorted((c for c in counts if c > ops.SKINNY_MAX_ROWS), reverse=True)
+    assert ModelRunner.tune_products(runner, counts) == large + [8] * few
+    assert ran == [8] * few + large
