@@ -2052,9 +2052,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_join_bf16_kernel(const bf16_t
 }
 
 // How cw_gemm_bf16_join cuts a product on a card of ``units`` compute units: outputs a workgroup, of ``*slots`` that its kernel has
-// room for, and waves. 0: it does not take the product. Few rows of x beside the weights only: every workgroup takes in all of x, and from
-// about 72 K elements on the planes and the norm that adds them are the faster way (see the kernel: 8 rows of 8960 are even, 16 lose). Up to 16
-// outputs a compute unit in one round, so that all units stream; a K of up to 2048 is one trip to memory for eight waves, whose
+// room for, and waves. 0: it does not take the product. Few rows of x beside the weights only, up to 72 K elements: every workgroup takes in
+// all of x. Up to 16 outputs a compute unit in one round, so that all units stream; a K of up to 2048 is one trip to memory for eight waves, whose
 // workgroup has room for 8 outputs: on a card of fewer units, where more come to one, it has sixteen.
 static int join_plan(int M, int N, int K, int units, int* slots, int* waves) {
   if (M < 1 || M > 16 || N < 64 || N > 16 * units || K < 256 || (K & 7) || (int64_t)M * K > 72 * 1024) return 0;
@@ -2069,6 +2068,19 @@ CW_EXPORT int cw_gemm_bf16_join_rule(int M, int N, int K, int units) {
   int slots = 0, waves = 0;
   const int rows = units > 0 ? join_plan(M, N, K, units, &slots, &waves) : 0;
   return rows ? rows | slots << 8 | waves << 16 : 0;
+}
+
+// Is that also the faster way for a layer, against planes (of whole lines from 64 MB on) and the norm that adds them? Up to 64 K elements of x; where a
+// workgroup has more than 8 outputs and its K is more than the one trip of 16 waves with 8 operands each, up to 16 K. Decode steps, us, a feed-forward's output
+// as planes / joined (its mixer's joined), rows: 896 x 4864 1 712 / 673, 8 758 / 733; 1536 x 8960 1 1182 / 1180, 2 1191 / 1185, 4 1210 / 1205, 8 1244 /
+// 1257; 2048 x 11008 1 1826 / 1808, 2 1845 / 1826, 4 1866 / 1856; 2560 x 9728 1 2234 / 2223, 2 2247 / 2244, 4 2278 / 2297; 4096 x 14336 1 1720 / 1711, 2 1732 /
+// 1731, 4 1758 / 1777; 3584 x 18944 1 2892 / 2907, 2 2919 / 2961. A mixer's, whose norm would be made inside the gate/up product: 1536 x 1536 8
+// 1377 / 1244, 3584 x 3584 1 2963 / 2892, 8 3096 / 3025, 16 3265 / 3244, 4096 x 4096 16 1951 / 1939.
+CW_EXPORT int cw_gemm_bf16_join_pays(int M, int N, int K) {
+  int slots, waves;
+  if (!join_plan(M, N, K, cw_num_compute_units(), &slots, &waves)) return 0;
+  const int64_t x = (int64_t)M * K;
+  return x <= 64 * 1024 && (slots <= 8 || K <= 4096 || x <= 16 * 1024) ? 1 : 0;
 }
 
 // The number of sums of squares that cw_gemm_bf16_join leaves of a row (zeros up to a multiple of 4 at the end), 0 where it does not take these sizes.

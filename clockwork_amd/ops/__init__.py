@@ -122,6 +122,7 @@ def _declare(name: str, lib: ctypes.CDLL) -> None:
             "cw_gemm_bf16_group": [I, P, P, P, P, I, I, P],
             "cw_gemm_bf16_join_parts": [I, I, I],
             "cw_gemm_bf16_join_rule": [I, I, I, I],
+            "cw_gemm_bf16_join_pays": [I, I, I],
             "cw_gemm_bf16_join": [P, P, P, P, I, P, P, I, I, I, P],
             "cw_gemm_bf16_swiglu_begun": [P, P, I, F, P, P, L, I, I, I, P],
             "cw_gemm_qkv_rope_bf16": [P, L, P, P, I, P, P, P, P, P, P, L, I, I, I, I, I, P],
@@ -444,6 +445,12 @@ def linear_join_ok(M: int, weight: torch.Tensor, norm_weight: torch.Tensor) -> b
     return (weight.dtype == torch.bfloat16 and weight.is_contiguous() and _aligned(weight) and norm_weight.numel() == weight.shape[0]
             and norm_weight.dtype in (torch.bfloat16, torch.float32)
             and _load("gemm").cw_gemm_bf16_join_parts(M, weight.shape[0], weight.shape[1]) > 0)
+
+
+def linear_join_pays(M: int, weight: torch.Tensor, norm_weight: torch.Tensor) -> bool:
+    """Does ``linear_join`` take the product, and is it the faster way to a block's output? By the rule of
+    ``cw_gemm_bf16_join_pays`` (csrc/gemm.hip)."""
+    return linear_join_ok(M, weight, norm_weight) and bool(_load("gemm").cw_gemm_bf16_join_pays(M, weight.shape[0], weight.shape[1]))
 
 
 def linear_join(x: torch.Tensor, weight: torch.Tensor, resid: torch.Tensor, norm_weight: torch.Tensor, eps: float) -> BegunNorm:

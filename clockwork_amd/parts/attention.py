@@ -352,8 +352,8 @@ class PagedAttention(Part):
         return takes is not None and own_method(self, PagedAttention) and cache.writes and takes(n_tokens, self.qkv_weight, self.spec.head_dim)
 
     def joins_stream(self, n_tokens: int, norm) -> bool:
-        """Can ``forward_joined`` add that many rows to the stream and begin ``norm``?"""
-        return own_method(self, PagedAttention) and self.out_bias is None and ops.linear_join_ok(n_tokens, self.out_weight, norm.weight)
+        """Does ``forward_joined`` add that many rows to the stream and begin ``norm``?"""
+        return own_method(self, PagedAttention) and self.out_bias is None and ops.linear_join_pays(n_tokens, self.out_weight, norm.weight)
 
     def forward_joined(self, x, ctx, cache: EntryCache, resid, norm) -> "ops.BegunNorm":
         """``forward``, its output added to ``resid`` and ``norm`` of that begun."""

@@ -43,8 +43,8 @@ class SwiGLU(Part):
         return own_method(self, SwiGLU) and ops.swiglu_begun_ok(n_tokens, self.gate_up)
 
     def joins_stream(self, n_tokens: int, norm) -> bool:
-        """Can ``forward_joined`` add that many rows to the stream and begin ``norm``?"""
-        return own_method(self, SwiGLU) and ops.linear_join_ok(n_tokens, self.down, norm.weight)
+        """Does ``forward_joined`` add that many rows to the stream and begin ``norm``?"""
+        return own_method(self, SwiGLU) and ops.linear_join_pays(n_tokens, self.down, norm.weight)
 
     def forward_joined(self, x, ctx, resid, norm) -> "ops.BegunNorm":
         """``forward``, its output added to ``resid`` and ``norm`` of that begun."""

@@ -312,6 +312,22 @@ def test_chunks_of_a_row_of_logits_have_few_enough_tokens_for_float64_sums(n, V)
     assert 1 <= chunks <= 64 and 4 * -(-per // 1024) * 2 ** 40 <= 2 ** 53
 
 
+@pytest.mark.parametrize("N,K,rows,not_rows", [(896, 4864, (1, 8, 13), (14, 16)), (1536, 8960, (1, 4, 7), (8, 16)), (2048, 11008, (1, 4, 5), (6, 8)), (3584, 18944, (), (1, 2, 3)),
+                                               (2560, 9728, (1,), (2, 4, 8)), (4096, 14336, (1,), (2, 4)), (1536, 1536, (1, 8, 16), ()), (3584, 3584, (1, 8, 16), ()), (4096, 4096, (16,), ())])
+def test_outputs_join_the_stream_where_that_is_the_faster_way(N, K, rows, not_rows):
+    """The parts ask what pays; the kernel takes more than that (few rows of a long K, timed both ways in whole steps)."""
+    import torch
+
+    from clockwork_amd.parts.mlp import SwiGLU
+
+    ffn, norm = SwiGLU.__new__(SwiGLU), SimpleNamespace(weight=torch.ones(N))
+    ffn.down = torch.zeros(1, dtype=torch.bfloat16).expand(N, K)
+    assert not ffn.joins_stream(1, norm)   # rows with gaps
+    ffn.down = torch.empty(N, K, dtype=torch.bfloat16)
+    assert all(ffn.joins_stream(M, norm) for M in rows) and not any(ffn.joins_stream(M, norm) for M in not_rows)
+    assert all(ops.linear_join_ok(M, ffn.down, norm.weight) == (M <= 16 and M * K <= 72 * 1024) for M in (*rows, *not_rows, 17))
+
+
 def test_few_rows_join_the_stream_between_blocks_only():
     """The mixer's output begins the second norm and the feed-forward's the next block's first one, where the parts take such
     rows and another block follows; the last block leaves its outputs to the final norm."""
